@@ -864,9 +864,11 @@ inline size_t wide_smem(unsigned mt) { return (size_t)mt * NL * FT * sizeof(floa
 // The bit-count backward: a wave per region, three workgroups per CU resident (its 5 x MT sums and the rest take ~160
 // registers at 24 taps: three waves per SIMD);
 // the smallest grid that gives every wave the same number of regions as the resident grid would.
-inline unsigned bits_grid_x(unsigned ftiles, size_t P)
+// At 32 taps they take ~200: two waves per SIMD, two workgroups per CU. (A step of 8 models on 2048 sequences of 90-200 nt,
+// max + average pooling, 32 taps: 7.3 ms through the per-wave LDS tables that any longer filter takes, 0.115 ms this way.)
+inline unsigned bits_grid_x(unsigned mt, unsigned ftiles, size_t P)
 {
-    unsigned gx = 768u / ftiles;
+    unsigned gx = (mt == 32 ? 512u : 768u) / ftiles;
     if (gx < 1) gx = 1;
     // at least two regions per wave: the fold of a workgroup's sums and its slab cost about as much as two regions
     // (measured on a calibration batch of 256 regions x 23 tiles: 26.7 us with two, 29.6 with three, 34.5 with five
@@ -975,16 +977,21 @@ int launch_fprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
 }
 
 template <int PT, int MT>
+int launch_bits(hipStream_t st, unsigned gx, unsigned ftiles, size_t smem, size_t m, size_t F, const uint8_t* X, size_t N, const uint32_t* R,
+                size_t P, const float* pooled, const uint32_t* argmax, const float* dpooled, const unsigned long long* act, float* slabs, size_t stride)
+{
+    auto kern = scanpool_bprop_bits_kernel<PT, MT>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), smem, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
+    return 0;
+}
+
+template <int PT, int MT>
 int launch_dense(hipStream_t st, unsigned gx, unsigned ftiles, size_t smem, const float* W, const float* bias, size_t m, size_t F,
                   const uint8_t* X, size_t N, const uint32_t* R, size_t P, const float* pooled, const uint32_t* argmax,
                   const float* dpooled, const unsigned long long* act, float* slabs, size_t stride)
 {
-    if (act) {
-        auto kern = scanpool_bprop_bits_kernel<PT, MT>;
-        DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-        hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), smem, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
-        return 0;
-    }
+    if (act) return launch_bits<PT, MT>(st, gx, ftiles, smem, m, F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
     auto kern = scanpool_bprop_dense_kernel<PT, MT>;
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, slabs, stride);
@@ -999,8 +1006,21 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
     const unsigned ftiles = dbk::divup(F, FT);
     DBK_CHECK(ftiles <= 65535u, "ValueError: too many filters (%zu) for one launch", F);
     const size_t nW = 4 * m * F, stride = nW + F;
-    const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : (m <= 24 ? 24 : 0));    // the register budget of the dense kernel ends at 24 taps
-    if (mt == 0) {
+    const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : (m <= 24 ? 24 : (m <= 32 ? 32 : 0)));
+    // Average pooling without the forward pass's activity masks: the matrix-core forward writes them again (into the
+    // stream's second scratch buffer, with its pooled values beside them), and the bit-count kernel takes them from
+    // there; less than half the time of recomputing the map through the letter table, whose registers moreover end at 24
+    // taps: longer filters take this way at every size.
+    const size_t mask_bytes = N * ftiles * sizeof(unsigned long long), pooled_bytes = P * F * 2 * sizeof(float);
+    if (PT != DBK_PT_MAX && !act && !dbk::deferred() && (mfma_pays(m, ftiles, P) || mt == 32) && mask_bytes + pooled_bytes <= ((size_t)1 << 30)) {   // (at most 1 GiB of scratch for it)
+        unsigned char* scratch = (unsigned char*)dbk::workspace(mask_bytes + pooled_bytes, st, 1);
+        DBK_CHECK(scratch != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", mask_bytes + pooled_bytes, dbk::workspace_error());
+        unsigned long long* masks = reinterpret_cast<unsigned long long*>(scratch);
+        const int rc = launch_fprop_mfma<PT>(st, ftiles, W, bias, m, F, X, N, R, P, reinterpret_cast<float*>(scratch + mask_bytes), nullptr, masks);
+        if (rc) return rc;
+        act = masks;
+    }
+    if (mt == 0 || (mt == 32 && PT != DBK_PT_MAX && !act)) {
         // any filter length: one kernel does both halves through per-wave LDS tables
         unsigned nw = 4;
         const size_t lutb = PT == DBK_PT_MAX ? 0 : m * NL * FT * sizeof(float);
@@ -1021,35 +1041,25 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
         else hipLaunchKernelGGL(reduce_slabs_kernel, dim3(dbk::ew_grid(stride)), dim3(256), 0, st, dW, dbias, (const float*)slabs, nW, F, gx, overwrite);
         DBK_LAUNCH_OK();
     }
-    // Average pooling without the forward pass's activity masks: the matrix-core forward writes them again (into the
-    // stream's second scratch buffer, with its pooled values beside them), and the bit-count kernel takes them from
-    // there; less than half the time of recomputing the map through the letter table.
-    const size_t mask_bytes = N * ftiles * sizeof(unsigned long long), pooled_bytes = P * F * 2 * sizeof(float);
-    if (PT != DBK_PT_MAX && !act && !dbk::deferred() && mfma_pays(m, ftiles, P) && mask_bytes + pooled_bytes <= ((size_t)1 << 30)) {   // (at most 1 GiB of scratch for it)
-        unsigned char* scratch = (unsigned char*)dbk::workspace(mask_bytes + pooled_bytes, st, 1);
-        DBK_CHECK(scratch != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", mask_bytes + pooled_bytes, dbk::workspace_error());
-        unsigned long long* masks = reinterpret_cast<unsigned long long*>(scratch);
-        const int rc = launch_fprop_mfma<PT>(st, ftiles, W, bias, m, F, X, N, R, P, reinterpret_cast<float*>(scratch + mask_bytes), nullptr, masks);
-        if (rc) return rc;
-        act = masks;
-    }
     // with max+avg pooling the dense half carries the maxima along
     const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P);
-    const unsigned gxs = PT == DBK_PT_MAX ? (max_bits ? bits_grid_x(ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
-    const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? bits_grid_x(ftiles, P) : dense_grid_x(mt, ftiles, P);
-    const size_t smem_s = sparse_smem(m), smem_d = dense_smem(mt);
+    const unsigned gxs = PT == DBK_PT_MAX ? (max_bits ? bits_grid_x(mt, ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
+    const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? bits_grid_x(mt, ftiles, P) : dense_grid_x(mt, ftiles, P);
+    const size_t smem_s = sparse_smem(m), smem_d = mt == 32 ? bits_smem(mt) : dense_smem(mt);
     DBK_CHECK(smem_s <= lds_limit() && smem_d <= lds_limit(), "ValueError: filter length %zu does not fit in LDS", m);
     float* slabs = (float*)dbk::workspace(stride * (gxs + gxd) * sizeof(float), st);
     DBK_CHECK(slabs != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", stride * (gxs + gxd) * sizeof(float), dbk::workspace_error());
     if (gxs && max_bits) {
-        auto kern = mt == 8 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 8> : mt == 16 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 16> : scanpool_bprop_bits_kernel<DBK_PT_MAX, 24>;
+        auto kern = mt == 8 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 8> : mt == 16 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 16>
+                  : mt == 24 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 24> : scanpool_bprop_bits_kernel<DBK_PT_MAX, 32>;
         const size_t smem_b = bits_smem(mt);
         DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_b));
         hipLaunchKernelGGL(kern, dim3(gxs, ftiles), dim3(256), smem_b, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled,
                            (const unsigned long long*)nullptr, slabs, stride);
     } else if (gxs) {
         constexpr int PS = PT == DBK_PT_AVG ? DBK_PT_MAX : PT;
-        auto kern = mt == 8 ? scanpool_bprop_sparse_kernel<PS, 8> : mt == 16 ? scanpool_bprop_sparse_kernel<PS, 16> : scanpool_bprop_sparse_kernel<PS, 24>;
+        auto kern = mt == 8 ? scanpool_bprop_sparse_kernel<PS, 8> : mt == 16 ? scanpool_bprop_sparse_kernel<PS, 16>
+                  : mt == 24 ? scanpool_bprop_sparse_kernel<PS, 24> : scanpool_bprop_sparse_kernel<PS, 32>;
         DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_s));
         hipLaunchKernelGGL(kern, dim3(gxs, ftiles), dim3(64), smem_s, st, (unsigned)m, (unsigned)F, X, N, P, pooled, argmax, dpooled, slabs, stride);
     }
@@ -1059,7 +1069,8 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
         int rc;
         if (mt == 8) rc = launch_dense<PD, 8>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
         else if (mt == 16) rc = launch_dense<PD, 16>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
-        else rc = launch_dense<PD, 24>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
+        else if (mt == 24) rc = launch_dense<PD, 24>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
+        else rc = launch_bits<PD, 32>(st, gxd, ftiles, smem_d, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
         if (rc) return rc;
     }
     if (dbk::deferred_sums* later = dbk::deferred()) { later->slabs = slabs; later->slab_stride = stride; later->nslab = gxs + gxd; }
@@ -1131,7 +1142,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 24 ? 
     wg_t wg;
     const unsigned gi = multi_locate(a, wg);
     const dbk::scan_group& j = a.g[gi];
-    if constexpr (MT == 16 || MT == 24) {
+    if constexpr (MT == 16 || MT == 24 || MT == 32) {
         if (a.wide[gi]) {
             if (j.ptype == DBK_PT_MAX)
                 scanpool_fprop_mfma_body<DBK_PT_MAX, true, false, MT / 4>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, nullptr);
@@ -1170,7 +1181,7 @@ __global__ __launch_bounds__(256) void scanpool_bprop_multi_kernel(const multi_a
     }
 }
 
-inline unsigned multi_tier(size_t m) { return m <= 8 ? 8u : (m <= 16 ? 16u : (m <= 24 ? 24u : 0u)); }
+inline unsigned multi_tier(size_t m) { return m <= 8 ? 8u : (m <= 16 ? 16u : (m <= 24 ? 24u : (m <= 32 ? 32u : 0u))); }
 
 template <typename K>
 int launch_multi(K kern, hipStream_t st, size_t smem, const multi_args& a)
@@ -1201,7 +1212,7 @@ bool scan_multi_takes(size_t m, size_t N, size_t P, unsigned n, const scan_group
         // a max-pooling group on a batch large enough for the k-mer table goes there when stepped alone (other sums, other bits)
         if (g[i].ptype == DBK_PT_MAX && dbk_scanpool_kmer::takes(m, g[i].F, N, P)) return false;
     }
-    return fprop_smem(multi_tier(m), m) <= lds_limit() && wide_smem(24) <= lds_limit() && sparse_smem(m) <= lds_limit() && dense_smem(multi_tier(m)) <= lds_limit();
+    return fprop_smem(multi_tier(m), m) <= lds_limit() && wide_smem(24) <= lds_limit() && sparse_smem(m) <= lds_limit() && bits_smem(multi_tier(m)) <= lds_limit();
 }
 
 int scan_fprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size_t P, unsigned n, const scan_group* g)
@@ -1216,7 +1227,7 @@ int scan_fprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
     for (unsigned i = 0; i < n; ++i) {
         a.g[i] = g[i];
         a.ftiles[i] = dbk::divup(g[i].F, FT);
-        a.wide[i] = mfma_pays(m, a.ftiles[i], P) && m <= 24;      // the kernel body the group's own launch would choose
+        a.wide[i] = mfma_pays(m, a.ftiles[i], P);                 // the kernel body the group's own launch would choose
         // the groups share the GPU: the grids are sized so that all of them are resident together, and a workgroup
         // amortises its filter tile's table over more regions (a region's results do not depend on the grid)
         a.gx[i] = a.wide[i] ? mfma_grid_x(tiles, P) : fprop_grid_x(mt, tiles, P);
@@ -1227,7 +1238,8 @@ int scan_fprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
     if (any_wide && MFMA_SMEM > smem) smem = MFMA_SMEM;
     if (mt == 8) return launch_multi(scanpool_fprop_multi_kernel<8>, st, smem, a);
     if (mt == 16) return launch_multi(scanpool_fprop_multi_kernel<16>, st, smem, a);
-    return launch_multi(scanpool_fprop_multi_kernel<24>, st, smem, a);
+    if (mt == 24) return launch_multi(scanpool_fprop_multi_kernel<24>, st, smem, a);
+    return launch_multi(scanpool_fprop_multi_kernel<32>, st, smem, a);
 }
 
 int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size_t P, unsigned n, scan_group* g)
@@ -1241,7 +1253,7 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
         a.ftiles[i] = dbk::divup(g[i].F, FT);
         // as the group's own launch would choose: the bit-count kernel, or the sparse one for max pooling over long regions
         a.wide[i] = g[i].ptype != DBK_PT_MAX || bits_takes_max(N, P);
-        a.gx[i] = a.wide[i] ? bits_grid_x(a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
+        a.gx[i] = a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
         a.first[i + 1] = a.first[i] + a.gx[i] * a.ftiles[i];
         g[i].slab_stride = 4 * m * (size_t)g[i].F + g[i].F;
         g[i].nslab = a.gx[i];
@@ -1254,11 +1266,12 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
         slabs += g[i].slab_stride * a.gx[i];
         a.g[i] = g[i];
     }
-    const size_t ss = sparse_smem(m), sd = dense_smem(mt);
+    const size_t ss = sparse_smem(m), sd = bits_smem(mt);
     const size_t smem = ss > sd ? ss : sd;
     if (mt == 8) return launch_multi(scanpool_bprop_multi_kernel<8>, st, smem, a);
     if (mt == 16) return launch_multi(scanpool_bprop_multi_kernel<16>, st, smem, a);
-    return launch_multi(scanpool_bprop_multi_kernel<24>, st, smem, a);
+    if (mt == 24) return launch_multi(scanpool_bprop_multi_kernel<24>, st, smem, a);
+    return launch_multi(scanpool_bprop_multi_kernel<32>, st, smem, a);
 }
 
 }  // namespace dbk

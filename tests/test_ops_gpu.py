@@ -557,6 +557,16 @@ def test_scanpool_bprop_with_activity_masks_equals_recomputation(ks, ptype, B, l
         ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, path="kmer", act=act)
 
 
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("B,lo,hi,m,F", [(9, 0, 90, 25, 70), (600, 20, 70, 32, 16), (40, 100, 300, 31, 130), (3, 150, 400, 32, 64)])
+def test_scanpool_bprop_25_to_32_taps(ks, ptype, B, lo, hi, m, F):
+    """The longest tap tier of the bit-count and the sparse backward, with and without masks from the forward pass (without,
+    the call forms them itself at every size): the checks of the shorter tiers at its edges."""
+    test_scanpool_bprop(ks, ptype, B, lo, hi, m, F)
+    if ptype != "max":
+        test_scanpool_bprop_with_activity_masks_equals_recomputation(ks, ptype, B, lo, hi, m, F)
+
+
 @pytest.mark.parametrize("ptype", ["avg", "all"])
 @pytest.mark.parametrize("B,lo,hi,m,F", [(600, 0, 70, 24, 70), (520, 30, 45, 16, 16), (530, 1, 150, 7, 40), (130, 100, 260, 24, 300)])
 def test_scanpool_bprop_many_regions_kernel(ks, ptype, B, lo, hi, m, F):
