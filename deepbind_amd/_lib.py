@@ -89,6 +89,11 @@ _SIGNATURES = {
     "dbk_counter_add": [_P, _P, _U64],
     "dbk_l1_decay": [_P, _I, _P, _P, _P, _Z],
     "dbk_head_fprop": [_P, _Z, _I, _I, _I, _P, _I, _P, _P, _P, _P, _P, _P, _I, _P],
+    "dbk_pack_text": [_P, _P, _P, _Z, _Z, _I, _P, _P],
+    "dbk_pack_windows": [_P, _P, _P, _P, _Z, _Z, _Z, _Z, _Z, _I, _P, _P],
+    "dbk_mutation_map_takes": [_Z, _Z, _I, _Z],
+    "dbk_mutation_map": [_P, _P, _P, _Z, _Z, _P, _Z, _P, _Z, _Z, _I, _Z, _P, _P, _P, _P, _P, _I, _I, _P, _P],
+    "dbk_gather_maps": [_P, _I, _P, _Z, _Z, _I, _P, _P, _P],
     "dbk_train_step": [_P, _P],
     "dbk_train_steps": [_P, _Z, _P],
     "dbk_train_step_single_workspace": [_P, _P],

@@ -1,0 +1,425 @@
+// Device side of the prediction-time callers: packing of sequence text into the scan's input stream, the scores of every
+// single-letter change of a batch (mutation maps), and the compaction of gradient maps.
+//
+// Reference: kangaroo/kangaroo/util.py:50-56,68-74 (letters), data.py:274-354 (packed stream, reverse-complement rows),
+// predict.py:145-345 (predictions, mutation maps, window scans). There every change is one full pass of the net over the
+// whole batch, the stream mutated on the host.
+#include "dbk_common.h"
+#include "scan_common.h"
+
+namespace {
+
+using namespace dbk_scan;
+
+__device__ __forceinline__ unsigned code_of_char(unsigned c)
+{
+    c |= 32u;                                                       // (letters only differ in this bit from their capitals)
+    return c == 'a' ? 0u : c == 'c' ? 1u : c == 'g' ? 2u : (c == 't' || c == 'u') ? 3u : 255u;
+}
+__device__ __forceinline__ uint8_t strand_code(unsigned ch, bool rev)
+{
+    // 'A'..'z' is the only range where setting bit 5 maps a letter to a letter: '!'..'Z' minus 32 are no letters
+    const unsigned c = ch >= 'A' ? code_of_char(ch) : 255u;
+    return (uint8_t)(rev && c < 4u ? 3u - c : c);
+}
+
+// One wave per row (strand of a sequence): its leading pad, then its letters; the last row adds the closing pad.
+// Row r of sequence s starts at padding * r + (strands * offsets[s] + (reverse row ? length : 0)).
+__global__ __launch_bounds__(256) void k_pack_text(const uint8_t* __restrict__ text, const uint32_t* __restrict__ offsets, size_t nseq,
+                                                   unsigned padding, unsigned strands, uint8_t* __restrict__ X, uint32_t* __restrict__ R)
+{
+    const unsigned lane = threadIdx.x & 63;
+    const size_t nrow = nseq * strands, step = (size_t)gridDim.x * (blockDim.x >> 6);
+    for (size_t r = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); r < nrow; r += step) {
+        const size_t s = strands == 2 ? r >> 1 : r;
+        const bool rev = strands == 2 && (r & 1);
+        const uint32_t o = offsets[s], len = offsets[s + 1] - o;
+        const size_t a = (size_t)padding * r + (size_t)strands * o + (rev ? len : 0);
+        for (uint32_t i = lane; i < padding; i += 64) X[a + i] = 255;
+        uint8_t* dst = X + a + padding;
+        for (uint32_t i = lane; i < len; i += 64) dst[i] = strand_code(text[o + (rev ? len - 1 - i : i)], rev);
+        if (r + 1 == nrow)
+            for (uint32_t i = lane; i < padding; i += 64) dst[len + i] = 255;
+        if (lane == 0) { R[2 * r] = (uint32_t)a; R[2 * r + 1] = (uint32_t)(a + padding + len); }
+    }
+}
+
+// Windows of `window` letters every `stride` letters of every sequence, N past its ends; the first window of a sequence
+// starts window - 1 letters before it. first[s] .. first[s + 1] - 1 are sequence s's windows. One thread per byte of X.
+__global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict__ text, const uint32_t* __restrict__ offsets,
+                                                      const uint32_t* __restrict__ first, unsigned nseq, unsigned window, unsigned stride,
+                                                      unsigned padding, unsigned strands, size_t nbyte, uint8_t* __restrict__ X, uint32_t* __restrict__ R)
+{
+    const unsigned span = padding + window;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < nbyte; e += (size_t)gridDim.x * blockDim.x) {
+        const size_t r = e / span;
+        const unsigned o = (unsigned)(e - r * span);
+        const size_t w = strands == 2 ? r >> 1 : r;
+        if (o == 0 && w < first[nseq]) { R[2 * r] = (uint32_t)e; R[2 * r + 1] = (uint32_t)(e + span); }
+        uint8_t v = 255;
+        if (o >= padding && w < first[nseq]) {
+            unsigned lo = 0, hi = nseq - 1;                         // the sequence that holds window w
+            while (lo < hi) { const unsigned mid = (lo + hi + 1) >> 1; if (first[mid] <= w) lo = mid; else hi = mid - 1; }
+            const bool rev = strands == 2 && (r & 1);
+            const unsigned in = rev ? window - 1 - (o - padding) : o - padding;
+            const long at = (long)((w - first[lo]) * stride) + in - (long)(window - 1);
+            const uint32_t base = offsets[lo], len = offsets[lo + 1] - base;
+            if (at >= 0 && at < (long)len) v = strand_code(text[base + at], rev);
+        }
+        X[e] = v;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// mutation maps
+// ---------------------------------------------------------------------------------------------
+// S[4 * p + c] = the net's output for the region around stream position p with the letter at p changed to c, for every
+// letter p of every region (not its leading pad).
+//
+// A change at p moves the `m` rows whose windows hold p and nothing else, so a workgroup takes a few consecutive letters
+// of one region: it scans the region once (16 lanes of filters x 16 lanes of rows, the letter table of 16 filters in
+// LDS), keeps the maximum and the sum of the rows no change of its letters can reach and, one by one, the rows some change
+// can; a wave then takes a letter at a time, its lanes being 4 new letters x 16 filters, scans the m rows of each anew -
+// taps in ascending order, as the forward pass does, so that a change to the letter that is there gives the score that is
+// there - and pools them with what is kept. More than 16 filters take further passes; pooled values meet the dense head in LDS.
+// What bounds it is LDS reads, one per (row, tap): m * m per letter and filter tile, where the reference's way (a pass of the
+// whole net per change) scans length + m - 1 rows per change, and launches 15 kernels for it.
+// Measured: 32 sequences of 60-101 letters, both strands, 16 filters of 24 taps: 0.047 ms, the whole call
+// 0.13 ms from strings to host arrays (74-84 ms when the batch was re-scored once per letter and base).
+//
+// The reference changes letter i of EVERY region in pass i; where a region is shorter than its neighbour's i that lands in
+// the pad behind it, which is the next region's leading pad. Those entries are scored with both changes, the rows of either window anew.
+constexpr unsigned MUT_F = 16, MUT_MAXK = 128, MUT_MAXH = 64;
+constexpr unsigned MUT_TILE = 512;                                  // rows of the region scanned between two stagings of letters
+
+struct mut_args {
+    const float *W, *bias, *W1, *b1, *W2, *b2, *in_scale;
+    const uint8_t* X;
+    const uint32_t* R;
+    size_t N, P;
+    unsigned m, F, k, hidden;
+    int ptype, logistic, strands;
+    float *S, *base;                                                // changed scores (4 per stream position), unchanged ones (per region)
+};
+
+// Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending; the letters at index
+// `at` and `at2` read as `other`. A letter is read once for the four rows it meets.
+template <bool TWO = false>
+__device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, unsigned at,
+                                      unsigned other, float (&z)[4], unsigned at2 = ~0u)
+{
+    z[0] = z[1] = z[2] = z[3] = 0.0f;
+    unsigned l[4];
+#pragma unroll
+    for (unsigned u = 0; u < 3; ++u) l[u + 1] = p + u == at || (TWO && p + u == at2) ? other : let[p + u];
+#pragma unroll 4
+    for (unsigned j = 0; j < m; ++j) {
+        l[0] = l[1]; l[1] = l[2]; l[2] = l[3];
+        l[3] = p + 3 + j == at || (TWO && p + 3 + j == at2) ? other : let[p + 3 + j];
+        const float* t = lut_f + j * NL * MUT_F;
+#pragma unroll
+        for (unsigned u = 0; u < 4; ++u) z[u] += t[l[u]];
+    }
+}
+
+// LDS, in this order: letter table [m][NL][16], rows a change can reach [pos + m - 1][16] (rectified), two fold areas [2][16][16],
+// pooled values [pos + 1][4][k], rows of the region's head, i.e. those whose windows hold letters of its leading pad, [m][16]; letters of a
+// tile of rows and their windows, letters of the rows a change can reach, letters of the head rows.
+// (scan4 looks 3 rows past the last one asked for.)
+__host__ __device__ inline unsigned mut_tile_letters(unsigned m) { return (MUT_TILE + m + 3 + 3) & ~3u; }
+__host__ __device__ inline unsigned mut_reach_letters(unsigned pos, unsigned m) { return (pos + 2 * m + 4 + 3) & ~3u; }
+inline size_t mut_smem(unsigned pos, size_t m, size_t k)
+{
+    return ((size_t)m * NL * MUT_F + (pos + m - 1) * MUT_F + 2 * 16 * MUT_F + (pos + 1) * 4 * k + m * MUT_F) * sizeof(float) +
+           mut_tile_letters((unsigned)m) + mut_reach_letters(pos, (unsigned)m) + mut_reach_letters(0, (unsigned)m);
+}
+
+template <unsigned MUT_POS>
+__global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
+{
+    extern __shared__ __align__(16) float msm[];
+    const unsigned m = a.m, pad = m - 1;
+    const size_t r = blockIdx.x;
+    const unsigned ra = a.R[2 * r], rb = a.R[2 * r + 1];
+    const unsigned len = rb - ra > pad ? rb - ra - pad : 0u;
+    const unsigned i0 = blockIdx.y * MUT_POS;
+    if (i0 >= len && blockIdx.y != 0) return;
+    const unsigned npos = i0 < len ? (len - i0 < MUT_POS ? len - i0 : MUT_POS) : 0u;
+    const unsigned tid = threadIdx.x, lane = tid & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    float* lut = msm;
+    float* rows = lut + m * NL * MUT_F;
+    float* fold = rows + (MUT_POS + m - 1) * MUT_F;
+    float* pooled = fold + 2 * 16 * MUT_F;
+    float* head = pooled + (MUT_POS + 1) * 4 * a.k;
+    uint8_t* tile = reinterpret_cast<uint8_t*>(head + m * MUT_F);
+    uint8_t* let = tile + mut_tile_letters(m);
+    uint8_t* hlet = let + mut_reach_letters(MUT_POS, m);
+    const size_t n = a.N >= m ? a.N - m + 1 : 0;                   // rows the scan defines; later rows are relu(bias)
+    // rows some change of these letters reaches: [s0, s1)
+    const unsigned q0 = ra + pad + i0;                             // stream position of the first letter
+    const unsigned s0 = q0 - pad, s1 = npos ? q0 + npos : s0;
+    auto stage = [&](uint8_t* to, size_t from, unsigned count) {   // letters as offsets into a tap's part of the table
+        for (unsigned e = tid; e < count; e += 256) to[e] = (uint8_t)((from + e < a.N ? letter_of(a.X[from + e]) : 5u) * MUT_F);
+    };
+    stage(let, s0, mut_reach_letters(MUT_POS, m));
+    // the change of the region before this one that lands in this one's leading pad
+    const bool shorter_before = a.strands == 1 && r > 0;
+    const unsigned pa = shorter_before ? a.R[2 * r - 2] : 0u, pb = shorter_before ? a.R[2 * r - 1] : 0u;
+    // (pass `i` of the reference: letter i of every region, i.e. stream position pad + pa + i of that one)
+    auto spills = [&](unsigned pass) { return shorter_before && pb - pa > pass && pad + pa + pass >= pb && pad + pa + pass < ra + pad; };
+    bool spill_here = false;
+    for (unsigned i = 0; i < npos; ++i) spill_here |= spills(i0 + i);
+    // rows of the head that no change of these letters reaches: with a spill they are kept one by one as well
+    const unsigned h1 = spill_here ? (s0 < ra + pad ? s0 : ra + pad) : ra;
+    if (spill_here) stage(hlet, ra, mut_reach_letters(0, m));
+    const unsigned f = tid & 15u, rl = tid >> 4;
+    const unsigned kper = a.ptype == DBK_PT_ALL ? 2u : 1u;
+    const float count = (float)(rb - ra);
+    const float* lut_f = lut + f;
+
+    for (unsigned f0 = 0; f0 < a.F; f0 += MUT_F) {
+        const bool on = f0 + f < a.F;
+        const float bf = on ? a.bias[f0 + f] : 0.0f;
+        __syncthreads();                                            // the previous tile's table and rows are no longer read
+        for (unsigned e = tid; e < m * MUT_F; e += 256) {
+            const unsigned j = e / MUT_F, c = f0 + e % MUT_F;
+            float w[4];
+#pragma unroll
+            for (int l = 0; l < 4; ++l) w[l] = c < a.F ? a.W[(size_t)(4 * j + l) * a.F + c] : 0.0f;
+            float z = w[0];
+            z += w[1]; z += w[2]; z += w[3];
+            float* t = lut + (size_t)j * NL * MUT_F + e % MUT_F;
+            t[0] = w[0]; t[MUT_F] = w[1]; t[2 * MUT_F] = w[2]; t[3 * MUT_F] = w[3]; t[4 * MUT_F] = z * 0.25f; t[5 * MUT_F] = 0.0f;
+        }
+        // ---- the region as it is: rows out of reach folded, rows in reach kept
+        float mx = 0.0f, sum = 0.0f;
+        for (unsigned t0 = ra; t0 < rb; t0 += MUT_TILE) {
+            __syncthreads();
+            stage(tile, t0, mut_tile_letters(m));
+            __syncthreads();
+            const unsigned t1 = rb - t0 < MUT_TILE ? rb : t0 + MUT_TILE;
+            for (unsigned p = t0 + 4 * rl; p < t1; p += 64) {
+                float z[4];
+                scan4(lut_f, tile, p - t0, m, ~0u, 0u, z);
+#pragma unroll
+                for (unsigned u = 0; u < 4; ++u) {
+                    if (p + u >= t1) break;
+                    float v = (p + u < n ? z[u] : 0.0f) + bf;
+                    v = v > 0.0f ? v : 0.0f;
+                    if (p + u >= s0 && p + u < s1) rows[(p + u - s0) * MUT_F + f] = v;
+                    else if (p + u < h1) head[(p + u - ra) * MUT_F + f] = v;
+                    else { mx = v > mx ? v : mx; sum += v; }
+                }
+            }
+        }
+        fold[rl * MUT_F + f] = mx;
+        fold[(16 + rl) * MUT_F + f] = sum;
+        __syncthreads();
+        mx = 0.0f; sum = 0.0f;
+#pragma unroll
+        for (unsigned t = 0; t < 16; ++t) {
+            const float v = fold[t * MUT_F + f];
+            mx = v > mx ? v : mx;
+            sum += fold[(16 + t) * MUT_F + f];
+        }
+        // ---- one letter per wave at a time (the item behind the last one is the region unchanged): lane = (new letter, filter)
+        const unsigned c = lane >> 4, coff = c * MUT_F;
+        for (unsigned i = wave; i < npos + (i0 == 0 ? 1u : 0u); i += 4) {
+            float bm = mx, bs = sum;
+            auto pool = [&](float v) { bm = v > bm ? v : bm; bs += v; };
+            // rows [lo, hi) among the kept ones are scanned anew: those of letter q0 + i's windows, and with a spill the head as well
+            const bool both = i < npos && spills(i0 + i);
+            const unsigned q2 = pad + pa + i0 + i;
+            unsigned hp = 0;                                         // rows of the head to scan anew
+            if (both) {
+                hp = q2 + 1 - ra;                                    // rows ra .. q2 hold it
+                if (hp > h1 - ra) hp = h1 - ra;
+                for (unsigned p = 0; p < hp; p += 4) {
+                    float z[4];
+                    scan4(lut_f, hlet, p, m, q2 - ra, coff, z);
+#pragma unroll
+                    for (unsigned u = 0; u < 4; ++u)
+                        if (p + u < hp) {
+                            const float v = ((size_t)ra + p + u < n ? z[u] : 0.0f) + bf;
+                            pool(v > 0.0f ? v : 0.0f);
+                        }
+                }
+            }
+            for (unsigned p = hp; p < h1 - ra; ++p) pool(head[p * MUT_F + f]);
+            const unsigned rest = s1 - s0;
+            unsigned lo = i < npos ? i : rest, hi = i < npos ? i + m : rest;
+            if (both && q2 >= s0) lo = 0;
+            for (unsigned p = 0; p < lo; ++p) pool(rows[p * MUT_F + f]);
+            for (unsigned p = lo; p < hi; p += 4) {
+                float z[4];
+                if (both) scan4<true>(lut_f, let, p, m, i + pad, coff, z, q2 - s0);
+                else scan4(lut_f, let, p, m, i + pad, coff, z);
+#pragma unroll
+                for (unsigned u = 0; u < 4; ++u)
+                    if (p + u < hi) {
+                        const float v = ((size_t)s0 + p + u < n ? z[u] : 0.0f) + bf;
+                        pool(v > 0.0f ? v : 0.0f);
+                    }
+            }
+            for (unsigned p = hi; p < rest; ++p) pool(rows[p * MUT_F + f]);
+            if (on) {
+                float* to = pooled + (i * 4 + c) * a.k + (f0 + f) * kper;
+                if (a.ptype == DBK_PT_MAX) to[0] = bm;
+                else if (a.ptype == DBK_PT_AVG) to[0] = bs / count;
+                else { to[0] = bm; to[1] = bs / count; }
+            }
+        }
+    }
+    __syncthreads();
+    // ---- the dense head: 16 lanes per (letter, change) item, hidden units dealt over them
+    const float sc = a.in_scale ? a.in_scale[0] : 1.0f;
+    const unsigned nitem = (npos + (i0 == 0 ? 1u : 0u)) * 4, g = tid >> 4, hl = tid & 15u;
+    for (unsigned it = g; it < nitem; it += 16) {
+        const float* x = pooled + it * a.k;
+        float out = 0.0f;
+        if (a.hidden > 0) {
+            for (unsigned h = hl; h < a.hidden; h += 16) {
+                float z = 0.0f;
+#pragma unroll 8
+                for (unsigned kk = 0; kk < a.k; ++kk) z = __builtin_fmaf(x[kk] * sc, a.W1[(size_t)kk * a.hidden + h], z);
+                z += a.b1[h];
+                out += (z > 0.0f ? z : 0.0f) * a.W2[h];
+            }
+        } else {
+            for (unsigned kk = hl; kk < a.k; kk += 16) out += x[kk] * sc * a.W1[kk];
+        }
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1) out += __shfl_xor(out, d, 16);
+        out += a.hidden > 0 ? a.b2[0] : a.b1[0];
+        if (a.logistic) out = 1.0f / (1.0f + expf(-out));
+        if (hl == 0) {
+            const unsigned i = it >> 2, c = it & 3u;
+            if (i < npos) a.S[4 * ((size_t)q0 + i) + c] = out;
+            else if (c == 0) a.base[r] = out;
+        }
+    }
+}
+
+// The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
+// is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. One workgroup per sequence.
+__global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const float* __restrict__ S,
+                                                      const float* __restrict__ base, float* __restrict__ Z, float* __restrict__ map)
+{
+    const size_t s = blockIdx.x, r = s * (unsigned)strands;
+    const unsigned ra = R[2 * r], len = R[2 * r + 1] - ra - pad;
+    const size_t out = ((size_t)ra - (size_t)pad * r) / (unsigned)strands;       // letters of the sequences before this one
+    float z = base[r];
+    if (strands == 2) z = base[r + 1] > z ? base[r + 1] : z;
+    const unsigned mirror = strands == 2 ? R[2 * r + 3] - 1 : 0u;
+    for (unsigned e = threadIdx.x; e < 4 * len; e += blockDim.x) {
+        const unsigned i = e >> 2, c = e & 3u;
+        float v = S[4 * ((size_t)ra + pad + i) + c];
+        if (strands == 2) {
+            const float w = S[4 * (size_t)(mirror - i) + 3 - c];
+            v = w > v ? w : v;
+        }
+        map[4 * out + e] = (z > v ? z : v) > 0.0f ? v - z : 0.0f;
+    }
+    if (threadIdx.x == 0) Z[s] = z;
+}
+
+// The rows of dX (4 values per stream position) that belong to the winning strand's letters, one sequence after another.
+// Z: the rows' predictions; with both strands the forward row wins ties. One workgroup per sequence.
+template <typename T, typename T4>
+__global__ __launch_bounds__(256) void k_gather_maps(const uint32_t* __restrict__ R, unsigned pad, int strands, const T* __restrict__ Z,
+                                                     const T4* __restrict__ dX, T4* __restrict__ map)
+{
+    const size_t s = blockIdx.x;
+    size_t r = s * (unsigned)strands;
+    const size_t out = ((size_t)R[2 * r] - (size_t)pad * r) / (unsigned)strands;
+    if (strands == 2 && Z[r] < Z[r + 1]) r += 1;
+    const unsigned ra = R[2 * r], len = R[2 * r + 1] - ra - pad;
+    for (unsigned i = threadIdx.x; i < len; i += blockDim.x) map[out + i] = dX[(size_t)ra + pad + i];
+}
+
+}  // namespace
+
+extern "C" {
+
+int dbk_pack_text(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, size_t nseq, size_t padding, int strands,
+                  uint8_t* X, uint32_t* R)
+{
+    DBK_CHECK(strands == 1 || strands == 2, "ValueError: strands must be 1 or 2");
+    if (nseq == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(offsets && X && R, "ValueError: null pointer argument");
+    unsigned grid = dbk::divup(nseq * strands, 4);
+    if (grid > 8192u) grid = 8192u;
+    hipLaunchKernelGGL(k_pack_text, dim3(grid), dim3(256), 0, dbk::as_stream(stream), text, offsets, nseq, (unsigned)padding, (unsigned)strands, X, R);
+    DBK_LAUNCH_OK();
+}
+
+int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, const uint32_t* first, size_t nseq, size_t nwindow,
+                     size_t window, size_t stride, size_t padding, int strands, uint8_t* X, uint32_t* R)
+{
+    DBK_CHECK(strands == 1 || strands == 2, "ValueError: strands must be 1 or 2");
+    DBK_CHECK(window >= 1 && stride >= 1, "ValueError: window and stride must be >= 1");
+    if (nseq == 0 || nwindow == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(offsets && first && X && R, "ValueError: null pointer argument");
+    const size_t nbyte = nwindow * strands * (padding + window) + padding;
+    hipLaunchKernelGGL(k_pack_windows, dim3(dbk::ew_grid(nbyte)), dim3(256), 0, dbk::as_stream(stream), text, offsets, first, (unsigned)nseq,
+                       (unsigned)window, (unsigned)stride, (unsigned)padding, (unsigned)strands, nbyte, X, R);
+    DBK_LAUNCH_OK();
+}
+
+int dbk_mutation_map_takes(size_t m, size_t nfilter, int ptype, size_t hidden)
+{
+    const size_t k = nfilter * (ptype == DBK_PT_ALL ? 2 : 1);
+    return m >= 1 && m <= 64 && nfilter >= 1 && k <= MUT_MAXK && hidden <= MUT_MAXH &&
+           (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL) && mut_smem(16, m, k) <= 65536;
+}
+
+int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* X, size_t N,
+                     const uint32_t* regions, size_t nregion, size_t longest, int ptype, size_t hidden, const float* W1, const float* b1,
+                     const float* W2, const float* b2, const float* in_scale, int apply_logistic, int strands, float* Z, float* map)
+{
+    DBK_CHECK(strands == 1 || (strands == 2 && nregion % 2 == 0), "ValueError: strands must be 1, or 2 with an even number of regions");
+    DBK_CHECK(dbk_mutation_map_takes(m, nfilter, ptype, hidden), "NotImplementedError: the mutation map kernel does not take %zu filters of %zu taps with %zu hidden units and pooling %d",
+              nfilter, m, hidden, ptype);
+    if (nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(W && bias && X && regions && W1 && b1 && Z && map, "ValueError: null pointer argument");
+    DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
+    // letters per workgroup: 16 where that still gives every CU several workgroups, else fewer, as a workgroup's first scan of
+    // its region costs less than an idle CU (64 regions of up to 101 letters: 159 us a call with 4, 179 with 16; 256 of 101: 312 / 288)
+    const size_t letters = longest > 0 ? longest : 1;
+    const unsigned pos = nregion * dbk::divup(letters, 16) >= 1024 ? 16u : nregion * dbk::divup(letters, 8) >= 1024 ? 8u : 4u;
+    const unsigned gy = dbk::divup(letters, pos);
+    DBK_CHECK(nregion <= 0x7fffffffu && gy <= 65535u, "ValueError: too many regions (%zu) or letters per region (%zu) for one launch", nregion, longest);
+    hipStream_t st = dbk::as_stream(stream);
+    float* scratch = (float*)dbk::workspace((4 * N + nregion) * sizeof(float), st);
+    DBK_CHECK(scratch != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", (4 * N + nregion) * sizeof(float), dbk::workspace_error());
+    mut_args a;
+    a.W = W; a.bias = bias; a.W1 = W1; a.b1 = b1; a.W2 = W2; a.b2 = b2; a.in_scale = in_scale;
+    a.X = X; a.R = regions; a.N = N; a.P = nregion;
+    a.m = (unsigned)m; a.F = (unsigned)nfilter; a.k = (unsigned)(nfilter * (ptype == DBK_PT_ALL ? 2 : 1)); a.hidden = (unsigned)hidden;
+    a.ptype = ptype; a.logistic = apply_logistic; a.strands = strands;
+    a.S = scratch; a.base = scratch + 4 * N;
+    auto kern = pos == 16 ? k_mutation_scores<16> : (pos == 8 ? k_mutation_scores<8> : k_mutation_scores<4>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(256), mut_smem(pos, m, a.k), st, a);
+    hipLaunchKernelGGL(k_mutation_map, dim3((unsigned)(nregion / strands)), dim3(256), 0, st, regions, (unsigned)(m - 1), strands,
+                       (const float*)a.S, (const float*)a.base, Z, map);
+    DBK_LAUNCH_OK();
+}
+
+int dbk_gather_maps(dbk_stream_t stream, int dtype, const uint32_t* regions, size_t nregion, size_t padding, int strands, const void* Z,
+                    const void* dX, void* map)
+{
+    DBK_DTYPE_OK(dtype);
+    DBK_CHECK(strands == 1 || (strands == 2 && nregion % 2 == 0), "ValueError: strands must be 1, or 2 with an even number of regions");
+    if (nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(regions && Z && dX && map, "ValueError: null pointer argument");
+    const dim3 grid((unsigned)(nregion / strands));
+    if (dtype == DBK_F32)
+        hipLaunchKernelGGL((k_gather_maps<float, float4>), grid, dim3(256), 0, dbk::as_stream(stream), regions, (unsigned)padding, strands,
+                           (const float*)Z, (const float4*)dX, (float4*)map);
+    else
+        hipLaunchKernelGGL((k_gather_maps<double, double4>), grid, dim3(256), 0, dbk::as_stream(stream), regions, (unsigned)padding, strands,
+                           (const double*)Z, (const double4*)dX, (double4*)map);
+    DBK_LAUNCH_OK();
+}
+
+}  // extern "C"

@@ -44,10 +44,18 @@ def ord2acgt(x):
     return _ORD2ACGT[np.asarray(x, dtype=np.uint8).ravel()].tobytes().decode("latin-1")
 
 
+_NORMAL_TABLE = _ORD2ACGT[_ACGT2ORD].tobytes()
+_COMPLEMENT_TABLE = _COMPLEMENT.tobytes()
+
+
+def normalize(b):
+    """The letters the packed stream knows, from bytes: ACGT (U as T, either case), N for anything else."""
+    return b.translate(_NORMAL_TABLE).decode("latin-1")
+
+
 def revcomp(s):
     """Reverse complement of a DNA/RNA string (U pairs to A, unknown letters to N)."""
-    b = np.frombuffer(s.encode("latin-1"), dtype=np.uint8)
-    return _COMPLEMENT[b[::-1]].tobytes().decode("latin-1")
+    return s.encode("latin-1")[::-1].translate(_COMPLEMENT_TABLE).decode("latin-1")
 
 
 def insert_reverse_complements(seqs):

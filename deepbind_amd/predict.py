@@ -3,14 +3,15 @@ mutation maps and sliding-window scans for one trained model.
 
 Mirrors the reference's prediction module (code/libs/kangaroo/kangaroo/predict.py:145-345):
 `maskout_revcomp`, `gen_convnet_predictions` and `gen_convnet_predictionmaps`, with the model
-evaluation replaced by `SequenceNet` calls. The mutation map re-scores the batch once per
-(position, base) as the reference does, but mutates the packed stream and collects the
-differences on the device, so a batch costs 4 x (longest region) small launches and one copy
-back instead of as many host round trips.
+evaluation replaced by `SequenceNet` calls. Strings go to the device as they are: packing them, cutting
+windows out of them and picking a map's rows are kernels. A mutation map is one launch that re-scans only the
+rows a changed letter moves (nets whose shape that kernel does not take re-score the batch once per (position,
+base), as the reference does, the stream mutated and the differences collected on the device).
 """
 import numpy as np
 import torch
 
+from . import _lib
 from . import data as _data
 
 _RCINDEX = (3, 2, 1, 0)
@@ -59,6 +60,69 @@ def _finite_diff(net, Xd, Rd, R, Z, dX):
             dX[(pad + a + i)[rows], j] = dZ[(rows // 2) if rc else rows, 0]
 
 
+class _Text(object):
+    """Sequence strings as the device takes them: their letters end to end, and where each begins."""
+
+    def __init__(self, seqs):
+        seqs = [s if isinstance(s, str) else bytes(s).decode("latin-1") for s in seqs]
+        self.bytes = np.frombuffer("".join(seqs).encode("latin-1"), dtype=np.uint8)
+        self.lens = np.fromiter(map(len, seqs), dtype=np.int64, count=len(seqs))
+        self.offsets = np.zeros(len(seqs) + 1, dtype=np.int64)
+        np.cumsum(self.lens, out=self.offsets[1:])
+
+    def upload(self, device, *tables):
+        """One copy to the device: (offsets, the further uint32 tables, letters)."""
+        words = [np.asarray(t, dtype=np.uint32) for t in (self.offsets,) + tables]
+        buf = torch.from_numpy(np.concatenate([w.view(np.uint8) for w in words] + [self.bytes])).to(device)
+        out, at = [], 0
+        for w in words:
+            out.append(buf[at:at + w.nbytes])
+            at += w.nbytes
+        return out + [buf[at:]]
+
+    def strings(self, reverse=None):
+        """The sequences in the packed stream's letters (ACGT, else N); those marked in `reverse` as their reverse complement."""
+        fwd = _data.normalize(self.bytes.tobytes())
+        n, o = len(fwd), self.offsets.tolist()
+        if reverse is None or not reverse.any():
+            return [fwd[a:b] for a, b in zip(o[:-1], o[1:])]
+        rev = _data.revcomp(fwd)
+        return [rev[n - b:n - a] if r else fwd[a:b] for a, b, r in zip(o[:-1], o[1:], reverse.tolist())]
+
+
+def _pack(net, text):
+    """(X, R) of the batch on the device, as data.pack_sequences lays them out."""
+    strands, pad, n = (2 if net.reverse_complement else 1), net.m - 1, len(text.lens)
+    offsets, letters = text.upload(net.device)
+    X = torch.empty((strands * (n * pad + len(text.bytes)) + pad, 1), dtype=torch.uint8, device=net.device)
+    R = torch.empty((n * strands, 2), dtype=torch.uint32, device=net.device)
+    _lib.call("dbk_pack_text", _lib.stream(), _lib.ptr(letters), _lib.ptr(offsets), n, pad, strands, _lib.ptr(X), _lib.ptr(R))
+    return X, R
+
+
+def _split(maps, text):
+    o = text.offsets.tolist()
+    return [maps[a:b] for a, b in zip(o[:-1], o[1:])]
+
+
+def _mutation_maps(net, X, R, text):
+    """(Z (nseq, 1), map (letters, 4)) of the batch, or None when the kernel does not take the net's shape."""
+    ptype = _lib.str2pooltype[net.pool]
+    if net.dtype != torch.float32 or not _lib.dll().dbk_mutation_map_takes(net.m, net.nfilter, ptype, net.hidden):
+        return None
+    p = net.p
+    Wc = p["Wc"] if net.input_dropout <= 0 else p["Wc"] * (1.0 - net.input_dropout)
+    scale = (1.0 - net.dropout) if net.use_dropout else None
+    n = len(text.lens)
+    out = torch.empty(n + 4 * len(text.bytes), dtype=torch.float32, device=net.device)       # (one copy back to the host)
+    Z, maps = out[:n], out[n:]
+    _lib.call("dbk_mutation_map", _lib.stream(), _lib.ptr(Wc), _lib.ptr(p["bc"]), net.m, net.nfilter, _lib.ptr(X), X.numel(), _lib.ptr(R),
+              R.shape[0], int(text.lens.max()), ptype, net.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")),
+              _lib.ptr(p.get("b2")), _lib.ptr(scale), int(net.loss == "nll"), 2 if net.reverse_complement else 1, _lib.ptr(Z), _lib.ptr(maps))
+    out = out.cpu().numpy()
+    return out[:n].reshape(-1, 1), out[n:].reshape(-1, 4)
+
+
 def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     """Scores a list of sequence strings with a single-model SequenceNet.
 
@@ -71,28 +135,43 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     rc, pad = net.reverse_complement, net.m - 1
     preds, gmaps = [], ([] if want_gmaps else None)
     for s0 in range(0, len(seqs), batchsize):
-        X, R = _data.pack_sequences(seqs[s0:s0 + batchsize], pad, reverse_complement=rc)
-        Xd = torch.from_numpy(X).to(net.device)
-        Rd = torch.from_numpy(R).to(net.device)
+        text = _Text(seqs[s0:s0 + batchsize])
+        X, R = _pack(net, text)
         if not want_gmaps:
-            preds.append(net.predict(Xd, Rd).cpu().numpy())
+            preds.append(net.predict(X, R).cpu().numpy())
             continue
-        Zall, dX = net.input_gradients(Xd, Rd)
+        fused = _mutation_maps(net, X, R, text) if want_gmaps == "finite_diff" else None
+        if fused is not None:
+            preds.append(fused[0])
+            gmaps += zip(text.strings(), _split(fused[1], text))
+            continue
+        Zall, dX = net.input_gradients(X, R)
         Zh, Zmask = maskout_revcomp(Zall.cpu().numpy(), rc)
         preds.append(Zh)
-        Ri = R.astype(np.int64)
         if want_gmaps == "finite_diff":
-            _finite_diff(net, Xd, Rd, Ri, torch.from_numpy(Zh).to(net.device), dX)
+            Rh = R.cpu().numpy().astype(np.int64)
+            _finite_diff(net, X, R, Rh, torch.from_numpy(Zh).to(net.device), dX)
             dXh = dX.cpu().numpy()
-            fwd = Ri[::2] if rc else Ri
-            gmaps += [(_data.ord2acgt(X[a + pad:b]), dXh[a + pad:b].copy()) for a, b in fwd]
-        else:
-            dXh = dX.cpu().numpy()
-            maps = [(_data.ord2acgt(X[a + pad:b]), dXh[a + pad:b].copy()) for a, b in Ri]
-            if Zmask is not None:
-                maps = [mp for mp, keep in zip(maps, Zmask.ravel()) if keep]
-            gmaps += maps
+            gmaps += [(s, dXh[a + pad:b].copy()) for s, (a, b) in zip(text.strings(), Rh[::2] if rc else Rh)]
+            continue
+        maps = torch.empty((len(text.bytes), 4), dtype=dX.dtype, device=dX.device)
+        _lib.call("dbk_gather_maps", _lib.stream(), _lib.dtype_code(dX), _lib.ptr(R), R.shape[0], pad, 2 if rc else 1, _lib.ptr(Zall),
+                  _lib.ptr(dX), _lib.ptr(maps))
+        reverse = Zmask.reshape(-1, 2)[:, 1] if Zmask is not None else None
+        gmaps += zip(text.strings(reverse), _split(maps.cpu().numpy(), text))
     return np.vstack(preds), gmaps
+
+
+def _score_windows(net, raws, nwin, windowsize, stride):
+    """Predictions of all windows of a few sequences: the windows are cut on the device."""
+    text = _Text(raws)
+    strands, pad, total = (2 if net.reverse_complement else 1), net.m - 1, int(sum(nwin))
+    offsets, first, letters = text.upload(net.device, np.concatenate([[0], np.cumsum(nwin)]))
+    X = torch.empty((total * strands * (pad + windowsize) + pad, 1), dtype=torch.uint8, device=net.device)
+    R = torch.empty((total * strands, 2), dtype=torch.uint32, device=net.device)
+    _lib.call("dbk_pack_windows", _lib.stream(), _lib.ptr(letters), _lib.ptr(offsets), _lib.ptr(first), len(raws), total, windowsize, stride,
+              pad, strands, _lib.ptr(X), _lib.ptr(R))
+    return net.predict(X, R).cpu().numpy()
 
 
 def gen_predictionmaps(net, seqs, stride=1, windowsize=20, want_gmaps=False):
@@ -103,17 +182,20 @@ def gen_predictionmaps(net, seqs, stride=1, windowsize=20, want_gmaps=False):
     if want_gmaps and stride != 1:
         # the reference's aggregation (predict.py:330-340) slices rows that only line up for stride 1
         raise ValueError("window-averaged gradient maps need stride 1 (got %d)" % stride)
+    assert net.ninst == 1, "prediction maps are defined for one model at a time"
     pmaps, gmaps = [], ([] if want_gmaps else None)
     chunk = 32
     for c0 in range(0, len(seqs), chunk):
         raws = list(seqs[c0:c0 + chunk])
-        windows, nwin = [], []
-        for raw in raws:
-            padseq = "N" * (windowsize - 1) + raw + "N" * (windowsize - 1)
-            w = [padseq[i:i + windowsize] for i in range(0, max(1, len(padseq) - windowsize + 1), stride)]
-            windows += w
-            nwin.append(len(w))
-        Z, wmaps = gen_predictions(net, windows, want_gmaps=want_gmaps, batchsize=len(windows))
+        nwin = [len(range(0, max(1, len(raw) + windowsize - 1), stride)) for raw in raws]
+        if want_gmaps or windowsize < 2:         # (one-letter windows have no N around them: an empty sequence's window is empty)
+            windows = []
+            for raw in raws:
+                padseq = "N" * (windowsize - 1) + raw + "N" * (windowsize - 1)
+                windows += [padseq[i:i + windowsize] for i in range(0, max(1, len(padseq) - windowsize + 1), stride)]
+            Z, wmaps = gen_predictions(net, windows, want_gmaps=want_gmaps, batchsize=len(windows))
+        else:
+            Z = _score_windows(net, raws, nwin, windowsize, stride)
         edges = np.cumsum([0] + nwin)
         for i, raw in enumerate(raws):
             pmaps.append(Z[edges[i]:edges[i + 1]].ravel().copy())

@@ -415,6 +415,34 @@ int dbk_head_train(dbk_stream_t stream, size_t n, int nblock, int k, int hidden,
  * captured HIP graph draws fresh masks on every replay). */
 int dbk_counter_add(dbk_stream_t stream, uint64_t* counter, uint64_t delta);
 
+/* ------------------------------------------------------------------ prediction-time callers */
+
+/* Text to packed stream: nseq sequences of bytes, sequence s at text[offsets[s]] .. text[offsets[s+1] - 1], become X
+ * (strands * (nseq * padding + letters) + padding bytes: A, C, G, T/U in either case -> 0..3, anything else and the pads ->
+ * 255) and its region table R (nseq * strands, 2). strands = 2 interleaves every sequence with its reverse complement.
+ * reference: kangaroo/kangaroo/util.py:50-56,68-74, data.py:274-354 (on the host there). */
+int dbk_pack_text(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, size_t nseq, size_t padding, int strands,
+                  uint8_t* X, uint32_t* R);
+/* The same for every window of `window` letters, `stride` apart, of sequences with window - 1 N on either side:
+ * sequence s has the windows first[s] .. first[s+1] - 1 (first[nseq] = nwindow). X: nwindow * strands * (padding + window) +
+ * padding bytes. reference: kangaroo/kangaroo/predict.py:279-300. */
+int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, const uint32_t* first, size_t nseq, size_t nwindow,
+                     size_t window, size_t stride, size_t padding, int strands, uint8_t* X, uint32_t* R);
+/* Scores and mutation maps of one model: Z (nregion / strands) the net's outputs (with strands = 2 the larger of each
+ * pair's), map (letters of all sequences, 4): output with that letter changed to that base, minus the output, where the
+ * larger of the two is positive, else 0. X, regions as dbk_pack_text lays them out for padding = m - 1; longest: the longest
+ * sequence's letters. Weights as in dbk_head_fprop with nblock = 1 and no feature columns. Entries of a sequence shorter than
+ * the one before it see the reference's spill of that one's changes into the pad between them.
+ * dbk_mutation_map_takes: 1 for shapes the kernel takes. reference: kangaroo/kangaroo/predict.py:201-240. */
+int dbk_mutation_map_takes(size_t m, size_t nfilter, int ptype, size_t hidden);
+int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* X, size_t N,
+                     const uint32_t* regions, size_t nregion, size_t longest, int ptype, size_t hidden, const float* W1, const float* b1,
+                     const float* W2, const float* b2, const float* in_scale, int apply_logistic, int strands, float* Z, float* map);
+/* map (letters of all sequences, 4): the rows of dX (N, 4) at every sequence's letters, with strands = 2 those of the row of
+ * the pair whose prediction Z (nregion) is larger. reference: kangaroo/kangaroo/predict.py:188-199. */
+int dbk_gather_maps(dbk_stream_t stream, int dtype, const uint32_t* regions, size_t nregion, size_t padding, int strands, const void* Z,
+                    const void* dX, void* map);
+
 /* ------------------------------------------------------------------ one whole optimiser step */
 
 /* Everything one step of a group of `nmodel` same-architecture models touches. The parameters, their

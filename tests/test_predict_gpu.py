@@ -96,3 +96,52 @@ def test_gen_predictionmaps(rc, stride, want):
         assert gm is None
     with pytest.raises(ValueError):
         predict.gen_predictionmaps(net, seqs, stride=2, windowsize=12, want_gmaps=True)
+
+
+@pytest.mark.parametrize("pool,hidden,loss,rc,m,F", [("max", 32, "nll", True, 24, 16), ("all", 40, "nll", False, 32, 17), ("avg", 0, "mse", False, 1, 3),
+                                                     ("all", 0, "mse", True, 9, 33), ("max", 5, "mse", False, 17, 64)])
+def test_mutation_map_kernel_edges(pool, hidden, loss, rc, m, F):
+    """Lengths around a workgroup's 16 letters (one letter to several workgroups, a sequence shorter than its neighbours by more and
+    by less than the pad), filters beyond one and two tiles of 16, one tap, hidden units beyond a pass of 16 lanes."""
+    from deepbind_amd import _lib, predict
+    rng = np.random.default_rng(7 * m + F)
+    p = _params(rng, m, F, pool, hidden)
+    seqs = ["".join("ACGT"[v] for v in rng.integers(0, 4, n)) for n in (1, 15, 16, 17, 40, 33)]
+    seqs[3] = "n" + seqs[3][1:].lower().replace("t", "u")
+    out = "logistic" if loss == "nll" else "linear"
+    Zr, mr = orc.gen_predictions({k: v.astype(np.float64) for k, v in p.items()}, seqs, pool, hidden, out, reverse_complement=rc,
+                                 want_gmaps="finite_diff")
+    net = _net(p, m, F, pool, hidden, loss, rc, 0.0)
+    assert _lib.dll().dbk_mutation_map_takes(m, F, _lib.str2pooltype[pool], hidden) == 1
+    Z, maps = predict.gen_predictions(net, seqs, want_gmaps="finite_diff")
+    assert_close(Z, Zr, ACT, "Z")
+    scale = max(np.abs(b).max() for _, b in mr)
+    for (sa, a), (sb, b) in zip(maps, mr):
+        assert sa == sb and a.shape == b.shape
+        assert np.abs(a - b).max() <= GRAD * scale, (len(sa), np.abs(a - b).max(), scale)
+
+
+@pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("m,window,stride", [(1, 2, 1), (24, 20, 3), (8, 65, 7)])
+def test_text_and_windows_are_packed_as_on_the_host(rc, m, window, stride):
+    from deepbind_amd import _lib, data, predict
+    from deepbind_amd.model import SequenceNet
+    net = SequenceNet(1, 4, m, reverse_complement=rc)
+    every = "".join(chr(c) for c in range(256))
+    seqs = ["ACGTUacgtuNn.-", "", every, "G", "TT" * 90]
+    X, R = predict._pack(net, predict._Text(seqs))
+    Xr, Rr = data.pack_sequences(seqs, m - 1, reverse_complement=rc)
+    assert np.array_equal(X.cpu().numpy(), Xr) and np.array_equal(R.cpu().numpy(), Rr)
+    text = predict._Text(seqs)
+    assert text.strings() == [data.ord2acgt(data.acgt2ord(s)) for s in seqs]
+    assert text.strings(np.ones(len(seqs), bool)) == [data.revcomp(data.ord2acgt(data.acgt2ord(s))) for s in seqs]
+    # windows: what predict sees, captured instead of scored
+    seen = []
+    net.predict = lambda X, R, F=None: seen.append((X.cpu().numpy(), R.cpu().numpy())) or torch.zeros((R.shape[0] // (2 if rc else 1), 1))
+    predict.gen_predictionmaps(net, seqs, stride=stride, windowsize=window)
+    cut = []
+    for s in seqs:
+        padded = "N" * (window - 1) + s + "N" * (window - 1)
+        cut += [padded[i:i + window] for i in range(0, max(1, len(padded) - window + 1), stride)]
+    Xr, Rr = data.pack_sequences(cut, m - 1, reverse_complement=rc)
+    assert np.array_equal(seen[0][0], Xr) and np.array_equal(seen[0][1], Rr)
