@@ -97,6 +97,7 @@ _SIGNATURES = {
     "dbk_train_step": [_P, _P],
     "dbk_train_steps": [_P, _Z, _P],
     "dbk_train_step_single_workspace": [_P, _P],
+    "dbk_longest_region": [_P, _P, _Z, _P],
     "dbk_train_step_single": [_P, _P, _P, _Z],
     "dbk_train_step_args_size": [],
 }
@@ -117,6 +118,7 @@ class TrainStepArgs(ctypes.Structure):
         ("pooled", _P), ("argmax", _P), ("Z", _P), ("dpooled", _P), ("loss", _P), ("act", _P),
         ("L", _P), ("L_ready", _I),
         ("nfeat", _Z), ("feats", _P),
+        ("ycol", _P), ("ldY", _Z),
     ]
 
 _dll = None
@@ -156,7 +158,10 @@ def call(name, *args):
 
 def stream():
     """The current HIP stream of the current device, as the void* the library expects."""
-    return c_void_p(torch.cuda.current_stream().cuda_stream)
+    # (the raw handle: building torch's stream object costs as much as a whole call of the library)
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def ptr(t):

@@ -61,6 +61,7 @@ struct head_group {                         // the dense head of one group (argu
     uint64_t seed; uint64_t* counter;
     const float *W1, *b1, *W2, *b2, *Y;
     const uint8_t* Ymask;
+    const uint32_t* ycol; unsigned ldy;     // the group's columns of Y and Ymask and their rows' length (ycol null: all of them, in order)
     float *Z, *dpooled;
     // filled in by head_train_multi
     float* partial; unsigned nchunk, pstride;
@@ -70,6 +71,12 @@ bool scan_multi_takes(size_t m, size_t N, size_t P, unsigned n, const scan_group
 int scan_fprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size_t P, unsigned n, const scan_group* g);
 int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size_t P, unsigned n, scan_group* g);
 int head_train_multi(hipStream_t st, size_t nrow, unsigned n, head_group* g);
+// dbk_head_train with the models' columns of Y and Ymask picked by ycol (null: as dbk_head_train)
+int head_train(dbk_stream_t stream, size_t n, int nblock, int k, int hidden, int loss_kind, int reverse_complement,
+               const float* pooled, int nfeat, const float* feats, const float* rate, const float* U, uint64_t seed, uint64_t offset,
+               uint64_t* counter, uint64_t counter_advance, const float* W1, const float* b1, const float* W2, const float* b2,
+               const float* Y, const uint8_t* Ymask, const uint32_t* ycol, unsigned ldy,
+               float* Z, float* dpooled, float* dW1, float* db1, float* dW2, float* db2, float* loss);
 
 // dbk_set_exact_scan: the drop-in scan operators keep to the kernels that add in the reference's order at every size
 bool exact_scan();

@@ -31,6 +31,11 @@ struct head_args {
     unsigned long long counter_advance;
     const float *W1, *b1, *W2, *b2, *Y;
     const uint8_t* Ymask;
+    // model b's targets are column ycol[b] (ycol null: b) of Y and Ymask, whose rows are ldy apart: the groups of a calibration
+    // batch read their models' columns out of the batch's own matrices
+    const uint32_t* ycol;
+    unsigned ldy;
+    __device__ __forceinline__ size_t target(size_t row, unsigned b) const { return row * ldy + (ycol ? ycol[b] : b); }
     float *Z, *dpooled, *dW1, *db1, *dW2, *db2, *loss;
     float* partial;                // [chunk][model][pstride]: dW1 (k*h1), db1 (h1), dW2 (h1), db2, loss sum
     unsigned nchunk, pstride;
@@ -85,8 +90,9 @@ __device__ __forceinline__ void head_train_h32(const head_args& a, const unsigne
     const size_t r_mine = r0 + 8u * wave + (lane & 7u);
     const bool live_mine = lane < 8u && r_mine < a.n;
     const size_t zi_mine = live_mine ? r_mine * a.nblock + b : 0;
-    const float y_mine = live_mine ? a.Y[zi_mine] : 0.0f;
-    const bool use_mine = (live_mine && a.Ymask) ? a.Ymask[zi_mine] != 0 : true;
+    const size_t yi_mine = live_mine ? a.target(r_mine, b) : 0;
+    const float y_mine = live_mine ? a.Y[yi_mine] : 0.0f;
+    const bool use_mine = (live_mine && a.Ymask) ? a.Ymask[yi_mine] != 0 : true;
     const float b1v = a.b1[(size_t)b * H + j], w2v = a.W2[(size_t)b * H + j], bias2 = a.b2[b];
     const float inv_n = 1.0f / (float)a.n;
     {   // the chunk's inputs, dropout applied (element numbering of the stand-alone dropout kernels): four consecutive
@@ -297,8 +303,9 @@ __device__ __forceinline__ void head_train_body(const head_args& a, const unsign
     const float bias2 = hidden > 0 ? a.b2[b] : 0.0f;
     // this row's target and mask are needed only after the forward pass: requested now, they arrive meanwhile
     const size_t zi = live ? r * a.nblock + b : 0;
-    const float y_row = live ? a.Y[zi] : 0.0f;
-    const bool use_row = (live && a.Ymask) ? a.Ymask[zi] != 0 : true;
+    const size_t yi = live ? a.target(r, b) : 0;
+    const float y_row = live ? a.Y[yi] : 0.0f;
+    const bool use_row = (live && a.Ymask) ? a.Ymask[yi] != 0 : true;
     const float p_drop = a.rate ? a.rate[b] : 0.0f;
     const unsigned long long off = a.counter ? a.counter[0] : a.offset;
     const float inv_n = 1.0f / (float)a.n;
@@ -550,6 +557,7 @@ int dbk::head_train_multi(hipStream_t st, size_t nrow, unsigned n, dbk::head_gro
         a.pooled = g[i].pooled; a.rate = g[i].rate; a.U = nullptr; a.seed = g[i].seed; a.offset = 0;
         a.counter = (unsigned long long*)g[i].counter; a.counter_advance = 0;
         a.W1 = g[i].W1; a.b1 = g[i].b1; a.W2 = g[i].W2; a.b2 = g[i].b2; a.Y = g[i].Y; a.Ymask = g[i].Ymask;
+        a.ycol = g[i].ycol; a.ldy = g[i].ycol ? g[i].ldy : (unsigned)g[i].nblock;
         a.Z = g[i].Z; a.dpooled = g[i].dpooled; a.dW1 = a.db1 = a.dW2 = a.db2 = a.loss = nullptr;
         a.partial = g[i].partial; a.nchunk = g[i].nchunk; a.pstride = g[i].pstride;
     }
@@ -558,11 +566,11 @@ int dbk::head_train_multi(hipStream_t st, size_t nrow, unsigned n, dbk::head_gro
     DBK_LAUNCH_OK();
 }
 
-extern "C" int dbk_head_train(dbk_stream_t stream, size_t n, int nblock, int k, int hidden, int loss_kind, int reverse_complement,
+int dbk::head_train(dbk_stream_t stream, size_t n, int nblock, int k, int hidden, int loss_kind, int reverse_complement,
                               const float* pooled, int nfeat, const float* feats, const float* rate, const float* U, uint64_t seed, uint64_t offset,
                               uint64_t* counter, uint64_t counter_advance,
                               const float* W1, const float* b1, const float* W2, const float* b2,
-                              const float* Y, const uint8_t* Ymask,
+                              const float* Y, const uint8_t* Ymask, const uint32_t* ycol, unsigned ldy,
                               float* Z, float* dpooled, float* dW1, float* db1, float* dW2, float* db2, float* loss)
 {
     DBK_CHECK(nblock >= 1 && k >= 1 && nfeat >= 0 && hidden >= 0, "ValueError: bad head shape (nblock=%d, k=%d, nfeat=%d, hidden=%d)", nblock, k, nfeat, hidden);
@@ -579,7 +587,7 @@ extern "C" int dbk_head_train(dbk_stream_t stream, size_t n, int nblock, int k, 
     head_args a;
     a.n = n; a.nblock = nblock; a.k = k; a.kf = nfeat; a.feats = feats; a.hidden = hidden; a.loss_kind = loss_kind; a.revcomp = reverse_complement;
     a.pooled = pooled; a.rate = rate; a.U = U; a.seed = seed; a.offset = offset; a.counter = (unsigned long long*)counter; a.counter_advance = counter_advance;
-    a.W1 = W1; a.b1 = b1; a.W2 = W2; a.b2 = b2; a.Y = Y; a.Ymask = Ymask;
+    a.W1 = W1; a.b1 = b1; a.W2 = W2; a.b2 = b2; a.Y = Y; a.Ymask = Ymask; a.ycol = ycol; a.ldy = ycol ? ldy : (unsigned)nblock;
     a.Z = Z; a.dpooled = dpooled; a.dW1 = dW1; a.db1 = db1; a.dW2 = dW2; a.db2 = db2; a.loss = loss;
     a.nchunk = (unsigned)nchunk;
     a.pstride = (unsigned)((k + nfeat) * h1 + 2 * h1 + 2);
@@ -597,4 +605,15 @@ extern "C" int dbk_head_train(dbk_stream_t stream, size_t n, int nblock, int k, 
         hipLaunchKernelGGL(k_head_reduce, dim3(dbk::ew_grid((size_t)nblock * a.pstride)), dim3(256), 0, dbk::as_stream(stream), a);
     }
     DBK_LAUNCH_OK();
+}
+
+extern "C" int dbk_head_train(dbk_stream_t stream, size_t n, int nblock, int k, int hidden, int loss_kind, int reverse_complement,
+                              const float* pooled, int nfeat, const float* feats, const float* rate, const float* U, uint64_t seed, uint64_t offset,
+                              uint64_t* counter, uint64_t counter_advance,
+                              const float* W1, const float* b1, const float* W2, const float* b2,
+                              const float* Y, const uint8_t* Ymask,
+                              float* Z, float* dpooled, float* dW1, float* db1, float* dW2, float* db2, float* loss)
+{
+    return dbk::head_train(stream, n, nblock, k, hidden, loss_kind, reverse_complement, pooled, nfeat, feats, rate, U, seed, offset, counter, counter_advance,
+                           W1, b1, W2, b2, Y, Ymask, nullptr, 0, Z, dpooled, dW1, db1, dW2, db2, loss);
 }

@@ -837,6 +837,7 @@ bool plan(const dbk_train_step_args* a, single_args& s, unsigned& MT, size_t& ld
     if (F > 64 || a->hidden > 64 || !a->nesterov || a->input_rate > 0.0f || a->nregion < 1 || a->N >= 0xffffff00ull) return false;
     if (a->ptype != DBK_PT_MAX && a->ptype != DBK_PT_AVG && a->ptype != DBK_PT_ALL) return false;
     if (a->reverse_complement && (a->nregion & 1)) return false;
+    if (a->ycol) return false;                    // (picked target columns: groups of a calibration batch, which share launches)
     s.nmodel = (unsigned)a->nmodel; s.nfilter = (unsigned)a->nfilter; s.F = (unsigned)F;
     s.Fp = F <= 16 ? 16u : (F <= 32 ? 32u : 64u);
     s.lgFp = ilog2(s.Fp);
@@ -865,6 +866,43 @@ bool plan(const dbk_train_step_args* a, single_args& s, unsigned& MT, size_t& ld
 }
 
 }  // namespace
+
+namespace {
+
+__global__ __launch_bounds__(256) void k_longest_region(const uint32_t* __restrict__ R, unsigned P, unsigned* __restrict__ out)
+{
+    __shared__ unsigned part[4];
+    unsigned rows = 0;
+    for (unsigned r = threadIdx.x; r < P; r += 256) {
+        const uint2 ab = reinterpret_cast<const uint2*>(R)[r];
+        rows = max(rows, ab.y > ab.x ? ab.y - ab.x : 0u);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) rows = max(rows, (unsigned)__shfl_xor((int)rows, d, 64));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = rows;
+    __syncthreads();
+    if (threadIdx.x == 0) out[0] = max(max(part[0], part[1]), max(part[2], part[3]));
+}
+
+}  // namespace
+
+// A new minibatch pays for this once before its first step: one launch and one read-back (the same from elementwise
+// operations of the host's array library: five launches and a read-back, ~60 us a minibatch against ~20).
+extern "C" int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, size_t nregion, unsigned* rows)
+{
+    DBK_CHECK(rows, "ValueError: null pointer argument");
+    *rows = 0;
+    if (nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(regions && ((uintptr_t)regions & 7) == 0 && nregion < ((size_t)1 << 31), "ValueError: regions must be an 8-byte aligned table of fewer than 2^31 rows");
+    hipStream_t st = dbk::as_stream(stream);
+    unsigned* word = (unsigned*)dbk::workspace(sizeof(unsigned), st);
+    DBK_CHECK(word != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
+    hipLaunchKernelGGL(k_longest_region, dim3(1), dim3(256), 0, st, regions, (unsigned)nregion, word);
+    DBK_HIP(hipMemcpyAsync(rows, word, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    DBK_HIP(hipStreamSynchronize(st));
+    dbk::clear_error();
+    return 0;
+}
 
 extern "C" int dbk_train_step_single_workspace(const dbk_train_step_args* a, size_t* work_bytes)
 {

@@ -166,6 +166,7 @@ int check_args(const dbk_train_step_args* a)
     DBK_CHECK(a->ptype == DBK_PT_AVG || a->argmax, "ValueError: max / all pooling needs the argmax work buffer");
     DBK_CHECK(a->input_rate <= 0.0f || (a->Xdrop && a->Mdrop), "ValueError: input dropout needs the Xdrop and Mdrop work buffers");
     DBK_CHECK(!(a->rate || a->input_rate > 0.0f) || a->counter, "ValueError: dropout needs the device generator position");
+    DBK_CHECK(!a->ycol || (a->ldY >= 1 && a->ldY < ((size_t)1 << 32)), "ValueError: picked target columns need the targets' row length");
     const block_sizes z = sizes_of(a);
     const size_t need[6] = { a->off_Wc + z.nWc, a->off_bc + z.F, a->off_W1 + z.nW1, a->off_b1 + z.nb1,
                              a->off_W2 + z.nW2, a->off_b2 + z.nb2 };
@@ -246,10 +247,10 @@ extern "C" int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* a)
                             a->pooled, a->argmax, act);
     if (rc) return rc;
     const uint64_t draws = a->rate ? (a->nregion * k * a->nmodel + 3) / 4 : 0;
-    rc = dbk_head_train(stream, a->nregion, (int)a->nmodel, (int)k, (int)a->hidden, a->loss_kind, a->reverse_complement,
+    rc = dbk::head_train(stream, a->nregion, (int)a->nmodel, (int)k, (int)a->hidden, a->loss_kind, a->reverse_complement,
                         a->pooled, (int)a->nfeat, a->feats, a->rate, nullptr, a->seed, 0, a->counter, draws,
                         P + a->off_W1, P + a->off_b1, a->hidden ? P + a->off_W2 : nullptr, a->hidden ? P + a->off_b2 : nullptr,
-                        a->Y, a->Ymask, a->Z, a->dpooled,
+                        a->Y, a->Ymask, a->ycol, (unsigned)a->ldY, a->Z, a->dpooled,
                         dP + a->off_W1, dP + a->off_b1, a->hidden ? dP + a->off_W2 : nullptr, a->hidden ? dP + a->off_b2 : nullptr,
                         a->loss);
     if (rc) return rc;
@@ -277,7 +278,7 @@ extern "C" int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* a)
 // One step of each of several groups that train on the same batch: every phase of the step is ONE launch holding
 // all the groups' grids, so groups too small to fill the GPU run side by side on one stream. A group's kernels,
 // grids and summation orders are those of its own dbk_train_step, hence the same bits. Taken for up to 8 groups
-// with a look-ahead vector each (Nesterov), filters of at most 24 taps and one shared region table; any other
+// with a look-ahead vector each (Nesterov), filters of at most 32 taps and one shared region table; any other
 // call steps the groups one after the other.
 extern "C" int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_train_step_args* const* args)
 {
@@ -355,7 +356,7 @@ extern "C" int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_tra
         hg[i].pooled = a->pooled; hg[i].rate = a->rate; hg[i].seed = a->seed; hg[i].counter = a->counter;
         hg[i].W1 = P + a->off_W1; hg[i].b1 = P + a->off_b1;
         hg[i].W2 = a->hidden ? P + a->off_W2 : nullptr; hg[i].b2 = a->hidden ? P + a->off_b2 : nullptr;
-        hg[i].Y = a->Y; hg[i].Ymask = a->Ymask; hg[i].Z = a->Z; hg[i].dpooled = a->dpooled;
+        hg[i].Y = a->Y; hg[i].Ymask = a->Ymask; hg[i].ycol = a->ycol; hg[i].ldy = (unsigned)a->ldY; hg[i].Z = a->Z; hg[i].dpooled = a->dpooled;
         hg[i].partial = nullptr; hg[i].nchunk = 0; hg[i].pstride = 0;
     }
     rc = dbk::head_train_multi(st, a0->nregion, n, hg);

@@ -65,7 +65,9 @@ class SequenceNet(object):
         self._last_single = False            # the last natively issued step went through the single-launch kernel
         self.step_count = 0
         self._step_args = None               # argument block and work buffers of the natively issued step
-        self._step_bufs = {}
+        self._step_bufs = {}                 # per batch shape: the step's work buffers, views of the vectors below
+        self._step_store = {}                # one growing vector per work buffer, shared by all batch shapes
+        self._works = []                     # single-launch workspaces: [tensor, steps issued on it]; the last one is in use
         self._step_sig, self._step_buf, self._step_nesterov = None, None, None
         # Nesterov look-ahead kept beside the parameters by the natively issued step (each step's update kernel
         # leaves the next step's look-ahead there); valid while nothing else has touched P, mP or mrate
@@ -189,7 +191,7 @@ class SequenceNet(object):
         if "work" not in buf:
             need = ctypes.c_size_t(0)
             _lib.call("dbk_train_step_single_workspace", ctypes.addressof(self._step_args), ctypes.addressof(need))
-            buf["work"] = torch.zeros(need.value, dtype=torch.uint8, device=self.P.device) if need.value else None
+            buf["work"] = self._workspace(need.value) if need.value else None
         if buf["work"] is None:
             return None
         # the longest region of this very tensor object in its present state: an address alone says nothing (a new
@@ -198,10 +200,20 @@ class SequenceNet(object):
         if ent is None or ent[0]() is not R or ent[1] != R._version:
             if len(self._single_rows) >= 256:
                 self._single_rows.clear()
-            Rl = R.to(torch.int64)           # one read-back per region table: the kernel keeps whole regions in LDS
-            rows = int((Rl[:, 1] - Rl[:, 0]).max().item()) if R.shape[0] else 0
-            ent = self._single_rows[id(R)] = (weakref.ref(R), R._version, rows)
+            rows = ctypes.c_uint(0)          # one read-back per region table: the kernel keeps whole regions in LDS
+            _lib.call("dbk_longest_region", _lib.stream(), _lib.ptr(R), R.shape[0], ctypes.addressof(rows))
+            ent = self._single_rows[id(R)] = (weakref.ref(R), R._version, rows.value)
         return buf["work"] if ent[2] <= 256 else None
+
+    def _workspace(self, need):
+        """A single-launch workspace of at least `need` bytes. Batches of all shapes share one: what a launch leaves in it
+        carries the launch's number, so nothing a launch of another shape left is taken for this one's."""
+        if not self._works or self._works[-1][0].numel() < need:
+            self._works.append([torch.zeros((need + need // 4 + 255) // 256 * 256, dtype=torch.uint8, device=self.P.device), 0])
+            for buf in self._step_bufs.values():
+                if buf.get("work") is not None:
+                    del buf["work"]          # (looked up again with the batch's next step)
+        return self._works[-1][0]
 
     SINGLE_HEADER = 32768                    # bytes of a single-launch workspace before the gradient shares
 
@@ -210,16 +222,17 @@ class SequenceNet(object):
         workspace, changed nothing (parameters, momentum, generator position), so the host's step counter and
         generator mirror are set back to what the device actually did, and the workspace's header is zeroed so that
         the next step runs again."""
-        for buf in self._step_bufs.values():
-            work = buf.get("work")
-            if work is None:
-                continue
+        own = [w for w, _ in self._works]
+        entries = self._works + [[buf["work"], buf.get("issued", 0)] for buf in self._step_bufs.values()
+                                 if buf.get("work") is not None and not any(buf["work"] is w for w in own)]
+        for entry in entries:
+            work, issued = entry
             torch.cuda.synchronize()
             stepped, status = (int(v) for v in work[0:8].view(torch.int32).tolist())
             if status:
-                dropped = max(buf.get("issued", 0) - stepped, 0)
+                dropped = max(issued - stepped, 0)
                 work[:self.SINGLE_HEADER].zero_()
-                buf["issued"] = 0
+                entry[1] = 0
                 self.step_count -= dropped
                 self._rng_offset = int(self.rng_counter.item())
                 self._L_versions = None
@@ -229,7 +242,9 @@ class SequenceNet(object):
     def _count_single_launch(self, buf):
         """Book-keeping after a single-launch step was issued on the workspace in `buf` (or a graph holding one
         replayed): the status word is looked at every 256 launches, so that an abandoned step does not go unnoticed."""
-        buf["issued"] = buf.get("issued", 0) + 1
+        for entry in self._works:
+            if entry[0] is buf["work"]:
+                entry[1] += 1
         self._single_calls += 1
         if self._single_calls % 256 == 0:
             self._check_single_status()
@@ -516,13 +531,14 @@ class SequenceNet(object):
         return Z
 
     # ------------------------------------------------------------------ one optimiser step
-    def _prepare_step(self, X, R, Y, Ymask=None, F=None):
+    def _prepare_step(self, X, R, Y, Ymask=None, F=None, cols=None):
         """Fills this net's dbk_train_step_args block for one step on the batch and returns the step's work
-        buffers (made on the current stream, where the step is issued)."""
+        buffers (made on the current stream, where the step is issued). cols: the columns of Y and Ymask that are this
+        net's models' (device int32), None for all."""
         a = self._step_args
         # the same batch tensors as in the previous step (a training loop over resident batches): only the switches move
         sig = (X.data_ptr(), X.numel(), R.data_ptr(), R.shape[0], R._version, Y.data_ptr(), Y.numel(),
-               None if Ymask is None else Ymask.data_ptr(), None if F is None else F.data_ptr())
+               None if Ymask is None else Ymask.data_ptr(), None if F is None else F.data_ptr(), None if cols is None else cols.data_ptr())
         if a is not None and sig == self._step_sig and not self.nesterov_changed():
             if self.nesterov:
                 versions = (self.P._version, self.mP._version, self.mrate._version)
@@ -534,9 +550,10 @@ class SequenceNet(object):
         ks._u8(X)
         ks._regions(R)
         ni, P = self.ninst, R.shape[0]
+        want = (P, ni if cols is None else Y.shape[-1])
         _lib.require(R.shape[1] == 2, "ValueError: the fused path takes 2-column regions")
-        _lib.require(Y.dtype == torch.float32 and tuple(Y.shape) == (P, ni), "ValueError: Y must be float32 (rows x models)")
-        _lib.require(Ymask is None or (Ymask.dtype == torch.bool and tuple(Ymask.shape) == (P, ni)), "ValueError: Ymask must be bool (rows x models)")
+        _lib.require(Y.dtype == torch.float32 and tuple(Y.shape) == want, "ValueError: Y must be float32 (rows x models)")
+        _lib.require(Ymask is None or (Ymask.dtype == torch.bool and tuple(Ymask.shape) == want), "ValueError: Ymask must be bool (rows x models)")
         if a is None:
             a = self._step_args = _lib.TrainStepArgs()
             off = {name: int(o) for (name, _, _), o in zip(self.layout, self.offsets[:-1])}
@@ -550,20 +567,9 @@ class SequenceNet(object):
             a.off_W2, a.off_b2 = off.get("W2", 0), off.get("b2", 0)
             a.rate = self.dropout.data_ptr() if self.use_dropout else None
             a.counter = self.rng_counter.data_ptr()
-        key = (X.numel(), P)
-        buf = self._step_bufs.get(key)
-        if buf is None:
-            if len(self._step_bufs) >= 4:
-                self._step_bufs.clear()
-            dev = self.P.device
-            buf = self._step_bufs[key] = dict(
-                pooled=torch.empty((P, self.k * ni), dtype=torch.float32, device=dev),
-                dpooled=torch.empty((P, self.k * ni), dtype=torch.float32, device=dev),
-                argmax=torch.empty((P, self.nfilter * ni), dtype=ks.uindex, device=dev) if self.pool != "avg" else None,
-                Z=torch.empty((P, ni), dtype=torch.float32, device=dev),
-                act=ks.activity_words(X, self.p["Wc"]) if self.pool != "max" else None,
-                Xdrop=torch.empty(X.numel(), dtype=torch.uint8, device=dev) if self.input_dropout > 0 else None,
-                Mdrop=torch.empty(X.numel(), dtype=torch.bool, device=dev) if self.input_dropout > 0 else None)
+            a.input_rate = self.input_dropout
+            a.loss = None
+        buf = self._step_buffers(X.numel(), P)
         a.nesterov, a.seed = int(bool(self.nesterov)), int(self.rng_seed)
         if self.nesterov:
             if self._L is None:
@@ -579,16 +585,47 @@ class SequenceNet(object):
         pv = lambda t: None if t is None else _lib.ptr(t).value          # checks device + contiguity
         a.X, a.N, a.regions, a.nregion = pv(X), X.numel(), pv(R), P
         a.Y, a.Ymask = pv(Y), pv(Ymask)
+        a.ycol, a.ldY = pv(cols), Y.shape[-1]
         _lib.require(F is None or (F.dtype == torch.float32 and tuple(F.shape) == (P, self.nfeat)), "ValueError: F must be float32 (rows x feature_columns)")
         a.nfeat, a.feats = self.nfeat, pv(F)
-        a.input_rate = self.input_dropout
-        for name, t in buf.items():
-            if name not in ("work", "issued"):
-                setattr(a, name, None if t is None else t.data_ptr())
+        for name in self._STEP_BUFFERS:
+            t = buf[name]
+            setattr(a, name, None if t is None else t.data_ptr())
         a.decay = self.decay_vec.data_ptr() if self.weight_decay_start <= self.step_count else None
         a.freeze_scan = int(self.step_count < self.start_training)
-        a.loss = None
         self._step_sig, self._step_buf, self._step_nesterov = sig, buf, (bool(self.nesterov), int(self.rng_seed))
+        return buf
+
+    _STEP_BUFFERS = ("pooled", "dpooled", "argmax", "Z", "act", "Xdrop", "Mdrop")
+
+    def _step_buffers(self, N, P):
+        """The step's work buffers for a batch of N letters and P regions: views of vectors that grow with the largest batch,
+        so that an epoch of ragged minibatches allocates nothing once it has seen its largest one. (A captured graph keeps
+        the views it was captured with, and through them the memory.)"""
+        buf = self._step_bufs.get((N, P))
+        if buf is not None:
+            return buf
+        if len(self._step_bufs) >= 64:
+            self._step_bufs.clear()
+        ni, F = self.ninst, self.nfilter * self.ninst
+        f32, words = torch.float32, (F + 63) // 64
+        wanted = [("pooled", P, self.k * ni, f32), ("dpooled", P, self.k * ni, f32), ("Z", P, ni, f32)]
+        if self.pool != "avg":
+            wanted.append(("argmax", P, F, ks.uindex))
+        if self.pool != "max":
+            wanted.append(("act", N, words, torch.int64))
+        if self.input_dropout > 0:
+            wanted += [("Xdrop", N, 0, torch.uint8), ("Mdrop", N, 0, torch.bool)]
+        buf = dict.fromkeys(self._STEP_BUFFERS)
+        for name, rows, cols, dtype in wanted:
+            n = rows * max(cols, 1)
+            store = self._step_store.get(name)
+            if store is None or store.numel() < n:
+                # (a quarter more than asked for: the epoch's other minibatches are about as large)
+                store = self._step_store[name] = torch.empty(n + n // 4, dtype=dtype, device=self.P.device)
+                self._step_bufs.clear()      # (views of the vector that was outgrown would keep it alive)
+            buf[name] = store[:n].view(rows, cols) if cols else store[:n]
+        self._step_bufs[N, P] = buf
         return buf
 
     def nesterov_changed(self):
@@ -660,7 +697,7 @@ class SequenceNet(object):
 
 
 def _native_steps(jobs):
-    """jobs: list of (net, X, R, Y, Ymask[, F]), nets that step on the same batch. One dbk_train_steps call per eight
+    """jobs: list of (net, X, R, Y, Ymask[, F[, cols]]), nets that step on the same batch. One dbk_train_steps call per eight
     nets on the current stream: every phase of the step is one launch holding all the nets' grids, so nets too
     small to fill the GPU run side by side without extra streams. Each net gets the bits of its own step."""
     if len(jobs) == 1:
@@ -671,7 +708,7 @@ def _native_steps(jobs):
         chunk = jobs[i:i + 8]
         blocks = (ctypes.c_void_p * len(chunk))()
         for j, (net, X, R, Y, Ymask, *rest) in enumerate(chunk):
-            net._prepare_step(X, R, Y, Ymask, rest[0] if rest else None)
+            net._prepare_step(X, R, Y, Ymask, *rest)
             blocks[j] = ctypes.addressof(net._step_args)
         _lib.call("dbk_train_steps", _lib.stream(), len(chunk), blocks)
         for net, X, R, *_ in chunk:
@@ -749,6 +786,7 @@ def _graphed_step(jobs):
         for net, *_ in jobs:
             net._L_versions = None              # (the warm-up step's look-ahead belongs to parameters that were put back)
         state["graphs"], state["decay"] = graphs, decay_flags()
+        state["buffers"] = [(net._step_buf, net._L) for net, *_ in jobs]                      # (the graph's nodes point into them)
         state["single"] = [(net, net._step_buf) for net, *_ in jobs if net._last_single]      # workspaces of single-launch steps in the graph
 
     def step():
@@ -784,7 +822,8 @@ class ModelGroup(object):
             kw = {k: (np.asarray(v)[idx] if np.ndim(v) else v) for k, v in per_model.items()}
             self.groups.append((idx, SequenceNet(len(idx), nfilter, m, pool=key[0], hidden=key[1], loss=loss, **kw)))
         self.streams = None
-        self._batch_key, self._batch, self._targets = None, None, None
+        # every group reads its models' columns out of the batch's own target matrices
+        self._cols = [torch.as_tensor(idx, dtype=torch.int32, device=net.device) for idx, net in self.groups]
 
     def _streams(self):
         if self.streams is None:
@@ -810,16 +849,10 @@ class ModelGroup(object):
                 return run
             _side_by_side(self._streams(), [one(gi, idx, net) for gi, (idx, net) in enumerate(self.groups)])
             return
-        key = tuple((t.data_ptr(), t._version, tuple(t.shape)) for t in (X, R, Y, Ymask) if t is not None)
-        if key != self._batch_key:
-            # each group's columns of the targets, kept until the batch changes
-            self._targets = []
-            for idx, _ in self.groups:
-                ii = torch.as_tensor(idx, device=Y.device)
-                self._targets.append((Y.index_select(1, ii).contiguous(),
-                                      Ymask.index_select(1, ii).contiguous() if Ymask is not None else None))
-            self._batch_key, self._batch = key, (X, R, Y, Ymask)
-        _native_steps([(net, X, R, Yg, Mg, F) for (_, net), (Yg, Mg) in zip(self.groups, self._targets)])
+        if len(self.groups) == 1:
+            self.groups[0][1]._native_step(X, R, Y, Ymask, F)
+            return
+        _native_steps([(net, X, R, Y, Ymask, F, cols) for (_, net), cols in zip(self.groups, self._cols)])
 
     def make_graphed_step(self, X, R, Y, Ymask=None, F=None):
         """One HIP graph holding the fused training step of every architecture group on a static batch."""

@@ -477,6 +477,8 @@ typedef struct dbk_train_step_args {
     size_t nfeat; const float* feats;       /* shared feature columns (nregion, nfeat) entering the first dense layer after each model's
                                                pooled features: W1 is ((k+nfeat)*nmodel, hidden|1); feats NULL = all zeros
                                                (reference: kangaroo/kangaroo/model.py:101-112, data.py:59-69) */
+    const uint32_t* ycol; size_t ldY;       /* device: model b's targets are column ycol[b] of Y and Ymask (nregion, ldY), which a calibration
+                                               batch's groups then share; NULL: Y and Ymask are (nregion, nmodel) */
 } dbk_train_step_args;
 
 /* One optimiser step, all launches issued from native code on `stream`:
@@ -493,7 +495,7 @@ int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* args);
  * one calibration batch. Every phase of the step is one launch that holds the grids of all the groups, so
  * groups that are each too small to fill the GPU run side by side on one stream, with no second stream and
  * no event. Each group's results are the bits its own dbk_train_step gives. Up to 8 groups, each with a
- * look-ahead vector (Nesterov) and filters of at most 24 taps, are taken together; any other call steps
+ * look-ahead vector (Nesterov) and filters of at most 32 taps, are taken together; any other call steps
  * the groups one after the other on `stream`.
  * reference: the per-architecture loop over one shared minibatch in the calibration search, which trains
  * all sampled models on the same batches (deepity/deepity/hpsearch.py:314-330, sgd.py:98-135). */
@@ -508,7 +510,7 @@ int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_train_step_arg
  * dP, mP, P, loss and advances the generator position. Deterministic; within the tolerances of dbk_train_step,
  * not its bits (other summation orders).
  * work: caller-owned device memory of dbk_train_step_single_workspace() bytes, 16-byte aligned, ZERO before its
- * first use and from then on passed unchanged to every call with the same nregion. Word 0 (uint32) counts the
+ * first use and from then on passed unchanged to every call (batches of any shape it is large enough for). Word 0 (uint32) counts the
  * launches that stepped; word 1 is a status: 1 = a workgroup waited too long (at the barrier or for its
  * reverse-complement partner), 2 = a region had more than 256 rows. Whether a launch steps is decided once for the
  * whole grid (a compare-and-swap on one word of the workspace): an abandoned launch changes no parameter, neither
@@ -519,6 +521,8 @@ int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_train_step_arg
  * (use dbk_train_step).
  * reference: the body of the trainer's loop, deepity/deepity/sgd.py:98-135, as dbk_train_step. */
 int dbk_train_step_single_workspace(const dbk_train_step_args* args, size_t* work_bytes);
+/* Rows of the longest of nregion (start, end) regions, read back to the host (waits for the stream). */
+int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, size_t nregion, unsigned* rows);
 int dbk_train_step_single(dbk_stream_t stream, const dbk_train_step_args* args, void* work, size_t work_bytes);
 /* sizeof(dbk_train_step_args) as the library was built, for bindings that mirror the block field by field. */
 int dbk_train_step_args_size(void);

@@ -282,3 +282,27 @@ def test_region_table_cache_follows_the_tensor_not_its_address():
     assert net.step_count == 2
     for pname in a:
         assert np.abs(a[pname] - b[pname]).max() <= GRAD * np.abs(b[pname]).max(), pname
+
+
+@pytest.mark.parametrize("nm,rc,pool", [(1, False, "all"), (1, True, "max"), (2, False, "avg")])
+def test_minibatches_of_changing_shape_share_buffers_and_workspace(nm, rc, pool):
+    """An epoch of minibatches that grow and shrink in letters and rows (also across one workgroup per region, 256) gives the
+    bits of a net that starts every step with buffers and a workspace of its own."""
+    rng = np.random.default_rng(31)
+    m, batches = 11, []
+    for rows in (16, 40, 6, 300, 128):
+        X, R = _batch(rng, rows, m, 20, 60, reverse_complement=rc)
+        batches.append((dev(X), dev(R), dev(rng.random((len(R), nm)).astype(np.float32))))
+    net, own = [_net(np.random.default_rng(32), nm, 16, m, pool, 8, "mse", rate=0.05, momentum=0.9, dropout=0.5, reverse_complement=rc)[0] for _ in range(2)]
+    for X, R, Y in batches + batches[::-1]:
+        net.train_step(X, R, Y)
+        own._check_single_status()
+        own._step_bufs.clear(); own._step_store.clear(); own._works.clear()
+        own._step_sig = None
+        own.train_step(X, R, Y)
+        assert net._last_single and own._last_single
+    assert len(net._works) <= len(batches) and len(net._step_bufs) == len(batches)
+    a, b = net.get_params(), own.get_params()
+    for name in a:
+        assert np.array_equal(a[name], b[name]), name
+    assert np.array_equal(host(net.mP), host(own.mP)) and int(net.rng_counter.item()) == int(own.rng_counter.item())

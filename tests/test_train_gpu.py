@@ -852,3 +852,32 @@ def test_nets_stepped_through_one_call_end_with_the_bits_of_their_own_steps(case
         assert np.abs(host(a.mP)).max() > 0
         assert a.step_count == b.step_count == 4 and a._rng_offset == b._rng_offset
         assert host(a.rng_counter) == host(b.rng_counter)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_group_reads_its_models_columns_of_the_shared_targets(masked):
+    """The groups of a calibration batch pick their models' target (and mask) columns inside the kernels: over minibatches of
+    changing shape each group ends with the bits of a net of its own that is handed those columns."""
+    from deepbind_amd import data
+    from deepbind_amd.model import ModelGroup, SequenceNet
+    rng = np.random.default_rng(41)
+    pools, hiddens = ["max", "all", "max", "all", "avg", "max"], [32, 0, 32, 0, 8, 0]
+    m, ncol = 26, len(pools)
+    kw = dict(loss="nll", rate=0.05, momentum=0.9, weight_decay_start=0, decay_conv=1e-4)
+    grp = ModelGroup(pools, hiddens, 16, m, **kw)
+    nets = []
+    for idx, net in grp.groups:
+        net.init_params(init_conv=0.1, init_full=0.1, seed=idx[0])
+        nets.append(SequenceNet(len(idx), 16, m, pool=net.pool, hidden=net.hidden, **kw))
+        nets[-1].set_params(net.get_params())
+    for rows in (20, 70, 33):
+        ords = [rng.integers(0, 4, int(n)).astype(np.uint8) for n in rng.integers(20, 50, rows)]
+        X, R = data.pack_ordinals(ords, m - 1)
+        Y, M = (rng.random((rows, ncol)) < 0.5).astype(np.float32), rng.random((rows, ncol)) < 0.7
+        Xd, Rd = dev(X), dev(R)
+        grp.train_step(Xd, Rd, dev(Y), dev(M) if masked else None)
+        for (idx, _), net in zip(grp.groups, nets):
+            net.single_launch = False
+            net.train_step(Xd, Rd, dev(np.ascontiguousarray(Y[:, idx])), dev(np.ascontiguousarray(M[:, idx])) if masked else None)
+    for (idx, net), own in zip(grp.groups, nets):
+        assert np.array_equal(host(net.P), host(own.P)) and np.array_equal(host(net.mP), host(own.mP)), idx
