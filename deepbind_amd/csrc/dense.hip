@@ -584,6 +584,99 @@ __global__ __launch_bounds__(256) void k_head16(size_t n, int nblock, int k, int
     }
 }
 
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true)); }
+// z[u] += (input KK of the 16-lane row, held by lane KK % 16) * w[u][KK], inputs ascending
+template <int HU, int K, int KK, int KI>
+__device__ __forceinline__ void head_lanes_inputs(const float (&x)[KI], const float (&w)[HU][K], float (&z)[HU])
+{
+    const float v = lane_move<0x150 + KK % 16>(x[KK / 16]);
+#pragma unroll
+    for (int u = 0; u < HU; ++u) z[u] = __builtin_fmaf(v, w[u][KK], z[u]);
+    if constexpr (KK + 1 < K) head_lanes_inputs<HU, K, KK + 1>(x, w, z);
+}
+
+// Scoring head, 16 lanes per (row, model) item, the model's weights in their registers (lane l holds the columns
+// l, l + 16, .. of W1, HU of them over KI x 16 inputs; HU = 0: no hidden layer, lane l holds inputs l, l + 16, ..), the row's
+// inputs read as one coalesced load per 16 and handed round by lane moves, the output sum folded by lane moves. No LDS, no
+// barrier: what bounds a small call is the chain weights -> inputs -> ~60 instructions, which a thread per row (k_head) runs
+// as 544 dependent multiply-adds behind a staging of the weights, and a bulk call the vector issue (15 instructions an item at
+// 16 inputs, 27 at 32). A wave's four items are `mg` adjacent models of 4 / mg rows, four such steps in flight together.
+// Measured against k_head / k_head16 (us a call, host included): 64 rows x 1 model (16 -> 32 -> 1) 7.6 against 11.9, 4156 x 1 (32 -> 1)
+// 7.0 / 10.3, 100 000 x 1 (16 -> 32 -> 1) 9.3 / 44, 20 000 x 24 (32 -> 32 -> 1) 41 / 258, 20 000 x 24 (32 -> 1) 15 / 243.
+template <int KI, int HU>
+__global__ __launch_bounds__(256) void k_head_lanes(size_t n, int nblock, int k, int kf, int kw, int hidden, int mg, const float* __restrict__ pooled,
+                                                    const float* __restrict__ feats, const float* __restrict__ in_scale, const float* __restrict__ W1, const float* __restrict__ b1,
+                                                    const float* __restrict__ W2, const float* __restrict__ b2, bool apply_logistic,
+                                                    float* __restrict__ scores)
+{
+    constexpr int K = KI * 16, NR = 4;
+    const int kt = k + kf;                              // the model's own inputs, then the shared feature columns (see k_head)
+    const unsigned hl = threadIdx.x & 15u, g = (threadIdx.x >> 4) & 3u;
+    const unsigned b = blockIdx.x * (unsigned)mg + (g & (unsigned)(mg - 1));
+    const bool live = b < (unsigned)nblock;
+    const unsigned bb = live ? b : 0u, per = 4u / (unsigned)mg;
+    const size_t wave = (size_t)blockIdx.y * 4 + (threadIdx.x >> 6), step = (size_t)gridDim.y * 4 * per;
+    float w[HU > 0 ? HU : 1][HU > 0 ? K : KI], bias1[HU > 0 ? HU : 1], w2[HU > 0 ? HU : 1];
+    if (HU > 0) {
+#pragma unroll
+        for (int u = 0; u < HU; ++u) {
+            const int h = (int)hl + 16 * u;
+            const bool in = h < hidden;
+#pragma unroll
+            for (int kk = 0; kk < K; ++kk) w[u][kk] = in && kk < kt ? W1[((size_t)bb * kw + kk) * hidden + h] : 0.0f;
+            bias1[u] = in ? b1[(size_t)bb * hidden + h] : 0.0f;
+            w2[u] = in ? W2[(size_t)bb * hidden + h] : 0.0f;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < KI; ++i) w[0][i] = (int)hl + 16 * i < kt ? W1[(size_t)bb * kw + hl + 16 * i] : 0.0f;
+    }
+    const float sc = in_scale ? in_scale[bb] : 1.0f, last = HU > 0 ? b2[bb] : b1[bb];
+    const size_t rowlen = (size_t)k * nblock;
+    const float* src = pooled + (size_t)bb * k + hl;
+    for (size_t r = wave * per + g / (unsigned)mg; __ballot(r < n) != 0; r += NR * step) {
+        float x[NR][KI];
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+#pragma unroll
+            for (int i = 0; i < KI; ++i) {
+                const size_t row = r + j * step;
+                const int kk = (int)hl + 16 * i;
+                x[j][i] = row >= n ? 0.0f : kk < k ? src[row * rowlen + 16 * i] * sc : kk < kt ? feats[row * (size_t)kf + (kk - k)] : 0.0f;
+            }
+        float mine = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            if (__ballot(r + j * step < n) == 0) break;
+            float out = 0.0f;
+            if constexpr (HU > 0) {
+                float z[HU];
+#pragma unroll
+                for (int u = 0; u < HU; ++u) z[u] = 0.0f;
+                head_lanes_inputs<HU, K, 0>(x[j], w, z);
+#pragma unroll
+                for (int u = 0; u < HU; ++u) {
+                    const float a = z[u] + bias1[u];
+                    out += (a > 0.0f ? a : 0.0f) * w2[u];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < KI; ++i) out += x[j][i] * w[0][i];
+            }
+            out += lane_move<0xB1>(out);                           // lane ^ 1, lane ^ 2, the mirrored lane of the eight, of the sixteen
+            out += lane_move<0x4E>(out);
+            out += lane_move<0x141>(out);
+            out += lane_move<0x140>(out);
+            mine = hl == (unsigned)j ? out : mine;
+        }
+        mine += last;
+        if (apply_logistic) mine = 1.0f / (1.0f + expf(-mine));
+        const size_t row = r + hl * step;                          // lane j of the group stores row j of the four
+        if (live && hl < (unsigned)NR && row < n) scores[row * (size_t)nblock + b] = mine;
+    }
+}
+
 // Row-slice count for the kernels that stage 16 models' weights per workgroup: about 1024 workgroups in all
 // (a few per CU), so that staging is paid once per many rows.
 inline unsigned row_slices(size_t n, unsigned rows_per_pass, unsigned ngroups)
@@ -923,6 +1016,28 @@ int dbk_head_fprop(dbk_stream_t stream, size_t n, int nblock, int k, int hidden,
     unsigned gx = dbk::divup(n, 256);
     if (gx > 2048u) gx = 2048u;
     const size_t smem16 = ((size_t)kk_all * hidden + 2 * (size_t)hidden) * HG * sizeof(float);
+    // The lane-per-item kernel's weights feed four rows each (9 instructions an item at 16 inputs against 15): worth it where its
+    // groups of 16 models are mostly full. 100 000 rows x 64 models (16 -> 32 -> 1): 165 us against 275; x 8 models: 45 / 37.
+    const bool grouped = n >= 4096 && hidden > 0 && (hidden & 3) == 0 && k <= 16 && nblock >= 12;
+    // (Whether the feature columns are given or left out as zeros must not change the kernel: kw, not kk_all, decides.)
+    if (!grouped && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
+        const int mg = nblock >= 4 ? 4 : (nblock >= 2 ? 2 : 1);
+        const unsigned cols = dbk::divup(nblock, mg);
+        unsigned gy = dbk::divup(n, 4 * (4 / mg));                 // a row step per wave ...
+        if (gy > 2048u / cols) gy = 2048u / cols;                  // ... until the GPU is full: then the weights serve several
+        if (gy < 1) gy = 1;
+        const dim3 grid(cols, gy);
+#define DBK_HEAD_LANES(KI, HU)                                                                                                        \
+        if (kk_all <= KI * 16 && hidden <= HU * 16) {                                                                                       \
+            hipLaunchKernelGGL((k_head_lanes<KI, HU>), grid, dim3(256), 0, dbk::as_stream(stream), n, nblock, k, kf, kw, hidden, mg, pooled, feats, in_scale, \
+                               W1, b1, W2, b2, apply_logistic != 0, scores);                                                           \
+            DBK_LAUNCH_OK();                                                                                                           \
+        }
+        DBK_HEAD_LANES(1, 0) DBK_HEAD_LANES(2, 0) DBK_HEAD_LANES(4, 0)
+        DBK_HEAD_LANES(1, 1) DBK_HEAD_LANES(1, 2) DBK_HEAD_LANES(2, 1) DBK_HEAD_LANES(2, 2) DBK_HEAD_LANES(1, 4) DBK_HEAD_LANES(4, 1)
+        DBK_HEAD_LANES(2, 4) DBK_HEAD_LANES(4, 2)
+#undef DBK_HEAD_LANES
+    }
     if (hidden > 0 && (hidden & 3) == 0 && smem16 <= 65536 && n >= 4096) {
         // bulk scoring: 16 models per workgroup, coalesced reads of the feature matrix
         const unsigned gy = row_slices(n, kk_all <= 16 ? 64 : (kk_all <= 32 ? 32 : 16), dbk::divup(nblock, HG));

@@ -696,6 +696,27 @@ def test_head_fprop(ds):
     assert_close(host(got0), ref0, ACT, "scores (no hidden)")
 
 
+@pytest.mark.parametrize("n,k,h,nb", [(1, 1, 1, 1), (5, 17, 33, 3), (4097, 12, 0, 4), (70, 64, 32, 2), (301, 33, 16, 5), (9001, 16, 32, 1),
+                                      (4096, 32, 32, 13), (2, 64, 0, 6), (33, 32, 64, 7)])
+def test_head_fprop_lane_groups(ds, n, k, h, nb):
+    """The 16-lanes-per-item kernel: inputs and hidden units that fill no group of 16, one to four models side by side and more, a
+    single row, several steps per wave with a ragged end."""
+    rng = np.random.default_rng(n + k + h + nb)
+    Pl = np.abs(rng.standard_normal((n, k * nb))).astype(np.float32)
+    W1 = (rng.standard_normal((k * nb, h or 1)) * 0.3).astype(np.float32); b1 = (rng.standard_normal((1, (h or 1) * nb)) * 0.1).astype(np.float32)
+    W2 = (rng.standard_normal((h * nb, 1)) * 0.3).astype(np.float32) if h else None
+    b2 = (rng.standard_normal((1, nb)) * 0.1).astype(np.float32) if h else None
+    rate = rng.choice([0.0, 0.25, 0.5], size=nb).astype(np.float32)
+    f64 = lambda v: v.astype(np.float64)
+    ref = orc.bias_fprop(orc.blockwise_dot(orc.dropout_fp_test(f64(Pl), f64(rate)), f64(W1), nb), f64(b1))
+    if h:
+        ref = orc.bias_fprop(orc.blockwise_dot(orc.relu_fprop(ref), f64(W2), nb), f64(b2))
+    for logistic in (False, True):
+        got = ds.head_fprop(dev(Pl), dev(W1), dev(b1), None if W2 is None else dev(W2), None if b2 is None else dev(b2), nblock=nb,
+                            in_scale=1 - rate, apply_logistic=logistic)
+        assert_close(host(got), orc.logistic(ref) if logistic else ref, ACT, "scores")
+
+
 @pytest.mark.parametrize("k,h,nb", [(16, 32, 37), (32, 8, 16), (16, 64, 5)])
 def test_head_fprop_bulk_rows(ds, k, h, nb):
     """Row counts that take the 16-models-per-workgroup kernel; model count not a multiple of 16; dropout rescale."""
