@@ -102,6 +102,22 @@ struct mut_args {
     float *S, *base;                                                // changed scores (4 per stream position), unchanged ones (per region)
 };
 
+// The letter table of filters c0 .. c0 + 15 (filters >= c1: zeros), [tap][letter][16], by all `nt` threads of the workgroup.
+__device__ __forceinline__ void letter_table16(float* __restrict__ lut, const float* __restrict__ W, unsigned m, size_t F, unsigned c0, unsigned c1,
+                                               unsigned nt)
+{
+    for (unsigned e = threadIdx.x; e < m * MUT_F; e += nt) {
+        const unsigned j = e / MUT_F, c = c0 + e % MUT_F;
+        float w[4];
+#pragma unroll
+        for (int l = 0; l < 4; ++l) w[l] = c < c1 ? W[(size_t)(4 * j + l) * F + c] : 0.0f;
+        float z = w[0];
+        z += w[1]; z += w[2]; z += w[3];
+        float* t = lut + (size_t)j * NL * MUT_F + e % MUT_F;
+        t[0] = w[0]; t[MUT_F] = w[1]; t[2 * MUT_F] = w[2]; t[3 * MUT_F] = w[3]; t[4 * MUT_F] = z * 0.25f; t[5 * MUT_F] = 0.0f;
+    }
+}
+
 // Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending; the letters at index
 // `at` and `at2` read as `other`. A letter is read once for the four rows it meets.
 template <bool TWO = false>
@@ -181,16 +197,7 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
         const bool on = f0 + f < a.F;
         const float bf = on ? a.bias[f0 + f] : 0.0f;
         __syncthreads();                                            // the previous tile's table and rows are no longer read
-        for (unsigned e = tid; e < m * MUT_F; e += 256) {
-            const unsigned j = e / MUT_F, c = f0 + e % MUT_F;
-            float w[4];
-#pragma unroll
-            for (int l = 0; l < 4; ++l) w[l] = c < a.F ? a.W[(size_t)(4 * j + l) * a.F + c] : 0.0f;
-            float z = w[0];
-            z += w[1]; z += w[2]; z += w[3];
-            float* t = lut + (size_t)j * NL * MUT_F + e % MUT_F;
-            t[0] = w[0]; t[MUT_F] = w[1]; t[2 * MUT_F] = w[2]; t[3 * MUT_F] = w[3]; t[4 * MUT_F] = z * 0.25f; t[5 * MUT_F] = 0.0f;
-        }
+        letter_table16(lut, a.W, m, a.F, f0, a.F, 256);
         // ---- the region as it is: rows out of reach folded, rows in reach kept
         float mx = 0.0f, sum = 0.0f;
         for (unsigned t0 = ra; t0 < rb; t0 += MUT_TILE) {
@@ -300,6 +307,114 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// scores of few sequences
+// ---------------------------------------------------------------------------------------------
+// Scan, pooling and dense head of one (region, model) per workgroup of NT threads, for calls that are all latency: 16 lanes of
+// filters x NT / 16 lanes of rows, four rows each at a time; lane h of the first wave holds hidden unit h's weights, on
+// their way while the region is scanned. One launch and two round trips to memory (bounds, then letters and weights) where
+// the scan kernel and the head cost a launch and three each. KM: pooled features per model, at most.
+// Measured: 64 sequences x 101 nt, 16 filters of 24 taps, 16 -> 32 -> 1: 5.9 us, the whole call 10.0 with its host side (scan kernel
+// 11.5 + head 4.1, the call 17.8).
+struct small_args {
+    const float *W, *bias, *W1, *b1, *W2, *b2, *in_scale;
+    const uint8_t* X;
+    const uint32_t* R;
+    size_t N;
+    unsigned m, nmodel, nfilter, k, hidden;
+    int ptype, logistic;
+    float* scores;
+};
+
+inline size_t small_smem(size_t m, unsigned nt) { return ((size_t)m * NL * MUT_F + nt / 64 * 2 * MUT_F + 2 * MUT_F) * sizeof(float) + mut_tile_letters((unsigned)m); }
+
+template <int KM, int NT>
+__global__ __launch_bounds__(NT) void k_predict_small(const small_args a)
+{
+    extern __shared__ __align__(16) float msm[];
+    const unsigned m = a.m, tid = threadIdx.x, lane = tid & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const unsigned b = blockIdx.y, f = tid & 15u, rl = tid >> 4;
+    const size_t r = blockIdx.x;
+    float* lut = msm;
+    float* part = lut + m * NL * MUT_F;                             // [waves][2][16]: maxima, sums
+    float* x = part + NT / 64 * 2 * MUT_F;                          // pooled features
+    uint8_t* tile = reinterpret_cast<uint8_t*>(x + 2 * MUT_F);
+    const unsigned ra = a.R[2 * r], rb = a.R[2 * r + 1];
+    const unsigned c0 = b * a.nfilter;
+    const size_t F = (size_t)a.nmodel * a.nfilter;
+    const float bf = f < a.nfilter ? a.bias[c0 + f] : 0.0f;
+    letter_table16(lut, a.W, m, F, c0, c0 + a.nfilter, NT);
+    float w[KM], b1v = 0.0f, w2v = 0.0f;
+    if (wave == 0) {
+        const unsigned h1 = a.hidden ? a.hidden : 1u;
+        const bool in = lane < h1;
+        // without a hidden layer lane l holds input l's weight
+        if (a.hidden) {
+#pragma unroll
+            for (int kk = 0; kk < KM; ++kk) w[kk] = in && kk < (int)a.k ? a.W1[((size_t)b * a.k + kk) * h1 + lane] : 0.0f;
+            w2v = in ? a.W2[(size_t)b * h1 + lane] : 0.0f;
+        } else w[0] = lane < a.k ? a.W1[(size_t)b * a.k + lane] : 0.0f;
+        b1v = in ? a.b1[(size_t)b * h1 + lane] : 0.0f;
+    }
+    const size_t n = a.N >= m ? a.N - m + 1 : 0;                   // rows the scan defines; later rows are relu(bias)
+    float mx = 0.0f, sum = 0.0f;
+    for (unsigned t0 = ra; t0 < rb; t0 += MUT_TILE) {
+        if (t0 != ra) __syncthreads();
+        const unsigned t1 = rb - t0 < MUT_TILE ? rb : t0 + MUT_TILE, count = t1 - t0 + m + 3;
+        for (unsigned e = tid; e < count; e += NT) tile[e] = (uint8_t)((t0 + (size_t)e < a.N ? letter_of(a.X[t0 + (size_t)e]) : 5u) * MUT_F);
+        __syncthreads();
+        for (unsigned p = t0 + 4 * rl; p < t1; p += NT / 4) {
+            float z[4];
+            scan4(lut + f, tile, p - t0, m, ~0u, 0u, z);
+#pragma unroll
+            for (unsigned u = 0; u < 4; ++u)
+                if (p + u < t1) {
+                    float v = (p + u < n ? z[u] : 0.0f) + bf;
+                    v = v > 0.0f ? v : 0.0f;
+                    mx = v > mx ? v : mx;
+                    sum += v;
+                }
+        }
+    }
+#pragma unroll
+    for (int d = 16; d <= 32; d <<= 1) {
+        const float v = __shfl_xor(mx, d, 64);
+        mx = v > mx ? v : mx;
+        sum += __shfl_xor(sum, d, 64);
+    }
+    if (lane < MUT_F) { part[(2 * wave) * MUT_F + f] = mx; part[(2 * wave + 1) * MUT_F + f] = sum; }
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane < MUT_F) {
+        for (unsigned v = 1; v < NT / 64; ++v) {
+            const float o = part[(2 * v) * MUT_F + f];
+            mx = o > mx ? o : mx;
+            sum += part[(2 * v + 1) * MUT_F + f];
+        }
+        const float sc = a.in_scale ? a.in_scale[b] : 1.0f, avg = sum / (float)(rb - ra);
+        if (a.ptype == DBK_PT_ALL) { x[2 * f] = mx * sc; x[2 * f + 1] = avg * sc; }
+        else x[f] = (a.ptype == DBK_PT_MAX ? mx : avg) * sc;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float out;
+    if (a.hidden) {
+        float z = 0.0f;
+#pragma unroll
+        for (int kk = 0; kk < KM; ++kk) z = __builtin_fmaf(kk < (int)a.k ? x[kk] : 0.0f, w[kk], z);
+        z += b1v;
+        out = (z > 0.0f ? z : 0.0f) * w2v;
+    } else out = lane < a.k ? x[lane] * w[0] : 0.0f;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) out += __shfl_xor(out, d, 64);
+    if (lane == 0) {
+        out += a.hidden ? a.b2[b] : b1v;
+        if (a.logistic) out = 1.0f / (1.0f + expf(-out));
+        a.scores[r * a.nmodel + b] = out;
+    }
+}
+
 // The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
 // is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. One workgroup per sequence.
 __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const float* __restrict__ S,
@@ -363,6 +478,34 @@ int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* o
     const size_t nbyte = nwindow * strands * (padding + window) + padding;
     hipLaunchKernelGGL(k_pack_windows, dim3(dbk::ew_grid(nbyte)), dim3(256), 0, dbk::as_stream(stream), text, offsets, first, (unsigned)nseq,
                        (unsigned)window, (unsigned)stride, (unsigned)padding, (unsigned)strands, nbyte, X, R);
+    DBK_LAUNCH_OK();
+}
+
+int dbk_predict_small_takes(size_t m, size_t nmodel, size_t nfilter, size_t N, size_t nregion, int ptype, size_t hidden)
+{
+    // Every workgroup stages its model's weights: worth it while the call is one wave of latency. Measured with 24 taps (us a call,
+    // this kernel / scan kernel + head): 2000 x 101 nt 15 / 18, 4000 x 101 nt 27 / 21, 900 x 500 nt 24 / 23, 100 x 101 nt x 32 models 22 / 17.
+    return m >= 1 && m <= 64 && nfilter >= 1 && nfilter <= MUT_F && hidden <= 64 && N * nmodel * m <= 6000000 && nregion < ((size_t)1 << 31) && nmodel <= 65535 &&
+           (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL);
+}
+
+int dbk_predict_small(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nmodel, size_t nfilter, const uint8_t* X, size_t N,
+                      const uint32_t* regions, size_t nregion, int ptype, size_t hidden, const float* W1, const float* b1, const float* W2,
+                      const float* b2, const float* in_scale, int apply_logistic, float* scores)
+{
+    if (nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(dbk_predict_small_takes(m, nmodel, nfilter, N, nregion, ptype, hidden), "NotImplementedError: dbk_predict_small takes up to 6e6 rows x models x taps, "
+              "models of up to 16 filters of up to 64 taps and 64 hidden units");
+    DBK_CHECK(W && bias && X && regions && W1 && b1 && scores, "ValueError: null pointer argument");
+    DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
+    small_args a;
+    a.W = W; a.bias = bias; a.W1 = W1; a.b1 = b1; a.W2 = W2; a.b2 = b2; a.in_scale = in_scale; a.X = X; a.R = regions; a.N = N;
+    a.m = (unsigned)m; a.nmodel = (unsigned)nmodel; a.nfilter = (unsigned)nfilter; a.k = (unsigned)(nfilter * (ptype == DBK_PT_ALL ? 2 : 1));
+    a.hidden = (unsigned)hidden; a.ptype = ptype; a.logistic = apply_logistic; a.scores = scores;
+    const bool wide = N > 64 * nregion;                             // 512 threads scan 128 rows at once
+    auto kern = a.k <= 16 ? (wide ? k_predict_small<16, 512> : k_predict_small<16, 256>) : (wide ? k_predict_small<32, 512> : k_predict_small<32, 256>);
+    const unsigned nt = wide ? 512u : 256u;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nregion, (unsigned)nmodel), dim3(nt), small_smem(m, nt), dbk::as_stream(stream), a);
     DBK_LAUNCH_OK();
 }
 

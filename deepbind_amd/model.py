@@ -390,6 +390,17 @@ class SequenceNet(object):
     def predict(self, X, R, F=None):
         """Test-mode predictions through the fused scoring head (dropout rescale folded in)."""
         p = self.p
+        P, ptype = R.shape[0], _lib.str2pooltype[self.pool]
+        if self.mode == "fused" and self.dtype == torch.float32 and self.nfeat == 0 and R.shape[1] == 2 and _lib.dll().dbk_predict_small_takes(
+                self.m, self.ninst, self.nfilter, X.numel(), P, ptype, self.hidden):
+            # a handful of sequences: one launch for everything
+            Wc = p["Wc"] if self.input_dropout <= 0 else p["Wc"] * (1.0 - self.input_dropout)
+            scale = (1.0 - self.dropout) if self.use_dropout else None
+            Z = torch.empty((P, self.ninst), dtype=torch.float32, device=X.device)
+            _lib.call("dbk_predict_small", _lib.stream(), _lib.ptr(Wc), _lib.ptr(p["bc"]), self.m, self.ninst, self.nfilter, _lib.ptr(ks._u8(X)),
+                      X.numel(), _lib.ptr(ks._regions(R)), P, ptype, self.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")),
+                      _lib.ptr(p.get("b2")), _lib.ptr(scale), int(self.loss == "nll"), _lib.ptr(Z))
+            return ds.pair_max(Z) if self.reverse_complement else Z
         pooled, _, _ = self._conv_forward(X, R, False)
         if self.dtype != torch.float32:
             Z = self.forward(X, R, F=F)["Z"]

@@ -145,3 +145,28 @@ def test_text_and_windows_are_packed_as_on_the_host(rc, m, window, stride):
         cut += [padded[i:i + window] for i in range(0, max(1, len(padded) - window + 1), stride)]
     Xr, Rr = data.pack_sequences(cut, m - 1, reverse_complement=rc)
     assert np.array_equal(seen[0][0], Xr) and np.array_equal(seen[0][1], Rr)
+
+
+@pytest.mark.parametrize("pool,hidden,loss,rc,m,F,nm,lo,hi", [("max", 32, "nll", False, 24, 16, 1, 101, 101), ("all", 0, "mse", True, 32, 16, 3, 0, 40),
+                                                              ("avg", 64, "mse", False, 1, 1, 5, 1, 9), ("all", 33, "nll", False, 11, 7, 2, 490, 1100),
+                                                              ("max", 1, "mse", True, 64, 12, 1, 60, 70)])
+def test_single_launch_scores(pool, hidden, loss, rc, m, F, nm, lo, hi):
+    """The one-launch scoring kernel: regions below and above 64 rows on average and beyond one tile of 512, models whose filters and
+    pooled features fill no group of 16, hidden units up to a wave; against the oracle's forward pass."""
+    from deepbind_amd import _lib, data
+    from deepbind_amd.model import SequenceNet
+    rng = np.random.default_rng(m + F + nm)
+    seqs = _seqs(rng, 9, lo, hi)
+    net = SequenceNet(nm, F, m, pool=pool, hidden=hidden, loss=loss, dropout=0.25, reverse_complement=rc)
+    params = {name: (rng.standard_normal(shape) * (0.3 if name == "Wc" else 0.2)).astype(np.float32) for name, shape, _ in net.layout}
+    net.set_params(params)
+    X, R = data.pack_sequences(seqs, m - 1, reverse_complement=rc)
+    X[rng.random(len(X)) < 0.02] = 254
+    assert _lib.dll().dbk_predict_small_takes(m, nm, F, X.size, len(R), _lib.str2pooltype[pool], hidden) == 1
+    got = net.predict(torch.from_numpy(X).cuda(), torch.from_numpy(R).cuda()).cpu().numpy()
+    st = orc.model_forward({k: v.astype(np.float64) for k, v in params.items()}, X, R, nm, pool, hidden, out="logistic" if loss == "nll" else "linear",
+                           dropout=(np.full(nm, 0.25), None))
+    want = st["Zout"]
+    if rc:
+        want = want.reshape(-1, 2, nm).max(axis=1)
+    assert_close(got, want, ACT, "scores")
