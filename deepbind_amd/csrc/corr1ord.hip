@@ -11,6 +11,7 @@
 #include "dbk_common.h"
 #include "scan_common.h"
 #include "mfma_common.h"
+#include "corr1ord_mm.h"
 #include <type_traits>
 
 namespace {
@@ -195,7 +196,7 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_kernel(T* __restrict__ d
 // positions, so the letters of a 16-position window are read once into scalar registers.
 // ---------------------------------------------------------------------------------------------
 constexpr unsigned WSUBS = 4;             // windows of PSUB positions per wave and staging round
-constexpr unsigned WSUBS_W = 8;           // the same for the filter-gradient kernel
+constexpr unsigned WSUBS_W = 8;           // the same for the register-plane kernel
 
 // forward: every (position, tap) is one LDS read with an immediate offset; taps in ascending order,
 // so the sums are bit-identical to the any-length kernel's. A workgroup builds its filter tile's
@@ -313,164 +314,6 @@ __global__ __launch_bounds__(256) void corr1ord_wide_kernel(const float* __restr
                 if (f + 3 < F) dst[3] = acc[p].w;
             }
         }
-    }
-}
-
-// filter gradient, pass 1: a lane keeps its filter's whole [letter][tap] column in registers; the window's
-// letters (scalars) pick the register plane each gradient value is added into through the register index
-// mode: one addition per (position, tap). "Mean of the four" letters collect in a plane of their own that
-// is spread over the four channels (x 1/4) at the end.
-// Workgroup y walks chunks y, y+gridDim.y, ... in ascending order; its waves are folded in wave order.
-template <int MT>
-__global__ __launch_bounds__(256) void corr1ord_bprop_W_window_kernel(float* __restrict__ partial, unsigned m, unsigned F,
-                                                                      const uint8_t* __restrict__ X, size_t n,
-                                                                      const float* __restrict__ dZ)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    float* fold = reinterpret_cast<float*>(smem);                          // [MT*4][FT]
-    uint8_t* xl = smem + (size_t)MT * 4 * FT * sizeof(float);
-    const unsigned nw = blockDim.x >> 6, chunk = nw * WSUBS_W * PSUB;
-    const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const unsigned f0 = blockIdx.x * FT, f = f0 + lane;
-    const size_t N = n + m - 1;
-    grad_planes<MT> planes;                                                // [letter][tap] accumulators in fixed registers
-    planes.clear();
-    for (size_t c0 = (size_t)blockIdx.y * chunk; c0 < n; c0 += (size_t)gridDim.y * chunk) {
-        const unsigned rows = (unsigned)((n - c0) < chunk ? (n - c0) : chunk);
-        __syncthreads();
-        stage(xl, X, N, c0, window_span<MT>(rows));
-        __syncthreads();
-        // the next window's gradient rows are requested before this window's additions start
-        float g[PSUB], gn[PSUB];
-        auto fetch = [&](unsigned p0, float (&dst)[PSUB]) {
-#pragma unroll
-            for (int p = 0; p < PSUB; ++p) dst[p] = (f < F && p0 + p < rows) ? dZ[(c0 + p0 + p) * F + f] : 0.0f;
-        };
-        fetch(wave * PSUB, g);
-#pragma unroll 1
-        for (unsigned s = 0; s < WSUBS_W; ++s) {
-            const unsigned p0 = (s * nw + wave) * PSUB;
-            if (p0 >= rows) break;
-            fetch(p0 + nw * PSUB, gn);                                     // all zero past the chunk's rows
-            unsigned wq[window<MT>::words];
-            load_window<MT>(xl, p0, wq);
-            grad_planes_window<MT>(planes, wq, g);                         // one add per (position, tap)
-#pragma unroll
-            for (int p = 0; p < PSUB; ++p) g[p] = gn[p];
-        }
-    }
-    float aw[MT][4];
-    grad_planes_read<MT>(planes, aw);
-    float* mine = fold + lane;
-    for (unsigned w = 0; w < nw; ++w) {
-        __syncthreads();
-        if (wave == w) {
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-                if ((unsigned)j < m) {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        float* cell = mine + (j * 4 + c) * FT;
-                        *cell = w == 0 ? aw[j][c] : *cell + aw[j][c];
-                    }
-                }
-        }
-    }
-    __syncthreads();
-    float* out = partial + (size_t)blockIdx.y * (4 * m) * F;
-    for (unsigned e = threadIdx.x; e < m * 4 * FT; e += blockDim.x) {
-        const unsigned row = e / FT, fl = e % FT;
-        if (f0 + fl < F) out[(size_t)row * F + f0 + fl] = fold[e];
-    }
-}
-
-// input gradient: a wave owns RPW consecutive rows and walks the filter tiles; a lane holds its filter's
-// [tap][channel] weights in registers and a ring of the last MT gradient rows, so each row of dZ is read
-// once per tile and each (row, tap, channel) is one multiply-add. Row sums over the 64 filters of a tile
-// go through LDS eight rows at a time: every lane parks its 32 partial sums, then lane v < 32 adds up
-// value v over the 64 lanes in lane order (a fixed order); tiles are added in ascending order into the
-// wave's rows in LDS.
-constexpr int XR_STRIDE = 65;             // odd row stride: the 32 column sums read 32 different banks
-constexpr int XR_AHEAD = 4;               // rows of dZ in flight per lane
-
-template <int MT, int RPW>
-__global__ __launch_bounds__(256) void corr1ord_bprop_X_ring_kernel(float* __restrict__ dX, size_t n, const float* __restrict__ W,
-                                                                    unsigned m, unsigned F, const float* __restrict__ dZ)
-{
-    static_assert(RPW % MT == 0 && MT % 8 == 0 && MT % XR_AHEAD == 0, "a wave's rows are walked in blocks of MT, reduced eight at a time");
-    __shared__ float rows_acc[4][RPW * 4];
-    __shared__ float parts[4][32 * XR_STRIDE];
-    const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const size_t i0 = ((size_t)blockIdx.x * 4 + wave) * RPW;
-    if (i0 >= n) return;                                                   // (no barriers in this kernel)
-    float* acc = rows_acc[wave];
-    float* part = parts[wave];
-    for (unsigned e = lane; e < RPW * 4; e += 64) acc[e] = 0.0f;
-    const unsigned ftiles = (F + FT - 1) / FT;
-    for (unsigned t = 0; t < ftiles; ++t) {
-        const unsigned f = t * FT + lane;
-        const bool live = f < F;
-        float w[MT][4];
-#pragma unroll
-        for (int k = 0; k < MT; ++k) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) w[k][c] = (live && (unsigned)k < m) ? W[(size_t)(4 * k + c) * F + f] : 0.0f;
-        }
-        // ring slot r holds row i with i % MT == r (i0 is a multiple of MT); start with the MT-1 rows before i0
-        float ring[MT];
-        ring[0] = 0.0f;
-#pragma unroll
-        for (int r = 1; r < MT; ++r) {
-            const bool have = i0 + r >= (size_t)MT;                         // row i0 - MT + r exists
-            ring[r] = (live && have) ? dZ[(i0 - MT + r) * F + f] : 0.0f;
-        }
-        // rows are fetched XR_AHEAD positions before they are used (MT is a multiple of XR_AHEAD, so the
-        // slot of a row is a compile-time index)
-        float pre[XR_AHEAD];
-#pragma unroll
-        for (int d = 0; d < XR_AHEAD; ++d) pre[d] = (live && i0 + d < n) ? dZ[(i0 + d) * F + f] : 0.0f;
-#pragma unroll 1
-        for (unsigned b0 = 0; b0 < RPW; b0 += MT) {
-            if (i0 + b0 >= n) break;
-#pragma unroll
-            for (int u = 0; u < MT; ++u) {
-                ring[u] = pre[u % XR_AHEAD];
-                {
-                    const size_t i = i0 + b0 + u + XR_AHEAD;
-                    pre[u % XR_AHEAD] = (live && i < n) ? dZ[i * F + f] : 0.0f;
-                }
-                float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-#pragma unroll
-                for (int k = 0; k < MT; ++k) {
-                    const float dz = ring[(u - k + MT) % MT];              // row i - k
-                    s0 = __builtin_fmaf(dz, w[k][0], s0);
-                    s1 = __builtin_fmaf(dz, w[k][1], s1);
-                    s2 = __builtin_fmaf(dz, w[k][2], s2);
-                    s3 = __builtin_fmaf(dz, w[k][3], s3);
-                }
-                float* mine = part + ((u & 7) * 4) * XR_STRIDE + lane;
-                mine[0 * XR_STRIDE] = s0;
-                mine[1 * XR_STRIDE] = s1;
-                mine[2 * XR_STRIDE] = s2;
-                mine[3 * XR_STRIDE] = s3;
-                if ((u & 7) == 7) {
-                    // the wave's own LDS accesses execute in program order; no other wave touches `part`
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane < 32) {
-                        const float* col = part + lane * XR_STRIDE;
-                        float tot = 0.0f;
-#pragma unroll 16
-                        for (int l = 0; l < 64; ++l) tot += col[l];
-                        acc[(b0 + u - 7) * 4 + lane] += tot;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                }
-            }
-        }
-    }
-    for (unsigned e = lane; e < RPW * 4; e += 64) {
-        const size_t i = i0 + e / 4;
-        if (i < n) dX[i * 4 + (e & 3)] += acc[e];
     }
 }
 
@@ -817,7 +660,9 @@ void launch_bprop_W_mfma_mb(hipStream_t st, float* partial, unsigned gy, unsigne
     hipLaunchKernelGGL(corr1ord_bprop_W_mfma_kernel<MB>, dim3(dbk::divup(F, 128), gy), dim3(256), 0, st, partial, (unsigned)m, (unsigned)F, X, n, dZ, rounds);
 }
 
-// Bulk sizes only: below, the partial results (one 4m x F block per workgroup) cost more than the rows.
+// Bulk sizes only: below, the partial results (one 4m x F block per workgroup) cost more than the rows, and the float32 products of
+// corr1ord_mm.h take over (us a call, this / those: 123 000 rows x 64 filters of 24 taps 34 / 43, 20 000 x 256 17 / 28; 60 000 x 48
+// of 16 taps 29 / 24 through the vector kernel that came before).
 inline bool bprop_W_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 32 && n * F >= ((size_t)1 << 22) && n >= 4096; }
 
 inline int launch_bprop_W_mfma(hipStream_t st, float* dW, size_t m, size_t F, const uint8_t* X, size_t n, const float* dZ)
@@ -839,26 +684,6 @@ inline int launch_bprop_W_mfma(hipStream_t st, float* dW, size_t m, size_t F, co
     default: launch_bprop_W_mfma_mb<4>(st, partial, (unsigned)gy, rounds, m, F, X, n, dZ); break;
     }
     hipLaunchKernelGGL(reduce_partials_quarters_kernel, dim3((unsigned)dbk::divup(nelem, 64)), dim3(256), 0, st, dW, (const float*)partial, nelem, (unsigned)gy);
-    DBK_LAUNCH_OK();
-}
-
-// float32 filters of at most 24 taps: register-resident gradient columns
-inline int launch_bprop_W_window(hipStream_t st, float* dW, size_t m, size_t F, const uint8_t* X, size_t n, const float* dZ)
-{
-    const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : 24);
-    const unsigned ftiles = dbk::divup(F, FT), chunk = 4 * WSUBS_W * PSUB;
-    const unsigned nchunk = dbk::divup(n, chunk);
-    unsigned gy = (mt == 8 ? 768u : 512u) / ftiles;           // three workgroups fit a CU with 8 taps' register planes, else two
-    if (gy < 1) gy = 1;
-    if (gy > nchunk) gy = nchunk;
-    const size_t nelem = 4 * m * F;
-    float* partial = (float*)dbk::workspace(nelem * gy * sizeof(float), st);
-    DBK_CHECK(partial != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", nelem * gy * sizeof(float), dbk::workspace_error());
-    const size_t smem = (size_t)mt * 4 * FT * sizeof(float) + ((chunk + mt - 1 + 7) & ~(size_t)3);
-    auto kern = mt == 8 ? corr1ord_bprop_W_window_kernel<8> : mt == 16 ? corr1ord_bprop_W_window_kernel<16> : corr1ord_bprop_W_window_kernel<24>;
-    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    hipLaunchKernelGGL(kern, dim3(ftiles, gy), dim3(256), smem, st, partial, (unsigned)m, (unsigned)F, X, n, dZ);
-    hipLaunchKernelGGL(reduce_partials_kernel<float>, dim3(dbk::ew_grid(nelem)), dim3(256), 0, st, dW, (const float*)partial, nelem, gy);
     DBK_LAUNCH_OK();
 }
 
@@ -1027,7 +852,10 @@ __global__ __launch_bounds__(64 * MB) void corr1ord_bprop_X_mfma_kernel(float* _
     for (size_t e = threadIdx.x; e < nout; e += NT) dX[o0 * 4 + e] += out[e];
 }
 
-inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 64 && n * F >= ((size_t)1 << 22) && n >= 4096; }
+// A launch per 128 filters with the weights' pieces formed per workgroup, against the float32 products of corr1ord_mm.h (us a call, this /
+// those): 100 000 rows x 128 filters of 24 taps 51 / 54, 120 000 x 128 of 32 taps 55 / 72, 1.0 M x 256 450 / 943; 60 000 x 128 50 / 41,
+// 40 000 x 256 95 / 72, 200 000 x 96 111 / 82.
+inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 128 && n * F >= 12000000; }
 
 inline int launch_bprop_X_mfma(hipStream_t st, float* dX, size_t n, const float* W, size_t m, size_t F, const float* dZ)
 {
@@ -1054,15 +882,45 @@ inline int launch_bprop_X_mfma(hipStream_t st, float* dX, size_t n, const float*
     DBK_LAUNCH_OK();
 }
 
-inline int launch_bprop_X_ring(hipStream_t st, float* dX, size_t n, const float* W, size_t m, size_t F, const float* dZ)
+// Filters of up to 32 taps on the 16 x 16 x 4 products (corr1ord_mm.h).
+template <typename T>
+int launch_bprop_W_mm(hipStream_t st, T* dW, size_t m, size_t F, const uint8_t* X, size_t n, const T* dZ)
 {
-    if (m <= 8) {
-        hipLaunchKernelGGL((corr1ord_bprop_X_ring_kernel<8, 96>), dim3(dbk::divup(n, 4 * 96)), dim3(256), 0, st, dX, n, W, (unsigned)m, (unsigned)F, dZ);
-    } else if (m <= 16) {
-        hipLaunchKernelGGL((corr1ord_bprop_X_ring_kernel<16, 96>), dim3(dbk::divup(n, 4 * 96)), dim3(256), 0, st, dX, n, W, (unsigned)m, (unsigned)F, dZ);
-    } else {
-        hipLaunchKernelGGL((corr1ord_bprop_X_ring_kernel<24, 96>), dim3(dbk::divup(n, 4 * 96)), dim3(256), 0, st, dX, n, W, (unsigned)m, (unsigned)F, dZ);
+    using namespace dbk_corr_mm;
+    const unsigned groups = dbk::divup(F, 16);
+    // two workgroups per CU; a wave with fewer than 64 rows would spend its time on the fold
+    size_t slices = 512 / groups;
+    if (slices > n / 256) slices = n / 256;
+    if (slices < 1) slices = 1;
+    const unsigned rows = (unsigned)(dbk::divup(n, slices * 4 * 32) * 32);
+    slices = dbk::divup(n, (size_t)rows * 4);
+    const size_t nelem = 4 * m * F;
+    T* partial = (T*)dbk::workspace(nelem * slices * sizeof(T), st);
+    DBK_CHECK(partial != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", nelem * slices * sizeof(T), dbk::workspace_error());
+    const dim3 grid(groups, (unsigned)slices);
+#define DBK_GO(TT)                                                                                                    \
+    {                                                                                                                 \
+        const size_t smem = TT * 256 * 4 * sizeof(T);                                                                  \
+        auto kern = corr1ord_bprop_W_mm_kernel<T, TT>;                                                                \
+        DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));       \
+        hipLaunchKernelGGL(kern, grid, dim3(256), smem, st, partial, (unsigned)m, (unsigned)F, X, n, dZ, rows);       \
     }
+    if (m <= 8) DBK_GO(2) else if (m <= 16) DBK_GO(4) else if (m <= 24) DBK_GO(6) else DBK_GO(8)
+#undef DBK_GO
+    hipLaunchKernelGGL(reduce_partials_kernel<T>, dim3(dbk::ew_grid(nelem)), dim3(256), 0, st, dW, (const T*)partial, nelem, (unsigned)slices);
+    DBK_LAUNCH_OK();
+}
+
+template <typename T>
+int launch_bprop_X_mm(hipStream_t st, T* dX, size_t n, const T* W, size_t m, size_t F, const T* dZ)
+{
+    using namespace dbk_corr_mm;
+    // fewer than two workgroups of 256 rows per CU: 64 rows each, whose bits then depend on the size of the call
+    const bool few = !dbk::exact_scan() && n < 512 * 256;
+    const size_t smem = cx_smem<T>(m, few ? 1 : 4);
+    auto kern = few ? corr1ord_bprop_X_mm_kernel<T, 1> : corr1ord_bprop_X_mm_kernel<T, 4>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3(dbk::divup(n, few ? 64 : 256)), dim3(256), smem, st, dX, n, W, (unsigned)m, (unsigned)F, dZ);
     DBK_LAUNCH_OK();
 }
 
@@ -1125,8 +983,9 @@ int dbk_corr1ord_bprop_W(dbk_stream_t stream, int dtype, void* dW, size_t m, siz
     if (n == 0 || nfilter == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(dW && X && dZ, "ValueError: null pointer argument");
     if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_W_mfma_takes(m, nfilter, n)) return launch_bprop_W_mfma(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
-    if (dtype == DBK_F32 && m <= 24) return launch_bprop_W_window(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
+    if (dtype == DBK_F32 && m <= 32) return launch_bprop_W_mm<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F32) return launch_bprop_W<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
+    if (dtype == DBK_F64 && m <= 32) return launch_bprop_W_mm<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);
     return launch_bprop_W<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);
 }
 
@@ -1139,8 +998,9 @@ int dbk_corr1ord_bprop_X(dbk_stream_t stream, int dtype, void* dX, size_t n, siz
     if (n == 0 || nfilter == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(dX && W && dZ, "ValueError: null pointer argument");
     if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_X_mfma_takes(m, nfilter, n)) return launch_bprop_X_mfma(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
-    if (dtype == DBK_F32 && m <= 24) return launch_bprop_X_ring(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
+    if (dtype == DBK_F32 && m <= 64) return launch_bprop_X_mm<float>(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
     if (dtype == DBK_F32) return launch_bprop_X<float>(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
+    if (dtype == DBK_F64 && m <= 64) return launch_bprop_X_mm<double>(dbk::as_stream(stream), (double*)dX, n, (const double*)W, m, nfilter, (const double*)dZ);
     return launch_bprop_X<double>(dbk::as_stream(stream), (double*)dX, n, (const double*)W, m, nfilter, (const double*)dZ);
 }
 

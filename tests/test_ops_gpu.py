@@ -186,6 +186,31 @@ def test_corr1ord_bprop_X(ks, n, m, F, dtype):
     assert np.array_equal(host(dX), host(dX2))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,m,F", [(1, 1, 1), (63, 8, 15), (64, 9, 17), (257, 32, 33), (1000, 25, 16), (3000, 33, 5), (131329, 24, 3), (700, 64, 20)])
+def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype):
+    """Both gradients at the edges of the 16 x 16 x 4 kernels: rows around a block of 64 and a chunk of 256, fewer rows than taps, each tap
+    tier and the first length beyond it, filters that leave most of a group of 16 empty, calls of one block per workgroup and of four;
+    every letter code."""
+    rng = np.random.default_rng(n + m + F)
+    tol = GRAD if dtype == np.float32 else 1e-12
+    X = random_codes(rng, n + m - 1, 0.05, 0.05).reshape(-1, 1)
+    dZ = np.zeros((n + m - 1, F), dtype); dZ[:n] = rng.standard_normal((n, F))
+    W = (rng.standard_normal((4 * m, F)) * 0.1).astype(dtype)
+    ref = np.ones((4 * m, F)); orc.corr1ord_bprop_W(ref, X, dZ.astype(np.float64))
+    dW = dev(np.ones((4 * m, F), dtype))
+    ks.corr1ord_bprop_W(dW, dev(X), dev(dZ), 4)
+    assert_close(host(dW), ref, tol, "dW")
+    refx = np.ones((n + m - 1, 4)); orc.corr1ord_bprop_X(refx, W.astype(np.float64), dZ.astype(np.float64))
+    outs = []
+    for _ in range(2):
+        dX = dev(np.ones((n + m - 1, 4), dtype))
+        ks.corr1ord_bprop_X(dX, dev(W), dev(dZ), 4)
+        outs.append(host(dX))
+    assert_close(outs[0], refx, tol, "dX")
+    assert np.array_equal(outs[0], outs[1])
+
+
 # ------------------------------------------------------------------------------------------ pooling
 def _regions(rng, P, lo, hi, gap=0):
     lens = rng.integers(lo, hi + 1, size=P)
