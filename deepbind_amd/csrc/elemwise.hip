@@ -297,7 +297,7 @@ template <typename T> __global__ void k_add_rowvec(const T* X, const T* b, T* Z,
 }
 // Column sums in a fixed order. Workgroup (x, y) takes 64 columns and row slice y; wave w sums rows
 // w, w+4, ... of the slice in ascending order (four rows in flight), the four waves are combined in
-// wave order, and k_colsum_fold adds the slices in ascending order: the summation order depends only
+// wave order, and k_colsum_fold adds the slices in a fixed order: the summation order depends only
 // on the shape.
 template <typename T> __global__ __launch_bounds__(256) void k_colsum(const T* __restrict__ X, T* __restrict__ out, size_t n, size_t m,
                                                                       size_t rows_per_slice)
@@ -323,13 +323,36 @@ template <typename T> __global__ __launch_bounds__(256) void k_colsum(const T* _
     __syncthreads();
     if (w == 0 && c < m) out[(size_t)blockIdx.y * m + c] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
 }
-template <typename T> __global__ void k_colsum_fold(const T* __restrict__ partial, T* __restrict__ out, size_t m, unsigned nslice)
+// A workgroup folds 64 columns: its 16 waves take every 16th slice, eight loads in flight each, and the 16 sums are added in wave
+// order. (One thread per column adding slice after slice: 20-25 us of the 35-230 us that the column sums of 64-256 columns take.)
+// rep > 1: the 64 columns are `rep` rows of a matrix of 64 / rep columns that k_colsum took side by side; their sums are added in row
+// order, and the ntail rows that fill no such group after them. (48 of 64 lanes idle otherwise: 496 000 rows x 16 columns 78 -> 10 us.)
+template <typename T> __global__ __launch_bounds__(1024) void k_colsum_fold(const T* __restrict__ partial, T* __restrict__ out, size_t m, unsigned nslice,
+                                                                            unsigned rep, const T* __restrict__ tail, unsigned ntail)
 {
-    GRID_STRIDE(c, m) {
-        T s = partial[c];
+    __shared__ T part[16][64];
+    const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t c = (size_t)blockIdx.x * 64 + lane;
+    T s = (T)0;
+    if (c < m) {
 #pragma unroll 8
-        for (unsigned y = 1; y < nslice; ++y) s += partial[(size_t)y * m + c];
-        out[c] = s;
+        for (unsigned y = w; y < nslice; y += 16) s += partial[(size_t)y * m + c];
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && c < m) {
+#pragma unroll
+        for (unsigned v = 1; v < 16; ++v) s += part[v][lane];
+        if (rep == 1) { out[c] = s; return; }
+        part[0][lane] = s;                                          // (m is 64 here: one workgroup, all lanes)
+    }
+    if (rep == 1) return;
+    __syncthreads();
+    const unsigned cols = 64 / rep;
+    if (w == 0 && lane < cols) {
+        for (unsigned v = 1; v < rep; ++v) s += part[0][v * cols + lane];
+        for (unsigned t = 0; t < ntail; ++t) s += tail[(size_t)t * cols + lane];
+        out[lane] = s;
     }
 }
 template <typename T> __global__ void k_relu(const T* X, T* Z, size_t n)
@@ -501,6 +524,12 @@ inline unsigned pack_grid(size_t n, size_t per_pack) { return (unsigned)dbk::div
 template <typename T>
 int launch_colsum(hipStream_t st, const T* X, T* out, size_t n, size_t m)
 {
+    // rows of 1, 2, 4 .. 32 columns: as many as make 64 side by side
+    const unsigned rep = n >= 4096 && m < 64 && 64 % m == 0 ? (unsigned)(64 / m) : 1u;
+    const T* tail = X + n / rep * rep * m;
+    const unsigned ntail = (unsigned)(n % rep);
+    n /= rep;
+    m *= rep;
     const unsigned tiles = dbk::divup(m, 64);
     // slices of at least 256 rows, about 2048 workgroups in all
     size_t nslice = (n + 255) / 256;
@@ -508,14 +537,14 @@ int launch_colsum(hipStream_t st, const T* X, T* out, size_t n, size_t m)
     if (nslice > cap) nslice = cap;
     if (nslice < 1) nslice = 1;
     const size_t rows_per = (n + nslice - 1) / nslice;
-    if (nslice == 1) {
+    if (nslice == 1 && rep == 1) {
         hipLaunchKernelGGL(k_colsum<T>, dim3(tiles, 1), dim3(256), 0, st, X, out, n, m, rows_per);
         return 0;
     }
     T* partial = (T*)dbk::workspace(nslice * m * sizeof(T), st);
     if (!partial) { dbk::set_error("MemoryError: could not allocate %zu bytes of scratch (%s)", nslice * m * sizeof(T), dbk::workspace_error()); return 1; }
     hipLaunchKernelGGL(k_colsum<T>, dim3(tiles, (unsigned)nslice), dim3(256), 0, st, X, partial, n, m, rows_per);
-    hipLaunchKernelGGL(k_colsum_fold<T>, dim3(dbk::ew_grid(m)), dim3(256), 0, st, (const T*)partial, out, m, (unsigned)nslice);
+    hipLaunchKernelGGL(k_colsum_fold<T>, dim3(dbk::divup(m, 64)), dim3(1024), 0, st, (const T*)partial, out, m, (unsigned)nslice, rep, tail, ntail);
     return 0;
 }
 

@@ -1309,3 +1309,31 @@ def test_poolrgn_packed_and_plain_columns_agree(ks, F):
         ks.poolrgn_bprop(dUa, Rd, dP, Ia if want else None, ptype)
         ks.poolrgn_bprop(dUb, Rd, dP, Ib if want else None, ptype)
         assert torch.equal(dUa, dUb), ptype
+
+
+@pytest.mark.parametrize("n,m,dtype", [(4096, 1, np.float32), (4099, 2, np.float64), (70003, 16, np.float32), (5001, 32, np.float64)])
+def test_column_sums_of_few_columns(sm, n, m, dtype):
+    """Several rows side by side in the 64 lanes, with and without rows left over."""
+    test_column_sums(sm, n, m, dtype)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("P,F,step", [(37, 16, False), (501, 8, True), (9001, 16, False), (2, 64, True)])
+def test_poolrgn_max_in_runs(ks, P, F, step, dtype):
+    """Maximum pooling with 16 and with 4 lanes per region and pack against the one-column kernel (the same map off a 16-byte boundary):
+    regions of one row and of fewer rows than lanes, ties, row steps, rows that are NaN or minus infinity."""
+    rng = np.random.default_rng(P + F)
+    lens = rng.integers(1, 50, size=P)
+    starts = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    R = np.stack([starts, starts + lens] + ([rng.integers(1, 4, size=P)] if step else []), 1).astype(np.uint32)
+    U = rng.standard_normal((int(lens.sum()), F)).astype(dtype)
+    U[rng.random(U.shape) < 0.3] = 0.5
+    U[rng.random(U.shape) < 0.05] = np.nan
+    U[rng.random(U.shape) < 0.2] = -np.inf
+    Ud = dev(U)
+    base = torch.empty(U.size + 1, dtype=Ud.dtype, device="cuda")
+    Uoff = base[1:].reshape(U.shape)
+    Uoff.copy_(Ud)
+    Pa, Ia = ks.poolrgn(Ud, dev(R), "max", want_argmax=True)
+    Pb, Ib = ks.poolrgn(Uoff, dev(R), "max", want_argmax=True)
+    assert np.array_equal(host(Pa), host(Pb), equal_nan=True) and np.array_equal(host(Ia), host(Ib))
