@@ -95,6 +95,8 @@ _SIGNATURES = {
     "dbk_predict_small": [_P, _P, _P, _Z, _Z, _Z, _P, _Z, _P, _Z, _I, _Z, _P, _P, _P, _P, _P, _I, _P],
     "dbk_mutation_map_takes": [_Z, _Z, _I, _Z],
     "dbk_mutation_map": [_P, _P, _P, _Z, _Z, _P, _Z, _P, _Z, _Z, _I, _Z, _P, _P, _P, _P, _P, _I, _I, _P, _P],
+    "dbk_gradient_map_takes": [_Z, _Z, _Z, _Z, _I, _Z],
+    "dbk_gradient_map": [_P, _P, _P, _Z, _Z, _P, _P, _Z, _Z, _Z, _I, _Z, _P, _P, _P, _P, _P, _I, _I, _P, _P, _P],
     "dbk_gather_maps": [_P, _I, _P, _Z, _Z, _I, _P, _P, _P],
     "dbk_train_step": [_P, _P],
     "dbk_train_steps": [_P, _Z, _P],

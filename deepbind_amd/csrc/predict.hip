@@ -415,6 +415,193 @@ __global__ __launch_bounds__(NT) void k_predict_small(const small_args a)
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// gradient maps
+// ---------------------------------------------------------------------------------------------
+// One workgroup per sequence takes it from its letters to the map: both strands scanned (as k_predict_small does, keeping each
+// filter's first largest row and, where a mean is pooled, a bit per row and filter that says the rectifier let it through) and
+// put through the head; then the winning strand's score goes back through the head, the pooling and the filters. A letter's
+// windows are rows of its own sequence, so nothing leaves the workgroup, no feature map is written, and the strand that lost is not
+// taken back at all. Layer by layer the same took 23 launches over three maps of rows x filters.
+// What bounds it is latency with the maximum, LDS reads with the mean (16 bytes per letter, base, tap and four filters). Measured: 1000 sequences of 101
+// letters, both strands, 16 filters of 24 taps: 26 us a launch (layer by layer 170 us of kernels,
+// 210 until the last of them ended), the call from strings to host arrays 0.90 -> 0.55 ms.
+constexpr unsigned GRAD_MAXROWS = 2048;                             // rows of a region: their bits are 2 x 2 bytes of LDS each
+
+struct grad_args {
+    const float *W, *bias, *W1, *b1, *W2, *b2, *in_scale;
+    const uint8_t* text;
+    const uint32_t* offsets;
+    unsigned m, F, k, hidden, rows_max;
+    int ptype, logistic, strands;
+    float *Z, *map;
+    uint8_t* letters;
+};
+
+__host__ __device__ inline unsigned grad_letters(unsigned rows_max, unsigned m) { return (rows_max + m + 3 + 3 + 3) & ~3u; }
+inline size_t grad_smem(size_t m, unsigned rows_max)
+{
+    return ((size_t)m * (NL + 4) * MUT_F + 3 * 16 * MUT_F + 2 * 2 * MUT_F + 2 * 64 + 2 * 2 * MUT_F + 2 * MUT_F + 4) * sizeof(float) +
+           2 * ((rows_max + 1) & ~1u) * sizeof(uint16_t) + grad_letters(rows_max, (unsigned)m);
+}
+
+__global__ __launch_bounds__(256) void k_gradient_map(const grad_args a)
+{
+    extern __shared__ __align__(16) float msm[];
+    const unsigned m = a.m, pad = m - 1, tid = threadIdx.x, lane = tid & 63;
+    const unsigned f = tid & 15u, rl = tid >> 4;
+    const size_t s = blockIdx.x;
+    const unsigned base = a.offsets[s], len = a.offsets[s + 1] - base, rows = pad + len;
+    float* lut = msm;                                               // [tap][letter][16]
+    float* wt = lut + m * NL * MUT_F;                               // [tap][base][16], times the mean's gradient
+    float* fold = wt + m * 4 * MUT_F;                               // largest value [16][16], sum [16][16], its row [16][16]
+    unsigned* frow = reinterpret_cast<unsigned*>(fold + 2 * 16 * MUT_F);
+    float* x = fold + 3 * 16 * MUT_F;                               // pooled features of either strand [2][32]
+    float* hid = x + 2 * 2 * MUT_F;                                 // hidden units [2][64]
+    unsigned* arg = reinterpret_cast<unsigned*>(hid + 2 * 64);      // row of the maximum [2][16]
+    float* dmax = reinterpret_cast<float*>(arg + 2 * MUT_F);        // gradients of the pooled values [16], [16]
+    float* davg = dmax + MUT_F;
+    float* zs = davg + 3 * MUT_F;                                   // scores [2]
+    uint16_t* bits = reinterpret_cast<uint16_t*>(zs + 4);           // [2][rows]
+    const unsigned nbits = (a.rows_max + 1) & ~1u;
+    uint8_t* tile = reinterpret_cast<uint8_t*>(bits + 2 * nbits);
+    const bool mean = a.ptype != DBK_PT_MAX;
+    const float bf = f < a.F ? a.bias[f] : 0.0f, sc = a.in_scale ? a.in_scale[0] : 1.0f;
+    letter_table16(lut, a.W, m, a.F, 0, a.F, 256);
+    for (int st = 0; st < a.strands; ++st) {
+        __syncthreads();                                            // the other strand's letters are no longer read
+        for (unsigned e = tid; e < rows + m + 3; e += 256) {
+            const unsigned i = e - pad;                             // (wraps for the pad before the letters)
+            tile[e] = (uint8_t)((i < len ? letter_of(strand_code(a.text[base + (st ? len - 1 - i : i)], st != 0)) : 4u) * MUT_F);
+        }
+        __syncthreads();
+        float mx = -1.0f, sum = 0.0f;
+        unsigned at = ~0u;
+        for (unsigned p = 4 * rl; p < rows; p += 64) {
+            float z[4];
+            scan4(lut + f, tile, p, m, ~0u, 0u, z);
+#pragma unroll
+            for (unsigned u = 0; u < 4; ++u) {
+                float v = z[u] + bf;
+                v = v > 0.0f && p + u < rows ? v : 0.0f;
+                if (v > mx && p + u < rows) { mx = v; at = p + u; }
+                sum += v;
+                if (mean) {
+                    const unsigned on = (unsigned)(__ballot(v > 0.0f) >> (lane & 48u));
+                    if (f == 0 && p + u < rows) bits[st * nbits + p + u] = (uint16_t)on;
+                }
+            }
+        }
+        fold[rl * MUT_F + f] = mx;
+        fold[(16 + rl) * MUT_F + f] = sum;
+        frow[rl * MUT_F + f] = at;
+        __syncthreads();
+        if (tid < 64) {
+            if (tid < a.F) {
+                mx = -1.0f; sum = 0.0f; at = ~0u;
+#pragma unroll
+                for (unsigned t = 0; t < 16; ++t) {
+                    const float v = fold[t * MUT_F + tid];
+                    const unsigned r = frow[t * MUT_F + tid];
+                    if (v > mx || (v == mx && r < at)) { mx = v; at = r; }       // the first of equal rows
+                    sum += fold[(16 + t) * MUT_F + tid];
+                }
+                const float avg = sum / (float)rows;
+                if (a.ptype == DBK_PT_ALL) { x[st * 2 * MUT_F + 2 * tid] = mx; x[st * 2 * MUT_F + 2 * tid + 1] = avg; }
+                else x[st * 2 * MUT_F + tid] = a.ptype == DBK_PT_MAX ? mx : avg;
+                arg[st * MUT_F + tid] = mx > 0.0f ? at : ~0u;        // (a maximum of nothing has no gradient)
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const float* xs = x + st * 2 * MUT_F;
+            float out = 0.0f;
+            if (a.hidden > 0) {
+                if (lane < a.hidden) {
+                    float z = 0.0f;
+#pragma unroll 8
+                    for (unsigned kk = 0; kk < a.k; ++kk) z = __builtin_fmaf(xs[kk] * sc, a.W1[(size_t)kk * a.hidden + lane], z);
+                    z += a.b1[lane];
+                    z = z > 0.0f ? z : 0.0f;
+                    hid[st * 64 + lane] = z;
+                    out = z * a.W2[lane];
+                }
+            } else if (lane < a.k) out = xs[lane] * sc * a.W1[lane];
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) out += __shfl_xor(out, d, 64);
+            out += a.hidden > 0 ? a.b2[0] : a.b1[0];
+            if (a.logistic) out = 1.0f / (1.0f + expf(-out));
+            if (lane == 0) zs[st] = out;
+        }
+    }
+    __syncthreads();
+    // ---- the strand that predicts more (the forward one wins ties), and its score's way back: eight lanes per pooled value
+    const unsigned win = a.strands == 2 && zs[0] < zs[1] ? 1u : 0u;
+    float dz = zs[win];
+    if (a.strands == 2 && !(zs[0] >= zs[1]) && win == 0) dz = 0.0f;  // (scores that do not compare pick neither row of the pair)
+    {
+        const unsigned kk = tid >> 3, h8 = tid & 7u;
+        float d = 0.0f;
+        if (kk < a.k) {
+            if (a.hidden > 0) {
+                for (unsigned h = h8; h < a.hidden; h += 8)
+                    d += (hid[win * 64 + h] > 0.0f ? dz * a.W2[h] : 0.0f) * a.W1[(size_t)kk * a.hidden + h];
+            } else if (h8 == 0) d = dz * a.W1[kk];
+        }
+#pragma unroll
+        for (int w = 4; w >= 1; w >>= 1) d += __shfl_xor(d, w, 8);
+        if (h8 == 0) {
+            d *= sc;
+            if (a.ptype == DBK_PT_ALL) {
+                if (kk & 1u) davg[kk >> 1] = kk < a.k ? d / (float)rows : 0.0f;
+                else dmax[kk >> 1] = kk < a.k ? d : 0.0f;
+            } else if (kk < MUT_F) {
+                if (a.ptype == DBK_PT_MAX) dmax[kk] = kk < a.k ? d : 0.0f;
+                else davg[kk] = kk < a.k ? d / (float)rows : 0.0f;
+            }
+        }
+    }
+    __syncthreads();
+    if (mean) {
+        for (unsigned e = tid; e < m * 4 * MUT_F; e += 256) {
+            const unsigned j = e / (4 * MUT_F), c = e / MUT_F % 4;
+            wt[e] = davg[e % MUT_F] * lut[(j * NL + c) * MUT_F + e % MUT_F];
+        }
+        __syncthreads();
+    }
+    for (unsigned e = tid; e < 4 * len; e += 256) {
+        const unsigned q = pad + (e >> 2), c = e & 3u;               // the letter's place among the region's rows
+        float g = 0.0f;
+        if (mean) {
+            const uint16_t* on = bits + win * nbits + q;
+#pragma unroll 2
+            for (unsigned j = 0; j < m; ++j) {
+                const unsigned b = on[-(int)j];
+                const float4* w = reinterpret_cast<const float4*>(wt + (j * 4 + c) * MUT_F);
+#pragma unroll
+                for (unsigned t = 0; t < 4; ++t) {
+                    const float4 v = w[t];
+                    g += b & (1u << (4 * t)) ? v.x : 0.0f;
+                    g += b & (2u << (4 * t)) ? v.y : 0.0f;
+                    g += b & (4u << (4 * t)) ? v.z : 0.0f;
+                    g += b & (8u << (4 * t)) ? v.w : 0.0f;
+                }
+            }
+        }
+        if (a.ptype != DBK_PT_AVG)
+            for (unsigned t = 0; t < a.F; ++t) {
+                const unsigned j = q - arg[win * MUT_F + t];         // (wraps past m where the maximum is another window's)
+                if (j < m) g += dmax[t] * lut[(j * NL + c) * MUT_F + t];
+            }
+        a.map[4 * (size_t)base + e] = g;
+    }
+    for (unsigned i = tid; i < len; i += 256) {
+        const unsigned c = strand_code(a.text[base + (win ? len - 1 - i : i)], win != 0);
+        a.letters[(size_t)base + i] = (uint8_t)(c == 0 ? 'A' : c == 1 ? 'C' : c == 2 ? 'G' : c == 3 ? 'T' : 'N');
+    }
+    if (tid == 0) a.Z[s] = zs[win];
+}
+
 // The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
 // is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. One workgroup per sequence.
 __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const float* __restrict__ S,
@@ -545,6 +732,34 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(256), mut_smem(pos, m, a.k), st, a);
     hipLaunchKernelGGL(k_mutation_map, dim3((unsigned)(nregion / strands)), dim3(256), 0, st, regions, (unsigned)(m - 1), strands,
                        (const float*)a.S, (const float*)a.base, Z, map);
+    DBK_LAUNCH_OK();
+}
+
+int dbk_gradient_map_takes(size_t m, size_t nfilter, size_t shortest, size_t longest, int ptype, size_t hidden)
+{
+    // One workgroup per sequence: a long one would keep it busy where the layer-by-layer kernels fill the chip. (An empty region
+    // - no letters and filters of one tap - has no rows of its own: the layers say what it gives.)
+    return m >= 1 && m <= 64 && nfilter >= 1 && nfilter <= MUT_F && hidden <= 64 && shortest + m > 1 && longest + m - 1 <= GRAD_MAXROWS &&
+           (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL) && grad_smem(m, (unsigned)(longest + m - 1)) <= 65536;
+}
+
+int dbk_gradient_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* text, const uint32_t* offsets,
+                     size_t nseq, size_t shortest, size_t longest, int ptype, size_t hidden, const float* W1, const float* b1, const float* W2,
+                     const float* b2, const float* in_scale, int apply_logistic, int strands, float* Z, float* map, uint8_t* letters)
+{
+    DBK_CHECK(strands == 1 || strands == 2, "ValueError: strands must be 1 or 2");
+    DBK_CHECK(dbk_gradient_map_takes(m, nfilter, shortest, longest, ptype, hidden), "NotImplementedError: the gradient map kernel does not take %zu filters of "
+              "%zu taps with %zu hidden units, pooling %d and sequences of %zu to %zu letters", nfilter, m, hidden, ptype, shortest, longest);
+    if (nseq == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(nseq <= 0x7fffffffu, "ValueError: too many sequences (%zu) for one launch", nseq);
+    DBK_CHECK(W && bias && offsets && W1 && b1 && Z && (longest == 0 || (text && map && letters)), "ValueError: null pointer argument");
+    DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
+    grad_args a;
+    a.W = W; a.bias = bias; a.W1 = W1; a.b1 = b1; a.W2 = W2; a.b2 = b2; a.in_scale = in_scale; a.text = text; a.offsets = offsets;
+    a.m = (unsigned)m; a.F = (unsigned)nfilter; a.k = (unsigned)(nfilter * (ptype == DBK_PT_ALL ? 2 : 1)); a.hidden = (unsigned)hidden;
+    a.rows_max = (unsigned)(longest + m - 1); a.ptype = ptype; a.logistic = apply_logistic; a.strands = strands;
+    a.Z = Z; a.map = map; a.letters = letters;
+    hipLaunchKernelGGL(k_gradient_map, dim3((unsigned)nseq), dim3(256), grad_smem(m, a.rows_max), dbk::as_stream(stream), a);
     DBK_LAUNCH_OK();
 }
 

@@ -123,6 +123,26 @@ def _mutation_maps(net, X, R, text):
     return out[:n].reshape(-1, 1), out[n:].reshape(-1, 4)
 
 
+def _gradient_maps(net, text):
+    """(Z (nseq, 1), map (letters, 4), the letters of the strands mapped) of the batch, or None when the kernel does not take it."""
+    ptype, shortest, longest = _lib.str2pooltype[net.pool], int(text.lens.min()), int(text.lens.max())
+    if net.dtype != torch.float32 or net.input_dropout > 0 or not _lib.dll().dbk_gradient_map_takes(net.m, net.nfilter, shortest, longest, ptype, net.hidden):
+        return None
+    p, n, L = net.p, len(text.lens), len(text.bytes)
+    offsets, letters = text.upload(net.device)
+    out = torch.empty(4 * n + 17 * L, dtype=torch.uint8, device=net.device)                  # (one copy back to the host)
+    Z, maps, strand = out[:4 * n], out[4 * n:4 * n + 16 * L], out[4 * n + 16 * L:]
+    _lib.call("dbk_gradient_map", _lib.stream(), _lib.ptr(p["Wc"]), _lib.ptr(p["bc"]), net.m, net.nfilter, _lib.ptr(letters), _lib.ptr(offsets), n,
+              shortest, longest, ptype, net.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")), _lib.ptr(p.get("b2")),
+              _lib.ptr((1.0 - net.dropout) if net.use_dropout else None), int(net.loss == "nll"), 2 if net.reverse_complement else 1,
+              _lib.ptr(Z), _lib.ptr(maps), _lib.ptr(strand))
+    out = out.cpu().numpy()
+    Z = out[:4 * n].view(np.float32).reshape(-1, 1)
+    if net.reverse_complement:
+        Z = Z[Z[:, 0] == Z[:, 0]]                    # (scores that do not compare select neither row of their pair)
+    return Z, out[4 * n:4 * n + 16 * L].view(np.float32).reshape(-1, 4), out[4 * n + 16 * L:].tobytes().decode("ascii")
+
+
 def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     """Scores a list of sequence strings with a single-model SequenceNet.
 
@@ -136,6 +156,11 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     preds, gmaps = [], ([] if want_gmaps else None)
     for s0 in range(0, len(seqs), batchsize):
         text = _Text(seqs[s0:s0 + batchsize])
+        fused = _gradient_maps(net, text) if want_gmaps and want_gmaps != "finite_diff" else None
+        if fused is not None:
+            preds.append(fused[0])
+            gmaps += zip(_split(fused[2], text), _split(fused[1], text))
+            continue
         X, R = _pack(net, text)
         if not want_gmaps:
             preds.append(net.predict(X, R).cpu().numpy())

@@ -445,6 +445,15 @@ int dbk_mutation_map_takes(size_t m, size_t nfilter, int ptype, size_t hidden);
 int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* X, size_t N,
                      const uint32_t* regions, size_t nregion, size_t longest, int ptype, size_t hidden, const float* W1, const float* b1,
                      const float* W2, const float* b2, const float* in_scale, int apply_logistic, int strands, float* Z, float* map);
+/* Scores and gradient maps of one model, from the sequences' text (as dbk_pack_text takes it): Z (nseq) the net's outputs (with strands = 2
+ * the larger of each pair's, the forward row on ties), map (letters of all sequences, 4) the back-propagated gradient of
+ * that output's half square at every letter of that strand, letters the strand's text in ACGTN. shortest, longest: the
+ * sequences' fewest and most letters. Weights as in dbk_head_fprop with nblock = 1 and no feature columns.
+ * dbk_gradient_map_takes: 1 for shapes the kernel takes. reference: kangaroo/kangaroo/predict.py:168-199. */
+int dbk_gradient_map_takes(size_t m, size_t nfilter, size_t shortest, size_t longest, int ptype, size_t hidden);
+int dbk_gradient_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* text, const uint32_t* offsets,
+                     size_t nseq, size_t shortest, size_t longest, int ptype, size_t hidden, const float* W1, const float* b1, const float* W2,
+                     const float* b2, const float* in_scale, int apply_logistic, int strands, float* Z, float* map, uint8_t* letters);
 /* map (letters of all sequences, 4): the rows of dX (N, 4) at every sequence's letters, with strands = 2 those of the row of
  * the pair whose prediction Z (nregion) is larger. reference: kangaroo/kangaroo/predict.py:188-199. */
 int dbk_gather_maps(dbk_stream_t stream, int dtype, const uint32_t* regions, size_t nregion, size_t padding, int strands, const void* Z,

@@ -170,3 +170,39 @@ def test_single_launch_scores(pool, hidden, loss, rc, m, F, nm, lo, hi):
     if rc:
         want = want.reshape(-1, 2, nm).max(axis=1)
     assert_close(got, want, ACT, "scores")
+
+
+@pytest.mark.parametrize("pool,hidden,loss,rc,rate,m,F", [("max", 64, "nll", True, 0.5, 24, 16), ("all", 33, "mse", True, 0.0, 32, 16), ("avg", 0, "mse", False, 0.25, 9, 5),
+                                                          ("all", 0, "nll", False, 0.0, 2, 1), ("max", 1, "mse", False, 0.0, 64, 13), ("avg", 8, "nll", True, 0.0, 13, 12)])
+def test_gradient_map_kernel_edges(pool, hidden, loss, rc, rate, m, F):
+    """Regions around 64 rows (a pass of the workgroup) and up to the kernel's 2048, one letter, none, all N (every row of a strand is as large), a
+    palindrome (the pair ties); against the oracle and, longest region apart, the layers in place of the kernel: maps differ from
+    those by round-off of sums of up to 2 m F terms."""
+    from deepbind_amd import _lib, predict
+    rng = np.random.default_rng(11 * m + F)
+    p = _params(rng, m, F, pool, hidden)
+    seqs = ["".join("ACGT"[v] for v in rng.integers(0, 4, n)) for n in (1, max(1, 65 - m), max(1, 66 - m), 130, 2049 - m)] + ["", "N" * 40, "ACGTUACGT"[:4] * 9]
+    seqs[3] = "n" + seqs[3][1:].lower().replace("t", "u")
+    out = "logistic" if loss == "nll" else "linear"
+    net = _net(p, m, F, pool, hidden, loss, rc, rate)
+    ptype = _lib.str2pooltype[pool]
+    takes = _lib.dll().dbk_gradient_map_takes
+    assert takes(m, F, 0, 2049 - m, ptype, hidden) == 1 and takes(m, F, 0, 2050 - m, ptype, hidden) == 0 and takes(1, F, 0, 9, ptype, hidden) == 0
+    assert takes(m, 17, 0, 9, ptype, hidden) == 0 and takes(m, F, 0, 9, ptype, 65) == 0 and takes(65, F, 0, 9, ptype, hidden) == 0
+    Z, maps = predict.gen_predictions(net, seqs, want_gmaps=True)
+    Zr, mr = orc.gen_predictions({k: v.astype(np.float64) for k, v in p.items()}, seqs, pool, hidden, out, dropout_rate=[rate] if rate else None,
+                                 reverse_complement=rc, want_gmaps=True)
+    assert_close(Z, Zr, ACT, "Z")
+    scale = max(np.abs(b).max() for _, b in mr if len(b))
+    for (sa, a), (sb, b) in zip(maps, mr):
+        assert sa == sb and a.shape == b.shape
+        assert len(b) == 0 or np.abs(a - b).max() <= GRAD * scale, (len(sa), np.abs(a - b).max(), scale)
+    fused = predict._gradient_maps
+    predict._gradient_maps = lambda net, text: None
+    try:
+        Zl, ml = predict.gen_predictions(net, seqs, want_gmaps=True)
+    finally:
+        predict._gradient_maps = fused
+    assert_close(Z, Zl, ACT, "Z, layer by layer")
+    for (sa, a), (sb, b) in zip(maps, ml):
+        assert sa == sb and (len(b) == 0 or np.abs(a - b).max() <= GRAD * scale)
