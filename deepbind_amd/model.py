@@ -239,11 +239,11 @@ class SequenceNet(object):
                 raise _lib.DeepbindError("RuntimeError: a single-launch training step was abandoned (%s); %d step(s) were not applied" %
                                          ("a workgroup waited too long" if status == 1 else "a region has more than 256 rows", dropped))
 
-    def _count_single_launch(self, buf):
-        """Book-keeping after a single-launch step was issued on the workspace in `buf` (or a graph holding one
+    def _count_single_launch(self, work):
+        """Book-keeping after a single-launch step was issued on the workspace `work` (or a graph holding one
         replayed): the status word is looked at every 256 launches, so that an abandoned step does not go unnoticed."""
         for entry in self._works:
-            if entry[0] is buf["work"]:
+            if entry[0] is work:
                 entry[1] += 1
         self._single_calls += 1
         if self._single_calls % 256 == 0:
@@ -664,7 +664,7 @@ class SequenceNet(object):
         self._last_single = work is not None
         self._finish_step(X, R)
         if work is not None and not torch.cuda.is_current_stream_capturing():
-            self._count_single_launch(buf)   # (may raise: a step that was abandoned must not be trained over in silence)
+            self._count_single_launch(work)  # (may raise: a step that was abandoned must not be trained over in silence)
         self.enforce_constraints()
         return buf["Z"]
 
@@ -798,7 +798,7 @@ def _graphed_step(jobs):
             net._L_versions = None              # (the warm-up step's look-ahead belongs to parameters that were put back)
         state["graphs"], state["decay"] = graphs, decay_flags()
         state["buffers"] = [(net._step_buf, net._L) for net, *_ in jobs]                      # (the graph's nodes point into them)
-        state["single"] = [(net, net._step_buf) for net, *_ in jobs if net._last_single]      # workspaces of single-launch steps in the graph
+        state["single"] = [(net, net._step_buf["work"]) for net, *_ in jobs if net._last_single]      # workspaces of single-launch steps in the graph
 
     def step():
         if state["graphs"] is None or state["decay"] != decay_flags():
@@ -813,8 +813,8 @@ def _graphed_step(jobs):
             if net.use_dropout:
                 net._rng_offset += (R.shape[0] * net.k * net.ninst + 3) // 4
             net.step_count += 1
-        for net, buf in state["single"]:
-            net._count_single_launch(buf)
+        for net, work in state["single"]:
+            net._count_single_launch(work)
 
     return step
 

@@ -306,3 +306,24 @@ def test_minibatches_of_changing_shape_share_buffers_and_workspace(nm, rc, pool)
     for name in a:
         assert np.array_equal(a[name], b[name]), name
     assert np.array_equal(host(net.mP), host(own.mP)) and int(net.rng_counter.item()) == int(own.rng_counter.item())
+
+
+def test_graphed_step_outlives_a_larger_workspace():
+    """A graph whose step is one launch keeps being replayed after an eager step on a larger minibatch has made the net a larger
+    workspace: the replays give the bits of eager steps."""
+    rng = np.random.default_rng(33)
+    batches = []
+    for rows in (6, 300):
+        X, R = _batch(rng, rows, 11, 20, 60)
+        batches.append((dev(X), dev(R), dev(rng.random((len(R), 2)).astype(np.float32))))
+    net, ref = [_net(np.random.default_rng(34), 2, 16, 11, "max", 8, "mse", rate=0.05, momentum=0.9, dropout=0.5)[0] for _ in range(2)]
+    step = net.make_graphed_step(*batches[0], force_graph=True)
+    for i in range(3):
+        step()
+        net.train_step(*batches[1])
+        ref.train_step(*batches[0])
+        ref.train_step(*batches[1])
+        a, b = net.get_params(), ref.get_params()
+        for name in a:
+            assert np.array_equal(a[name], b[name]), (i, name)
+    assert len(net._works) == 2 and net.step_count == ref.step_count == 6
