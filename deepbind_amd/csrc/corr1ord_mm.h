@@ -43,6 +43,8 @@ template <> struct mm16<float> {
 // a call with the reduction: float64, 123 000 rows x 64 filters of 24 taps 55 (the kernel with per-wave tables in LDS, one read-modify-
 // write per row and tap: 876); float32, 250 000 x 16 filters of 24 taps 45 (one register add per row and tap: 68), 60 000 x 16 of 32 taps 21
 // (tables in LDS: 497).
+// A product with a zero of the one-hot operand is no zero where dZ is infinite or not a number: a wave that has met such a value adds
+// its rows again one by one, each to the rows of dW its letters name and to no other.
 constexpr unsigned CW_CHUNK = 256;                                  // rows whose letters a wave stages at a time
 template <int TT> struct cw_lds { static constexpr unsigned letters = CW_CHUNK + 4 * TT + 4; };
 
@@ -63,12 +65,14 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_W_mm_kernel(T* __restrict_
 #pragma unroll
     for (int t = 0; t < TT; ++t) acc[t] = (acc_t)(T)0;
     const T* src = dZ + (f < F ? f : F - 1);
+    bool odd = false;
     auto fetch = [&](size_t p, T (&b)[8]) {                         // rows p + k, p + 4 + k, ..: eight steps
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const size_t row = p + 4u * u + k;
             const T v = src[(row < n ? row : n - 1) * F];
             b[u] = row < r1 && f < F ? v : (T)0;
+            odd |= !__builtin_isfinite(b[u]);
         }
     };
     T b[8], bn[8];
@@ -109,10 +113,24 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_W_mm_kernel(T* __restrict_
     }
     __syncthreads();                                                // (the letters are no longer read)
     T* tiles = reinterpret_cast<T*>(smem);                          // [wave][TT][16][16]
+    if (__ballot(odd) == 0) {
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+        for (int t = 0; t < TT; ++t)
 #pragma unroll
-        for (unsigned i = 0; i < 4; ++i) tiles[((wave * TT + t) * 16 + mm16<T>::row(i, k)) * 16 + col] = acc[t][i];
+            for (unsigned i = 0; i < 4; ++i) tiles[((wave * TT + t) * 16 + mm16<T>::row(i, k)) * 16 + col] = acc[t][i];
+    } else {
+        T* mine = tiles + wave * TT * 256u + col;                   // row 4 j + l of dW, this lane's filter; taps k, k + 4, .. are this lane's
+        for (unsigned j = k; j < 4u * TT; j += 4)
+            for (unsigned l = 0; l < 4; ++l) mine[(4 * j + l) * 16] = (T)0;
+        for (size_t p = r0; p < r1 && f < F; ++p) {
+            const T v = dZ[p * F + f];
+            for (unsigned j = k; j < m; j += 4) {
+                const unsigned letter = letter_of(X[p + j]);
+                for (unsigned l = 0; l < 4; ++l)
+                    if (letter == l || letter == 4u) mine[(4 * j + l) * 16] += letter == 4u ? v * (T)0.25 : v;
+            }
+        }
+    }
     __syncthreads();
     T* out = partial + (size_t)blockIdx.y * 4 * m * F;
     for (unsigned e = threadIdx.x; e < TT * 256u; e += 256u) {
@@ -155,6 +173,7 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_mm_kernel(T* __restrict_
     const unsigned w0 = NB == 4 ? 64u * wave : 0u, d0 = NB == 4 ? 0u : wave;
     constexpr unsigned DSTEP = NB == 4 ? 1u : 4u;
     const size_t q0 = (size_t)blockIdx.x * (64 * NB);
+    bool odd = false;
     acc_t acc = (acc_t)(T)0;
     const T* za = zs + (w0 + 4u * col) * CX_ST + k;                 // A: row 4 r + d of the wave's rows, r = col; d counted from -(m - 1)
     const T* wb = ws + ((m - 1 + 3) * 4u + col) * CX_ST + k;        // B: (s, c) = col at d = -(m - 1): tap s + m - 1
@@ -163,11 +182,15 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_mm_kernel(T* __restrict_
         for (unsigned e = tid; e < (64 * NB + m - 1) * 16; e += 256) {
             const unsigned r = e >> 4, fl = f0 + (e & 15u);
             const size_t row = q0 + r;                              // + (m - 1): offset by the rows before the workgroup's
-            zs[r * CX_ST + (e & 15u)] = row >= m - 1 && row - (m - 1) < n && fl < F ? dZ[(row - (m - 1)) * F + fl] : (T)0;
+            const T v = row >= m - 1 && row - (m - 1) < n && fl < F ? dZ[(row - (m - 1)) * F + fl] : (T)0;
+            zs[r * CX_ST + (e & 15u)] = v;
+            odd |= !__builtin_isfinite(v);
         }
         for (unsigned e = tid; e < (m + 6) * 4 * 16; e += 256) {
             const unsigned r = e >> 4, fl = f0 + (e & 15u);
-            ws[r * CX_ST + (e & 15u)] = r >= 12 && r - 12 < 4 * m && fl < F ? W[(size_t)(r - 12) * F + fl] : (T)0;
+            const T v = r >= 12 && r - 12 < 4 * m && fl < F ? W[(size_t)(r - 12) * F + fl] : (T)0;
+            ws[r * CX_ST + (e & 15u)] = v;
+            odd |= !__builtin_isfinite(v);
         }
         __syncthreads();
 #pragma unroll 4
@@ -176,8 +199,20 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_mm_kernel(T* __restrict_
             for (unsigned s = 0; s < 4; ++s) acc = mm16<T>::mul(za[d * CX_ST + 4 * s], wb[-(int)(d * 4 * CX_ST) + (int)(4 * s)], acc);
         }
     }
+    // (a zero beside an infinite value or one that is not a number is no zero of the sum: such rows are added without it)
+    if (__syncthreads_or(odd)) {
+        for (unsigned e = tid; e < 64 * NB * 4; e += 256) {
+            const size_t q = q0 + (e >> 2);
+            if (q >= n) break;
+            const T* w = W + (size_t)(e & 3u) * F;
+            T sum = (T)0;
+            for (unsigned j = 0; j < m && j <= q; ++j)
+                for (unsigned f = 0; f < F; ++f) sum += dZ[(q - j) * F + f] * w[(size_t)4 * j * F + f];
+            dX[q * 4 + (e & 3u)] += sum;
+        }
+        return;
+    }
     if (NB == 1) {
-        __syncthreads();
         acc_t* parts = reinterpret_cast<acc_t*>(smem);              // [wave][lane]: less than the staged rows
         parts[tid] = acc;
         __syncthreads();

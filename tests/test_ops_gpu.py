@@ -211,6 +211,28 @@ def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype)
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,m,F", [(300, 8, 5), (131329, 9, 3), (700, 32, 20)])
+def test_corr1ord_gradients_of_infinite_values(ks, n, m, F, dtype):
+    """A gradient that is infinite or not a number reaches the letters of its own windows and nothing else, infinite weights the rows
+    their taps reach: no product with a zero operand shows."""
+    rng = np.random.default_rng(n + m)
+    X = random_codes(rng, n + m - 1, 0.05, 0.05).reshape(-1, 1)
+    dZ = np.zeros((n + m - 1, F), dtype); dZ[:n] = rng.standard_normal((n, F))
+    W = (rng.standard_normal((4 * m, F)) * 0.1).astype(dtype)
+    dZ[n // 2, 1], dZ[n - 2, 2], W[4 * (m - 1) + 1, 0] = np.inf, np.nan, -np.inf
+    with np.errstate(invalid="ignore"):
+        ref = np.ones((4 * m, F)); orc.corr1ord_bprop_W(ref, X, dZ.astype(np.float64))
+        refx = np.ones((n + m - 1, 4)); orc.corr1ord_bprop_X(refx, W.astype(np.float64), dZ.astype(np.float64))
+    dW, dX = dev(np.ones((4 * m, F), dtype)), dev(np.ones((n + m - 1, 4), dtype))
+    ks.corr1ord_bprop_W(dW, dev(X), dev(dZ), 4)
+    ks.corr1ord_bprop_X(dX, dev(W), dev(dZ), 4)
+    for got, want, name in ((host(dW), ref, "dW"), (host(dX), refx, "dX")):
+        odd = ~np.isfinite(want)
+        assert np.array_equal(odd, ~np.isfinite(got)) and np.array_equal(want[odd], got[odd].astype(np.float64), equal_nan=True), name
+        assert_close(np.where(odd, 0, got), np.where(odd, 0, want), GRAD if dtype == np.float32 else 1e-12, name)
+
+
 # ------------------------------------------------------------------------------------------ pooling
 def _regions(rng, P, lo, hi, gap=0):
     lens = rng.integers(lo, hi + 1, size=P)
