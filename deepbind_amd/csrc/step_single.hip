@@ -874,8 +874,8 @@ __global__ __launch_bounds__(256) void k_longest_region(const uint32_t* __restri
     __shared__ unsigned part[4];
     unsigned rows = 0;
     for (unsigned r = threadIdx.x; r < P; r += 256) {
-        const uint2 ab = reinterpret_cast<const uint2*>(R)[r];
-        rows = max(rows, ab.y > ab.x ? ab.y - ab.x : 0u);
+        const uint32_t a = R[2 * (size_t)r], b = R[2 * (size_t)r + 1];
+        rows = max(rows, b > a ? b - a : 0u);
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) rows = max(rows, (unsigned)__shfl_xor((int)rows, d, 64));
@@ -893,7 +893,7 @@ extern "C" int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, 
     DBK_CHECK(rows, "ValueError: null pointer argument");
     *rows = 0;
     if (nregion == 0) { dbk::clear_error(); return 0; }
-    DBK_CHECK(regions && ((uintptr_t)regions & 7) == 0 && nregion < ((size_t)1 << 31), "ValueError: regions must be an 8-byte aligned table of fewer than 2^31 rows");
+    DBK_CHECK(regions && nregion < ((size_t)1 << 31), "ValueError: regions must be a table of fewer than 2^31 rows");
     hipStream_t st = dbk::as_stream(stream);
     unsigned* word = (unsigned*)dbk::workspace(sizeof(unsigned), st);
     DBK_CHECK(word != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
