@@ -599,7 +599,7 @@ __global__ __launch_bounds__(256) void k_gradient_map(const grad_args a)
         const unsigned c = strand_code(a.text[base + (win ? len - 1 - i : i)], win != 0);
         a.letters[(size_t)base + i] = (uint8_t)(c == 0 ? 'A' : c == 1 ? 'C' : c == 2 ? 'G' : c == 3 ? 'T' : 'N');
     }
-    if (tid == 0) a.Z[s] = zs[win];
+    if (tid == 0) a.Z[s] = a.strands == 2 && !(zs[0] >= zs[1]) && win == 0 ? __uint_as_float(0x7fc00000u) : zs[win];
 }
 
 // The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
@@ -620,7 +620,9 @@ __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict
             const float w = S[4 * (size_t)(mirror - i) + 3 - c];
             v = w > v ? w : v;
         }
-        map[4 * out + e] = (z > v ? z : v) > 0.0f ? v - z : 0.0f;
+        // (a product with 1 or 0, so that scores that are infinite or not a number show)
+        const float d = v - z;
+        map[4 * out + e] = (z > v ? z : v) > 0.0f ? d : v == v && z == z ? d * 0.0f : d;
     }
     if (threadIdx.x == 0) Z[s] = z;
 }

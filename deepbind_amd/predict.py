@@ -108,7 +108,7 @@ def _split(maps, text):
 def _mutation_maps(net, X, R, text):
     """(Z (nseq, 1), map (letters, 4)) of the batch, or None when the kernel does not take the net's shape."""
     ptype = _lib.str2pooltype[net.pool]
-    if net.dtype != torch.float32 or not _lib.dll().dbk_mutation_map_takes(net.m, net.nfilter, ptype, net.hidden):
+    if net.dtype != torch.float32 or int(text.lens.max()) > 4 * 65535 or not _lib.dll().dbk_mutation_map_takes(net.m, net.nfilter, ptype, net.hidden):
         return None
     p = net.p
     Wc = p["Wc"] if net.input_dropout <= 0 else p["Wc"] * (1.0 - net.input_dropout)
@@ -124,7 +124,7 @@ def _mutation_maps(net, X, R, text):
 
 
 def _gradient_maps(net, text):
-    """(Z (nseq, 1), map (letters, 4), the letters of the strands mapped) of the batch, or None when the kernel does not take it."""
+    """(Z (rows, 1), [(letters, map (length, 4)) of the strand mapped]) of the batch, or None when the kernel does not take it."""
     ptype, shortest, longest = _lib.str2pooltype[net.pool], int(text.lens.min()), int(text.lens.max())
     if net.dtype != torch.float32 or net.input_dropout > 0 or not _lib.dll().dbk_gradient_map_takes(net.m, net.nfilter, shortest, longest, ptype, net.hidden):
         return None
@@ -138,9 +138,11 @@ def _gradient_maps(net, text):
               _lib.ptr(Z), _lib.ptr(maps), _lib.ptr(strand))
     out = out.cpu().numpy()
     Z = out[:4 * n].view(np.float32).reshape(-1, 1)
-    if net.reverse_complement:
-        Z = Z[Z[:, 0] == Z[:, 0]]                    # (scores that do not compare select neither row of their pair)
-    return Z, out[4 * n:4 * n + 16 * L].view(np.float32).reshape(-1, 4), out[4 * n + 16 * L:].tobytes().decode("ascii")
+    gmaps = list(zip(_split(out[4 * n + 16 * L:].tobytes().decode("ascii"), text), _split(out[4 * n:4 * n + 16 * L].view(np.float32).reshape(-1, 4), text)))
+    keep = Z[:, 0] == Z[:, 0]
+    if net.reverse_complement and not keep.all():    # (scores that do not compare select neither row of their pair)
+        return Z[keep], [gmap for gmap, k in zip(gmaps, keep) if k]
+    return Z, gmaps
 
 
 def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
@@ -159,7 +161,7 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
         fused = _gradient_maps(net, text) if want_gmaps and want_gmaps != "finite_diff" else None
         if fused is not None:
             preds.append(fused[0])
-            gmaps += zip(_split(fused[2], text), _split(fused[1], text))
+            gmaps += fused[1]
             continue
         X, R = _pack(net, text)
         if not want_gmaps:
@@ -182,8 +184,9 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
         maps = torch.empty((len(text.bytes), 4), dtype=dX.dtype, device=dX.device)
         _lib.call("dbk_gather_maps", _lib.stream(), _lib.dtype_code(dX), _lib.ptr(R), R.shape[0], pad, 2 if rc else 1, _lib.ptr(Zall),
                   _lib.ptr(dX), _lib.ptr(maps))
-        reverse = Zmask.reshape(-1, 2)[:, 1] if Zmask is not None else None
-        gmaps += zip(text.strings(reverse), _split(maps.cpu().numpy(), text))
+        pairs = Zmask.reshape(-1, 2) if Zmask is not None else None
+        new = zip(text.strings(None if pairs is None else pairs[:, 1]), _split(maps.cpu().numpy(), text))
+        gmaps += new if pairs is None else [gmap for gmap, keep in zip(new, pairs.any(axis=1)) if keep]
     return np.vstack(preds), gmaps
 
 
@@ -194,7 +197,7 @@ def _score_windows(net, raws, nwin, windowsize, stride):
     offsets, first, letters = text.upload(net.device, np.concatenate([[0], np.cumsum(nwin)]))
     X = torch.empty((total * strands * (pad + windowsize) + pad, 1), dtype=torch.uint8, device=net.device)
     R = torch.empty((total * strands, 2), dtype=torch.uint32, device=net.device)
-    _lib.call("dbk_pack_windows", _lib.stream(), _lib.ptr(letters), _lib.ptr(offsets), _lib.ptr(first), len(raws), total, windowsize, stride,
+    _lib.call("dbk_pack_windows", _lib.stream(), _lib.ptr(letters), _lib.ptr(offsets), _lib.ptr(first), len(raws), total, int(windowsize), int(stride),
               pad, strands, _lib.ptr(X), _lib.ptr(R))
     return net.predict(X, R).cpu().numpy()
 
