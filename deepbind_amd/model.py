@@ -391,7 +391,7 @@ class SequenceNet(object):
         """Test-mode predictions through the fused scoring head (dropout rescale folded in)."""
         p = self.p
         P, ptype = R.shape[0], _lib.str2pooltype[self.pool]
-        if self.mode == "fused" and self.dtype == torch.float32 and self.nfeat == 0 and R.shape[1] == 2 and _lib.dll().dbk_predict_small_takes(
+        if self.mode == "fused" and self.dtype == torch.float32 and self.nfeat == 0 and F is None and R.shape[1] == 2 and _lib.dll().dbk_predict_small_takes(
                 self.m, self.ninst, self.nfilter, X.numel(), P, ptype, self.hidden):
             # a handful of sequences: one launch for everything
             Wc = p["Wc"] if self.input_dropout <= 0 else p["Wc"] * (1.0 - self.input_dropout)
@@ -860,10 +860,18 @@ class ModelGroup(object):
                 return run
             _side_by_side(self._streams(), [one(gi, idx, net) for gi, (idx, net) in enumerate(self.groups)])
             return
+        Y, Ymask = self._columns(Y), self._columns(Ymask)
         if len(self.groups) == 1:
             self.groups[0][1]._native_step(X, R, Y, Ymask, F)
             return
         _native_steps([(net, X, R, Y, Ymask, F, cols) for (_, net), cols in zip(self.groups, self._cols)])
+
+    def _columns(self, t):
+        """The models' columns of a target matrix, contiguous (which a program's own matrix mostly is: then it is used as it is)."""
+        if t is None or (t.shape[-1] == self.nmodel and t.is_contiguous()):
+            return t
+        _lib.require(t.shape[-1] >= self.nmodel, "ValueError: Y and Ymask must have a column per model")
+        return t[:, :self.nmodel].contiguous()
 
     def make_graphed_step(self, X, R, Y, Ymask=None, F=None):
         """One HIP graph holding the fused training step of every architecture group on a static batch."""

@@ -206,3 +206,58 @@ def test_gradient_map_kernel_edges(pool, hidden, loss, rc, rate, m, F):
     assert_close(Z, Zl, ACT, "Z, layer by layer")
     for (sa, a), (sb, b) in zip(maps, ml):
         assert sa == sb and (len(b) == 0 or np.abs(a - b).max() <= GRAD * scale)
+
+
+@pytest.mark.parametrize("which", ["b2", "W1"])
+def test_pairs_whose_scores_do_not_compare(which, monkeypatch):
+    """Scores that are not a number - of every strand, or only of strands on which one filter never fires - select neither row of a
+    pair: such sequences have no entry among the predictions or the maps, by the one-workgroup kernel as by the layers."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(5)
+    p = _params(rng, 8, 4, "max", 8)
+    if which == "b2":
+        p["b2"][:] = np.nan
+    else:
+        p["W1"][0, 0] = np.inf                          # 0 x inf where filter 0 stays at zero
+        p["bc"][0, 0] = -2.0
+    seqs = _seqs(rng, 40, 10, 14, 0.0)
+    net = _net(p, 8, 4, "max", 8, "nll", True, 0.0)
+    Z, maps = predict.gen_predictions(net, seqs, want_gmaps=True)
+    monkeypatch.setattr(predict, "_gradient_maps", lambda *a: None)
+    Zr, ref = predict.gen_predictions(net, seqs, want_gmaps=True)
+    monkeypatch.undo()
+    assert len(maps) == len(Z) == len(Zr) == len(ref) < len(seqs) or which == "W1"
+    assert [s for s, _ in maps] == [s for s, _ in ref] and np.allclose(Z, Zr, atol=1e-6, equal_nan=True)
+
+
+def test_feature_columns_and_wide_targets():
+    """Maps of nets with shared feature columns (absent: zeros) are those of the net without them; a group takes target
+    matrices with further columns behind its models' and ones that are not contiguous, and refuses ones with fewer."""
+    from deepbind_amd import predict
+    from deepbind_amd._lib import DeepbindError
+    from deepbind_amd.model import ModelGroup, SequenceNet
+    rng = np.random.default_rng(6)
+    p = _params(rng, 8, 4, "max", 8)
+    seqs = _seqs(rng, 5, 10, 14)
+    plain = _net(p, 8, 4, "max", 8, "nll", False, 0.0)
+    net = SequenceNet(1, 4, 8, pool="max", hidden=8, loss="nll", feature_columns=2)
+    net.set_params(dict(p, W1=np.concatenate([p["W1"], rng.standard_normal((2, 8)).astype(np.float32)])))
+    for mode in (True, "finite_diff"):
+        (Z, maps), (Zr, ref) = [predict.gen_predictions(n, seqs, want_gmaps=mode) for n in (net, plain)]
+        assert_close(Z, Zr, ACT, "predictions")
+        assert_close(np.concatenate([g for _, g in maps]), np.concatenate([g for _, g in ref]), GRAD, "maps")
+    X, R = [torch.from_numpy(v).cuda() for v in __import__("deepbind_amd.data", fromlist=["data"]).pack_sequences(seqs, 7)]
+    Y = rng.random((5, 3)).astype(np.float32)
+    wide = torch.from_numpy(np.concatenate([Y, Y + 1], axis=1)).cuda()
+    for pools in (["max", "all", "max"], ["max"] * 3):
+        out = []
+        for t in (wide[:, :3].contiguous(), wide, wide.t().contiguous().t(), wide[:, :3]):
+            grp = ModelGroup(pools, [0] * 3, 4, 8, loss="mse", rate=0.05, momentum=0.9)
+            for _, n in grp.groups:
+                n.init_params(init_conv=0.1, init_full=0.1, seed=3)
+            grp.train_step(X, R, t)
+            out.append([n.P.cpu().numpy() for _, n in grp.groups])
+        for o in out[1:]:
+            assert all(np.array_equal(a, b) for a, b in zip(out[0], o))
+        with pytest.raises(DeepbindError):
+            grp.train_step(X, R, wide[:, :2].contiguous())
