@@ -853,9 +853,10 @@ __global__ __launch_bounds__(64 * MB) void corr1ord_bprop_X_mfma_kernel(float* _
 }
 
 // A launch per 128 filters with the weights' pieces formed per workgroup, against the float32 products of corr1ord_mm.h (us a call, this /
-// those): 100 000 rows x 128 filters of 24 taps 51 / 54, 120 000 x 128 of 32 taps 55 / 72, 1.0 M x 256 450 / 943; 60 000 x 128 50 / 41,
-// 40 000 x 256 95 / 72, 200 000 x 96 111 / 82.
-inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 128 && n * F >= 12000000; }
+// those, 24 taps): 50 000 rows x 256 filters 96 / 52, 100 000 x 128 52 / 50, 100 000 x 256 98 / 87 (12 taps: 97 / 58), 150 000 x 256
+// 123 / 119, 120 000 x 128 of 32 taps 56 / 62, 250 000 x 128 66 / 80, 250 000 x 256 127 / 150, 500 000 x 256 235 / 305. Its launch costs ~50 us up to
+// ~120 000 rows whatever the taps, so rows x steps of the other kernel decide.
+inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 128 && n * (m + 3) >= 4100000; }
 
 inline int launch_bprop_X_mfma(hipStream_t st, float* dX, size_t n, const float* W, size_t m, size_t F, const float* dZ)
 {
@@ -915,10 +916,14 @@ template <typename T>
 int launch_bprop_X_mm(hipStream_t st, T* dX, size_t n, const T* W, size_t m, size_t F, const T* dZ)
 {
     using namespace dbk_corr_mm;
-    // fewer than two workgroups of 256 rows per CU: 64 rows each, whose bits then depend on the size of the call
-    const bool few = !dbk::exact_scan() && n < 512 * 256;
+    // fewer workgroups of 256 rows than fill the CUs' LDS twice (two fit in float64, five in float32): 64 rows each, whose bits then depend on
+    // the size of the call. 64 / 256 rows, us a call, 64 filters of 24 taps: float64 90 000 rows 39 / 46, 180 000 63 / 85, 250 000 86 / 86; float32
+    // 90 000 22 / 26, 123 000 27 / 26, 180 000 37 / 35, 250 000 48 / 44.
+    const bool few = !dbk::exact_scan() && n < (sizeof(T) == 8 ? 1024 : 512) * 256;
     const size_t smem = cx_smem<T>(m, few ? 1 : 4);
-    auto kern = few ? corr1ord_bprop_X_mm_kernel<T, 1> : corr1ord_bprop_X_mm_kernel<T, 4>;
+    auto kern = m <= 24 ? (few ? corr1ord_bprop_X_mm_kernel<T, 1, 24> : corr1ord_bprop_X_mm_kernel<T, 4, 24>)
+              : m <= 32 ? (few ? corr1ord_bprop_X_mm_kernel<T, 1, 32> : corr1ord_bprop_X_mm_kernel<T, 4, 32>)
+                        : (few ? corr1ord_bprop_X_mm_kernel<T, 1, 64> : corr1ord_bprop_X_mm_kernel<T, 4, 64>);
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3(dbk::divup(n, few ? 64 : 256)), dim3(256), smem, st, dX, n, W, (unsigned)m, (unsigned)F, dZ);
     DBK_LAUNCH_OK();

@@ -150,16 +150,18 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_W_mm_kernel(T* __restrict_
 // W lie in LDS at a stride of 17, so that the 16 lanes that read rows four apart, or 16 rows of W, meet no bank twice. Per
 // product one element of either operand per lane; one fixed order (filter tiles, d, filters, ascending), so that a row's bits do
 // not depend on its place in the batch.
-// Bound by the matrix pipe at F (m + 3) / 4 products of 64 (float64) or 32 (float32) clocks per 64 rows. Measured, us a call: float64,
-// 123 000 rows x 64 filters of 24 taps 63 (one wave per row: 444); float32, 250 000 x 16 filters 14 (one wave per 96 rows and 64
-// filters, multiply-adds with the weights in registers: 70), 123 000 x 64 31 (55).
+// The next 16 filters' columns are requested while these are multiplied and wait in registers (sized for up to MT taps): with the loads
+// behind the barrier a call of few waves spent most of its time on their latency (us a call, before / now: 123 000 rows x 64 filters
+// of 24 taps float64 70 / 48, float32 34 / 27; 20 000 x 256 95 / 48, 64 / 29; 250 000 x 64 of 8 taps 95 / 52, 42 / 28).
+// Bound by the matrix pipe at F (m + 3) / 4 products of 64 (float64) or 32 (float32) clocks per 64 rows, the LDS reads of its operands beside
+// it. Against the kernels before: float64, 123 000 x 64 444 us (one wave per row); float32, 250 000 x 16 filters 15 against 70
+// (one wave per 96 rows and 64 filters, multiply-adds with the weights in registers), 123 000 x 64 55.
 constexpr unsigned CX_ST = 17;
 // NB blocks of 64 rows per workgroup: 4, a wave each; or 1, whose steps d the four waves share out (wave w takes d = w, w + 4, ..,
-// and the four sums are added in wave order), for calls whose rows would otherwise leave CUs idle: float32, 20 000 rows x 256 filters
-// 59 us against 104, float64 92 against 211.
+// and the four sums are added in wave order), for calls whose rows would otherwise leave CUs idle.
 template <typename T> inline size_t cx_smem(size_t m, unsigned nb) { return ((64 * nb + m - 1) + (m + 6) * 4) * CX_ST * sizeof(T); }
 
-template <typename T, unsigned NB>
+template <typename T, unsigned NB, unsigned MT>
 __global__ __launch_bounds__(256) void corr1ord_bprop_X_mm_kernel(T* __restrict__ dX, size_t n, const T* __restrict__ W, unsigned m, unsigned F,
                                                                   const T* __restrict__ dZ)
 {
@@ -177,22 +179,44 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_mm_kernel(T* __restrict_
     acc_t acc = (acc_t)(T)0;
     const T* za = zs + (w0 + 4u * col) * CX_ST + k;                 // A: row 4 r + d of the wave's rows, r = col; d counted from -(m - 1)
     const T* wb = ws + ((m - 1 + 3) * 4u + col) * CX_ST + k;        // B: (s, c) = col at d = -(m - 1): tap s + m - 1
+    constexpr unsigned ZE = ((64 * NB + MT - 1) * 16 + 255) / 256, WE = ((MT + 6) * 64 + 255) / 256;
+    const unsigned nz = (64 * NB + m - 1) * 16, nw = (m + 6) * 64, er = tid >> 4, ef = tid & 15u;
+    T zr[ZE], wr[WE];
+    auto fetch = [&](unsigned f0) {                                 // the next 16 filters' columns: always an element of the matrix, kept or not below
+        const unsigned fl = f0 + ef < F ? f0 + ef : F - 1;
+#pragma unroll
+        for (unsigned i = 0; i < ZE; ++i) {
+            size_t row = q0 + er + 16 * i;                          // + (m - 1): offset by the rows before the workgroup's
+            row = row < m - 1 ? 0 : row - (m - 1);
+            zr[i] = dZ[(row < n ? row : n - 1) * F + fl];
+        }
+#pragma unroll
+        for (unsigned i = 0; i < WE; ++i) {
+            const unsigned r = er + 16 * i;
+            wr[i] = W[(size_t)(r < 12 ? 0 : r - 12 < 4 * m ? r - 12 : 4 * m - 1) * F + fl];
+        }
+    };
+    fetch(0);
     for (unsigned f0 = 0; f0 < F; f0 += 16) {
         __syncthreads();
-        for (unsigned e = tid; e < (64 * NB + m - 1) * 16; e += 256) {
-            const unsigned r = e >> 4, fl = f0 + (e & 15u);
-            const size_t row = q0 + r;                              // + (m - 1): offset by the rows before the workgroup's
-            const T v = row >= m - 1 && row - (m - 1) < n && fl < F ? dZ[(row - (m - 1)) * F + fl] : (T)0;
-            zs[r * CX_ST + (e & 15u)] = v;
-            odd |= !__builtin_isfinite(v);
-        }
-        for (unsigned e = tid; e < (m + 6) * 4 * 16; e += 256) {
-            const unsigned r = e >> 4, fl = f0 + (e & 15u);
-            const T v = r >= 12 && r - 12 < 4 * m && fl < F ? W[(size_t)(r - 12) * F + fl] : (T)0;
-            ws[r * CX_ST + (e & 15u)] = v;
-            odd |= !__builtin_isfinite(v);
-        }
+#pragma unroll
+        for (unsigned i = 0; i < ZE; ++i)
+            if (tid + 256 * i < nz) {
+                const size_t row = q0 + er + 16 * i;
+                const T v = row >= m - 1 && row - (m - 1) < n && f0 + ef < F ? zr[i] : (T)0;
+                zs[(er + 16 * i) * CX_ST + ef] = v;
+                odd |= !__builtin_isfinite(v);
+            }
+#pragma unroll
+        for (unsigned i = 0; i < WE; ++i)
+            if (tid + 256 * i < nw) {
+                const unsigned r = er + 16 * i;
+                const T v = r >= 12 && r - 12 < 4 * m && f0 + ef < F ? wr[i] : (T)0;
+                ws[r * CX_ST + ef] = v;
+                odd |= !__builtin_isfinite(v);
+            }
         __syncthreads();
+        if (f0 + 16 < F) fetch(f0 + 16);
 #pragma unroll 4
         for (unsigned d = d0; d < m + 3; d += DSTEP) {
 #pragma unroll

@@ -187,7 +187,7 @@ def test_corr1ord_bprop_X(ks, n, m, F, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n,m,F", [(1, 1, 1), (63, 8, 15), (64, 9, 17), (257, 32, 33), (1000, 25, 16), (3000, 33, 5), (131329, 24, 3), (700, 64, 20)])
+@pytest.mark.parametrize("n,m,F", [(1, 1, 1), (63, 8, 15), (64, 9, 17), (257, 32, 33), (1000, 25, 16), (3000, 33, 5), (131329, 24, 3), (700, 64, 20), (262401, 9, 17)])
 def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype):
     """Both gradients at the edges of the 16 x 16 x 4 kernels: rows around a block of 64 and a chunk of 256, fewer rows than taps, each tap
     tier and the first length beyond it, filters that leave most of a group of 16 empty, calls of one block per workgroup and of four;
@@ -209,6 +209,12 @@ def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype)
         outs.append(host(dX))
     assert_close(outs[0], refx, tol, "dX")
     assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (228001, 15, 128), (228001, 14, 128)])
+def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
+    """Either side of the size from which 128 filters and more go through the split-operand products, and a second launch of few filters."""
+    test_corr1ord_bprop_X(ks, n, m, F, np.float32)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
