@@ -44,7 +44,7 @@ int dbk_device_count(void);
  * at EVERY size, so that a row's result does not depend on the size of the batch it arrives in: dbk_corr1ord
  * then adds the taps in the reference's order (corr1ord.cuh:139-157: its bits) for any number of rows, and the two
  * gradients keep one summation order. Off (the default) float32 calls switch to the split-operand matrix-core kernels at bulk sizes
- * (2^25 map values for the forward, 2^22 for the filter gradient, ~150 000 rows for the input gradient): the same sums in another order, 1.5-2x faster.
+ * (2^25 map values for the forward, 2^22 for the filter gradient, ~140 000 rows for the input gradient): the same sums in another order, 1.5-2x faster.
  * Process-wide; returns the previous setting. No counterpart in the reference (it has one kernel per operator). */
 int dbk_set_exact_scan(int on);
 /* Blocks until `stream` has drained. reference: api_sync, smat_cuda/cuda_context.cpp:198-202 */

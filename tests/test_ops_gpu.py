@@ -211,7 +211,7 @@ def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype)
     assert np.array_equal(outs[0], outs[1])
 
 
-@pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (228001, 15, 128), (228001, 14, 128)])
+@pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (208401, 15, 128), (208301, 15, 128)])
 def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
     """Either side of the size from which 128 filters and more go through the split-operand products, and a second launch of few filters."""
     test_corr1ord_bprop_X(ks, n, m, F, np.float32)
