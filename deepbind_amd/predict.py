@@ -129,12 +129,13 @@ def _gradient_maps(net, text):
     if net.dtype != torch.float32 or net.input_dropout > 0 or not _lib.dll().dbk_gradient_map_takes(net.m, net.nfilter, shortest, longest, ptype, net.hidden):
         return None
     p, n, L = net.p, len(text.lens), len(text.bytes)
+    scale = (1.0 - net.dropout) if net.use_dropout else None
     offsets, letters = text.upload(net.device)
     out = torch.empty(4 * n + 17 * L, dtype=torch.uint8, device=net.device)                  # (one copy back to the host)
     Z, maps, strand = out[:4 * n], out[4 * n:4 * n + 16 * L], out[4 * n + 16 * L:]
     _lib.call("dbk_gradient_map", _lib.stream(), _lib.ptr(p["Wc"]), _lib.ptr(p["bc"]), net.m, net.nfilter, _lib.ptr(letters), _lib.ptr(offsets), n,
               shortest, longest, ptype, net.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")), _lib.ptr(p.get("b2")),
-              _lib.ptr((1.0 - net.dropout) if net.use_dropout else None), int(net.loss == "nll"), 2 if net.reverse_complement else 1,
+              _lib.ptr(scale), int(net.loss == "nll"), 2 if net.reverse_complement else 1,
               _lib.ptr(Z), _lib.ptr(maps), _lib.ptr(strand))
     out = out.cpu().numpy()
     Z = out[:4 * n].view(np.float32).reshape(-1, 1)

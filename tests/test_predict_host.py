@@ -1,0 +1,51 @@
+"""Host side of the prediction-time callers, without a GPU: what is refused, and what is alive when the library is called."""
+import types
+import weakref
+
+import numpy as np
+import pytest
+import torch
+
+from deepbind_amd import _lib, predict
+
+
+def _net(**kw):
+    net = dict(ninst=1, m=4, nfilter=2, pool="max", hidden=0, loss="nll", dtype=torch.float32, input_dropout=0.0, use_dropout=True,
+               dropout=torch.full((1,), 0.25), reverse_complement=False, device="cpu", mode="fused", nfeat=0,
+               p=dict(Wc=torch.zeros(16, 2), bc=torch.zeros(1, 2), W1=torch.zeros(2, 1), b1=torch.zeros(1, 1)))
+    net.update(kw)
+    return types.SimpleNamespace(**net)
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """The library's calls, recorded in place of being made; every tensor whose address a call takes must be alive when it is made
+    (freed before, its memory is another thread's to take while the launch that reads it is not yet on the stream)."""
+    taken, made = [], []
+
+    def ptr(t):
+        if t is not None:
+            taken.append(weakref.ref(t))
+
+    def call(name, *args):
+        made.append(name)
+        assert all(ref() is not None for ref in taken), "%s was given the address of a tensor that is gone" % name
+        taken.clear()
+
+    monkeypatch.setattr(_lib, "ptr", ptr)
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(_lib, "stream", lambda: None)
+    return made
+
+
+@pytest.mark.parametrize("rc", [False, True])
+def test_tensors_live_until_the_call_that_reads_them(calls, rc):
+    net = _net(reverse_complement=rc, hidden=3)
+    net.p.update(W1=torch.zeros(2, 3), b1=torch.zeros(1, 3), W2=torch.zeros(3, 1), b2=torch.zeros(1, 1))
+    text = predict._Text(["ACGT", "GGN"])
+    assert predict._gradient_maps(net, text) is not None
+    X, R = predict._pack(net, text)
+    assert predict._mutation_maps(net, X, R, text) is not None
+    net.predict = lambda X, R: torch.zeros(R.shape[0], 1)
+    predict._score_windows(net, ["ACGT"], [9], 6, 1)
+    assert calls == ["dbk_gradient_map", "dbk_pack_text", "dbk_mutation_map", "dbk_pack_windows"]
