@@ -61,10 +61,13 @@ def _finite_diff(net, Xd, Rd, R, Z, dX):
 
 
 class _Text(object):
-    """Sequence strings as the device takes them: their letters end to end, and where each begins."""
+    """Sequences as the device takes them: their letters end to end, and where each begins. Strings, or anything whose
+    buffer holds letters unless `strings` says that only strings will do (reverse complements and windows of a sequence)."""
 
-    def __init__(self, seqs):
-        seqs = [s if isinstance(s, str) else bytes(s).decode("latin-1") for s in seqs]
+    def __init__(self, seqs, strings=False):
+        if strings and not all(isinstance(s, str) for s in seqs):
+            raise TypeError("sequences must be strings")
+        seqs = [s if isinstance(s, str) else np.frombuffer(s, dtype=np.uint8).tobytes().decode("latin-1") for s in seqs]
         self.bytes = np.frombuffer("".join(seqs).encode("latin-1"), dtype=np.uint8)
         self.lens = np.fromiter(map(len, seqs), dtype=np.int64, count=len(seqs))
         self.offsets = np.zeros(len(seqs) + 1, dtype=np.int64)
@@ -158,7 +161,7 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     rc, pad = net.reverse_complement, net.m - 1
     preds, gmaps = [], ([] if want_gmaps else None)
     for s0 in range(0, len(seqs), batchsize):
-        text = _Text(seqs[s0:s0 + batchsize])
+        text = _Text(seqs[s0:s0 + batchsize], strings=rc)
         fused = _gradient_maps(net, text) if want_gmaps and want_gmaps != "finite_diff" else None
         if fused is not None:
             preds.append(fused[0])
@@ -193,7 +196,7 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
 
 def _score_windows(net, raws, nwin, windowsize, stride):
     """Predictions of all windows of a few sequences: the windows are cut on the device."""
-    text = _Text(raws)
+    text = _Text(raws, strings=True)
     strands, pad, total = (2 if net.reverse_complement else 1), net.m - 1, int(sum(nwin))
     offsets, first, letters = text.upload(net.device, np.concatenate([[0], np.cumsum(nwin)]))
     X = torch.empty((total * strands * (pad + windowsize) + pad, 1), dtype=torch.uint8, device=net.device)

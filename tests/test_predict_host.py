@@ -50,3 +50,18 @@ def test_tensors_live_until_the_call_that_reads_them(calls, rc):
     net.predict = lambda X, R: torch.zeros(R.shape[0], 1)
     predict._score_windows(net, ["ACGT"], [9], 6, 1)
     assert calls == ["dbk_gradient_map", "dbk_pack_text", "dbk_mutation_map", "dbk_pack_windows"]
+
+
+@pytest.mark.parametrize("mode", [False, True, "finite_diff"])
+def test_what_is_no_sequence_is_refused(calls, mode):
+    """A number is no sequence (bytes(5) would make five letters of it), nor a list of numbers; bytes are one where no reverse complement
+    is taken and no window cut."""
+    for seqs in ([5], [[65, 67]], [None], ["ACGT", 7]):
+        with pytest.raises(TypeError):
+            predict.gen_predictions(_net(), seqs, want_gmaps=mode)
+    with pytest.raises(TypeError):
+        predict.gen_predictions(_net(reverse_complement=True), [b"ACGT"], want_gmaps=mode)
+    with pytest.raises(TypeError):
+        predict.gen_predictionmaps(_net(), [b"ACGT"], want_gmaps=mode is True)
+    assert not calls
+    assert predict._Text([b"AC", bytearray(b"g"), np.frombuffer(b"TN", np.uint8), b""]).strings() == ["AC", "G", "TN", ""]
