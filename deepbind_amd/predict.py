@@ -214,19 +214,23 @@ def gen_predictionmaps(net, seqs, stride=1, windowsize=20, want_gmaps=False):
     if want_gmaps and stride != 1:
         # the reference's aggregation (predict.py:330-340) slices rows that only line up for stride 1
         raise ValueError("window-averaged gradient maps need stride 1 (got %d)" % stride)
-    assert net.ninst == 1, "prediction maps are defined for one model at a time"
     pmaps, gmaps = [], ([] if want_gmaps else None)
     chunk = 32
     for c0 in range(0, len(seqs), chunk):
         raws = list(seqs[c0:c0 + chunk])
-        nwin = [len(range(0, max(1, len(raw) + windowsize - 1), stride)) for raw in raws]
         if want_gmaps or windowsize < 2:         # (one-letter windows have no N around them: an empty sequence's window is empty)
-            windows = []
+            windows, nwin = [], []
             for raw in raws:
                 padseq = "N" * (windowsize - 1) + raw + "N" * (windowsize - 1)
-                windows += [padseq[i:i + windowsize] for i in range(0, max(1, len(padseq) - windowsize + 1), stride)]
+                cut = [padseq[i:i + windowsize] for i in range(0, max(1, len(padseq) - windowsize + 1), stride)]
+                windows += cut
+                nwin.append(len(cut))
             Z, wmaps = gen_predictions(net, windows, want_gmaps=want_gmaps, batchsize=len(windows))
         else:
+            assert net.ninst == 1, "prediction maps are defined for one model at a time"
+            if stride < 1:
+                raise ValueError("windows are cut every stride letters, at least 1 (got %d)" % stride)
+            nwin = [len(range(0, max(1, len(raw) + windowsize - 1), stride)) for raw in raws]
             Z = _score_windows(net, raws, nwin, windowsize, stride)
         edges = np.cumsum([0] + nwin)
         for i, raw in enumerate(raws):

@@ -65,3 +65,15 @@ def test_what_is_no_sequence_is_refused(calls, mode):
         predict.gen_predictionmaps(_net(), [b"ACGT"], want_gmaps=mode is True)
     assert not calls
     assert predict._Text([b"AC", bytearray(b"g"), np.frombuffer(b"TN", np.uint8), b""]).strings() == ["AC", "G", "TN", ""]
+
+
+def test_strides_and_windows_below_one(monkeypatch):
+    """A stride below one is refused; windows of no letter are scored as they are cut, as many of them as there are."""
+    for stride in (0, -1, -7):
+        with pytest.raises(ValueError):
+            predict.gen_predictionmaps(_net(predict=lambda X, R: torch.zeros(R.shape[0], 1)), ["ACGTACGT"], stride=stride, windowsize=4)
+    seen = []
+    monkeypatch.setattr(predict, "gen_predictions", lambda net, seqs, **kw: seen.extend(seqs) or (np.arange(len(seqs)).reshape(-1, 1), None))
+    pmaps, _ = predict.gen_predictionmaps(_net(), ["ACG", "", "TT"], windowsize=0)
+    assert seen == [""] * 8 and [p.tolist() for p in pmaps] == [[0, 1, 2, 3], [4], [5, 6, 7]]
+    assert predict.gen_predictionmaps(_net(ninst=2), [])[0] == []
