@@ -11,6 +11,8 @@ namespace {
 
 using namespace dbk_scan;
 
+constexpr double MAX_BOUND = 4294967295.0;                          // region bounds are 32-bit
+
 __device__ __forceinline__ unsigned code_of_char(unsigned c)
 {
     c |= 32u;                                                       // (letters only differ in this bit from their capitals)
@@ -650,6 +652,8 @@ int dbk_pack_text(dbk_stream_t stream, const uint8_t* text, const uint32_t* offs
 {
     DBK_CHECK(strands == 1 || strands == 2, "ValueError: strands must be 1 or 2");
     if (nseq == 0) { dbk::clear_error(); return 0; }
+    // (the letters, which only the device knows here, count too: the caller sizes X and sees to it)
+    DBK_CHECK((double)nseq * strands * (double)padding <= MAX_BOUND, "ValueError: the stream of %zu sequences has more than 2^32 - 1 bytes", nseq);
     DBK_CHECK(offsets && X && R, "ValueError: null pointer argument");
     unsigned grid = dbk::divup(nseq * strands, 4);
     if (grid > 8192u) grid = 8192u;
@@ -663,6 +667,7 @@ int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* o
     DBK_CHECK(strands == 1 || strands == 2, "ValueError: strands must be 1 or 2");
     DBK_CHECK(window >= 1 && stride >= 1, "ValueError: window and stride must be >= 1");
     if (nseq == 0 || nwindow == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK((double)nwindow * strands * ((double)padding + (double)window) <= MAX_BOUND, "ValueError: the stream of %zu windows has more than 2^32 - 1 bytes", nwindow);
     DBK_CHECK(offsets && first && X && R, "ValueError: null pointer argument");
     const size_t nbyte = nwindow * strands * (padding + window) + padding;
     hipLaunchKernelGGL(k_pack_windows, dim3(dbk::ew_grid(nbyte)), dim3(256), 0, dbk::as_stream(stream), text, offsets, first, (unsigned)nseq,

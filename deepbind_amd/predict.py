@@ -8,6 +8,8 @@ windows out of them and picking a map's rows are kernels. A mutation map is one 
 rows a changed letter moves (nets whose shape that kernel does not take re-score the batch once per (position,
 base), as the reference does, the stream mutated and the differences collected on the device).
 """
+import itertools
+
 import numpy as np
 import torch
 
@@ -15,6 +17,7 @@ from . import _lib
 from . import data as _data
 
 _RCINDEX = (3, 2, 1, 0)
+_STREAM_MAX = 2 ** 32 - 1        # bytes of a packed stream, and letters of a batch: region bounds and text offsets are 32-bit
 
 
 def maskout_revcomp(Z, reverse_complement):
@@ -75,6 +78,7 @@ class _Text(object):
 
     def upload(self, device, *tables):
         """One copy to the device: (offsets, the further uint32 tables, letters)."""
+        _lib.require(len(self.bytes) <= _STREAM_MAX, "ValueError: more than 2^32 - 1 letters in one batch")
         words = [np.asarray(t, dtype=np.uint32) for t in (self.offsets,) + tables]
         buf = torch.from_numpy(np.concatenate([w.view(np.uint8) for w in words] + [self.bytes])).to(device)
         out, at = [], 0
@@ -96,8 +100,10 @@ class _Text(object):
 def _pack(net, text):
     """(X, R) of the batch on the device, as data.pack_sequences lays them out."""
     strands, pad, n = (2 if net.reverse_complement else 1), net.m - 1, len(text.lens)
+    N = strands * (n * pad + len(text.bytes)) + pad
+    _lib.require(N <= _STREAM_MAX, "ValueError: a batch of %d letters packs to more than 2^32 - 1 bytes; score in smaller batches" % len(text.bytes))
     offsets, letters = text.upload(net.device)
-    X = torch.empty((strands * (n * pad + len(text.bytes)) + pad, 1), dtype=torch.uint8, device=net.device)
+    X = torch.empty((N, 1), dtype=torch.uint8, device=net.device)
     R = torch.empty((n * strands, 2), dtype=torch.uint32, device=net.device)
     _lib.call("dbk_pack_text", _lib.stream(), _lib.ptr(letters), _lib.ptr(offsets), n, pad, strands, _lib.ptr(X), _lib.ptr(R))
     return X, R
@@ -194,10 +200,26 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     return np.vstack(preds), gmaps
 
 
+def _cut(raws, nwin, windowsize, stride):
+    """The windows of the sequences, one after another, as strings."""
+    for raw, n in zip(raws, nwin):
+        padseq = "N" * (windowsize - 1) + raw + "N" * (windowsize - 1)
+        for i in range(n):
+            yield padseq[i * stride:i * stride + windowsize]
+
+
 def _score_windows(net, raws, nwin, windowsize, stride):
-    """Predictions of all windows of a few sequences: the windows are cut on the device."""
-    text = _Text(raws, strings=True)
+    """Predictions of all windows of a few sequences: the windows are cut on the device. (Sequences whose windows pack to
+    more than region bounds can say are cut on the host, a batch at a time.)"""
     strands, pad, total = (2 if net.reverse_complement else 1), net.m - 1, int(sum(nwin))
+    span = strands * (pad + windowsize)
+    if total * span + pad > _STREAM_MAX:
+        windows, Z = _cut(raws, nwin, windowsize, stride), []
+        most = max(1, min(2 ** 20, (_STREAM_MAX - pad) // span))
+        for batch in iter(lambda: list(itertools.islice(windows, most)), []):
+            Z.append(gen_predictions(net, batch, batchsize=len(batch))[0])
+        return np.vstack(Z)
+    text = _Text(raws, strings=True)
     offsets, first, letters = text.upload(net.device, np.concatenate([[0], np.cumsum(nwin)]))
     X = torch.empty((total * strands * (pad + windowsize) + pad, 1), dtype=torch.uint8, device=net.device)
     R = torch.empty((total * strands, 2), dtype=torch.uint32, device=net.device)

@@ -419,13 +419,14 @@ int dbk_counter_add(dbk_stream_t stream, uint64_t* counter, uint64_t delta);
 
 /* Text to packed stream: nseq sequences of bytes, sequence s at text[offsets[s]] .. text[offsets[s+1] - 1], become X
  * (strands * (nseq * padding + letters) + padding bytes: A, C, G, T/U in either case -> 0..3, anything else and the pads ->
- * 255) and its region table R (nseq * strands, 2). strands = 2 interleaves every sequence with its reverse complement.
+ * 255) and its region table R (nseq * strands, 2). strands = 2 interleaves every sequence with its reverse complement. Region
+ * bounds are 32-bit: X must have fewer than 2^32 bytes (only the device knows the letters, so the caller sees to it).
  * reference: kangaroo/kangaroo/util.py:50-56,68-74, data.py:274-354 (on the host there). */
 int dbk_pack_text(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, size_t nseq, size_t padding, int strands,
                   uint8_t* X, uint32_t* R);
 /* The same for every window of `window` letters, `stride` apart, of sequences with window - 1 N on either side:
  * sequence s has the windows first[s] .. first[s+1] - 1 (first[nseq] = nwindow). X: nwindow * strands * (padding + window) +
- * padding bytes. reference: kangaroo/kangaroo/predict.py:279-300. */
+ * padding bytes; refused where the last region would end past 2^32 - 1. reference: kangaroo/kangaroo/predict.py:279-300. */
 int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, const uint32_t* first, size_t nseq, size_t nwindow,
                      size_t window, size_t stride, size_t padding, int strands, uint8_t* X, uint32_t* R);
 /* Scores (nregion, nmodel) of few sequences in one launch: scan, bias, rectifier, pooling and dense head, as

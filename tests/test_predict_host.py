@@ -77,3 +77,44 @@ def test_strides_and_windows_below_one(monkeypatch):
     pmaps, _ = predict.gen_predictionmaps(_net(), ["ACG", "", "TT"], windowsize=0)
     assert seen == [""] * 8 and [p.tolist() for p in pmaps] == [[0, 1, 2, 3], [4], [5, 6, 7]]
     assert predict.gen_predictionmaps(_net(ninst=2), [])[0] == []
+
+
+class _Letters(object):
+    """So many letters, none of them in memory."""
+
+    def __init__(self, n):
+        self.n = n
+
+    def __len__(self):
+        return self.n
+
+
+def test_streams_that_region_bounds_cannot_address_are_refused(calls):
+    text = predict._Text(["A"])
+    for letters, n, rc in ((2 ** 32, 1, False), (2 ** 32 - 4, 1, False), (2 ** 31 - 5, 2, True)):
+        text.bytes, text.lens = _Letters(letters), np.zeros(n, np.int64)
+        with pytest.raises(_lib.DeepbindError, match="2\\^32"):
+            predict._pack(_net(reverse_complement=rc), text)
+    text.bytes = _Letters(2 ** 32)
+    with pytest.raises(_lib.DeepbindError, match="2\\^32"):
+        text.upload("cpu")
+    lib, one = _lib.dll(), 1                                       # (refused for their sizes, before anything is read or launched)
+    for strands, nwindow in ((1, 2 ** 32 // 83 + 1), (2, 2 ** 31 // 83 + 1)):
+        assert lib.dbk_pack_windows(None, one, one, one, 1, nwindow, 60, 1, 23, strands, one, one) != 0
+        assert b"2^32" in lib.dbk_last_error()
+    assert lib.dbk_pack_text(None, one, one, 2 ** 27, 32, 1, one, one) != 0 and b"2^32" in lib.dbk_last_error()
+
+
+@pytest.mark.parametrize("rc", [False, True])
+def test_windows_beyond_one_stream_are_cut_on_the_host(rc, monkeypatch):
+    """Every batch packs to no more bytes than a stream may have, and together they are the windows the device would cut."""
+    net, raws, w, stride = _net(reverse_complement=rc), ["ACGTACGTAA", "", "TTG"], 5, 2
+    span = (2 if rc else 1) * (net.m - 1 + w)
+    nwin = [len(range(0, max(1, len(s) + w - 1), stride)) for s in raws]
+    for most in (1, 3, 6):
+        monkeypatch.setattr(predict, "_STREAM_MAX", most * span + net.m - 1)
+        seen = []
+        monkeypatch.setattr(predict, "gen_predictions", lambda net, seqs, **kw: seen.append(list(seqs)) or (np.array([[hash(s) % 1000] for s in seqs]), None))
+        Z = predict._score_windows(net, raws, nwin, w, stride)
+        cut = [("N" * (w - 1) + s + "N" * (w - 1))[i:i + w] for s in raws for i in range(0, max(1, len(s) + w - 1), stride)]
+        assert sum(seen, []) == cut and all(len(b) <= most for b in seen) and Z.ravel().tolist() == [hash(s) % 1000 for s in cut]
