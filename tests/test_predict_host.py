@@ -103,6 +103,7 @@ def test_streams_that_region_bounds_cannot_address_are_refused(calls):
         assert lib.dbk_pack_windows(None, one, one, one, 1, nwindow, 60, 1, 23, strands, one, one) != 0
         assert b"2^32" in lib.dbk_last_error()
     assert lib.dbk_pack_text(None, one, one, 2 ** 27, 32, 1, one, one) != 0 and b"2^32" in lib.dbk_last_error()
+    assert lib.dbk_pack_text(None, None, None, 0, 32, 1, None, None) == 0 and lib.dbk_last_error() == b""
 
 
 @pytest.mark.parametrize("rc", [False, True])
