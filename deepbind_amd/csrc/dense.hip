@@ -677,6 +677,24 @@ __global__ __launch_bounds__(256) void k_head_lanes(size_t n, int nblock, int k,
     }
 }
 
+// Where k_head16, whose weights in LDS feed four rows (two beyond 16 inputs, one beyond 32) of 16 models each, is the better of the two: it
+// spends about a microsecond per 32 multiply-adds of an item before the first row is out, and then fewer instructions an item than
+// k_head_lanes' padded 16 x 16 blocks - by most where a block is mostly padding (few hidden units), by none where its inputs are no whole
+// packs or LDS holds few workgroups of it. The line is the measured break-even in rows x models of 50 shapes; within 1.3 % of always
+// taking the faster one over 2907 calls of 4096 to 300 000 rows, 1 to 64 models. us a call, k_head16 / k_head_lanes: 100 000 x 24
+// models (32 -> 8 -> 1) 82 / 166, 30 000 x 8 (16 -> 4) 6.5 / 9.9, 100 000 x 16 (16 -> 32) 66 / 89; 30 000 x 16 (16 -> 32) 27 / 25,
+// 10 000 x 24 (32 -> 8) 14 / 13, 30 000 x 12 (24 -> 16) 36 / 24.
+inline bool head16_pays(size_t n, int nblock, int inputs, int hidden)
+{
+    const size_t smem = ((size_t)inputs * hidden + 2 * (size_t)hidden) * HG * sizeof(float);
+    if (n < 4096 || hidden == 0 || (hidden & 3) || smem > 65536 || nblock < (hidden <= 4 ? 4 : 6)) return false;
+    const size_t items = n * (size_t)nblock, macs = (size_t)inputs * hidden;
+    if (inputs > 16 && inputs != 32 && inputs != 64) return inputs < 24 && items >= 1000000;
+    if (hidden <= 4) return items >= 500 * macs;
+    if (inputs <= 16 && items >= 4000000) return true;
+    return macs <= (inputs == 32 ? 512u : 640u) && items >= 160000 && items >= 1200 * macs;
+}
+
 // Row-slice count for the kernels that stage 16 models' weights per workgroup: about 1024 workgroups in all
 // (a few per CU), so that staging is paid once per many rows.
 inline unsigned row_slices(size_t n, unsigned rows_per_pass, unsigned ngroups)
@@ -1016,10 +1034,9 @@ int dbk_head_fprop(dbk_stream_t stream, size_t n, int nblock, int k, int hidden,
     unsigned gx = dbk::divup(n, 256);
     if (gx > 2048u) gx = 2048u;
     const size_t smem16 = ((size_t)kk_all * hidden + 2 * (size_t)hidden) * HG * sizeof(float);
-    // The lane-per-item kernel's weights feed four rows each (9 instructions an item at 16 inputs against 15): worth it where its
-    // groups of 16 models are mostly full. 100 000 rows x 64 models (16 -> 32 -> 1): 165 us against 275; x 8 models: 45 / 37.
-    const bool grouped = n >= 4096 && hidden > 0 && (hidden & 3) == 0 && k <= 16 && nblock >= 12;
-    // (Whether the feature columns are given or left out as zeros must not change the kernel: kw, not kk_all, decides.)
+    // (Whether the feature columns are given or left out as zeros must not change the bits: what does not depend on it decides. k_head, which
+    // takes over from k_head16 where given columns do not fit in LDS, adds in k_head16's order.)
+    const bool grouped = head16_pays(n, nblock, k, hidden);
     if (!grouped && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
         const int mg = nblock >= 4 ? 4 : (nblock >= 2 ? 2 : 1);
         const unsigned cols = dbk::divup(nblock, mg);

@@ -770,6 +770,29 @@ def test_head_fprop_lane_groups(ds, n, k, h, nb):
         assert_close(host(got), orc.logistic(ref) if logistic else ref, ACT, "scores")
 
 
+@pytest.mark.parametrize("n,k,h,nb,nfeat", [(10001, 32, 8, 33, 0), (4097, 16, 4, 9, 0), (62501, 20, 16, 16, 0), (30001, 16, 60, 12, 0), (9001, 16, 64, 70, 0),
+                                            (40001, 16, 32, 16, 16), (4500, 64, 4, 30, 0), (26001, 64, 8, 25, 0), (11000, 5, 64, 35, 3)])
+def test_head_fprop_either_side_of_the_bulk_rule(ds, n, k, h, nb, nfeat):
+    """Shapes that the 16-models-per-workgroup kernel takes by rows x models, and ones that do not fit its LDS: for all of them the scores
+    are the oracle's, and feature columns left out give the bits of columns of zeros."""
+    rng = np.random.default_rng(n + k + h + nb)
+    Pl = np.abs(rng.standard_normal((n, k * nb))).astype(np.float32)
+    W1 = (rng.standard_normal(((k + nfeat) * nb, h)) * 0.2).astype(np.float32); b1 = (rng.standard_normal((1, h * nb)) * 0.1).astype(np.float32)
+    W2 = (rng.standard_normal((h * nb, 1)) * 0.2).astype(np.float32); b2 = (rng.standard_normal((1, nb)) * 0.1).astype(np.float32)
+    F = rng.standard_normal((n, nfeat)).astype(np.float32) if nfeat else None
+    X = Pl.astype(np.float64).reshape(n, nb, k)
+    if nfeat:
+        X = np.concatenate([X, np.broadcast_to(F.astype(np.float64)[:, None], (n, nb, nfeat))], axis=2)
+    A = np.einsum("nbk,bkh->nbh", X, W1.astype(np.float64).reshape(nb, k + nfeat, h)) + b1.reshape(nb, h)
+    ref = (np.maximum(A, 0) * W2.reshape(nb, h)).sum(axis=2) + b2
+    args = [dev(Pl), dev(W1), dev(b1), dev(W2), dev(b2)]
+    got = ds.head_fprop(*args, nblock=nb, nfeat=nfeat, feats=None if F is None else dev(F))
+    assert_close(host(got), ref, ACT, "scores")
+    if nfeat:
+        none, zeros = [host(ds.head_fprop(*args, nblock=nb, nfeat=nfeat, feats=f)) for f in (None, dev(F * 0))]
+        assert np.array_equal(none, zeros)
+
+
 @pytest.mark.parametrize("k,h,nb", [(16, 32, 37), (32, 8, 16), (16, 64, 5)])
 def test_head_fprop_bulk_rows(ds, k, h, nb):
     """Row counts that take the 16-models-per-workgroup kernel; model count not a multiple of 16; dropout rescale."""
