@@ -677,9 +677,14 @@ int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* o
 
 int dbk_predict_small_takes(size_t m, size_t nmodel, size_t nfilter, size_t N, size_t nregion, int ptype, size_t hidden)
 {
-    // Every workgroup stages its model's weights: worth it while the call is one wave of latency. Measured with 24 taps (us a call,
-    // this kernel / scan kernel + head): 2000 x 101 nt 15 / 18, 4000 x 101 nt 27 / 21, 900 x 500 nt 24 / 23, 100 x 101 nt x 32 models 22 / 17.
+    // Every workgroup stages its model's weights: worth it while the call is a few waves of latency. One model's 16 filters leave the scan
+    // kernel 48 of a tile's 64 lanes idle: up to 6e6 rows x taps (us a call, this kernel / scan kernel + head: 24 taps, 2000 x 101 nt 15 /
+    // 18; 4 taps, 65 217 x 20 nt 94 / 240; 8 taps, 3358 x 60 nt 15 / 26). Where models share a tile, the workgroups that a GPU holds
+    // at once, 2048, are the line besides: 16 models of 8 filters of 8 taps, 69 x 60 nt 6.6 / 10.4, 699 x 60 nt 41 / 17; of 4 taps, 4076 x
+    // 20 nt 71 / 39. Of 3758 calls of 4 to 64 taps, 20 to 2000 nt, 1 to 64 models of 1 to 16 filters, 37 of those it takes are more than 5 %
+    // slower than the scan kernel + head, by at most 8 us.
     return m >= 1 && m <= 64 && nfilter >= 1 && nfilter <= MUT_F && hidden <= 64 && N * nmodel * m <= 6000000 && nregion < ((size_t)1 << 31) && nmodel <= 65535 &&
+           (nmodel == 1 || nregion * nmodel <= 2048) &&
            (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL);
 }
 
@@ -689,7 +694,7 @@ int dbk_predict_small(dbk_stream_t stream, const float* W, const float* bias, si
 {
     if (nregion == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(dbk_predict_small_takes(m, nmodel, nfilter, N, nregion, ptype, hidden), "NotImplementedError: dbk_predict_small takes up to 6e6 rows x models x taps, "
-              "models of up to 16 filters of up to 64 taps and 64 hidden units");
+              "one model or up to 2048 regions x models, models of up to 16 filters of up to 64 taps and 64 hidden units");
     DBK_CHECK(W && bias && X && regions && W1 && b1 && scores, "ValueError: null pointer argument");
     DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
     small_args a;

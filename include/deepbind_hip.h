@@ -430,8 +430,8 @@ int dbk_pack_text(dbk_stream_t stream, const uint8_t* text, const uint32_t* offs
 int dbk_pack_windows(dbk_stream_t stream, const uint8_t* text, const uint32_t* offsets, const uint32_t* first, size_t nseq, size_t nwindow,
                      size_t window, size_t stride, size_t padding, int strands, uint8_t* X, uint32_t* R);
 /* Scores (nregion, nmodel) of few sequences in one launch: scan, bias, rectifier, pooling and dense head, as
- * dbk_scanpool_fprop followed by dbk_head_fprop (no feature columns). Up to 6e6 rows x models x taps, models of up to 16
- * filters of up to 64 taps and up to 64 hidden units (dbk_predict_small_takes). */
+ * dbk_scanpool_fprop followed by dbk_head_fprop (no feature columns). Up to 6e6 rows x models x taps, one model or up to
+ * 2048 regions x models, models of up to 16 filters of up to 64 taps and up to 64 hidden units (dbk_predict_small_takes). */
 int dbk_predict_small_takes(size_t m, size_t nmodel, size_t nfilter, size_t N, size_t nregion, int ptype, size_t hidden);
 int dbk_predict_small(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nmodel, size_t nfilter, const uint8_t* X, size_t N,
                       const uint32_t* regions, size_t nregion, int ptype, size_t hidden, const float* W1, const float* b1, const float* W2,

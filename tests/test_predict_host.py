@@ -119,3 +119,11 @@ def test_windows_beyond_one_stream_are_cut_on_the_host(rc, monkeypatch):
         Z = predict._score_windows(net, raws, nwin, w, stride)
         cut = [("N" * (w - 1) + s + "N" * (w - 1))[i:i + w] for s in raws for i in range(0, max(1, len(s) + w - 1), stride)]
         assert sum(seen, []) == cut and all(len(b) <= most for b in seen) and Z.ravel().tolist() == [hash(s) % 1000 for s in cut]
+
+
+def test_calls_that_fill_the_gpu_are_not_scored_in_one_launch():
+    """A workgroup per region and model: one model, or few enough of both; the scan kernel and the head take the rest."""
+    takes = _lib.dll().dbk_predict_small_takes
+    assert takes(24, 1, 16, 64 * 124 + 23, 64, 0, 32) == 1 and takes(8, 1, 16, 700000, 7000, 0, 0) == 1
+    assert takes(8, 16, 8, 128 * 67 + 7, 128, 0, 32) == 1 and takes(8, 16, 8, 129 * 67 + 7, 129, 0, 32) == 0
+    assert takes(4, 64, 16, 23020, 1019, 3, 32) == 0 and takes(24, 1, 16, 250001, 2000, 0, 32) == 0
