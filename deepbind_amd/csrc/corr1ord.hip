@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void corr1ord_bprop_X_kernel(T* __restrict__ d
 // positions, so the letters of a 16-position window are read once into scalar registers.
 // ---------------------------------------------------------------------------------------------
 constexpr unsigned WSUBS = 4;             // windows of PSUB positions per wave and staging round
-constexpr unsigned WSUBS_W = 8;           // the same for the register-plane kernel
+constexpr unsigned WSUBS_W = 8;           // the same for the register-plane kernels
 
 // forward: every (position, tap) is one LDS read with an immediate offset; taps in ascending order,
 // so the sums are bit-identical to the any-length kernel's. A workgroup builds its filter tile's
@@ -314,6 +314,74 @@ __global__ __launch_bounds__(256) void corr1ord_wide_kernel(const float* __restr
                 if (f + 3 < F) dst[3] = acc[p].w;
             }
         }
+    }
+}
+
+// filter gradient, pass 1: a lane keeps its filter's whole [letter][tap] column in registers; the window's
+// letters (scalars) pick the register plane each gradient value is added into through the register index
+// mode: one addition per (position, tap). "Mean of the four" letters collect in a plane of their own that
+// is spread over the four channels (x 1/4) at the end.
+// Workgroup y walks chunks y, y+gridDim.y, ... in ascending order; its waves are folded in wave order.
+template <int MT>
+__global__ __launch_bounds__(256) void corr1ord_bprop_W_window_kernel(float* __restrict__ partial, unsigned m, unsigned F,
+                                                                      const uint8_t* __restrict__ X, size_t n,
+                                                                      const float* __restrict__ dZ)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* fold = reinterpret_cast<float*>(smem);                          // [MT*4][FT]
+    uint8_t* xl = smem + (size_t)MT * 4 * FT * sizeof(float);
+    const unsigned nw = blockDim.x >> 6, chunk = nw * WSUBS_W * PSUB;
+    const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned f0 = blockIdx.x * FT, f = f0 + lane;
+    const size_t N = n + m - 1;
+    grad_planes<MT> planes;                                                // [letter][tap] accumulators in fixed registers
+    planes.clear();
+    for (size_t c0 = (size_t)blockIdx.y * chunk; c0 < n; c0 += (size_t)gridDim.y * chunk) {
+        const unsigned rows = (unsigned)((n - c0) < chunk ? (n - c0) : chunk);
+        __syncthreads();
+        stage(xl, X, N, c0, window_span<MT>(rows));
+        __syncthreads();
+        // the next window's gradient rows are requested before this window's additions start
+        float g[PSUB], gn[PSUB];
+        auto fetch = [&](unsigned p0, float (&dst)[PSUB]) {
+#pragma unroll
+            for (int p = 0; p < PSUB; ++p) dst[p] = (f < F && p0 + p < rows) ? dZ[(c0 + p0 + p) * F + f] : 0.0f;
+        };
+        fetch(wave * PSUB, g);
+#pragma unroll 1
+        for (unsigned s = 0; s < WSUBS_W; ++s) {
+            const unsigned p0 = (s * nw + wave) * PSUB;
+            if (p0 >= rows) break;
+            fetch(p0 + nw * PSUB, gn);                                     // all zero past the chunk's rows
+            unsigned wq[window<MT>::words];
+            load_window<MT>(xl, p0, wq);
+            grad_planes_window<MT>(planes, wq, g);                         // one add per (position, tap)
+#pragma unroll
+            for (int p = 0; p < PSUB; ++p) g[p] = gn[p];
+        }
+    }
+    float aw[MT][4];
+    grad_planes_read<MT>(planes, aw);
+    float* mine = fold + lane;
+    for (unsigned w = 0; w < nw; ++w) {
+        __syncthreads();
+        if (wave == w) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+                if ((unsigned)j < m) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        float* cell = mine + (j * 4 + c) * FT;
+                        *cell = w == 0 ? aw[j][c] : *cell + aw[j][c];
+                    }
+                }
+        }
+    }
+    __syncthreads();
+    float* out = partial + (size_t)blockIdx.y * (4 * m) * F;
+    for (unsigned e = threadIdx.x; e < m * 4 * FT; e += blockDim.x) {
+        const unsigned row = e / FT, fl = e % FT;
+        if (f0 + fl < F) out[(size_t)row * F + f0 + fl] = fold[e];
     }
 }
 
@@ -687,6 +755,34 @@ inline int launch_bprop_W_mfma(hipStream_t st, float* dW, size_t m, size_t F, co
     DBK_LAUNCH_OK();
 }
 
+// float32 filters of at most 24 taps: register-resident gradient columns. The float32 products of corr1ord_mm.h go over the rows once per
+// 16 filters; where two such passes over many rows are too few for the split-operand products (32 filters on) they are slower than this
+// kernel's one (us a call, products / this: 20 filters of 8 taps 600 000 rows 78 / 79, 1.0 M 115 / 94, 4.0 M 510 / 242; of 24 taps 1.0 M 142 /
+// 139, 2.0 M 261 / 231), and past the caches so is one pass of 16 filters of few taps (4.0 M x 16 of 8 taps 254 / 232; of 16 taps 280 / 326).
+inline bool bprop_W_window_takes(size_t m, size_t F, size_t n)
+{
+    return m <= 24 && ((F > 16 && F < 32 && n >= 750000) || (F == 16 && m <= 8 && n >= 3500000));
+}
+
+inline int launch_bprop_W_window(hipStream_t st, float* dW, size_t m, size_t F, const uint8_t* X, size_t n, const float* dZ)
+{
+    const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : 24);
+    const unsigned ftiles = dbk::divup(F, FT), chunk = 4 * WSUBS_W * PSUB;
+    const unsigned nchunk = dbk::divup(n, chunk);
+    unsigned gy = (mt == 8 ? 768u : 512u) / ftiles;           // three workgroups fit a CU with 8 taps' register planes, else two
+    if (gy < 1) gy = 1;
+    if (gy > nchunk) gy = nchunk;
+    const size_t nelem = 4 * m * F;
+    float* partial = (float*)dbk::workspace(nelem * gy * sizeof(float), st);
+    DBK_CHECK(partial != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", nelem * gy * sizeof(float), dbk::workspace_error());
+    const size_t smem = (size_t)mt * 4 * FT * sizeof(float) + ((chunk + mt - 1 + 7) & ~(size_t)3);
+    auto kern = mt == 8 ? corr1ord_bprop_W_window_kernel<8> : mt == 16 ? corr1ord_bprop_W_window_kernel<16> : corr1ord_bprop_W_window_kernel<24>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3(ftiles, gy), dim3(256), smem, st, partial, (unsigned)m, (unsigned)F, X, n, dZ);
+    hipLaunchKernelGGL(reduce_partials_kernel<float>, dim3(dbk::ew_grid(nelem)), dim3(256), 0, st, dW, (const float*)partial, nelem, gy);
+    DBK_LAUNCH_OK();
+}
+
 // ---------------------------------------------------------------------------------------------
 // input gradient on the matrix cores (float32, filters of up to 32 taps, bulk sizes)
 // ---------------------------------------------------------------------------------------------
@@ -988,6 +1084,7 @@ int dbk_corr1ord_bprop_W(dbk_stream_t stream, int dtype, void* dW, size_t m, siz
     if (n == 0 || nfilter == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(dW && X && dZ, "ValueError: null pointer argument");
     if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_W_mfma_takes(m, nfilter, n)) return launch_bprop_W_mfma(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
+    if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_W_window_takes(m, nfilter, n)) return launch_bprop_W_window(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F32 && m <= 32) return launch_bprop_W_mm<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F32) return launch_bprop_W<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F64 && m <= 32) return launch_bprop_W_mm<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);

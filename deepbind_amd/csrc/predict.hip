@@ -682,7 +682,7 @@ int dbk_predict_small_takes(size_t m, size_t nmodel, size_t nfilter, size_t N, s
     // 18; 4 taps, 65 217 x 20 nt 94 / 240; 8 taps, 3358 x 60 nt 15 / 26). Where models share a tile, the workgroups that a GPU holds
     // at once, 2048, are the line besides: 16 models of 8 filters of 8 taps, 69 x 60 nt 6.6 / 10.4, 699 x 60 nt 41 / 17; of 4 taps, 4076 x
     // 20 nt 71 / 39. Of 3758 calls of 4 to 64 taps, 20 to 2000 nt, 1 to 64 models of 1 to 16 filters, 37 of those it takes are more than 5 %
-    // slower than the scan kernel + head, by at most 8 us.
+    // slower than the scan kernel + head, by at most 9 us.
     return m >= 1 && m <= 64 && nfilter >= 1 && nfilter <= MUT_F && hidden <= 64 && N * nmodel * m <= 6000000 && nregion < ((size_t)1 << 31) && nmodel <= 65535 &&
            (nmodel == 1 || nregion * nmodel <= 2048) &&
            (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL);

@@ -211,6 +211,12 @@ def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype)
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("N,m,F", [(750030, 24, 17), (750021, 5, 31), (749990, 16, 20)])
+def test_corr1ord_bprop_W_many_rows_of_few_filters(ks, N, m, F):
+    """Either side of the row count from which 17 to 31 filters go through the register-plane kernel."""
+    test_corr1ord_bprop_W(ks, N, m, F, True, np.float32)
+
+
 @pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (208401, 15, 128), (208301, 15, 128)])
 def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
     """Either side of the size from which 128 filters and more go through the split-operand products, and a second launch of few filters."""
