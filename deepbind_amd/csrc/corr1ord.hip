@@ -1008,6 +1008,20 @@ int launch_bprop_W_mm(hipStream_t st, T* dW, size_t m, size_t F, const uint8_t* 
     DBK_LAUNCH_OK();
 }
 
+// Few rows of many filters: the products' workgroups, one per 64 rows, pass over the filters 16 at a time whatever the rows, while the kernel
+// of one wave per row (below) spends its time on the rows it has. The line is where the two measured the same (microseconds: a row's share
+// of 64 filters and a tap against a pass over 16 filters; in float32 a wave's row of many filters costs more than its share). us a call,
+// products / wave per row: float64, 24 taps, 300 rows x 1000 filters 137 / 68, 2000 x 64 11 / 9, 4000 x 64 11 / 16; 4 taps, 4000 x 256
+// 22 / 12; float32, 24 taps, 1000 x 256 26 / 18, 8000 x 256 26 / 39; 32 taps, 300 x 1000 109 / 79.
+template <typename T>
+bool bprop_X_few_rows(size_t m, size_t F, size_t n)
+{
+    const bool f64 = sizeof(T) == 8;
+    const double row = (f64 ? 1.45e-4 : F <= 512 ? 6.5e-5 : 2.3e-4) * (double)m * dbk::divup(F, 64);
+    const double pass = f64 ? 0.95 + 0.047 * (double)m : 0.65 + 0.032 * (double)m;
+    return F > (f64 ? 16 : 32) && row * (double)n < pass * dbk::divup(F, 16);
+}
+
 template <typename T>
 int launch_bprop_X_mm(hipStream_t st, T* dX, size_t n, const T* W, size_t m, size_t F, const T* dZ)
 {
@@ -1100,9 +1114,10 @@ int dbk_corr1ord_bprop_X(dbk_stream_t stream, int dtype, void* dX, size_t n, siz
     if (n == 0 || nfilter == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(dX && W && dZ, "ValueError: null pointer argument");
     if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_X_mfma_takes(m, nfilter, n)) return launch_bprop_X_mfma(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
-    if (dtype == DBK_F32 && m <= 64) return launch_bprop_X_mm<float>(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
+    const bool few = !dbk::exact_scan() && (dtype == DBK_F32 ? bprop_X_few_rows<float>(m, nfilter, n) : bprop_X_few_rows<double>(m, nfilter, n));
+    if (dtype == DBK_F32 && m <= 64 && !few) return launch_bprop_X_mm<float>(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
     if (dtype == DBK_F32) return launch_bprop_X<float>(dbk::as_stream(stream), (float*)dX, n, (const float*)W, m, nfilter, (const float*)dZ);
-    if (dtype == DBK_F64 && m <= 64) return launch_bprop_X_mm<double>(dbk::as_stream(stream), (double*)dX, n, (const double*)W, m, nfilter, (const double*)dZ);
+    if (dtype == DBK_F64 && m <= 64 && !few) return launch_bprop_X_mm<double>(dbk::as_stream(stream), (double*)dX, n, (const double*)W, m, nfilter, (const double*)dZ);
     return launch_bprop_X<double>(dbk::as_stream(stream), (double*)dX, n, (const double*)W, m, nfilter, (const double*)dZ);
 }
 
