@@ -952,7 +952,13 @@ __global__ __launch_bounds__(64 * MB) void corr1ord_bprop_X_mfma_kernel(float* _
 // those, 24 taps): 50 000 rows x 256 filters 96 / 52, 100 000 x 128 52 / 50, 100 000 x 256 98 / 87 (12 taps: 97 / 58), 150 000 x 256
 // 123 / 119, 120 000 x 128 of 32 taps 56 / 62, 250 000 x 128 66 / 80, 250 000 x 256 127 / 150, 500 000 x 256 235 / 305. Its launch costs ~50 us up to
 // ~120 000 rows whatever the taps, so rows x steps of the other kernel decide.
-inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n) { return m <= 32 && F >= 128 && n * (m + 3) >= 3750000; }
+// (Filters that do not fill a launch of 128 take unaligned loads: 113 to 127 pay only at two blocks of eight taps, and until a workgroup
+// gets more than its 1024 rows: 127 of 16 taps, 250 000 rows 61 / 74, 400 000 88 / 117, 600 000 219 / 165; of 24 taps 400 000 160 / 144.)
+inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n)
+{
+    if (F > 112 && F < 128) return m > 12 && m <= 16 && n >= 230000 && n <= 512 * 1024;
+    return m <= 32 && F >= 128 && n * (m + 3) >= 3750000;
+}
 
 inline int launch_bprop_X_mfma(hipStream_t st, float* dX, size_t n, const float* W, size_t m, size_t F, const float* dZ)
 {

@@ -217,7 +217,7 @@ def test_corr1ord_bprop_W_many_rows_of_few_filters(ks, N, m, F):
     test_corr1ord_bprop_W(ks, N, m, F, True, np.float32)
 
 
-@pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (208401, 15, 128), (208301, 15, 128)])
+@pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (208401, 15, 128), (208301, 15, 128), (240001, 16, 127), (229999, 13, 113)])
 def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
     """Either side of the size from which 128 filters and more go through the split-operand products, and a second launch of few filters."""
     test_corr1ord_bprop_X(ks, n, m, F, np.float32)
