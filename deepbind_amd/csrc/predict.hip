@@ -723,7 +723,7 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     DBK_CHECK(dbk_mutation_map_takes(m, nfilter, ptype, hidden), "NotImplementedError: the mutation map kernel does not take %zu filters of %zu taps with %zu hidden units and pooling %d",
               nfilter, m, hidden, ptype);
     if (nregion == 0) { dbk::clear_error(); return 0; }
-    DBK_CHECK(W && bias && X && regions && W1 && b1 && Z && map, "ValueError: null pointer argument");
+    DBK_CHECK(W && bias && X && regions && W1 && b1 && Z && (longest == 0 || map), "ValueError: null pointer argument");
     DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
     // letters per workgroup: 16 where that still gives every CU several workgroups, else fewer, as a workgroup's first scan of
     // its region costs less than an idle CU (64 regions of up to 101 letters: 159 us a call with 4, 179 with 16; 256 of 101: 312 / 288)

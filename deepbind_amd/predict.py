@@ -192,8 +192,9 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
             gmaps += [(s, dXh[a + pad:b].copy()) for s, (a, b) in zip(text.strings(), Rh[::2] if rc else Rh)]
             continue
         maps = torch.empty((len(text.bytes), 4), dtype=dX.dtype, device=dX.device)
-        _lib.call("dbk_gather_maps", _lib.stream(), _lib.dtype_code(dX), _lib.ptr(R), R.shape[0], pad, 2 if rc else 1, _lib.ptr(Zall),
-                  _lib.ptr(dX), _lib.ptr(maps))
+        if len(text.bytes):                  # (a batch of empty sequences has no letter to gather for, and no memory for them)
+            _lib.call("dbk_gather_maps", _lib.stream(), _lib.dtype_code(dX), _lib.ptr(R), R.shape[0], pad, 2 if rc else 1, _lib.ptr(Zall),
+                      _lib.ptr(dX), _lib.ptr(maps))
         pairs = Zmask.reshape(-1, 2) if Zmask is not None else None
         new = zip(text.strings(None if pairs is None else pairs[:, 1]), _split(maps.cpu().numpy(), text))
         gmaps += new if pairs is None else [gmap for gmap, keep in zip(new, pairs.any(axis=1)) if keep]

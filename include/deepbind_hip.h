@@ -439,7 +439,7 @@ int dbk_predict_small(dbk_stream_t stream, const float* W, const float* bias, si
 /* Scores and mutation maps of one model: Z (nregion / strands) the net's outputs (with strands = 2 the larger of each
  * pair's), map (letters of all sequences, 4): output with that letter changed to that base, minus the output, where the
  * larger of the two is positive, else 0. X, regions as dbk_pack_text lays them out for padding = m - 1; longest: the longest
- * sequence's letters. Weights as in dbk_head_fprop with nblock = 1 and no feature columns. Entries of a sequence shorter than
+ * sequence's letters (0: map may be null). Weights as in dbk_head_fprop with nblock = 1 and no feature columns. Entries of a sequence shorter than
  * the one before it see the reference's spill of that one's changes into the pad between them.
  * dbk_mutation_map_takes: 1 for shapes the kernel takes. reference: kangaroo/kangaroo/predict.py:201-240. */
 int dbk_mutation_map_takes(size_t m, size_t nfilter, int ptype, size_t hidden);

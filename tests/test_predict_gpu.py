@@ -208,6 +208,24 @@ def test_gradient_map_kernel_edges(pool, hidden, loss, rc, rate, m, F):
         assert sa == sb and (len(b) == 0 or np.abs(a - b).max() <= GRAD * scale)
 
 
+@pytest.mark.parametrize("mode", [True, "finite_diff"])
+@pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("pool,m,F", [("max", 8, 4), ("all", 24, 17), ("avg", 2, 16)])
+def test_batches_of_empty_sequences(pool, m, F, rc, mode):
+    """No letter in a whole batch - alone, and as what a longer list ends in: scored, with empty maps; by the map kernels and by the layers
+    (more than 16 filters have no gradient map kernel)."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(m + F)
+    p = _params(rng, m, F, pool, 5)
+    net = _net(p, m, F, pool, 5, "nll", rc, 0.0)
+    p64 = {k: v.astype(np.float64) for k, v in p.items()}
+    for seqs, batch in (([""], 2048), (["", ""], 2048), (["ACGT", "GATTACA", ""], 2)):
+        Z, maps = predict.gen_predictions(net, seqs, want_gmaps=mode, batchsize=batch)
+        Zr = np.vstack([orc.gen_predictions(p64, [s], pool, 5, "logistic", reverse_complement=rc, want_gmaps=False)[0] for s in seqs])
+        assert_close(Z, Zr, ACT, "Z")
+        assert [g.shape for _, g in maps] == [(len(s), 4) for s in seqs] and maps[-1][0] == ""
+
+
 @pytest.mark.parametrize("which", ["b2", "W1"])
 def test_pairs_whose_scores_do_not_compare(which, monkeypatch):
     """Scores that are not a number - of every strand, or only of strands on which one filter never fires - select neither row of a

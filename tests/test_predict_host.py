@@ -52,6 +52,17 @@ def test_tensors_live_until_the_call_that_reads_them(calls, rc):
     assert calls == ["dbk_gradient_map", "dbk_pack_text", "dbk_mutation_map", "dbk_pack_windows"]
 
 
+def test_batches_of_empty_sequences_gather_nothing(calls):
+    """A tensor of no elements has no address: what is asked of the library for a batch without a letter names none of them, or takes null."""
+    net = _net(nfilter=17, reverse_complement=True)
+    net.input_gradients = lambda X, R: (torch.ones(R.shape[0], 1), torch.zeros(X.numel(), 4))
+    Z, maps = predict.gen_predictions(net, ["", ""], want_gmaps=True)
+    assert calls == ["dbk_pack_text"] and [(s, g.shape) for s, g in maps] == [("", (0, 4))] * 2
+    lib, one = _lib.dll(), 1                                       # (a null map is refused where there are letters for it)
+    assert lib.dbk_mutation_map(None, one, one, 4, 2, one, 10, one, 1, 4, 0, 0, one, one, None, None, None, 0, 1, one, None) != 0
+    assert b"null pointer" in lib.dbk_last_error()
+
+
 @pytest.mark.parametrize("mode", [False, True, "finite_diff"])
 def test_what_is_no_sequence_is_refused(calls, mode):
     """A number is no sequence (bytes(5) would make five letters of it), nor a list of numbers; bytes are one where no reverse complement
