@@ -68,7 +68,7 @@ class SequenceNet(object):
         self._step_bufs = {}                 # per batch shape: the step's work buffers, views of the vectors below
         self._step_store = {}                # one growing vector per work buffer, shared by all batch shapes
         self._works = []                     # single-launch workspaces: [tensor, steps issued on it]; the last one is in use
-        self._step_sig, self._step_buf, self._step_nesterov = None, None, None
+        self._step_sig, self._step_buf, self._step_switches = None, None, None
         # Nesterov look-ahead kept beside the parameters by the natively issued step (each step's update kernel
         # leaves the next step's look-ahead there); valid while nothing else has touched P, mP or mrate
         self._L, self._L_versions = None, None
@@ -550,7 +550,7 @@ class SequenceNet(object):
         # the same batch tensors as in the previous step (a training loop over resident batches): only the switches move
         sig = (X.data_ptr(), X.numel(), R.data_ptr(), R.shape[0], R._version, Y.data_ptr(), Y.numel(),
                None if Ymask is None else Ymask.data_ptr(), None if F is None else F.data_ptr(), None if cols is None else cols.data_ptr())
-        if a is not None and sig == self._step_sig and not self.nesterov_changed():
+        if a is not None and sig == self._step_sig and self._step_switches == self._switches():
             if self.nesterov:
                 versions = (self.P._version, self.mP._version, self.mrate._version)
                 a.L_ready = int(self._L_versions == versions)
@@ -578,10 +578,9 @@ class SequenceNet(object):
             a.off_W2, a.off_b2 = off.get("W2", 0), off.get("b2", 0)
             a.rate = self.dropout.data_ptr() if self.use_dropout else None
             a.counter = self.rng_counter.data_ptr()
-            a.input_rate = self.input_dropout
             a.loss = None
         buf = self._step_buffers(X.numel(), P)
-        a.nesterov, a.seed = int(bool(self.nesterov)), int(self.rng_seed)
+        a.nesterov, a.seed, a.input_rate = int(bool(self.nesterov)), int(self.rng_seed), self.input_dropout
         if self.nesterov:
             if self._L is None:
                 self._L = torch.empty_like(self.P)
@@ -604,7 +603,7 @@ class SequenceNet(object):
             setattr(a, name, None if t is None else t.data_ptr())
         a.decay = self.decay_vec.data_ptr() if self.weight_decay_start <= self.step_count else None
         a.freeze_scan = int(self.step_count < self.start_training)
-        self._step_sig, self._step_buf, self._step_nesterov = sig, buf, (bool(self.nesterov), int(self.rng_seed))
+        self._step_sig, self._step_buf, self._step_switches = sig, buf, self._switches()
         return buf
 
     _STEP_BUFFERS = ("pooled", "dpooled", "argmax", "Z", "act", "Xdrop", "Mdrop")
@@ -613,8 +612,9 @@ class SequenceNet(object):
         """The step's work buffers for a batch of N letters and P regions: views of vectors that grow with the largest batch,
         so that an epoch of ragged minibatches allocates nothing once it has seen its largest one. (A captured graph keeps
         the views it was captured with, and through them the memory.)"""
+        drops = self.input_dropout > 0
         buf = self._step_bufs.get((N, P))
-        if buf is not None:
+        if buf is not None and (buf["Xdrop"] is not None or not drops):
             return buf
         if len(self._step_bufs) >= 64:
             self._step_bufs.clear()
@@ -625,7 +625,7 @@ class SequenceNet(object):
             wanted.append(("argmax", P, F, ks.uindex))
         if self.pool != "max":
             wanted.append(("act", N, words, torch.int64))
-        if self.input_dropout > 0:
+        if drops:
             wanted += [("Xdrop", N, 0, torch.uint8), ("Mdrop", N, 0, torch.bool)]
         buf = dict.fromkeys(self._STEP_BUFFERS)
         for name, rows, cols, dtype in wanted:
@@ -639,8 +639,9 @@ class SequenceNet(object):
         self._step_bufs[N, P] = buf
         return buf
 
-    def nesterov_changed(self):
-        return self._step_nesterov != (bool(self.nesterov), int(self.rng_seed))
+    def _switches(self):
+        """What a program may change between two steps on the same batch, as the argument block holds it."""
+        return bool(self.nesterov), int(self.rng_seed), float(self.input_dropout)
 
     def _finish_step(self, X, R):
         """Host-side mirrors of what a natively issued step moved on the device."""
