@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict_
 // of one region: it scans the region once (16 lanes of filters x 16 lanes of rows, the letter table of 16 filters in
 // LDS), keeps the maximum and the sum of the rows no change of its letters can reach and, one by one, the rows some change
 // can; a wave then takes a letter at a time, its lanes being 4 new letters x 16 filters, scans the m rows of each anew -
-// taps in ascending order, as the forward pass does, so that a change to the letter that is there gives the score that is
-// there - and pools them with what is kept. More than 16 filters take further passes; pooled values meet the dense head in LDS.
+// taps in ascending order, as the forward pass does - and pools them with what is kept. (Rows of a mean are added in an order that depends on
+// where the workgroup's letters lie, so the score of the letter that is there comes from k_mutation_map.) More than 16 filters take further passes; pooled values meet the dense head in LDS.
 // What bounds it is LDS reads, one per (row, tap): m * m per letter and filter tile, where the reference's way (a pass of the
 // whole net per change) scans length + m - 1 rows per change, and launches 15 kernels for it.
 // Measured: 32 sequences of 60-101 letters, both strands, 16 filters of 24 taps: 0.047 ms, the whole call
@@ -152,6 +152,13 @@ inline size_t mut_smem(unsigned pos, size_t m, size_t k)
            mut_tile_letters((unsigned)m) + mut_reach_letters(pos, (unsigned)m) + mut_reach_letters(0, (unsigned)m);
 }
 
+// Pass `pass` of the reference changes letter `pass` of every region: whether what it does to the region [pa, pb) before this one (none: !before)
+// lands at stream position pad + pa + pass in the leading pad of this one, which begins at ra.
+__device__ __forceinline__ bool spilled_pass(unsigned pass, unsigned pad, bool before, unsigned pa, unsigned pb, unsigned ra)
+{
+    return before && pb - pa > pass && pad + pa + pass >= pb && pad + pa + pass < ra + pad;
+}
+
 template <unsigned MUT_POS>
 __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
 {
@@ -183,8 +190,7 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
     // the change of the region before this one that lands in this one's leading pad
     const bool shorter_before = a.strands == 1 && r > 0;
     const unsigned pa = shorter_before ? a.R[2 * r - 2] : 0u, pb = shorter_before ? a.R[2 * r - 1] : 0u;
-    // (pass `i` of the reference: letter i of every region, i.e. stream position pad + pa + i of that one)
-    auto spills = [&](unsigned pass) { return shorter_before && pb - pa > pass && pad + pa + pass >= pb && pad + pa + pass < ra + pad; };
+    auto spills = [&](unsigned pass) { return spilled_pass(pass, pad, shorter_before, pa, pb, ra); };
     bool spill_here = false;
     for (unsigned i = 0; i < npos; ++i) spill_here |= spills(i0 + i);
     // rows of the head that no change of these letters reaches: with a spill they are kept one by one as well
@@ -605,9 +611,11 @@ __global__ __launch_bounds__(256) void k_gradient_map(const grad_args a)
 }
 
 // The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
-// is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. One workgroup per sequence.
-__global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const float* __restrict__ S,
-                                                      const float* __restrict__ base, float* __restrict__ Z, float* __restrict__ map)
+// is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. The letter that is there is no change: its score
+// is the score, whatever order the workgroup that formed the changed one added its rows in. One workgroup per sequence.
+__global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const uint8_t* __restrict__ X,
+                                                      const float* __restrict__ S, const float* __restrict__ base, float* __restrict__ Z,
+                                                      float* __restrict__ map)
 {
     const size_t s = blockIdx.x, r = s * (unsigned)strands;
     const unsigned ra = R[2 * r], len = R[2 * r + 1] - ra - pad;
@@ -615,6 +623,8 @@ __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict
     float z = base[r];
     if (strands == 2) z = base[r + 1] > z ? base[r + 1] : z;
     const unsigned mirror = strands == 2 ? R[2 * r + 3] - 1 : 0u;
+    const bool before = strands == 1 && r > 0;
+    const unsigned pa = before ? R[2 * r - 2] : 0u, pb = before ? R[2 * r - 1] : 0u;
     for (unsigned e = threadIdx.x; e < 4 * len; e += blockDim.x) {
         const unsigned i = e >> 2, c = e & 3u;
         float v = S[4 * ((size_t)ra + pad + i) + c];
@@ -622,6 +632,7 @@ __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict
             const float w = S[4 * (size_t)(mirror - i) + 3 - c];
             v = w > v ? w : v;
         }
+        if (X[(size_t)ra + pad + i] == c && !spilled_pass(i, pad, before, pa, pb, ra)) v = z;
         // (a product with 1 or 0, so that scores that are infinite or not a number show)
         const float d = v - z;
         map[4 * out + e] = (z > v ? z : v) > 0.0f ? d : v == v && z == z ? d * 0.0f : d;
@@ -742,7 +753,7 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     a.S = scratch; a.base = scratch + 4 * N;
     auto kern = pos == 16 ? k_mutation_scores<16> : (pos == 8 ? k_mutation_scores<8> : k_mutation_scores<4>);
     hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(256), mut_smem(pos, m, a.k), st, a);
-    hipLaunchKernelGGL(k_mutation_map, dim3((unsigned)(nregion / strands)), dim3(256), 0, st, regions, (unsigned)(m - 1), strands,
+    hipLaunchKernelGGL(k_mutation_map, dim3((unsigned)(nregion / strands)), dim3(256), 0, st, regions, (unsigned)(m - 1), strands, X,
                        (const float*)a.S, (const float*)a.base, Z, map);
     DBK_LAUNCH_OK();
 }

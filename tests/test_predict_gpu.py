@@ -122,6 +122,22 @@ def test_mutation_map_kernel_edges(pool, hidden, loss, rc, m, F):
 
 
 @pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("pool,hidden,m,F", [("avg", 6, 24, 16), ("all", 0, 9, 33), ("max", 5, 16, 16), ("avg", 0, 1, 4)])
+def test_mutation_to_the_letter_that_is_there_is_none(pool, hidden, m, F, rc):
+    """Exactly zero at every sequence's own letters, wherever in the sequence the workgroup that scores them begins. (Longer sequences
+    first: a shorter one before would have its changes spill into the next.)"""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(3 * m + F)
+    net = _net(_params(rng, m, F, pool, hidden), m, F, pool, hidden, "nll", rc, 0.0)
+    seqs = ["".join("ACGT"[v] for v in rng.integers(0, 4, n)) for n in (131, 90, 90, 37, 2)]
+    _, maps = predict.gen_predictions(net, seqs, want_gmaps="finite_diff")
+    for s, (letters, g) in zip(seqs, maps):
+        own = ["ACGT".index(ch) for ch in s]
+        assert letters == s and (g[np.arange(len(s)), own] == 0).all()
+    assert any((g != 0).any() for _, g in maps)
+
+
+@pytest.mark.parametrize("rc", [False, True])
 @pytest.mark.parametrize("m,window,stride", [(1, 2, 1), (24, 20, 3), (8, 65, 7)])
 def test_text_and_windows_are_packed_as_on_the_host(rc, m, window, stride):
     from deepbind_amd import _lib, data, predict
