@@ -1375,7 +1375,8 @@ def test_poolrgn_packed_and_plain_columns_agree(ks, F):
         assert torch.equal(dUa, dUb), ptype
 
 
-@pytest.mark.parametrize("n,m,dtype", [(4096, 1, np.float32), (4099, 2, np.float64), (70003, 16, np.float32), (5001, 32, np.float64)])
+@pytest.mark.parametrize("n,m,dtype", [(4096, 1, np.float32), (4099, 2, np.float64), (70003, 16, np.float32), (5001, 32, np.float64),
+                                         (16383, 1, np.float64), (16447, 1, np.float32)])
 def test_column_sums_of_few_columns(sm, n, m, dtype):
     """Several rows side by side in the 64 lanes, with and without rows left over."""
     test_column_sums(sm, n, m, dtype)
