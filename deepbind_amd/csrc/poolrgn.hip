@@ -381,8 +381,11 @@ int launch_fwd(hipStream_t st, const T* U, size_t F, const uint32_t* R, size_t P
         const dim3 grid(dbk::divup(P * (F / (16 / sizeof(T))), 256)), block(256);
         const unsigned F32 = (unsigned)F, P32 = (unsigned)P;
         const size_t items = P * (F / (16 / sizeof(T)));
-        if (ptype == DBK_PT_MAX && items <= 131072) {               // (fewer than eight waves per SIMD with a lane per item)
-            if (items <= 32768)
+        // Too few items to fill the GPU with a lane each. The regions' lengths are only known on the device: the lines lie where regions of a
+        // few rows are no slower either (us, lane per item / this; 16 lanes per item: 16 000 items of 12 rows 4.0 / 4.0, of 124 34 / 10, but
+        // 32 000 of 12 rows 3.9 / 5.1; four: 64 000 of 12 rows 4.2 / 4.1, 100 000 of 124 50 / 40, but 130 000 of 12 rows 4.4 / 5.5).
+        if (ptype == DBK_PT_MAX && items <= 98304) {
+            if (items <= 16384)
                 hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 16>), dim3(dbk::divup(items, 16)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
             else
                 hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 4>), dim3(dbk::divup(items, 64)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
