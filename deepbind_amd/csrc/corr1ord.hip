@@ -761,7 +761,19 @@ inline int launch_bprop_W_mfma(hipStream_t st, float* dW, size_t m, size_t F, co
 // 139, 2.0 M 261 / 231), and past the caches so is one pass of 16 filters of few taps (4.0 M x 16 of 8 taps 254 / 232; of 16 taps 280 / 326).
 inline bool bprop_W_window_takes(size_t m, size_t F, size_t n)
 {
-    return m <= 24 && ((F > 16 && F < 32 && n >= 750000) || (F == 16 && m <= 8 && n >= 3500000));
+    return m <= 24 && ((F > 16 && F < 32 && n >= 750000) || (F == 16 && m <= 8 && n >= 3500000)
+                       // one to four taps, just below the split-operand products (their tiles hold eight): 28 000 x 100 of one tap 20.1 / 18.1,
+                       // 80 000 x 48 25.1 / 23.1; 64 filters of three and four taps 1 to 5 % the other way
+                       || (m <= 4 && F > 32 && F < 128 && F % 64 != 0 && n * F >= 2800000));
+}
+
+// The float64 products' smallest tile is eight taps by 16 filters: of one to three taps over many gradient values most of it is padding, and the
+// any-length kernel, one pass for 64 filters, is the better one. us a call, products / that kernel: one tap, 57 000 rows x 1000 filters
+// 286 / 121, 28 000 x 1000 115 / 76, 14 000 x 1000 61 / 67, 221 000 x 128 111 / 96; three, 49 000 x 1000
+// 245 / 148; four taps never below 57 M values.
+inline bool bprop_W_few_taps(size_t m, size_t F, size_t n)
+{
+    return m <= 3 && F > 32 && (double)n * (double)F >= (9e6 + 6e6 * (double)m) * (F > 256 ? 1.0 : F >= 100 ? 1.35 : 1.9);
 }
 
 inline int launch_bprop_W_window(hipStream_t st, float* dW, size_t m, size_t F, const uint8_t* X, size_t n, const float* dZ)
@@ -1107,7 +1119,7 @@ int dbk_corr1ord_bprop_W(dbk_stream_t stream, int dtype, void* dW, size_t m, siz
     if (dtype == DBK_F32 && !dbk::exact_scan() && bprop_W_window_takes(m, nfilter, n)) return launch_bprop_W_window(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F32 && m <= 32) return launch_bprop_W_mm<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
     if (dtype == DBK_F32) return launch_bprop_W<float>(dbk::as_stream(stream), (float*)dW, m, nfilter, X, n, (const float*)dZ);
-    if (dtype == DBK_F64 && m <= 32) return launch_bprop_W_mm<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);
+    if (dtype == DBK_F64 && m <= 32 && (dbk::exact_scan() || !bprop_W_few_taps(m, nfilter, n))) return launch_bprop_W_mm<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);
     return launch_bprop_W<double>(dbk::as_stream(stream), (double*)dW, m, nfilter, X, n, (const double*)dZ);
 }
 

@@ -217,6 +217,13 @@ def test_corr1ord_bprop_W_many_rows_of_few_filters(ks, N, m, F):
     test_corr1ord_bprop_W(ks, N, m, F, True, np.float32)
 
 
+@pytest.mark.parametrize("N,m,F,dtype", [(15010, 1, 1000, np.float64), (14990, 1, 1000, np.float64), (283600, 2, 100, np.float64), (283400, 2, 100, np.float64),
+                                         (27005, 3, 1000, np.float64), (58340, 1, 48, np.float32), (58330, 1, 48, np.float32), (28010, 4, 100, np.float32)])
+def test_corr1ord_bprop_W_few_taps(ks, N, m, F, dtype):
+    """Either side of the gradient values from which filters of a few taps go through the kernels without padding."""
+    test_corr1ord_bprop_W(ks, N, m, F, True, dtype)
+
+
 @pytest.mark.parametrize("n,m,F", [(117150, 32, 130), (208401, 15, 128), (208301, 15, 128), (240001, 16, 127), (229999, 13, 113)])
 def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
     """Either side of the size from which 128 filters and more go through the split-operand products, and a second launch of few filters."""
