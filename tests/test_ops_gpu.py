@@ -308,6 +308,35 @@ def test_poolrgn_step_and_overlapping_regions(ks):
         assert_close(host(dU), ref, GRAD, "dU " + ptype)
 
 
+@pytest.mark.parametrize("dtype,P,F,stepped", [(np.float32, 17000, 64, False), (np.float32, 5500, 200, True), (np.float64, 9000, 64, True)])
+def test_poolrgn_bprop_all_of_many_packs(ks, dtype, P, F, stepped):
+    """Max + average pooling from 262 144 packs on, where the maximum's share goes in as its row passes: regions of 1 to 20 rows (around
+    the eight of a round), with and without a step column of ones, some maxima in rows of no region. Whole numbers, so that any order of
+    the additions gives the oracle's bits; then normal ones, whose order is that of the kernel that takes maps off a 16-byte boundary."""
+    assert P * F * np.dtype(dtype).itemsize // 16 >= 262144
+    rng = np.random.default_rng(P + F)
+    R, N = _regions(rng, P, 1, 20, gap=1)
+    lens = (R[:, 1] - R[:, 0]).astype(np.int64)
+    Rk = np.concatenate([R, np.ones((P, 1), np.uint32)], axis=1) if stepped else R
+    own = (R[:, :1] + rng.integers(0, lens[:, None], (P, F))) * np.int64(F) + np.arange(F)
+    I = np.where(rng.random((P, F)) < 0.02, R[:, 1:].astype(np.int64) * F + np.arange(F), own).astype(np.uint32)
+    dP = rng.integers(-9, 10, (P, 2 * F)).astype(dtype)
+    dP[:, 1::2] *= lens[:, None]
+    ref = rng.integers(-9, 10, (N, F)).astype(dtype)
+    dU = dev(ref)
+    orc.poolrgn_bprop(ref, Rk, dP, I, "all")
+    ks.poolrgn_bprop(dU, dev(Rk), dev(dP), dev(I), "all")
+    assert np.array_equal(host(dU), ref)
+    start, dPn, Id = rng.standard_normal((N, F)).astype(dtype), dev(rng.standard_normal((P, 2 * F)).astype(dtype)), dev(own.astype(np.uint32))
+    out = []
+    for shift in (0, 1):
+        dU = torch.empty(N * F + 1, dtype=dPn.dtype, device="cuda")[shift:shift + N * F].view(N, F)
+        dU.copy_(dev(start))
+        ks.poolrgn_bprop(dU, dev(Rk), dPn, Id, "all")
+        out.append(host(dU))
+    assert np.array_equal(out[0], out[1])
+
+
 # ------------------------------------------------------------------------------------------ fused scan + pool
 def _chain_oracle(W, b, X, R, ptype):
     Z = np.zeros((X.size, W.shape[1]), W.dtype)
