@@ -43,8 +43,12 @@ int dbk_device_count(void);
 /* on != 0: from now on dbk_corr1ord, dbk_corr1ord_bprop_W and dbk_corr1ord_bprop_X keep to one kernel
  * at EVERY size, so that a row's result does not depend on the size of the batch it arrives in: dbk_corr1ord
  * then adds the taps in the reference's order (corr1ord.cuh:139-157: its bits) for any number of rows, and the two
- * gradients keep one summation order. Off (the default) float32 calls switch to the split-operand matrix-core kernels at bulk sizes
- * (2^25 map values for the forward, 2^22 for the filter gradient, ~140 000 rows for the input gradient): the same sums in another order, 1.5-2x faster.
+ * gradients keep one summation order. Off (the default) the same sums may come in another order where another kernel is the faster one:
+ * float32 calls on the split-operand matrix-core kernels at bulk sizes (2^25 map values for the forward, 2^22 for the filter gradient, 3.75 M
+ * rows x (taps + 3) of 128 filters and more for the input gradient, 230 000 rows of 113 to 127 filters of 13 to 16 taps); filter gradients of
+ * either type on vector kernels where the products would be mostly padding (many rows of 17 to 31 filters or of up to four taps); and input
+ * gradients of either type with four waves to 64 rows below 131 072 (float32) or 262 144 (float64) rows and a wave per row where few rows meet
+ * many filters.
  * Process-wide; returns the previous setting. No counterpart in the reference (it has one kernel per operator). */
 int dbk_set_exact_scan(int on);
 /* Blocks until `stream` has drained. reference: api_sync, smat_cuda/cuda_context.cpp:198-202 */

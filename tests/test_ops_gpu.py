@@ -93,6 +93,29 @@ def test_exact_scan_switch_keeps_the_reference_bits_at_bulk_sizes(ks):
     assert_close(grads["dW"], dWr, GRAD, "dW with the switch on vs the oracle")
 
 
+@pytest.mark.parametrize("n,m,F,dtype", [(131073 + 500, 9, 20, np.float32), (125100, 27, 130, np.float32), (262145 + 500, 9, 20, np.float64)])
+def test_exact_scan_switch_keeps_input_gradient_rows_the_same_in_calls_of_any_size(ks, n, m, F, dtype):
+    """Rows of a bulk call - beyond the sizes from which 256 rows go to a workgroup instead of 64, and from which the split-operand products
+    would take them - have the bits that small calls of the same rows give them, wherever in the bulk call they lie."""
+    rng = np.random.default_rng(n)
+    Wd, dZ = dev((rng.standard_normal((4 * m, F)) * 0.1).astype(dtype)), dev(rng.standard_normal((n, F)).astype(dtype))
+
+    def rows(part):
+        out = torch.zeros((part.shape[0], 4), dtype=part.dtype, device="cuda")
+        ks.corr1ord_bprop_X(out, Wd, part, 4)
+        return host(out)
+
+    assert ks.set_exact_scan(True) is False
+    try:
+        bulk = rows(dZ)
+        for first, count in ((0, 1), (0, 63), (0, 3000), (77001, 300), (n - 130, 130)):
+            lead = min(first, m - 1)                                # the rows before, which the first ones' sums reach
+            assert np.array_equal(rows(dZ[first - lead:first + count].contiguous())[lead:], bulk[first:first + count]), (first, count)
+    finally:
+        assert ks.set_exact_scan(False) is True
+    assert_close(rows(dZ), bulk.astype(np.float64), GRAD if dtype == np.float32 else 1e-12, "dX, default path")
+
+
 @pytest.mark.parametrize("N,m,F", [(300000, 24, 128), (600001, 11, 70), (1100000, 32, 32)])
 def test_corr1ord_bulk_sizes_on_the_matrix_cores(ks, N, m, F):
     """From 2^25 map values on, float32 maps come from the matrix-core kernel: the same sums in another order, so the
