@@ -248,20 +248,26 @@ def test_pairs_whose_scores_do_not_compare(which, monkeypatch):
     pair: such sequences have no entry among the predictions or the maps, by the one-workgroup kernel as by the layers."""
     from deepbind_amd import predict
     rng = np.random.default_rng(5)
-    p = _params(rng, 8, 4, "max", 8)
+    hidden = 8 if which == "b2" else 0                  # (a hidden unit's rectifier would take such a value for zero)
+    p = _params(rng, 8, 4, "max", hidden)
     if which == "b2":
         p["b2"][:] = np.nan
     else:
         p["W1"][0, 0] = np.inf                          # 0 x inf where filter 0 stays at zero
         p["bc"][0, 0] = -2.0
     seqs = _seqs(rng, 40, 10, 14, 0.0)
-    net = _net(p, 8, 4, "max", 8, "nll", True, 0.0)
+    net = _net(p, 8, 4, "max", hidden, "nll", True, 0.0)
     Z, maps = predict.gen_predictions(net, seqs, want_gmaps=True)
     monkeypatch.setattr(predict, "_gradient_maps", lambda *a: None)
     Zr, ref = predict.gen_predictions(net, seqs, want_gmaps=True)
     monkeypatch.undo()
-    assert len(maps) == len(Z) == len(Zr) == len(ref) < len(seqs) or which == "W1"
+    assert len(maps) == len(Z) == len(Zr) == len(ref)
+    assert (len(maps) == 0) if which == "b2" else (0 < len(maps) < len(seqs))
     assert [s for s, _ in maps] == [s for s, _ in ref] and np.allclose(Z, Zr, atol=1e-6, equal_nan=True)
+    scale = max([np.abs(b[np.isfinite(b)]).max(initial=0.0) for _, b in ref], default=0.0)
+    for (_, a), (_, b) in zip(maps, ref):
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[np.isinf(a)], b[np.isinf(b)])
+        assert np.abs(a - b)[np.isfinite(a) & np.isfinite(b)].max(initial=0.0) <= GRAD * scale
 
 
 def test_feature_columns_and_wide_targets():
