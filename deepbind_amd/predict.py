@@ -161,7 +161,9 @@ def gen_predictions(net, seqs, want_gmaps=False, batchsize=2048):
     Returns (predictions (nseq, 1) float32, gmaps). gmaps is None, or a list of
     (sequence string, (len, 4) float32 map): with want_gmaps=True the back-propagated input
     gradient (with reverse complements only the winning strand's entry, whose string is that
-    strand's), with want_gmaps="finite_diff" the mutation map of the forward strand.
+    strand's), with want_gmaps="finite_diff" the mutation map of the forward strand. The maps of one
+    batch are disjoint parts of one array, written to by nobody else: a program that keeps a few maps of
+    many for long copies those, or it keeps their whole batch (up to `batchsize` sequences).
     (reference: predict.py:168-260)"""
     assert net.ninst == 1, "prediction maps are defined for one model at a time"
     rc, pad = net.reverse_complement, net.m - 1
