@@ -222,7 +222,10 @@ class SequenceNet(object):
         workspace, changed nothing (parameters, momentum, generator position), so the host's step counter and
         generator mirror are set back to what the device actually did, and the workspace's header is zeroed so that
         the next step runs again."""
-        for entry in self._works:
+        own = [w for w, _ in self._works]
+        entries = self._works + [[buf["work"], buf.get("issued", 0)] for buf in self._step_bufs.values()
+                                 if buf.get("work") is not None and not any(buf["work"] is w for w in own)]
+        for entry in entries:
             work, issued = entry
             torch.cuda.synchronize()
             stepped, status = (int(v) for v in work[0:8].view(torch.int32).tolist())
