@@ -223,7 +223,8 @@ class SequenceNet(object):
         generator mirror are set back to what the device actually did, and the workspace's header is zeroed so that
         the next step runs again."""
         own = [w for w, _ in self._works]
-        entries = self._works + [[buf["work"], buf.get("issued", 0)] for buf in self._step_bufs.values()
+        # (a workspace that a program put beside a batch's buffers itself is looked at too; what it issued there was not counted)
+        entries = self._works + [[buf["work"], 0] for buf in self._step_bufs.values()
                                  if buf.get("work") is not None and not any(buf["work"] is w for w in own)]
         for entry in entries:
             work, issued = entry
