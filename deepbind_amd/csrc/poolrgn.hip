@@ -382,11 +382,14 @@ int launch_fwd(hipStream_t st, const T* U, size_t F, const uint32_t* R, size_t P
         const unsigned F32 = (unsigned)F, P32 = (unsigned)P;
         const size_t items = P * (F / (16 / sizeof(T)));
         // Too few items to fill the GPU with a lane each. The regions' lengths are only known on the device: the lines lie where regions of a
-        // few rows are no slower either (us, lane per item / this; 16 lanes per item: 16 000 items of 12 rows 4.0 / 4.0, of 124 34 / 10, but
-        // 32 000 of 12 rows 3.9 / 5.1; four: 64 000 of 12 rows 4.2 / 4.1, 100 000 of 124 50 / 40, but 130 000 of 12 rows 4.4 / 5.5).
+        // few rows are no slower either. us, lane per item / this, for regions of 12 and of 124 rows: 16 000 items, 16 lanes each, 4.0 / 4.0
+        // and 34 / 10 (at 32 000 items 3.9 / 5.1 and 35 / 17); 32 000, eight lanes, 4.0 / 3.9 and 35 / 13.6; 64 000, four, 4.2 / 4.1 and
+        // 24 / 12 (at 130 000 4.4 / 5.5 for 12 rows).
         if (ptype == DBK_PT_MAX && items <= 98304) {
             if (items <= 16384)
                 hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 16>), dim3(dbk::divup(items, 16)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
+            else if (items <= 32768)
+                hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 8>), dim3(dbk::divup(items, 32)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
             else
                 hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 4>), dim3(dbk::divup(items, 64)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
             DBK_LAUNCH_OK();

@@ -1442,9 +1442,9 @@ def test_column_sums_of_few_columns(sm, n, m, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("P,F,step", [(37, 16, False), (501, 8, True), (9001, 16, False), (2, 64, True)])
+@pytest.mark.parametrize("P,F,step", [(37, 16, False), (501, 8, True), (9001, 16, False), (2, 64, True), (6001, 16, False), (3001, 16, True)])
 def test_poolrgn_max_in_runs(ks, P, F, step, dtype):
-    """Maximum pooling with 16 and with 4 lanes per region and pack against the one-column kernel (the same map off a 16-byte boundary):
+    """Maximum pooling with 16, 8 and 4 lanes per region and pack against the one-column kernel (the same map off a 16-byte boundary):
     regions of one row and of fewer rows than lanes, ties, row steps, rows that are NaN or minus infinity."""
     rng = np.random.default_rng(P + F)
     lens = rng.integers(1, 50, size=P)
