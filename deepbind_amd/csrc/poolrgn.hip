@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void poolrgn_pack_kernel(const T* __restrict__
 // maxima meet by lane exchanges, the earlier run winning ties, so the result is the first strict maximum as above (a region's
 // first row counts whatever it holds, later rows only where they exceed: a NaN behaves as in the one-lane kernel). With a lane per
 // item 2000 regions x 16 columns keep 125 waves busy with 124 dependent rows each: 34 us for 16 MB, under 9 this way; 1000
-// regions x 64 doubles 36 us, 16.
+// regions x 64 doubles 35 us, 14.
 template <typename T, int SPLIT>
 __global__ __launch_bounds__(256) void poolrgn_max_split_kernel(const T* __restrict__ U, unsigned F, const uint32_t* __restrict__ R, unsigned P, bool per_step,
                                                                 T* __restrict__ pooled, uint32_t* __restrict__ argmax)
@@ -383,8 +383,8 @@ int launch_fwd(hipStream_t st, const T* U, size_t F, const uint32_t* R, size_t P
         const size_t items = P * (F / (16 / sizeof(T)));
         // Too few items to fill the GPU with a lane each. The regions' lengths are only known on the device: the lines lie where regions of a
         // few rows are no slower either. us, lane per item / this, for regions of 12 and of 124 rows: 16 000 items, 16 lanes each, 4.0 / 4.0
-        // and 34 / 10 (at 32 000 items 3.9 / 5.1 and 35 / 17); 32 000, eight lanes, 4.0 / 3.9 and 35 / 13.6; 64 000, four, 4.2 / 4.1 and
-        // 24 / 12 (at 130 000 4.4 / 5.5 for 12 rows).
+        // and 34 / 10 (at 32 000 items 3.9 / 5.1 and 33 / 18); 32 000, eight lanes, 4.0 / 3.9 and 35 / 13.6; 64 000, four, 3.9 / 3.8 and
+        // 35 / 20 (at 130 000 5.4 / 6.5 for 12 rows).
         if (ptype == DBK_PT_MAX && items <= 98304) {
             if (items <= 16384)
                 hipLaunchKernelGGL((poolrgn_max_split_kernel<T, 16>), dim3(dbk::divup(items, 16)), block, 0, st, U, F32, R, P32, per_step, pooled, argmax);
