@@ -1036,7 +1036,8 @@ bool bprop_X_few_rows(size_t m, size_t F, size_t n)
 {
     const bool f64 = sizeof(T) == 8;
     const double row = (f64 ? 1.45e-4 : F <= 512 ? 6.5e-5 : 2.3e-4) * (double)m * dbk::divup(F, 64);
-    const double pass = f64 ? 0.95 + 0.047 * (double)m : 0.65 + 0.032 * (double)m;
+    const double pass = f64 ? 0.95 + 0.047 * (double)m : 0.65 + 0.032 * (double)m + (m > 24 ? 0.2 : 0.0);
+    if (m > 24 && n <= m / 2) return true;                         // (a workgroup's filters would be staged for a few rows: 12 x 32 filters of 64 taps 8.9 / 3.8)
     return F > (f64 ? 16 : 32) && row * (double)n < pass * dbk::divup(F, 16);
 }
 

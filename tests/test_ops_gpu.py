@@ -254,7 +254,8 @@ def test_corr1ord_bprop_X_bulk_rows(ks, n, m, F):
 
 
 @pytest.mark.parametrize("n,m,F,dtype", [(2400, 24, 1000, np.float64), (2300, 24, 1000, np.float64), (1500, 64, 300, np.float32), (1, 4, 17, np.float32),
-                                         (1190, 24, 31, np.float64), (1210, 24, 31, np.float64)])
+                                         (1190, 24, 31, np.float64), (1210, 24, 31, np.float64),
+                                         (32, 64, 20, np.float32), (33, 64, 20, np.float32), (12, 25, 3, np.float64), (13, 25, 3, np.float64)])
 def test_corr1ord_bprop_X_few_rows_of_many_filters(ks, n, m, F, dtype):
     """Either side of the line between the kernel of one wave per row and the products."""
     test_corr1ord_bprop_X(ks, n, m, F, dtype)
