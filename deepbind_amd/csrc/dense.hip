@@ -684,15 +684,31 @@ __global__ __launch_bounds__(256) void k_head_lanes(size_t n, int nblock, int k,
 // taking the faster one over 2907 calls of 4096 to 300 000 rows, 1 to 64 models. us a call, k_head16 / k_head_lanes: 100 000 x 24
 // models (32 -> 8 -> 1) 82 / 166, 30 000 x 8 (16 -> 4) 6.5 / 9.9, 100 000 x 16 (16 -> 32) 66 / 89; 30 000 x 16 (16 -> 32) 27 / 25,
 // 10 000 x 24 (32 -> 8) 14 / 13, 30 000 x 12 (24 -> 16) 36 / 24.
+// (Inputs that fill no group of 16, few hidden units: 20 000 x 48 (20 -> 8) 34 / 51, 48 000 x 12 (20 -> 4) 24 / 34, 80 000 x 3 (16 -> 4) 8 / 12,
+// 50 000 x 6 (24 -> 4) 19 / 25; 8000 x 6 of each 60 to 90 % the other way.)
 inline bool head16_pays(size_t n, int nblock, int inputs, int hidden)
 {
     const size_t smem = ((size_t)inputs * hidden + 2 * (size_t)hidden) * HG * sizeof(float);
-    if (n < 4096 || hidden == 0 || (hidden & 3) || smem > 65536 || nblock < (hidden <= 4 ? 4 : 6)) return false;
+    if (n < 4096 || hidden == 0 || (hidden & 3) || smem > 65536) return false;
     const size_t items = n * (size_t)nblock, macs = (size_t)inputs * hidden;
-    if (inputs > 16 && inputs != 32 && inputs != 64) return inputs < 24 && items >= 1000000;
+    if (hidden <= 4 && nblock >= 3 && (inputs == 32 || (inputs <= 16 && items >= 300000))) return true;
+    if (nblock < (hidden <= 4 && (inputs <= 16 || inputs == 64) ? 4 : 6)) return false;
+    if (inputs > 16 && inputs < 24) return items >= 100000 && items >= (macs < 1000 ? 1000 * macs : 1000000);
+    if (inputs >= 24 && inputs < 32) return (inputs & 7) ? hidden <= 12 && items >= 1600 * macs : hidden <= 4 && items >= 800000;
+    if (inputs > 32 && inputs < 64) return false;
+    if (inputs == 64 && hidden <= 8 && nblock >= 11 && items >= 300 * macs) return true;
     if (hidden <= 4) return items >= 500 * macs;
     if (inputs <= 16 && items >= 4000000) return true;
     return macs <= (inputs == 32 ? 512u : 640u) && items >= 160000 && items >= 1200 * macs;
+}
+
+// Where k_head, a thread per row and model, is the better one still: so few inputs that most of k_head_lanes' 16 are padding, and enough rows x
+// models to fill the GPU with threads. us a call, k_head / k_head_lanes: 2740 x 90 (1 -> 32 -> 1) 8.8 / 12.5, 2458 x 64 (3 -> 20) 8.2 / 9.9,
+// 84 000 x 64 (1 -> 1) 62 / 75; of 643 calls of up to three inputs it takes, four are more than 6 % slower than k_head_lanes.
+inline bool head_rows_pay(size_t n, int nblock, int inputs, int hidden)
+{
+    const size_t items = n * (size_t)nblock;
+    return hidden > 0 ? inputs <= 3 && n < 4096 && items >= 24000 : inputs == 1 && items >= 18000;
 }
 
 // Row-slice count for the kernels that stage 16 models' weights per workgroup: about 1024 workgroups in all
@@ -1035,9 +1051,9 @@ int dbk_head_fprop(dbk_stream_t stream, size_t n, int nblock, int k, int hidden,
     if (gx > 2048u) gx = 2048u;
     const size_t smem16 = ((size_t)kk_all * hidden + 2 * (size_t)hidden) * HG * sizeof(float);
     // (Whether the feature columns are given or left out as zeros must not change the bits: what does not depend on it decides. k_head, which
-    // takes over from k_head16 where given columns do not fit in LDS, adds in k_head16's order.)
+    // takes over from k_head16 where given columns do not fit in LDS, adds in k_head16's order; kw counts them in either case.)
     const bool grouped = head16_pays(n, nblock, k, hidden);
-    if (!grouped && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
+    if (!grouped && !head_rows_pay(n, nblock, kw, hidden) && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
         const int mg = nblock >= 4 ? 4 : (nblock >= 2 ? 2 : 1);
         const unsigned cols = dbk::divup(nblock, mg);
         unsigned gy = dbk::divup(n, 4 * (4 / mg));                 // a row step per wave ...

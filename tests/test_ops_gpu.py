@@ -823,7 +823,7 @@ def test_head_fprop(ds):
 
 
 @pytest.mark.parametrize("n,k,h,nb", [(1, 1, 1, 1), (5, 17, 33, 3), (4097, 12, 0, 4), (70, 64, 32, 2), (301, 33, 16, 5), (9001, 16, 32, 1),
-                                      (4096, 32, 32, 13), (2, 64, 0, 6), (33, 32, 64, 7)])
+                                      (4096, 32, 32, 13), (2, 64, 0, 6), (33, 32, 64, 7), (9001, 1, 0, 2), (8999, 1, 0, 2)])
 def test_head_fprop_lane_groups(ds, n, k, h, nb):
     """The 16-lanes-per-item kernel: inputs and hidden units that fill no group of 16, one to four models side by side and more, a
     single row, several steps per wave with a ragged end."""
@@ -844,9 +844,11 @@ def test_head_fprop_lane_groups(ds, n, k, h, nb):
 
 
 @pytest.mark.parametrize("n,k,h,nb,nfeat", [(10001, 32, 8, 33, 0), (4097, 16, 4, 9, 0), (62501, 20, 16, 16, 0), (30001, 16, 60, 12, 0), (9001, 16, 64, 70, 0),
-                                            (40001, 16, 32, 16, 16), (4500, 64, 4, 30, 0), (26001, 64, 8, 25, 0), (11000, 5, 64, 35, 3)])
+                                            (40001, 16, 32, 16, 16), (4500, 64, 4, 30, 0), (26001, 64, 8, 25, 0), (11000, 5, 64, 35, 3),
+                                            (14001, 20, 8, 12, 0), (4099, 32, 4, 3, 0), (27801, 26, 8, 12, 2), (100100, 16, 4, 3, 0), (4101, 64, 8, 38, 0),
+                                            (2741, 1, 32, 9, 0), (2741, 1, 32, 8, 1), (2000, 2, 20, 13, 1), (2000, 2, 20, 13, 2)])
 def test_head_fprop_either_side_of_the_bulk_rule(ds, n, k, h, nb, nfeat):
-    """Shapes that the 16-models-per-workgroup kernel takes by rows x models, and ones that do not fit its LDS: for all of them the scores
+    """Shapes that the 16-models-per-workgroup kernel takes by rows x models, ones that do not fit its LDS, and few inputs: for all of them the scores
     are the oracle's, and feature columns left out give the bits of columns of zeros."""
     rng = np.random.default_rng(n + k + h + nb)
     Pl = np.abs(rng.standard_normal((n, k * nb))).astype(np.float32)
