@@ -680,8 +680,8 @@ __global__ __launch_bounds__(256) void k_head_lanes(size_t n, int nblock, int k,
 // Where k_head16, whose weights in LDS feed four rows (two beyond 16 inputs, one beyond 32) of 16 models each, is the better of the two: it
 // spends about a microsecond per 32 multiply-adds of an item before the first row is out, and then fewer instructions an item than
 // k_head_lanes' padded 16 x 16 blocks - by most where a block is mostly padding (few hidden units), by none where its inputs are no whole
-// packs or LDS holds few workgroups of it. The line is the measured break-even in rows x models of 50 shapes; within 1.3 % of always
-// taking the faster one over 2907 calls of 4096 to 300 000 rows, 1 to 64 models. us a call, k_head16 / k_head_lanes: 100 000 x 24
+// packs or LDS holds few workgroups of it. The line is the measured break-even in rows x models of 100 shapes; of 3085 calls of 1 to 200 000
+// rows, 1 to 90 models, 14 are more than 6 % slower than with k_head16 and k_head alone. us a call, k_head16 / k_head_lanes: 100 000 x 24
 // models (32 -> 8 -> 1) 82 / 166, 30 000 x 8 (16 -> 4) 6.5 / 9.9, 100 000 x 16 (16 -> 32) 66 / 89; 30 000 x 16 (16 -> 32) 27 / 25,
 // 10 000 x 24 (32 -> 8) 14 / 13, 30 000 x 12 (24 -> 16) 36 / 24.
 // (Inputs that fill no group of 16, few hidden units: 20 000 x 48 (20 -> 8) 34 / 51, 48 000 x 12 (20 -> 4) 24 / 34, 80 000 x 3 (16 -> 4) 8 / 12,
