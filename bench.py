@@ -319,10 +319,10 @@ def ops_throughput(reps=5):
             rec("scanpool_bprop[all, masks]", timed(lambda: ks.scanpool_bprop(W, b, X, R, pt, P, I, dP, dW, db, overwrite=True, act=act)),
                 N + 2 * nout + B * F * 4 + N * F // 8, adds)
             del act
-    rec("scanpool_fprop table[max]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "max", path="kmer")), N + B * F * 4, adds)
-    rec("scanpool_fprop table[max, argmax]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "max", want_argmax=True, path="kmer")),
+    rec("scanpool_fprop bulk[max]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "max", path="kmer")), N + B * F * 4, adds)
+    rec("scanpool_fprop bulk[max, argmax]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "max", want_argmax=True, path="kmer")),
         N + 2 * B * F * 4, adds)
-    rec("scanpool_fprop table[all, argmax]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "all", want_argmax=True, path="kmer")),
+    rec("scanpool_fprop bulk[all, argmax]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "all", want_argmax=True, path="kmer")),
         N + 3 * B * F * 4, adds)
     del X, R, W, b, dW, db, dX, P, I, dP
     # shorter filters at bulk-scoring size (65 536 sequences x 101 nt): up to 18 taps the table kernel walks through
@@ -336,7 +336,7 @@ def ops_throughput(reps=5):
         W = torch.randn(4 * m2, F, device="cuda") * 0.1
         b = torch.randn(1, F, device="cuda") * 0.1
         for path in ("kmer", "mfma"):
-            rec("scanpool_fprop %s[max] %d x %d nt, %d taps" % ("table" if path == "kmer" else "matrix cores", B2, L, m2),
+            rec("scanpool_fprop %s[max] %d x %d nt, %d taps" % ("bulk" if path == "kmer" else "matrix cores", B2, L, m2),
                 timed(lambda: ks.scanpool_fprop(W, b, X, R, "max", path=path)), X.numel() + B2 * F * 4, float(X.numel()) * F * m2)
         del X, R, W, b
     # per-model dense layer at bulk-scoring size: 100 000 rows, 64 models, 16 -> 32

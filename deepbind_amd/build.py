@@ -24,9 +24,9 @@ FLAGS = [
 ]
 
 
-# The running max of the k-mer kernel must compile to bare v_max / v_max3 instructions; with NaNs
-# honoured every fmaxf gets two extra canonicalising ops. Infinities stay honoured (-inf seeds the max).
-EXTRA = {"scanpool_kmer.hip": ["-fno-honor-nans"]}
+# The running max of the bulk scan must compile to bare v_max / v_max3 instructions; with NaNs
+# honoured every fmaxf gets two extra canonicalising ops. Infinities stay honoured.
+EXTRA = {"scanpool_digits.hip": ["-fno-honor-nans"]}
 
 
 def _compile(src):

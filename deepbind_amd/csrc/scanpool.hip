@@ -3,8 +3,8 @@
 // The (N, F) activation map is never written: a workgroup owns a tile of 64 filters (one lane per
 // filter) and walks whole regions, each wave scanning 16 positions at a time in registers and
 // folding them straight into the region's running max / argmax / sum. This path takes any filter
-// length that fits in LDS, any region table and every letter code; the k-mer table kernel in
-// scanpool_kmer.hip is the fast path for bulk scoring and falls back to this one.
+// length that fits in LDS, any region table and every letter code; the kernel of scanpool_digits.hip is the fast path
+// for bulk scoring and leaves weights it cannot express to this one.
 //
 // Backward: the max part is 1-sparse (one position per region and filter), the average part is
 // dense and needs the forward recomputed for the ReLU mask. Both accumulate into per-wave private
@@ -53,8 +53,8 @@ __device__ __forceinline__ void scanpool_fprop_body(const wg_t wg, const float* 
                                                     unsigned long long* __restrict__ act)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    // when given, the launch only does work if the device flag is set (fallback behind the k-mer kernel)
-    if (run_if_flag && run_if_flag[0] == 0) return;
+    // when given (behind the bulk kernel: one flag per 32 filters), only the tiles that one of their two flags asks for
+    if (run_if_flag && (run_if_flag[2 * wg.y] | run_if_flag[2 * wg.y + 1]) == 0u) return;
     const unsigned nw = blockDim.x >> 6;
     const unsigned chunk = nw * XCH_SUBS * PSUB;
     // up to 16 taps: the lane's filter weights live in register planes and the scan needs no table in LDS
@@ -1193,8 +1193,8 @@ int launch_multi(K kern, hipStream_t st, size_t smem, const multi_args& a)
 
 }  // namespace dbk_scanpool_general
 
-namespace dbk_scanpool_kmer {
-bool takes(size_t m, size_t F, size_t N, size_t P);
+namespace dbk_scanpool_digits {
+bool takes(size_t m, size_t F, size_t N, size_t P, bool argmax);
 }
 
 namespace dbk {
@@ -1209,8 +1209,8 @@ bool scan_multi_takes(size_t m, size_t N, size_t P, unsigned n, const scan_group
         if (g[i].ptype != DBK_PT_MAX && g[i].ptype != DBK_PT_AVG && g[i].ptype != DBK_PT_ALL) return false;
         if (g[i].ptype != DBK_PT_MAX && !g[i].act) return false;      // the dense backward kernel here is the mask-driven one
         if (g[i].ptype != DBK_PT_AVG && !g[i].argmax) return false;
-        // a max-pooling group on a batch large enough for the k-mer table goes there when stepped alone (other sums, other bits)
-        if (g[i].ptype == DBK_PT_MAX && dbk_scanpool_kmer::takes(m, g[i].F, N, P)) return false;
+        // a max-pooling group on a batch large enough for the bulk kernel goes there when stepped alone (other sums, other bits)
+        if (g[i].ptype == DBK_PT_MAX && dbk_scanpool_digits::takes(m, g[i].F, N, P, true)) return false;
     }
     return fprop_smem(multi_tier(m), m) <= lds_limit() && wide_smem(24) <= lds_limit() && sparse_smem(m) <= lds_limit() && bits_smem(multi_tier(m)) <= lds_limit();
 }
@@ -1276,8 +1276,8 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
 
 }  // namespace dbk
 
-namespace dbk_scanpool_kmer {
-// Fast path (k-mer lookup table); returns -1 when the shape is outside what it handles.
+namespace dbk_scanpool_digits {
+// Bulk path (6-bit digits on the matrix cores); returns -1 when the shape is outside what it handles.
 int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
           const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax);
 }
@@ -1346,10 +1346,9 @@ int dbk_scanpool_fprop(dbk_stream_t stream, const float* W, const float* bias, s
               "ValueError: %zu rows x %zu filters overflow the 32-bit argmax index; score in smaller batches or without argmax", N, nfilter);
     if (nfilter == 0 || nregion == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(W && bias && X && regions && pooled, "ValueError: null pointer argument");
-    // the activity masks are written by the general kernel only (the k-mer table is worth its set-up for bulk scoring,
-    // where no backward pass follows)
+    // the activity masks are written by the general path only (the bulk kernel is for scoring, where no backward pass follows)
     if (!act) {
-        int rc = dbk_scanpool_kmer::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax);
+        int rc = dbk_scanpool_digits::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax);
         if (rc >= 0) return rc;
     }
     return dbk_scanpool_general::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax, nullptr,

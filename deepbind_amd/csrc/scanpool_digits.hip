@@ -1,0 +1,557 @@
+// Bulk path of the fused scan + bias + ReLU + region pooling forward: the scan as a product of 4-bit one-hot letters
+// with the weights' 6-bit digits on the matrix cores.
+//
+// Written as a product the scan is Z (positions x filters) = H (positions x 4m) . W (4m x filters), H holding the one-hot
+// letters of every position's window. v_mfma_scale_f32_32x32x64_f8f6f4 multiplies 4-bit by 6-bit floats with float32
+// accumulation, 64 values of the contraction index per 32 clocks - four times what the bf16 instruction does - and both
+// operands are exact in those formats:
+//  * H: a letter is 4.0 in its own row, "mean of the four" (N, padding: code 255 and any other non-letter) 1.0 in all
+//    four rows, code 254 nothing: the multiples 4, 1 and 0 of a quarter.
+//  * W: every filter's weights as 30-bit fixed point numbers against the filter's largest (32^5 .. 32^6 units), written
+//    in six digits of -16 .. 16: 1/8 .. 16/8 are exact in the 6-bit format (1 sign, 2 exponent, 3 fraction bits). The
+//    instruction's per-lane block scale carries the filter's and the digit's power of two.
+// So the products are exact and the float32 accumulator sees the small digits first. What is dropped is below 2^-29 of
+// the filter's largest weight; measured against float64 the sums are off by 3.3e-8 (16 taps, normal weights) where
+// float32 additions tap by tap are off by 7.6e-8 and through a table of 3-mer sums by 6.2e-8.
+//
+// A weight far below zero only has to keep its window closed: every window's rectified value is at most
+// T = sum over the taps of the largest weight (if positive) + the bias, so weights below -8 T are raised to -8 T (a
+// window of one such "mean of four" is still at most -2 T + T). Filters that fixed point does not express well (an
+// infinite or undefined weight, one positive weight more than 64 times the next) are left to the general kernel,
+// which is launched behind this one and does nothing where no tile of filters asks for it.
+//
+// Mapping: a workgroup of 16 waves (one per CU) owns 32 filters, whose digits stay in its registers (24 taps: 9
+// instructions' operands, 54 registers a lane). A wave takes a region at a time from the workgroup's counter and walks it
+// in tiles of 32 positions. 224 positions' letters at a time become one 16-byte entry per position in the wave's own
+// LDS: the one-hot nibbles of the eight letters from there on, which is half of an instruction's operand (lanes 0-31
+// take taps 0-7, lanes 32-63 taps 8-15), so a tile costs one or two 16-byte reads per lane. An entry's place is
+// q + q / 16: writes (four consecutive entries per lane) and reads are both free of bank conflicts.
+//
+// Bound: the matrix pipe, and through it the chip's power: an instruction takes its 34 clocks, at 1.5-1.6 GHz under this
+// load (2.3 GHz with all operands zero), 22 ns per SIMD. A table of 3-mer sums in LDS (one 4-byte read and add per three
+// taps), which this replaced, moved its 248 ns worth of LDS bytes per 32 x 32 tile of 24 taps; nine instructions are 198.
+// Measured, table / digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 11.1 ms; 65 536 x 101 x 256
+// filters, 24 taps 0.721 / 0.513, 16 taps 0.552 / 0.380; 20 000 x 500 x 256 x 8 taps 0.491 / 0.261; max + average, 20 000 x
+// 30-150 x 384 x 16 taps 0.275 / 0.215; with an argmax 65 536 x 101 x 256 x 24 taps 0.867 / 0.616; averages are off by
+// 5.6e-8 instead of 1.7e-7 (a tile's sum first, then the tiles').
+//
+// Reference chain being fused: kangaroo/_ext/corr1ord.py:97-117 -> deepity/std/elemwise.py:162-180,71-82
+// -> kangaroo/_ext/poolrgn.py:56-76 (kernels corr1ord.cuh:139-157, poolrgn.cuh:44-79).
+#include "dbk_common.h"
+#include "scan_common.h"
+#include "mfma_common.h"
+#include <mutex>
+
+namespace dbk_scanpool_general {
+int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
+          const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, const unsigned* run_if_flag,
+          unsigned long long* act);
+}
+
+namespace dbk_scanpool_digits {
+
+using dbk_mfma::f32x16_t;
+using dbk_mfma::load_letters4;
+
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+
+constexpr int FTILE = 32;                     // filters per workgroup: columns of a tile
+constexpr int ROWS = 32;                      // positions per tile
+constexpr int NDIGIT = 6;                     // digits per weight
+constexpr int NWAVE = 16;                     // waves per workgroup
+constexpr unsigned CHUNK = 224;               // rows whose letters are staged at a time: seven tiles
+constexpr unsigned ENTRIES = 304;             // entries of a wave: 256 positions, one entry of padding per 16, what a read past the last tile touches
+constexpr unsigned SLOT_BYTES = FTILE * 24;   // one digit of eight taps of all the tile's filters: 32 values of 6 bits per filter
+constexpr float CLOSED = -3.0e38f;            // the value of a row outside the region
+
+// the LDS entry of a position: consecutive positions of a lane and of neighbouring lanes fall into different banks
+__device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
+
+// ---------------------------------------------------------------------------------------------- the weights' digits
+// What a call keeps in its scratch, per tile of 32 filters: a flag (not expressible: the general kernel's), the filters'
+// exponents and the digits, [8-tap block][digit][filter][24 bytes].
+struct digit_store { unsigned* flags; int* expo; unsigned char* digits; };
+inline size_t tile_bytes(unsigned tb) { return FTILE * sizeof(int) + (size_t)tb * NDIGIT * SLOT_BYTES; }
+inline digit_store store_at(unsigned* flags, unsigned char* ws, unsigned ntile)
+{
+    digit_store s;
+    s.flags = flags;
+    s.expo = reinterpret_cast<int*>(ws);
+    s.digits = ws + (size_t)ntile * FTILE * sizeof(int);
+    return s;
+}
+
+// A workgroup splits one tile's weights: thread (g, fl) takes taps g, 8 + g, .. of filter fl. Latency only (4m x 32 values).
+template <int TB>
+__global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restrict__ W, const float* __restrict__ bias, unsigned m, unsigned F,
+                                                            unsigned f0, digit_store out)
+{
+    __shared__ float red[5][8][FTILE];                            // sums and maxima of the eight threads of a filter
+    __shared__ unsigned char dig[TB * NDIGIT * SLOT_BYTES];
+    __shared__ unsigned bad_tile;
+    const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
+    if (threadIdx.x == 0) bad_tile = 0u;
+    float w[TB][4];
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const unsigned tap = 8u * t + g;
+            w[t][c] = (tap < m && f < F) ? W[(size_t)(4 * tap + c) * F + f] : 0.0f;
+        }
+    const float b = f < F ? bias[f] : 0.0f;
+    float open = 0.0f, top = 0.0f, second = 0.0f, low = 0.0f;     // sum of the taps' best, the two largest weights, the most negative one
+    bool bad = (__float_as_uint(b) & 0x7fffffffu) >= 0x71000000u;     // (the file is compiled without NaN: test the bits)
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        float best = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const unsigned bits = __float_as_uint(w[t][c]) & 0x7fffffffu;
+            bad |= bits > 0x7f800000u || (bits == 0x7f800000u && w[t][c] > 0.0f);
+            best = fmaxf(best, w[t][c]);
+            second = fmaxf(second, fminf(top, w[t][c]));
+            top = fmaxf(top, w[t][c]);
+            low = fmaxf(low, -w[t][c]);
+        }
+        open += best;
+    }
+    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = second; red[3][g][fl] = low; red[4][g][fl] = bad ? 1.0f : 0.0f;
+    __syncthreads();
+    open = fmaxf(b, 0.0f); top = 0.0f; second = 0.0f; low = 0.0f;
+    float nbad = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        open += red[0][k][fl];
+        const float tk = red[1][k][fl], sk = red[2][k][fl];
+        second = fmaxf(fmaxf(second, sk), fminf(top, tk));
+        top = fmaxf(top, tk);
+        low = fmaxf(low, red[3][k][fl]);
+        nbad += red[4][k][fl];
+    }
+    const float floor_ = -8.0f * open;                            // nothing below keeps a window open
+    const float big = fmaxf(top, fminf(low, -floor_));
+    second = fmaxf(second, b);
+    int e = 0;
+    bad = nbad > 0.0f || (second > 0.0f && top > 64.0f * second) || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-25f);
+    if (!bad && big != 0.0f) e = (int)((__float_as_uint(big) >> 23) & 0xffu) - 127;
+    if (bad) bad_tile = 1u;                                       // (every writer writes the same)
+    // digits: x = w * 2^(3 - e) is below 16, each digit the nearest whole number, the remainder (exact) times 32
+    const float scale = __uint_as_float((unsigned)(127 + 3 - e) << 23);
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        float x[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[c] = bad ? 0.0f : fmaxf(w[t][c], floor_) * scale;
+#pragma unroll
+        for (int p = 0; p < NDIGIT; ++p) {
+            unsigned word = 0u;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float d = rintf(x[c]);
+                x[c] = (x[c] - d) * 32.0f;
+                const int i = (int)d;
+                const unsigned a = (unsigned)(i < 0 ? -i : i);
+                // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 15 are their own codes (denormal below 8), 16 is code 16
+                word |= (a | (i < 0 ? 32u : 0u)) << (6 * c);
+            }
+            unsigned char* o = dig + ((size_t)(t * NDIGIT + p) * FTILE + fl) * 24u + 3u * g;
+            o[0] = (unsigned char)word; o[1] = (unsigned char)(word >> 8); o[2] = (unsigned char)(word >> 16);
+        }
+    }
+    __syncthreads();
+    unsigned* dst = reinterpret_cast<unsigned*>(out.digits + (size_t)blockIdx.x * (TB * NDIGIT * SLOT_BYTES));
+    for (unsigned i = threadIdx.x; i < TB * NDIGIT * SLOT_BYTES / 4; i += 256) dst[i] = reinterpret_cast<const unsigned*>(dig)[i];
+    if (g == 0) out.expo[blockIdx.x * FTILE + fl] = e;
+    if (threadIdx.x == 0) out.flags[blockIdx.x] = bad_tile;
+}
+
+// ---------------------------------------------------------------------------------------------- letters
+// Four letter codes (bytes) as four 16-bit groups of one-hot nibbles, two registers. 6 is 4.0 and 2 is 1.0 in the 4-bit
+// format. The codes' low three bits (0-3 letters, 6: 254, 7: 255) select the byte of an eight-byte table each.
+__device__ __forceinline__ uint2 letter_nibbles(unsigned v)
+{
+    const unsigned sel = v & 0x07070707u;
+    const unsigned lo = __builtin_amdgcn_perm(0x22002222u, 0x00006006u, sel), hi = __builtin_amdgcn_perm(0x22002222u, 0x60060000u, sel);
+    return make_uint2(__builtin_amdgcn_perm(hi, lo, 0x05010400u), __builtin_amdgcn_perm(hi, lo, 0x07030602u));
+}
+// nonzero where a byte's upper six bits differ from each other: a code between 4 and 251, which counts as 255
+__device__ __forceinline__ unsigned odd_codes(unsigned v) { return (v ^ (v << 1)) & 0xf8f8f8f8u; }
+__device__ __forceinline__ unsigned plain_codes(unsigned v)
+{
+    unsigned r = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const unsigned c = (v >> (8 * k)) & 0xffu;
+        r |= ((c < 4u || c == 254u) ? c : 255u) << (8 * k);
+    }
+    return r;
+}
+
+// ---------------------------------------------------------------------------------------------- the products
+// instructions per tile: two 8-tap blocks (one per half wave) or two digits of one block at a time
+template <int TB> struct product_count { static constexpr int N = TB == 1 ? 3 : (TB == 2 ? 6 : (TB == 3 ? 9 : 12)); };
+
+template <int SEL>
+__device__ __forceinline__ f32x16_t product(const uint4& a, const unsigned (&b)[6], const f32x16_t& c, int scale)
+{
+    const i32x8_t av = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
+    const i32x8_t bv = {(int)b[0], (int)b[1], (int)b[2], (int)b[3], (int)b[4], (int)b[5], 0, 0};
+    // operand formats 4 (4-bit) and 2 (6-bit, two exponent bits); scale bytes are exponents + 127: 125 makes the 4.0 a one
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 4, 2, 0, 125, SEL, scale);
+}
+
+// which 8-tap block and digit the half wave h holds in operand i of a tile (operands in the order they are multiplied:
+// small digits first)
+template <int TB> __device__ __forceinline__ void operand_slot(int i, unsigned h, unsigned& block, unsigned& digit)
+{
+    if (TB == 1) { block = 0u; digit = 2u * (2 - i) + h; }                          // digit pairs (4,5) (2,3) (0,1)
+    else if (TB == 2) { block = h; digit = 5 - i; }
+    else if (TB == 3) {
+        const int j = 2 - i / 3, k = i % 3;                                         // block pair digit 2j + 1, digit 2j, third block's pair
+        if (k < 2) { block = h; digit = 2 * j + 1 - k; }
+        else { block = 2u; digit = 2u * j + h; }
+    } else { block = (i & 1 ? 2u : 0u) + h; digit = 5 - i / 2; }
+}
+
+template <int TB, int I>
+__device__ __forceinline__ void products(f32x16_t& acc, const uint4& a0, const uint4& a1, const unsigned (&B)[product_count<TB>::N][6], const int (&s)[3])
+{
+    if constexpr (I < product_count<TB>::N) {
+        if constexpr (TB == 1) acc = product<2 - I>(a0, B[I], acc, s[2]);
+        else if constexpr (TB == 2) { constexpr int p = 5 - I; acc = product<(p & 3)>(a0, B[I], acc, s[p >> 2]); }
+        else if constexpr (TB == 3) {
+            constexpr int j = 2 - I / 3, k = I % 3, p = 2 * j + 1 - k;
+            if constexpr (k < 2) acc = product<(p & 3)>(a0, B[I], acc, s[p >> 2]);
+            else acc = product<j>(a1, B[I], acc, s[2]);
+        } else { constexpr int p = 5 - I / 2; acc = product<(p & 3)>(I & 1 ? a1 : a0, B[I], acc, s[p >> 2]); }
+        products<TB, I + 1>(acc, a0, a1, B, s);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------- the scan
+template <int PT, bool WANT_ARGMAX, int TB>
+__global__ __launch_bounds__(NWAVE * 64) __attribute__((amdgpu_waves_per_eu(NWAVE / 4, NWAVE / 4)))
+void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsigned f0, unsigned F, const uint8_t* __restrict__ X, size_t N, size_t ndef,
+                            const uint32_t* __restrict__ R, unsigned P, unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int NI = product_count<TB>::N;
+    const unsigned tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
+    if (D.flags[tile] != 0u) return;                              // the general kernel takes these filters
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned col = lane & 31u, h = lane >> 5;
+    unsigned* counter = reinterpret_cast<unsigned*>(smem);
+    uint4* entries = reinterpret_cast<uint4*>(smem + 16) + (size_t)wave * ENTRIES;
+    // this workgroup's regions
+    const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
+    if (threadIdx.x == 0) counter[0] = lo;
+    // ---- this lane's operands: column `col` of the weights, the half wave's 32 rows of every product
+    unsigned B[NI][6];
+    {
+        const unsigned char* dig = D.digits + (size_t)tile * (TB * NDIGIT * SLOT_BYTES);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            unsigned block, digit;
+            operand_slot<TB>(i, h, block, digit);
+            const uint2* src = reinterpret_cast<const uint2*>(dig + ((size_t)(block * NDIGIT + digit) * FTILE + col) * 24u);
+            const uint2 q0 = src[0], q1 = src[1], q2 = src[2];
+            B[i][0] = q0.x; B[i][1] = q0.y; B[i][2] = q1.x; B[i][3] = q1.y; B[i][4] = q2.x; B[i][5] = q2.y;
+        }
+    }
+    // block scales: digit p counts 2^(e - 3 - 5 p), stored in eighths
+    const int e = D.expo[tile * FTILE + col] + 127;
+    int s[3];
+    s[0] = (e & 255) | ((e - 5) & 255) << 8 | ((e - 10) & 255) << 16 | (int)((unsigned)((e - 15) & 255) << 24);
+    s[1] = ((e - 20) & 255) | ((e - 25) & 255) << 8;
+    const int eh = e - 5 * (int)h;                                // pairs of digits of one block: 2 j + h
+    s[2] = (eh & 255) | ((eh - 10) & 255) << 8 | ((eh - 20) & 255) << 16;
+    const unsigned f = f0 + tile * FTILE + col;
+    const float bf = f < F ? bias[f] : 0.0f;
+    const unsigned rg = 4u * h;                                   // this half wave's rows lie 4 further down
+    // operands are read from entry tile * 34 + these (34 entries per 32 positions)
+    const unsigned at0 = place(col + (TB >= 2 ? 8u * h : 0u)), at1 = place(col + 16u + (TB == 4 ? 8u * h : 0u));
+    __syncthreads();
+
+    auto claim = [&]() -> unsigned {
+        unsigned v = 0u;
+        if (lane == 0u) v = atomicAdd(counter, 1u);
+        return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+    };
+    // 12 letters from position c + 4 * lane on
+    auto load12 = [&](unsigned c, unsigned (&v)[3]) {
+        const size_t o = (size_t)c + 4u * lane;
+        if ((size_t)c + 4u * 63u + 12u <= N) __builtin_memcpy(v, X + o, 12);
+        else {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) v[k] = load_letters4(X, N, o + 4 * k);
+        }
+    };
+    unsigned r = claim(), rn = claim();                           // the region in work, the one after it
+    unsigned a = 0u, b = 0u, an = 0u, bn = 0u;
+    if (r < hi) { a = R[2 * (size_t)r]; b = R[2 * (size_t)r + 1]; }
+    if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
+    unsigned letters[3] = {0u, 0u, 0u};
+    if (r < hi) load12(a, letters);
+
+    while (r < hi) {
+        float mx = CLOSED, sum = 0.0f;
+        unsigned xi = 0u;
+        unsigned c = a;
+        bool last;
+        do {
+            const unsigned left = b > c ? b - c : 0u;             // rows of the region from this chunk on
+            last = left <= CHUNK;
+            // ---- the chunk's entries
+            if (__any((odd_codes(letters[0]) | odd_codes(letters[1]) | odd_codes(letters[2])) != 0u)) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) letters[k] = plain_codes(letters[k]);
+            }
+            const uint2 n0 = letter_nibbles(letters[0]), n1 = letter_nibbles(letters[1]), n2 = letter_nibbles(letters[2]);
+            const unsigned p[6] = {n0.x, n0.y, n1.x, n1.y, n2.x, n2.y};
+            unsigned q[5];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) q[k] = __builtin_amdgcn_alignbit(p[k + 1], p[k], 16);
+            uint4* dst = entries + place(4u * lane);
+            __builtin_amdgcn_wave_barrier();
+            dst[0] = make_uint4(p[0], p[1], p[2], p[3]);
+            dst[1] = make_uint4(q[0], q[1], q[2], q[3]);
+            dst[2] = make_uint4(p[1], p[2], p[3], p[4]);
+            dst[3] = make_uint4(q[1], q[2], q[3], q[4]);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // the next chunk's letters travel while this one is multiplied
+            if (!last) load12(c + CHUNK, letters);
+            else if (rn < hi) load12(an, letters);
+            // ---- its tiles
+            const unsigned nrow = last ? left : CHUNK;
+            const uint4* src = entries;
+            for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34) {
+                uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
+                if ((size_t)c + t0 + ROWS > ndef) {
+                    // rows the scan does not define hold the rectified bias
+                    if ((size_t)c + t0 + col >= ndef) { a0 = make_uint4(0u, 0u, 0u, 0u); a1 = a0; }
+                }
+                f32x16_t z;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+                products<TB, 0>(z, a0, a1, B, s);
+                if (left - t0 < (unsigned)ROWS) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) z[i] = rg + ((i & 3) + 8 * (i >> 2)) < left - t0 ? z[i] : CLOSED;
+                }
+                if (PT != DBK_PT_AVG) {
+                    if (WANT_ARGMAX) {
+                        float bm = z[0];
+                        unsigned bi = 0u;
+#pragma unroll
+                        for (int i = 1; i < 16; ++i) {
+                            const bool gt = z[i] > bm;
+                            bm = gt ? z[i] : bm;
+                            bi = gt ? (unsigned)i : bi;
+                        }
+                        if (bm > mx) { mx = bm; xi = (c - a) + t0 + rg + (bi & 3u) + 8u * (bi >> 2); }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, z[i]), z[i + 1]);
+                    }
+                }
+                if (PT != DBK_PT_MAX) {
+                    float part = fmaxf(z[0] + bf, 0.0f);
+#pragma unroll
+                    for (int i = 1; i < 16; ++i) part += fmaxf(z[i] + bf, 0.0f);
+                    sum += part;                                  // (a tile's sum first: sums of sums round less)
+                }
+            }
+            c += CHUNK;
+        } while (!last);
+        // ---- the region's result: fold the two half waves (equal values keep the earlier row)
+        if (PT != DBK_PT_AVG) {
+            const float vm = __shfl_xor(mx, 32, 64);
+            if (WANT_ARGMAX) {
+                const unsigned vi = (unsigned)__shfl_xor((int)xi, 32, 64);
+                if (vm > mx || (vm == mx && vi < xi)) xi = vi;
+            }
+            mx = fmaxf(mx, vm) + bf;
+            if (WANT_ARGMAX && !(mx > 0.0f)) xi = 0u;             // nothing open: the region's first row
+            mx = fmaxf(mx, 0.0f);
+        }
+        if (PT != DBK_PT_MAX) sum = (sum + __shfl_xor(sum, 32, 64)) / (float)(b - a);
+        if (h == 0u && f < F) {
+            const size_t j = (size_t)r * F + f;
+            if (PT == DBK_PT_MAX) pooled[j] = mx;
+            else if (PT == DBK_PT_AVG) pooled[j] = sum;
+            else { pooled[2 * j] = mx; pooled[2 * j + 1] = sum; }
+            if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + xi) * F + f);
+        }
+        r = rn; a = an; b = bn;
+        rn = claim();
+        if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
+    }
+}
+
+constexpr size_t SMEM = 16 + (size_t)NWAVE * ENTRIES * 16;
+
+template <int PT, bool WANT_ARGMAX, int TB>
+int launch_pt(hipStream_t st, const digit_store& D, const float* bias, unsigned f0, unsigned ntile, size_t F, const uint8_t* X, size_t N, size_t ndef,
+              const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
+{
+    auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
+    unsigned nsplit = 256u / ntile;
+    if (nsplit < 1) nsplit = 1;
+    while (nsplit > 1 && (size_t)(nsplit - 1) * NWAVE >= P) --nsplit;           // no more waves than regions
+    hipLaunchKernelGGL(kern, dim3(ntile * nsplit), dim3(NWAVE * 64), SMEM, st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
+    return 0;
+}
+
+// the filters f0 .. f0 + 32 * ntile - 1: their digits, then the scan
+template <int TB>
+int launch(hipStream_t st, const digit_store& D, const float* W, const float* bias, unsigned f0, unsigned ntile, unsigned nflag, size_t m, size_t F,
+           const uint8_t* X, size_t N, const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax)
+{
+    const size_t ndef = N >= m ? N - m + 1 : 0;                    // rows the scan defines
+    hipLaunchKernelGGL(weight_digits_kernel<TB>, dim3(nflag), dim3(256), 0, st, W, bias, (unsigned)m, (unsigned)F, f0, D);
+    if (ptype == DBK_PT_AVG) return launch_pt<DBK_PT_AVG, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+    if (ptype == DBK_PT_MAX)
+        return argmax ? launch_pt<DBK_PT_MAX, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
+                      : launch_pt<DBK_PT_MAX, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+    return argmax ? launch_pt<DBK_PT_ALL, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
+                  : launch_pt<DBK_PT_ALL, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+}
+
+// Whether a call of this size goes to the digit kernel when the choice is left to the library, in rows x 64-filter tiles
+// (what the general path's time follows). The smallest call takes three launches (digits, scan, the general kernel's look
+// at the flags), 16-18 us. Measured break-even without argmax, 25 to 400 letters, 16 to 384 filters: up to 8 taps, where
+// the general path has no matrix-core kernel, 0.15-0.25 M (at 0.5 M 17 us against 36, at 4 M 47 against 257); 9 to 32 taps
+// 0.45-0.55 M (24 taps, 101 letters x 64 filters: 20 us against 19 at 0.5 M, 27 / 33 at 1 M, 72 / 129 at 4 M; 32 taps
+// 26 / 26, 37 / 46, 107 / 171). With an argmax (a training step's forward pass) it lies at 0.9 M rows x tiles; such calls
+// come here from the size on at which a group of models is better stepped alone than in the shared launches.
+bool takes(size_t m, size_t F, size_t N, size_t P, bool argmax)
+{
+    if (m > (argmax ? 24u : 32u) || N == 0 || N > 0x7fffff00u || P > 0x7fff0000u) return false;
+    if (argmax) return (double)N * dbk::divup(F, FTILE) >= (m > 12 ? 4.0e6 : 2.0e6);
+    return (double)N * dbk::divup(F, 2 * FTILE) >= (m > 8 ? 0.6e6 : 0.25e6);
+}
+
+// A call's scratch: one flag per 32 filters (an even number of them: the general kernel looks at pairs), then the digits of
+// up to PASS_TILES tiles; more filters than that are taken in several passes.
+constexpr unsigned PASS_TILES = 2048;
+inline size_t flag_bytes(size_t F) { return (2 * (size_t)dbk::divup(F, 2 * FTILE) * sizeof(unsigned) + 255) & ~(size_t)255; }
+inline size_t scratch_bytes(size_t m, size_t F)
+{
+    const size_t nflag = 2 * (size_t)dbk::divup(F, 2 * FTILE), tiles = nflag < PASS_TILES ? nflag : PASS_TILES;
+    return flag_bytes(F) + tiles * tile_bytes((unsigned)((m + 7) / 8));
+}
+
+// force: take this path whenever the shape allows, regardless of problem size.
+// ws: device scratch of scratch_bytes(m, F) bytes the caller provides, or null to take the stream's grow-on-demand buffer.
+int fprop_impl(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
+               const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, bool force, unsigned char* ws = nullptr)
+{
+    if (ptype != DBK_PT_MAX && ptype != DBK_PT_AVG && ptype != DBK_PT_ALL) return -1;
+    if (ptype == DBK_PT_AVG && argmax != nullptr) return -1;
+    if (m > 32 || (force && m > 24) || N == 0 || N > 0x7fffff00u || P > 0x7fff0000u) return -1;
+    if (!force && !takes(m, F, N, P, argmax != nullptr)) return -1;
+    const unsigned tb = (unsigned)((m + 7) / 8), ntile = dbk::divup(F, FTILE), nflag = 2 * dbk::divup(F, 2 * FTILE);
+    DBK_CHECK(nflag / 2 <= 65535u, "ValueError: too many filters (%zu) for one launch", F);
+    if (!ws) {
+        ws = (unsigned char*)dbk::workspace(scratch_bytes(m, F), st);
+        // (a stream under capture whose scratch has not grown yet, or no memory: the general path needs none)
+        if (!ws && !force) return -1;
+        if (!ws) { dbk::set_error("MemoryError: could not allocate %zu bytes of scratch (%s)", scratch_bytes(m, F), dbk::workspace_error()); return 1; }
+    }
+    unsigned* flags = reinterpret_cast<unsigned*>(ws);
+    for (unsigned t0 = 0; t0 < ntile; t0 += PASS_TILES) {
+        const unsigned nt = ntile - t0 < PASS_TILES ? ntile - t0 : PASS_TILES, nf = nflag - t0 < PASS_TILES ? nflag - t0 : PASS_TILES;
+        const digit_store D = store_at(flags + t0, ws + flag_bytes(F), nf);
+        int rc;
+        switch (tb) {
+        case 1: rc = launch<1>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
+        case 2: rc = launch<2>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
+        case 3: rc = launch<3>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
+        default: rc = launch<4>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
+        }
+        if (rc != 0) return rc;
+    }
+    // filters whose weights the digits do not express: the general kernel, gated on the tiles' flags so that no host
+    // synchronisation is needed
+    return dbk_scanpool_general::fprop(st, W, bias, m, F, X, N, R, P, ptype, pooled, argmax, flags, nullptr);
+}
+
+int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
+          const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax)
+{
+    return fprop_impl(st, W, bias, m, F, X, N, R, P, ptype, pooled, argmax, false);
+}
+
+// ---- scratch that is part of the loaded code object, for callers that must not allocate ------------------
+// Every device the library runs on holds its own copy of this array, at its own address, from the moment the code
+// object is loaded there until the process ends. The array's name is a host-side handle, not a device address:
+// host code asks the runtime for the address once per device and passes that pointer to the kernels.
+// (24 taps: 2048 tiles' digits and exponents, 28.6 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
+constexpr size_t STATIC_SCRATCH_BYTES = size_t(29) << 20;
+constexpr size_t STATIC_SEQUENCE_BYTES = (size_t(64) << 20) - 127; // sequence bytes a call may bring
+static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * sizeof(int) + 3 * NDIGIT * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
+static __device__ __align__(256) unsigned char scratch[STATIC_SCRATCH_BYTES];
+static unsigned char* g_static_scratch[64] = {nullptr};
+static std::mutex g_static_scratch_mutex;
+
+// Address of the current device's copy of `scratch` (looked up on the first call per device); null on failure.
+static unsigned char* static_scratch()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { dbk::set_error("RuntimeError: no current device below 64"); return nullptr; }
+    std::lock_guard<std::mutex> lock(g_static_scratch_mutex);
+    if (!g_static_scratch[dev]) {
+        unsigned char* p = nullptr;
+        hipError_t e = hipGetSymbolAddress((void**)&p, HIP_SYMBOL(scratch));
+        if (e != hipSuccess || !p) {
+            dbk::set_error("RuntimeError: hipGetSymbolAddress(scratch) failed on device %d: %s", dev, hipGetErrorString(e));
+            return nullptr;
+        }
+        g_static_scratch[dev] = p;
+    }
+    return g_static_scratch[dev];
+}
+
+}  // namespace dbk_scanpool_digits
+
+extern "C" int dbk_scanpool_fprop_kmer_static(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter,
+                                              const uint8_t* X, size_t N, const uint32_t* regions, size_t nregion, int ptype,
+                                              float* pooled, uint32_t* argmax)
+{
+    using namespace dbk_scanpool_digits;
+    DBK_CHECK(m >= 1, "ValueError: filter length must be >= 1");
+    if (nfilter == 0 || nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(W && bias && X && regions && pooled, "ValueError: null pointer argument");
+    DBK_CHECK(!(argmax && ptype == DBK_PT_AVG), "ValueError: pooledmaps_argmax can only be used for max/all pooling.");
+    DBK_CHECK(!argmax || (double)N * (double)nfilter <= 4294967296.0,
+              "ValueError: %zu rows x %zu filters overflow the 32-bit argmax index; score in smaller batches or without argmax", N, nfilter);
+    DBK_CHECK(N <= STATIC_SEQUENCE_BYTES,
+              "ValueError: %zu sequence bytes; the entry point with the built-in buffer takes at most %zu per call; "
+              "score in smaller batches or call dbk_scanpool_fprop_kmer", N, STATIC_SEQUENCE_BYTES);
+    unsigned char* ws = static_scratch();
+    if (!ws) return 2;
+    // The flags and the digits are rewritten from the weights by the call's first launch, so nothing of an earlier call's
+    // contents is read.
+    int rc = fprop_impl(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax, true, ws);
+    DBK_CHECK(rc >= 0, "NotImplementedError: the bulk path takes max / avg / all pooling and filter length <= 24");
+    return rc;
+}
+
+extern "C" int dbk_scanpool_fprop_kmer(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter,
+                                       const uint8_t* X, size_t N, const uint32_t* regions, size_t nregion, int ptype,
+                                       float* pooled, uint32_t* argmax)
+{
+    DBK_CHECK(m >= 1, "ValueError: filter length must be >= 1");
+    if (nfilter == 0 || nregion == 0) { dbk::clear_error(); return 0; }
+    DBK_CHECK(W && bias && X && regions && pooled, "ValueError: null pointer argument");
+    DBK_CHECK(!(argmax && ptype == DBK_PT_AVG), "ValueError: pooledmaps_argmax can only be used for max/all pooling.");
+    DBK_CHECK(!argmax || (double)N * (double)nfilter <= 4294967296.0,
+              "ValueError: %zu rows x %zu filters overflow the 32-bit argmax index; score in smaller batches or without argmax", N, nfilter);
+    int rc = dbk_scanpool_digits::fprop_impl(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax, true);
+    DBK_CHECK(rc >= 0, "NotImplementedError: the bulk path takes max / avg / all pooling and filter length <= 24");
+    return rc;
+}

@@ -172,9 +172,9 @@ def scanpool_fprop(W, b, X, regions, ptype, want_argmax=False, path="auto", act=
     path: "auto" lets the library choose; "general" / "mfma" / "wide" / "kmer" force the general path (which picks its
     kernel by size), its matrix-core kernel for many regions (filters of up to 32 taps; sums in another order than
     the lookup kernels', equal to round-off), the four-filters-per-lane lookup kernel (9-24 taps; the bits of the
-    one-filter-per-lane kernel) or the table kernel; "kmer_static" is the table kernel
-    with the scratch buffer that is built into the library (no allocation inside the call; at most 64 MiB of
-    sequence bytes; calls that overlap on one GPU must not use it together).
+    one-filter-per-lane kernel) or the bulk kernel (6-bit digits on the matrix cores, filters of up to 24 taps);
+    "kmer_static" is the bulk kernel with the scratch buffer that is built into the library (no allocation inside the
+    call; at most 64 MiB of sequence bytes; calls that overlap on one GPU must not use it together).
     out (optional): (pooled, argmax|None) tensors to write into instead of new ones, so that the call allocates nothing.
     act (optional, from activity_words): receives 1 bit per row and filter - rectifier open or not - which
     scanpool_bprop takes in place of recomputing the map (general kernel only).
@@ -210,7 +210,7 @@ def scanpool_fprop(W, b, X, regions, ptype, want_argmax=False, path="auto", act=
     if path not in ("kmer", "kmer_static"):
         args.append(_act(act, X, F))
     else:
-        require(act is None, "ValueError: the table kernel does not write activity masks")
+        require(act is None, "ValueError: the bulk kernel does not write activity masks")
     call(entry, *args)
     return pooled, argmax
 

@@ -135,7 +135,7 @@ int dbk_dropoutord_mirror(dbk_stream_t stream, const uint8_t* X, uint8_t* Z, uin
  * every tile of 64 filters, the mask of filters whose rectifier is open there (bit l = filter tile*64 + l):
  * what the reference's relu node keeps as its output for the backward pass (elemwise.py:78), 1 bit per
  * value. Hand it to dbk_scanpool_bprop and the average-pooling gradient needs no recomputation. With act
- * the general kernel runs (the table kernel does not write it). */
+ * the general kernel runs (the bulk kernel does not write it). */
 int dbk_scanpool_fprop(dbk_stream_t stream,
                        const float* W, const float* bias, size_t m, size_t nfilter,
                        const uint8_t* X, size_t N,
@@ -172,9 +172,11 @@ int dbk_scanpool_fprop_mfma(dbk_stream_t stream,
                             const uint32_t* regions, size_t nregion, int ptype,
                             float* pooled, uint32_t* argmax, uint64_t* act);
 
-/* Same contract through the 3-mer lookup-table kernel regardless of problem size; fails with
- * NotImplementedError for shapes that kernel does not take (filter length > 24, avg/all pooling,
- * argmax requested). Inputs it cannot express (code 254, regions outside the sequence) are detected
+/* Same contract through the bulk kernel regardless of problem size (dbk_scanpool_fprop picks it for scoring calls of
+ * some 10^5 rows x filter tiles on, for filters of up to 32 taps): the scan as a product of the windows' one-hot letters
+ * with the weights as six 6-bit digits each on the matrix cores, accumulated in float32 (v_mfma_scale_f32_32x32x64_f8f6f4).
+ * Fails with NotImplementedError for shapes this entry point does not take (filter length > 24, sum pooling). Filters whose
+ * weights the digits do not express (infinite or undefined ones, one positive weight far beyond all others) are detected
  * on the device and computed by the general kernel inside the same call. */
 int dbk_scanpool_fprop_kmer(dbk_stream_t stream,
                             const float* W, const float* bias, size_t m, size_t nfilter,
@@ -184,9 +186,9 @@ int dbk_scanpool_fprop_kmer(dbk_stream_t stream,
 
 /* dbk_scanpool_fprop_kmer for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid allocation): same arguments, same kernels, same results, but the call's
- * scratch (a flag word and one index byte per sequence byte) lies in a buffer that is part of the loaded
+ * scratch (the weights' digits) lies in a buffer that is part of the loaded
  * library instead of a grow-on-demand allocation, so the call never allocates, frees or synchronises.
- * Limit: N <= 64 MiB of sequence bytes per call (ValueError beyond; the buffer's 64.0005 MiB are held on every
+ * Limit: N <= 64 MiB - 127 sequence bytes per call (ValueError beyond; the buffer's 29 MiB are held on every
  * GPU the library runs on until the process ends). All calls on one GPU share the buffer: calls that overlap
  * on one GPU (different streams, different host threads) race; calls ordered on one stream do not.
  * No counterpart in the reference (its wrappers allocate per call, kangaroo/_ext/kangaroo_smat.py:121-132). */

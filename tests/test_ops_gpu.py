@@ -1126,6 +1126,99 @@ def test_scanpool_kmer_argmax_takes_the_first_of_exactly_equal_rows(ks):
         assert np.array_equal(host(I) % F, np.broadcast_to(np.arange(F), (2, F)))
 
 
+def _bulk_case(seed, rows, m, F, odd_codes=True):
+    """Regions of exactly the given numbers of rows (0 allowed), every letter code among the bytes."""
+    rng = np.random.default_rng(seed)
+    edges = np.concatenate([[0], np.cumsum(rows)])
+    X = rng.integers(0, 4, int(edges[-1]) + m - 1).astype(np.uint8)
+    X[rng.random(X.size) < 0.03] = 255
+    if odd_codes:
+        X[rng.random(X.size) < 0.02] = 254
+        k = rng.random(X.size) < 0.02
+        X[k] = rng.choice([4, 5, 77, 251, 252, 253], int(k.sum()))
+    R = np.stack([edges[:-1], edges[1:]], axis=1).astype(np.uint32)
+    W = (rng.standard_normal((4 * m, F)) * 0.1).astype(np.float32)
+    b = (rng.standard_normal((1, F)) * 0.05 - 0.02).astype(np.float32)
+    return rng, W, b, X.reshape(-1, 1), R
+
+
+def _within_rounding(got, want, W, b, ptype):
+    """float32 sums of m + 1 terms, then a mean: every rounding is at most 2^-24 of the sum of the terms' sizes, the mean's
+    partial sums (16 rows, tiles, two halves) add some 50 more."""
+    m = W.shape[0] // 4
+    size = np.abs(W.astype(np.float64)).reshape(m, 4, -1).max(axis=1).sum(axis=0) + np.abs(b.ravel().astype(np.float64))
+    bound = (m + 50) * 2.0 ** -24 * np.repeat(size, 2 if ptype == "all" else 1)
+    assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m,F", [(1, 32), (7, 33), (8, 16), (9, 64), (16, 31), (17, 40), (24, 96)])
+def test_bulk_scan_at_the_edges_of_its_tiles(ks, ptype, m, F):
+    """Regions that end one row before, at and after a tile of 32 rows and a staged stretch of 224, codes that are no
+    letter, rows past the stream's last window, streams and tables off their natural boundaries."""
+    rows = [1, 31, 32, 33, 63, 64, 65, 223, 224, 225, 255, 256, 257, 447, 448, 449, 480, 2, 700]
+    rng, W, b, X, R = _bulk_case(100 + m, rows, m, F)
+    R[-1, 1] = X.size                                                   # the last region runs into rows the scan does not define
+    A, Pr, Ir = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
+    store, table = dev(np.concatenate([[np.uint8(9)], X.ravel()])), dev(np.concatenate([[0], R.view(np.int32).ravel()]).astype(np.int32))
+    for Xd, Rd in ((dev(X), dev(R)), (store[1:].view(-1, 1), table[1:].view(-1, 2))):
+        Rd = Rd if Rd.dtype == dev(R).dtype else Rd.view(dev(R).dtype)
+        P, _ = ks.scanpool_fprop(dev(W), dev(b), Xd, Rd, ptype, path="kmer")
+        _within_rounding(host(P), Pr, W, b, ptype)
+        if ptype != "avg":
+            Pa, I = ks.scanpool_fprop(dev(W), dev(b), Xd, Rd, ptype, want_argmax=True, path="kmer")
+            assert np.array_equal(host(Pa), host(P))
+            moved = host(I) != Ir
+            assert np.abs(A.ravel()[host(I)[moved]] - A.ravel()[Ir[moved]]).max(initial=0.0) <= 1e-5
+    empty = np.concatenate([R[:3], [[5, 5]], R[3:5]]).astype(np.uint32)
+    P, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(empty), ptype, path="kmer")
+    Pg, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(empty), ptype, path="general")
+    assert np.array_equal(np.isnan(host(P)), np.isnan(host(Pg))) and np.allclose(host(P), host(Pg), rtol=0, atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [25, 29, 32])
+def test_bulk_scan_of_25_to_32_taps(ks, ptype, m):
+    """The longest filters reach the bulk kernel by the library's own choice: few rows of very many filters."""
+    F = 64 * 320
+    rng, W, b, X, R = _bulk_case(40 + m, [300, 1, 33, 224, 500, 64, 900], m, F)
+    P, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype)
+    pick = np.sort(rng.choice(F, 96, replace=False))
+    _, Pr, _ = _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R, ptype)
+    cols = pick if ptype != "all" else np.stack([2 * pick, 2 * pick + 1], axis=1).ravel()
+    _within_rounding(host(P)[:, cols], Pr, W[:, pick], b[:, pick], ptype)
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+def test_bulk_scan_leaves_weights_it_cannot_express_to_the_general_kernel(ks, ptype):
+    """Filters with infinite or undefined weights, one weight or bias beyond all others, or sizes near the type's ends sit
+    between ordinary ones; weights far below zero (they only close their windows) are expressed."""
+    m, F = 16, 130
+    rng, W, b, X, R = _bulk_case(9, [40, 300, 33, 224, 64], m, F, odd_codes=False)
+    W[5, 3] = np.inf                                                    # filters 0-63: the general kernel's
+    W[:, 40] *= 1e-30
+    W[9, 41] = 1e6
+    W[7, 70] = -np.inf                                                  # filters 64-129: expressed
+    W[:, 71] = -np.abs(W[:, 71])
+    W[20, 72] = -1e9
+    W[:, 73] = 0.0
+    W[:, 74] *= 1e10
+    W[:, 75] *= 1e-20
+    b[0, 76] = -0.6
+    Wd, bd, Xd, Rd = dev(W), dev(b), dev(X), dev(R)
+    P, _ = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, path="kmer")
+    want = ptype != "avg"
+    I = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, want_argmax=want, path="kmer")[1]
+    k = 2 if ptype == "all" else 1
+    Pg, Ig = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, want_argmax=want, path="general")
+    P, Pg = host(P), host(Pg)
+    assert np.array_equal(P[:, :64 * k], Pg[:, :64 * k], equal_nan=True)
+    scale = np.maximum(np.abs(Pg).max(axis=0), 1e-30)
+    assert np.all(np.abs(P - Pg)[:, 64 * k:] <= 1e-5 * scale[64 * k:]) and np.all(P[:, 71 * k:72 * k][:, :1] >= 0)
+    if want:
+        assert (host(I) == host(Ig)).mean() > 0.99
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
