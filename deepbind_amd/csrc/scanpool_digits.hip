@@ -51,13 +51,13 @@ int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F,
 namespace dbk_scanpool_digits {
 
 using dbk_mfma::f32x16_t;
-using dbk_mfma::load_letters4;
 
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 
 constexpr int FTILE = 32;                     // filters per workgroup: columns of a tile
 constexpr int ROWS = 32;                      // positions per tile
 constexpr int NDIGIT = 6;                     // digits per weight
+constexpr int NTOP = 3;                       // of them, the first ones that find a maximum's place
 constexpr int NWAVE = 16;                     // waves per workgroup
 constexpr unsigned CHUNK = 224;               // rows whose letters are staged at a time: seven tiles
 constexpr unsigned ENTRIES = 304;             // entries of a wave: 256 positions, one entry of padding per 16, what a read past the last tile touches
@@ -69,16 +69,46 @@ __device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
 
 // ---------------------------------------------------------------------------------------------- the weights' digits
 // What a call keeps in its scratch, per tile of 32 filters: a flag (not expressible: the general kernel's), the filters'
-// exponents and the digits, [8-tap block][digit][filter][24 bytes].
-struct digit_store { unsigned* flags; int* expo; unsigned char* digits; };
-inline size_t tile_bytes(unsigned tb) { return FTILE * sizeof(int) + (size_t)tb * NDIGIT * SLOT_BYTES; }
-inline digit_store store_at(unsigned* flags, unsigned char* ws, unsigned ntile)
+// exponents, the digits, [8-tap block][digit][filter][24 bytes], and, to find a maximum's place, NTOP digits per weight in
+// units of the filter's own (no power of two) with what the scan has to know of them.
+struct digit_facts {
+    float unit;         // digit NTOP - 1's step
+    float above;        // the most that a window's weights lie above those digits, in units, and some slack
+    float lowest;       // weights below count as this
+    int whole;          // weights times 2^whole add up to less than 2^30 over any window
+};
+struct digit_store { unsigned* flags; int* expo; digit_facts* facts; unsigned char *digits, *top; };
+inline size_t tile_bytes(unsigned tb) { return FTILE * (sizeof(int) + sizeof(digit_facts)) + (size_t)tb * (NDIGIT + NTOP) * SLOT_BYTES; }
+inline digit_store store_at(unsigned* flags, unsigned char* ws, unsigned ntile, unsigned tb)
 {
     digit_store s;
     s.flags = flags;
     s.expo = reinterpret_cast<int*>(ws);
-    s.digits = ws + (size_t)ntile * FTILE * sizeof(int);
+    s.facts = reinterpret_cast<digit_facts*>(s.expo + (size_t)ntile * FTILE);
+    s.digits = reinterpret_cast<unsigned char*>(s.facts + (size_t)ntile * FTILE);
+    s.top = s.digits + (size_t)ntile * tb * NDIGIT * SLOT_BYTES;
     return s;
+}
+
+// x, of magnitude up to 16.5, as ND digits base 32, each the nearest whole number; what remains, in units of the next digit
+template <int ND>
+__device__ __forceinline__ void split_digits(float (&x)[4], unsigned char* o)
+{
+#pragma unroll
+    for (int p = 0; p < ND; ++p) {
+        unsigned word = 0u;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float d = rintf(x[c]);
+            x[c] = (x[c] - d) * 32.0f;                            // (exact)
+            const int i = (int)d;
+            const unsigned a = (unsigned)(i < 0 ? -i : i);
+            // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 15 are their own codes (denormal below 8), 16 is code 16
+            word |= (a | (i < 0 ? 32u : 0u)) << (6 * c);
+        }
+        unsigned char* q = o + (size_t)p * SLOT_BYTES;
+        q[0] = (unsigned char)word; q[1] = (unsigned char)(word >> 8); q[2] = (unsigned char)(word >> 16);
+    }
 }
 
 // A workgroup splits one tile's weights: thread (g, fl) takes taps g, 8 + g, .. of filter fl. Latency only (4m x 32 values).
@@ -86,8 +116,8 @@ template <int TB>
 __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restrict__ W, const float* __restrict__ bias, unsigned m, unsigned F,
                                                             unsigned f0, digit_store out)
 {
-    __shared__ float red[5][8][FTILE];                            // sums and maxima of the eight threads of a filter
-    __shared__ unsigned char dig[TB * NDIGIT * SLOT_BYTES];
+    __shared__ float red[6][8][FTILE];                            // sums and maxima of the eight threads of a filter
+    __shared__ unsigned char dig[TB * (NDIGIT + NTOP) * SLOT_BYTES];
     __shared__ unsigned bad_tile;
     const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
     if (threadIdx.x == 0) bad_tile = 0u;
@@ -101,6 +131,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         }
     const float b = f < F ? bias[f] : 0.0f;
     float open = 0.0f, top = 0.0f, second = 0.0f, low = 0.0f;     // sum of the taps' best, the two largest weights, the most negative one
+    float size = 0.0f;                                            // sum of the taps' largest magnitudes
     bool bad = (__float_as_uint(b) & 0x7fffffffu) >= 0x71000000u;     // (the file is compiled without NaN: test the bits)
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
@@ -136,33 +167,58 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
     bad = nbad > 0.0f || (second > 0.0f && top > 64.0f * second) || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-25f);
     if (!bad && big != 0.0f) e = (int)((__float_as_uint(big) >> 23) & 0xffu) - 127;
     if (bad) bad_tile = 1u;                                       // (every writer writes the same)
-    // digits: x = w * 2^(3 - e) is below 16, each digit the nearest whole number, the remainder (exact) times 32
-    const float scale = __uint_as_float((unsigned)(127 + 3 - e) << 23);
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
-        float x[4];
+        float z = 0.0f;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) x[c] = bad ? 0.0f : fmaxf(w[t][c], floor_) * scale;
-#pragma unroll
-        for (int p = 0; p < NDIGIT; ++p) {
-            unsigned word = 0u;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float d = rintf(x[c]);
-                x[c] = (x[c] - d) * 32.0f;
-                const int i = (int)d;
-                const unsigned a = (unsigned)(i < 0 ? -i : i);
-                // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 15 are their own codes (denormal below 8), 16 is code 16
-                word |= (a | (i < 0 ? 32u : 0u)) << (6 * c);
-            }
-            unsigned char* o = dig + ((size_t)(t * NDIGIT + p) * FTILE + fl) * 24u + 3u * g;
-            o[0] = (unsigned char)word; o[1] = (unsigned char)(word >> 8); o[2] = (unsigned char)(word >> 16);
+        for (int c = 0; c < 4; ++c) {
+            w[t][c] = bad ? 0.0f : fmaxf(w[t][c], floor_);
+            z = fmaxf(z, fabsf(w[t][c]));
         }
+        size += z;
     }
+    red[5][g][fl] = size;
     __syncthreads();
+    size = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) size += red[5][k][fl];
+    // all the digits: x = w * 2^(3 - e), below 16. The first ones by themselves: x = w / unit with a window's x at most
+    // 240 (so that its sum, in 1/1024, leaves room for a row's number below it: see the scan) and a weight's at most 16.4
+    const float scale = __uint_as_float((unsigned)(127 + 3 - e) << 23);
+    const float finest = bad ? 1.0f : fmaxf(fmaxf(size * (1.0f / 240.0f), big * (1.0f / 16.4f)), 1.0e-30f), per = 1.0f / finest;
+    float above = 0.0f;                                           // the most that the weights exceed those digits by, in units of the next digit
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        float x[4], y[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { x[c] = w[t][c] * scale; y[c] = w[t][c] * per; }
+        split_digits<NDIGIT>(x, dig + ((size_t)t * NDIGIT * FTILE + fl) * 24u + 3u * g);
+        split_digits<NTOP>(y, dig + ((size_t)(TB * NDIGIT + t * NTOP) * FTILE + fl) * 24u + 3u * g);
+        above += fmaxf(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])), 0.0f);     // (a letter that counts nothing exceeds nothing)
+    }
+    red[0][g][fl] = above;
+    __syncthreads();
+    const unsigned* src = reinterpret_cast<const unsigned*>(dig);
     unsigned* dst = reinterpret_cast<unsigned*>(out.digits + (size_t)blockIdx.x * (TB * NDIGIT * SLOT_BYTES));
-    for (unsigned i = threadIdx.x; i < TB * NDIGIT * SLOT_BYTES / 4; i += 256) dst[i] = reinterpret_cast<const unsigned*>(dig)[i];
-    if (g == 0) out.expo[blockIdx.x * FTILE + fl] = e;
+    for (unsigned i = threadIdx.x; i < TB * NDIGIT * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
+    src += TB * NDIGIT * SLOT_BYTES / 4;
+    dst = reinterpret_cast<unsigned*>(out.top + (size_t)blockIdx.x * (TB * NTOP * SLOT_BYTES));
+    for (unsigned i = threadIdx.x; i < TB * NTOP * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
+    if (g == 0) {
+        above = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) above += red[0][k][fl];
+        out.expo[blockIdx.x * FTILE + fl] = e;
+        digit_facts k;
+        k.unit = finest * (1.0f / 1024.0f);
+        // a quarter of a unit for the rows' numbers, a quarter for the rounding of a window's sum and of the scaled weights
+        // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
+        k.above = above * (1.00001f / 32.0f) + 0.5f;
+        k.lowest = floor_;
+        const int se = size > 0.0f ? (int)((__float_as_uint(size) >> 23) & 0xffu) - 127 : 0;
+        k.whole = 29 - se;                                        // size < 2^(se + 1)
+        out.facts[blockIdx.x * FTILE + fl] = k;
+    }
     if (threadIdx.x == 0) out.flags[blockIdx.x] = bad_tile;
 }
 
@@ -188,17 +244,99 @@ __device__ __forceinline__ unsigned plain_codes(unsigned v)
     return r;
 }
 
+// B bytes of X from o on, which run past its end: bytes past the end are undefined (they only reach windows that are closed).
+// Kept small and out of the way: only a stream's last stretches come here.
+template <int B>
+__device__ __forceinline__ void load_tail(const uint8_t* __restrict__ X, size_t N, size_t o, unsigned (&v)[B / 4])
+{
+#pragma unroll
+    for (int k = 0; k < B / 4; ++k) v[k] = 0u;
+#pragma unroll 1
+    for (unsigned i = 0; i < B; ++i) {
+        const unsigned c = o + i < N ? X[o + i] : 0u;
+#pragma unroll
+        for (int k = 0; k < B / 4; ++k) v[k] |= (i >> 2) == (unsigned)k ? c << (8u * (i & 3u)) : 0u;
+    }
+}
+
+// The twelve letters from position c + 4 * lane on.
+__device__ __forceinline__ void load12(const uint8_t* __restrict__ X, size_t N, unsigned c, unsigned lane, unsigned (&v)[3])
+{
+    const size_t o = (size_t)c + 4u * lane;
+    if ((size_t)c + 4u * 63u + 12u <= N) __builtin_memcpy(v, X + o, 12);
+    else load_tail<12>(X, N, o, v);
+}
+
+// A wave's 256 positions (each lane: its twelve letters) into its entries: the nibbles of eight letters per position.
+__device__ __forceinline__ void stage(uint4* entries, unsigned lane, unsigned (&v)[3])
+{
+    if (__any((odd_codes(v[0]) | odd_codes(v[1]) | odd_codes(v[2])) != 0u)) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[k] = plain_codes(v[k]);
+    }
+    const uint2 n0 = letter_nibbles(v[0]), n1 = letter_nibbles(v[1]), n2 = letter_nibbles(v[2]);
+    const unsigned p[6] = {n0.x, n0.y, n1.x, n1.y, n2.x, n2.y};
+    unsigned q[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) q[k] = __builtin_amdgcn_alignbit(p[k + 1], p[k], 16);
+    uint4* dst = entries + place(4u * lane);
+    __builtin_amdgcn_wave_barrier();
+    dst[0] = make_uint4(p[0], p[1], p[2], p[3]);
+    dst[1] = make_uint4(q[0], q[1], q[2], q[3]);
+    dst[2] = make_uint4(p[1], p[2], p[3], p[4]);
+    dst[3] = make_uint4(q[1], q[2], q[3], q[4]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The next region of the workgroup's, the same in all lanes.
+__device__ __forceinline__ unsigned claim(unsigned* counter, unsigned lane)
+{
+    unsigned v = 0u;
+    if (lane == 0u) v = atomicAdd(counter, 1u);
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
+}
+
+// Where a lane's operands lie: tile t of a staged stretch reads entries 34 t + these (34 entries per 32 positions). The
+// first holds its half wave's block of taps 0-15, the second that of taps 16-31.
+template <int TB> __device__ __forceinline__ unsigned first_operand(unsigned col, unsigned h) { return place(col + (TB >= 2 ? 8u * h : 0u)); }
+template <int TB> __device__ __forceinline__ unsigned second_operand(unsigned col, unsigned h) { return place(col + 16u + (TB == 4 ? 8u * h : 0u)); }
+
+// Rows from c on that the scan defines, as far as a staged stretch is concerned.
+__device__ __forceinline__ unsigned defined_rows(size_t ndef, unsigned c)
+{
+    return (size_t)c >= ndef ? 0u : (ndef - c < 2 * CHUNK ? (unsigned)(ndef - c) : 2 * CHUNK);
+}
+// Rows the scan does not define hold the rectified bias: no letter in their windows. Only the stream's last tiles come here;
+// the empty statement keeps it a branch (as selects it would be a third of a tile's vector instructions).
+__device__ __forceinline__ void close_undefined(uint4& a0, uint4& a1, bool defined)
+{
+    asm volatile("");
+    if (!defined) { a0 = make_uint4(0u, 0u, 0u, 0u); a1 = a0; }
+}
+
 // ---------------------------------------------------------------------------------------------- the products
 // instructions per tile: two 8-tap blocks (one per half wave) or two digits of one block at a time
 template <int TB> struct product_count { static constexpr int N = TB == 1 ? 3 : (TB == 2 ? 6 : (TB == 3 ? 9 : 12)); };
 
+// (operand formats 4: 4-bit, and 2: 6-bit with two exponent bits; a scale is a power of two plus 127)
 template <int SEL>
-__device__ __forceinline__ f32x16_t product(const uint4& a, const unsigned (&b)[6], const f32x16_t& c, int scale)
+__device__ __forceinline__ f32x16_t product(const uint4& a, const unsigned (&b)[6], const f32x16_t& c, int scale, int one = 125)
 {
     const i32x8_t av = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
     const i32x8_t bv = {(int)b[0], (int)b[1], (int)b[2], (int)b[3], (int)b[4], (int)b[5], 0, 0};
-    // operand formats 4 (4-bit) and 2 (6-bit, two exponent bits); scale bytes are exponents + 127: 125 makes the 4.0 a one
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 4, 2, 0, 125, SEL, scale);
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, 4, 2, 0, one, SEL, scale);      // (one = 2^-2: the 4.0 of a letter)
+}
+
+// Block scales of a filter of exponent `expo`: digit p counts 2^(expo - 3 - 5 p) and is stored in eighths. s[0] and s[1]: the
+// digits one by one; s[2]: pairs of digits 2 j, 2 j + 1 of one block, this half wave's.
+__device__ __forceinline__ void digit_scales(int expo, unsigned h, int (&s)[3])
+{
+    const int e = expo + 127, eh = e - 5 * (int)h;
+    s[0] = (e & 255) | ((e - 5) & 255) << 8 | ((e - 10) & 255) << 16 | (int)((unsigned)((e - 15) & 255) << 24);
+    s[1] = ((e - 20) & 255) | ((e - 25) & 255) << 8;
+    s[2] = (eh & 255) | ((eh - 10) & 255) << 8 | ((eh - 20) & 255) << 16;
 }
 
 // which 8-tap block and digit the half wave h holds in operand i of a tile (operands in the order they are multiplied:
@@ -212,6 +350,20 @@ template <int TB> __device__ __forceinline__ void operand_slot(int i, unsigned h
         if (k < 2) { block = h; digit = 2 * j + 1 - k; }
         else { block = 2u; digit = 2u * j + h; }
     } else { block = (i & 1 ? 2u : 0u) + h; digit = 5 - i / 2; }
+}
+
+// a lane's operands: column `col` of the weights, the half wave's 32 rows of every product
+template <int TB>
+__device__ __forceinline__ void load_operands(const unsigned char* digits, unsigned col, unsigned h, unsigned (&B)[product_count<TB>::N][6])
+{
+#pragma unroll
+    for (int i = 0; i < product_count<TB>::N; ++i) {
+        unsigned block, digit;
+        operand_slot<TB>(i, h, block, digit);
+        const uint2* src = reinterpret_cast<const uint2*>(digits + ((block * NDIGIT + digit) * FTILE + col) * 24u);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { const uint2 v = src[k]; B[i][2 * k] = v.x; B[i][2 * k + 1] = v.y; }
+    }
 }
 
 template <int TB, int I>
@@ -246,53 +398,22 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
     // this workgroup's regions
     const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
     if (threadIdx.x == 0) counter[0] = lo;
-    // ---- this lane's operands: column `col` of the weights, the half wave's 32 rows of every product
     unsigned B[NI][6];
-    {
-        const unsigned char* dig = D.digits + (size_t)tile * (TB * NDIGIT * SLOT_BYTES);
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            unsigned block, digit;
-            operand_slot<TB>(i, h, block, digit);
-            const uint2* src = reinterpret_cast<const uint2*>(dig + ((size_t)(block * NDIGIT + digit) * FTILE + col) * 24u);
-            const uint2 q0 = src[0], q1 = src[1], q2 = src[2];
-            B[i][0] = q0.x; B[i][1] = q0.y; B[i][2] = q1.x; B[i][3] = q1.y; B[i][4] = q2.x; B[i][5] = q2.y;
-        }
-    }
-    // block scales: digit p counts 2^(e - 3 - 5 p), stored in eighths
-    const int e = D.expo[tile * FTILE + col] + 127;
+    load_operands<TB>(D.digits + (size_t)tile * (TB * NDIGIT * SLOT_BYTES), col, h, B);
     int s[3];
-    s[0] = (e & 255) | ((e - 5) & 255) << 8 | ((e - 10) & 255) << 16 | (int)((unsigned)((e - 15) & 255) << 24);
-    s[1] = ((e - 20) & 255) | ((e - 25) & 255) << 8;
-    const int eh = e - 5 * (int)h;                                // pairs of digits of one block: 2 j + h
-    s[2] = (eh & 255) | ((eh - 10) & 255) << 8 | ((eh - 20) & 255) << 16;
+    digit_scales(D.expo[tile * FTILE + col], h, s);
     const unsigned f = f0 + tile * FTILE + col;
     const float bf = f < F ? bias[f] : 0.0f;
     const unsigned rg = 4u * h;                                   // this half wave's rows lie 4 further down
-    // operands are read from entry tile * 34 + these (34 entries per 32 positions)
-    const unsigned at0 = place(col + (TB >= 2 ? 8u * h : 0u)), at1 = place(col + 16u + (TB == 4 ? 8u * h : 0u));
+    const unsigned at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
     __syncthreads();
 
-    auto claim = [&]() -> unsigned {
-        unsigned v = 0u;
-        if (lane == 0u) v = atomicAdd(counter, 1u);
-        return (unsigned)__builtin_amdgcn_readfirstlane((int)v);
-    };
-    // 12 letters from position c + 4 * lane on
-    auto load12 = [&](unsigned c, unsigned (&v)[3]) {
-        const size_t o = (size_t)c + 4u * lane;
-        if ((size_t)c + 4u * 63u + 12u <= N) __builtin_memcpy(v, X + o, 12);
-        else {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) v[k] = load_letters4(X, N, o + 4 * k);
-        }
-    };
-    unsigned r = claim(), rn = claim();                           // the region in work, the one after it
+    unsigned r = claim(counter, lane), rn = claim(counter, lane);                           // the region in work, the one after it
     unsigned a = 0u, b = 0u, an = 0u, bn = 0u;
     if (r < hi) { a = R[2 * (size_t)r]; b = R[2 * (size_t)r + 1]; }
     if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
     unsigned letters[3] = {0u, 0u, 0u};
-    if (r < hi) load12(a, letters);
+    if (r < hi) load12(X, N, a, lane, letters);
 
     while (r < hi) {
         float mx = CLOSED, sum = 0.0f;
@@ -302,37 +423,17 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
         do {
             const unsigned left = b > c ? b - c : 0u;             // rows of the region from this chunk on
             last = left <= CHUNK;
-            // ---- the chunk's entries
-            if (__any((odd_codes(letters[0]) | odd_codes(letters[1]) | odd_codes(letters[2])) != 0u)) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) letters[k] = plain_codes(letters[k]);
-            }
-            const uint2 n0 = letter_nibbles(letters[0]), n1 = letter_nibbles(letters[1]), n2 = letter_nibbles(letters[2]);
-            const unsigned p[6] = {n0.x, n0.y, n1.x, n1.y, n2.x, n2.y};
-            unsigned q[5];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) q[k] = __builtin_amdgcn_alignbit(p[k + 1], p[k], 16);
-            uint4* dst = entries + place(4u * lane);
-            __builtin_amdgcn_wave_barrier();
-            dst[0] = make_uint4(p[0], p[1], p[2], p[3]);
-            dst[1] = make_uint4(q[0], q[1], q[2], q[3]);
-            dst[2] = make_uint4(p[1], p[2], p[3], p[4]);
-            dst[3] = make_uint4(q[1], q[2], q[3], q[4]);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            stage(entries, lane, letters);
             // the next chunk's letters travel while this one is multiplied
-            if (!last) load12(c + CHUNK, letters);
-            else if (rn < hi) load12(an, letters);
+            if (!last) load12(X, N, c + CHUNK, lane, letters);
+            else if (rn < hi) load12(X, N, an, lane, letters);
             // ---- its tiles
             const unsigned nrow = last ? left : CHUNK;
+            const unsigned defined = defined_rows(ndef, c);
             const uint4* src = entries;
             for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34) {
                 uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
-                if ((size_t)c + t0 + ROWS > ndef) {
-                    // rows the scan does not define hold the rectified bias
-                    if ((size_t)c + t0 + col >= ndef) { a0 = make_uint4(0u, 0u, 0u, 0u); a1 = a0; }
-                }
+                if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
                 f32x16_t z;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) z[i] = 0.0f;
@@ -386,9 +487,336 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
             if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + xi) * F + f);
         }
         r = rn; a = an; b = bn;
-        rn = claim();
+        rn = claim(counter, lane);
         if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
     }
+}
+
+// ---------------------------------------------------------------------------------------------- plain maxima
+// Max pooling with filters of 17 to 32 taps: half the products. A region's maximum is one window, so the products only have
+// to find its place; its value is then added up from the weights themselves (whole numbers of 2^-30 of the largest sum that
+// a window can have: one rounding in the end). The first NTOP digits of every weight give every
+// window's sum to within what the digits left out can amount to. The value of the largest sum's window being known, it is
+// the maximum unless the second largest sum plus the most that the left out digits can add to any window (`above`, per
+// filter) reaches it. Where that is so (0.1 % of the filters and regions of 500 random letters, and windows that repeat),
+// the region is scanned once more with all the digits for the 32 filters concerned.
+//
+// Sums of NTOP digits are whole numbers of 1/4 unit (a "mean of the four" counts quarters) below 2^18 units, which leaves
+// float32 four bits below: a lane's 16 rows start from 15/64 .. 0 units instead of zero, so the maximum carries its row's
+// number with it, and a tile only notes that it was the best so far. The second largest comes with the largest: v_max3 and
+// v_med3 give the top two of three, 20 instructions for a tile's 16 rows and the two so far.
+//
+// A wave takes 64 filters at a time (the staging of the letters, the operand reads and the walk serve both halves), 12
+// waves per workgroup: three per SIMD at up to 168 registers. At a region's end lanes 0-31 hold the
+// first 32 filters and lanes 32-63 the others, and each adds up its own filter's window.
+constexpr int MAX_WAVES = 12;
+constexpr int PAIR = 2 * FTILE;               // filters per workgroup
+
+template <int TB> struct place_count { static constexpr int N = TB == 3 ? 5 : 6; };
+
+// which block and digit operand i of a tile holds; digit NTOP stands for an empty half
+template <int TB> __device__ __forceinline__ void place_slot(int i, unsigned h, unsigned& block, unsigned& digit)
+{
+    if (TB == 3) {
+        if (i < 3) { block = h; digit = 2 - i; }
+        else { block = 2u; digit = i == 3 ? 1u + h : (h ? (unsigned)NTOP : 0u); }
+    } else { block = (i & 1 ? 2u : 0u) + h; digit = 2 - i / 2; }
+}
+
+// In units of digit NTOP - 1: the digits' scales are the same for every filter. single: digits 0, 1, 2 by byte; pair: bytes
+// for this half wave's digits (0, none) and (1, 2).
+template <int TB>
+__device__ __forceinline__ f32x16_t place_sums(const f32x16_t& rows, const uint4& a0, const uint4& a1, const unsigned (&B)[place_count<TB>::N][6], int single, int pair)
+{
+    f32x16_t z;
+    if constexpr (TB == 3) {
+        z = product<2>(a0, B[0], rows, single);
+        z = product<1>(a0, B[1], z, single);
+        z = product<0>(a0, B[2], z, single);
+        z = product<1>(a1, B[3], z, pair);
+        z = product<0>(a1, B[4], z, pair);
+    } else {
+        z = product<2>(a0, B[0], rows, single);
+        z = product<1>(a0, B[2], z, single);
+        z = product<0>(a0, B[4], z, single);
+        z = product<2>(a1, B[1], z, single);
+        z = product<1>(a1, B[3], z, single);
+        z = product<0>(a1, B[5], z, single);
+    }
+    return z;
+}
+
+// The maximum over a region from all the digits, and its row: this half wave's, without the bias.
+template <bool WANT_ARGMAX, int TB>
+__device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, size_t N, size_t ndef, unsigned a, unsigned b, uint4* entries,
+                                              const unsigned char* digits, unsigned lane, int expo)
+{
+    asm volatile("" : "+v"(lane));                                // (opaque: nothing of this is held in registers across the regions)
+    const unsigned col = lane & 31u, h = lane >> 5, at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
+    int s[3];
+    digit_scales(expo, h, s);
+    unsigned B[product_count<TB>::N][6];
+    load_operands<TB>(digits, col, h, B);
+    float mx = CLOSED;
+    unsigned xi = 0u;
+    for (unsigned c = a;; c += CHUNK) {
+        const unsigned left = b > c ? b - c : 0u;
+        unsigned letters[3];
+        load12(X, N, c, lane, letters);
+        stage(entries, lane, letters);
+        const unsigned nrow = left < CHUNK ? left : CHUNK, defined = defined_rows(ndef, c);
+        const uint4* src = entries;
+        for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34) {
+            uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
+            if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
+            f32x16_t z;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+            products<TB, 0>(z, a0, a1, B, s);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const unsigned row = 4u * h + ((i & 3) + 8 * (i >> 2));
+                const float v = row < left - t0 ? z[i] : CLOSED;
+                if (WANT_ARGMAX) xi = v > mx ? (c - a) + t0 + row : xi;
+                mx = fmaxf(mx, v);
+            }
+        }
+        if (left <= CHUNK) break;
+    }
+    return make_float2(mx, __uint_as_float(xi));
+}
+
+// the two largest of a tile's 16 rows and of those so far; the tile of the largest
+__device__ __forceinline__ void top_two(const f32x16_t& z, float& m1, float& m2, unsigned& t1, unsigned t)
+{
+    auto max3 = [](float x, float y, float w) { return fmaxf(fmaxf(x, y), w); };
+    auto med3 = [](float x, float y, float w) { return __builtin_amdgcn_fmed3f(x, y, w); };
+    float g[5], k[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        g[i] = max3(z[3 * i], z[3 * i + 1], z[3 * i + 2]);
+        k[i] = med3(z[3 * i], z[3 * i + 1], z[3 * i + 2]);
+    }
+    const float u0 = max3(g[0], g[1], g[2]), v0 = med3(g[0], g[1], g[2]);
+    const float u1 = max3(g[3], g[4], z[15]), v1 = med3(g[3], g[4], z[15]);
+    const float top = max3(u0, u1, m1), v2 = med3(u0, u1, m1);
+    m2 = max3(max3(max3(max3(m2, k[0], k[1]), k[2], k[3]), k[4], v0), v1, v2);
+    t1 = top > m1 ? t : t1;
+    m1 = top;
+}
+
+// Lanes 0-31 of x beside lanes 0-31 of y, and lanes 32-63 of x beside lanes 32-63 of y: (x, y) becomes what the low and the
+// high half wave held of the first value (in lanes 0-31) and of the second (in lanes 32-63).
+__device__ __forceinline__ void swap_halves(unsigned& x, unsigned& y)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0];
+    y = r[1];
+}
+__device__ __forceinline__ void swap_halves(float& x, float& y)
+{
+    unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+    swap_halves(a, b);
+    x = __uint_as_float(a);
+    y = __uint_as_float(b);
+}
+
+template <bool WANT_ARGMAX, int TB>
+__global__ __launch_bounds__(MAX_WAVES * 64) __attribute__((amdgpu_waves_per_eu(MAX_WAVES / 4, MAX_WAVES / 4)))
+void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __restrict__ W, const float* __restrict__ bias, unsigned f0, unsigned m, unsigned F,
+                                const uint8_t* __restrict__ X, size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P, unsigned nsplit,
+                                float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int NI = place_count<TB>::N;
+    constexpr unsigned TAPS = 8u * TB, TILE_DIGITS = TB * NDIGIT * SLOT_BYTES;
+    const unsigned tile = 2u * (blockIdx.x / nsplit), split = blockIdx.x % nsplit;
+    const bool two = tile + 1u < ntile;                           // (an odd last tile is scanned beside nothing)
+    // (a tile that is the general kernel's is scanned along with its neighbour; the general kernel writes over it)
+    if (D.flags[tile] != 0u && (!two || D.flags[tile + 1] != 0u)) return;
+    const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned col = lane & 31u, h = lane >> 5;
+    unsigned* counter = reinterpret_cast<unsigned*>(smem);
+    uint4* entries = reinterpret_cast<uint4*>(smem + 16) + (size_t)wave * ENTRIES;
+    int* table = reinterpret_cast<int*>(smem + 16 + MAX_WAVES * ENTRIES * 16);      // [8 TB taps][8 codes][64 filters]: the weights as whole numbers
+    unsigned char* digits = reinterpret_cast<unsigned char*>(table + TAPS * 8 * PAIR);
+    float4* about = reinterpret_cast<float4*>(digits + 2 * TILE_DIGITS);            // [64 filters]: bias, unit, above, exponents
+    const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
+    if (threadIdx.x == 0) counter[0] = lo;
+    const unsigned fbase = f0 + tile * FTILE;
+    for (unsigned i = threadIdx.x; i < (two ? 2u : 1u) * TILE_DIGITS / 16; i += MAX_WAVES * 64)
+        reinterpret_cast<uint4*>(digits)[i] = reinterpret_cast<const uint4*>(D.digits + (size_t)tile * TILE_DIGITS)[i];
+    for (unsigned i = threadIdx.x; i < TAPS * PAIR; i += MAX_WAVES * 64) {
+        const unsigned tap = i / PAIR, fl = i % PAIR, f = fbase + fl;
+        const bool in = tap < m && f < F && (two || fl < FTILE);
+        const digit_facts k = D.facts[tile * FTILE + (in ? fl : 0u)];
+        const float scale = __uint_as_float((unsigned)(127 + k.whole) << 23);
+        int w[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w[c] = in ? (int)rintf(fmaxf(W[(size_t)(4 * tap + c) * F + f], k.lowest) * scale) : 0;
+        const int mean = (int)(((long long)w[0] + w[1] + w[2] + w[3] + 2) >> 2);
+        int* row = table + (size_t)tap * 8 * PAIR + fl;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) row[c * PAIR] = c < 4 ? w[c & 3] : (c == 6 ? 0 : mean);      // codes mod 8: 254 is 6
+    }
+    if (threadIdx.x < PAIR) {
+        const unsigned f = fbase + threadIdx.x;
+        const bool in = f < F && (two || threadIdx.x < FTILE);
+        const digit_facts k = D.facts[tile * FTILE + (in ? threadIdx.x : 0u)];
+        // (filters past the last: closed whatever their sums)
+        about[threadIdx.x] = make_float4(in ? bias[f] : CLOSED, k.unit, k.above,
+                                         __uint_as_float((unsigned)(k.whole + 1024) << 16 | (unsigned)(D.expo[tile * FTILE + (in ? threadIdx.x : 0u)] + 1024)));
+    }
+    __syncthreads();
+    unsigned B[2][NI][6];
+    auto load_places = [&](unsigned ln) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                unsigned block, digit;
+                place_slot<TB>(i, ln >> 5, block, digit);
+                const bool none = digit == (unsigned)NTOP || (q == 1 && !two);
+                const uint2* src = reinterpret_cast<const uint2*>(D.top + (none ? (size_t)0 : (size_t)(tile + q) * (TB * NTOP * SLOT_BYTES) +
+                                                                            ((block * NTOP + digit) * FTILE + (ln & 31u)) * 24u));
+#pragma unroll
+                for (int k = 0; k < 3; ++k) { const uint2 v = src[k]; B[q][i][2 * k] = none ? 0u : v.x; B[q][i][2 * k + 1] = none ? 0u : v.y; }
+            }
+    };
+    load_places(lane);
+    // a unit is digit 2's step: digit p counts 2^(5 (2 - p)), stored in eighths
+    const int single = 140 | 135 << 8 | 130 << 16, pair = 140 | (135 - 5 * (int)h) << 8;
+    f32x16_t rows;                                                // what the rows start from, in 1/64 of a unit
+#pragma unroll
+    for (int i = 0; i < 16; ++i) rows[i] = (float)(15 - i) * (1.0f / 64.0f);
+    const unsigned at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
+
+    unsigned r = claim(counter, lane), rn = claim(counter, lane); // the region in work, the one after it
+    unsigned a = 0u, b = 0u, an = 0u, bn = 0u;
+    if (r < hi) { a = R[2 * (size_t)r]; b = R[2 * (size_t)r + 1]; }
+    if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
+    a = (unsigned)__builtin_amdgcn_readfirstlane((int)a); b = (unsigned)__builtin_amdgcn_readfirstlane((int)b);
+    unsigned letters[3] = {0u, 0u, 0u};
+    if (r < hi) load12(X, N, a, lane, letters);
+
+    while (r < hi) {
+        float m1[2] = {CLOSED, CLOSED}, m2[2] = {CLOSED, CLOSED}; // the two largest sums so far
+        unsigned t1[2] = {0u, 0u}, t = 0u;                        // the tile of the largest, the tile in work
+        unsigned c = a;
+        bool last;
+        do {
+            const unsigned left = b > c ? b - c : 0u;             // rows of the region from this stretch on
+            last = left <= CHUNK;
+            stage(entries, lane, letters);
+            // the next stretch's letters travel while this one is multiplied
+            if (!last) load12(X, N, c + CHUNK, lane, letters);
+            else if (rn < hi) load12(X, N, (unsigned)__builtin_amdgcn_readfirstlane((int)an), lane, letters);
+            const unsigned nrow = last ? left : CHUNK;
+            const unsigned defined = defined_rows(ndef, c);
+            const uint4* src = entries;
+            for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34, ++t) {
+                uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
+                if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
+                const unsigned rest = left - t0;                  // (rows of the region from this tile on)
+                const int inside = (int)(rest < 64u ? rest : 64u) - 4 * (int)h;
+                auto half = [&](int q) {
+                    f32x16_t z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
+                    if (rest < (unsigned)ROWS) {
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) z[i] = (i & 3) + 8 * (i >> 2) < inside ? z[i] : CLOSED;
+                    }
+                    top_two(z, m1[q], m2[q], t1[q], t);
+                };
+                half(0);
+                half(1);
+            }
+            c += CHUNK;
+        } while (!last);
+        // ---- each filter's two half waves side by side: the largest sum, its place, the second largest
+        unsigned mine = lane;                                     // (opaque: addresses are formed from it here, not held in registers)
+        asm volatile("" : "+v"(mine));
+        swap_halves(m1[0], m1[1]);
+        swap_halves(m2[0], m2[1]);
+        swap_halves(t1[0], t1[1]);
+        const bool upper = m1[1] > m1[0];
+        const float best = fmaxf(m1[0], m1[1]), second = fmaxf(fminf(m1[0], m1[1]), fmaxf(m2[0], m2[1]));
+        const unsigned i = 15u - ((unsigned)(int)(best * 64.0f) & 15u);
+        unsigned row = (upper ? t1[1] : t1[0]) * ROWS + (upper ? 4u : 0u) + (i & 3u) + 8u * (i >> 2);
+        const float4 filter = about[mine];
+        const bool open = (best + filter.z) * filter.y + filter.x > 0.0f;      // else every window's rectified value is zero
+        // ---- its value from the weights
+        float value = 0.0f;
+        const size_t at = (size_t)a + row;
+        if (open && at < ndef) {
+            unsigned v[2 * TB];
+            if (at + TAPS <= N) __builtin_memcpy(v, X + at, TAPS);
+            else load_tail<TAPS>(X, N, at, v);
+            int sum = 0;
+#pragma unroll
+            for (int k = 0; k < 2 * TB; ++k) {
+                if (odd_codes(v[k]) != 0u) v[k] = plain_codes(v[k]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sum += (table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
+            }
+            value = (float)sum * __uint_as_float((unsigned)(127 + 1024 - (int)(__float_as_uint(filter.w) >> 16)) << 23);
+        }
+        const bool unsure = open && !((second + filter.z) * filter.y < value);
+        const unsigned long long who = __ballot(unsure);
+        if (who != 0ull) {
+            // ---- too close to call: all the digits, for the 32 filters concerned
+#pragma unroll 1
+            for (unsigned q = 0; q < 2; ++q) {
+                if ((unsigned)(who >> (32u * q)) == 0u) continue;
+                const float2 all = region_maximum<WANT_ARGMAX, TB>(X, N, ndef, a, b, entries, digits + q * TILE_DIGITS, mine,
+                                                                   (int)(__float_as_uint(about[32u * q + (mine & 31u)].w) & 0xffffu) - 1024);
+                const float oz = __shfl_xor(all.x, 32, 64);
+                const unsigned xi = __float_as_uint(all.y), oi = (unsigned)__shfl_xor((int)xi, 32, 64);
+                if (unsure && (mine >> 5) == q) {
+                    value = fmaxf(all.x, oz);
+                    row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
+                }
+            }
+            load_places(mine);                                    // (not held over the pass: its operands take their registers)
+        }
+        value = open ? fmaxf(value + filter.x, 0.0f) : 0.0f;
+        const unsigned f = fbase + mine;
+        if (f < F && (two || mine < FTILE)) {
+            const size_t j = (size_t)r * F + f;
+            pooled[j] = value;
+            if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + (value > 0.0f ? row : 0u)) * F + f);   // nothing open: the first row
+        }
+        r = rn;
+        a = (unsigned)__builtin_amdgcn_readfirstlane((int)an); b = (unsigned)__builtin_amdgcn_readfirstlane((int)bn);
+        rn = claim(counter, lane);
+        if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
+    }
+}
+
+// workgroups per group of filters: one workgroup per CU in all, no more waves than regions
+inline unsigned splits(unsigned groups, unsigned waves, size_t P)
+{
+    unsigned n = 256u / groups;
+    if (n < 1) n = 1;
+    while (n > 1 && (size_t)(n - 1) * waves >= P) --n;
+    return n;
+}
+
+constexpr size_t max_smem(int tb)
+{
+    return 16 + (size_t)MAX_WAVES * ENTRIES * 16 + (size_t)tb * (8 * 8 * PAIR * sizeof(float) + 2 * NDIGIT * SLOT_BYTES) + PAIR * 16;
+}
+static_assert(max_smem(4) <= 160 * 1024, "LDS of a CU");
+
+template <bool WANT_ARGMAX, int TB>
+int launch_max(hipStream_t st, const digit_store& D, const float* W, const float* bias, unsigned f0, unsigned ntile, size_t m, size_t F, const uint8_t* X,
+               size_t N, size_t ndef, const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
+{
+    auto kern = scanpool_digits_max_kernel<WANT_ARGMAX, TB>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_smem(TB)));
+    const unsigned groups = (ntile + 1) / 2, nsplit = splits(groups, MAX_WAVES, P);
+    hipLaunchKernelGGL(kern, dim3(groups * nsplit), dim3(MAX_WAVES * 64), max_smem(TB), st, D, ntile, W, bias, f0, (unsigned)m, (unsigned)F, X, N, ndef, R,
+                       (unsigned)P, nsplit, pooled, argmax);
+    return 0;
 }
 
 constexpr size_t SMEM = 16 + (size_t)NWAVE * ENTRIES * 16;
@@ -399,26 +827,40 @@ int launch_pt(hipStream_t st, const digit_store& D, const float* bias, unsigned 
 {
     auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB>;
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
-    unsigned nsplit = 256u / ntile;
-    if (nsplit < 1) nsplit = 1;
-    while (nsplit > 1 && (size_t)(nsplit - 1) * NWAVE >= P) --nsplit;           // no more waves than regions
+    const unsigned nsplit = splits(ntile, NWAVE, P);
     hipLaunchKernelGGL(kern, dim3(ntile * nsplit), dim3(NWAVE * 64), SMEM, st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
     return 0;
 }
 
-// the filters f0 .. f0 + 32 * ntile - 1: their digits, then the scan
+// the filters f0 .. f0 + 32 * ntile - 1: their digits, then the scan (half: plain maxima with half the products)
 template <int TB>
 int launch(hipStream_t st, const digit_store& D, const float* W, const float* bias, unsigned f0, unsigned ntile, unsigned nflag, size_t m, size_t F,
-           const uint8_t* X, size_t N, const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax)
+           const uint8_t* X, size_t N, const uint32_t* R, size_t P, int ptype, bool half, float* pooled, uint32_t* argmax)
 {
     const size_t ndef = N >= m ? N - m + 1 : 0;                    // rows the scan defines
     hipLaunchKernelGGL(weight_digits_kernel<TB>, dim3(nflag), dim3(256), 0, st, W, bias, (unsigned)m, (unsigned)F, f0, D);
+    if constexpr (TB >= 3) {
+        if (half)
+            return argmax ? launch_max<true, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax)
+                          : launch_max<false, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax);
+    }
     if (ptype == DBK_PT_AVG) return launch_pt<DBK_PT_AVG, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
     if (ptype == DBK_PT_MAX)
         return argmax ? launch_pt<DBK_PT_MAX, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
                       : launch_pt<DBK_PT_MAX, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
     return argmax ? launch_pt<DBK_PT_ALL, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
                   : launch_pt<DBK_PT_ALL, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+}
+
+// Whether plain maxima go through half the products: filters of more than 16 taps, more than 32 of them (a wave takes 64),
+// regions of 80 rows on average and eight of them per wave. Measured, all the products / half of them, 24 taps: 100 000 x
+// 500 letters x 1024 filters 10.4 / 8.1 ms, 65 536 x 101 x 256 0.515 / 0.461, 8192 x 101 x 256 0.080 / 0.078, 100 000 x 40 x
+// 64 0.134 / 0.137, 2000 x 500 x 64 0.034 / 0.049; 16 taps, 65 536 x 101 x 256 0.361 / 0.368. A caller who asks for this
+// path by name gets them whatever the number of regions: a region's result then does not depend on what is beside it.
+bool half_the_products(size_t m, size_t F, size_t N, size_t P, int ptype, bool force)
+{
+    if (ptype != DBK_PT_MAX || m <= 16 || F <= FTILE || N < 80 * P) return false;
+    return force || P * dbk::divup(F, PAIR) >= (size_t)256 * MAX_WAVES * 8;
 }
 
 // Whether a call of this size goes to the digit kernel when the choice is left to the library, in rows x 64-filter tiles
@@ -437,7 +879,7 @@ bool takes(size_t m, size_t F, size_t N, size_t P, bool argmax)
 
 // A call's scratch: one flag per 32 filters (an even number of them: the general kernel looks at pairs), then the digits of
 // up to PASS_TILES tiles; more filters than that are taken in several passes.
-constexpr unsigned PASS_TILES = 2048;
+constexpr unsigned PASS_TILES = 1024;
 inline size_t flag_bytes(size_t F) { return (2 * (size_t)dbk::divup(F, 2 * FTILE) * sizeof(unsigned) + 255) & ~(size_t)255; }
 inline size_t scratch_bytes(size_t m, size_t F)
 {
@@ -463,15 +905,16 @@ int fprop_impl(hipStream_t st, const float* W, const float* bias, size_t m, size
         if (!ws) { dbk::set_error("MemoryError: could not allocate %zu bytes of scratch (%s)", scratch_bytes(m, F), dbk::workspace_error()); return 1; }
     }
     unsigned* flags = reinterpret_cast<unsigned*>(ws);
+    const bool half = half_the_products(m, F, N, P, ptype, force);
     for (unsigned t0 = 0; t0 < ntile; t0 += PASS_TILES) {
         const unsigned nt = ntile - t0 < PASS_TILES ? ntile - t0 : PASS_TILES, nf = nflag - t0 < PASS_TILES ? nflag - t0 : PASS_TILES;
-        const digit_store D = store_at(flags + t0, ws + flag_bytes(F), nf);
+        const digit_store D = store_at(flags + t0, ws + flag_bytes(F), nf, tb);
         int rc;
         switch (tb) {
-        case 1: rc = launch<1>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
-        case 2: rc = launch<2>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
-        case 3: rc = launch<3>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
-        default: rc = launch<4>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, pooled, argmax); break;
+        case 1: rc = launch<1>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, half, pooled, argmax); break;
+        case 2: rc = launch<2>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, half, pooled, argmax); break;
+        case 3: rc = launch<3>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, half, pooled, argmax); break;
+        default: rc = launch<4>(st, D, W, bias, t0 * FTILE, nt, nf, m, F, X, N, R, P, ptype, half, pooled, argmax); break;
         }
         if (rc != 0) return rc;
     }
@@ -490,10 +933,10 @@ int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F,
 // Every device the library runs on holds its own copy of this array, at its own address, from the moment the code
 // object is loaded there until the process ends. The array's name is a host-side handle, not a device address:
 // host code asks the runtime for the address once per device and passes that pointer to the kernels.
-// (24 taps: 2048 tiles' digits and exponents, 28.6 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
-constexpr size_t STATIC_SCRATCH_BYTES = size_t(29) << 20;
+// (24 taps: 1024 tiles' digits, 21.9 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
+constexpr size_t STATIC_SCRATCH_BYTES = size_t(22) << 20;
 constexpr size_t STATIC_SEQUENCE_BYTES = (size_t(64) << 20) - 127; // sequence bytes a call may bring
-static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * sizeof(int) + 3 * NDIGIT * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
+static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * (sizeof(int) + sizeof(digit_facts)) + 3 * (NDIGIT + NTOP) * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
 static __device__ __align__(256) unsigned char scratch[STATIC_SCRATCH_BYTES];
 static unsigned char* g_static_scratch[64] = {nullptr};
 static std::mutex g_static_scratch_mutex;

@@ -1176,6 +1176,57 @@ def test_bulk_scan_at_the_edges_of_its_tiles(ks, ptype, m, F):
     assert np.array_equal(np.isnan(host(P)), np.isnan(host(Pg))) and np.allclose(host(P), host(Pg), rtol=0, atol=1e-5, equal_nan=True)
 
 
+@pytest.mark.parametrize("m,F", [(17, 33), (20, 64), (24, 96), (24, 130)])
+def test_bulk_maxima_that_are_close_are_settled_by_all_the_digits(ks, m, F):
+    """Long filters' maxima are placed by half of the products; where two windows' sums are closer than those tell, the region
+    is scanned again. Windows that recur letter by letter, weights whose sums tie between different windows, filters that
+    stay closed, windows of nothing but padding: the value, and the first of the rows that attain it."""
+    rng = np.random.default_rng(m + F)
+    unit = rng.integers(0, 4, 37, dtype=np.uint8)
+    seqs = [np.tile(unit, 8), rng.integers(0, 4, 300).astype(np.uint8), np.full(150, 2, np.uint8), np.tile(unit[::-1], 3),
+            np.full(100, 255, np.uint8), rng.integers(0, 4, 501).astype(np.uint8), np.tile(rng.integers(0, 4, 2).astype(np.uint8), 120)]
+    from deepbind_amd import data
+    X, R = data.pack_ordinals(seqs, m - 1)
+    X[X.size // 2] = 254
+    W = (rng.integers(-8, 9, (4 * m, F)) / 8.0).astype(np.float32)        # every sum is exact: ties are ties
+    W[:, 3] = rng.standard_normal(4 * m) * 0.1
+    W[:, 4] = W[0, 4]
+    W[:, 5] = 0.0
+    b = (rng.integers(-4, 5, (1, F)) / 8.0).astype(np.float32)
+    b[0, 6] = -50.0
+    A, Pr, _ = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, "max")
+    P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", want_argmax=True, path="kmer")
+    P, I = host(P), host(I)
+    assert np.array_equal(host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", path="kmer")[0]), P)
+    exact = np.arange(F) != 3
+    assert np.array_equal(P[:, exact], Pr[:, exact].astype(np.float32)) and np.abs(P - Pr).max() <= 1e-5
+    first = np.stack([A[a:e].argmax(axis=0) + a for a, e in R.astype(int)])
+    assert np.array_equal((I // F)[:, exact], first[:, exact]) and np.array_equal(I % F, np.broadcast_to(np.arange(F), I.shape))
+    a3 = A[I[:, 3] // F, 3]
+    assert np.abs(a3 - Pr[:, 3]).max() <= 1e-5
+
+
+@pytest.mark.parametrize("m", [17, 25, 32])
+def test_bulk_maxima_of_long_filters_by_the_library_s_choice(ks, m):
+    """Enough regions and filters that the library itself takes half of the products, an odd number of filter tiles."""
+    F = 32 * 513
+    rng, W, b, X, R = _bulk_case(70 + m, list(rng_rows(m, 110, 60, 190)), m, F, odd_codes=False)
+    P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", want_argmax=m <= 24)
+    P = host(P)
+    pick = np.sort(np.concatenate([rng.choice(F, 90, replace=False), [F - 1, F - 33]]))
+    A, Pr, Ir = _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R, "max")
+    _within_rounding(P[:, pick], Pr, W[:, pick], b[:, pick], "max")
+    if I is not None:
+        rows = host(I)[:, pick] // F
+        moved = rows != Ir // len(pick)
+        cols = np.broadcast_to(np.arange(len(pick)), rows.shape)
+        assert moved.mean() < 0.001 and np.abs(A[rows[moved], cols[moved]] - Pr[moved]).max(initial=0.0) <= 1e-5
+
+
+def rng_rows(seed, n, lo, hi):
+    return np.random.default_rng(seed).integers(lo, hi, n)
+
+
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("m", [25, 29, 32])
 def test_bulk_scan_of_25_to_32_taps(ks, ptype, m):
@@ -1214,7 +1265,7 @@ def test_bulk_scan_leaves_weights_it_cannot_express_to_the_general_kernel(ks, pt
     P, Pg = host(P), host(Pg)
     assert np.array_equal(P[:, :64 * k], Pg[:, :64 * k], equal_nan=True)
     scale = np.maximum(np.abs(Pg).max(axis=0), 1e-30)
-    assert np.all(np.abs(P - Pg)[:, 64 * k:] <= 1e-5 * scale[64 * k:]) and np.all(P[:, 71 * k:72 * k][:, :1] >= 0)
+    assert np.all(np.abs(P[:, 64 * k:] - Pg[:, 64 * k:]) <= 1e-5 * scale[64 * k:]) and np.all(P[:, 71 * k:72 * k][:, :1] >= 0)
     if want:
         assert (host(I) == host(Ig)).mean() > 0.99
 
