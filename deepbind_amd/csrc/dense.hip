@@ -677,6 +677,112 @@ __global__ __launch_bounds__(256) void k_head_lanes(size_t n, int nblock, int k,
     }
 }
 
+// The sum of the four rows of 16 lanes, in every lane.
+__device__ __forceinline__ float sum_rows16(float v)
+{
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// Scoring head on the float32 matrix instruction (v_mfma_f32_16x16x4_f32: products and sums as fused multiply-adds in
+// float32), for bulk calls with a hidden layer. A wave owns one model, whose W1 (16 KI inputs x 16 HU units, transposed) is
+// the first operand and stays in registers, and takes 16 rows at a time as the second: lane (row, q) loads inputs 4 q .. 4 q + 3
+// of every 16 as 16 bytes, step j of four multiplies element j of those (the contraction's order is the same for both
+// operands, so no value has to move). The result has a row's hidden units in four lanes, four per lane and tile: bias,
+// rectifier and W2 are three instructions each, the output sum two lane swaps. 4 waves: adjacent models of the same rows.
+// Bound by the matrix pipe (512 clocks per 16 rows of 32 inputs and 32 units) beside the one pass over the features.
+// Measured, us a call, the kernels below and above / this one: 30 000 rows x 24 models, 32 -> 32 -> 1 55 / 30, 16 -> 32 35 / 18;
+// 100 000 x 24, 32 -> 32 185 / 93; 100 000 x 64, 24 -> 32 498 / 229; 8000 x 64, 32 -> 32 44 / 23; 100 000 x 1, 32 -> 64 32 / 11.
+template <int KI, int HU>
+__global__ __launch_bounds__(256) void k_head_mm(size_t n, int nblock, int k, int kf, int kw, int hidden, int mg, unsigned cols, const float* __restrict__ pooled,
+                                                 const float* __restrict__ feats, const float* __restrict__ in_scale, const float* __restrict__ W1,
+                                                 const float* __restrict__ b1, const float* __restrict__ W2, const float* __restrict__ b2,
+                                                 bool apply_logistic, float* __restrict__ scores)
+{
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    constexpr int NR = 4;                               // 16-row blocks in flight
+    const int kt = k + kf;                              // the model's own inputs, then the shared feature columns (see k_head)
+    const unsigned lane = threadIdx.x & 63u, col = lane & 15u, q = lane >> 4, wave = threadIdx.x >> 6;
+    // workgroups go round the eight XCDs: those that share rows (models side by side) are made to share an L2 as well
+    const unsigned xcd = blockIdx.x & 7u, turn = blockIdx.x >> 3, slices = gridDim.x / cols, slice = (turn / cols) * 8u + xcd;
+    const unsigned b = (turn % cols) * (unsigned)mg + (wave & (unsigned)(mg - 1)), per = 4u / (unsigned)mg;
+    if (b >= (unsigned)nblock) return;                  // (no barrier below)
+    float a[KI][4][HU];
+    f32x4_t bias1[HU], w2[HU];
+#pragma unroll
+    for (int u = 0; u < HU; ++u) {
+        const int h = 16 * u + (int)col;
+#pragma unroll
+        for (int i = 0; i < KI; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int kk = 16 * i + 4 * (int)q + j;
+                a[i][j][u] = h < hidden && kk < kt ? W1[((size_t)b * kw + kk) * hidden + h] : 0.0f;
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int hr = 16 * u + 4 * (int)q + i;
+            bias1[u][i] = hr < hidden ? b1[(size_t)b * hidden + hr] : 0.0f;
+            w2[u][i] = hr < hidden ? W2[(size_t)b * hidden + hr] : 0.0f;
+        }
+    }
+    const float sc = in_scale ? in_scale[b] : 1.0f, last = b2[b];
+    const size_t rowlen = (size_t)k * nblock;
+    const bool packs = kf == 0 && (k & 3) == 0 && (reinterpret_cast<uintptr_t>(pooled) & 15u) == 0;
+    const size_t step = (size_t)slices * per * (16 * NR);
+    for (size_t base = ((size_t)slice * per + wave / (unsigned)mg) * (16 * NR); base < n; base += step) {
+        float x[NR][KI][4];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const size_t row = base + 16 * r + col, at = (row < n ? row : n - 1) * rowlen + (size_t)b * k;
+#pragma unroll
+            for (int i = 0; i < KI; ++i) {
+                const int k0 = 16 * i + 4 * (int)q;
+                if (packs) {
+                    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (k0 < k) v = *reinterpret_cast<const float4*>(pooled + at + k0);
+                    x[r][i][0] = v.x * sc; x[r][i][1] = v.y * sc; x[r][i][2] = v.z * sc; x[r][i][3] = v.w * sc;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int kk = k0 + j;
+                        x[r][i][j] = kk < k ? pooled[at + kk] * sc : (kk < kt ? feats[(row < n ? row : n - 1) * (size_t)kf + (kk - k)] : 0.0f);
+                    }
+                }
+            }
+        }
+        float mine = 0.0f;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            f32x4_t z[HU];
+#pragma unroll
+            for (int u = 0; u < HU; ++u) z[u] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < KI; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int u = 0; u < HU; ++u) z[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][j][u], x[r][i][j], z[u], 0, 0, 0);
+            float out = 0.0f;
+#pragma unroll
+            for (int u = 0; u < HU; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = z[u][i] + bias1[u][i];
+                    out += (v > 0.0f ? v : 0.0f) * w2[u][i];
+                }
+            out = sum_rows16(out);
+            mine = q == (unsigned)r ? out : mine;
+        }
+        mine += last;
+        if (apply_logistic) mine = 1.0f / (1.0f + expf(-mine));
+        const size_t row = base + lane;                 // lane (col, q) keeps row 16 q + col
+        if (row < n) scores[row * (size_t)nblock + b] = mine;
+    }
+}
+
 // Where k_head16, whose weights in LDS feed four rows (two beyond 16 inputs, one beyond 32) of 16 models each, is the better of the two: it
 // spends about a microsecond per 32 multiply-adds of an item before the first row is out, and then fewer instructions an item than
 // k_head_lanes' padded 16 x 16 blocks - by most where a block is mostly padding (few hidden units), by none where its inputs are no whole
@@ -700,6 +806,25 @@ inline bool head16_pays(size_t n, int nblock, int inputs, int hidden)
     if (hidden <= 4) return items >= 500 * macs;
     if (inputs <= 16 && items >= 4000000) return true;
     return macs <= (inputs == 32 ? 512u : 640u) && items >= 160000 && items >= 1200 * macs;
+}
+
+// Where the matrix instruction is the better one: from some thousand rows x models on, except where k_head16 (`grouped`) runs and most of
+// the 16 x 16 blocks would be padding, or where a bulk call is so large that its rows no longer come from the last-level cache and
+// k_head16's 1 KB row segments do better than 256 bytes. us a call, k_head16 / k_head_mm: 100 000 x 24, 32 -> 4 74 / 91, 32 -> 8 83 / 91,
+// 32 -> 16 99 / 92; 100 000 x 64, 16 -> 16 105 / 157, 16 -> 32 144 / 147, 8 -> 16 102 / 88; 30 000 x 64, 16 -> 16 39 / 31; 100 000 x 40,
+// 4 -> 32 59 / 65; 30 000 x 24, 4 -> 32 20 / 16.
+inline bool head_mm_pays(size_t n, int nblock, int inputs, int hidden, bool grouped)
+{
+    const size_t items = n * (size_t)nblock;
+    if (hidden == 0 || items < 8192) return false;
+    if (!grouped) return true;
+    if (inputs <= 4) return items < (hidden <= 8 ? 1000000u : 3000000u);
+    if (inputs < 16) return hidden > 28 || items < (hidden > 16 ? 3000000u : 6000000u);
+    if (inputs > 16 && inputs < 32) return true;
+    if (hidden <= 4) return items < 500000;
+    if (hidden <= 8) return items < (inputs == 16 ? 700000u : 1600000u);
+    if (hidden <= 16) return items < 2500000;
+    return inputs > 16 || hidden > 28 || items < 3000000;
 }
 
 // Where k_head, a thread per row and model, is the better one still: so few inputs that most of k_head_lanes' 16 are padding, and enough rows x
@@ -1053,7 +1178,23 @@ int dbk_head_fprop(dbk_stream_t stream, size_t n, int nblock, int k, int hidden,
     // (Whether the feature columns are given or left out as zeros must not change the bits: what does not depend on it decides. k_head, which
     // takes over from k_head16 where given columns do not fit in LDS, adds in k_head16's order; kw counts them in either case.)
     const bool grouped = head16_pays(n, nblock, k, hidden);
-    if (!grouped && !head_rows_pay(n, nblock, kw, hidden) && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
+    const bool by_rows = !grouped && head_rows_pay(n, nblock, kw, hidden);
+    if (!by_rows && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32) && head_mm_pays(n, nblock, k, hidden, grouped)) {
+        const int mg = nblock >= 4 ? 4 : (nblock >= 2 ? 2 : 1);
+        const unsigned cols = dbk::divup(nblock, mg);
+        unsigned gy = (dbk::divup(n, 64 * (4 / mg)) + 7u) & ~7u;   // slices of rows: a multiple of the XCDs
+        if (gy > 2048u / cols) gy = (2048u / cols) & ~7u;
+        if (gy < 8) gy = 8;
+#define DBK_HEAD_MM(KI, HU)                                                                                                        \
+        if (kk_all <= KI * 16 && hidden <= HU * 16) {                                                                                       \
+            hipLaunchKernelGGL((k_head_mm<KI, HU>), dim3(cols * gy), dim3(256), 0, dbk::as_stream(stream), n, nblock, k, kf, kw, hidden, mg, cols, pooled, feats, in_scale, \
+                               W1, b1, W2, b2, apply_logistic != 0, scores);                                                           \
+            DBK_LAUNCH_OK();                                                                                                           \
+        }
+        DBK_HEAD_MM(1, 1) DBK_HEAD_MM(1, 2) DBK_HEAD_MM(2, 1) DBK_HEAD_MM(2, 2) DBK_HEAD_MM(1, 4) DBK_HEAD_MM(4, 1) DBK_HEAD_MM(2, 4) DBK_HEAD_MM(4, 2)
+#undef DBK_HEAD_MM
+    }
+    if (!grouped && !by_rows && kw <= 64 && hidden <= 64 && (kw <= 32 || hidden <= 32)) {
         const int mg = nblock >= 4 ? 4 : (nblock >= 2 ? 2 : 1);
         const unsigned cols = dbk::divup(nblock, mg);
         unsigned gy = dbk::divup(n, 4 * (4 / mg));                 // a row step per wave ...

@@ -868,6 +868,35 @@ def test_head_fprop_either_side_of_the_bulk_rule(ds, n, k, h, nb, nfeat):
         assert np.array_equal(none, zeros)
 
 
+@pytest.mark.parametrize("n,k,h,nb,nfeat", [(8193, 16, 32, 1, 0), (4097, 32, 17, 2, 0), (2731, 7, 33, 3, 0), (1700, 30, 5, 5, 3), (2063, 33, 32, 4, 0),
+                                            (8200, 64, 9, 1, 0), (12289, 12, 64, 7, 4), (64 * 130 + 1, 16, 16, 1, 0)])
+def test_head_fprop_on_the_matrix_instruction(ds, n, k, h, nb, nfeat):
+    """Calls that go through the float32 matrix instruction: inputs that are no whole packs of four (or lie off a 16-byte
+    boundary), inputs and units that fill no group of 16, rows past a multiple of 64, one to seven models, feature columns, an
+    infinite input. float32 sums of k + nfeat and h terms: each rounding is 2^-24 of the terms' sizes."""
+    rng = np.random.default_rng(n + k + h)
+    Pl = np.abs(rng.standard_normal((n, k * nb))).astype(np.float32)
+    W1 = (rng.standard_normal(((k + nfeat) * nb, h)) * 0.2).astype(np.float32); b1 = (rng.standard_normal((1, h * nb)) * 0.1).astype(np.float32)
+    W2 = (rng.standard_normal((h * nb, 1)) * 0.2).astype(np.float32); b2 = (rng.standard_normal((1, nb)) * 0.1).astype(np.float32)
+    F = rng.standard_normal((n, nfeat)).astype(np.float32) if nfeat else None
+    rate = rng.choice([0.0, 0.25, 0.5], size=nb).astype(np.float32)
+    X = Pl.astype(np.float64).reshape(n, nb, k) * (1 - rate.astype(np.float64))[:, None]
+    if nfeat:
+        X = np.concatenate([X, np.broadcast_to(F.astype(np.float64)[:, None], (n, nb, nfeat))], axis=2)
+    w1, w2 = W1.astype(np.float64).reshape(nb, k + nfeat, h), W2.astype(np.float64).reshape(nb, h)
+    A = np.einsum("nbk,bkh->nbh", X, w1) + b1.reshape(nb, h)
+    size = (np.einsum("nbk,bkh->nbh", np.abs(X), np.abs(w1)) + np.abs(b1.reshape(nb, h))) @ np.eye(h)
+    ref, bound = (np.maximum(A, 0) * w2).sum(axis=2) + b2, (k + nfeat + h + 6) * 2.0 ** -24 * ((size * np.abs(w2)).sum(axis=2) + np.abs(b2))
+    store = torch.zeros(n * k * nb + 1, device="cuda")
+    store[1:] = dev(Pl).reshape(-1)
+    for P in (dev(Pl), store[1:].view(n, k * nb)):
+        got = ds.head_fprop(P, dev(W1), dev(b1), dev(W2), dev(b2), nblock=nb, in_scale=1 - rate, nfeat=nfeat, feats=None if F is None else dev(F))
+        assert np.all(np.abs(host(got) - ref) <= bound)
+    Pl[n - 1, 0] = np.inf
+    got = host(ds.head_fprop(dev(Pl), dev(W1), dev(b1), dev(W2), dev(b2), nblock=nb, in_scale=1 - rate, nfeat=nfeat, feats=None if F is None else dev(F)))
+    assert not np.isfinite(got[n - 1, 0]) and np.all(np.abs(got[:-1] - ref[:-1]) <= bound[:-1])
+
+
 @pytest.mark.parametrize("k,h,nb", [(16, 32, 37), (32, 8, 16), (16, 64, 5)])
 def test_head_fprop_bulk_rows(ds, k, h, nb):
     """Row counts that take the 16-models-per-workgroup kernel; model count not a multiple of 16; dropout rescale."""
