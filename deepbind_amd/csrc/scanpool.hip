@@ -635,52 +635,17 @@ __global__ void reduce_slabs_kernel(float* __restrict__ dW, float* __restrict__ 
     }
 }
 
-// The mask-driven backward through bit counts. At every row of a region whose rectifier is open the average-pooling
-// gradient is the SAME number c = dpooled / rows, so the filter gradient needs no pass over the rows:
-//     dW[tap][letter][f] += c * popcount(open_f & (is_letter >> tap))
-// with one bit per row: open_f from the forward pass's activity masks (stored one 64-bit lane mask per row; turned
-// into one row mask per lane = filter with a six-stage butterfly of lane exchanges), is_letter from five ballots over the chunk's
-// letters (wave-uniform, shifted in scalar registers). A wave walks whole regions in chunks of 64 rows: per chunk
-// ~7 vector instructions per (tap, letter) whatever the number of rows, against one half-rate index-mode add per
-// (row, tap) in the kernels above: a third of their issue slots at 53 rows, a fifth at 64. The max-pooling gradient
-// lands on one row per (region, filter): that row's letters are cut out of the same letter bits, once per region.
-// A lane keeps the 5 x MT sums of its filter in registers over all its regions (ascending), the waves fold them
-// into the workgroup's slab as above. Deterministic; c * count is rounded once where the kernels above add c count
-// times, so the sums agree with theirs to rounding, not bit for bit.
-// PT: DBK_PT_AVG / ALL read the masks; DBK_PT_MAX needs none.
-// Transposes the 64 x 64 bit matrix whose row i is lane i's (lo, hi): afterwards bit i of lane j is what bit j of
-// lane i was. Six butterfly stages (block sizes 32 ... 1): a lane and its partner lane ^ d swap the off-diagonal
-// d x d blocks they hold between them.
-__device__ __forceinline__ void transpose_masks(unsigned& lo, unsigned& hi, unsigned lane)
-{
-    {   // d = 32: whole words change places
-        const unsigned plo = (unsigned)__shfl_xor((int)lo, 32, 64), phi = (unsigned)__shfl_xor((int)hi, 32, 64);
-        if (lane & 32u) lo = phi; else hi = plo;
-    }
-#pragma unroll
-    for (unsigned d = 16; d >= 1; d >>= 1) {
-        // bits whose index has bit d clear, within a word
-        const unsigned keep = d == 16 ? 0x0000ffffu : d == 8 ? 0x00ff00ffu : d == 4 ? 0x0f0f0f0fu : d == 2 ? 0x33333333u : 0x55555555u;
-        const unsigned plo = (unsigned)__shfl_xor((int)lo, (int)d, 64), phi = (unsigned)__shfl_xor((int)hi, (int)d, 64);
-        if (lane & d) {
-            lo = ((plo >> d) & keep) | (lo & ~keep);
-            hi = ((phi >> d) & keep) | (hi & ~keep);
-        } else {
-            lo = (lo & keep) | ((plo & keep) << d);
-            hi = (hi & keep) | ((phi & keep) << d);
-        }
-    }
-}
-template <int PT, int MT>
+// The max-pooling gradient of short regions. It lands on one row per (region, filter): that row's letters are cut out of the
+// region's letters held as one bit per (letter, position), from five ballots per chunk of 64 rows (wave-uniform, shifted in scalar
+// registers), once per region. A wave walks whole regions; a lane keeps the 5 x MT sums of its filter in registers over all its
+// regions (ascending), the waves fold them into the workgroup's slab as above. Deterministic.
+template <int MT>
 __device__ __forceinline__ void scanpool_bprop_bits_body(const wg_t wg, unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
                                                          const uint32_t* __restrict__ R, size_t P,
                                                          const float* __restrict__ pooled, const uint32_t* __restrict__ argmax,
-                                                         const float* __restrict__ dpooled,
-                                                         const unsigned long long* __restrict__ act,
-                                                         float* __restrict__ slabs, size_t stride)
+                                                         const float* __restrict__ dpooled, float* __restrict__ slabs, size_t stride)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    constexpr bool DENSE = PT != DBK_PT_MAX, PEAK = PT != DBK_PT_AVG;
     const unsigned nw = blockDim.x >> 6;
     const unsigned lane = threadIdx.x & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned f0 = wg.y * FT, f = f0 + lane;
@@ -692,25 +657,22 @@ __device__ __forceinline__ void scanpool_bprop_bits_body(const wg_t wg, unsigned
         for (int t = 0; t < MT; ++t) acc[l][t] = 0.0f;
     float db = 0.0f;
 
-    struct pooled_in { float davg, pmax, dmax; unsigned arg; };
+    struct pooled_in { float pmax, dmax; unsigned arg; };
     auto load_pooled = [&](size_t r_) -> pooled_in {
-        pooled_in q = { 0.0f, 0.0f, 0.0f, 0u };
+        pooled_in q = { 0.0f, 0.0f, 0u };
         if (f < F && r_ < P) {
             const size_t j0 = r_ * F + f;
-            if (PT == DBK_PT_AVG) q.davg = dpooled[j0];
-            else if (PT == DBK_PT_ALL) { q.davg = dpooled[2 * j0 + 1]; q.pmax = pooled[2 * j0]; q.dmax = dpooled[2 * j0]; q.arg = argmax[j0]; }
-            else { q.pmax = pooled[j0]; q.dmax = dpooled[j0]; q.arg = argmax[j0]; }
+            q.pmax = pooled[j0]; q.dmax = dpooled[j0]; q.arg = argmax[j0];
         }
         return q;
     };
     auto bound = [&](size_t r_, unsigned which) -> size_t { return r_ < P ? (unsigned)__builtin_amdgcn_readfirstlane((int)R[2 * r_ + which]) : 0u; };
-    struct raw { unsigned x0, x1; unsigned long long mk; };       // a chunk as loaded: two letters per lane, the row's mask
-    auto load_chunk = [&](size_t c0, size_t bend) -> raw {
-        raw w = { 254u, 254u, 0ull };
+    struct raw { unsigned x0, x1; };                               // a chunk as loaded: two letters per lane
+    auto load_chunk = [&](size_t c0) -> raw {
+        raw w = { 254u, 254u };
         const size_t g0 = c0 + lane, g1 = g0 + 64;
         if (g0 < N) w.x0 = X[g0];
         if (lane < (unsigned)MT - 1 && g1 < N) w.x1 = X[g1];
-        if (DENSE && g0 < bend) w.mk = act[g0 * wg.gy + wg.y];
         return w;
     };
 
@@ -720,72 +682,45 @@ __device__ __forceinline__ void scanpool_bprop_bits_body(const wg_t wg, unsigned
     size_t nna = bound(r + 2 * step, 0), nnb = bound(r + 2 * step, 1);
     pooled_in q = load_pooled(r), nq = load_pooled(r + step);
     size_t c0 = a;
-    raw cur = r < P ? load_chunk(c0, b) : raw{ 254u, 254u, 0ull };
-    float gavg = 0.0f, gmax = 0.0f;
+    raw cur = r < P ? load_chunk(c0) : raw{ 254u, 254u };
+    float gmax = 0.0f;
     size_t imax = ~(size_t)0;
     unsigned tm[5] = { 0u, 0u, 0u, 0u, 0u };                        // letters of the taps at the winning row: bit t of tm[l]
     while (r < P) {                                                // uniform over the wave
         // ---- the chunk after this one is requested before this one is worked on
         const bool last = c0 + 64 >= b;
-        const size_t nc0 = last ? na : c0 + 64, nend = last ? nb : b;
+        const size_t nc0 = last ? na : c0 + 64;
         const bool more = last ? r + step < P : true;
-        raw nxt = { 254u, 254u, 0ull };
-        if (more) nxt = load_chunk(nc0, nend);
+        raw nxt = { 254u, 254u };
+        if (more) nxt = load_chunk(nc0);
         if (c0 == a) {
-            if (DENSE) gavg = b > a ? q.davg / (float)(b - a) : 0.0f;
-            if (PEAK) {
-                gmax = 0.0f; imax = ~(size_t)0;
-                if (q.pmax > 0.0f) { gmax = q.dmax; imax = q.arg / F; }
+            gmax = 0.0f; imax = ~(size_t)0;
+            if (q.pmax > 0.0f) { gmax = q.dmax; imax = q.arg / F; }
 #pragma unroll
-                for (int l = 0; l < 5; ++l) tm[l] = 0u;
-            }
+            for (int l = 0; l < 5; ++l) tm[l] = 0u;
         }
         // ---- one bit per (letter, position) of the chunk: positions c0 .. c0 + 63 and the MT - 1 behind them
         const unsigned v0 = letter_of(cur.x0), v1 = letter_of(cur.x1);
         unsigned long long L0[5], L1[5];
 #pragma unroll
         for (int l = 0; l < 5; ++l) { L0[l] = __ballot(v0 == (unsigned)l); L1[l] = __ballot(v1 == (unsigned)l); }
-        const size_t nrel = n > c0 ? n - c0 : 0;                   // rows of the chunk the scan defines
-        if (DENSE) {
-            // ---- one bit per row for this lane's filter: bit i of lane f = bit f of row i's mask
-            const unsigned mlo = (unsigned)cur.mk, mhi = (unsigned)(cur.mk >> 32);
-            unsigned tlo = mlo, thi = mhi;
-            transpose_masks(tlo, thi, lane);
-            db += gavg * (float)(__popc(tlo) + __popc(thi));
-            const unsigned long long keep = nrel >= 64 ? ~0ull : ((1ull << nrel) - 1ull);
-            tlo &= (unsigned)keep;
-            thi &= (unsigned)(keep >> 32);
+        // ---- the winning row of this lane's filter, if it lies in the chunk: its taps' letters
+        const bool here = imax >= c0 && imax - c0 < 64;
+        const unsigned rel = here ? (unsigned)(imax - c0) : 0u;
+        if (here) db += gmax;
+        const bool counts = here && imax < n;
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                for (int l = 0; l < 5; ++l) {
-                    const unsigned long long sh = t == 0 ? L0[l] : (L0[l] >> t) | (L1[l] << (64 - t));   // is_letter at row + t
-                    const unsigned cnt = __popc(tlo & (unsigned)sh) + __popc(thi & (unsigned)(sh >> 32));
-                    acc[l][t] = __builtin_fmaf(gavg, (float)cnt, acc[l][t]);
-                }
-            }
-        }
-        if (PEAK) {
-            // ---- the winning row of this lane's filter, if it lies in the chunk: its taps' letters
-            const bool here = imax >= c0 && imax - c0 < 64;
-            const unsigned rel = here ? (unsigned)(imax - c0) : 0u;
-            if (here) db += gmax;
-            const bool counts = here && imax < n;
-#pragma unroll
-            for (int l = 0; l < 5; ++l) {
-                const unsigned long long cut = rel == 0 ? L0[l] : (L0[l] >> rel) | (L1[l] << (64 - rel));
-                tm[l] |= counts ? (unsigned)cut : 0u;              // (MT <= 32 taps: the low word is all that is looked at)
-            }
-            if (last) {
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                    for (int l = 0; l < 5; ++l) acc[l][t] = __builtin_fmaf(gmax, (float)((tm[l] >> t) & 1u), acc[l][t]);
-                }
-            }
+        for (int l = 0; l < 5; ++l) {
+            const unsigned long long cut = rel == 0 ? L0[l] : (L0[l] >> rel) | (L1[l] << (64 - rel));
+            tm[l] |= counts ? (unsigned)cut : 0u;                  // (MT <= 32 taps: the low word is all that is looked at)
         }
         // ---- on to the next chunk / region
         if (last) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int l = 0; l < 5; ++l) acc[l][t] = __builtin_fmaf(gmax, (float)((tm[l] >> t) & 1u), acc[l][t]);
+            }
             r += step;
             a = na; b = nb; q = nq;
             na = nna; nb = nnb;
@@ -798,15 +733,266 @@ __device__ __forceinline__ void scanpool_bprop_bits_body(const wg_t wg, unsigned
     fold_waves_into_slab<MT>(smem, [&](int j, int c) { return acc[c][j] + 0.25f * acc[4][j]; }, db, m, F, f0, slabs + (size_t)wg.x * stride);
 }
 
-template <int PT, int MT>
+template <int MT>
 __global__ __launch_bounds__(256) void scanpool_bprop_bits_kernel(unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
                                                                   const uint32_t* __restrict__ R, size_t P,
                                                                   const float* __restrict__ pooled, const uint32_t* __restrict__ argmax,
-                                                                  const float* __restrict__ dpooled,
-                                                                  const unsigned long long* __restrict__ act,
-                                                                  float* __restrict__ slabs, size_t stride)
+                                                                  const float* __restrict__ dpooled, float* __restrict__ slabs, size_t stride)
 {
-    scanpool_bprop_bits_body<PT, MT>(this_wg(), m, F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
+    scanpool_bprop_bits_body<MT>(this_wg(), m, F, X, N, R, P, pooled, argmax, dpooled, slabs, stride);
+}
+
+// The mask-driven backward of average (and max + average) pooling, counted on the matrix cores. At every row of a region
+// whose rectifier is open the average-pooling gradient is the SAME number c = dpooled / rows, so the filter gradient needs
+// no pass over the rows but counts:
+//     dW[tap][letter][f] += c * #{rows of the region: open_f(row) and letter(row + tap) = letter}
+// and the counts are a product of bits, letters (4m x rows) times open rows (rows x filters), which
+// v_mfma_scale_f32_32x32x64_f8f6f4 forms 64 rows at a time and exactly: in its 4-bit format the bit pattern 0001 is 0.5, so
+// a word of 32 bits is made an operand by three shifts and four masks (the order of the contraction index is free as long
+// as both sides share it: dword d, nibble i is row 4 i + d). A letter is 0100 = 2, a "mean of the four" 0001 = 0.5 in all four
+// of its rows: with the 0.5 of an open row the 1 and the quarter they count.
+// The max-pooling gradient lands on one row per (region, filter): that is a column of bits too, with one set. A wave takes
+// 16 filters; columns 0-15 of its products are their open rows, columns 16-31 their winning rows, and at the end of a region
+// every column's counts are added to its sums with its own factor (a lane's, that is). The four waves of a workgroup share
+// the regions and write the four quarters of its slab: no fold through LDS.
+// The open rows come from the forward pass's activity masks, one 64-bit lane mask per row: a 16 x 16 bit transpose
+// among the lanes (16 rows of this wave's 16 filters per row of lanes) makes them one word of 32 rows per column.
+// Deterministic; c * count is rounded once where the kernels above add c count times, so the sums agree with theirs to
+// rounding, not bit for bit. PT: DBK_PT_AVG or DBK_PT_ALL.
+// What bounds it: instruction issue, ~90 vector and as many scalar instructions per chunk and wave beside the m / 8 products (matrix
+// cores busy a tenth of the time), with two to three waves per SIMD (sums, counts: 4 MT registers). Against one lane per filter that
+// counts by population counts, 10 instructions per (tap, letter) and chunk (us, kernel and reduction of its slabs, before / after):
+// 2048 regions of 90-200 rows x 128 filters, max + average, 32 taps 70 / 43, 24 taps 60 / 40, 8 taps 36 / 31; 20 000 x 101 x 256,
+// 24 taps 356 / 227; 128 x 101 x 64, 24 taps 26 / 16; 50 x 3000 x 64 339 / 34. Requesting a chunk's inputs in the step before,
+// with copies at its end, cost 15 to 25 % of that. Error of dW against float64 8.5e-8 (8.9e-8 before), of the bias 8.6e-8 (9.6e-8).
+typedef int i32x8_t __attribute__((ext_vector_type(8)));
+// 32 bits as 32 values 0 or 0.5 of the 4-bit format
+__device__ __forceinline__ i32x8_t bits_as_halves(unsigned w)
+{
+    const unsigned k = 0x11111111u;
+    return i32x8_t{(int)(w & k), (int)((w >> 1) & k), (int)((w >> 2) & k), (int)((w >> 3) & k), 0, 0, 0, 0};
+}
+// ... as 0 or 2
+__device__ __forceinline__ i32x8_t bits_as_twos(unsigned w)
+{
+    const unsigned k = 0x44444444u;
+    return i32x8_t{(int)((w << 2) & k), (int)((w << 1) & k), (int)(w & k), (int)((w >> 1) & k), 0, 0, 0, 0};
+}
+__device__ __forceinline__ f32x16_t count_product(const i32x8_t& letters, const i32x8_t& rows, const f32x16_t& c)
+{
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(letters, rows, c, 4, 4, 0, 127, 0, 127);      // (4-bit formats; block scales 1)
+}
+// Transposes a 16 x 16 bit matrix per row of 16 lanes: bit i of v is column i of this lane's row, afterwards row i of this lane's
+// column. Four butterfly stages (block sizes 8 ... 1): a lane and its partner lane ^ d swap the off-diagonal d x d blocks they
+// hold between them. The value is held twice, in both halves of the word, so that the shift of either side is a rotation.
+struct transpose16 {
+    unsigned keep[4], turn[4];
+    __device__ __forceinline__ explicit transpose16(unsigned lane)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const unsigned d = 8u >> k, clear = d == 8u ? 0x00ff00ffu : d == 4u ? 0x0f0f0f0fu : d == 2u ? 0x33333333u : 0x55555555u;
+            keep[k] = lane & d ? ~clear : clear;
+            turn[k] = lane & d ? d : 16u - d;
+        }
+    }
+    __device__ __forceinline__ unsigned stage(unsigned v, unsigned partner, int k) const
+    {
+        const unsigned other = __builtin_amdgcn_alignbit(partner, partner, turn[k]);
+        return other ^ ((v ^ other) & keep[k]);
+    }
+    __device__ __forceinline__ unsigned operator()(unsigned v) const
+    {
+        v |= v << 16;
+        v = stage(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true), 0);       // lane ^ 8
+        const int x7 = __builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, true);                    // lane ^ 7
+        v = stage(v, (unsigned)__builtin_amdgcn_mov_dpp(x7, 0x1b, 0xf, 0xf, true), 1);            // ^ 3: lane ^ 4
+        v = stage(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, true), 2);        // lane ^ 2
+        return stage(v, (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true), 3);     // lane ^ 1
+    }
+};
+
+template <int PT, int MT>
+__device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
+                                                           const uint32_t* __restrict__ R, size_t P,
+                                                           const float* __restrict__ pooled, const uint32_t* __restrict__ argmax,
+                                                           const float* __restrict__ dpooled,
+                                                           const unsigned long long* __restrict__ act,
+                                                           float* __restrict__ slabs, size_t stride)
+{
+    constexpr bool PEAK = PT == DBK_PT_ALL;
+    constexpr int NB = MT / 8;                                     // blocks of eight taps: 32 rows (tap, letter) of the product
+    constexpr unsigned NONE = ~0u;
+    const unsigned lane = threadIdx.x & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const unsigned col = lane & 31u, h = lane >> 5;
+    const bool peak = (lane & 16u) != 0u;                          // this lane's column: winning rows, or open rows
+    const unsigned f = wg.y * FT + 16u * wave + (lane & 15u);
+    const size_t n = N + 1 >= (size_t)m + 1 ? N - m + 1 : 0;      // rows the scan defines; later rows carry bias only
+    const unsigned short* act16 = reinterpret_cast<const unsigned short*>(act) + 4 * (size_t)wg.y + wave;
+    const transpose16 transpose(lane);
+    // as a row of the letters' operand: letter col & 3 of tap col >> 2 of each block
+    const unsigned not0 = col & 1u ? 0u : ~0u, not1 = col & 2u ? 0u : ~0u, tap = col >> 2;
+    f32x16_t sums[NB], counts[NB];
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) { sums[t][i] = 0.0f; counts[t][i] = 0.0f; }
+    float db = 0.0f;
+    // A wave's regions are wg.x, wg.x + gx, ...: lane i holds the bounds of the i-th of 64 of them.
+    const size_t step = wg.gx;
+    const unsigned nregion = N != 0 && wg.x < P ? (unsigned)((P - wg.x + step - 1) / step) : 0u;     // (without rows every region is empty)
+    unsigned va = 0u, vb = 0u;
+    auto load_bounds = [&](unsigned k) {
+        const size_t e = wg.x + ((size_t)k + lane) * step, r_ = e < P ? e : P - 1;
+        va = R[2 * r_]; vb = R[2 * r_ + 1];
+        __builtin_amdgcn_s_waitcnt(0x0f70);                        // vmcnt(0), here: else every step that may come this way waits for all that is under way
+    };
+    // What a chunk needs - its letters (two per lane) and masks, a region's first one its factors - is requested two chunks ahead, into
+    // the registers that the chunk in work has just left (a copy on the way would wait for what is still under way), without
+    // branches on the lane: past the end the last letter and row are read, and not used.
+    struct chunk_in { unsigned x0, x1, mk, arg; float g, pmax; };
+    struct place { unsigned k, a, b, c; };                         // a chunk: which of the wave's regions, its bounds, first row
+    auto advance = [&](place& k) {
+        if (k.b > k.c && k.b - k.c > 64u) { k.c += 64u; return; }
+        ++k.k;
+        if ((k.k & 63u) == 0u) load_bounds(k.k);
+        k.a = k.c = (unsigned)__builtin_amdgcn_readlane((int)va, (int)(k.k & 63u));
+        k.b = (unsigned)__builtin_amdgcn_readlane((int)vb, (int)(k.k & 63u));
+    };
+    // chunks up to here lie inside the text, and inside the rows that the scan defines
+    const bool any_inside = N >= 128, any_defined = n >= 64;
+    const unsigned inside = (unsigned)(N - 128 < 0xffffffffull ? N - 128 : 0xffffffffull), defined = (unsigned)(n - 64 < 0xffffffffull ? n - 64 : 0xffffffffull);
+    const unsigned fe = f < F ? f : F - 1u, row_words = 4u * wg.gy;
+    auto request_chunk = [&](const place& k, chunk_in& in) {
+        size_t base = k.c;
+        unsigned e0 = lane, e1 = lane + 64u, em = lane * row_words;
+        if (!(any_inside && k.c <= inside)) {
+            if (base >= N) base = N - 1;
+            const unsigned more = N - 1 - base < 128 ? (unsigned)(N - 1 - base) : 128u;
+            e0 = e0 < more ? e0 : more; e1 = e1 < more ? e1 : more; em = e0 * row_words;
+        }
+        in.x0 = (X + base)[e0];
+        in.x1 = (X + base)[e1];
+        in.mk = (act16 + base * row_words)[em];
+        if (k.c == k.a) {
+            const size_t r_ = wg.x + (size_t)k.k * step, j0 = (r_ < P ? r_ : P - 1) * F;
+            if (PEAK) { in.g = (dpooled + 2 * j0)[2u * fe + (peak ? 0u : 1u)]; in.pmax = (pooled + 2 * j0)[2u * fe]; in.arg = (argmax + j0)[fe]; }
+            else in.g = (dpooled + j0)[fe];
+        }
+    };
+    chunk_in in0 = { 254u, 254u, 0u, 0u, 0.0f, 0.0f }, in1 = in0;
+    place now = { 0u, 0u, 0u, 0u }, next = now;
+    if (nregion != 0u) {
+        load_bounds(0u);
+        now.a = now.c = (unsigned)__builtin_amdgcn_readlane((int)va, 0);
+        now.b = (unsigned)__builtin_amdgcn_readlane((int)vb, 0);
+        request_chunk(now, in0);
+        next = now;
+        advance(next);
+        request_chunk(next, in1);
+    }
+    float g = 0.0f;                                                // this column's factor
+    unsigned top = NONE, open = 0u;                                // its winning row; how many of its bits were set (this half wave's)
+    auto work = [&](chunk_in& in) {
+        const unsigned c = now.c, left = now.b > c ? now.b - c : 0u;      // rows of the region from this chunk on
+        const bool first = c == now.a, last = left <= 64u;
+        // ---- the letters: one bit per (letter, position) of the chunk, positions c .. c + 63 and the MT - 1 behind them
+        if (!(any_inside && c <= inside)) {
+            if ((size_t)c + lane >= N) in.x0 = 254u;
+            if ((size_t)c + 64 + lane >= N) in.x1 = 254u;
+        }
+        const unsigned long long V0 = __ballot(in.x0 < 4u), E0 = __ballot((in.x0 & 1u) != 0u), T0 = __ballot((in.x0 & 2u) != 0u);
+        const unsigned V1 = (unsigned)__ballot(in.x1 < 4u), E1 = (unsigned)__ballot((in.x1 & 1u) != 0u), T1 = (unsigned)__ballot((in.x1 & 2u) != 0u);
+        const unsigned long long Z0 = __ballot(in.x0 == 254u);
+        const unsigned Z1 = (unsigned)__ballot(in.x1 == 254u);
+        // ---- the columns: 32 rows' bits
+        const unsigned v = transpose(lane < left ? in.mk : 0u);
+        if (first) {
+            g = now.b > now.a && f < F ? in.g / (float)(now.b - now.a) : 0.0f;
+            if (peak) {
+                const bool any = PEAK && in.pmax > 0.0f && f < F;
+                g = any ? in.g : 0.0f;
+                top = any ? in.arg / F : NONE;
+            }
+        }
+        // ---- what comes after the next chunk is on its way while this one is worked on
+        place after = next;
+        advance(after);
+        request_chunk(after, in);
+        if (now.k < nregion) {
+            const auto halves = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+            unsigned bits = __builtin_amdgcn_perm(halves[1], halves[0], 0x05040100u);
+            const unsigned rel = top - c - 32u * h;
+            if (peak) bits = PEAK && top != NONE && rel < 32u ? 1u << (rel & 31u) : 0u;
+            open += (unsigned)__popc(bits);
+            if (!(any_defined && c <= defined)) {                      // rows that the scan does not define
+                const size_t nrel = n > c ? n - c : 0;
+                if (nrel < 64) bits &= (unsigned)(((1ull << nrel) - 1ull) >> (32u * h));
+            }
+            // ---- the counts
+            const i32x8_t B = bits_as_halves(bits);
+            auto letter = [&](unsigned v_, unsigned e, unsigned t) -> unsigned { return (e ^ not0) & (t ^ not1) & v_; };
+            const unsigned w0 = letter((unsigned)V0, (unsigned)E0, (unsigned)T0), w1 = letter((unsigned)(V0 >> 32), (unsigned)(E0 >> 32), (unsigned)(T0 >> 32)), w2 = letter(V1, E1, T1);
+            const unsigned wl = h ? w1 : w0, wh = h ? w2 : w1;         // from this half wave's first row on
+            i32x8_t A[NB];
+#pragma unroll
+            for (int t = 0; t < NB; ++t) A[t] = bits_as_twos(__builtin_amdgcn_alignbit(wh, wl, 8u * t + tap));
+            const unsigned long long M0 = ~(V0 | Z0);              // neither a letter nor nothing: the mean of the four
+            const unsigned M1 = ~(V1 | Z1);
+            if ((M0 | M1) != 0ull) {
+                const unsigned ml = h ? (unsigned)(M0 >> 32) : (unsigned)M0, mh = h ? M1 : (unsigned)(M0 >> 32);
+#pragma unroll
+                for (int t = 0; t < NB; ++t) A[t] = A[t] | bits_as_halves(__builtin_amdgcn_alignbit(mh, ml, 8u * t + tap));
+            }
+            if (first) {
+#pragma unroll
+                for (int t = 0; t < NB; ++t) counts[t] = count_product(A[t], B, f32x16_t{});
+            } else {
+#pragma unroll
+                for (int t = 0; t < NB; ++t) counts[t] = count_product(A[t], B, counts[t]);
+            }
+            // ---- a region's end
+            if (last) {
+                db = __builtin_fmaf(g, (float)open, db);
+                open = 0u;
+#pragma unroll
+                for (int t = 0; t < NB; ++t)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sums[t][i] = __builtin_fmaf(g, counts[t][i], sums[t][i]);
+            }
+        }
+        now = next;
+        next = after;
+    };
+    // (no way out between the two: the compiler's waits cover every path, and one that leaves a request out would make them longer)
+    while (now.k < nregion) {                                      // uniform over the wave
+        work(in0);
+        work(in1);
+    }
+    // ---- this wave's quarter of the slab: a filter's two columns side by side, register i's sums in lanes 0-15 and 32-47, register
+    // i + 1's in the others. Register i holds letter i & 3 of tap 2 (i >> 2) + h of its block.
+    float* out = slabs + (size_t)wg.x * stride;
+#pragma unroll
+    for (int t = 0; t < NB; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(sums[t][i]), __float_as_uint(sums[t][i + 1]), false, false);
+            const unsigned j = 8u * t + 2u * (i >> 2) + h;
+            if (j < m && f < F) out[(size_t)(4u * j + (i & 3) + (peak ? 1u : 0u)) * F + f] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        }
+    const auto d16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(db), __float_as_uint(db), false, false);
+    db = __uint_as_float(d16[0]) + __uint_as_float(d16[1]);
+    const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(db), __float_as_uint(db), false, false);
+    if (lane < 16u && f < F) out[(size_t)4 * m * F + f] = __uint_as_float(d32[0]) + __uint_as_float(d32[1]);
+}
+
+template <int PT, int MT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 32 ? 2 : 3)))
+void scanpool_bprop_counts_kernel(unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N, const uint32_t* __restrict__ R, size_t P,
+                                  const float* __restrict__ pooled, const uint32_t* __restrict__ argmax, const float* __restrict__ dpooled,
+                                  const unsigned long long* __restrict__ act, float* __restrict__ slabs, size_t stride)
+{
+    scanpool_bprop_counts_body<PT, MT>(this_wg(), m, F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
 }
 
 // Launch shapes, shared by the single-group launchers and the multi-group ones.
@@ -861,11 +1047,9 @@ inline unsigned wide_grid_x(unsigned ftiles, size_t P)
     return gx;
 }
 inline size_t wide_smem(unsigned mt) { return (size_t)mt * NL * FT * sizeof(float) + 4 * (mt == 16 ? wide_shape<16>::xbytes : wide_shape<24>::xbytes); }
-// The bit-count backward: a wave per region, three workgroups per CU resident (its 5 x MT sums and the rest take ~160
-// registers at 24 taps: three waves per SIMD);
+// The bit kernel of max pooling: a wave per region, three workgroups per CU resident (its 5 x MT sums and the rest take ~150
+// registers at 24 taps: three waves per SIMD; ~190 at 32: two);
 // the smallest grid that gives every wave the same number of regions as the resident grid would.
-// At 32 taps they take ~200: two waves per SIMD, two workgroups per CU. (A step of 8 models on 2048 sequences of 90-200 nt,
-// max + average pooling, 32 taps: 7.3 ms through the per-wave LDS tables that any longer filter takes, 0.115 ms this way.)
 inline unsigned bits_grid_x(unsigned mt, unsigned ftiles, size_t P)
 {
     unsigned gx = (mt == 32 ? 512u : 768u) / ftiles;
@@ -877,7 +1061,20 @@ inline unsigned bits_grid_x(unsigned mt, unsigned ftiles, size_t P)
     const size_t per_wave = (P + (size_t)gx * 4 - 1) / ((size_t)gx * 4);
     return (unsigned)((P + 4 * per_wave - 1) / (4 * per_wave));
 }
-// Max pooling goes through it while the regions are short on average (it visits every 64-row chunk of a region to
+// The counting backward: as many workgroups as are resident at once (two per CU with 32 taps, else three, the third only
+// where each of them gets many regions), every workgroup the same number of regions, at least eight chunks of 64 rows (the
+// sums' way out and their reduction cost about as much). us with the third, without: 20 000 regions x 101 x 256 filters 240 / 277, 2048 x
+// 145 x 128 42 / 41. us with eight regions, four: 128 x 101 x 64 17.8 / 14.6, 256 x 30 x 512 16.8 / 18.4; 50 x 3000 x 64 216 / 113, one 34.
+inline unsigned counts_grid_x(unsigned mt, unsigned ftiles, size_t N, size_t P)
+{
+    size_t gx = (mt < 32 && P * ftiles >= 16 * 768 ? 768u : 512u) / ftiles;
+    if (gx < 1) gx = 1;
+    const size_t chunks = N / (64 * P) > 0 ? N / (64 * P) : 1, least = chunks < 8 ? (8 + chunks - 1) / chunks : 1;
+    if (gx > (P + least - 1) / least) gx = (P + least - 1) / least;
+    const size_t per_group = (P + gx - 1) / gx;
+    return (unsigned)((P + per_group - 1) / per_group);
+}
+// Max pooling goes through the bit kernel while the regions are short on average (it visits every 64-row chunk of a region to
 // find each filter's winning row; the sparse kernel goes straight to that row).
 inline bool bits_takes_max(size_t N, size_t P) { return N <= 128 * P; }
 inline size_t bits_smem(unsigned) { return FOLD_BYTES; }
@@ -977,12 +1174,11 @@ int launch_fprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
 }
 
 template <int PT, int MT>
-int launch_bits(hipStream_t st, unsigned gx, unsigned ftiles, size_t smem, size_t m, size_t F, const uint8_t* X, size_t N, const uint32_t* R,
-                size_t P, const float* pooled, const uint32_t* argmax, const float* dpooled, const unsigned long long* act, float* slabs, size_t stride)
+int launch_counts(hipStream_t st, unsigned gx, unsigned ftiles, size_t m, size_t F, const uint8_t* X, size_t N, const uint32_t* R,
+                  size_t P, const float* pooled, const uint32_t* argmax, const float* dpooled, const unsigned long long* act, float* slabs, size_t stride)
 {
-    auto kern = scanpool_bprop_bits_kernel<PT, MT>;
-    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), smem, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
+    auto kern = scanpool_bprop_counts_kernel<PT, MT>;
+    hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), 0, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
     return 0;
 }
 
@@ -991,7 +1187,7 @@ int launch_dense(hipStream_t st, unsigned gx, unsigned ftiles, size_t smem, cons
                   const uint8_t* X, size_t N, const uint32_t* R, size_t P, const float* pooled, const uint32_t* argmax,
                   const float* dpooled, const unsigned long long* act, float* slabs, size_t stride)
 {
-    if (act) return launch_bits<PT, MT>(st, gx, ftiles, smem, m, F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
+    if (act) return launch_counts<PT, MT>(st, gx, ftiles, m, F, X, N, R, P, pooled, argmax, dpooled, act, slabs, stride);
     auto kern = scanpool_bprop_dense_kernel<PT, MT>;
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(256), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled, slabs, stride);
@@ -1008,7 +1204,7 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
     const size_t nW = 4 * m * F, stride = nW + F;
     const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : (m <= 24 ? 24 : (m <= 32 ? 32 : 0)));
     // Average pooling without the forward pass's activity masks: the matrix-core forward writes them again (into the
-    // stream's second scratch buffer, with its pooled values beside them), and the bit-count kernel takes them from
+    // stream's second scratch buffer, with its pooled values beside them), and the counting kernel takes them from
     // there; less than half the time of recomputing the map through the letter table, whose registers moreover end at 24
     // taps: longer filters take this way at every size.
     const size_t mask_bytes = N * ftiles * sizeof(unsigned long long), pooled_bytes = P * F * 2 * sizeof(float);
@@ -1044,18 +1240,18 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
     // with max+avg pooling the dense half carries the maxima along
     const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P);
     const unsigned gxs = PT == DBK_PT_MAX ? (max_bits ? bits_grid_x(mt, ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
-    const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? bits_grid_x(mt, ftiles, P) : dense_grid_x(mt, ftiles, P);
+    const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? counts_grid_x(mt, ftiles, N, P) : dense_grid_x(mt, ftiles, P);
     const size_t smem_s = sparse_smem(m), smem_d = mt == 32 ? bits_smem(mt) : dense_smem(mt);
     DBK_CHECK(smem_s <= lds_limit() && smem_d <= lds_limit(), "ValueError: filter length %zu does not fit in LDS", m);
     float* slabs = (float*)dbk::workspace(stride * (gxs + gxd) * sizeof(float), st);
     DBK_CHECK(slabs != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", stride * (gxs + gxd) * sizeof(float), dbk::workspace_error());
     if (gxs && max_bits) {
-        auto kern = mt == 8 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 8> : mt == 16 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 16>
-                  : mt == 24 ? scanpool_bprop_bits_kernel<DBK_PT_MAX, 24> : scanpool_bprop_bits_kernel<DBK_PT_MAX, 32>;
+        auto kern = mt == 8 ? scanpool_bprop_bits_kernel<8> : mt == 16 ? scanpool_bprop_bits_kernel<16>
+                  : mt == 24 ? scanpool_bprop_bits_kernel<24> : scanpool_bprop_bits_kernel<32>;
         const size_t smem_b = bits_smem(mt);
         DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_b));
         hipLaunchKernelGGL(kern, dim3(gxs, ftiles), dim3(256), smem_b, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled,
-                           (const unsigned long long*)nullptr, slabs, stride);
+                           slabs, stride);
     } else if (gxs) {
         constexpr int PS = PT == DBK_PT_AVG ? DBK_PT_MAX : PT;
         auto kern = mt == 8 ? scanpool_bprop_sparse_kernel<PS, 8> : mt == 16 ? scanpool_bprop_sparse_kernel<PS, 16>
@@ -1070,7 +1266,7 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
         if (mt == 8) rc = launch_dense<PD, 8>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
         else if (mt == 16) rc = launch_dense<PD, 16>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
         else if (mt == 24) rc = launch_dense<PD, 24>(st, gxd, ftiles, smem_d, W, bias, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
-        else rc = launch_bits<PD, 32>(st, gxd, ftiles, smem_d, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
+        else rc = launch_counts<PD, 32>(st, gxd, ftiles, m, F, X, N, R, P, pooled, argmax, dpooled, act, sd, stride);
         if (rc) return rc;
     }
     if (dbk::deferred_sums* later = dbk::deferred()) { later->slabs = slabs; later->slab_stride = stride; later->nslab = gxs + gxd; }
@@ -1161,23 +1357,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 24 ? 
         scanpool_fprop_body<DBK_PT_AVG, false, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, nullptr, nullptr, j.act);
 }
 
-// The bit-count kernel; for max pooling over long regions the one-wave sparse kernel in the first wave of the
+// The counting kernel; for max pooling the bit kernel, over long regions the one-wave sparse kernel in the first wave of the
 // workgroup (the other waves leave at once).
 template <int MT>
-__global__ __launch_bounds__(256) void scanpool_bprop_multi_kernel(const multi_args a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 32 ? 2 : 3))) void scanpool_bprop_multi_kernel(const multi_args a)
 {
     wg_t wg;
     const unsigned gi = multi_locate(a, wg);
     const dbk::scan_group& j = a.g[gi];
     if (j.ptype == DBK_PT_MAX) {
         if (a.wide[gi])
-            scanpool_bprop_bits_body<DBK_PT_MAX, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, nullptr, j.slabs, j.slab_stride);
+            scanpool_bprop_bits_body<MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.slabs, j.slab_stride);
         else if (threadIdx.x < 64)
             scanpool_bprop_sparse_body<DBK_PT_MAX, MT>(wg, a.m, j.F, j.X, a.N, a.P, j.pooled, j.argmax, j.dpooled, j.slabs, j.slab_stride);
     } else if (j.ptype == DBK_PT_ALL) {
-        scanpool_bprop_bits_body<DBK_PT_ALL, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.act, j.slabs, j.slab_stride);
+        scanpool_bprop_counts_body<DBK_PT_ALL, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.act, j.slabs, j.slab_stride);
     } else {
-        scanpool_bprop_bits_body<DBK_PT_AVG, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.act, j.slabs, j.slab_stride);
+        scanpool_bprop_counts_body<DBK_PT_AVG, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.act, j.slabs, j.slab_stride);
     }
 }
 
@@ -1251,9 +1447,9 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
     size_t total = 0;
     for (unsigned i = 0; i < n; ++i) {
         a.ftiles[i] = dbk::divup(g[i].F, FT);
-        // as the group's own launch would choose: the bit-count kernel, or the sparse one for max pooling over long regions
+        // as the group's own launch would choose: the counting kernel, for max pooling the bit kernel or, over long regions, the sparse one
         a.wide[i] = g[i].ptype != DBK_PT_MAX || bits_takes_max(N, P);
-        a.gx[i] = a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
+        a.gx[i] = g[i].ptype != DBK_PT_MAX ? counts_grid_x(mt, a.ftiles[i], N, P) : a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
         a.first[i + 1] = a.first[i] + a.gx[i] * a.ftiles[i];
         g[i].slab_stride = 4 * m * (size_t)g[i].F + g[i].F;
         g[i].nslab = a.gx[i];
