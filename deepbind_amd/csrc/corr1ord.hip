@@ -964,11 +964,11 @@ __global__ __launch_bounds__(64 * MB) void corr1ord_bprop_X_mfma_kernel(float* _
 // those, 24 taps): 50 000 rows x 256 filters 96 / 52, 100 000 x 128 52 / 50, 100 000 x 256 98 / 87 (12 taps: 97 / 58), 150 000 x 256
 // 123 / 119, 120 000 x 128 of 32 taps 56 / 62, 250 000 x 128 66 / 80, 250 000 x 256 127 / 150, 500 000 x 256 235 / 305. Its launch costs ~50 us up to
 // ~120 000 rows whatever the taps, so rows x steps of the other kernel decide.
-// (Filters that do not fill a launch of 128 take unaligned loads: 113 to 127 pay only at two blocks of eight taps, and until a workgroup
-// gets more than its 1024 rows: 127 of 16 taps, 250 000 rows 61 / 74, 400 000 88 / 117, 600 000 219 / 165; of 24 taps 400 000 160 / 144.)
+// (Filters that do not fill a launch of 128 take unaligned loads: 113 to 127 pay only at two blocks of eight taps:
+// 127 of 16 taps, 250 000 rows 61 / 74, 400 000 88 / 117, 600 000 163 / 193, 1.0 M 243 / 277; of 24 taps 400 000 160 / 144.)
 inline bool bprop_X_mfma_takes(size_t m, size_t F, size_t n)
 {
-    if (F > 112 && F < 128) return m > 12 && m <= 16 && n >= 230000 && n <= 512 * 1024;
+    if (F > 112 && F < 128) return m > 12 && m <= 16 && n >= 230000;
     return m <= 32 && F >= 128 && n * (m + 3) >= 3750000;
 }
 
@@ -977,9 +977,12 @@ inline int launch_bprop_X_mfma(hipStream_t st, float* dX, size_t n, const float*
     // two workgroups fit a CU: about 512 of them in all, so that the weights' pieces are formed once per many rows
     // (512 rows per workgroup: 0.61 ms at 1.0 M rows x 256 filters; 1/512 of the rows: 0.54 ms; at most 1024, the result
     // rows in LDS and the rows of dZ requested a block ahead: 0.51 ms)
-    unsigned rows = (unsigned)(((n + 511) / 512 + 31) / 32 * 32);
+    // Where that takes several rounds of 512, they are made alike: 600 000 rows are two rounds of 608 rows, not one of 1024 and a
+    // second of 74 workgroups (us a call, rows of 1024 / rounds alike: 600 000 rows x 128 filters x 16 taps 191 / 128, 560 000 x 256 x
+    // 24 368 / 277, 800 000 x 256 x 32 444 / 394, 1.1 M x 256 x 24 554 / 496, 1.2 M x 128 x 12 290 / 241).
+    const size_t rounds = (n + 512 * (size_t)GX_WGROWS - 1) / (512 * (size_t)GX_WGROWS);
+    unsigned rows = (unsigned)(((n + 512 * rounds - 1) / (512 * rounds) + 31) / 32 * 32);
     if (rows < GX_ROWS) rows = GX_ROWS;
-    if (rows > GX_WGROWS) rows = GX_WGROWS;
     const unsigned gx = (unsigned)dbk::divup(n, rows), mb = (unsigned)((4 * m + 31) / 32);
     for (size_t f0 = 0; f0 < F; f0 += GX_FILTERS) {
         const bool whole = F % 4 == 0 && f0 + GX_FILTERS <= F;
