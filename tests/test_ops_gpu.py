@@ -683,6 +683,26 @@ def test_scanpool_bprop_with_activity_masks_equals_recomputation(ks, ptype, B, l
         ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, path="kmer", act=act)
 
 
+@pytest.mark.parametrize("n,m,F", [(512 * 1024, 16, 128), (512 * 1024 + 1, 16, 128), (512 * 1056 - 31, 9, 130), (600000, 15, 127), (1024 * 1024 + 33, 8, 128)])
+def test_corr1ord_bprop_X_in_rounds(ks, n, m, F):
+    """Bulk maps around the sizes where the workgroups' rows are divided into another number of rounds: every row of the result, the
+    last of a workgroup and the first of the next among them, against float64. Bound: F m products a value, of unit-variance terms,
+    float32 sums: 1e-5 of the largest."""
+    g = torch.Generator(device="cuda").manual_seed(n % 1000)
+    W = torch.randn(4 * m, F, device="cuda", generator=g) * 0.1
+    dZ = torch.randn(n, F, device="cuda", generator=g)
+    dX = torch.zeros(n, 4, device="cuda")
+    ks.corr1ord_bprop_X(dX, W, dZ, 4)
+    ref = torch.zeros(n, 4, device="cuda", dtype=torch.float64)
+    for a in range(0, n, 1 << 17):
+        e = min(n, a + (1 << 17))
+        Y = (dZ[a:e].double() @ W.double().T).reshape(e - a, m, 4)
+        for k in range(m):
+            stop = min(e, n - k)
+            ref[a + k:stop + k] += Y[:stop - a, k]
+    assert ((dX - ref).abs().max() / ref.abs().max()).item() < 1e-5
+
+
 @pytest.mark.parametrize("ptype", ["avg", "all"])
 @pytest.mark.parametrize("lengths,m,F", [((1, 63, 64, 65, 0, 127, 128, 129, 300), 8, 16), ((64, 0, 2, 192, 31, 33), 9, 1), ((40,) * 70, 16, 17),
                                          ((53, 200, 64), 24, 65), ((1, 0, 700, 5) * 3, 25, 48), ((100,) * 9, 32, 130), ((0, 2, 1) * 17000, 8, 16),
