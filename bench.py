@@ -24,6 +24,8 @@ if ROOT not in sys.path:
 
 FP32_VECTOR_PEAK_TFLOPS = 157.3     # MI355X published FP32 vector peak (FMA = 2 FLOP)
 FP32_ADD_ISSUE_PEAK_TADDS = 78.6    # the same peak for a stream of plain adds (1 FLOP per lane-operation)
+MATRIX_F8F6F4_PEAK_TFLOPS = 10066.0  # 32 x 32 x 64 multiply-adds of 4-bit by 6-bit floats per 32 clocks and SIMD, 1 024 SIMDs at 2.4 GHz
+MATRIX_OPS_PER_INSTRUCTION = 2.0 * 32 * 32 * 64
 HBM_PEAK_GBS = 8000.0
 
 
@@ -132,16 +134,16 @@ def train_cpu_baseline(cfg, groups, nsteps=2, budget_s=12.0):
                       % (spec.nmodel, runs)}
 
 
-def measured_traffic(workload):
-    """HBM bytes per launch of the dominant kernel as measured offline with rocprofv3 --pmc
-    FETCH_SIZE / WRITE_SIZE (scaled by a copy kernel of known size) for the full-size workload;
-    None when no measurement is on file for this workload."""
+def measured_counter(workload, name):
+    """A figure per launch of the dominant kernel as measured offline with rocprofv3 --pmc for the full-size workload: HBM bytes
+    (FETCH_SIZE / WRITE_SIZE, scaled by a copy kernel of known size) or matrix instructions (SQ_INSTS_MFMA); None when no measurement
+    is on file for this workload."""
     if workload != "config5":
         return None
-    path = os.path.join(ROOT, "profiles", "scanpool_kmer_config5_counters.md")
+    path = os.path.join(ROOT, "profiles", "scan_digits_counters.md")
     try:
         for line in open(path):
-            if line.startswith("traffic_bytes_per_launch:"):
+            if line.startswith(name + ":"):
                 return int(line.split(":")[1])
     except OSError:
         pass
@@ -325,8 +327,7 @@ def ops_throughput(reps=5):
     rec("scanpool_fprop bulk[all, argmax]", timed(lambda: ks.scanpool_fprop(W, b, X, R, "all", want_argmax=True, path="kmer")),
         N + 3 * B * F * 4, adds)
     del X, R, W, b, dW, db, dX, P, I, dP
-    # shorter filters at bulk-scoring size (65 536 sequences x 101 nt): up to 18 taps the table kernel walks through
-    # regions that follow each other without a fresh start
+    # shorter filters at bulk-scoring size (65 536 sequences x 101 nt)
     B2 = 65536
     codes = rng.integers(0, 4, (B2, L), dtype=np.uint8)
     codes[rng.random((B2, L)) < 0.01] = 255
@@ -422,6 +423,8 @@ def main():
     adds_per_s = adds / (scan_ms * 1e-3)
     # algorithmic HBM bytes of the scan+pool launch: sequence bytes in, filters in, pooled features out
     hbm_bytes = cfg["X"].size + p["Wc"].nbytes + p["bc"].nbytes + nseq * spec.F * 4
+    matrix_instructions = measured_counter(args.workload, "matrix_instructions_per_launch")
+    matrix_tflops = None if matrix_instructions is None else matrix_instructions * MATRIX_OPS_PER_INSTRUCTION / (scan_ms * 1e-3) / 1e12
     out = {
         "metric": "seq_positions_per_sec_fwd_scan_pool",
         "value": positions * args.steps / elapsed,
@@ -437,15 +440,15 @@ def main():
         "sequences_per_s": nseq * args.steps / elapsed,
         "model_sequences_per_s": nseq * spec.nmodel * args.steps / elapsed,
         "roofline": {
-            # compute-bound on the FP32 vector ALUs (a gather-add: no matrix instruction is issued)
-            "bound": "fp32_valu", "bound_detail": "FP32 vector ALU gather-add, no MFMA instruction issued; peak = published 157.3 TFLOP/s FP32 vector "
-                                                  "(FMA-counted); a stream of plain adds tops out at 78.6 T adds/s",
-            "achieved": adds_per_s / 1e12, "peak": FP32_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
-            "frac": adds_per_s / 1e12 / FP32_VECTOR_PEAK_TFLOPS,
-            "frac_vs_add_issue_peak": adds_per_s / 1e12 / FP32_ADD_ISSUE_PEAK_TADDS,
-            "traffic": measured_traffic(args.workload),
-            "traffic_source": "read from the committed counter profile profiles/scanpool_kmer_config5_counters.md (rocprofv3 --pmc FETCH_SIZE / "
-                              "WRITE_SIZE runs of this workload, scaled by a copy kernel of known size); not measured in this run",
+            # bound by the matrix cores: one-hot letters times the weights' 6-bit digits
+            "bound": "mfma_f8f6f4", "bound_detail": "matrix operations executed (4-bit letters x 6-bit digits of the float32 weights, three digits to place "
+                                                    "the maximum); peak at 2.4 GHz, of which the power limit leaves about two thirds under these operands",
+            "achieved": matrix_tflops, "peak": MATRIX_F8F6F4_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": None if matrix_tflops is None else matrix_tflops / MATRIX_F8F6F4_PEAK_TFLOPS,
+            "algorithmic_adds_T_per_s": adds_per_s / 1e12,
+            "traffic": measured_counter(args.workload, "traffic_bytes_per_launch"),
+            "traffic_source": "traffic and matrix instructions per launch are read from the committed counter profile profiles/scan_digits_counters.md "
+                              "(rocprofv3 --pmc runs of this workload); not measured in this run",
             "kernel": "fused scan+bias+relu+maxpool (dbk_scanpool_fprop launches)", "kernel_ms": scan_ms,
             "algorithmic_adds_per_launch": adds,
             "hbm": {"algorithmic_bytes_per_launch": hbm_bytes, "achieved_GBs": hbm_bytes / (scan_ms * 1e-3) / 1e9,
