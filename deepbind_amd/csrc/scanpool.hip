@@ -758,7 +758,8 @@ __global__ __launch_bounds__(256) void scanpool_bprop_bits_kernel(unsigned m, un
 // The open rows come from the forward pass's activity masks, one 64-bit lane mask per row: a 16 x 16 bit transpose
 // among the lanes (16 rows of this wave's 16 filters per row of lanes) makes them one word of 32 rows per column.
 // Deterministic; c * count is rounded once where the kernels above add c count times, so the sums agree with theirs to
-// rounding, not bit for bit. PT: DBK_PT_AVG or DBK_PT_ALL.
+// rounding, not bit for bit. PT: DBK_PT_AVG or DBK_PT_ALL; DBK_PT_MAX (small batches of short regions, counts_takes_max) has the
+// winning rows alone: a wave takes 32 filters, two waves a tile, and a workgroup two shares of the regions with a slab each.
 // What bounds it: instruction issue, ~90 vector and as many scalar instructions per chunk and wave beside the m / 8 products (matrix
 // cores busy a tenth of the time), with two to three waves per SIMD (sums, counts: 4 MT registers). Against one lane per filter that
 // counts by population counts, 10 instructions per (tap, letter) and chunk (us, kernel and reduction of its slabs, before / after):
@@ -820,13 +821,14 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
                                                            const unsigned long long* __restrict__ act,
                                                            float* __restrict__ slabs, size_t stride)
 {
-    constexpr bool PEAK = PT == DBK_PT_ALL;
+    constexpr bool DENSE = PT != DBK_PT_MAX, PEAK = PT != DBK_PT_AVG;
     constexpr int NB = MT / 8;                                     // blocks of eight taps: 32 rows (tap, letter) of the product
     constexpr unsigned NONE = ~0u;
     const unsigned lane = threadIdx.x & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
-    const bool peak = (lane & 16u) != 0u;                          // this lane's column: winning rows, or open rows
-    const unsigned f = wg.y * FT + 16u * wave + (lane & 15u);
+    const bool peak = !DENSE || (lane & 16u) != 0u;                // this lane's column: winning rows, or open rows
+    const unsigned f = wg.y * FT + (DENSE ? 16u * wave + (lane & 15u) : 32u * (wave & 1u) + col);
+    const unsigned share = DENSE ? wg.x : 2u * wg.x + (wave >> 1), shares = DENSE ? wg.gx : 2u * wg.gx;      // of the regions: a slab each
     const size_t n = N + 1 >= (size_t)m + 1 ? N - m + 1 : 0;      // rows the scan defines; later rows carry bias only
     const unsigned short* act16 = reinterpret_cast<const unsigned short*>(act) + 4 * (size_t)wg.y + wave;
     const transpose16 transpose(lane);
@@ -837,13 +839,13 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
     for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) { sums[t][i] = 0.0f; counts[t][i] = 0.0f; }
-    float db = 0.0f;
-    // A wave's regions are wg.x, wg.x + gx, ...: lane i holds the bounds of the i-th of 64 of them.
-    const size_t step = wg.gx;
-    const unsigned nregion = N != 0 && wg.x < P ? (unsigned)((P - wg.x + step - 1) / step) : 0u;     // (without rows every region is empty)
+    float db = 0.0f, db_odd = 0.0f;                                // (every other region's apart: shorter chains round less)
+    // A wave's regions are share, share + shares, ...: lane i holds the bounds of the i-th of 64 of them.
+    const size_t step = shares;
+    const unsigned nregion = N != 0 && share < P ? (unsigned)((P - share + step - 1) / step) : 0u;     // (without rows every region is empty)
     unsigned va = 0u, vb = 0u;
     auto load_bounds = [&](unsigned k) {
-        const size_t e = wg.x + ((size_t)k + lane) * step, r_ = e < P ? e : P - 1;
+        const size_t e = share + ((size_t)k + lane) * step, r_ = e < P ? e : P - 1;
         va = R[2 * r_]; vb = R[2 * r_ + 1];
         __builtin_amdgcn_s_waitcnt(0x0f70);                        // vmcnt(0), here: else every step that may come this way waits for all that is under way
     };
@@ -873,10 +875,11 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
         }
         in.x0 = (X + base)[e0];
         in.x1 = (X + base)[e1];
-        in.mk = (act16 + base * row_words)[em];
+        if (DENSE) in.mk = (act16 + base * row_words)[em];
         if (k.c == k.a) {
-            const size_t r_ = wg.x + (size_t)k.k * step, j0 = (r_ < P ? r_ : P - 1) * F;
-            if (PEAK) { in.g = (dpooled + 2 * j0)[2u * fe + (peak ? 0u : 1u)]; in.pmax = (pooled + 2 * j0)[2u * fe]; in.arg = (argmax + j0)[fe]; }
+            const size_t r_ = share + (size_t)k.k * step, j0 = (r_ < P ? r_ : P - 1) * F;
+            if (PEAK && DENSE) { in.g = (dpooled + 2 * j0)[2u * fe + (peak ? 0u : 1u)]; in.pmax = (pooled + 2 * j0)[2u * fe]; in.arg = (argmax + j0)[fe]; }
+            else if (PEAK) { in.g = (dpooled + j0)[fe]; in.pmax = (pooled + j0)[fe]; in.arg = (argmax + j0)[fe]; }
             else in.g = (dpooled + j0)[fe];
         }
     };
@@ -906,7 +909,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
         const unsigned long long Z0 = __ballot(in.x0 == 254u);
         const unsigned Z1 = (unsigned)__ballot(in.x1 == 254u);
         // ---- the columns: 32 rows' bits
-        const unsigned v = transpose(lane < left ? in.mk : 0u);
+        const unsigned v = DENSE ? transpose(lane < left ? in.mk : 0u) : 0u;
         if (first) {
             g = now.b > now.a && f < F ? in.g / (float)(now.b - now.a) : 0.0f;
             if (peak) {
@@ -953,7 +956,8 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
             }
             // ---- a region's end
             if (last) {
-                db = __builtin_fmaf(g, (float)open, db);
+                if (now.k & 1u) db_odd = __builtin_fmaf(g, (float)open, db_odd);
+                else db = __builtin_fmaf(g, (float)open, db);
                 open = 0u;
 #pragma unroll
                 for (int t = 0; t < NB; ++t)
@@ -971,7 +975,20 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
     }
     // ---- this wave's quarter of the slab: a filter's two columns side by side, register i's sums in lanes 0-15 and 32-47, register
     // i + 1's in the others. Register i holds letter i & 3 of tap 2 (i >> 2) + h of its block.
-    float* out = slabs + (size_t)wg.x * stride;
+    db += db_odd;
+    float* out = slabs + (size_t)share * stride;
+    if (!DENSE) {                                                  // (a column per filter: this wave's half of its slab as it is)
+#pragma unroll
+        for (int t = 0; t < NB; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const unsigned j = 8u * t + 2u * (i >> 2) + h;
+                if (j < m && f < F) out[(size_t)(4u * j + (i & 3)) * F + f] = sums[t][i];
+            }
+        const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(db), __float_as_uint(db), false, false);
+        if (h == 0u && f < F) out[(size_t)4 * m * F + f] = __uint_as_float(d32[0]) + __uint_as_float(d32[1]);
+        return;
+    }
 #pragma unroll
     for (int t = 0; t < NB; ++t)
 #pragma unroll
@@ -1074,6 +1091,11 @@ inline unsigned counts_grid_x(unsigned mt, unsigned ftiles, size_t N, size_t P)
     const size_t per_group = (P + gx - 1) / gx;
     return (unsigned)((P + per_group - 1) / per_group);
 }
+// Of max pooling it takes small batches of short regions (one chunk each, so that no chunk is walked for nothing); a workgroup has two
+// shares of the regions there. us a call, bit kernel / this: 256 regions of 53 rows x 1440 filters of 24 taps 27 / 22, 171 x 512 17.2 / 15.7,
+// 171 x 64 15.8 / 14.7, 512 x 16 of 8 taps 14.4 / 13.8, 768 of 61 x 256 of 32 taps 26.2 / 22.7, 768 of 37 x 512 of 8 taps 17.0 / 16.9; 128 of 119 rows x 64 16.0 / 16.4, 2048 of 77 rows x 256 of 8 taps 20.8 / 25.7, 20 000 of 60 x 64 50 / 57.
+inline bool counts_takes_max(size_t N, size_t P) { return P <= 768 && N <= 64 * P; }
+inline unsigned counts_max_grid_x(unsigned mt, unsigned ftiles, size_t N, size_t P) { return (counts_grid_x(mt, ftiles, N, P) + 1) / 2; }
 // Max pooling goes through the bit kernel while the regions are short on average (it visits every 64-row chunk of a region to
 // find each filter's winning row; the sparse kernel goes straight to that row).
 inline bool bits_takes_max(size_t N, size_t P) { return N <= 128 * P; }
@@ -1238,14 +1260,19 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
         DBK_LAUNCH_OK();
     }
     // with max+avg pooling the dense half carries the maxima along
-    const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P);
-    const unsigned gxs = PT == DBK_PT_MAX ? (max_bits ? bits_grid_x(mt, ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
+    const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P), max_counts = PT == DBK_PT_MAX && counts_takes_max(N, P);
+    const unsigned gxs = PT == DBK_PT_MAX ? (max_counts ? 2 * counts_max_grid_x(mt, ftiles, N, P) : max_bits ? bits_grid_x(mt, ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
     const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? counts_grid_x(mt, ftiles, N, P) : dense_grid_x(mt, ftiles, P);
     const size_t smem_s = sparse_smem(m), smem_d = mt == 32 ? bits_smem(mt) : dense_smem(mt);
     DBK_CHECK(smem_s <= lds_limit() && smem_d <= lds_limit(), "ValueError: filter length %zu does not fit in LDS", m);
     float* slabs = (float*)dbk::workspace(stride * (gxs + gxd) * sizeof(float), st);
     DBK_CHECK(slabs != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", stride * (gxs + gxd) * sizeof(float), dbk::workspace_error());
-    if (gxs && max_bits) {
+    if (max_counts) {
+        auto kern = mt == 8 ? scanpool_bprop_counts_kernel<DBK_PT_MAX, 8> : mt == 16 ? scanpool_bprop_counts_kernel<DBK_PT_MAX, 16>
+                  : mt == 24 ? scanpool_bprop_counts_kernel<DBK_PT_MAX, 24> : scanpool_bprop_counts_kernel<DBK_PT_MAX, 32>;
+        hipLaunchKernelGGL(kern, dim3(gxs / 2, ftiles), dim3(256), 0, st, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, dpooled,
+                           (const unsigned long long*)nullptr, slabs, stride);
+    } else if (gxs && max_bits) {
         auto kern = mt == 8 ? scanpool_bprop_bits_kernel<8> : mt == 16 ? scanpool_bprop_bits_kernel<16>
                   : mt == 24 ? scanpool_bprop_bits_kernel<24> : scanpool_bprop_bits_kernel<32>;
         const size_t smem_b = bits_smem(mt);
@@ -1366,7 +1393,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 32 ? 
     const unsigned gi = multi_locate(a, wg);
     const dbk::scan_group& j = a.g[gi];
     if (j.ptype == DBK_PT_MAX) {
-        if (a.wide[gi])
+        if (a.wide[gi] == 2u)
+            scanpool_bprop_counts_body<DBK_PT_MAX, MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, nullptr, j.slabs, j.slab_stride);
+        else if (a.wide[gi])
             scanpool_bprop_bits_body<MT>(wg, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.dpooled, j.slabs, j.slab_stride);
         else if (threadIdx.x < 64)
             scanpool_bprop_sparse_body<DBK_PT_MAX, MT>(wg, a.m, j.F, j.X, a.N, a.P, j.pooled, j.argmax, j.dpooled, j.slabs, j.slab_stride);
@@ -1448,18 +1477,19 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
     for (unsigned i = 0; i < n; ++i) {
         a.ftiles[i] = dbk::divup(g[i].F, FT);
         // as the group's own launch would choose: the counting kernel, for max pooling the bit kernel or, over long regions, the sparse one
-        a.wide[i] = g[i].ptype != DBK_PT_MAX || bits_takes_max(N, P);
-        a.gx[i] = g[i].ptype != DBK_PT_MAX ? counts_grid_x(mt, a.ftiles[i], N, P) : a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
+        a.wide[i] = g[i].ptype != DBK_PT_MAX ? 1u : counts_takes_max(N, P) ? 2u : bits_takes_max(N, P) ? 1u : 0u;
+        a.gx[i] = g[i].ptype != DBK_PT_MAX ? counts_grid_x(mt, a.ftiles[i], N, P) : a.wide[i] == 2u ? counts_max_grid_x(mt, a.ftiles[i], N, P)
+                : a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
         a.first[i + 1] = a.first[i] + a.gx[i] * a.ftiles[i];
         g[i].slab_stride = 4 * m * (size_t)g[i].F + g[i].F;
-        g[i].nslab = a.gx[i];
-        total += g[i].slab_stride * a.gx[i];
+        g[i].nslab = a.wide[i] == 2u ? 2 * a.gx[i] : a.gx[i];
+        total += g[i].slab_stride * g[i].nslab;
     }
     float* slabs = (float*)dbk::workspace(total * sizeof(float), st);
     DBK_CHECK(slabs != nullptr, "MemoryError: could not allocate %zu bytes of scratch (%s)", total * sizeof(float), dbk::workspace_error());
     for (unsigned i = 0; i < n; ++i) {
         g[i].slabs = slabs;
-        slabs += g[i].slab_stride * a.gx[i];
+        slabs += g[i].slab_stride * g[i].nslab;
         a.g[i] = g[i];
     }
     const size_t ss = sparse_smem(m), sd = bits_smem(mt);

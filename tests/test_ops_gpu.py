@@ -703,15 +703,16 @@ def test_corr1ord_bprop_X_in_rounds(ks, n, m, F):
     assert ((dX - ref).abs().max() / ref.abs().max()).item() < 1e-5
 
 
-@pytest.mark.parametrize("ptype", ["avg", "all"])
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("lengths,m,F", [((1, 63, 64, 65, 0, 127, 128, 129, 300), 8, 16), ((64, 0, 2, 192, 31, 33), 9, 1), ((40,) * 70, 16, 17),
                                          ((53, 200, 64), 24, 65), ((1, 0, 700, 5) * 3, 25, 48), ((100,) * 9, 32, 130), ((0, 2, 1) * 17000, 8, 16),
-                                         ((5,), 32, 16), ((0, 0), 7, 33)])
+                                         ((5,), 32, 16), ((0, 0), 7, 33), ((1, 0, 30, 41) * 192, 24, 130), ((20,) * 769, 24, 16)])
 def test_scanpool_bprop_counts_are_exact(ks, ptype, lengths, m, F):
     """With masks the gradient is counts times one number per (region, filter). With integers for those numbers (an average's gradient
     a multiple of its region's length) every sum is a whole number of quarters below 2^22, exact in float32 whatever the order: the
     result is the float64 one, bit for bit. Regions around the 64-row chunks, more of them than a wave keeps bounds of (64),
-    every tap tier, filters around the 16 of a wave and the 64 of a tile, N and code 254, a last region at the end of the text."""
+    every tap tier, filters around the 16 of a wave and the 64 of a tile, N and code 254, a last region at the end of the text. Maxima
+    alone are counted that way up to 768 short regions."""
     rng = np.random.default_rng(7 * m + F)
     n = np.array(lengths); pad = m - 1
     ends = np.cumsum(n + pad)
@@ -723,19 +724,25 @@ def test_scanpool_bprop_counts_are_exact(ks, ptype, lengths, m, F):
     Wd, bd, Xd, Rd = dev(W), dev(b), dev(X), dev(R)
     act = ks.activity_words(Xd, Wd)
     act.fill_(-1)
-    P, I = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, want_argmax=True, act=act)
+    if ptype == "max":
+        act.fill_(0)
+        P, I = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, want_argmax=True)
+    else:
+        P, I = ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, want_argmax=True, act=act)
     davg = rng.integers(-3, 4, (len(n), F)); dmax = rng.integers(-3, 4, (len(n), F))
     dP = (davg * n[:, None]).astype(np.float32)
     if ptype == "all":
         dP = np.stack([dmax, dP], 2).reshape(len(n), 2 * F).astype(np.float32)
+    elif ptype == "max":
+        dP = dmax.astype(np.float32)
     dW, db = dev(np.full(W.shape, 7.0, np.float32)), dev(np.full((1, F), 7.0, np.float32))
-    ks.scanpool_bprop(Wd, bd, Xd, Rd, ptype, P, I, dev(dP), dW, db, overwrite=True, act=act)
+    ks.scanpool_bprop(Wd, bd, Xd, Rd, ptype, P, I, dev(dP), dW, db, overwrite=True, act=None if ptype == "max" else act)
     region = np.full(N, -1); region[np.concatenate([np.arange(a, e) for a, e in R.astype(int)])] = np.repeat(np.arange(len(n)), n)
     words = host(act).view(np.uint64).reshape(N, -1)
     G = ((words[:, np.arange(F) // 64] >> (np.arange(F) % 64).astype(np.uint64)) & np.uint64(1)).astype(np.float64)
     G *= np.where(region[:, None] >= 0, davg[np.maximum(region, 0)], 0)
-    if ptype == "all":
-        won = host(P).reshape(len(n), F, 2)[:, :, 0] > 0
+    if ptype != "avg":
+        won = (host(P) if ptype == "max" else host(P).reshape(len(n), F, 2)[:, :, 0]) > 0
         np.add.at(G, (host(I).astype(np.uint32)[won] // F, np.nonzero(won)[1]), dmax[won])
     letters = np.full((256, 4), 0.25); letters[:4] = np.eye(4); letters[254] = 0.0
     rows = N - m + 1
