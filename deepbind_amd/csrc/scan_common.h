@@ -9,6 +9,10 @@ constexpr int FT = 64;        // filters per tile = lanes per wave
 constexpr int NL = 6;         // letters in the LDS table
 constexpr int PSUB = 16;      // positions accumulated in registers at a time
 
+// Who takes the filters of a tile in a bulk call: the bulk kernel itself (below TILE_LEFT), or the launch behind it, finite weights on
+// the matrix cores and infinite, undefined or extreme ones from the letter table.
+constexpr unsigned TILE_BULK = 0, TILE_LEFT = 2, TILE_NOT_FINITE = 3;
+
 __device__ __forceinline__ unsigned letter_of(unsigned code)
 {
     return code < 4u ? code : (code == 254u ? 5u : 4u);

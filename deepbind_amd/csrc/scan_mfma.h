@@ -72,7 +72,9 @@ struct mfma_block {
     bool valid;
 };
 
-template <int PT, bool WANT_ARGMAX, bool ACT, int KS>
+// ROWS_OPEN: averages add relu(z + b) row by row instead of max(z, -b) and then b times the number of rows, which in a region of few
+// rows rounds in the size of 16 b.
+template <int PT, bool WANT_ARGMAX, bool ACT, int KS, bool ROWS_OPEN = false>
 __device__ __forceinline__ void scanpool_fprop_mfma_body(const wg_t wg, const float* __restrict__ W, const float* __restrict__ bias,
                                                          unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
                                                          const uint32_t* __restrict__ R, size_t P,
@@ -223,9 +225,9 @@ __device__ __forceinline__ void scanpool_fprop_mfma_body(const wg_t wg, const fl
             if (bm > mz) { mz = bm; xi = (k.c0 - k.a) + rg + (bi & 3u) + 8u * (bi >> 2); }
         }
         if (PT != DBK_PT_MAX) {
-            float part = 16.0f * bf;
+            float part = ROWS_OPEN ? 0.0f : 16.0f * bf;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) part += plain_max(z[i], nb);
+            for (int i = 0; i < 16; ++i) part += ROWS_OPEN ? plain_max(z[i], nb) + bf : plain_max(z[i], nb);
             sum += part;
         }
         if (rows <= MFMA_ROWS) {

@@ -4,7 +4,7 @@
 // filter) and walks whole regions, each wave scanning 16 positions at a time in registers and
 // folding them straight into the region's running max / argmax / sum. This path takes any filter
 // length that fits in LDS, any region table and every letter code; the kernel of scanpool_digits.hip is the fast path
-// for bulk scoring and leaves weights it cannot express to this one.
+// for bulk scoring and leaves weights it cannot express to a launch of this file behind it.
 //
 // Backward: the max part is 1-sparse (one position per region and filter), the average part is
 // dense and needs the forward recomputed for the ReLU mask. Both accumulate into per-wave private
@@ -17,6 +17,7 @@
 // poolrgn_bprop.cuh:45-127, corr1ord_bprop.cuh:91-137.
 #include "dbk_common.h"
 #include "scan_common.h"
+#include <algorithm>
 
 namespace dbk_scanpool_general {
 
@@ -49,12 +50,9 @@ __device__ __forceinline__ void scanpool_fprop_body(const wg_t wg, const float* 
                                                     unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
                                                     const uint32_t* __restrict__ R, size_t P,
                                                     float* __restrict__ pooled, uint32_t* __restrict__ argmax,
-                                                    const unsigned* __restrict__ run_if_flag,
                                                     unsigned long long* __restrict__ act)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    // when given (behind the bulk kernel: one flag per 32 filters), only the tiles that one of their two flags asks for
-    if (run_if_flag && (run_if_flag[2 * wg.y] | run_if_flag[2 * wg.y + 1]) == 0u) return;
     const unsigned nw = blockDim.x >> 6;
     const unsigned chunk = nw * XCH_SUBS * PSUB;
     // up to 16 taps: the lane's filter weights live in register planes and the scan needs no table in LDS
@@ -155,10 +153,9 @@ __global__ __launch_bounds__(256) void scanpool_fprop_kernel(const float* __rest
                                                              unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
                                                              const uint32_t* __restrict__ R, size_t P,
                                                              float* __restrict__ pooled, uint32_t* __restrict__ argmax,
-                                                             const unsigned* __restrict__ run_if_flag,
                                                              unsigned long long* __restrict__ act)
 {
-    scanpool_fprop_body<PT, WANT_ARGMAX, MT>(this_wg(), W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act);
+    scanpool_fprop_body<PT, WANT_ARGMAX, MT>(this_wg(), W, bias, m, F, X, N, R, P, pooled, argmax, act);
 }
 
 // The same forward pass with four filters per lane, for batches of many regions (filters of 17-24 taps).
@@ -287,6 +284,44 @@ __global__ __launch_bounds__(256) void scanpool_fprop_wide_kernel(const float* _
 #include "scan_mfma.h"
 
 namespace dbk_scanpool_general {
+
+// What the bulk kernel (scanpool_digits.hip) leaves out: it writes a flag per 32 filters, and this launch, behind it on the
+// stream, takes the 64-filter tiles of which one asks for it: finite weights on the matrix cores, in three bf16 pieces whatever
+// their sizes; infinite and undefined ones, which a product would spread over windows that do not hold them, one by one from the
+// letter table. The workgroups are dealt over the tiles that are left, not over all, so that a few of many have the whole GPU.
+// Where nothing is left the launch costs 4-5 us. Measured, 20 000 x 500 letters x 512 filters, ms with nothing, one tile of eight and all
+// tiles left: max pooling of 24 taps 0.98, 1.21, 2.36, of 8 taps 0.54, 0.66, 1.24, of 32 taps 1.11, 1.39, -; average of 24 taps 1.32, 1.53, 2.31.
+// (One lookup per tap from the letter table, by a grid of all tiles of which most workgroups left at once: 24 taps 7.4 and 9.2, 8 taps 2.8 and 4.1.)
+// (the form with its table in LDS: the register planes of 16 taps are pinned beyond the registers of three waves per SIMD)
+constexpr int left_lookup_taps(int ks) { return ks == 8 ? 32 : 24; }
+template <int PT, bool WANT_ARGMAX, int KS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void scanpool_fprop_left_kernel(const float* __restrict__ W, const float* __restrict__ bias,
+                                                                  unsigned m, unsigned F, const uint8_t* __restrict__ X, size_t N,
+                                                                  const uint32_t* __restrict__ R, size_t P,
+                                                                  float* __restrict__ pooled, uint32_t* __restrict__ argmax,
+                                                                  const unsigned* __restrict__ flags, unsigned ftiles)
+{
+    const unsigned lane = threadIdx.x & 63u;
+    auto asked = [&](unsigned t0) -> unsigned long long {
+        const unsigned t = t0 + lane;
+        return __ballot(t < ftiles && (flags[2 * t] >= TILE_LEFT || flags[2 * t + 1] >= TILE_LEFT));
+    };
+    unsigned left = 0u;
+    for (unsigned t0 = 0; t0 < ftiles; t0 += 64u) left += (unsigned)__popcll(asked(t0));
+    if (left == 0u) return;
+    const unsigned gx = gridDim.x / left;                         // workgroups per tile (the grid has no fewer than tiles)
+    if (blockIdx.x >= left * gx) return;
+    unsigned t0 = 0u, nth = blockIdx.x % left;                     // the nth of the tiles that are left
+    unsigned long long who = asked(0u);
+    while ((unsigned)__popcll(who) <= nth) { nth -= (unsigned)__popcll(who); t0 += 64u; who = asked(t0); }
+    for (; nth != 0u; --nth) who &= who - 1ull;
+    const unsigned tile = t0 + (unsigned)__builtin_ctzll(who);
+    const wg_t wg = {blockIdx.x / left, tile, gx, ftiles};
+    if (flags[2 * tile] == TILE_NOT_FINITE || flags[2 * tile + 1] == TILE_NOT_FINITE)
+        scanpool_fprop_body<PT, WANT_ARGMAX, left_lookup_taps(KS)>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);
+    else
+        scanpool_fprop_mfma_body<PT, WANT_ARGMAX, false, KS, true>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);
+}
 
 // ---------------------------------------------------------------------------------------------
 // backward
@@ -1111,16 +1146,16 @@ inline size_t dense_smem(unsigned mt)
 template <int PT, int MT>
 int launch_fprop_mt(hipStream_t st, unsigned gx, unsigned ftiles, unsigned nw, size_t smem, const float* W, const float* bias, size_t m,
                      size_t F, const uint8_t* X, size_t N, const uint32_t* R, size_t P, float* pooled, uint32_t* argmax,
-                     const unsigned* run_if_flag, unsigned long long* act)
+                     unsigned long long* act)
 {
     if (argmax) {
         auto kern = scanpool_fprop_kernel<PT, true, MT>;
         DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-        hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(nw * 64), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, run_if_flag, act);
+        hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(nw * 64), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, act);
     } else {
         auto kern = scanpool_fprop_kernel<PT, false, MT>;
         DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-        hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(nw * 64), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, run_if_flag, act);
+        hipLaunchKernelGGL(kern, dim3(gx, ftiles), dim3(nw * 64), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, act);
     }
     return 0;
 }
@@ -1174,7 +1209,7 @@ int launch_fprop_mfma(hipStream_t st, unsigned ftiles, const float* W, const flo
 
 template <int PT>
 int launch_fprop_pt(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
-                    const uint32_t* R, size_t P, float* pooled, uint32_t* argmax, const unsigned* run_if_flag, unsigned long long* act)
+                    const uint32_t* R, size_t P, float* pooled, uint32_t* argmax, unsigned long long* act)
 {
     const unsigned nw = 4;
     const unsigned mt = m <= 8 ? 8 : (m <= 16 ? 16 : (m <= 24 ? 24 : (m <= 32 ? 32 : 0)));    // 0: any-length kernel
@@ -1182,18 +1217,43 @@ int launch_fprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
     DBK_CHECK(smem <= lds_limit(), "ValueError: filter length %zu needs %zu bytes of LDS (limit %zu)", m, smem, lds_limit());
     unsigned ftiles = dbk::divup(F, FT);
     DBK_CHECK(ftiles <= 65535u, "ValueError: too many filters (%zu) for one launch", F);
-    if (!run_if_flag && mfma_pays(m, ftiles, P)) return launch_fprop_mfma<PT>(st, ftiles, W, bias, m, F, X, N, R, P, pooled, argmax, act);
+    if (mfma_pays(m, ftiles, P)) return launch_fprop_mfma<PT>(st, ftiles, W, bias, m, F, X, N, R, P, pooled, argmax, act);
     const unsigned gx = fprop_grid_x(mt, ftiles, P);
     int rc = 0;
     switch (mt) {
-    case 8:  rc = launch_fprop_mt<PT, 8>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act); break;
-    case 16: rc = launch_fprop_mt<PT, 16>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act); break;
-    case 24: rc = launch_fprop_mt<PT, 24>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act); break;
-    case 32: rc = launch_fprop_mt<PT, 32>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act); break;
-    default: rc = launch_fprop_mt<PT, 0>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act); break;
+    case 8:  rc = launch_fprop_mt<PT, 8>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, act); break;
+    case 16: rc = launch_fprop_mt<PT, 16>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, act); break;
+    case 24: rc = launch_fprop_mt<PT, 24>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, act); break;
+    case 32: rc = launch_fprop_mt<PT, 32>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, act); break;
+    default: rc = launch_fprop_mt<PT, 0>(st, gx, ftiles, nw, smem, W, bias, m, F, X, N, R, P, pooled, argmax, act); break;
     }
     if (rc) return rc;
     DBK_LAUNCH_OK();
+}
+
+template <int PT, int KS>
+int launch_fprop_left_ks(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N, const uint32_t* R,
+                         size_t P, float* pooled, uint32_t* argmax, const unsigned* flags)
+{
+    const unsigned ftiles = dbk::divup(F, FT);
+    const size_t smem = std::max(MFMA_SMEM, fprop_smem(left_lookup_taps(KS), m)), items = ftiles * P;
+    const unsigned grid = std::max(ftiles, items < 768 ? (unsigned)items : 768u);   // three workgroups per CU are resident
+    auto kern = argmax && PT != DBK_PT_AVG ? scanpool_fprop_left_kernel<PT, PT != DBK_PT_AVG, KS> : scanpool_fprop_left_kernel<PT, false, KS>;
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, flags, ftiles);
+    DBK_LAUNCH_OK();
+}
+
+template <int PT>
+int launch_fprop_left(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N, const uint32_t* R,
+                      size_t P, float* pooled, uint32_t* argmax, const unsigned* flags)
+{
+    switch ((mfma_ksteps(m) + 1) / 2) {
+    case 1:  return launch_fprop_left_ks<PT, 2>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
+    case 2:  return launch_fprop_left_ks<PT, 4>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
+    case 3:  return launch_fprop_left_ks<PT, 6>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
+    default: return launch_fprop_left_ks<PT, 8>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
+    }
 }
 
 template <int PT, int MT>
@@ -1327,13 +1387,23 @@ int fprop_wide(hipStream_t st, const float* W, const float* bias, size_t m, size
 }
 
 int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
-          const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, const unsigned* run_if_flag,
-          unsigned long long* act)
+          const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, unsigned long long* act)
 {
     switch (ptype) {
-    case DBK_PT_MAX: return launch_fprop_pt<DBK_PT_MAX>(st, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act);
-    case DBK_PT_AVG: return launch_fprop_pt<DBK_PT_AVG>(st, W, bias, m, F, X, N, R, P, pooled, nullptr, run_if_flag, act);
-    default:         return launch_fprop_pt<DBK_PT_ALL>(st, W, bias, m, F, X, N, R, P, pooled, argmax, run_if_flag, act);
+    case DBK_PT_MAX: return launch_fprop_pt<DBK_PT_MAX>(st, W, bias, m, F, X, N, R, P, pooled, argmax, act);
+    case DBK_PT_AVG: return launch_fprop_pt<DBK_PT_AVG>(st, W, bias, m, F, X, N, R, P, pooled, nullptr, act);
+    default:         return launch_fprop_pt<DBK_PT_ALL>(st, W, bias, m, F, X, N, R, P, pooled, argmax, act);
+    }
+}
+
+// The tiles that the bulk kernel left out (flags: one per 32 filters), for filters of up to 32 taps.
+int fprop_left(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
+               const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, const unsigned* flags)
+{
+    switch (ptype) {
+    case DBK_PT_MAX: return launch_fprop_left<DBK_PT_MAX>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
+    case DBK_PT_AVG: return launch_fprop_left<DBK_PT_AVG>(st, W, bias, m, F, X, N, R, P, pooled, nullptr, flags);
+    default:         return launch_fprop_left<DBK_PT_ALL>(st, W, bias, m, F, X, N, R, P, pooled, argmax, flags);
     }
 }
 
@@ -1378,11 +1448,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MT == 24 ? 
         }
     }
     if (j.ptype == DBK_PT_MAX)
-        scanpool_fprop_body<DBK_PT_MAX, true, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, nullptr, nullptr);
+        scanpool_fprop_body<DBK_PT_MAX, true, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, nullptr);
     else if (j.ptype == DBK_PT_ALL)
-        scanpool_fprop_body<DBK_PT_ALL, true, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, nullptr, j.act);
+        scanpool_fprop_body<DBK_PT_ALL, true, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, j.argmax, j.act);
     else
-        scanpool_fprop_body<DBK_PT_AVG, false, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, nullptr, nullptr, j.act);
+        scanpool_fprop_body<DBK_PT_AVG, false, MT>(wg, j.W, j.bias, a.m, j.F, j.X, a.N, a.R, a.P, j.pooled, nullptr, j.act);
 }
 
 // The counting kernel; for max pooling the bit kernel, over long regions the one-wave sparse kernel in the first wave of the
@@ -1525,7 +1595,7 @@ int dbk_scanpool_fprop_general(dbk_stream_t stream, const float* W, const float*
               "ValueError: %zu rows x %zu filters overflow the 32-bit argmax index; score in smaller batches or without argmax", N, nfilter);
     if (nfilter == 0 || nregion == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(W && bias && X && regions && pooled, "ValueError: null pointer argument");
-    return dbk_scanpool_general::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax, nullptr,
+    return dbk_scanpool_general::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax,
                                        reinterpret_cast<unsigned long long*>(act));
 }
 
@@ -1578,7 +1648,7 @@ int dbk_scanpool_fprop(dbk_stream_t stream, const float* W, const float* bias, s
         int rc = dbk_scanpool_digits::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax);
         if (rc >= 0) return rc;
     }
-    return dbk_scanpool_general::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax, nullptr,
+    return dbk_scanpool_general::fprop(dbk::as_stream(stream), W, bias, m, nfilter, X, N, regions, nregion, ptype, pooled, argmax,
                                        reinterpret_cast<unsigned long long*>(act));
 }
 

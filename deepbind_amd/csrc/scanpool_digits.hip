@@ -17,8 +17,8 @@
 // A weight far below zero only has to keep its window closed: every window's rectified value is at most
 // T = sum over the taps of the largest weight (if positive) + the bias, so weights below -8 T are raised to -8 T (a
 // window of one such "mean of four" is still at most -2 T + T). Filters that fixed point does not express well (an
-// infinite or undefined weight, one positive weight more than 64 times the next) are left to the general kernel,
-// which is launched behind this one and does nothing where no tile of filters asks for it.
+// infinite or undefined weight, one positive weight more than 64 times the next) are left to a launch behind this one
+// (scanpool_fprop_left_kernel), which does nothing where no tile of filters asks for it.
 //
 // Mapping: a workgroup of 16 waves (one per CU) owns 32 filters, whose digits stay in its registers (24 taps: 9
 // instructions' operands, 54 registers a lane). A wave takes a region at a time from the workgroup's counter and walks it
@@ -43,14 +43,16 @@
 #include <mutex>
 
 namespace dbk_scanpool_general {
-int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
-          const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, const unsigned* run_if_flag,
-          unsigned long long* act);
+int fprop_left(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
+               const uint32_t* R, size_t P, int ptype, float* pooled, uint32_t* argmax, const unsigned* flags);
 }
 
 namespace dbk_scanpool_digits {
 
 using dbk_mfma::f32x16_t;
+using dbk_scan::TILE_BULK;
+using dbk_scan::TILE_LEFT;
+using dbk_scan::TILE_NOT_FINITE;
 
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 
@@ -68,7 +70,7 @@ constexpr float CLOSED = -3.0e38f;            // the value of a row outside the 
 __device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
 
 // ---------------------------------------------------------------------------------------------- the weights' digits
-// What a call keeps in its scratch, per tile of 32 filters: a flag (not expressible: the general kernel's), the filters'
+// What a call keeps in its scratch, per tile of 32 filters: a flag (TILE_BULK, or who takes it instead), the filters'
 // exponents, the digits, [8-tap block][digit][filter][24 bytes], and, to find a maximum's place, NTOP digits per weight in
 // units of the filter's own (no power of two) with what the scan has to know of them.
 struct digit_facts {
@@ -118,9 +120,9 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
 {
     __shared__ float red[6][8][FTILE];                            // sums and maxima of the eight threads of a filter
     __shared__ unsigned char dig[TB * (NDIGIT + NTOP) * SLOT_BYTES];
-    __shared__ unsigned bad_tile;
+    __shared__ unsigned worst;                                    // of the tile's filters
     const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
-    if (threadIdx.x == 0) bad_tile = 0u;
+    if (threadIdx.x == 0) worst = TILE_BULK;
     float w[TB][4];
 #pragma unroll
     for (int t = 0; t < TB; ++t)
@@ -132,14 +134,16 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
     const float b = f < F ? bias[f] : 0.0f;
     float open = 0.0f, top = 0.0f, second = 0.0f, low = 0.0f;     // sum of the taps' best, the two largest weights, the most negative one
     float size = 0.0f;                                            // sum of the taps' largest magnitudes
-    bool bad = (__float_as_uint(b) & 0x7fffffffu) >= 0x71000000u;     // (the file is compiled without NaN: test the bits)
+    const unsigned bias_bits = __float_as_uint(b) & 0x7fffffffu;      // (the file is compiled without NaN: test the bits)
+    bool finite = bias_bits < 0x7f800000u, closing = false;           // closing: minus infinity among the weights
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         float best = 0.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const unsigned bits = __float_as_uint(w[t][c]) & 0x7fffffffu;
-            bad |= bits > 0x7f800000u || (bits == 0x7f800000u && w[t][c] > 0.0f);
+            finite &= bits < 0x7f800000u || __float_as_uint(w[t][c]) == 0xff800000u;
+            closing |= bits == 0x7f800000u;
             best = fmaxf(best, w[t][c]);
             second = fmaxf(second, fminf(top, w[t][c]));
             top = fmaxf(top, w[t][c]);
@@ -147,10 +151,10 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         }
         open += best;
     }
-    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = second; red[3][g][fl] = low; red[4][g][fl] = bad ? 1.0f : 0.0f;
+    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = second; red[3][g][fl] = low; red[4][g][fl] = (finite ? 0.0f : 1.0f) + (closing ? 64.0f : 0.0f);
     __syncthreads();
     open = fmaxf(b, 0.0f); top = 0.0f; second = 0.0f; low = 0.0f;
-    float nbad = 0.0f;
+    float odd = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         open += red[0][k][fl];
@@ -158,15 +162,17 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         second = fmaxf(fmaxf(second, sk), fminf(top, tk));
         top = fmaxf(top, tk);
         low = fmaxf(low, red[3][k][fl]);
-        nbad += red[4][k][fl];
+        odd += red[4][k][fl];
     }
     const float floor_ = -8.0f * open;                            // nothing below keeps a window open
     const float big = fmaxf(top, fminf(low, -floor_));
     second = fmaxf(second, b);
     int e = 0;
-    bad = nbad > 0.0f || (second > 0.0f && top > 64.0f * second) || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-25f);
+    // sizes near the type's ends, where a weight's bf16 pieces or a sum may leave it, go with the infinite and undefined ones
+    const bool far = ((unsigned)odd & 63u) != 0u || bias_bits >= 0x71000000u || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-32f);
+    const bool bad = far || (second > 0.0f && top > 64.0f * second) || (big != 0.0f && big < 1.0e-25f);
     if (!bad && big != 0.0f) e = (int)((__float_as_uint(big) >> 23) & 0xffu) - 127;
-    if (bad) bad_tile = 1u;                                       // (every writer writes the same)
+    if (bad) atomicMax(&worst, far || odd >= 64.0f ? TILE_NOT_FINITE : TILE_LEFT);
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         float z = 0.0f;
@@ -219,7 +225,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         k.whole = 29 - se;                                        // size < 2^(se + 1)
         out.facts[blockIdx.x * FTILE + fl] = k;
     }
-    if (threadIdx.x == 0) out.flags[blockIdx.x] = bad_tile;
+    if (threadIdx.x == 0) out.flags[blockIdx.x] = worst;
 }
 
 // ---------------------------------------------------------------------------------------------- letters
@@ -381,6 +387,12 @@ __device__ __forceinline__ void products(f32x16_t& acc, const uint4& a0, const u
     }
 }
 
+// Whether the launch behind this one takes a tile: it takes tiles of 64 filters, that is pairs.
+__device__ __forceinline__ bool left_out(const unsigned* __restrict__ flags, unsigned tile)
+{
+    return flags[tile & ~1u] >= TILE_LEFT || flags[tile | 1u] >= TILE_LEFT;
+}
+
 // ---------------------------------------------------------------------------------------------- the scan
 template <int PT, bool WANT_ARGMAX, int TB>
 __global__ __launch_bounds__(NWAVE * 64) __attribute__((amdgpu_waves_per_eu(NWAVE / 4, NWAVE / 4)))
@@ -390,7 +402,7 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NI = product_count<TB>::N;
     const unsigned tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
-    if (D.flags[tile] != 0u) return;                              // the general kernel takes these filters
+    if (left_out(D.flags, tile)) return;
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
     unsigned* counter = reinterpret_cast<unsigned*>(smem);
@@ -632,8 +644,7 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
     constexpr unsigned TAPS = 8u * TB, TILE_DIGITS = TB * NDIGIT * SLOT_BYTES;
     const unsigned tile = 2u * (blockIdx.x / nsplit), split = blockIdx.x % nsplit;
     const bool two = tile + 1u < ntile;                           // (an odd last tile is scanned beside nothing)
-    // (a tile that is the general kernel's is scanned along with its neighbour; the general kernel writes over it)
-    if (D.flags[tile] != 0u && (!two || D.flags[tile + 1] != 0u)) return;
+    if (left_out(D.flags, tile)) return;
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
     unsigned* counter = reinterpret_cast<unsigned*>(smem);
@@ -864,8 +875,8 @@ bool half_the_products(size_t m, size_t F, size_t N, size_t P, int ptype, bool f
 }
 
 // Whether a call of this size goes to the digit kernel when the choice is left to the library, in rows x 64-filter tiles
-// (what the general path's time follows). The smallest call takes three launches (digits, scan, the general kernel's look
-// at the flags), 16-18 us. Measured break-even without argmax, 25 to 400 letters, 16 to 384 filters: up to 8 taps, where
+// (what the general path's time follows). The smallest call takes three launches (digits, scan, the look at the
+// flags), 16-18 us. Measured break-even without argmax, 25 to 400 letters, 16 to 384 filters: up to 8 taps, where
 // the general path has no matrix-core kernel, 0.15-0.25 M (at 0.5 M 17 us against 36, at 4 M 47 against 257); 9 to 32 taps
 // 0.45-0.55 M (24 taps, 101 letters x 64 filters: 20 us against 19 at 0.5 M, 27 / 33 at 1 M, 72 / 129 at 4 M; 32 taps
 // 26 / 26, 37 / 46, 107 / 171). With an argmax (a training step's forward pass) it lies at 0.9 M rows x tiles; such calls
@@ -877,7 +888,7 @@ bool takes(size_t m, size_t F, size_t N, size_t P, bool argmax)
     return (double)N * dbk::divup(F, 2 * FTILE) >= (m > 8 ? 0.6e6 : 0.25e6);
 }
 
-// A call's scratch: one flag per 32 filters (an even number of them: the general kernel looks at pairs), then the digits of
+// A call's scratch: one flag per 32 filters (an even number of them: the launch behind looks at pairs), then the digits of
 // up to PASS_TILES tiles; more filters than that are taken in several passes.
 constexpr unsigned PASS_TILES = 1024;
 inline size_t flag_bytes(size_t F) { return (2 * (size_t)dbk::divup(F, 2 * FTILE) * sizeof(unsigned) + 255) & ~(size_t)255; }
@@ -918,9 +929,8 @@ int fprop_impl(hipStream_t st, const float* W, const float* bias, size_t m, size
         }
         if (rc != 0) return rc;
     }
-    // filters whose weights the digits do not express: the general kernel, gated on the tiles' flags so that no host
-    // synchronisation is needed
-    return dbk_scanpool_general::fprop(st, W, bias, m, F, X, N, R, P, ptype, pooled, argmax, flags, nullptr);
+    // filters whose weights the digits do not express, by the tiles' flags, so that no host synchronisation is needed
+    return dbk_scanpool_general::fprop_left(st, W, bias, m, F, X, N, R, P, ptype, pooled, argmax, flags);
 }
 
 int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,

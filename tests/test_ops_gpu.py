@@ -1366,6 +1366,109 @@ def test_bulk_scan_leaves_weights_it_cannot_express_to_the_general_kernel(ks, pt
         assert (host(I) == host(Ig)).mean() > 0.99
 
 
+def _closed_tiles(W, tiles, weight):
+    """One filter of each of the given tiles of 32 gets a weight beyond all others at one letter of its middle tap."""
+    for t in tiles:
+        W[4 * (W.shape[0] // 8) + 2, min(32 * t + 7, W.shape[1] - 1)] = weight
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("tiles", [(0,), (1,), (0, 1), (4,), (1, 2, 4), (0, 1, 2, 3, 4)])
+@pytest.mark.parametrize("m", [1, 8, 16, 20, 24])
+def test_bulk_scan_beside_tiles_that_are_left_out(ks, m, tiles, ptype):
+    """Tiles of 32 filters that the digits do not express, first or second of their pair of tiles, both, the odd last one, all of
+    them: the launch behind the bulk kernel writes them, and only them and their neighbours."""
+    F = 32 * 4 + 9
+    rng, W, b, X, R = _bulk_case(500 + m, [200, 1, 33, 224, 500, 64, 110], m, F)
+    plain = W.copy()
+    _closed_tiles(W, tiles, 3e6)
+    want = ptype != "avg"
+    P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=want, path="kmer")
+    assert np.array_equal(host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")[0]), host(P))
+    A, Pr, Ir = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
+    _within_rounding(host(P), Pr, W, b, ptype)
+    if want:
+        moved = host(I) != Ir
+        # (two windows whose float32 sums of m + 1 terms may tie)
+        tie = (m + 1) * 2.0 ** -23 * (np.abs(W.astype(np.float64)).reshape(m, 4, F).max(axis=1).sum(axis=0) + np.abs(b.ravel()))
+        assert moved[:, np.abs(W).max(axis=0) < 1e6].mean() < 0.01
+        assert np.all(np.abs(A.ravel()[host(I)[moved]] - A.ravel()[Ir[moved]]) <= np.broadcast_to(tie, moved.shape)[moved])
+    # the tiles of 64 filters in which nothing is left out keep their bits
+    Pp, _ = ks.scanpool_fprop(dev(plain), dev(b), dev(X), dev(R), ptype, path="kmer")
+    k = 2 if ptype == "all" else 1
+    for t in range(3):
+        if t not in {u // 2 for u in tiles}:
+            assert np.array_equal(host(P)[:, 64 * k * t:64 * k * (t + 1)], host(Pp)[:, 64 * k * t:64 * k * (t + 1)])
+
+
+@pytest.mark.parametrize("weight", [3e6, np.inf, np.nan])
+def test_bulk_scan_of_25_to_32_taps_beside_tiles_that_are_left_out(ks, weight):
+    m, F = 32, 64 * 320 + 40
+    rng, W, b, X, R = _bulk_case(61, [300, 1, 33, 224, 500, 64, 900], m, F, odd_codes=False)
+    tiles = (0, 5, 320, 640, 641)
+    _closed_tiles(W, tiles, weight)
+    Wd, bd, Xd, Rd = dev(W), dev(b), dev(X), dev(R)
+    for ptype in ("max", "avg", "all"):
+        P, Pg = [host(ks.scanpool_fprop(Wd, bd, Xd, Rd, ptype, path=p)[0]) for p in ("auto", "general")]
+        pick = np.sort(np.concatenate([[32 * t + min(7, F - 1 - 32 * t) for t in tiles], rng.choice(F, 60, replace=False)]))
+        cols = pick if ptype != "all" else np.stack([2 * pick, 2 * pick + 1], axis=1).ravel()
+        if np.isfinite(weight):
+            _within_rounding(P[:, cols], _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R, ptype)[1], W[:, pick], b[:, pick], ptype)
+        else:
+            # (the general path takes this call in products, where an undefined weight reaches windows that do not hold it)
+            ok = [c for c, f in zip(cols, pick.repeat(len(cols) // len(pick))) if np.isfinite(W[:, f]).all()]
+            assert_close(P[:, ok], Pg[:, ok], ACT, "filters beside the tiles left out")
+            if ptype == "max":                                           # (the first region's 300 rows hold the letter)
+                f = 32 * 5 + 7
+                assert (P[0, f] == np.inf) if weight == np.inf else (np.isnan(P[0, f]) or np.isfinite(P[0, f]))
+
+
+def test_bulk_scan_of_more_filters_than_one_pass_takes(ks):
+    """Over 1024 tiles of 32 filters, with tiles that are left out on both sides of the line."""
+    m, F = 24, 32 * 1024 + 33
+    rng, W, b, X, R = _bulk_case(62, [120, 33, 64, 100], m, F, odd_codes=False)
+    _closed_tiles(W, (3, 1023, 1024), 3e6)
+    P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", want_argmax=True, path="kmer")
+    pick = np.unique(np.concatenate([rng.choice(F, 80, replace=False), np.arange(32 * 1022, F), [96 + 7, 64, 127]]))
+    A, Pr, Ir = _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R, "max")
+    _within_rounding(host(P)[:, pick], Pr, W[:, pick], b[:, pick], "max")
+    rows = host(I)[:, pick] // F
+    moved = rows != Ir // len(pick)
+    # (beside a weight of 3e6 the others are below float32's last place: many rows tie there)
+    assert moved[:, np.abs(W[:, pick]).max(axis=0) < 1e6].mean() < 0.001 and np.array_equal(host(I)[:, pick] % F, np.broadcast_to(pick, rows.shape))
+
+
+def test_bulk_scan_left_out_tiles_under_capture(ks):
+    """The entry point with the built-in scratch in a graph: replays after the weights have changed, from tiles that are left out to none
+    and back, with other work between them, are the eager call's bits."""
+    m, F = 20, 96
+    rng, W0, b, X, R = _bulk_case(63, [200, 33, 224, 500, 110], m, F, odd_codes=False)
+    _, W1, _, _, _ = _bulk_case(64, [200], m, F)
+    W2 = W1.copy()
+    _closed_tiles(W2, (1,), 3e6)
+    _closed_tiles(W2, (2,), np.inf)
+    bd, Xd, Rd = dev(b), dev(X), dev(R)
+    want = [[host(x) for x in ks.scanpool_fprop(dev(W), bd, Xd, Rd, "all", want_argmax=True, path="kmer")] for W in (W0, W1, W2)]
+    Wd = dev(W0).clone()
+    out = (torch.empty((len(R), 2 * F), device="cuda"), torch.empty_like(ks.scanpool_fprop(Wd, bd, Xd, Rd, "all", want_argmax=True, path="kmer")[1]))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ks.scanpool_fprop(Wd, bd, Xd, Rd, "all", want_argmax=True, path="kmer_static", out=out)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ks.scanpool_fprop(Wd, bd, Xd, Rd, "all", want_argmax=True, path="kmer_static", out=out)
+    for i in (0, 2, 1, 2, 0):
+        Wd.copy_(dev((W0, W1, W2)[i]))
+        out[0].fill_(-1.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        ks.scanpool_fprop(dev(W1), bd, Xd, Rd, "max", path="kmer")
+        assert np.array_equal(host(out[0]), want[i][0], equal_nan=True) and np.array_equal(host(out[1]), want[i][1]), i
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
