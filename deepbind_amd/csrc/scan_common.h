@@ -9,9 +9,10 @@ constexpr int FT = 64;        // filters per tile = lanes per wave
 constexpr int NL = 6;         // letters in the LDS table
 constexpr int PSUB = 16;      // positions accumulated in registers at a time
 
-// Who takes the filters of a tile in a bulk call: the bulk kernel itself (below TILE_LEFT), or the launch behind it, finite weights on
-// the matrix cores and infinite, undefined or extreme ones from the letter table.
-constexpr unsigned TILE_BULK = 0, TILE_LEFT = 2, TILE_NOT_FINITE = 3;
+// What a bulk call notes of a tile's filters, one bit each. Without TILE_LEFT and TILE_NOT_FINITE the bulk kernel takes them (a weight of
+// minus infinity only closes its windows); else the launch behind it does, weights that are all finite on the matrix cores, others from
+// the letter table.
+constexpr unsigned TILE_BULK = 0, TILE_CLOSING = 1, TILE_LEFT = 2, TILE_NOT_FINITE = 4;
 
 __device__ __forceinline__ unsigned letter_of(unsigned code)
 {

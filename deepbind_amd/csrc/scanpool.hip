@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     const unsigned lane = threadIdx.x & 63u;
     auto asked = [&](unsigned t0) -> unsigned long long {
         const unsigned t = t0 + lane;
-        return __ballot(t < ftiles && (flags[2 * t] >= TILE_LEFT || flags[2 * t + 1] >= TILE_LEFT));
+        return __ballot(t < ftiles && ((flags[2 * t] | flags[2 * t + 1]) & (TILE_LEFT | TILE_NOT_FINITE)) != 0u);
     };
     unsigned left = 0u;
     for (unsigned t0 = 0; t0 < ftiles; t0 += 64u) left += (unsigned)__popcll(asked(t0));
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     for (; nth != 0u; --nth) who &= who - 1ull;
     const unsigned tile = t0 + (unsigned)__builtin_ctzll(who);
     const wg_t wg = {blockIdx.x / left, tile, gx, ftiles};
-    if (flags[2 * tile] == TILE_NOT_FINITE || flags[2 * tile + 1] == TILE_NOT_FINITE)
+    if (((flags[2 * tile] | flags[2 * tile + 1]) & (TILE_CLOSING | TILE_NOT_FINITE)) != 0u)
         scanpool_fprop_body<PT, WANT_ARGMAX, left_lookup_taps(KS)>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);
     else
         scanpool_fprop_mfma_body<PT, WANT_ARGMAX, false, KS, true>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);

@@ -51,6 +51,7 @@ namespace dbk_scanpool_digits {
 
 using dbk_mfma::f32x16_t;
 using dbk_scan::TILE_BULK;
+using dbk_scan::TILE_CLOSING;
 using dbk_scan::TILE_LEFT;
 using dbk_scan::TILE_NOT_FINITE;
 
@@ -70,7 +71,7 @@ constexpr float CLOSED = -3.0e38f;            // the value of a row outside the 
 __device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
 
 // ---------------------------------------------------------------------------------------------- the weights' digits
-// What a call keeps in its scratch, per tile of 32 filters: a flag (TILE_BULK, or who takes it instead), the filters'
+// What a call keeps in its scratch, per tile of 32 filters: a flag (TILE_LEFT and its like), the filters'
 // exponents, the digits, [8-tap block][digit][filter][24 bytes], and, to find a maximum's place, NTOP digits per weight in
 // units of the filter's own (no power of two) with what the scan has to know of them.
 struct digit_facts {
@@ -120,9 +121,9 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
 {
     __shared__ float red[6][8][FTILE];                            // sums and maxima of the eight threads of a filter
     __shared__ unsigned char dig[TB * (NDIGIT + NTOP) * SLOT_BYTES];
-    __shared__ unsigned worst;                                    // of the tile's filters
+    __shared__ unsigned tile;                                     // what is noted of its filters
     const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
-    if (threadIdx.x == 0) worst = TILE_BULK;
+    if (threadIdx.x == 0) tile = TILE_BULK;
     float w[TB][4];
 #pragma unroll
     for (int t = 0; t < TB; ++t)
@@ -172,7 +173,8 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
     const bool far = ((unsigned)odd & 63u) != 0u || bias_bits >= 0x71000000u || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-32f);
     const bool bad = far || (second > 0.0f && top > 64.0f * second) || (big != 0.0f && big < 1.0e-25f);
     if (!bad && big != 0.0f) e = (int)((__float_as_uint(big) >> 23) & 0xffu) - 127;
-    if (bad) atomicMax(&worst, far || odd >= 64.0f ? TILE_NOT_FINITE : TILE_LEFT);
+    const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (odd >= 64.0f ? TILE_CLOSING : TILE_BULK);
+    if (notes != TILE_BULK) atomicOr(&tile, notes);
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         float z = 0.0f;
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         k.whole = 29 - se;                                        // size < 2^(se + 1)
         out.facts[blockIdx.x * FTILE + fl] = k;
     }
-    if (threadIdx.x == 0) out.flags[blockIdx.x] = worst;
+    if (threadIdx.x == 0) out.flags[blockIdx.x] = tile;
 }
 
 // ---------------------------------------------------------------------------------------------- letters
@@ -390,7 +392,7 @@ __device__ __forceinline__ void products(f32x16_t& acc, const uint4& a0, const u
 // Whether the launch behind this one takes a tile: it takes tiles of 64 filters, that is pairs.
 __device__ __forceinline__ bool left_out(const unsigned* __restrict__ flags, unsigned tile)
 {
-    return flags[tile & ~1u] >= TILE_LEFT || flags[tile | 1u] >= TILE_LEFT;
+    return ((flags[tile & ~1u] | flags[tile | 1u]) & (TILE_LEFT | TILE_NOT_FINITE)) != 0u;
 }
 
 // ---------------------------------------------------------------------------------------------- the scan

@@ -1401,6 +1401,25 @@ def test_bulk_scan_beside_tiles_that_are_left_out(ks, m, tiles, ptype):
             assert np.array_equal(host(P)[:, 64 * k * t:64 * k * (t + 1)], host(Pp)[:, 64 * k * t:64 * k * (t + 1)])
 
 
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [8, 20])
+def test_bulk_scan_closing_weights_beside_a_filter_that_is_left_out(ks, m, ptype):
+    """Weights of minus infinity only close their windows, also where another filter of their tile of 32, or of the tile beside it,
+    sends them to the launch behind the bulk kernel."""
+    F = 32 * 4
+    rng, W, b, X, R = _bulk_case(520 + m, [200, 1, 33, 224, 500, 64, 110], m, F)
+    _closed_tiles(W, (0, 3), 3e6)
+    closing = [1, 20, 40, 70, 100]                                       # beside the first, in its pair, the pair's first, beside the second
+    for f in closing:
+        W[rng.choice(4 * m, 2, replace=False), f] = -np.inf
+    want = ptype != "avg"
+    P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=want, path="kmer")
+    A, Pr, Ir = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
+    _within_rounding(host(P), Pr, np.where(np.isinf(W), 0, W), b, ptype)
+    if want:
+        assert (host(I) != Ir)[:, np.abs(np.where(np.isinf(W), 0, W)).max(axis=0) < 1e6].mean() < 0.01
+
+
 @pytest.mark.parametrize("weight", [3e6, np.inf, np.nan])
 def test_bulk_scan_of_25_to_32_taps_beside_tiles_that_are_left_out(ks, weight):
     m, F = 32, 64 * 320 + 40
