@@ -78,7 +78,7 @@ struct digit_facts {
     float unit;         // digit NTOP - 1's step
     float above;        // the most that a window's weights lie above those digits, in units, and some slack
     float lowest;       // weights below count as this
-    int whole;          // weights times 2^whole add up to less than 2^30 over any window
+    int whole;          // what an open window's weights and the bias come to, times 2^whole, is below 2^30
 };
 struct digit_store { unsigned* flags; int* expo; digit_facts* facts; unsigned char *digits, *top; };
 inline size_t tile_bytes(unsigned tb) { return FTILE * (sizeof(int) + sizeof(digit_facts)) + (size_t)tb * (NDIGIT + NTOP) * SLOT_BYTES; }
@@ -223,8 +223,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
         k.above = above * (1.00001f / 32.0f) + 0.5f;
         k.lowest = floor_;
-        const int se = size > 0.0f ? (int)((__float_as_uint(size) >> 23) & 0xffu) - 127 : 0;
-        k.whole = 29 - se;                                        // size < 2^(se + 1)
+        k.whole = open > 0.0f && !bad ? 29 - ((int)((__float_as_uint(open) >> 23) & 0xffu) - 127) : 0;
         out.facts[blockIdx.x * FTILE + fl] = k;
     }
     if (threadIdx.x == 0) out.flags[blockIdx.x] = tile;
@@ -508,12 +507,12 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
 
 // ---------------------------------------------------------------------------------------------- plain maxima
 // Max pooling with filters of 17 to 32 taps: half the products. A region's maximum is one window, so the products only have
-// to find its place; its value is then added up from the weights themselves (whole numbers of 2^-30 of the largest sum that
-// a window can have: one rounding in the end). The first NTOP digits of every weight give every
+// to find its place; its value is then added up from the weights themselves, as whole numbers below 2^-29 of the most that an open
+// window comes to, with one rounding in the end (weights that only close windows may wrap: no winning window holds them). The first NTOP digits of every weight give every
 // window's sum to within what the digits left out can amount to. The value of the largest sum's window being known, it is
 // the maximum unless the second largest sum plus the most that the left out digits can add to any window (`above`, per
 // filter) reaches it. Where that is so (0.1 % of the filters and regions of 500 random letters, and windows that repeat),
-// the region is scanned once more with all the digits for the 32 filters concerned.
+// the region is scanned once more with all the digits, for the 32 filters concerned, to find the place.
 //
 // Sums of NTOP digits are whole numbers of 1/4 unit (a "mean of the four" counts quarters) below 2^18 units, which leaves
 // float32 four bits below: a lane's 16 rows start from 15/64 .. 0 units instead of zero, so the maximum carries its row's
@@ -561,7 +560,7 @@ __device__ __forceinline__ f32x16_t place_sums(const f32x16_t& rows, const uint4
 }
 
 // The maximum over a region from all the digits, and its row: this half wave's, without the bias.
-template <bool WANT_ARGMAX, int TB>
+template <int TB>
 __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, size_t N, size_t ndef, unsigned a, unsigned b, uint4* entries,
                                               const unsigned char* digits, unsigned lane, int expo)
 {
@@ -587,12 +586,19 @@ __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, 
 #pragma unroll
             for (int i = 0; i < 16; ++i) z[i] = 0.0f;
             products<TB, 0>(z, a0, a1, B, s);
+            if (left - t0 < (unsigned)ROWS) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const unsigned row = 4u * h + ((i & 3) + 8 * (i >> 2));
-                const float v = row < left - t0 ? z[i] : CLOSED;
-                if (WANT_ARGMAX) xi = v > mx ? (c - a) + t0 + row : xi;
-                mx = fmaxf(mx, v);
+                for (int i = 0; i < 16; ++i) z[i] = 4u * h + ((i & 3) + 8 * (i >> 2)) < left - t0 ? z[i] : CLOSED;
+            }
+            float best = z[0];
+#pragma unroll
+            for (int i = 1; i < 15; i += 2) best = fmaxf(fmaxf(best, z[i]), z[i + 1]);
+            best = fmaxf(best, z[15]);
+            if (__any(best > mx)) {                               // (where rows repeat, the first tiles alone)
+                unsigned at = 15u;
+#pragma unroll
+                for (int i = 14; i >= 0; --i) at = z[i] == best ? (unsigned)i : at;
+                if (best > mx) { mx = best; xi = (c - a) + t0 + 4u * h + (at & 3u) + 8u * (at >> 2); }
             }
         }
         if (left <= CHUNK) break;
@@ -664,13 +670,15 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
         const bool in = tap < m && f < F && (two || fl < FTILE);
         const digit_facts k = D.facts[tile * FTILE + (in ? fl : 0u)];
         const float scale = __uint_as_float((unsigned)(127 + k.whole) << 23);
-        int w[4];
+        // (what 32 bits do not hold is in no open window)
+        auto held = [](long long v) -> int { return v > -0x7fffffffll ? (int)v : -0x7fffffff; };
+        long long w[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) w[c] = in ? (int)rintf(fmaxf(W[(size_t)(4 * tap + c) * F + f], k.lowest) * scale) : 0;
-        const int mean = (int)(((long long)w[0] + w[1] + w[2] + w[3] + 2) >> 2);
+        for (int c = 0; c < 4; ++c) w[c] = in ? (long long)rintf(fmaxf(W[(size_t)(4 * tap + c) * F + f], k.lowest) * scale) : 0ll;
+        const int mean = held((w[0] + w[1] + w[2] + w[3] + 2) >> 2);
         int* row = table + (size_t)tap * 8 * PAIR + fl;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) row[c * PAIR] = c < 4 ? w[c & 3] : (c == 6 ? 0 : mean);      // codes mod 8: 254 is 6
+        for (int c = 0; c < 8; ++c) row[c * PAIR] = c < 4 ? held(w[c & 3]) : (c == 6 ? 0 : mean);      // codes mod 8: 254 is 6
     }
     if (threadIdx.x < PAIR) {
         const unsigned f = fbase + threadIdx.x;
@@ -758,37 +766,36 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
         const float4 filter = about[mine];
         const bool open = (best + filter.z) * filter.y + filter.x > 0.0f;      // else every window's rectified value is zero
         // ---- its value from the weights
-        float value = 0.0f;
-        const size_t at = (size_t)a + row;
-        if (open && at < ndef) {
+        auto value_at = [&](unsigned row_, float exponents) -> float {
+            const size_t at = (size_t)a + row_;
+            if (!open || at >= ndef) return 0.0f;
             unsigned v[2 * TB];
             if (at + TAPS <= N) __builtin_memcpy(v, X + at, TAPS);
             else load_tail<TAPS>(X, N, at, v);
-            int sum = 0;
+            unsigned sum = 0u;                                    // (the sum fits, whatever its parts run through)
 #pragma unroll
             for (int k = 0; k < 2 * TB; ++k) {
                 if (odd_codes(v[k]) != 0u) v[k] = plain_codes(v[k]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) sum += (table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
+                for (int j = 0; j < 4; ++j) sum += (unsigned)(table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
             }
-            value = (float)sum * __uint_as_float((unsigned)(127 + 1024 - (int)(__float_as_uint(filter.w) >> 16)) << 23);
-        }
+            return (float)(int)sum * __uint_as_float((unsigned)(127 + 1024 - (int)(__float_as_uint(exponents) >> 16)) << 23);
+        };
+        float value = value_at(row, filter.w);
         const bool unsure = open && !((second + filter.z) * filter.y < value);
         const unsigned long long who = __ballot(unsure);
         if (who != 0ull) {
-            // ---- too close to call: all the digits, for the 32 filters concerned
+            // ---- too close to call: its place from all the digits, for the 32 filters concerned
 #pragma unroll 1
             for (unsigned q = 0; q < 2; ++q) {
                 if ((unsigned)(who >> (32u * q)) == 0u) continue;
-                const float2 all = region_maximum<WANT_ARGMAX, TB>(X, N, ndef, a, b, entries, digits + q * TILE_DIGITS, mine,
-                                                                   (int)(__float_as_uint(about[32u * q + (mine & 31u)].w) & 0xffffu) - 1024);
+                const float2 all = region_maximum<TB>(X, N, ndef, a, b, entries, digits + q * TILE_DIGITS, mine,
+                                                      (int)(__float_as_uint(about[32u * q + (mine & 31u)].w) & 0xffffu) - 1024);
                 const float oz = __shfl_xor(all.x, 32, 64);
                 const unsigned xi = __float_as_uint(all.y), oi = (unsigned)__shfl_xor((int)xi, 32, 64);
-                if (unsure && (mine >> 5) == q) {
-                    value = fmaxf(all.x, oz);
-                    row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
-                }
+                if (unsure && (mine >> 5) == q) row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
             }
+            value = value_at(row, about[mine].w);
             load_places(mine);                                    // (not held over the pass: its operands take their registers)
         }
         value = open ? fmaxf(value + filter.x, 0.0f) : 0.0f;

@@ -1488,6 +1488,40 @@ def test_bulk_scan_left_out_tiles_under_capture(ks):
         assert np.array_equal(host(out[0]), want[i][0], equal_nan=True) and np.array_equal(host(out[1]), want[i][1]), i
 
 
+def _forbid(rng, W, kind):
+    """Weights far below zero, which only close their windows: at half of the taps on average, at each of twelve taps, infinite ones."""
+    m, F = W.shape[0] // 4, W.shape[1]
+    if kind == "twelve taps":
+        W[:] = rng.uniform(-0.05, 0.05, W.shape)
+        for t in range(min(m, 12)):
+            W[4 * t + rng.integers(0, 4, F), np.arange(F)] = -30.0
+    else:
+        for f in range(F):
+            W[rng.choice(4 * m, m // 2, replace=False), f] = -1e9 if kind == "half the taps" else -np.inf
+
+
+@pytest.mark.parametrize("kind", ["half the taps", "twelve taps", "infinite"])
+@pytest.mark.parametrize("m", [17, 24, 32])
+def test_bulk_maxima_of_long_filters_that_forbid_letters(ks, m, kind):
+    """The maximum is the sum of the winning window's weights, each within 2^-30 of T, what an open window comes to at most, however far
+    below zero the weights are that close other windows; then it is rounded twice."""
+    F = 96 if m <= 24 else 32 * 513
+    rng, W, b, X, R = _bulk_case(80 + m, [500, 300, 224, 700, 96, 450] + ([] if m <= 24 else [100] * 100), m, F, odd_codes=m <= 24)
+    _forbid(rng, W, kind)
+    pick = np.arange(F) if m <= 24 else np.sort(rng.choice(F, 96, replace=False))
+    A, Pr, Ir = _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R, "max")
+    T = np.maximum(W[:, pick].astype(np.float64).reshape(m, 4, -1), 0).max(axis=1).sum(axis=0) + np.maximum(b[0, pick], 0)
+    for want in ((False, True) if m <= 24 else (False,)):
+        P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", want_argmax=want, path="kmer" if m <= 24 else "auto")
+        P = host(P)[:, pick]
+        assert (Pr > 0).mean() > 0.2
+        assert np.all(np.abs(P - Pr) <= 2.0 ** -23 * (Pr + np.abs(b[0, pick])) + m * 2.0 ** -30 * T)
+        if want:
+            rows, cols = host(I) // F, np.broadcast_to(np.arange(F), Pr.shape)
+            moved = rows != Ir // F
+            assert moved.mean() < 0.01 and np.all(Pr[moved] - A[rows[moved], cols[moved]] <= m * 2.0 ** -25 * T[cols[moved]])
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
