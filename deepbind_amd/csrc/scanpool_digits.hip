@@ -75,7 +75,7 @@ __device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
 // exponents, the digits, [8-tap block][digit][filter][24 bytes], and, to find a maximum's place, NTOP digits per weight in
 // units of the filter's own (no power of two) with what the scan has to know of them.
 struct digit_facts {
-    float unit;         // digit NTOP - 1's step
+    float unit;         // digit NTOP - 1's step; zero where every window's sum is zero, or closed
     float above;        // the most that a window's weights lie above those digits, in units, and some slack
     float lowest;       // weights below count as this
     int whole;          // what an open window's weights and the bias come to, times 2^whole, is below 2^30
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         for (int k = 0; k < 8; ++k) above += red[0][k][fl];
         out.expo[blockIdx.x * FTILE + fl] = e;
         digit_facts k;
-        k.unit = finest * (1.0f / 1024.0f);
+        k.unit = size > 0.0f ? finest * (1.0f / 1024.0f) : 0.0f;
         // a quarter of a unit for the rows' numbers, a quarter for the rounding of a window's sum and of the scaled weights
         // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
         k.above = above * (1.00001f / 32.0f) + 0.5f;
@@ -764,7 +764,8 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
         const unsigned i = 15u - ((unsigned)(int)(best * 64.0f) & 15u);
         unsigned row = (upper ? t1[1] : t1[0]) * ROWS + (upper ? 4u : 0u) + (i & 3u) + 8u * (i >> 2);
         const float4 filter = about[mine];
-        const bool open = (best + filter.z) * filter.y + filter.x > 0.0f;      // else every window's rectified value is zero
+        // else every window's rectified value is zero (a region without rows has no best)
+        const bool open = best > CLOSED && (best + filter.z) * filter.y + filter.x > 0.0f;
         // ---- its value from the weights
         auto value_at = [&](unsigned row_, float exponents) -> float {
             const size_t at = (size_t)a + row_;
@@ -782,7 +783,7 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
             return (float)(int)sum * __uint_as_float((unsigned)(127 + 1024 - (int)(__float_as_uint(exponents) >> 16)) << 23);
         };
         float value = value_at(row, filter.w);
-        const bool unsure = open && !((second + filter.z) * filter.y < value);
+        const bool unsure = open && filter.y > 0.0f && !((second + filter.z) * filter.y < value);     // (windows all alike: the first row)
         const unsigned long long who = __ballot(unsure);
         if (who != 0ull) {
             // ---- too close to call: its place from all the digits, for the 32 filters concerned

@@ -1522,6 +1522,26 @@ def test_bulk_maxima_of_long_filters_that_forbid_letters(ks, m, kind):
             assert moved.mean() < 0.01 and np.all(Pr[moved] - A[rows[moved], cols[moved]] <= m * 2.0 ** -25 * T[cols[moved]])
 
 
+@pytest.mark.parametrize("m", [18, 24])
+def test_bulk_maxima_of_filters_whose_windows_are_all_alike(ks, m):
+    """Weights of zero, or none above it: nothing, or the bias, at the first row, and nothing where a region has no rows."""
+    F = 70
+    rng, W, b, X, R = _bulk_case(97 + m, [300, 224, 500, 90, 200], m, F)
+    W[:, :8] = 0.0
+    W[:, 8:16] = -np.abs(W[:, 8:16])
+    W[:, 16:20] = np.where(rng.random((4 * m, 4)) < 0.5, -np.inf, 0.0)
+    b[0, :20] = np.tile([0.3, -0.3, 0.0, 1e-12], 5)
+    R = np.concatenate([R, [[7, 7]]]).astype(np.uint32)
+    A, Pr, Ir = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R[:-1], "max")
+    P, I = [host(x) for x in ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", want_argmax=True, path="kmer")]
+    Pg = host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", path="general")[0])
+    assert np.array_equal(P[-1], Pg[-1])
+    _within_rounding(P[:-1], Pr, np.where(np.isinf(W), 0, W), b, "max")
+    alike = np.array([f for f in range(8)] + [9, 10, 13, 14])
+    assert np.array_equal(P[:-1, alike], Pr[:, alike].astype(np.float32)) and np.array_equal(I[:-1, alike], Ir[:, alike])
+    assert np.array_equal(host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", path="kmer")[0]), P)
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
