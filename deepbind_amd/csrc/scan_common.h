@@ -9,10 +9,10 @@ constexpr int FT = 64;        // filters per tile = lanes per wave
 constexpr int NL = 6;         // letters in the LDS table
 constexpr int PSUB = 16;      // positions accumulated in registers at a time
 
-// What a bulk call notes of a tile's filters, one bit each. Without TILE_LEFT and TILE_NOT_FINITE the bulk kernel takes them (a weight of
-// minus infinity only closes its windows); else the launch behind it does, weights that are all finite on the matrix cores, others from
-// the letter table.
-constexpr unsigned TILE_BULK = 0, TILE_CLOSING = 1, TILE_LEFT = 2, TILE_NOT_FINITE = 4;
+// What a bulk call notes of a tile's filters, one bit each: weights that only close their windows (far below zero, minus infinity), of them
+// minus infinity, weights that the bulk kernel does not express, finite or not. Without the last two the bulk kernel takes the tile; else
+// the launch behind it does, weights that are all finite on the matrix cores, others from the letter table.
+constexpr unsigned TILE_BULK = 0, TILE_CLOSES = 1, TILE_INFINITE = 2, TILE_LEFT = 4, TILE_NOT_FINITE = 8;
 
 __device__ __forceinline__ unsigned letter_of(unsigned code)
 {

@@ -317,7 +317,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     for (; nth != 0u; --nth) who &= who - 1ull;
     const unsigned tile = t0 + (unsigned)__builtin_ctzll(who);
     const wg_t wg = {blockIdx.x / left, tile, gx, ftiles};
-    if (((flags[2 * tile] | flags[2 * tile + 1]) & (TILE_CLOSING | TILE_NOT_FINITE)) != 0u)
+    if (((flags[2 * tile] | flags[2 * tile + 1]) & (TILE_INFINITE | TILE_NOT_FINITE)) != 0u)
         scanpool_fprop_body<PT, WANT_ARGMAX, left_lookup_taps(KS)>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);
     else
         scanpool_fprop_mfma_body<PT, WANT_ARGMAX, false, KS, true>(wg, W, bias, m, F, X, N, R, P, pooled, argmax, nullptr);

@@ -15,8 +15,11 @@
 // float32 additions tap by tap are off by 7.6e-8 and through a table of 3-mer sums by 6.2e-8.
 //
 // A weight far below zero only has to keep its window closed: every window's rectified value is at most
-// T = sum over the taps of the largest weight (if positive) + the bias, so weights below -8 T are raised to -8 T (a
-// window of one such "mean of four" is still at most -2 T + T). Filters that fixed point does not express well (an
+// T = sum over the taps of the largest weight (if positive) + the bias, so a window with a weight below -4.125 T is closed, a
+// "mean of the four" (-1.03 T + T) as well. Such weights are no part of the digits, whose unit they would make coarse (and
+// with it the sums: an instruction adds to a float32 with the precision of its largest operands, as they would be with a
+// first digit in every place): tiles that have them take one more product per 16 taps, -7.5 times a power of two above T in the
+// place of every such weight. Filters that fixed point does not express well (an
 // infinite or undefined weight, one positive weight more than 64 times the next) are left to a launch behind this one
 // (scanpool_fprop_left_kernel), which does nothing where no tile of filters asks for it.
 //
@@ -41,6 +44,7 @@
 #include "scan_common.h"
 #include "mfma_common.h"
 #include <mutex>
+#include <type_traits>
 
 namespace dbk_scanpool_general {
 int fprop_left(hipStream_t st, const float* W, const float* bias, size_t m, size_t F, const uint8_t* X, size_t N,
@@ -51,7 +55,8 @@ namespace dbk_scanpool_digits {
 
 using dbk_mfma::f32x16_t;
 using dbk_scan::TILE_BULK;
-using dbk_scan::TILE_CLOSING;
+using dbk_scan::TILE_CLOSES;
+using dbk_scan::TILE_INFINITE;
 using dbk_scan::TILE_LEFT;
 using dbk_scan::TILE_NOT_FINITE;
 
@@ -72,16 +77,18 @@ __device__ __forceinline__ unsigned place(unsigned q) { return q + (q >> 4); }
 
 // ---------------------------------------------------------------------------------------------- the weights' digits
 // What a call keeps in its scratch, per tile of 32 filters: a flag (TILE_LEFT and its like), the filters'
-// exponents, the digits, [8-tap block][digit][filter][24 bytes], and, to find a maximum's place, NTOP digits per weight in
-// units of the filter's own (no power of two) with what the scan has to know of them.
+// exponents, the digits, [8-tap block][digit][filter][24 bytes], to find a maximum's place NTOP digits per weight in
+// units of the filter's own (no power of two) with what the scan has to know of them, and the weights that close windows,
+// [8-tap block][filter][24 bytes].
 struct digit_facts {
     float unit;         // digit NTOP - 1's step; zero where every window's sum is zero, or closed
     float above;        // the most that a window's weights lie above those digits, in units, and some slack
-    float lowest;       // weights below count as this
+    float lowest;       // weights below only close their windows
     int whole;          // what an open window's weights and the bias come to, times 2^whole, is below 2^30
+    unsigned shut;      // block scales of a closing weight: beside all the digits, beside the first ones
 };
-struct digit_store { unsigned* flags; int* expo; digit_facts* facts; unsigned char *digits, *top; };
-inline size_t tile_bytes(unsigned tb) { return FTILE * (sizeof(int) + sizeof(digit_facts)) + (size_t)tb * (NDIGIT + NTOP) * SLOT_BYTES; }
+struct digit_store { unsigned* flags; int* expo; digit_facts* facts; unsigned char *digits, *top, *shut; };
+inline size_t tile_bytes(unsigned tb) { return FTILE * (sizeof(int) + sizeof(digit_facts)) + (size_t)tb * (NDIGIT + NTOP + 1) * SLOT_BYTES; }
 inline digit_store store_at(unsigned* flags, unsigned char* ws, unsigned ntile, unsigned tb)
 {
     digit_store s;
@@ -90,10 +97,12 @@ inline digit_store store_at(unsigned* flags, unsigned char* ws, unsigned ntile, 
     s.facts = reinterpret_cast<digit_facts*>(s.expo + (size_t)ntile * FTILE);
     s.digits = reinterpret_cast<unsigned char*>(s.facts + (size_t)ntile * FTILE);
     s.top = s.digits + (size_t)ntile * tb * NDIGIT * SLOT_BYTES;
+    s.shut = s.top + (size_t)ntile * tb * NTOP * SLOT_BYTES;
     return s;
 }
 
-// x, of magnitude up to 16.5, as ND digits base 32, each the nearest whole number; what remains, in units of the next digit
+// x, of magnitude up to 32, as ND digits base 32, each the nearest number that the 6-bit format has (in eighths: 0 .. 16, the even
+// ones up to 32); what remains, in units of the next digit
 template <int ND>
 __device__ __forceinline__ void split_digits(float (&x)[4], unsigned char* o)
 {
@@ -102,25 +111,28 @@ __device__ __forceinline__ void split_digits(float (&x)[4], unsigned char* o)
         unsigned word = 0u;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const float d = rintf(x[c]);
+            const float d = fabsf(x[c]) <= 16.0f ? rintf(x[c]) : 2.0f * rintf(0.5f * x[c]);
             x[c] = (x[c] - d) * 32.0f;                            // (exact)
             const int i = (int)d;
             const unsigned a = (unsigned)(i < 0 ? -i : i);
-            // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 15 are their own codes (denormal below 8), 16 is code 16
-            word |= (a | (i < 0 ? 32u : 0u)) << (6 * c);
+            // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 16 are their own codes (denormal below 8), 18 .. 32 17 .. 24
+            const unsigned code = a <= 16u ? a : 8u + (a >> 1);
+            word |= (code | (i < 0 ? 32u : 0u)) << (6 * c);
         }
         unsigned char* q = o + (size_t)p * SLOT_BYTES;
         q[0] = (unsigned char)word; q[1] = (unsigned char)(word >> 8); q[2] = (unsigned char)(word >> 16);
     }
 }
 
+__device__ __forceinline__ int exponent_of(float v) { return (int)((__float_as_uint(v) >> 23) & 0xffu) - 127; }
+
 // A workgroup splits one tile's weights: thread (g, fl) takes taps g, 8 + g, .. of filter fl. Latency only (4m x 32 values).
 template <int TB>
 __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restrict__ W, const float* __restrict__ bias, unsigned m, unsigned F,
                                                             unsigned f0, digit_store out)
 {
-    __shared__ float red[6][8][FTILE];                            // sums and maxima of the eight threads of a filter
-    __shared__ unsigned char dig[TB * (NDIGIT + NTOP) * SLOT_BYTES];
+    __shared__ float red[7][8][FTILE];                            // sums and maxima of the eight threads of a filter
+    __shared__ unsigned char dig[TB * (NDIGIT + NTOP + 1) * SLOT_BYTES];
     __shared__ unsigned tile;                                     // what is noted of its filters
     const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
     if (threadIdx.x == 0) tile = TILE_BULK;
@@ -133,8 +145,7 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
             w[t][c] = (tap < m && f < F) ? W[(size_t)(4 * tap + c) * F + f] : 0.0f;
         }
     const float b = f < F ? bias[f] : 0.0f;
-    float open = 0.0f, top = 0.0f, second = 0.0f, low = 0.0f;     // sum of the taps' best, the two largest weights, the most negative one
-    float size = 0.0f;                                            // sum of the taps' largest magnitudes
+    float open = 0.0f, top = 0.0f, second = 0.0f;                 // sum of the taps' best, the two largest weights
     const unsigned bias_bits = __float_as_uint(b) & 0x7fffffffu;      // (the file is compiled without NaN: test the bits)
     bool finite = bias_bits < 0x7f800000u, closing = false;           // closing: minus infinity among the weights
 #pragma unroll
@@ -148,58 +159,78 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
             best = fmaxf(best, w[t][c]);
             second = fmaxf(second, fminf(top, w[t][c]));
             top = fmaxf(top, w[t][c]);
-            low = fmaxf(low, -w[t][c]);
         }
         open += best;
     }
-    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = second; red[3][g][fl] = low; red[4][g][fl] = (finite ? 0.0f : 1.0f) + (closing ? 64.0f : 0.0f);
+    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = (finite ? 0.0f : 1.0f) + (closing ? 64.0f : 0.0f); red[3][g][fl] = second;
     __syncthreads();
-    open = fmaxf(b, 0.0f); top = 0.0f; second = 0.0f; low = 0.0f;
+    open = fmaxf(b, 0.0f); top = 0.0f; second = 0.0f;
     float odd = 0.0f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         open += red[0][k][fl];
-        const float tk = red[1][k][fl], sk = red[2][k][fl];
-        second = fmaxf(fmaxf(second, sk), fminf(top, tk));
+        const float tk = red[1][k][fl];
+        second = fmaxf(fmaxf(second, red[3][k][fl]), fminf(top, tk));
         top = fmaxf(top, tk);
-        low = fmaxf(low, red[3][k][fl]);
-        odd += red[4][k][fl];
+        odd += red[2][k][fl];
     }
-    const float floor_ = -8.0f * open;                            // nothing below keeps a window open
-    const float big = fmaxf(top, fminf(low, -floor_));
-    second = fmaxf(second, b);
-    int e = 0;
-    // sizes near the type's ends, where a weight's bf16 pieces or a sum may leave it, go with the infinite and undefined ones
-    const bool far = ((unsigned)odd & 63u) != 0u || bias_bits >= 0x71000000u || !(big < 1.0e30f) || (big != 0.0f && big < 1.0e-32f);
-    const bool bad = far || (second > 0.0f && top > 64.0f * second) || (big != 0.0f && big < 1.0e-25f);
-    if (!bad && big != 0.0f) e = (int)((__float_as_uint(big) >> 23) & 0xffu) - 127;
-    const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (odd >= 64.0f ? TILE_CLOSING : TILE_BULK);
-    if (notes != TILE_BULK) atomicOr(&tile, notes);
+    // ---- the weights that an open window can hold: all but those below -4.125 times the most that a window and the bias come to
+    const float lowest = -4.125f * open;
+    float mid = 0.0f, size = 0.0f;                                // of those: the largest magnitude, the sum over the taps of the largest
+    bool closed = false;
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
-        float z = 0.0f;
+        float most = 0.0f;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            w[t][c] = bad ? 0.0f : fmaxf(w[t][c], floor_);
-            z = fmaxf(z, fabsf(w[t][c]));
+            if (w[t][c] < lowest) closed = true;
+            else most = fmaxf(most, fabsf(w[t][c]));
         }
-        size += z;
+        mid = fmaxf(mid, most);
+        size += most;
     }
-    red[5][g][fl] = size;
+    red[4][g][fl] = mid; red[5][g][fl] = size; red[6][g][fl] = closed ? 1.0f : 0.0f;
     __syncthreads();
-    size = 0.0f;
+    mid = 0.0f; size = 0.0f;
+    float any = 0.0f;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) size += red[5][k][fl];
-    // all the digits: x = w * 2^(3 - e), below 16. The first ones by themselves: x = w / unit with a window's x at most
-    // 240 (so that its sum, in 1/1024, leaves room for a row's number below it: see the scan) and a weight's at most 16.4
+    for (int k = 0; k < 8; ++k) {
+        mid = fmaxf(mid, red[4][k][fl]);
+        size += red[5][k][fl];
+        any = fmaxf(any, red[6][k][fl]);
+    }
+    // ---- all the digits: x = w * 2^(3 - e), the largest weight below 16, the others that count below 32, one that closes its
+    // windows CLOSING, beyond `lowest`
+    // ---- all the digits: x = w * 2^(3 - e), the largest weight below 16, the others that count below 32
+    const bool none = mid == 0.0f && !(any > 0.0f && open > 0.0f);    // every window's sum is zero, or closed with no bias to open it
+    int e = 0;
+    if (mid > 0.0f) e = exponent_of(top) > exponent_of(mid) - 1 ? exponent_of(top) : exponent_of(mid) - 1;
+    // sizes near the type's ends, where a weight's bf16 pieces or a sum may leave it, go with the infinite and undefined ones
+    const bool far = ((unsigned)odd & 63u) != 0u || bias_bits >= 0x71000000u || !(open < 1.0e30f) || !(mid < 1.0e30f) || (mid != 0.0f && mid < 1.0e-32f);
+    second = fmaxf(second, b);
+    const bool bad = far || (second > 0.0f && top > 64.0f * second) || e < -84 || (!none && open < 1.0e-25f);
+    const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (odd >= 64.0f ? TILE_INFINITE : TILE_BULK) | (any > 0.0f ? TILE_CLOSES : TILE_BULK);
+    if (notes != TILE_BULK) atomicOr(&tile, notes);
+    if (bad) e = 0;
+    // The first ones by themselves: x = w / unit with a window's x at most 240 (so that its sum, in 1/1024, leaves room for a row's
+    // number below it: see the scan) and a weight's at most 16.4
     const float scale = __uint_as_float((unsigned)(127 + 3 - e) << 23);
-    const float finest = bad ? 1.0f : fmaxf(fmaxf(size * (1.0f / 240.0f), big * (1.0f / 16.4f)), 1.0e-30f), per = 1.0f / finest;
+    const float finest = bad || none ? 1.0f : fmaxf(fmaxf(size * (1.0f / 240.0f), mid * (1.0f / 16.4f)), fmaxf(any > 0.0f ? open * 0x1.0p-40f : 0.0f, 1.0e-30f));
+    const float per = 1.0f / finest;
     float above = 0.0f;                                           // the most that the weights exceed those digits by, in units of the next digit
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         float x[4], y[4];
+        unsigned shut = 0u;                                       // 63: -7.5
 #pragma unroll
-        for (int c = 0; c < 4; ++c) { x[c] = w[t][c] * scale; y[c] = w[t][c] * per; }
+        for (int c = 0; c < 4; ++c) {
+            const bool closes = w[t][c] < lowest;
+            x[c] = bad || closes ? 0.0f : w[t][c] * scale;
+            y[c] = bad || closes ? 0.0f : w[t][c] * per;
+            shut |= closes ? 63u << (6 * c) : 0u;
+        }
+        unsigned char* q = dig + ((size_t)(TB * (NDIGIT + NTOP) + t) * FTILE + fl) * 24u + 3u * g;
+        q[0] = (unsigned char)shut; q[1] = (unsigned char)(shut >> 8); q[2] = (unsigned char)(shut >> 16);
         split_digits<NDIGIT>(x, dig + ((size_t)t * NDIGIT * FTILE + fl) * 24u + 3u * g);
         split_digits<NTOP>(y, dig + ((size_t)(TB * NDIGIT + t * NTOP) * FTILE + fl) * 24u + 3u * g);
         above += fmaxf(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])), 0.0f);     // (a letter that counts nothing exceeds nothing)
@@ -212,18 +243,22 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
     src += TB * NDIGIT * SLOT_BYTES / 4;
     dst = reinterpret_cast<unsigned*>(out.top + (size_t)blockIdx.x * (TB * NTOP * SLOT_BYTES));
     for (unsigned i = threadIdx.x; i < TB * NTOP * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
+    src += TB * NTOP * SLOT_BYTES / 4;
+    dst = reinterpret_cast<unsigned*>(out.shut + (size_t)blockIdx.x * (TB * SLOT_BYTES));
+    for (unsigned i = threadIdx.x; i < TB * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
     if (g == 0) {
         above = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) above += red[0][k][fl];
         out.expo[blockIdx.x * FTILE + fl] = e;
         digit_facts k;
-        k.unit = size > 0.0f ? finest * (1.0f / 1024.0f) : 0.0f;
+        k.unit = none ? 0.0f : finest * (1.0f / 1024.0f);
         // a quarter of a unit for the rows' numbers, a quarter for the rounding of a window's sum and of the scaled weights
         // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
         k.above = above * (1.00001f / 32.0f) + 0.5f;
-        k.lowest = floor_;
-        k.whole = open > 0.0f && !bad ? 29 - ((int)((__float_as_uint(open) >> 23) & 0xffu) - 127) : 0;
+        k.lowest = lowest;
+        k.whole = open > 0.0f && !bad ? 29 - exponent_of(open) : 0;   // open < 2^(exponent + 1)
+        k.shut = open > 0.0f && !bad ? (unsigned)(130 + exponent_of(open)) | (unsigned)(130 + exponent_of(open * per * 1024.0f)) << 8 : 127u | 127u << 8;
         out.facts[blockIdx.x * FTILE + fl] = k;
     }
     if (threadIdx.x == 0) out.flags[blockIdx.x] = tile;
@@ -337,12 +372,12 @@ __device__ __forceinline__ f32x16_t product(const uint4& a, const unsigned (&b)[
 }
 
 // Block scales of a filter of exponent `expo`: digit p counts 2^(expo - 3 - 5 p) and is stored in eighths. s[0] and s[1]: the
-// digits one by one; s[2]: pairs of digits 2 j, 2 j + 1 of one block, this half wave's.
-__device__ __forceinline__ void digit_scales(int expo, unsigned h, int (&s)[3])
+// digits one by one; s[2]: pairs of digits 2 j, 2 j + 1 of one block, this half wave's. Byte 2 of s[1]: that of weights that close windows.
+__device__ __forceinline__ void digit_scales(int expo, unsigned shut, unsigned h, int (&s)[3])
 {
     const int e = expo + 127, eh = e - 5 * (int)h;
     s[0] = (e & 255) | ((e - 5) & 255) << 8 | ((e - 10) & 255) << 16 | (int)((unsigned)((e - 15) & 255) << 24);
-    s[1] = ((e - 20) & 255) | ((e - 25) & 255) << 8;
+    s[1] = ((e - 20) & 255) | ((e - 25) & 255) << 8 | (int)((shut & 255u) << 16);
     s[2] = (eh & 255) | ((eh - 10) & 255) << 8 | ((eh - 20) & 255) << 16;
 }
 
@@ -388,6 +423,31 @@ __device__ __forceinline__ void products(f32x16_t& acc, const uint4& a0, const u
     }
 }
 
+// The weights that close windows, -7.5 2^scale in the place of each, before anything else is added: nothing at all where the window has
+// none of them. `shut`: this half wave's and column's, in LDS, [block][filter][24 bytes], the blocks an even number (the last one may be empty).
+template <int TB> constexpr unsigned SHUT_BYTES = (TB <= 2 ? 2 : 4) * SLOT_BYTES;
+template <int TB, int SEL>
+__device__ __forceinline__ f32x16_t closed_windows(const f32x16_t& z, const uint4& a0, const uint4& a1, const unsigned char* shut, int scale)
+{
+    f32x16_t r = z;
+#pragma unroll
+    for (int i = 0; i < (TB <= 2 ? 1 : 2); ++i) {
+        unsigned B[6];
+        const uint2* src = reinterpret_cast<const uint2*>(shut + 2 * i * SLOT_BYTES);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { const uint2 v = src[k]; B[2 * k] = v.x; B[2 * k + 1] = v.y; }
+        r = product<SEL>(i == 0 ? a0 : a1, B, r, scale);
+    }
+    return r;
+}
+// a tile's from the scratch into LDS, by the whole workgroup
+template <int TB>
+__device__ __forceinline__ void load_shut(const unsigned char* from, unsigned char* shut, unsigned threads)
+{
+    for (unsigned i = threadIdx.x; i < SHUT_BYTES<TB> / 4; i += threads)
+        reinterpret_cast<unsigned*>(shut)[i] = i < TB * SLOT_BYTES / 4 ? reinterpret_cast<const unsigned*>(from)[i] : 0u;
+}
+
 // Whether the launch behind this one takes a tile: it takes tiles of 64 filters, that is pairs.
 __device__ __forceinline__ bool left_out(const unsigned* __restrict__ flags, unsigned tile)
 {
@@ -395,26 +455,28 @@ __device__ __forceinline__ bool left_out(const unsigned* __restrict__ flags, uns
 }
 
 // ---------------------------------------------------------------------------------------------- the scan
-template <int PT, bool WANT_ARGMAX, int TB>
-__global__ __launch_bounds__(NWAVE * 64) __attribute__((amdgpu_waves_per_eu(NWAVE / 4, NWAVE / 4)))
-void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsigned f0, unsigned F, const uint8_t* __restrict__ X, size_t N, size_t ndef,
-                            const uint32_t* __restrict__ R, unsigned P, unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+// CLOSES: some of the tile's filters have weights that close windows. (Two bodies, so that the products of those take no registers in the other.)
+template <int PT, bool WANT_ARGMAX, int TB, bool CLOSES>
+__device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsigned tile, unsigned split, const float* __restrict__ bias, unsigned f0, unsigned F,
+                                                     const uint8_t* __restrict__ X, size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P,
+                                                     unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NI = product_count<TB>::N;
-    const unsigned tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
-    if (left_out(D.flags, tile)) return;
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
     unsigned* counter = reinterpret_cast<unsigned*>(smem);
     uint4* entries = reinterpret_cast<uint4*>(smem + 16) + (size_t)wave * ENTRIES;
+    unsigned char* shut = smem + 16 + (size_t)NWAVE * ENTRIES * 16;
+    if (CLOSES) load_shut<TB>(D.shut + (size_t)tile * (TB * SLOT_BYTES), shut, NWAVE * 64);
     // this workgroup's regions
     const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
     if (threadIdx.x == 0) counter[0] = lo;
     unsigned B[NI][6];
     load_operands<TB>(D.digits + (size_t)tile * (TB * NDIGIT * SLOT_BYTES), col, h, B);
     int s[3];
-    digit_scales(D.expo[tile * FTILE + col], h, s);
+    digit_scales(D.expo[tile * FTILE + col], D.facts[tile * FTILE + col].shut, h, s);
+    shut += (h * FTILE + col) * 24u;
     const unsigned f = f0 + tile * FTILE + col;
     const float bf = f < F ? bias[f] : 0.0f;
     const unsigned rg = 4u * h;                                   // this half wave's rows lie 4 further down
@@ -450,6 +512,7 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
                 f32x16_t z;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+                if (CLOSES) z = closed_windows<TB, 2>(z, a0, a1, shut, s[1]);
                 products<TB, 0>(z, a0, a1, B, s);
                 if (left - t0 < (unsigned)ROWS) {
 #pragma unroll
@@ -503,6 +566,19 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
         rn = claim(counter, lane);
         if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
     }
+}
+
+template <int PT, bool WANT_ARGMAX, int TB>
+__global__ __launch_bounds__(NWAVE * 64) __attribute__((amdgpu_waves_per_eu(NWAVE / 4, NWAVE / 4)))
+void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsigned f0, unsigned F, const uint8_t* __restrict__ X, size_t N, size_t ndef,
+                            const uint32_t* __restrict__ R, unsigned P, unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+{
+    const unsigned tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
+    if (left_out(D.flags, tile)) return;
+    if ((D.flags[tile] & TILE_CLOSES) != 0u)
+        scanpool_digits_body<PT, WANT_ARGMAX, TB, true>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
+    else
+        scanpool_digits_body<PT, WANT_ARGMAX, TB, false>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
 }
 
 // ---------------------------------------------------------------------------------------------- plain maxima
@@ -560,14 +636,15 @@ __device__ __forceinline__ f32x16_t place_sums(const f32x16_t& rows, const uint4
 }
 
 // The maximum over a region from all the digits, and its row: this half wave's, without the bias.
-template <int TB>
+template <int TB, bool CLOSES>
 __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, size_t N, size_t ndef, unsigned a, unsigned b, uint4* entries,
-                                              const unsigned char* digits, unsigned lane, int expo)
+                                              const unsigned char* digits, const unsigned char* shut, unsigned lane, int expo, unsigned scale)
 {
     asm volatile("" : "+v"(lane));                                // (opaque: nothing of this is held in registers across the regions)
     const unsigned col = lane & 31u, h = lane >> 5, at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
     int s[3];
-    digit_scales(expo, h, s);
+    digit_scales(expo, scale, h, s);
+    shut += (h * FTILE + col) * 24u;
     unsigned B[product_count<TB>::N][6];
     load_operands<TB>(digits, col, h, B);
     float mx = CLOSED;
@@ -585,6 +662,7 @@ __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, 
             f32x16_t z;
 #pragma unroll
             for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+            if (CLOSES) z = closed_windows<TB, 2>(z, a0, a1, shut, s[1]);
             products<TB, 0>(z, a0, a1, B, s);
             if (left - t0 < (unsigned)ROWS) {
 #pragma unroll
@@ -641,30 +719,34 @@ __device__ __forceinline__ void swap_halves(float& x, float& y)
     y = __uint_as_float(b);
 }
 
-template <bool WANT_ARGMAX, int TB>
-__global__ __launch_bounds__(MAX_WAVES * 64) __attribute__((amdgpu_waves_per_eu(MAX_WAVES / 4, MAX_WAVES / 4)))
-void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __restrict__ W, const float* __restrict__ bias, unsigned f0, unsigned m, unsigned F,
-                                const uint8_t* __restrict__ X, size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P, unsigned nsplit,
-                                float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+template <bool WANT_ARGMAX, int TB, bool CLOSES>
+__device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, unsigned tile, unsigned split, bool two, const float* __restrict__ W,
+                                                         const float* __restrict__ bias, unsigned f0, unsigned m, unsigned F, const uint8_t* __restrict__ X,
+                                                         size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P, unsigned nsplit,
+                                                         float* __restrict__ pooled, uint32_t* __restrict__ argmax)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NI = place_count<TB>::N;
     constexpr unsigned TAPS = 8u * TB, TILE_DIGITS = TB * NDIGIT * SLOT_BYTES;
-    const unsigned tile = 2u * (blockIdx.x / nsplit), split = blockIdx.x % nsplit;
-    const bool two = tile + 1u < ntile;                           // (an odd last tile is scanned beside nothing)
-    if (left_out(D.flags, tile)) return;
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
     unsigned* counter = reinterpret_cast<unsigned*>(smem);
     uint4* entries = reinterpret_cast<uint4*>(smem + 16) + (size_t)wave * ENTRIES;
     int* table = reinterpret_cast<int*>(smem + 16 + MAX_WAVES * ENTRIES * 16);      // [8 TB taps][8 codes][64 filters]: the weights as whole numbers
+    // all the digits, or (LDS does not hold both) the weights that close windows
     unsigned char* digits = reinterpret_cast<unsigned char*>(table + TAPS * 8 * PAIR);
+    unsigned char* shut = digits;
     float4* about = reinterpret_cast<float4*>(digits + 2 * TILE_DIGITS);            // [64 filters]: bias, unit, above, exponents
     const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
     if (threadIdx.x == 0) counter[0] = lo;
     const unsigned fbase = f0 + tile * FTILE;
-    for (unsigned i = threadIdx.x; i < (two ? 2u : 1u) * TILE_DIGITS / 16; i += MAX_WAVES * 64)
-        reinterpret_cast<uint4*>(digits)[i] = reinterpret_cast<const uint4*>(D.digits + (size_t)tile * TILE_DIGITS)[i];
+    if (CLOSES) {
+        load_shut<TB>(D.shut + (size_t)tile * (TB * SLOT_BYTES), shut, MAX_WAVES * 64);
+        if (two) load_shut<TB>(D.shut + (size_t)(tile + 1) * (TB * SLOT_BYTES), shut + SHUT_BYTES<TB>, MAX_WAVES * 64);
+    } else {
+        for (unsigned i = threadIdx.x; i < (two ? 2u : 1u) * TILE_DIGITS / 16; i += MAX_WAVES * 64)
+            reinterpret_cast<uint4*>(digits)[i] = reinterpret_cast<const uint4*>(D.digits + (size_t)tile * TILE_DIGITS)[i];
+    }
     for (unsigned i = threadIdx.x; i < TAPS * PAIR; i += MAX_WAVES * 64) {
         const unsigned tap = i / PAIR, fl = i % PAIR, f = fbase + fl;
         const bool in = tap < m && f < F && (two || fl < FTILE);
@@ -686,7 +768,7 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
         const digit_facts k = D.facts[tile * FTILE + (in ? threadIdx.x : 0u)];
         // (filters past the last: closed whatever their sums)
         about[threadIdx.x] = make_float4(in ? bias[f] : CLOSED, k.unit, k.above,
-                                         __uint_as_float((unsigned)(k.whole + 1024) << 16 | (unsigned)(D.expo[tile * FTILE + (in ? threadIdx.x : 0u)] + 1024)));
+                                         __uint_as_float((unsigned)(k.whole + 128) << 24 | (unsigned)(D.expo[tile * FTILE + (in ? threadIdx.x : 0u)] + 128) << 16 | k.shut));
     }
     __syncthreads();
     unsigned B[2][NI][6];
@@ -707,6 +789,9 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
     load_places(lane);
     // a unit is digit 2's step: digit p counts 2^(5 (2 - p)), stored in eighths
     const int single = 140 | 135 << 8 | 130 << 16, pair = 140 | (135 - 5 * (int)h) << 8;
+    // (of weights that close windows: those of the first 32 filters, of the others)
+    const int shut_scales = (int)(((__float_as_uint(about[col].w) >> 8) & 255u) | (__float_as_uint(about[FTILE + col].w) & 0xff00u));
+    const unsigned char* shut_here = shut + (h * FTILE + col) * 24u;
     f32x16_t rows;                                                // what the rows start from, in 1/64 of a unit
 #pragma unroll
     for (int i = 0; i < 16; ++i) rows[i] = (float)(15 - i) * (1.0f / 64.0f);
@@ -738,18 +823,23 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
             for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34, ++t) {
                 uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
                 if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
-                const unsigned rest = left - t0;                  // (rows of the region from this tile on)
+                const unsigned rest = left - t0;              // (rows of the region from this tile on)
                 const int inside = (int)(rest < 64u ? rest : 64u) - 4 * (int)h;
-                auto half = [&](int q) {
-                    f32x16_t z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
+                auto half = [&](auto second_half) {
+                    constexpr int q = decltype(second_half)::value;
+                    f32x16_t z;
+                    if constexpr (CLOSES)
+                        z = place_sums<TB>(closed_windows<TB, q>(rows, a0, a1, shut_here + q * SHUT_BYTES<TB>, shut_scales), a0, a1, B[q], single, pair);
+                    else
+                        z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
                     if (rest < (unsigned)ROWS) {
 #pragma unroll
                         for (int i = 0; i < 16; ++i) z[i] = (i & 3) + 8 * (i >> 2) < inside ? z[i] : CLOSED;
                     }
                     top_two(z, m1[q], m2[q], t1[q], t);
                 };
-                half(0);
-                half(1);
+                half(std::integral_constant<int, 0>{});
+                half(std::integral_constant<int, 1>{});
             }
             c += CHUNK;
         } while (!last);
@@ -780,7 +870,7 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
 #pragma unroll
                 for (int j = 0; j < 4; ++j) sum += (unsigned)(table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
             }
-            return (float)(int)sum * __uint_as_float((unsigned)(127 + 1024 - (int)(__float_as_uint(exponents) >> 16)) << 23);
+            return (float)(int)sum * __uint_as_float((unsigned)(127 + 128 - (int)(__float_as_uint(exponents) >> 24)) << 23);
         };
         float value = value_at(row, filter.w);
         const bool unsure = open && filter.y > 0.0f && !((second + filter.z) * filter.y < value);     // (windows all alike: the first row)
@@ -790,8 +880,9 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
 #pragma unroll 1
             for (unsigned q = 0; q < 2; ++q) {
                 if ((unsigned)(who >> (32u * q)) == 0u) continue;
-                const float2 all = region_maximum<TB>(X, N, ndef, a, b, entries, digits + q * TILE_DIGITS, mine,
-                                                      (int)(__float_as_uint(about[32u * q + (mine & 31u)].w) & 0xffffu) - 1024);
+                const unsigned expo = __float_as_uint(about[32u * q + (mine & 31u)].w);
+                const float2 all = region_maximum<TB, CLOSES>(X, N, ndef, a, b, entries, CLOSES ? D.digits + (size_t)(tile + q) * TILE_DIGITS : digits + q * TILE_DIGITS, shut + q * SHUT_BYTES<TB>,
+                                                      mine, (int)((expo >> 16) & 255u) - 128, expo & 255u);
                 const float oz = __shfl_xor(all.x, 32, 64);
                 const unsigned xi = __float_as_uint(all.y), oi = (unsigned)__shfl_xor((int)xi, 32, 64);
                 if (unsure && (mine >> 5) == q) row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
@@ -813,6 +904,21 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
     }
 }
 
+template <bool WANT_ARGMAX, int TB>
+__global__ __launch_bounds__(MAX_WAVES * 64) __attribute__((amdgpu_waves_per_eu(MAX_WAVES / 4, MAX_WAVES / 4)))
+void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __restrict__ W, const float* __restrict__ bias, unsigned f0, unsigned m, unsigned F,
+                                const uint8_t* __restrict__ X, size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P, unsigned nsplit,
+                                float* __restrict__ pooled, uint32_t* __restrict__ argmax)
+{
+    const unsigned tile = 2u * (blockIdx.x / nsplit), split = blockIdx.x % nsplit;
+    const bool two = tile + 1u < ntile;                           // (an odd last tile is scanned beside nothing)
+    if (left_out(D.flags, tile)) return;
+    if (((D.flags[tile] | (two ? D.flags[tile + 1] : 0u)) & TILE_CLOSES) != 0u)
+        scanpool_digits_max_body<WANT_ARGMAX, TB, true>(D, tile, split, two, W, bias, f0, m, F, X, N, ndef, R, P, nsplit, pooled, argmax);
+    else
+        scanpool_digits_max_body<WANT_ARGMAX, TB, false>(D, tile, split, two, W, bias, f0, m, F, X, N, ndef, R, P, nsplit, pooled, argmax);
+}
+
 // workgroups per group of filters: one workgroup per CU in all, no more waves than regions
 inline unsigned splits(unsigned groups, unsigned waves, size_t P)
 {
@@ -824,9 +930,9 @@ inline unsigned splits(unsigned groups, unsigned waves, size_t P)
 
 constexpr size_t max_smem(int tb)
 {
-    return 16 + (size_t)MAX_WAVES * ENTRIES * 16 + (size_t)tb * (8 * 8 * PAIR * sizeof(float) + 2 * NDIGIT * SLOT_BYTES) + PAIR * 16;
+    return 16 + (size_t)MAX_WAVES * ENTRIES * 16 + (size_t)tb * (8 * 8 * PAIR * sizeof(int) + 2 * NDIGIT * SLOT_BYTES) + PAIR * 16;
 }
-static_assert(max_smem(4) <= 160 * 1024, "LDS of a CU");
+static_assert(max_smem(4) <= 160 * 1024 && SHUT_BYTES<4> <= 3 * NDIGIT * SLOT_BYTES, "LDS of a CU");
 
 template <bool WANT_ARGMAX, int TB>
 int launch_max(hipStream_t st, const digit_store& D, const float* W, const float* bias, unsigned f0, unsigned ntile, size_t m, size_t F, const uint8_t* X,
@@ -840,16 +946,16 @@ int launch_max(hipStream_t st, const digit_store& D, const float* W, const float
     return 0;
 }
 
-constexpr size_t SMEM = 16 + (size_t)NWAVE * ENTRIES * 16;
+constexpr size_t scan_smem(int tb) { return 16 + (size_t)NWAVE * ENTRIES * 16 + (tb <= 2 ? SHUT_BYTES<2> : SHUT_BYTES<4>); }
 
 template <int PT, bool WANT_ARGMAX, int TB>
 int launch_pt(hipStream_t st, const digit_store& D, const float* bias, unsigned f0, unsigned ntile, size_t F, const uint8_t* X, size_t N, size_t ndef,
               const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
 {
     auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB>;
-    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SMEM));
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_smem(TB)));
     const unsigned nsplit = splits(ntile, NWAVE, P);
-    hipLaunchKernelGGL(kern, dim3(ntile * nsplit), dim3(NWAVE * 64), SMEM, st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
+    hipLaunchKernelGGL(kern, dim3(ntile * nsplit), dim3(NWAVE * 64), scan_smem(TB), st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
     return 0;
 }
 
@@ -953,10 +1059,10 @@ int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F,
 // Every device the library runs on holds its own copy of this array, at its own address, from the moment the code
 // object is loaded there until the process ends. The array's name is a host-side handle, not a device address:
 // host code asks the runtime for the address once per device and passes that pointer to the kernels.
-// (24 taps: 1024 tiles' digits, 21.9 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
-constexpr size_t STATIC_SCRATCH_BYTES = size_t(22) << 20;
+// (24 taps: 1024 tiles' digits, 24.4 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
+constexpr size_t STATIC_SCRATCH_BYTES = size_t(24) << 20;
 constexpr size_t STATIC_SEQUENCE_BYTES = (size_t(64) << 20) - 127; // sequence bytes a call may bring
-static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * (sizeof(int) + sizeof(digit_facts)) + 3 * (NDIGIT + NTOP) * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
+static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * (sizeof(int) + sizeof(digit_facts)) + 3 * (NDIGIT + NTOP + 1) * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
 static __device__ __align__(256) unsigned char scratch[STATIC_SCRATCH_BYTES];
 static unsigned char* g_static_scratch[64] = {nullptr};
 static std::mutex g_static_scratch_mutex;

@@ -188,7 +188,7 @@ int dbk_scanpool_fprop_kmer(dbk_stream_t stream,
  * serving loops, harnesses that forbid allocation): same arguments, same kernels, same results, but the call's
  * scratch (the weights' digits) lies in a buffer that is part of the loaded
  * library instead of a grow-on-demand allocation, so the call never allocates, frees or synchronises.
- * Limit: N <= 64 MiB - 127 sequence bytes per call (ValueError beyond; the buffer's 22 MiB are held on every
+ * Limit: N <= 64 MiB - 127 sequence bytes per call (ValueError beyond; the buffer's 24 MiB are held on every
  * GPU the library runs on until the process ends). All calls on one GPU share the buffer: calls that overlap
  * on one GPU (different streams, different host threads) race; calls ordered on one stream do not.
  * No counterpart in the reference (its wrappers allocate per call, kangaroo/_ext/kangaroo_smat.py:121-132). */

@@ -1542,6 +1542,27 @@ def test_bulk_maxima_of_filters_whose_windows_are_all_alike(ks, m):
     assert np.array_equal(host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", path="kmer")[0]), P)
 
 
+@pytest.mark.parametrize("ptype", ["max", "avg"])
+@pytest.mark.parametrize("kind", ["half the taps", "twelve taps", "infinite"])
+@pytest.mark.parametrize("m", [4, 8, 16, 20, 24])
+def test_bulk_scan_of_filters_that_forbid_letters_is_as_close_as_float32(ks, m, kind, ptype):
+    """Every window of filters with weights far below zero, as a region of its own: those that hold none of them are no further from
+    float64 than a float32 sum tap by tap, the others are closed."""
+    F, n = 96, 3000
+    rng, W, b, X, _ = _bulk_case(90 + m, [n], m, F, odd_codes=False)
+    _forbid(rng, W, kind)
+    b[:] = 0.0
+    R = np.stack([np.arange(n), np.arange(n) + 1], axis=1).astype(np.uint32)
+    want = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)[1]
+    with np.errstate(invalid="ignore"):
+        plain = _chain_oracle(W, b, X, R, ptype)[1]
+    P = host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")[0])
+    some = want > 0.05 * want.max()
+    assert some.sum() > 500 and np.array_equal(P == 0, want == 0)
+    off = lambda got: np.sqrt(np.mean(((got[some] - want[some]) / want[some]) ** 2))
+    assert off(P) <= off(plain)
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
