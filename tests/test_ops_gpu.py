@@ -1563,6 +1563,30 @@ def test_bulk_scan_of_filters_that_forbid_letters_is_as_close_as_float32(ks, m, 
     assert off(P) <= off(plain)
 
 
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [5, 8, 16, 24])
+@pytest.mark.parametrize("count,size", [(1, 1e4), (2, 20.0), (2, 150.0), (2, 1e4), (3, 1e6)])
+def test_bulk_scan_of_weights_beyond_most_others(ks, count, size, m, ptype):
+    """Filters with several weights far above the others, all for one letter, over regions that do not hold it: from some hundred times
+    the others on their values are rounded in the size of the weights that they are sums of."""
+    F = 96
+    rng, W, b, X, R = _bulk_case(95 + m, [300, 33, 224, 500, 64], m, F, odd_codes=False)
+    X[X == 0] = 3
+    X[X == 255] = 1
+    small = W.copy()
+    small[0::4] = 0.0
+    for f in range(0, F, 2):
+        W[4 * rng.choice(m, count, replace=False), f] = 0.1 * size
+    P = host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")[0])
+    want = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)[1]
+    if size > 1e3:
+        _within_rounding(P, want, small, b, ptype)
+    plain = _chain_oracle(W, b, X, R, ptype)[1]
+    some = want > 0
+    off = lambda got: np.sqrt(np.mean(((got[some] - want[some]) / want[some]) ** 2))
+    assert off(P) <= (2.0 * off(plain) if size > 1e3 else 6e-7)
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
