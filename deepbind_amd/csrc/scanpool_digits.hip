@@ -265,7 +265,9 @@ __global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restr
         k.unit = none ? 0.0f : finest * (1.0f / 1024.0f);
         // a quarter of a unit for the rows' numbers, a quarter for the rounding of a window's sum and of the scaled weights
         // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
-        k.above = above * (1.00001f / 32.0f) + 0.5f;
+        // and of all the digits' (below 1/32): a place that is sure is the one that all the digits find. A bias far above the weights makes the
+        // value coarse, by 2^-30 of it per tap.
+        k.above = above * (1.00001f / 32.0f) + 0.5f + (float)(8 * TB) * 0x1.0p-30f * (open * per * 1024.0f);
         k.lowest = lowest;
         k.whole = open > 0.0f && !bad ? 29 - exponent_of(open) : 0;   // open < 2^(exponent + 1)
         k.shut = open > 0.0f && !bad ? (unsigned)(130 + exponent_of(open)) | (unsigned)(130 + exponent_of(open * per * 1024.0f)) << 8 : 127u | 127u << 8;
@@ -597,8 +599,12 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
 // window comes to, with one rounding in the end (weights that only close windows may wrap: no winning window holds them). The first NTOP digits of every weight give every
 // window's sum to within what the digits left out can amount to. The value of the largest sum's window being known, it is
 // the maximum unless the second largest sum plus the most that the left out digits can add to any window (`above`, per
-// filter) reaches it. Where that is so (0.1 % of the filters and regions of 500 random letters, and windows that repeat),
-// the region is scanned once more with all the digits, for the 32 filters concerned, to find the place.
+// filter) reaches it. Where that is so (of normal weights over 500 random letters 0.1 % of the filters and regions), the region is
+// scanned once more with all the digits, for the 32 filters concerned, to find the place. In sequences that repeat the windows
+// tie in every filter: after two regions in a row that were unsure in both halves of its 64 filters a wave takes the next 15 to all the
+// digits at once. A place that is sure is the one that those find (`above` has their rounding in it), so that a result does not depend
+// on which regions a wave met before. Measured, 20 000 x 500 letters x 512 filters, ms, 24 / 32 taps: uniform letters 0.85 / 0.98, units of 7
+// letters that repeat 1.30 / 1.62 (every region twice 1.95 / 2.38; the table of 3-mer sums 1.35 / 2.7 whatever the letters).
 //
 // Sums of NTOP digits are whole numbers of 1/4 unit (a "mean of the four" counts quarters) below 2^18 units, which leaves
 // float32 four bits below: a lane's 16 rows start from 15/64 .. 0 units instead of zero, so the maximum carries its row's
@@ -609,6 +615,7 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
 // waves per workgroup: three per SIMD at up to 168 registers. At a region's end lanes 0-31 hold the
 // first 32 filters and lanes 32-63 the others, and each adds up its own filter's window.
 constexpr int MAX_WAVES = 12;
+constexpr unsigned AT_ONCE = 15;              // regions that go to all the digits at once before the places are tried again
 constexpr int PAIR = 2 * FTILE;               // filters per workgroup
 
 template <int TB> struct place_count { static constexpr int N = TB == 3 ? 5 : 6; };
@@ -645,10 +652,10 @@ __device__ __forceinline__ f32x16_t place_sums(const f32x16_t& rows, const uint4
     return z;
 }
 
-// The maximum over a region from all the digits, and its row: this half wave's, without the bias.
+// The maximum over a region from all the digits, and its row: this half wave's, without the bias, of the filters wanted (a bit each).
 template <int TB, bool CLOSES>
 __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, size_t N, size_t ndef, unsigned a, unsigned b, uint4* entries,
-                                              const unsigned char* digits, const unsigned char* shut, unsigned lane, int expo, unsigned scale)
+                                              const unsigned char* digits, const unsigned char* shut, unsigned lane, int expo, unsigned scale, unsigned wanted)
 {
     asm volatile("" : "+v"(lane));                                // (opaque: nothing of this is held in registers across the regions)
     const unsigned col = lane & 31u, h = lane >> 5, at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
@@ -682,11 +689,12 @@ __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, 
 #pragma unroll
             for (int i = 1; i < 15; i += 2) best = fmaxf(fmaxf(best, z[i]), z[i + 1]);
             best = fmaxf(best, z[15]);
-            if (__any(best > mx)) {                               // (where rows repeat, the first tiles alone)
+            const bool further = best > mx && ((wanted >> col) & 1u) != 0u;
+            if (__any(further)) {                                 // (where rows repeat, the first tiles alone)
                 unsigned at = 15u;
 #pragma unroll
                 for (int i = 14; i >= 0; --i) at = z[i] == best ? (unsigned)i : at;
-                if (best > mx) { mx = best; xi = (c - a) + t0 + 4u * h + (at & 3u) + 8u * (at >> 2); }
+                if (further) { mx = best; xi = (c - a) + t0 + 4u * h + (at & 3u) + 8u * (at >> 2); }
             }
         }
         if (left <= CHUNK) break;
@@ -815,102 +823,135 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
     unsigned letters[3] = {0u, 0u, 0u};
     if (r < hi) load12(X, N, a, lane, letters);
 
-    while (r < hi) {
-        float m1[2] = {CLOSED, CLOSED}, m2[2] = {CLOSED, CLOSED}; // the two largest sums so far
-        unsigned t1[2] = {0u, 0u}, t = 0u;                        // the tile of the largest, the tile in work
-        unsigned c = a;
-        bool last;
-        do {
-            const unsigned left = b > c ? b - c : 0u;             // rows of the region from this stretch on
-            last = left <= CHUNK;
-            stage(entries, lane, letters);
-            // the next stretch's letters travel while this one is multiplied
-            if (!last) load12(X, N, c + CHUNK, lane, letters);
-            else if (rn < hi) load12(X, N, (unsigned)__builtin_amdgcn_readfirstlane((int)an), lane, letters);
-            const unsigned nrow = last ? left : CHUNK;
-            const unsigned defined = defined_rows(ndef, c);
-            const uint4* src = entries;
-            for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34, ++t) {
-                uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
-                if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
-                const unsigned rest = left - t0;              // (rows of the region from this tile on)
-                const int inside = (int)(rest < 64u ? rest : 64u) - 4 * (int)h;
-                auto half = [&](auto second_half) {
-                    constexpr int q = decltype(second_half)::value;
-                    f32x16_t z;
-                    if constexpr (CLOSES)
-                        z = place_sums<TB>(closed_windows<TB, q>(rows, a0, a1, shut_here + q * SHUT_BYTES<TB>, shut_scales), a0, a1, B[q], single, pair);
-                    else
-                        z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
-                    if (rest < (unsigned)ROWS) {
+    // the value of a window (relative to the region), from the weights
+    auto value_at = [&](unsigned mine, bool open, unsigned row, float exponents) -> float {
+        const size_t at = (size_t)a + row;
+        if (!open || at >= ndef) return 0.0f;
+        unsigned v[2 * TB];
+        if (at + TAPS <= N) __builtin_memcpy(v, X + at, TAPS);
+        else load_tail<TAPS>(X, N, at, v);
+        unsigned sum = 0u;                                        // (the sum fits, whatever its parts run through)
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) z[i] = (i & 3) + 8 * (i >> 2) < inside ? z[i] : CLOSED;
-                    }
-                    top_two(z, m1[q], m2[q], t1[q], t);
-                };
-                half(std::integral_constant<int, 0>{});
-                half(std::integral_constant<int, 1>{});
-            }
-            c += CHUNK;
-        } while (!last);
-        // ---- each filter's two half waves side by side: the largest sum, its place, the second largest
-        unsigned mine = lane;                                     // (opaque: addresses are formed from it here, not held in registers)
-        asm volatile("" : "+v"(mine));
-        swap_halves(m1[0], m1[1]);
-        swap_halves(m2[0], m2[1]);
-        swap_halves(t1[0], t1[1]);
-        const bool upper = m1[1] > m1[0];
-        const float best = fmaxf(m1[0], m1[1]), second = fmaxf(fminf(m1[0], m1[1]), fmaxf(m2[0], m2[1]));
-        const unsigned i = 15u - ((unsigned)(int)(best * 64.0f) & 15u);
-        unsigned row = (upper ? t1[1] : t1[0]) * ROWS + (upper ? 4u : 0u) + (i & 3u) + 8u * (i >> 2);
-        const float4 filter = about[mine];
-        // else every window's rectified value is zero (a region without rows has no best)
-        const bool open = best > CLOSED && (best + filter.z) * filter.y + filter.x > 0.0f;
-        // ---- its value from the weights
-        auto value_at = [&](unsigned row_, float exponents) -> float {
-            const size_t at = (size_t)a + row_;
-            if (!open || at >= ndef) return 0.0f;
-            unsigned v[2 * TB];
-            if (at + TAPS <= N) __builtin_memcpy(v, X + at, TAPS);
-            else load_tail<TAPS>(X, N, at, v);
-            unsigned sum = 0u;                                    // (the sum fits, whatever its parts run through)
+        for (int k = 0; k < 2 * TB; ++k) {
+            if (odd_codes(v[k]) != 0u) v[k] = plain_codes(v[k]);
 #pragma unroll
-            for (int k = 0; k < 2 * TB; ++k) {
-                if (odd_codes(v[k]) != 0u) v[k] = plain_codes(v[k]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) sum += (unsigned)(table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
-            }
-            return (float)(int)sum * __uint_as_float((unsigned)(127 + 128 - (int)(__float_as_uint(exponents) >> 24)) << 23);
-        };
-        float value = value_at(row, filter.w);
-        const bool unsure = open && filter.y > 0.0f && !((second + filter.z) * filter.y < value);     // (windows all alike: the first row)
-        const unsigned long long who = __ballot(unsure);
-        if (who != 0ull) {
-            // ---- too close to call: its place from all the digits, for the 32 filters concerned
-#pragma unroll 1
-            for (unsigned q = 0; q < 2; ++q) {
-                if ((unsigned)(who >> (32u * q)) == 0u) continue;
-                const unsigned expo = __float_as_uint(about[32u * q + (mine & 31u)].w);
-                const float2 all = region_maximum<TB, CLOSES>(X, N, ndef, a, b, entries, CLOSES ? D.digits + (size_t)(tile + q) * TILE_DIGITS : digits + q * TILE_DIGITS, shut + q * SHUT_BYTES<TB>,
-                                                      mine, (int)((expo >> 16) & 255u) - 128, expo & 255u);
-                const float oz = __shfl_xor(all.x, 32, 64);
-                const unsigned xi = __float_as_uint(all.y), oi = (unsigned)__shfl_xor((int)xi, 32, 64);
-                if (unsure && (mine >> 5) == q) row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
-            }
-            value = value_at(row, about[mine].w);
-            load_places(mine);                                    // (not held over the pass: its operands take their registers)
+            for (int j = 0; j < 4; ++j) sum += (unsigned)(table + ((v[k] >> (8 * j)) & 7u) * PAIR + mine)[(4 * k + j) * 8 * PAIR];
         }
-        value = open ? fmaxf(value + filter.x, 0.0f) : 0.0f;
+        return (float)(int)sum * __uint_as_float((unsigned)(127 + 128 - (int)(__float_as_uint(exponents) >> 24)) << 23);
+    };
+    // the place from all the digits, for the halves of `who`
+    auto place_again = [&](unsigned mine, unsigned long long who, bool unsure, unsigned row) -> unsigned {
+#pragma unroll 1
+        for (unsigned q = 0; q < 2; ++q) {
+            if ((unsigned)(who >> (32u * q)) == 0u) continue;
+            const unsigned expo = __float_as_uint(about[32u * q + (mine & 31u)].w);
+            const float2 all = region_maximum<TB, CLOSES>(X, N, ndef, a, b, entries, CLOSES ? D.digits + (size_t)(tile + q) * TILE_DIGITS : digits + q * TILE_DIGITS,
+                                                          shut + q * SHUT_BYTES<TB>, mine, (int)((expo >> 16) & 255u) - 128, expo & 255u,
+                                                          (unsigned)(who >> (32u * q)));
+            const float oz = __shfl_xor(all.x, 32, 64);
+            const unsigned xi = __float_as_uint(all.y), oi = (unsigned)__shfl_xor((int)xi, 32, 64);
+            if (unsure && (mine >> 5) == q) row = oz > all.x || (oz == all.x && oi < xi) ? oi : xi;
+        }
+        return row;
+    };
+    auto keep = [&](unsigned mine, float value, unsigned row) {
         const unsigned f = fbase + mine;
         if (f < F && (two || mine < FTILE)) {
             const size_t j = (size_t)r * F + f;
             pooled[j] = value;
             if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + (value > 0.0f ? row : 0u)) * F + f);   // nothing open: the first row
         }
+    };
+    auto next_region = [&]() {
         r = rn;
         a = (unsigned)__builtin_amdgcn_readfirstlane((int)an); b = (unsigned)__builtin_amdgcn_readfirstlane((int)bn);
         rn = claim(counter, lane);
         if (rn < hi) { an = R[2 * (size_t)rn]; bn = R[2 * (size_t)rn + 1]; }
+    };
+    while (r < hi) {
+        unsigned ties = 0u;                                           // regions in a row that were unsure in both halves
+        while (r < hi && ties < 2u) {
+            float m1[2] = {CLOSED, CLOSED}, m2[2] = {CLOSED, CLOSED}; // the two largest sums so far
+            unsigned t1[2] = {0u, 0u}, t = 0u;                        // the tile of the largest, the tile in work
+            unsigned c = a;
+            bool last;
+            do {
+                const unsigned left = b > c ? b - c : 0u;             // rows of the region from this stretch on
+                last = left <= CHUNK;
+                stage(entries, lane, letters);
+                // the next stretch's letters travel while this one is multiplied
+                if (!last) load12(X, N, c + CHUNK, lane, letters);
+                else if (rn < hi) load12(X, N, (unsigned)__builtin_amdgcn_readfirstlane((int)an), lane, letters);
+                const unsigned nrow = last ? left : CHUNK;
+                const unsigned defined = defined_rows(ndef, c);
+                const uint4* src = entries;
+                for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34, ++t) {
+                    uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
+                    if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
+                    const unsigned rest = left - t0;              // (rows of the region from this tile on)
+                    const int inside = (int)(rest < 64u ? rest : 64u) - 4 * (int)h;
+                    auto half = [&](auto second_half) {
+                        constexpr int q = decltype(second_half)::value;
+                        f32x16_t z;
+                        if constexpr (CLOSES)
+                            z = place_sums<TB>(closed_windows<TB, q>(rows, a0, a1, shut_here + q * SHUT_BYTES<TB>, shut_scales), a0, a1, B[q], single, pair);
+                        else
+                            z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
+                        if (rest < (unsigned)ROWS) {
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) z[i] = (i & 3) + 8 * (i >> 2) < inside ? z[i] : CLOSED;
+                        }
+                        top_two(z, m1[q], m2[q], t1[q], t);
+                    };
+                    half(std::integral_constant<int, 0>{});
+                    half(std::integral_constant<int, 1>{});
+                }
+                c += CHUNK;
+            } while (!last);
+            // ---- each filter's two half waves side by side: the largest sum, its place, the second largest
+            unsigned mine = lane;                                     // (opaque: addresses are formed from it here, not held in registers)
+            asm volatile("" : "+v"(mine));
+            swap_halves(m1[0], m1[1]);
+            swap_halves(m2[0], m2[1]);
+            swap_halves(t1[0], t1[1]);
+            const bool upper = m1[1] > m1[0];
+            const float best = fmaxf(m1[0], m1[1]), second = fmaxf(fminf(m1[0], m1[1]), fmaxf(m2[0], m2[1]));
+            const unsigned i = 15u - ((unsigned)(int)(best * 64.0f) & 15u);
+            unsigned row = (upper ? t1[1] : t1[0]) * ROWS + (upper ? 4u : 0u) + (i & 3u) + 8u * (i >> 2);
+            const float4 filter = about[mine];
+            // else every window's rectified value is zero (a region without rows has no best)
+            const bool open = best > CLOSED && (best + filter.z) * filter.y + filter.x > 0.0f;
+            // ---- its value from the weights
+            float value = value_at(mine, open, row, filter.w);
+            const bool unsure = open && filter.y > 0.0f && !((second + filter.z) * filter.y < value);     // (windows all alike: the first row)
+            const unsigned long long who = __ballot(unsure);
+            if (!CLOSES) ties = (unsigned)who != 0u && (unsigned)(who >> 32) != 0u ? ties + 1u : 0u;
+            if (who != 0ull) {
+                // ---- too close to call: its place from all the digits, for the 32 filters concerned
+                row = place_again(mine, who, unsure, row);
+                value = value_at(mine, open, row, about[mine].w);
+                load_places(mine);                                    // (not held over the pass: its operands take their registers)
+            }
+            keep(mine, open ? fmaxf(value + filter.x, 0.0f) : 0.0f, row);
+            next_region();
+        }
+        // ---- two regions in a row were unsure in both halves (sequences that repeat: their windows tie): the next ones go to all the
+        // digits at once, before the places are tried again
+        if (CLOSES) break;                                        // (beside those weights' products registers would spill)
+#pragma unroll 1
+        for (unsigned k = 0; k < AT_ONCE && r < hi; ++k) {
+            unsigned mine = lane;
+            asm volatile("" : "+v"(mine));
+            const bool open = b > a;
+            const unsigned row = place_again(mine, open ? ~0ull : 0ull, open, 0u);
+            const float4 filter = about[mine];
+            keep(mine, open ? fmaxf(value_at(mine, open, row, filter.w) + filter.x, 0.0f) : 0.0f, row);
+            next_region();
+        }
+        unsigned again = lane;
+        asm volatile("" : "+v"(again));
+        load_places(again);                                       // (not held meanwhile, on any path)
+        if (r < hi) load12(X, N, a, again, letters);
     }
 }
 

@@ -1587,6 +1587,40 @@ def test_bulk_scan_of_weights_beyond_most_others(ks, count, size, m, ptype):
     assert off(P) <= (2.0 * off(plain) if size > 1e3 else 6e-7)
 
 
+@pytest.mark.parametrize("m", [18, 24])
+def test_bulk_maxima_of_many_sequences_that_repeat(ks, m):
+    """Waves that meet one repeating sequence after the other scan the next ones with all the digits at once, and come back to the places
+    where others follow: whichever way a region went, its maximum and the first row that attains it are the same."""
+    rng = np.random.default_rng(m)
+    F = 64 * 256                                                          # (one workgroup of 12 waves per 64 filters)
+    seqs = []
+    for n in (60, 250, 40, 150):
+        repeats = len(seqs) in (60, 310 + 40)
+        for _ in range(n):
+            unit = rng.integers(0, 4, int(rng.integers(1, 40))).astype(np.uint8)
+            rows = int(rng.integers(80, 130))
+            seqs.append(np.resize(unit, rows) if repeats else rng.integers(0, 4, rows).astype(np.uint8))
+    from deepbind_amd import data
+    X, R = data.pack_ordinals(seqs, m - 1)
+    R[100, 1] = R[100, 0]                                                 # a region without rows among those that repeat
+    W = (rng.integers(-8, 9, (4 * m, F)) / 8.0).astype(np.float32)        # every sum is exact: ties are ties
+    W[:, 64:128:3] = (rng.standard_normal((4 * m, 22)) * 0.1).astype(np.float32)
+    b = (rng.integers(-8, 5, (1, F)) / 8.0).astype(np.float32)
+    Wd, bd, Xd, Rd = dev(W), dev(b), dev(X), dev(R)
+    P, I = ks.scanpool_fprop(Wd, bd, Xd, Rd, "max", want_argmax=True, path="kmer")
+    for _ in range(3):
+        again = ks.scanpool_fprop(Wd, bd, Xd, Rd, "max", want_argmax=True, path="kmer")
+        assert torch.equal(again[0], P) and torch.equal(again[1], I)
+    assert torch.equal(ks.scanpool_fprop(Wd, bd, Xd, Rd, "max", path="kmer")[0], P)
+    pick = np.concatenate([np.arange(60, 130), np.sort(rng.choice(np.arange(130, F), 60, replace=False))])
+    some = np.arange(len(R)) != 100
+    A, Pr, Ir = _chain_oracle(W[:, pick].astype(np.float64), b[:, pick].astype(np.float64), X, R[some], "max")
+    P, I = host(P)[some][:, pick], host(I)[some][:, pick]
+    exact = ~np.isin(pick, np.arange(64, 128, 3))
+    assert np.array_equal(P[:, exact], Pr[:, exact].astype(np.float32)) and np.abs(P - Pr).max() <= 1e-5
+    assert np.array_equal((I // F)[:, exact], (Ir // len(pick))[:, exact]) and np.array_equal(I % F, np.broadcast_to(pick, I.shape))
+
+
 def test_scanpool_auto_path_bulk(ks):
     """A batch large enough for the library to pick the table kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
