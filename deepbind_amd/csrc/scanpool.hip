@@ -875,7 +875,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
     for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) { sums[t][i] = 0.0f; counts[t][i] = 0.0f; }
-    float db = 0.0f, db_odd = 0.0f;                                // (every other region's apart: shorter chains round less)
+    double db = 0.0;                                               // (two registers: in float32 a second chain would take as many, and round)
     // A wave's regions are share, share + shares, ...: lane i holds the bounds of the i-th of 64 of them.
     const size_t step = shares;
     const unsigned nregion = N != 0 && share < P ? (unsigned)((P - share + step - 1) / step) : 0u;     // (without rows every region is empty)
@@ -992,8 +992,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
             }
             // ---- a region's end
             if (last) {
-                if (now.k & 1u) db_odd = __builtin_fmaf(g, (float)open, db_odd);
-                else db = __builtin_fmaf(g, (float)open, db);
+                db = __builtin_fma((double)g, (double)open, db);
                 open = 0u;
 #pragma unroll
                 for (int t = 0; t < NB; ++t)
@@ -1011,7 +1010,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
     }
     // ---- this wave's quarter of the slab: a filter's two columns side by side, register i's sums in lanes 0-15 and 32-47, register
     // i + 1's in the others. Register i holds letter i & 3 of tap 2 (i >> 2) + h of its block.
-    db += db_odd;
+    float bias_sum = (float)db;
     float* out = slabs + (size_t)share * stride;
     if (!DENSE) {                                                  // (a column per filter: this wave's half of its slab as it is)
 #pragma unroll
@@ -1021,7 +1020,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
                 const unsigned j = 8u * t + 2u * (i >> 2) + h;
                 if (j < m && f < F) out[(size_t)(4u * j + (i & 3)) * F + f] = sums[t][i];
             }
-        const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(db), __float_as_uint(db), false, false);
+        const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(bias_sum), __float_as_uint(bias_sum), false, false);
         if (h == 0u && f < F) out[(size_t)4 * m * F + f] = __uint_as_float(d32[0]) + __uint_as_float(d32[1]);
         return;
     }
@@ -1033,9 +1032,9 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
             const unsigned j = 8u * t + 2u * (i >> 2) + h;
             if (j < m && f < F) out[(size_t)(4u * j + (i & 3) + (peak ? 1u : 0u)) * F + f] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
         }
-    const auto d16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(db), __float_as_uint(db), false, false);
-    db = __uint_as_float(d16[0]) + __uint_as_float(d16[1]);
-    const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(db), __float_as_uint(db), false, false);
+    const auto d16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(bias_sum), __float_as_uint(bias_sum), false, false);
+    bias_sum = __uint_as_float(d16[0]) + __uint_as_float(d16[1]);
+    const auto d32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(bias_sum), __float_as_uint(bias_sum), false, false);
     if (lane < 16u && f < F) out[(size_t)4 * m * F + f] = __uint_as_float(d32[0]) + __uint_as_float(d32[1]);
 }
 
