@@ -750,6 +750,25 @@ def test_scanpool_bprop_counts_are_exact(ks, ptype, lengths, m, F):
     assert np.array_equal(host(dW), ref.astype(np.float32)) and np.array_equal(host(db)[0], G.sum(0).astype(np.float32))
 
 
+def test_scanpool_bprop_bias_sums_of_small_batches(ks):
+    """The bias gradient of max pooling over a small batch: float64 sums within a wave, then some 30 partial sums in float32."""
+    P, L, m, F = 256, 30, 24, 1440
+    off = []
+    for seed in range(4):
+        rng = np.random.default_rng(seed)
+        from deepbind_amd import data
+        X, R = data.pack_uniform_ordinals(rng.integers(0, 4, (P, L)).astype(np.uint8), m - 1)
+        W, b = dev((rng.standard_normal((4 * m, F)) * 0.1).astype(np.float32)), dev((rng.standard_normal((1, F)) * 0.05).astype(np.float32))
+        Xd, Rd = dev(X), dev(R)
+        pooled, amax = ks.scanpool_fprop(W, b, Xd, Rd, "max", want_argmax=True)
+        g = rng.standard_normal((P, F)).astype(np.float32)
+        dW, db = torch.zeros_like(W), torch.zeros_like(b)
+        ks.scanpool_bprop(W, b, Xd, Rd, "max", pooled, amax, dev(g), dW, db)
+        want = (g.astype(np.float64) * (host(pooled) > 0)).sum(axis=0)
+        off.append(np.linalg.norm(host(db).ravel() - want) / np.linalg.norm(want))
+    assert np.mean(off) < 7.5e-8, off                                     # (float32 sums within a wave: 7.9e-8 to 8.1e-8)
+
+
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("B,lo,hi,m,F", [(9, 0, 90, 25, 70), (600, 20, 70, 32, 16), (40, 100, 300, 31, 130), (3, 150, 400, 32, 64)])
 def test_scanpool_bprop_25_to_32_taps(ks, ptype, B, lo, hi, m, F):
