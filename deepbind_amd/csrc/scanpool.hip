@@ -800,8 +800,8 @@ __global__ __launch_bounds__(256) void scanpool_bprop_bits_kernel(unsigned m, un
 // counts by population counts, 10 instructions per (tap, letter) and chunk (us, kernel and reduction of its slabs, before / after):
 // 2048 regions of 90-200 rows x 128 filters, max + average, 32 taps 70 / 43, 24 taps 60 / 40, 8 taps 36 / 31; 20 000 x 101 x 256,
 // 24 taps 356 / 227; 128 x 101 x 64, 24 taps 26 / 16; 50 x 3000 x 64 339 / 34. Requesting a chunk's inputs in the step before,
-// with copies at its end, cost 15 to 25 % of that. Error of dW against float64 8.5e-8 (8.9e-8 before), of the bias 8.6e-8 (9.6e-8).
-// Maxima alone: 8.1e-8 and 8.8e-8 (8.1e-8 and 8.6e-8 in the bit kernel).
+// with copies at its end, cost 15 to 25 % of that. Error of dW against float64 8.5e-8 (8.9e-8 before), of the bias 7.1e-8 (8.6e-8),
+// a float64 sum per wave. Maxima alone: 8.1e-8 and 6.9e-8 (8.1e-8 and 7.9e-8 in the bit kernel).
 typedef int i32x8_t __attribute__((ext_vector_type(8)));
 // 32 bits as 32 values 0 or 0.5 of the 4-bit format
 __device__ __forceinline__ i32x8_t bits_as_halves(unsigned w)
@@ -875,7 +875,7 @@ __device__ __forceinline__ void scanpool_bprop_counts_body(const wg_t wg, unsign
     for (int t = 0; t < NB; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) { sums[t][i] = 0.0f; counts[t][i] = 0.0f; }
-    double db = 0.0;                                               // (two registers: in float32 a second chain would take as many, and round)
+    double db = 0.0;                                               // (the registers of two float32 chains, which round more)
     // A wave's regions are share, share + shares, ...: lane i holds the bounds of the i-th of 64 of them.
     const size_t step = shares;
     const unsigned nregion = N != 0 && share < P ? (unsigned)((P - share + step - 1) / step) : 0u;     // (without rows every region is empty)
@@ -1129,7 +1129,12 @@ inline unsigned counts_grid_x(unsigned mt, unsigned ftiles, size_t N, size_t P)
 // Of max pooling it takes small batches of short regions (one chunk each, so that no chunk is walked for nothing); a workgroup has two
 // shares of the regions there. us a call, bit kernel / this: 256 regions of 53 rows x 1440 filters of 24 taps 27 / 22, 171 x 512 17.2 / 15.7,
 // 171 x 64 15.8 / 14.7, 512 x 16 of 8 taps 14.4 / 13.8, 768 of 61 x 256 of 32 taps 26.2 / 22.7, 768 of 37 x 512 of 8 taps 17.0 / 16.9; 128 of 119 rows x 64 16.0 / 16.4, 2048 of 77 rows x 256 of 8 taps 20.8 / 25.7, 20 000 of 60 x 64 50 / 57.
-inline bool counts_takes_max(size_t N, size_t P) { return P <= 768 && N <= 64 * P; }
+// Few taps leave the bit kernel little to do per region: it keeps the calls of many regions x filters (512 regions of 52 rows x 1024 filters
+// of 8 taps 14.1 / 15.4, 768 x 1024 15.7 / 18.6, 768 x 256 12.2 / 12.9, 256 x 1024 13.1 / 11.8; 16 taps 768 x 1024 22.6 / 23.9, 500 x 1024 19.2 / 19.1).
+inline bool counts_takes_max(unsigned mt, unsigned ftiles, size_t N, size_t P)
+{
+    return P <= (mt == 8 ? 512u : 768u) && N <= 64 * P && (mt > 16 || P * ftiles <= (mt == 8 ? 4096u : 8192u));
+}
 inline unsigned counts_max_grid_x(unsigned mt, unsigned ftiles, size_t N, size_t P) { return (counts_grid_x(mt, ftiles, N, P) + 1) / 2; }
 // Max pooling goes through the bit kernel while the regions are short on average (it visits every 64-row chunk of a region to
 // find each filter's winning row; the sparse kernel goes straight to that row).
@@ -1320,7 +1325,7 @@ int launch_bprop_pt(hipStream_t st, const float* W, const float* bias, size_t m,
         DBK_LAUNCH_OK();
     }
     // with max+avg pooling the dense half carries the maxima along
-    const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P), max_counts = PT == DBK_PT_MAX && counts_takes_max(N, P);
+    const bool max_bits = PT == DBK_PT_MAX && bits_takes_max(N, P), max_counts = PT == DBK_PT_MAX && counts_takes_max(mt, ftiles, N, P);
     const unsigned gxs = PT == DBK_PT_MAX ? (max_counts ? 2 * counts_max_grid_x(mt, ftiles, N, P) : max_bits ? bits_grid_x(mt, ftiles, P) : sparse_grid_x(ftiles, P)) : 0u;
     const unsigned gxd = PT == DBK_PT_MAX ? 0u : act ? counts_grid_x(mt, ftiles, N, P) : dense_grid_x(mt, ftiles, P);
     const size_t smem_s = sparse_smem(m), smem_d = mt == 32 ? bits_smem(mt) : dense_smem(mt);
@@ -1547,7 +1552,7 @@ int scan_bprop_multi(hipStream_t st, size_t m, size_t N, const uint32_t* R, size
     for (unsigned i = 0; i < n; ++i) {
         a.ftiles[i] = dbk::divup(g[i].F, FT);
         // as the group's own launch would choose: the counting kernel, for max pooling the bit kernel or, over long regions, the sparse one
-        a.wide[i] = g[i].ptype != DBK_PT_MAX ? 1u : counts_takes_max(N, P) ? 2u : bits_takes_max(N, P) ? 1u : 0u;
+        a.wide[i] = g[i].ptype != DBK_PT_MAX ? 1u : counts_takes_max(mt, a.ftiles[i], N, P) ? 2u : bits_takes_max(N, P) ? 1u : 0u;
         a.gx[i] = g[i].ptype != DBK_PT_MAX ? counts_grid_x(mt, a.ftiles[i], N, P) : a.wide[i] == 2u ? counts_max_grid_x(mt, a.ftiles[i], N, P)
                 : a.wide[i] ? bits_grid_x(mt, a.ftiles[i], P) : sparse_grid_x(a.ftiles[i], P);
         a.first[i + 1] = a.first[i] + a.gx[i] * a.ftiles[i];
