@@ -116,8 +116,7 @@ __device__ __forceinline__ void split_digits(float (&x)[4], unsigned char* o)
             const int i = (int)d;
             const unsigned a = (unsigned)(i < 0 ? -i : i);
             // a / 8 in 1 + 2 + 3 bits: the numbers 0 .. 16 are their own codes (denormal below 8), 18 .. 32 17 .. 24
-            const unsigned code = a <= 16u ? a : 8u + (a >> 1);
-            word |= (code | (i < 0 ? 32u : 0u)) << (6 * c);
+            word |= ((a <= 16u ? a : 8u + (a >> 1)) | (i < 0 ? 32u : 0u)) << (6 * c);
         }
         unsigned char* q = o + (size_t)p * SLOT_BYTES;
         q[0] = (unsigned char)word; q[1] = (unsigned char)(word >> 8); q[2] = (unsigned char)(word >> 16);
@@ -126,148 +125,122 @@ __device__ __forceinline__ void split_digits(float (&x)[4], unsigned char* o)
 
 __device__ __forceinline__ int exponent_of(float v) { return (int)((__float_as_uint(v) >> 23) & 0xffu) - 127; }
 
-// A workgroup splits one tile's weights: thread (g, fl) takes taps g, 8 + g, .. of filter fl. Latency only (4m x 32 values).
+// A workgroup splits one tile's weights, a thread per tap and filter. Latency only (4m x 32 values): with a thread per eight taps, which it
+// was, 24 taps took 10 us.
 template <int TB>
-__global__ __launch_bounds__(256) void weight_digits_kernel(const float* __restrict__ W, const float* __restrict__ bias, unsigned m, unsigned F,
-                                                            unsigned f0, digit_store out)
+__global__ __launch_bounds__(256 * TB) void weight_digits_kernel(const float* __restrict__ W, const float* __restrict__ bias, unsigned m, unsigned F,
+                                                                 unsigned f0, digit_store out)
 {
-    __shared__ float red[8][8][FTILE];                            // sums and maxima of the eight threads of a filter
-    __shared__ unsigned char dig[TB * (NDIGIT + NTOP + 1) * SLOT_BYTES];
-    __shared__ unsigned tile;                                     // what is noted of its filters
-    const unsigned fl = threadIdx.x & 31u, g = threadIdx.x >> 5, f = f0 + blockIdx.x * FTILE + fl;
-    if (threadIdx.x == 0) tile = TILE_BULK;
-    float w[TB][4];
+    constexpr unsigned THREADS = 256 * TB, PARTS = 4 * TB;        // a filter's sums: a part per wave (two taps)
+    __shared__ float parts[3][PARTS][FTILE];
+    __shared__ unsigned most[4][FTILE], fewest[FTILE];            // maxima of numbers that are not negative, as their bits; a minimum
+    __shared__ __align__(16) unsigned char dig[TB * (NDIGIT + NTOP + 1) * SLOT_BYTES];
+    __shared__ unsigned tile, closing[FTILE];                     // what is noted of the tile's filters; which of them have closing weights
+    const unsigned fl = threadIdx.x & 31u, tap = threadIdx.x >> 5, wave = threadIdx.x >> 6, f = f0 + blockIdx.x * FTILE + fl;
+    if (threadIdx.x < FTILE) {
+        most[0][fl] = most[1][fl] = most[2][fl] = most[3][fl] = closing[fl] = 0u;
+        fewest[fl] = 0x7f000000u;
+        tile = TILE_BULK;
+    }
+    float w[4];
 #pragma unroll
-    for (int t = 0; t < TB; ++t)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const unsigned tap = 8u * t + g;
-            w[t][c] = (tap < m && f < F) ? W[(size_t)(4 * tap + c) * F + f] : 0.0f;
-        }
+    for (int c = 0; c < 4; ++c) w[c] = (tap < m && f < F) ? W[(size_t)(4 * tap + c) * F + f] : 0.0f;
     const float b = f < F ? bias[f] : 0.0f;
-    float open = 0.0f, top = 0.0f;                                // sum of the taps' best, the largest weight
     const unsigned bias_bits = __float_as_uint(b) & 0x7fffffffu;      // (the file is compiled without NaN: test the bits)
-    bool finite = bias_bits < 0x7f800000u, closing = false;           // closing: minus infinity among the weights
+    bool finite = bias_bits < 0x7f800000u, infinite = false;          // infinite: minus infinity among the weights
+    float best = 0.0f;
 #pragma unroll
-    for (int t = 0; t < TB; ++t) {
-        float best = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const unsigned bits = __float_as_uint(w[t][c]) & 0x7fffffffu;
-            finite &= bits < 0x7f800000u || __float_as_uint(w[t][c]) == 0xff800000u;
-            closing |= bits == 0x7f800000u;
-            best = fmaxf(best, w[t][c]);
-        }
-        top = fmaxf(top, best);
-        open += best;
+    for (int c = 0; c < 4; ++c) {
+        const unsigned bits = __float_as_uint(w[c]) & 0x7fffffffu;
+        finite &= bits < 0x7f800000u || __float_as_uint(w[c]) == 0xff800000u;
+        infinite |= bits == 0x7f800000u;
+        best = fmaxf(best, w[c]);
     }
-    red[0][g][fl] = open; red[1][g][fl] = top; red[2][g][fl] = (finite ? 0.0f : 1.0f) + (closing ? 64.0f : 0.0f);
+    // a filter's sum over its taps: the wave's two first, then the waves' in order
+    auto part = [&](int k, float v) { const float two = v + __shfl_xor(v, 32, 64); if ((tap & 1u) == 0u) parts[k][wave][fl] = two; };
+    auto sum = [&](int k) { float v = 0.0f; for (unsigned i = 0; i < PARTS; ++i) v += parts[k][i][fl]; return v; };
+    part(0, best);
     __syncthreads();
-    open = fmaxf(b, 0.0f); top = 0.0f;
-    float odd = 0.0f;
+    // ---- what a window and the bias come to at most; the weights that an open window can hold: all but those below -4.125 times that
+    const float open = sum(0) + fmaxf(b, 0.0f), lowest = -4.125f * open;
+    float largest = 0.0f, smallest = 3.0e38f, finer = 3.0e38f;     // of those: the tap's largest, smallest, smallest that is not zero
+    bool closes[4], any_closes = false;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        open += red[0][k][fl];
-        top = fmaxf(top, red[1][k][fl]);
-        odd += red[2][k][fl];
-    }
-    // ---- the weights that an open window can hold: all but those below -4.125 times the most that a window and the bias come to
-    const float lowest = -4.125f * open;
-    float mid = 0.0f, size = 0.0f;                                // of those: the largest magnitude, the sum over the taps of the largest,
-    float least = 0.0f, finest_weight = 3.0e38f;                  // the largest over the taps of the smallest, the smallest that is not zero
-    bool closed = false;
-#pragma unroll
-    for (int t = 0; t < TB; ++t) {
-        float most = 0.0f, few = 3.0e38f;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const float v = fabsf(w[t][c]);
-            if (w[t][c] < lowest) closed = true;
-            else {
-                most = fmaxf(most, v);
-                few = fminf(few, v);
-                if (v > 0.0f) finest_weight = fminf(finest_weight, v);
-            }
+    for (int c = 0; c < 4; ++c) {
+        const float v = fabsf(w[c]);
+        closes[c] = w[c] < lowest;
+        any_closes |= closes[c];
+        if (!closes[c]) {
+            largest = fmaxf(largest, v);
+            smallest = fminf(smallest, v);
+            if (v > 0.0f) finer = fminf(finer, v);
         }
-        mid = fmaxf(mid, most);
-        size += most;
-        if (few < 3.0e38f) least = fmaxf(least, few);
     }
-    red[3][g][fl] = mid; red[4][g][fl] = size; red[5][g][fl] = closed ? 1.0f : 0.0f; red[6][g][fl] = least; red[7][g][fl] = finest_weight;
+    part(1, largest);
+    atomicMax(&most[0][fl], __float_as_uint(largest));
+    atomicMax(&most[3][fl], __float_as_uint(best));
+    if (smallest < 3.0e38f) atomicMax(&most[1][fl], __float_as_uint(smallest));
+    if (finer < 1.0e38f) atomicMin(&fewest[fl], __float_as_uint(finer));
+    if (any_closes) atomicOr(&closing[fl], 1u);
+    if (!finite) atomicMax(&most[2][fl], 1u);
+    if (infinite) atomicOr(&tile, TILE_INFINITE);
     __syncthreads();
-    mid = 0.0f; size = 0.0f; least = fabsf(b);
-    float any = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        mid = fmaxf(mid, red[3][k][fl]);
-        size += red[4][k][fl];
-        any = fmaxf(any, red[5][k][fl]);
-        least = fmaxf(least, red[6][k][fl]);
-        finest_weight = fminf(finest_weight, red[7][k][fl]);
-    }
-    least = fmaxf(least, finest_weight);                          // every open window that is not zero holds a weight, or the bias, of this size
-    // ---- all the digits: x = w * 2^(3 - e), the largest weight below 16, the others that count below 32, one that closes its
-    // windows CLOSING, beyond `lowest`
+    const float mid = __uint_as_float(most[0][fl]), size = sum(1);
+    const bool any = closing[fl] != 0u;
+    // every open window that is not zero holds a weight, or the bias, of this size
+    const float least = fmaxf(fmaxf(fabsf(b), __uint_as_float(most[1][fl])), __uint_as_float(fewest[fl]));
     // ---- all the digits: x = w * 2^(3 - e), the largest weight below 16, the others that count below 32
-    const bool none = mid == 0.0f && !(any > 0.0f && open > 0.0f);    // every window's sum is zero, or closed with no bias to open it
-    int e = 0;
-    if (mid > 0.0f) e = exponent_of(top) > exponent_of(mid) - 1 ? exponent_of(top) : exponent_of(mid) - 1;
+    const bool none = mid == 0.0f && !(any && open > 0.0f);       // every window's sum is zero, or closed with no bias to open it
+    const int e_top = exponent_of(__uint_as_float(most[3][fl])), e_mid = exponent_of(mid) - 1;
+    int e = mid > 0.0f ? (e_top > e_mid ? e_top : e_mid) : 0;
     // sizes near the type's ends, where a weight's bf16 pieces or a sum may leave it, go with the infinite and undefined ones
-    const bool far = ((unsigned)odd & 63u) != 0u || bias_bits >= 0x71000000u || !(open < 1.0e30f) || !(mid < 1.0e30f) || (mid != 0.0f && mid < 1.0e-32f);
+    const bool far = most[2][fl] != 0u || bias_bits >= 0x71000000u || !(open < 1.0e30f) || !(mid < 1.0e30f) || (mid != 0.0f && mid < 1.0e-32f);
     // The sums of windows without the largest weights are rounded in the size of those all the same. Where all of a window's weights may be
     // below a 256th of the largest, the tile is left out. Measured, root mean square of the windows' relative error, 8 / 24 taps, two weights
     // for one letter at about that many times the others, letters without it (a float32 sum tap by tap 0.8e-7 / 1.7e-7): once 0.5e-7 / 0.6e-7,
     // 15 times 2.4e-7 / 1.6e-7, 30 4.2e-7 / 3.3e-7, 120 1.9e-7 / 2.5e-7, 240 3.6e-7 / 5.0e-7, 970 1.5e-6 / 1.9e-6, 15 000 2.4e-5 / 3.1e-5.
     const bool bad = far || e < -84 || (!none && open < 1.0e-25f) || (mid > 0.0f && __uint_as_float((unsigned)(127 + e - 8) << 23) > least);
-    const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (odd >= 64.0f ? TILE_INFINITE : TILE_BULK) | (any > 0.0f ? TILE_CLOSES : TILE_BULK);
-    if (notes != TILE_BULK) atomicOr(&tile, notes);
+    const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (any ? TILE_CLOSES : TILE_BULK);
+    if (tap == 0u && notes != TILE_BULK) atomicOr(&tile, notes);
     if (bad) e = 0;
     // The first ones by themselves: x = w / unit with a window's x at most 240 (so that its sum, in 1/1024, leaves room for a row's
     // number below it: see the scan) and a weight's at most 16.4
     const float scale = __uint_as_float((unsigned)(127 + 3 - e) << 23);
-    const float finest = bad || none ? 1.0f : fmaxf(fmaxf(size * (1.0f / 240.0f), mid * (1.0f / 16.4f)), fmaxf(any > 0.0f ? open * 0x1.0p-40f : 0.0f, 1.0e-30f));
+    const float finest = bad || none ? 1.0f : fmaxf(fmaxf(size * (1.0f / 240.0f), mid * (1.0f / 16.4f)), fmaxf(any ? open * 0x1.0p-40f : 0.0f, 1.0e-30f));
     const float per = 1.0f / finest;
-    float above = 0.0f;                                           // the most that the weights exceed those digits by, in units of the next digit
+    float x[4], y[4];
+    unsigned shut = 0u;                                           // 63: -7.5
 #pragma unroll
-    for (int t = 0; t < TB; ++t) {
-        float x[4], y[4];
-        unsigned shut = 0u;                                       // 63: -7.5
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const bool closes = w[t][c] < lowest;
-            x[c] = bad || closes ? 0.0f : w[t][c] * scale;
-            y[c] = bad || closes ? 0.0f : w[t][c] * per;
-            shut |= closes ? 63u << (6 * c) : 0u;
-        }
-        unsigned char* q = dig + ((size_t)(TB * (NDIGIT + NTOP) + t) * FTILE + fl) * 24u + 3u * g;
-        q[0] = (unsigned char)shut; q[1] = (unsigned char)(shut >> 8); q[2] = (unsigned char)(shut >> 16);
-        split_digits<NDIGIT>(x, dig + ((size_t)t * NDIGIT * FTILE + fl) * 24u + 3u * g);
-        split_digits<NTOP>(y, dig + ((size_t)(TB * NDIGIT + t * NTOP) * FTILE + fl) * 24u + 3u * g);
-        above += fmaxf(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])), 0.0f);     // (a letter that counts nothing exceeds nothing)
+    for (int c = 0; c < 4; ++c) {
+        x[c] = bad || closes[c] ? 0.0f : w[c] * scale;
+        y[c] = bad || closes[c] ? 0.0f : w[c] * per;
+        shut |= closes[c] ? 63u << (6 * c) : 0u;
     }
-    red[0][g][fl] = above;
+    const unsigned block = tap >> 3, at = fl * 24u + 3u * (tap & 7u);
+    split_digits<NDIGIT>(x, dig + block * NDIGIT * SLOT_BYTES + at);
+    split_digits<NTOP>(y, dig + (TB * NDIGIT + block * NTOP) * SLOT_BYTES + at);
+    unsigned char* q = dig + (TB * (NDIGIT + NTOP) + block) * SLOT_BYTES + at;
+    q[0] = (unsigned char)shut; q[1] = (unsigned char)(shut >> 8); q[2] = (unsigned char)(shut >> 16);
+    // the most that the weights exceed the first digits by, in units of the next digit (a letter that counts nothing exceeds nothing)
+    part(2, fmaxf(fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3])), 0.0f));
     __syncthreads();
-    const unsigned* src = reinterpret_cast<const unsigned*>(dig);
-    unsigned* dst = reinterpret_cast<unsigned*>(out.digits + (size_t)blockIdx.x * (TB * NDIGIT * SLOT_BYTES));
-    for (unsigned i = threadIdx.x; i < TB * NDIGIT * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
-    src += TB * NDIGIT * SLOT_BYTES / 4;
-    dst = reinterpret_cast<unsigned*>(out.top + (size_t)blockIdx.x * (TB * NTOP * SLOT_BYTES));
-    for (unsigned i = threadIdx.x; i < TB * NTOP * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
-    src += TB * NTOP * SLOT_BYTES / 4;
-    dst = reinterpret_cast<unsigned*>(out.shut + (size_t)blockIdx.x * (TB * SLOT_BYTES));
-    for (unsigned i = threadIdx.x; i < TB * SLOT_BYTES / 4; i += 256) dst[i] = src[i];
-    if (g == 0) {
-        above = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) above += red[0][k][fl];
+    const uint2* src = reinterpret_cast<const uint2*>(dig);
+    auto give = [&](unsigned char* to, unsigned digits) {
+        uint2* dst = reinterpret_cast<uint2*>(to + (size_t)blockIdx.x * (TB * digits * SLOT_BYTES));
+        for (unsigned i = threadIdx.x; i < TB * digits * SLOT_BYTES / 8; i += THREADS) dst[i] = src[i];
+        src += TB * digits * SLOT_BYTES / 8;
+    };
+    give(out.digits, NDIGIT);
+    give(out.top, NTOP);
+    give(out.shut, 1u);
+    if (tap == 0u) {
         out.expo[blockIdx.x * FTILE + fl] = e;
         digit_facts k;
         k.unit = none ? 0.0f : finest * (1.0f / 1024.0f);
-        // a quarter of a unit for the rows' numbers, a quarter for the rounding of a window's sum and of the scaled weights
-        // (sums of at most 240 * 1024 units, half a dozen roundings of 2^-24)
-        // and of all the digits' (below 1/32): a place that is sure is the one that all the digits find. A bias far above the weights makes the
-        // value coarse, by 2^-30 of it per tap.
-        k.above = above * (1.00001f / 32.0f) + 0.5f + (float)(8 * TB) * 0x1.0p-30f * (open * per * 1024.0f);
+        // a quarter of a unit for the rounding of a window's sum and of the scaled weights (sums of at most 240 * 1024 units, half a dozen
+        // roundings of 2^-24) and of all the digits' (below 1/32), so that a place that is sure is the one that all the digits find. A bias
+        // far above the weights makes the value coarse, by 2^-30 of it per tap. (The rows' numbers only raise the second sum.)
+        k.above = sum(2) * (1.00001f / 32.0f) + 0.25f + (float)(8 * TB) * 0x1.0p-30f * (open * per * 1024.0f);
         k.lowest = lowest;
         k.whole = open > 0.0f && !bad ? 29 - exponent_of(open) : 0;   // open < 2^(exponent + 1)
         k.shut = open > 0.0f && !bad ? (unsigned)(130 + exponent_of(open)) | (unsigned)(130 + exponent_of(open * per * 1024.0f)) << 8 : 127u | 127u << 8;
@@ -604,7 +577,8 @@ void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsig
 // tie in every filter: after two regions in a row that were unsure in both halves of its 64 filters a wave takes the next 15 to all the
 // digits at once. A place that is sure is the one that those find (`above` has their rounding in it), so that a result does not depend
 // on which regions a wave met before. Measured, 20 000 x 500 letters x 512 filters, ms, 24 / 32 taps: uniform letters 0.85 / 0.98, units of 7
-// letters that repeat 1.30 / 1.62 (every region twice 1.95 / 2.38; the table of 3-mer sums 1.35 / 2.7 whatever the letters).
+// letters that repeat 1.30 / 2.4 (25 to 32 taps scan every region twice, as 24 did in 1.95; the table of 3-mer sums 1.35 / 2.7 whatever
+// the letters).
 //
 // Sums of NTOP digits are whole numbers of 1/4 unit (a "mean of the four" counts quarters) below 2^18 units, which leaves
 // float32 four bits below: a lane's 16 rows start from 15/64 .. 0 units instead of zero, so the maximum carries its row's
@@ -745,6 +719,8 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
 {
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NI = place_count<TB>::N;
+    // (beside a fourth block of taps or the products of closing weights registers would spill: a repeating region costs both ways there)
+    constexpr bool DIRECT = TB == 3 && !CLOSES;
     constexpr unsigned TAPS = 8u * TB, TILE_DIGITS = TB * NDIGIT * SLOT_BYTES;
     const unsigned lane = threadIdx.x & 63u, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned col = lane & 31u, h = lane >> 5;
@@ -770,15 +746,14 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
         const bool in = tap < m && f < F && (two || fl < FTILE);
         const digit_facts k = D.facts[tile * FTILE + (in ? fl : 0u)];
         const float scale = __uint_as_float((unsigned)(127 + k.whole) << 23);
-        // (what 32 bits do not hold is in no open window)
-        auto held = [](long long v) -> int { return v > -0x7fffffffll ? (int)v : -0x7fffffff; };
-        long long w[4];
+        float w[4];                                               // (what 32 bits do not hold is in no open window)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) w[c] = in ? (long long)rintf(fmaxf(W[(size_t)(4 * tap + c) * F + f], k.lowest) * scale) : 0ll;
-        const int mean = held((w[0] + w[1] + w[2] + w[3] + 2) >> 2);
+        for (int c = 0; c < 4; ++c) w[c] = in ? rintf(fmaxf(W[(size_t)(4 * tap + c) * F + f], k.lowest) * scale) : 0.0f;
+        const double sum = ((double)w[0] + (double)w[1]) + ((double)w[2] + (double)w[3]);
+        const int mean = (int)rint(fmax(0.25 * sum, -2147483647.0));
         int* row = table + (size_t)tap * 8 * PAIR + fl;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) row[c * PAIR] = c < 4 ? held(w[c & 3]) : (c == 6 ? 0 : mean);      // codes mod 8: 254 is 6
+        for (int c = 0; c < 8; ++c) row[c * PAIR] = c < 4 ? (int)fmaxf(w[c & 3], -2147483520.0f) : (c == 6 ? 0 : mean);      // codes mod 8: 254 is 6
     }
     if (threadIdx.x < PAIR) {
         const unsigned f = fbase + threadIdx.x;
@@ -893,8 +868,13 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
                     auto half = [&](auto second_half) {
                         constexpr int q = decltype(second_half)::value;
                         f32x16_t z;
-                        if constexpr (CLOSES)
-                            z = place_sums<TB>(closed_windows<TB, q>(rows, a0, a1, shut_here + q * SHUT_BYTES<TB>, shut_scales), a0, a1, B[q], single, pair);
+                        if constexpr (CLOSES) {
+                            float zero = 0.0f;                    // (opaque: the rows' numbers are formed anew, for their registers)
+                            asm volatile("" : "+v"(zero));
+#pragma unroll
+                            for (int i = 0; i < 16; ++i) z[i] = zero + (float)(15 - i) * (1.0f / 64.0f);
+                            z = place_sums<TB>(closed_windows<TB, q>(z, a0, a1, shut_here + q * SHUT_BYTES<TB>, shut_scales), a0, a1, B[q], single, pair);
+                        }
                         else
                             z = place_sums<TB>(rows, a0, a1, B[q], single, pair);
                         if (rest < (unsigned)ROWS) {
@@ -925,11 +905,12 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
             float value = value_at(mine, open, row, filter.w);
             const bool unsure = open && filter.y > 0.0f && !((second + filter.z) * filter.y < value);     // (windows all alike: the first row)
             const unsigned long long who = __ballot(unsure);
-            if (!CLOSES) ties = (unsigned)who != 0u && (unsigned)(who >> 32) != 0u ? ties + 1u : 0u;
+            if (DIRECT) ties = (unsigned)who != 0u && (unsigned)(who >> 32) != 0u ? ties + 1u : 0u;
             if (who != 0ull) {
                 // ---- too close to call: its place from all the digits, for the 32 filters concerned
-                row = place_again(mine, who, unsure, row);
-                value = value_at(mine, open, row, about[mine].w);
+                const unsigned found = place_again(mine, who, unsure, row);
+                if (__any(found != row)) value = value_at(mine, open, found, about[mine].w);
+                row = found;
                 load_places(mine);                                    // (not held over the pass: its operands take their registers)
             }
             keep(mine, open ? fmaxf(value + filter.x, 0.0f) : 0.0f, row);
@@ -937,7 +918,7 @@ __device__ __forceinline__ void scanpool_digits_max_body(const digit_store& D, u
         }
         // ---- two regions in a row were unsure in both halves (sequences that repeat: their windows tie): the next ones go to all the
         // digits at once, before the places are tried again
-        if (CLOSES) break;                                        // (beside those weights' products registers would spill)
+        if (!DIRECT) break;
 #pragma unroll 1
         for (unsigned k = 0; k < AT_ONCE && r < hi; ++k) {
             unsigned mine = lane;
@@ -1016,7 +997,7 @@ int launch(hipStream_t st, const digit_store& D, const float* W, const float* bi
            const uint8_t* X, size_t N, const uint32_t* R, size_t P, int ptype, bool half, float* pooled, uint32_t* argmax)
 {
     const size_t ndef = N >= m ? N - m + 1 : 0;                    // rows the scan defines
-    hipLaunchKernelGGL(weight_digits_kernel<TB>, dim3(nflag), dim3(256), 0, st, W, bias, (unsigned)m, (unsigned)F, f0, D);
+    hipLaunchKernelGGL(weight_digits_kernel<TB>, dim3(nflag), dim3(256 * TB), 0, st, W, bias, (unsigned)m, (unsigned)F, f0, D);
     if constexpr (TB >= 3) {
         if (half)
             return argmax ? launch_max<true, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax)
