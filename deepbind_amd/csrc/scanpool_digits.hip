@@ -33,7 +33,8 @@
 // Bound: the matrix pipe, and through it the chip's power: an instruction takes its 34 clocks, at 1.5-1.6 GHz under this
 // load (2.3 GHz with all operands zero), 22 ns per SIMD. A table of 3-mer sums in LDS (one 4-byte read and add per three
 // taps), which this replaced, moved its 248 ns worth of LDS bytes per 32 x 32 tile of 24 taps; nine instructions are 198.
-// Measured, table / digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 11.1 ms; 65 536 x 101 x 256
+// Measured, table / all digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 10.4 ms (8.1 through half of the
+// products, scanpool_digits_max_kernel below); 65 536 x 101 x 256
 // filters, 24 taps 0.721 / 0.513, 16 taps 0.552 / 0.380; 20 000 x 500 x 256 x 8 taps 0.491 / 0.261; max + average, 20 000 x
 // 30-150 x 384 x 16 taps 0.275 / 0.215; with an argmax 65 536 x 101 x 256 x 24 taps 0.867 / 0.616; averages are off by
 // 5.6e-8 instead of 1.7e-7 (a tile's sum first, then the tiles').
@@ -1015,7 +1016,8 @@ int launch(hipStream_t st, const digit_store& D, const float* W, const float* bi
 // regions of 80 rows on average and eight of them per wave. Measured, all the products / half of them, 24 taps: 100 000 x
 // 500 letters x 1024 filters 10.4 / 8.1 ms, 65 536 x 101 x 256 0.515 / 0.461, 8192 x 101 x 256 0.080 / 0.078, 100 000 x 40 x
 // 64 0.134 / 0.137, 2000 x 500 x 64 0.034 / 0.049; 16 taps, 65 536 x 101 x 256 0.361 / 0.368. A caller who asks for this
-// path by name gets them whatever the number of regions: a region's result then does not depend on what is beside it.
+// path by name gets them whatever the number of regions; the regions' average length still decides, so a region's last bit may differ
+// between calls of short and of long company.
 bool half_the_products(size_t m, size_t F, size_t N, size_t P, int ptype, bool force)
 {
     if (ptype != DBK_PT_MAX || m <= 16 || F <= FTILE || N < 80 * P) return false;
@@ -1093,7 +1095,7 @@ int fprop(hipStream_t st, const float* W, const float* bias, size_t m, size_t F,
 // host code asks the runtime for the address once per device and passes that pointer to the kernels.
 // (24 taps: 1024 tiles' digits, 24.4 MB; flags of the 65 535 x 64 filters a launch may have, 0.5 MB)
 constexpr size_t STATIC_SCRATCH_BYTES = size_t(24) << 20;
-constexpr size_t STATIC_SEQUENCE_BYTES = (size_t(64) << 20) - 127; // sequence bytes a call may bring
+constexpr size_t STATIC_SEQUENCE_BYTES = (size_t(64) << 20) - 127; // sequence bytes a call may bring: the entry point's contract; the scratch does not depend on them
 static_assert(131070 * sizeof(unsigned) + 256 + PASS_TILES * (FTILE * (sizeof(int) + sizeof(digit_facts)) + 3 * (NDIGIT + NTOP + 1) * SLOT_BYTES) <= STATIC_SCRATCH_BYTES, "the largest call must fit");
 static __device__ __align__(256) unsigned char scratch[STATIC_SCRATCH_BYTES];
 static unsigned char* g_static_scratch[64] = {nullptr};

@@ -176,8 +176,9 @@ int dbk_scanpool_fprop_mfma(dbk_stream_t stream,
  * some 10^5 rows x filter tiles on, for filters of up to 32 taps): the scan as a product of the windows' one-hot letters
  * with the weights as six 6-bit digits each on the matrix cores, accumulated in float32 (v_mfma_scale_f32_32x32x64_f8f6f4).
  * Fails with NotImplementedError for shapes this entry point does not take (filter length > 24, sum pooling). Filters whose
- * weights the digits do not express (infinite or undefined ones, one positive weight far beyond all others) are detected
- * on the device and computed by the general kernel inside the same call. */
+ * weights the digits do not express (infinite or undefined ones, a few weights so far beyond the others that windows without them
+ * would lose their precision) are detected on the device, and their tiles of 64 filters computed by a launch of the general
+ * kernels inside the same call. */
 int dbk_scanpool_fprop_kmer(dbk_stream_t stream,
                             const float* W, const float* bias, size_t m, size_t nfilter,
                             const uint8_t* X, size_t N,
@@ -188,7 +189,8 @@ int dbk_scanpool_fprop_kmer(dbk_stream_t stream,
  * serving loops, harnesses that forbid allocation): same arguments, same kernels, same results, but the call's
  * scratch (the weights' digits) lies in a buffer that is part of the loaded
  * library instead of a grow-on-demand allocation, so the call never allocates, frees or synchronises.
- * Limit: N <= 64 MiB - 127 sequence bytes per call (ValueError beyond; the buffer's 24 MiB are held on every
+ * Limit: N <= 64 MiB - 127 sequence bytes per call (ValueError beyond: a limit of this entry point, which its scratch,
+ * sized by the filters alone, does not need; the buffer's 24 MiB are held on every
  * GPU the library runs on until the process ends). All calls on one GPU share the buffer: calls that overlap
  * on one GPU (different streams, different host threads) race; calls ordered on one stream do not.
  * No counterpart in the reference (its wrappers allocate per call, kangaroo/_ext/kangaroo_smat.py:121-132). */

@@ -1144,7 +1144,7 @@ def test_masks_dropout_and_loss_ops(ds, sm, ks):
     assert_close(host(sm.dot_tn(dev(X), dev(X))), X.T.astype(np.float64) @ X.astype(np.float64), ACT, "dot_tn")
 
 
-# ------------------------------------------------------------------------------------------ k-mer table fast path
+# ------------------------------------------------------------------------------------------ bulk path
 @pytest.mark.parametrize("B,lo,hi,m,F", [(64, 101, 101, 24, 16), (128, 38, 41, 16, 16), (300, 20, 40, 24, 144), (33, 1, 300, 11, 70),
                                           (50, 500, 500, 24, 64), (17, 0, 9, 5, 33), (700, 30, 60, 20, 40), (40, 90, 110, 2, 8),
                                           (1, 50, 50, 24, 32), (49, 10, 80, 24, 32)])
@@ -1160,7 +1160,7 @@ def test_scanpool_kmer_path_matches_oracle(ks, B, lo, hi, m, F):
 
 
 def test_scanpool_kmer_path_repeats_its_bits(ks):
-    """The table kernel's streams take regions as they become free, so which stream scans a region differs from call to
+    """The bulk kernel's waves take regions as they become free, so which stream scans a region differs from call to
     call; every region's result must not (same additions in the same order whoever performs them)."""
     rng, W, b, X, R = _fused_case(515, 3000, 5, 200, 24, 96, pn=0.03)
     Wd, bd, Xd, Rd = dev(W), dev(b), dev(X), dev(R)
@@ -1172,8 +1172,8 @@ def test_scanpool_kmer_path_repeats_its_bits(ks):
 
 
 def test_scanpool_kmer_path_device_side_fallbacks(ks):
-    """Code 254 and regions past the scan's last row cannot be expressed in the table: the call must
-    still return the right answer (the general kernel runs behind a device flag)."""
+    """Code 254 and regions past the scan's last row, which the bulk kernel takes itself (tiles that it leaves out:
+    test_bulk_scan_beside_tiles_that_are_left_out and those after it); more taps than the entry point takes are refused."""
     rng, W, b, X, R = _fused_case(4242, 60, 30, 50, 24, 48, pn=0.03, p254=0.02)
     assert (X == 254).any()
     A, Pr, _ = _chain_oracle(W, b, X, R, "max")
@@ -1192,14 +1192,13 @@ def test_scanpool_kmer_path_device_side_fallbacks(ks):
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("B,lo,hi,m,F", [(200, 101, 101, 24, 64), (150, 30, 60, 16, 40), (60, 1, 30, 24, 33), (90, 40, 90, 7, 32)])
 def test_scanpool_kmer_path_pooling_variants_and_argmax(ks, ptype, B, lo, hi, m, F):
-    """The table kernel's average / max+average pooling and its argmax (winning triple of positions, settled
-    exactly at the region's end) against the oracle, with the general kernel as a second opinion."""
+    """The bulk kernel's average / max+average pooling and its argmax against the oracle, with the general kernel as a second opinion."""
     rng, W, b, X, R = _fused_case(7000 + B + m + F, B, lo, hi, m, F, pn=0.04)
     b = b - 0.05                                                    # some filters never fire in some regions: argmax = first row
     A, Pr, Ir = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
     want = ptype != "avg"
     P, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=want, path="kmer")
-    assert_close(host(P), Pr, ACT, "pooled (%s, table kernel)" % ptype)
+    assert_close(host(P), Pr, ACT, "pooled (%s, bulk kernel)" % ptype)
     Pg, Ig = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=want, path="general")
     assert_close(host(P), host(Pg), ACT, "table vs general")
     if want:
@@ -1641,7 +1640,7 @@ def test_bulk_maxima_of_many_sequences_that_repeat(ks, m):
 
 
 def test_scanpool_auto_path_bulk(ks):
-    """A batch large enough for the library to pick the table kernel by itself."""
+    """A batch large enough for the library to pick the bulk kernel by itself."""
     rng, W, b, X, R = _fused_case(99, 2500, 100, 100, 24, 256, pn=0.01)
     P, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max")
     Pg, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), "max", path="general")
@@ -1654,7 +1653,7 @@ def test_scanpool_auto_path_bulk(ks):
 @pytest.mark.parametrize("B,lo,hi,m,F", [(200, 101, 101, 24, 64), (150, 30, 60, 16, 40), (77, 24, 24, 24, 16), (500, 1, 5, 24, 32),
                                           (300, 60, 200, 16, 64), (100, 500, 500, 12, 32), (400, 40, 70, 5, 16), (64, 101, 101, 18, 96)])
 def test_scanpool_kmer_regions_in_any_order(ks, B, lo, hi, m, F):
-    """Regions need not be sorted or contiguous for the table kernel: shuffling the region table
+    """Regions need not be sorted or contiguous for the bulk kernel: shuffling the region table
     permutes the output rows and nothing else - not a bit. (With filters of up to 18 taps a stream walks through regions
     that follow each other in the text without a fresh start and splits the block in which one ends between the two;
     shuffled, every region gets a fresh start: the two ways must agree exactly.)"""
@@ -1671,7 +1670,7 @@ def test_scanpool_kmer_regions_in_any_order(ks, B, lo, hi, m, F):
 @pytest.mark.parametrize("B,lo,hi,m", [(4000, 20, 60, 16), (13000, 5, 30, 11), (4000, 20, 60, 24), (13000, 1, 40, 20), (5000, 30, 30, 24),
                                         (4500, 101, 101, 18)])
 def test_scanpool_kmer_walks_on_through_regions_at_bulk_sizes(ks, B, lo, hi, m):
-    """Enough regions per workgroup (1 024 filters: eight workgroups per tile) that every stream of the table kernel
+    """Enough regions per workgroup (1 024 filters: eight workgroups per tile) that every wave of the bulk kernel
     claims several regions at a time and goes on from one into the next where they follow each other in the text (runs
     of up to eight with at most 18 taps, pairs with 19-24 and for average pooling): the packed table, the same with a third of the regions
     dropped (runs and pairs break off, second halves of claims are scanned alone), with regions cut in two that touch,
@@ -1699,7 +1698,7 @@ def test_scanpool_kmer_walks_on_through_regions_at_bulk_sizes(ks, B, lo, hi, m):
             assert torch.equal(P, Pagain), "two calls, different bits (%s)" % name
         pick = np.sort(rng.choice(len(Rt), 40, replace=False))
         Pr, _ = oracle_c.scanpool(W, b, X, np.ascontiguousarray(Rt[pick]), 0)
-        assert_close(host(P)[pick], Pr, ACT, "table kernel vs C oracle, %s" % name)
+        assert_close(host(P)[pick], Pr, ACT, "bulk kernel vs C oracle, %s" % name)
         perm = rng.permutation(len(Rt))
         P2, _ = ks.scanpool_fprop(Wd, bd, Xd, dev(np.ascontiguousarray(Rt[perm])), "max", path="kmer")
         assert np.array_equal(host(P2), host(P)[perm]), "a region's result depends on its neighbours in the region table (%s)" % name
@@ -1790,7 +1789,7 @@ def test_scanpool_extreme_shapes(ks, ptype):
     assert same.mean() > 0.999                                       # the rest are float32 round-off ties between rows
     if ptype == "max":
         Pk, _ = ks.scanpool_fprop(Wd, bd, Xd, Rd, "max", path="kmer")
-        assert_close(host(Pk), Pr, ACT, "pooled (table kernel)")
+        assert_close(host(Pk), Pr, ACT, "pooled (bulk kernel)")
     # backward: linear in dpooled, so two calls with g and 2g must give dW2 = 2 dW1 (bit-exact) and run-to-run identical
     dP = dev(rng.standard_normal(Pr.shape).astype(np.float32))
     outs = []
@@ -1804,7 +1803,7 @@ def test_scanpool_extreme_shapes(ks, ptype):
 
 
 def test_config5_full_size_against_subsampled_checkers(ks, ds):
-    """The full bulk-scoring workload (100 000 x 500 nt, 1024 filters): rows of the table kernel's result are
+    """The full bulk-scoring workload (100 000 x 500 nt, 1024 filters): rows of the bulk kernel's result are
     checked against the general kernel and the plain-C oracle run on random subsets of the regions (same
     packed stream, region table subsampled), and a permuted region table must permute the rows and nothing else."""
     from deepbind_amd import synth
@@ -1819,14 +1818,14 @@ def test_config5_full_size_against_subsampled_checkers(ks, ds):
     Rs = np.ascontiguousarray(cfg["R"][pick])
     Pg, _ = ks.scanpool_fprop(W, b, X, dev(Rs), "max", path="general")
     sub = host(P[torch.as_tensor(pick, device="cuda")])
-    assert_close(sub, host(Pg), ACT, "table kernel vs general kernel on 1500 regions")
+    assert_close(sub, host(Pg), ACT, "bulk kernel vs general kernel on 1500 regions")
     few = pick[:120]
     Pc, _ = oracle_c.scanpool(p["Wc"], p["bc"], cfg["X"], np.ascontiguousarray(cfg["R"][few]), 0)
-    assert_close(sub[:120], Pc, ACT, "table kernel vs C oracle on 120 regions")
+    assert_close(sub[:120], Pc, ACT, "bulk kernel vs C oracle on 120 regions")
     perm = rng.permutation(100000)
     Pp, _ = ks.scanpool_fprop(W, b, X, dev(np.ascontiguousarray(cfg["R"][perm])), "max")
     assert torch.equal(Pp, P[torch.as_tensor(perm, device="cuda")])
-    # the pooling winners of the table kernel against the float32 evaluation in reference order (the plain-C oracle):
+    # the pooling winners of the bulk kernel against the float32 evaluation in reference order (the plain-C oracle):
     # at full size row * 1024 + filter does not fit the reference's 32-bit index, so the 120 regions are repacked as
     # a stream of their own (each region starts with its padding: every window reads the same letters as before)
     def repack(which):

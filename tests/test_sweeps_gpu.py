@@ -84,7 +84,7 @@ def _region_variant(rng, R, variant):
 
 def test_table_kernel_against_the_general_kernel_over_random_shapes(ks):
     """1-24 taps, any pooling, with and without argmax, empty regions included (their average is 0/0 on both paths):
-    the table kernel agrees with the general kernel, and the same regions in another order give the same bits."""
+    the bulk kernel agrees with the general kernel, and the same regions in another order give the same bits."""
     bad = []
     for case in range(120):
         rng = np.random.default_rng(100000 + case)

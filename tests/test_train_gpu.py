@@ -652,7 +652,7 @@ def test_gradcheck_float64_layer_by_layer(pool, hidden, loss, mode):
 
 @pytest.mark.parametrize("pool", ["max", "all"])
 def test_bulk_batch_training_step_uses_the_table_kernel_and_matches_layer_by_layer(pool):
-    """A batch large enough for the fused forward to pick the table kernel (with argmax for the backward pass):
+    """A batch large enough for the fused forward to pick the bulk kernel (with argmax for the backward pass):
     one training step must agree with the layer-by-layer drop-in operators, and be bit-stable."""
     from deepbind_amd import data
     from deepbind_amd.model import SequenceNet

@@ -1,4 +1,4 @@
-"""The allocation-free entry point of the table kernel (scratch built into the library) against the ordinary one."""
+"""The allocation-free entry point of the bulk kernel (scratch built into the library) against the ordinary one."""
 import numpy as np
 import pytest
 import torch
@@ -21,7 +21,7 @@ def test_static_scratch_entry_point_matches_the_allocating_one_on_consecutive_ca
     W = dev((rng.standard_normal((4 * m, F)) * 0.3).astype(np.float32))
     b = dev((rng.standard_normal((1, F)) * 0.1).astype(np.float32))
     # two calls in a row, the second over a smaller batch (the shared buffer still holds the first call's bytes),
-    # then one whose input makes the table kernel stand down (code 254) and one with avg pooling
+    # then one with code 254 among the letters and one with avg pooling
     cases = [(300, 200, "max", True, 0.0), (40, 57, "max", True, 0.0), (64, 101, "all", True, 0.0), (50, 80, "max", False, 0.01),
              (30, 61, "avg", False, 0.0)]
     for nseq, L, ptype, want_argmax, p254 in cases:
