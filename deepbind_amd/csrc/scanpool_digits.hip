@@ -20,7 +20,7 @@
 // with it the sums: an instruction adds to a float32 with the precision of its largest operands, as they would be with a
 // first digit in every place): tiles that have them take one more product per 16 taps, -7.5 times a power of two above T in the
 // place of every such weight. Filters that fixed point does not express well (an
-// infinite or undefined weight, windows that may hold nothing but weights below a 256th of the largest) are left to a launch behind
+// infinite or undefined weight, windows that may hold nothing but weights below a 256th to a 512th of the largest) are left to a launch behind
 // this one (scanpool_fprop_left_kernel), which does nothing where no tile of filters asks for it.
 //
 // Mapping: a workgroup of 16 waves (one per CU) owns 32 filters, whose digits stay in its registers (24 taps: 9
@@ -197,9 +197,11 @@ __global__ __launch_bounds__(256 * TB) void weight_digits_kernel(const float* __
     // sizes near the type's ends, where a weight's bf16 pieces or a sum may leave it, go with the infinite and undefined ones
     const bool far = most[2][fl] != 0u || bias_bits >= 0x71000000u || !(open < 1.0e30f) || !(mid < 1.0e30f) || (mid != 0.0f && mid < 1.0e-32f);
     // The sums of windows without the largest weights are rounded in the size of those all the same. Where all of a window's weights may be
-    // below a 256th of the largest, the tile is left out. Measured, root mean square of the windows' relative error, 8 / 24 taps, two weights
+    // below 2^(e - 8), that is a 256th to a 512th of the largest (a 1024th of negative ones), the tile is left out. Measured, root mean square of the windows' relative error, 8 / 24 taps, two weights
     // for one letter at about that many times the others, letters without it (a float32 sum tap by tap 0.8e-7 / 1.7e-7): once 0.5e-7 / 0.6e-7,
-    // 15 times 2.4e-7 / 1.6e-7, 30 4.2e-7 / 3.3e-7, 120 1.9e-7 / 2.5e-7, 240 3.6e-7 / 5.0e-7, 970 1.5e-6 / 1.9e-6, 15 000 2.4e-5 / 3.1e-5.
+    // 15 times 2.4e-7 / 1.6e-7, 30 4.2e-7 / 3.3e-7, 120 1.9e-7 / 2.5e-7, 240 3.6e-7 / 5.0e-7, 970 1.5e-6 / 1.9e-6, 15 000 2.4e-5 / 3.1e-5. Worst of 600 random sets of
+    // weights of fifteen kinds that the digits keep: 8.2e-7 (3 taps, heavy tails), a single window 1.2e-5 (20 taps, large negative weights that do not
+    // close; its value a small difference, float32 4e-6).
     const bool bad = far || e < -84 || (!none && open < 1.0e-25f) || (mid > 0.0f && __uint_as_float((unsigned)(127 + e - 8) << 23) > least);
     const unsigned notes = (far ? TILE_NOT_FINITE : bad ? TILE_LEFT : TILE_BULK) | (any ? TILE_CLOSES : TILE_BULK);
     if (tap == 0u && notes != TILE_BULK) atomicOr(&tile, notes);
