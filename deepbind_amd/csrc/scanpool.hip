@@ -1242,7 +1242,8 @@ int launch_fprop_left_ks(hipStream_t st, const float* W, const float* bias, size
     const unsigned ftiles = dbk::divup(F, FT);
     const size_t smem = std::max(MFMA_SMEM, fprop_smem(left_lookup_taps(KS), m)), items = ftiles * P;
     const unsigned grid = std::max(ftiles, items < 768 ? (unsigned)items : 768u);   // three workgroups per CU are resident
-    auto kern = argmax && PT != DBK_PT_AVG ? scanpool_fprop_left_kernel<PT, PT != DBK_PT_AVG, KS> : scanpool_fprop_left_kernel<PT, false, KS>;
+    constexpr bool ARG = PT != DBK_PT_AVG && KS < 8;               // (the bulk kernel takes more than 24 taps without an argmax only)
+    auto kern = ARG && argmax ? scanpool_fprop_left_kernel<PT, ARG, KS> : scanpool_fprop_left_kernel<PT, false, KS>;
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), smem, st, W, bias, (unsigned)m, (unsigned)F, X, N, R, P, pooled, argmax, flags, ftiles);
     DBK_LAUNCH_OK();

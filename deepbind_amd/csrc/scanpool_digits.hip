@@ -999,19 +999,20 @@ template <int TB>
 int launch(hipStream_t st, const digit_store& D, const float* W, const float* bias, unsigned f0, unsigned ntile, unsigned nflag, size_t m, size_t F,
            const uint8_t* X, size_t N, const uint32_t* R, size_t P, int ptype, bool half, float* pooled, uint32_t* argmax)
 {
+    constexpr bool ARG = TB < 4;                                   // (filters of more than 24 taps come without an argmax)
     const size_t ndef = N >= m ? N - m + 1 : 0;                    // rows the scan defines
     hipLaunchKernelGGL(weight_digits_kernel<TB>, dim3(nflag), dim3(256 * TB), 0, st, W, bias, (unsigned)m, (unsigned)F, f0, D);
     if constexpr (TB >= 3) {
         if (half)
-            return argmax ? launch_max<true, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax)
-                          : launch_max<false, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax);
+            return ARG && argmax ? launch_max<ARG, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax)
+                                 : launch_max<false, TB>(st, D, W, bias, f0, ntile, m, F, X, N, ndef, R, P, pooled, argmax);
     }
     if (ptype == DBK_PT_AVG) return launch_pt<DBK_PT_AVG, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
     if (ptype == DBK_PT_MAX)
-        return argmax ? launch_pt<DBK_PT_MAX, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
-                      : launch_pt<DBK_PT_MAX, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
-    return argmax ? launch_pt<DBK_PT_ALL, true, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
-                  : launch_pt<DBK_PT_ALL, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+        return ARG && argmax ? launch_pt<DBK_PT_MAX, ARG, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
+                             : launch_pt<DBK_PT_MAX, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+    return ARG && argmax ? launch_pt<DBK_PT_ALL, ARG, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax)
+                         : launch_pt<DBK_PT_ALL, false, TB>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
 }
 
 // Whether plain maxima go through half the products: filters of more than 16 taps, more than 32 of them (a wave takes 64),
