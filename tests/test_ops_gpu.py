@@ -1582,6 +1582,24 @@ def test_bulk_scan_of_filters_that_forbid_letters_is_as_close_as_float32(ks, m, 
 
 
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [4, 16, 24])
+@pytest.mark.parametrize("size,bias", [(1e-24, 0.0), (1e28, 0.0), (1e-20, 1e25), (1e-20, -1e25), (1e-12, 1e-3), (1e20, 1e-20), (1.0, -1e29)])
+def test_bulk_scan_of_weights_and_biases_of_any_size(ks, size, bias, m, ptype):
+    """Rectified sums are formed in units of a power of two above what an open window and the bias come to, from either end of the type's
+    range, and beside a bias that is far above or below the weights. (Filters of which nothing is open: every value is zero.)"""
+    F = 70
+    rng, W, b, X, R = _bulk_case(140 + m, [300, 1, 33, 224, 500, 64], m, F)
+    W = (W * np.float32(size)).astype(np.float32)
+    b = (b * np.float32(size) + np.float32(bias) * (1.0 + np.abs(b))).astype(np.float32)
+    W[:, 5] = -np.abs(W[:, 5])
+    W[:, 40] = 0.0
+    P = host(ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")[0])
+    want = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)[1]
+    _within_rounding(P, want, W, b, ptype)
+    assert np.all(P[want == 0.0] == 0.0)
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("m", [5, 8, 16, 24])
 @pytest.mark.parametrize("count,size", [(1, 1e4), (2, 20.0), (2, 150.0), (2, 1e4), (3, 1e6)])
 def test_bulk_scan_of_weights_beyond_most_others(ks, count, size, m, ptype):
