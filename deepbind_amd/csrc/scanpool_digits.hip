@@ -23,8 +23,8 @@
 // infinite or undefined weight, windows that may hold nothing but weights below a 256th to a 512th of the largest) are left to a launch behind
 // this one (scanpool_fprop_left_kernel), which does nothing where no tile of filters asks for it.
 //
-// Mapping: a workgroup of 16 waves (one per CU) owns 32 filters, whose digits stay in its registers (24 taps: 9
-// instructions' operands, 54 registers a lane). A wave takes a region at a time from the workgroup's counter and walks it
+// Mapping: a workgroup of 16 waves (one per CU) owns 32 filters, up to 16 taps one of 12 waves 64 of them; their digits stay in its registers
+// (24 taps: 9 instructions' operands, 54 registers a lane). A wave takes a region at a time from the workgroup's counter and walks it
 // in tiles of 32 positions. 224 positions' letters at a time become one 16-byte entry per position in the wave's own
 // LDS: the one-hot nibbles of the eight letters from there on, which is half of an instruction's operand (lanes 0-31
 // take taps 0-7, lanes 32-63 taps 8-15), so a tile costs one or two 16-byte reads per lane. An entry's place is
@@ -36,7 +36,7 @@
 // Measured, table / all digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 10.4 ms (8.1 through half of the
 // products, scanpool_digits_max_kernel below); 65 536 x 101 x 256
 // filters, 24 taps 0.721 / 0.513, 16 taps 0.552 / 0.380; 20 000 x 500 x 256 x 8 taps 0.491 / 0.261; max + average, 20 000 x
-// 30-150 x 384 x 16 taps 0.275 / 0.215; with an argmax 65 536 x 101 x 256 x 24 taps 0.867 / 0.616; averages are off by
+// 30-150 x 384 x 16 taps 0.275 / 0.215 (0.19 now: launch_sets, scanpool_digits_body); with an argmax 65 536 x 101 x 256 x 24 taps 0.867 / 0.616; averages are off by
 // 5.6e-8 instead of 1.7e-7 (a tile's sum first, then the tiles').
 //
 // Reference chain being fused: kangaroo/_ext/corr1ord.py:97-117 -> deepity/std/elemwise.py:162-180,71-82
@@ -398,18 +398,22 @@ __device__ __forceinline__ void load_operands(const unsigned char* digits, unsig
     }
 }
 
-template <int TB, int I>
-__device__ __forceinline__ void products(f32x16_t& acc, const uint4& a0, const uint4& a1, const unsigned (&B)[product_count<TB>::N][6], const int (&s)[3])
+// A tile's products with NT sets of filters, which take turns.
+template <int TB, int NT, int I>
+__device__ __forceinline__ void products(f32x16_t (&z)[NT], const uint4& a0, const uint4& a1, const unsigned (&B)[NT][product_count<TB>::N][6], const int (&s)[NT][3])
 {
     if constexpr (I < product_count<TB>::N) {
-        if constexpr (TB == 1) acc = product<2 - I>(a0, B[I], acc, s[2]);
-        else if constexpr (TB == 2) { constexpr int p = 5 - I; acc = product<(p & 3)>(a0, B[I], acc, s[p >> 2]); }
-        else if constexpr (TB == 3) {
-            constexpr int j = 2 - I / 3, k = I % 3, p = 2 * j + 1 - k;
-            if constexpr (k < 2) acc = product<(p & 3)>(a0, B[I], acc, s[p >> 2]);
-            else acc = product<j>(a1, B[I], acc, s[2]);
-        } else { constexpr int p = 5 - I / 2; acc = product<(p & 3)>(I & 1 ? a1 : a0, B[I], acc, s[p >> 2]); }
-        products<TB, I + 1>(acc, a0, a1, B, s);
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+            if constexpr (TB == 1) z[q] = product<2 - I>(a0, B[q][I], z[q], s[q][2]);
+            else if constexpr (TB == 2) { constexpr int p = 5 - I; z[q] = product<(p & 3)>(a0, B[q][I], z[q], s[q][p >> 2]); }
+            else if constexpr (TB == 3) {
+                constexpr int j = 2 - I / 3, k = I % 3, p = 2 * j + 1 - k;
+                if constexpr (k < 2) z[q] = product<(p & 3)>(a0, B[q][I], z[q], s[q][p >> 2]);
+                else z[q] = product<j>(a1, B[q][I], z[q], s[q][2]);
+            } else { constexpr int p = 5 - I / 2; z[q] = product<(p & 3)>(I & 1 ? a1 : a0, B[q][I], z[q], s[q][p >> 2]); }
+        }
+        products<TB, NT, I + 1>(z, a0, a1, B, s);
     }
 }
 
@@ -447,9 +451,27 @@ __device__ __forceinline__ bool left_out(const unsigned* __restrict__ flags, uns
 // a row's rectified sum and bias, both below one half in magnitude where it is not zero: one addition that clamps
 __device__ __forceinline__ float open_part(float z, float b) { return __builtin_amdgcn_fmed3f(z + b, 0.0f, 1.0f); }
 
+// Lanes 0-31 of x beside lanes 0-31 of y, and lanes 32-63 of x beside lanes 32-63 of y: (x, y) becomes what the low and the
+// high half wave held of the first value (in lanes 0-31) and of the second (in lanes 32-63).
+__device__ __forceinline__ void swap_halves(unsigned& x, unsigned& y)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    x = r[0];
+    y = r[1];
+}
+__device__ __forceinline__ void swap_halves(float& x, float& y)
+{
+    unsigned a = __float_as_uint(x), b = __float_as_uint(y);
+    swap_halves(a, b);
+    x = __uint_as_float(a);
+    y = __uint_as_float(b);
+}
+
 // ---------------------------------------------------------------------------------------------- the scan
 // CLOSES: some of the tile's filters have weights that close windows. (Two bodies, so that the products of those take no registers in the other.)
-template <int PT, bool WANT_ARGMAX, int TB, bool CLOSES>
+// NT: sets of 32 filters that a wave takes (a workgroup of 16 waves: one, of 12: two, see takes_two).
+template <int NT> constexpr int WAVES = NT == 2 ? 12 : NWAVE;
+template <int PT, bool WANT_ARGMAX, int TB, int NT, bool CLOSES>
 __device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsigned tile, unsigned split, const float* __restrict__ bias, unsigned f0, unsigned F,
                                                      const uint8_t* __restrict__ X, size_t N, size_t ndef, const uint32_t* __restrict__ R, unsigned P,
                                                      unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
@@ -460,22 +482,31 @@ __device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsig
     const unsigned col = lane & 31u, h = lane >> 5;
     unsigned* counter = reinterpret_cast<unsigned*>(smem);
     uint4* entries = reinterpret_cast<uint4*>(smem + 16) + (size_t)wave * ENTRIES;
-    unsigned char* shut = smem + 16 + (size_t)NWAVE * ENTRIES * 16;
-    if (CLOSES) load_shut<TB>(D.shut + (size_t)tile * (TB * SLOT_BYTES), shut, NWAVE * 64);
+    unsigned char* shut = smem + 16 + (size_t)WAVES<NT> * ENTRIES * 16;
+    if (CLOSES) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) load_shut<TB>(D.shut + (size_t)(tile + q) * (TB * SLOT_BYTES), shut + q * SHUT_BYTES<TB>, WAVES<NT> * 64);
+    }
     // this workgroup's regions
     const unsigned lo = (unsigned)((unsigned long long)P * split / nsplit), hi = (unsigned)((unsigned long long)P * (split + 1) / nsplit);
     if (threadIdx.x == 0) counter[0] = lo;
-    unsigned B[NI][6];
-    load_operands<TB>(D.digits + (size_t)tile * (TB * NDIGIT * SLOT_BYTES), col, h, B);
-    const unsigned f = f0 + tile * FTILE + col;
-    const float bf = f < F ? bias[f] : 0.0f;
+    const unsigned f = f0 + tile * FTILE + (NT == 2 ? lane : col);    // the filter whose results this lane writes (one set: lanes 0-31)
     // The sums come in units of 2^down, in which open windows and the bias stay below one half (`whole`), so that adding the bias and
     // rectifying is one instruction, which clamps to 0 .. 1. (16 of 61 vector instructions beside a tile's six products of 16 taps. The
     // whole call, us: max + average, 20 000 x 30-150 letters x 384 filters x 16 taps 231 -> 219; average, 30 000 x 101 x 256, 12 taps 208 -> 196, 24 taps 274 -> 262.)
-    int s[3];
-    const int down = 31 - D.facts[tile * FTILE + col].whole;
-    const float unit = power_of_two(down), bu = bf * power_of_two(-down);
-    digit_scales(D.expo[tile * FTILE + col] - down, D.facts[tile * FTILE + col].shut - (unsigned)down, h, s);
+    unsigned B[NT][NI][6];
+    int s[NT][3];
+    float bu[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const unsigned t = tile + q, g = f0 + t * FTILE + col;
+        load_operands<TB>(D.digits + (size_t)t * (TB * NDIGIT * SLOT_BYTES), col, h, B[q]);
+        const digit_facts& facts = D.facts[t * FTILE + col];
+        const int down = 31 - facts.whole;
+        bu[q] = g < F ? bias[g] * power_of_two(-down) : 0.0f;
+        digit_scales(D.expo[t * FTILE + col] - down, facts.shut - (unsigned)down, h, s[q]);
+    }
+    const float bf = f < F ? bias[f] : 0.0f, unit = power_of_two(31 - D.facts[tile * FTILE + (NT == 2 ? lane : col)].whole);
     shut += (h * FTILE + col) * 24u;
     const unsigned rg = 4u * h;                                   // this half wave's rows lie 4 further down
     const unsigned at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
@@ -489,8 +520,8 @@ __device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsig
     if (r < hi) load12(X, N, a, lane, letters);
 
     while (r < hi) {
-        float mx = CLOSED, sum = 0.0f;
-        unsigned xi = 0u;
+        float mx[2] = {CLOSED, CLOSED}, sum[2] = {0.0f, 0.0f};
+        unsigned xi[2] = {0u, 0u};
         unsigned c = a;
         bool last;
         do {
@@ -507,58 +538,74 @@ __device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsig
             for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34) {
                 uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
                 if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
-                f32x16_t z;
+                f32x16_t sums[NT];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-                if (CLOSES) z = closed_windows<TB, 2>(z, a0, a1, shut, s[1]);
-                products<TB, 0>(z, a0, a1, B, s);
-                if (left - t0 < (unsigned)ROWS) {
+                for (int q = 0; q < NT; ++q) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) z[i] = rg + ((i & 3) + 8 * (i >> 2)) < left - t0 ? z[i] : CLOSED;
+                    for (int i = 0; i < 16; ++i) sums[q][i] = 0.0f;
+                    if (CLOSES) sums[q] = closed_windows<TB, 2>(sums[q], a0, a1, shut + q * SHUT_BYTES<TB>, s[q][1]);
                 }
-                if (PT != DBK_PT_AVG) {
-                    if (WANT_ARGMAX) {
-                        float bm = z[0];
-                        unsigned bi = 0u;
+                products<TB, NT, 0>(sums, a0, a1, B, s);
+                if (left - t0 < (unsigned)ROWS) {
+                    unsigned inside = left - t0;                  // (opaque: the comparisons stay in this branch)
+                    asm volatile("" : "+v"(inside));
 #pragma unroll
-                        for (int i = 1; i < 16; ++i) {
-                            const bool gt = z[i] > bm;
-                            bm = gt ? z[i] : bm;
-                            bi = gt ? (unsigned)i : bi;
-                        }
-                        if (bm > mx) { mx = bm; xi = (c - a) + t0 + rg + (bi & 3u) + 8u * (bi >> 2); }
-                    } else {
+                    for (int i = 0; i < 16; ++i) {
+                        const bool in = rg + ((i & 3) + 8 * (i >> 2)) < inside;
 #pragma unroll
-                        for (int i = 0; i < 16; i += 2) mx = fmaxf(fmaxf(mx, z[i]), z[i + 1]);
+                        for (int q = 0; q < NT; ++q) sums[q][i] = in ? sums[q][i] : CLOSED;
                     }
                 }
-                if (PT != DBK_PT_MAX) {
-                    float part = open_part(z[0], bu);
 #pragma unroll
-                    for (int i = 1; i < 16; ++i) part += open_part(z[i], bu);
-                    sum += part;                                  // (a tile's sum first: sums of sums round less)
+                for (int q = 0; q < NT; ++q) {
+                    const f32x16_t& z = sums[q];
+                    if (PT != DBK_PT_AVG) {
+                        if (WANT_ARGMAX) {
+                            float bm = z[0];
+                            unsigned bi = 0u;
+#pragma unroll
+                            for (int i = 1; i < 16; ++i) {
+                                const bool gt = z[i] > bm;
+                                bm = gt ? z[i] : bm;
+                                bi = gt ? (unsigned)i : bi;
+                            }
+                            if (bm > mx[q]) { mx[q] = bm; xi[q] = (c - a) + t0 + rg + (bi & 3u) + 8u * (bi >> 2); }
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < 16; i += 2) mx[q] = fmaxf(fmaxf(mx[q], z[i]), z[i + 1]);
+                        }
+                    }
+                    if (PT != DBK_PT_MAX) {
+                        float part = open_part(z[0], bu[q]);
+#pragma unroll
+                        for (int i = 1; i < 16; ++i) part += open_part(z[i], bu[q]);
+                        sum[q] += part;                           // (a tile's sum first: sums of sums round less)
+                    }
                 }
             }
             c += CHUNK;
         } while (!last);
-        // ---- the region's result: fold the two half waves (equal values keep the earlier row)
+        // ---- the region's result: fold the two half waves (equal values keep the earlier row); two sets: the second's in lanes 32-63
         if (PT != DBK_PT_AVG) {
-            const float vm = __shfl_xor(mx, 32, 64);
+            if (NT == 2) swap_halves(mx[0], mx[1]); else mx[1] = __shfl_xor(mx[0], 32, 64);
             if (WANT_ARGMAX) {
-                const unsigned vi = (unsigned)__shfl_xor((int)xi, 32, 64);
-                if (vm > mx || (vm == mx && vi < xi)) xi = vi;
+                if (NT == 2) swap_halves(xi[0], xi[1]); else xi[1] = (unsigned)__shfl_xor((int)xi[0], 32, 64);
+                if (mx[1] > mx[0] || (mx[1] == mx[0] && xi[1] < xi[0])) xi[0] = xi[1];
             }
-            mx = fmaxf(mx, vm) * unit + bf;
-            if (WANT_ARGMAX && !(mx > 0.0f)) xi = 0u;             // nothing open: the region's first row
-            mx = fmaxf(mx, 0.0f);
+            mx[0] = fmaxf(mx[0], mx[1]) * unit + bf;
+            if (WANT_ARGMAX && !(mx[0] > 0.0f)) xi[0] = 0u;       // nothing open: the region's first row
+            mx[0] = fmaxf(mx[0], 0.0f);
         }
-        if (PT != DBK_PT_MAX) sum = (sum + __shfl_xor(sum, 32, 64)) / (float)(b - a) * unit;
-        if (h == 0u && f < F) {
+        if (PT != DBK_PT_MAX) {
+            if (NT == 2) swap_halves(sum[0], sum[1]); else sum[1] = __shfl_xor(sum[0], 32, 64);
+            sum[0] = (sum[0] + sum[1]) / (float)(b - a) * unit;
+        }
+        if ((NT == 2 || h == 0u) && f < F) {
             const size_t j = (size_t)r * F + f;
-            if (PT == DBK_PT_MAX) pooled[j] = mx;
-            else if (PT == DBK_PT_AVG) pooled[j] = sum;
-            else { pooled[2 * j] = mx; pooled[2 * j + 1] = sum; }
-            if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + xi) * F + f);
+            if (PT == DBK_PT_MAX) pooled[j] = mx[0];
+            else if (PT == DBK_PT_AVG) pooled[j] = sum[0];
+            else { pooled[2 * j] = mx[0]; pooled[2 * j + 1] = sum[0]; }
+            if (WANT_ARGMAX) argmax[j] = (uint32_t)(((size_t)a + xi[0]) * F + f);
         }
         r = rn; a = an; b = bn;
         rn = claim(counter, lane);
@@ -566,17 +613,17 @@ __device__ __forceinline__ void scanpool_digits_body(const digit_store& D, unsig
     }
 }
 
-template <int PT, bool WANT_ARGMAX, int TB>
-__global__ __launch_bounds__(NWAVE * 64) __attribute__((amdgpu_waves_per_eu(NWAVE / 4, NWAVE / 4)))
+template <int PT, bool WANT_ARGMAX, int TB, int NT>
+__global__ __launch_bounds__(WAVES<NT> * 64) __attribute__((amdgpu_waves_per_eu(WAVES<NT> / 4, WAVES<NT> / 4)))
 void scanpool_digits_kernel(digit_store D, const float* __restrict__ bias, unsigned f0, unsigned F, const uint8_t* __restrict__ X, size_t N, size_t ndef,
                             const uint32_t* __restrict__ R, unsigned P, unsigned nsplit, float* __restrict__ pooled, uint32_t* __restrict__ argmax)
 {
-    const unsigned tile = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
+    const unsigned tile = NT * (blockIdx.x / nsplit), split = blockIdx.x % nsplit;
     if (left_out(D.flags, tile)) return;
-    if ((D.flags[tile] & TILE_CLOSES) != 0u)
-        scanpool_digits_body<PT, WANT_ARGMAX, TB, true>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
+    if (((D.flags[tile] | D.flags[tile + NT - 1]) & TILE_CLOSES) != 0u)
+        scanpool_digits_body<PT, WANT_ARGMAX, TB, NT, true>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
     else
-        scanpool_digits_body<PT, WANT_ARGMAX, TB, false>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
+        scanpool_digits_body<PT, WANT_ARGMAX, TB, NT, false>(D, tile, split, bias, f0, F, X, N, ndef, R, P, nsplit, pooled, argmax);
 }
 
 // ---------------------------------------------------------------------------------------------- plain maxima
@@ -642,11 +689,11 @@ __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, 
 {
     asm volatile("" : "+v"(lane));                                // (opaque: nothing of this is held in registers across the regions)
     const unsigned col = lane & 31u, h = lane >> 5, at0 = first_operand<TB>(col, h), at1 = second_operand<TB>(col, h);
-    int s[3];
-    digit_scales(expo, scale, h, s);
+    int s[1][3];
+    digit_scales(expo, scale, h, s[0]);
     shut += (h * FTILE + col) * 24u;
-    unsigned B[product_count<TB>::N][6];
-    load_operands<TB>(digits, col, h, B);
+    unsigned B[1][product_count<TB>::N][6];
+    load_operands<TB>(digits, col, h, B[0]);
     float mx = CLOSED;
     unsigned xi = 0u;
     for (unsigned c = a;; c += CHUNK) {
@@ -659,11 +706,12 @@ __device__ __forceinline__ float2 region_maximum(const uint8_t* __restrict__ X, 
         for (unsigned t0 = 0; t0 < nrow; t0 += ROWS, src += 34) {
             uint4 a0 = src[at0], a1 = TB >= 3 ? src[at1] : a0;
             if (t0 + ROWS > defined) close_undefined(a0, a1, t0 + col < defined);
-            f32x16_t z;
+            f32x16_t sums[1];
+            f32x16_t& z = sums[0];
 #pragma unroll
             for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-            if (CLOSES) z = closed_windows<TB, 2>(z, a0, a1, shut, s[1]);
-            products<TB, 0>(z, a0, a1, B, s);
+            if (CLOSES) z = closed_windows<TB, 2>(z, a0, a1, shut, s[0][1]);
+            products<TB, 1, 0>(sums, a0, a1, B, s);
             if (left - t0 < (unsigned)ROWS) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) z[i] = 4u * h + ((i & 3) + 8 * (i >> 2)) < left - t0 ? z[i] : CLOSED;
@@ -702,22 +750,6 @@ __device__ __forceinline__ void top_two(const f32x16_t& z, float& m1, float& m2,
     m2 = max3(max3(max3(max3(m2, k[0], k[1]), k[2], k[3]), k[4], v0), v1, v2);
     t1 = top > m1 ? t : t1;
     m1 = top;
-}
-
-// Lanes 0-31 of x beside lanes 0-31 of y, and lanes 32-63 of x beside lanes 32-63 of y: (x, y) becomes what the low and the
-// high half wave held of the first value (in lanes 0-31) and of the second (in lanes 32-63).
-__device__ __forceinline__ void swap_halves(unsigned& x, unsigned& y)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
-    x = r[0];
-    y = r[1];
-}
-__device__ __forceinline__ void swap_halves(float& x, float& y)
-{
-    unsigned a = __float_as_uint(x), b = __float_as_uint(y);
-    swap_halves(a, b);
-    x = __uint_as_float(a);
-    y = __uint_as_float(b);
 }
 
 template <bool WANT_ARGMAX, int TB, bool CLOSES>
@@ -993,17 +1025,35 @@ int launch_max(hipStream_t st, const digit_store& D, const float* W, const float
     return 0;
 }
 
-constexpr size_t scan_smem(int tb) { return 16 + (size_t)NWAVE * ENTRIES * 16 + (tb <= 2 ? SHUT_BYTES<2> : SHUT_BYTES<4>); }
+template <int TB, int NT> constexpr size_t scan_smem() { return 16 + (size_t)WAVES<NT> * ENTRIES * 16 + NT * SHUT_BYTES<TB>; }
+
+// Whether a wave takes two sets of 32 filters at a time: one staging of the letters, one read of a tile's operands and one walk serve both,
+// and their products take turns instead of waiting for each other's sums. Up to 16 taps, whose digits leave the registers for it (24 taps, us, one /
+// two: average, 30 000 x 101 x 256 251 / 254, max + average 271 / 303). An odd last set is scanned beside nothing, which many others pay for.
+// Whole calls, us, one / two: max + average, 20 000 x 30-150 letters x 384 filters x 16 taps 205 / 193, 60 000 x 20-40 x 128 142 / 131; maximum,
+// 60 000 x 101 x 256, 8 taps 225 / 195, 16 taps 328 / 304; average, 30 000 x 101 x 256 x 12 taps 186 / 174; 5000 x 101 x 64 x 16 taps 25.5 / 25.4.
+inline bool takes_two(unsigned ntile) { return ntile % 2 == 0 || ntile > 16; }
+
+template <int PT, bool WANT_ARGMAX, int TB, int NT>
+int launch_sets(hipStream_t st, const digit_store& D, const float* bias, unsigned f0, unsigned ntile, size_t F, const uint8_t* X, size_t N, size_t ndef,
+                const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
+{
+    auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB, NT>;
+    constexpr size_t smem = scan_smem<TB, NT>();
+    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    const unsigned groups = (ntile + NT - 1) / NT, nsplit = splits(groups, WAVES<NT>, P);
+    hipLaunchKernelGGL(kern, dim3(groups * nsplit), dim3(WAVES<NT> * 64), smem, st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
+    return 0;
+}
 
 template <int PT, bool WANT_ARGMAX, int TB>
 int launch_pt(hipStream_t st, const digit_store& D, const float* bias, unsigned f0, unsigned ntile, size_t F, const uint8_t* X, size_t N, size_t ndef,
               const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
 {
-    auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB>;
-    DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_smem(TB)));
-    const unsigned nsplit = splits(ntile, NWAVE, P);
-    hipLaunchKernelGGL(kern, dim3(ntile * nsplit), dim3(NWAVE * 64), scan_smem(TB), st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
-    return 0;
+    if constexpr (TB <= 2) {
+        if (takes_two(ntile)) return launch_sets<PT, WANT_ARGMAX, TB, 2>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+    }
+    return launch_sets<PT, WANT_ARGMAX, TB, 1>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
 }
 
 // the filters f0 .. f0 + 32 * ntile - 1: their digits, then the scan (half: plain maxima with half the products)

@@ -1582,6 +1582,26 @@ def test_bulk_scan_of_filters_that_forbid_letters_is_as_close_as_float32(ks, m, 
 
 
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [8, 16])
+@pytest.mark.parametrize("F,closed", [(33, ()), (64, (0,)), (64, (1,)), (128, (1, 2)), (520, ()), (520, (16,))])
+def test_bulk_scan_of_two_sets_of_filters_at_a_time(ks, F, closed, m, ptype):
+    """Waves that take 64 filters: a second set of one filter, an odd last set beside nothing (17 sets), weights that close windows in
+    either set of a pair."""
+    rng, W, b, X, R = _bulk_case(160 + m, [300, 1, 32, 224, 0, 500, 64, 33], m, F)
+    R = R[R[:, 1] > R[:, 0]]
+    R[-1, 1] = X.size                                                   # the last region runs into rows the scan does not define
+    _closed_tiles(W, closed, np.float32(-1e9))
+    A, want, rows = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
+    P, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")
+    _within_rounding(host(P), want, np.where(W < -1e8, 0.0, W), b, ptype)
+    if ptype != "avg":
+        Pa, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=True, path="kmer")
+        assert np.array_equal(host(Pa), host(P))
+        moved = host(I) != rows
+        assert np.abs(A.ravel()[host(I)[moved]] - A.ravel()[rows[moved]]).max(initial=0.0) <= 1e-5
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("m", [4, 16, 24])
 @pytest.mark.parametrize("size,bias", [(1e-24, 0.0), (1e28, 0.0), (1e-20, 1e25), (1e-20, -1e25), (1e-12, 1e-3), (1e20, 1e-20), (1.0, -1e29)])
 def test_bulk_scan_of_weights_and_biases_of_any_size(ks, size, bias, m, ptype):
