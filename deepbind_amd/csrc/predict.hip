@@ -81,17 +81,20 @@ __global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict_
 // A change at p moves the `m` rows whose windows hold p and nothing else, so a workgroup takes a few consecutive letters
 // of one region: it scans the region once (16 lanes of filters x 16 lanes of rows, the letter table of 16 filters in
 // LDS), keeps the maximum and the sum of the rows no change of its letters can reach and, one by one, the rows some change
-// can; a wave then takes a letter at a time, its lanes being 4 new letters x 16 filters, scans the m rows of each anew -
-// taps in ascending order, as the forward pass does - and pools them with what is kept. (Rows of a mean are added in an order that depends on
+// can; a wave then takes a letter at a time, its lanes being 4 quarters of the m rows x 16 filters: the rows are scanned anew without that
+// letter, in two halves of its other taps, which leaves one addition for each of the four new ones, and pooled with what is kept (maps' error
+// against float64 2.1e-6 to 6.6e-6, 2.4e-6 to 6.9e-6 with every tap in one chain). (Rows of a mean are added in an order that depends on
 // where the workgroup's letters lie, so the score of the letter that is there comes from k_mutation_map.) More than 16 filters take further passes; pooled values meet the dense head in LDS.
-// What bounds it is LDS reads, one per (row, tap): m * m per letter and filter tile, where the reference's way (a pass of the
+// What bounds it is instruction issue and LDS reads, one per (row, tap): m * m / 4 per letter and filter tile and lane (m * m with a lane per new
+// letter, each of which scanned the rows by itself), where the reference's way (a pass of the
 // whole net per change) scans length + m - 1 rows per change, and launches 15 kernels for it.
-// Measured: 32 sequences of 60-101 letters, both strands, 16 filters of 24 taps: 0.047 ms, the whole call
-// 0.13 ms from strings to host arrays (74-84 ms when the batch was re-scored once per letter and base).
+// Measured: 32 sequences of 60-101 letters, both strands, 16 filters of 24 taps: 25 us (a lane per new letter 47), the whole call
+// 104 us from strings to host arrays (125) (74-84 ms when the batch was re-scored once per letter and base).
 //
 // The reference changes letter i of EVERY region in pass i; where a region is shorter than its neighbour's i that lands in
 // the pad behind it, which is the next region's leading pad. Those entries are scored with both changes, the rows of either window anew.
 constexpr unsigned MUT_F = 16, MUT_MAXK = 128, MUT_MAXH = 64;
+constexpr unsigned MUT_NT = 256;                                    // threads per workgroup
 constexpr unsigned MUT_TILE = 512;                                  // rows of the region scanned between two stagings of letters
 
 struct mut_args {
@@ -99,7 +102,7 @@ struct mut_args {
     const uint8_t* X;
     const uint32_t* R;
     size_t N, P;
-    unsigned m, F, k, hidden;
+    unsigned m, F, k, hidden, pos;                                  // pos: letters per workgroup
     int ptype, logistic, strands;
     float *S, *base;                                                // changed scores (4 per stream position), unchanged ones (per region)
 };
@@ -120,36 +123,69 @@ __device__ __forceinline__ void letter_table16(float* __restrict__ lut, const fl
     }
 }
 
-// Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending; the letters at index
-// `at` and `at2` read as `other`. A letter is read once for the four rows it meets.
-template <bool TWO = false>
-__device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, unsigned at,
-                                      unsigned other, float (&z)[4], unsigned at2 = ~0u)
+// Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending. A letter is read once for the four rows it meets.
+__device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, float (&z)[4])
 {
     z[0] = z[1] = z[2] = z[3] = 0.0f;
     unsigned l[4];
 #pragma unroll
-    for (unsigned u = 0; u < 3; ++u) l[u + 1] = p + u == at || (TWO && p + u == at2) ? other : let[p + u];
+    for (unsigned u = 0; u < 3; ++u) l[u + 1] = let[p + u];
 #pragma unroll 4
     for (unsigned j = 0; j < m; ++j) {
         l[0] = l[1]; l[1] = l[2]; l[2] = l[3];
-        l[3] = p + 3 + j == at || (TWO && p + 3 + j == at2) ? other : let[p + 3 + j];
+        l[3] = let[p + 3 + j];
         const float* t = lut_f + j * NL * MUT_F;
 #pragma unroll
         for (unsigned u = 0; u < 4; ++u) z[u] += t[l[u]];
     }
 }
 
-// LDS, in this order: letter table [m][NL][16], rows a change can reach [pos + m - 1][16] (rectified), two fold areas [2][16][16],
-// pooled values [pos + 1][4][k], rows of the region's head, i.e. those whose windows hold letters of its leading pad, [m][16]; letters of a
-// tile of rows and their windows, letters of the rows a change can reach, letters of the head rows.
-// (scan4 looks 3 rows past the last one asked for.)
-__host__ __device__ inline unsigned mut_tile_letters(unsigned m) { return (MUT_TILE + m + 3 + 3) & ~3u; }
-__host__ __device__ inline unsigned mut_reach_letters(unsigned pos, unsigned m) { return (pos + 2 * m + 4 + 3) & ~3u; }
-inline size_t mut_smem(unsigned pos, size_t m, size_t k)
+// Rows p .. p + NR - 1, in two halves of the taps, each ascending.
+template <unsigned NR>
+__device__ __forceinline__ void scan_rows(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, float (&z)[NR])
 {
-    return ((size_t)m * NL * MUT_F + (pos + m - 1) * MUT_F + 2 * 16 * MUT_F + (pos + 1) * 4 * k + m * MUT_F) * sizeof(float) +
-           mut_tile_letters((unsigned)m) + mut_reach_letters(pos, (unsigned)m) + mut_reach_letters(0, (unsigned)m);
+    float first[NR];
+    unsigned l[NR];
+#pragma unroll
+    for (unsigned u = 0; u < NR; ++u) z[u] = 0.0f;
+#pragma unroll
+    for (unsigned u = 0; u + 1 < NR; ++u) l[u + 1] = let[p + u];
+    auto taps = [&](unsigned from, unsigned to) __attribute__((always_inline)) {
+#pragma unroll 4
+        for (unsigned j = from; j < to; ++j) {
+#pragma unroll
+            for (unsigned u = 0; u + 1 < NR; ++u) l[u] = l[u + 1];
+            l[NR - 1] = let[p + NR - 1 + j];
+            const float* t = lut_f + j * NL * MUT_F;
+#pragma unroll
+            for (unsigned u = 0; u < NR; ++u) z[u] += t[l[u]];
+        }
+    };
+    const unsigned half = m / 2u;
+    taps(0u, half);
+#pragma unroll
+    for (unsigned u = 0; u < NR; ++u) { first[u] = z[u]; z[u] = 0.0f; }
+    taps(half, m);
+#pragma unroll
+    for (unsigned u = 0; u < NR; ++u) z[u] += first[u];
+}
+
+// LDS, in this order: letter table [m][NL][16], rows a change can reach [pos + m - 1][16] (rectified), two fold areas [2][NT / 16][16],
+// pooled values [pos + 1][4][k], rows of the region's head, i.e. those whose windows hold letters of its leading pad, [m][16]; letters of a
+// tile of rows and their windows, letters of the rows a change can reach, letters of the head rows, each wave's letters without the one it changes.
+// (The scans of a quarter of the rows run up to 11 rows past the last one, and look up to 7 further.) The head's first weights [k][hidden] where they are few.
+__host__ __device__ inline unsigned mut_tile_letters(unsigned m) { return (MUT_TILE + m + 7 + 3) & ~3u; }
+__host__ __device__ inline unsigned mut_reach_letters(unsigned pos, unsigned m) { return (pos + 2 * m + 20 + 3) & ~3u; }
+__host__ __device__ inline unsigned mut_head_weights(unsigned k, unsigned hidden) { const unsigned n = k * (hidden > 0 ? hidden : 1u); return n <= 2048u ? n : 0u; }
+inline size_t mut_smem(unsigned pos, size_t m, size_t k, size_t hidden)
+{
+    return ((size_t)m * NL * MUT_F + (pos + m - 1) * MUT_F + 2 * MUT_NT / 16 * MUT_F + (pos + 1) * 4 * k + m * MUT_F + mut_head_weights((unsigned)k, (unsigned)hidden)) * sizeof(float) +
+           mut_tile_letters((unsigned)m) + (1 + MUT_NT / 64) * mut_reach_letters(pos, (unsigned)m) + mut_reach_letters(0, (unsigned)m);
+}
+// what a call may ask for (65 536 bytes, while a workgroup had 256 threads and neither the head's weights nor the waves' letters in LDS)
+inline bool mut_fits(size_t m, size_t k)
+{
+    return mut_smem(16, m, k, 4096) - MUT_NT / 64 * mut_reach_letters(16, (unsigned)m) - 2 * (MUT_NT - 256) * sizeof(float) <= 65536 + 36;
 }
 
 // Pass `pass` of the reference changes letter `pass` of every region: whether what it does to the region [pa, pb) before this one (none: !before)
@@ -159,40 +195,71 @@ __device__ __forceinline__ bool spilled_pass(unsigned pass, unsigned pad, bool b
     return before && pb - pa > pass && pad + pa + pass >= pb && pad + pa + pass < ra + pad;
 }
 
-template <unsigned MUT_POS>
-__global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
+// NR: rows that a lane scans at a time. SPILLS: one strand only, where a change may lie in two regions (above).
+// v[c] of the four quarters of a wave put together: lanes 16 c .. 16 c + 15 get the one of v[c]
+template <typename Op>
+__device__ __forceinline__ float quarters(const float (&v)[4], Op op)
+{
+    float half[2];
+#pragma unroll
+    for (unsigned c = 0; c < 2; ++c) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[c]), __float_as_uint(v[c + 2]), false, false);
+        half[c] = op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(half[0]), __float_as_uint(half[1]), false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+template <unsigned NR, bool SPILLS>
+__global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
 {
     extern __shared__ __align__(16) float msm[];
     const unsigned m = a.m, pad = m - 1;
     const size_t r = blockIdx.x;
-    const unsigned ra = a.R[2 * r], rb = a.R[2 * r + 1];
-    const unsigned len = rb - ra > pad ? rb - ra - pad : 0u;
-    const unsigned i0 = blockIdx.y * MUT_POS;
-    if (i0 >= len && blockIdx.y != 0) return;
-    const unsigned npos = i0 < len ? (len - i0 < MUT_POS ? len - i0 : MUT_POS) : 0u;
     const unsigned tid = threadIdx.x, lane = tid & 63, wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     float* lut = msm;
     float* rows = lut + m * NL * MUT_F;
-    float* fold = rows + (MUT_POS + m - 1) * MUT_F;
-    float* pooled = fold + 2 * 16 * MUT_F;
-    float* head = pooled + (MUT_POS + 1) * 4 * a.k;
-    uint8_t* tile = reinterpret_cast<uint8_t*>(head + m * MUT_F);
+    float* fold = rows + (a.pos + m - 1) * MUT_F;
+    float* pooled = fold + 2 * MUT_NT / 16 * MUT_F;
+    float* head = pooled + (a.pos + 1) * 4 * a.k;
+    float* head_w = head + m * MUT_F;
+    const unsigned nhead_w = mut_head_weights(a.k, a.hidden);
+    // (the weights are on their way before the region's bounds and letters)
+    for (unsigned e = tid; e < nhead_w; e += MUT_NT) head_w[e] = a.W1[e];
+    letter_table16(lut, a.W, m, a.F, 0, a.F, MUT_NT);
+    const unsigned hl = tid & 15u;
+    float hidden_b[MUT_MAXH / 16], hidden_w[MUT_MAXH / 16];         // this lane's hidden units'
+#pragma unroll
+    for (unsigned q = 0; q < MUT_MAXH / 16; ++q) {
+        const bool one = hl + 16u * q < a.hidden;
+        hidden_b[q] = one ? a.b1[hl + 16u * q] : 0.0f;
+        hidden_w[q] = one ? a.W2[hl + 16u * q] : 0.0f;
+    }
+    const float last_b = a.hidden > 0 ? a.b2[0] : a.b1[0];
+    const unsigned ra = a.R[2 * r], rb = a.R[2 * r + 1];
+    const unsigned len = rb - ra > pad ? rb - ra - pad : 0u;
+    const unsigned i0 = blockIdx.y * a.pos;
+    if (i0 >= len && blockIdx.y != 0) return;
+    const unsigned npos = i0 < len ? (len - i0 < a.pos ? len - i0 : a.pos) : 0u;
+    uint8_t* tile = reinterpret_cast<uint8_t*>(head_w + nhead_w);
     uint8_t* let = tile + mut_tile_letters(m);
-    uint8_t* hlet = let + mut_reach_letters(MUT_POS, m);
+    uint8_t* hlet = let + mut_reach_letters(a.pos, m);
+    uint8_t* mine = hlet + mut_reach_letters(0, m) + wave * mut_reach_letters(a.pos, m);
     const size_t n = a.N >= m ? a.N - m + 1 : 0;                   // rows the scan defines; later rows are relu(bias)
     // rows some change of these letters reaches: [s0, s1)
     const unsigned q0 = ra + pad + i0;                             // stream position of the first letter
     const unsigned s0 = q0 - pad, s1 = npos ? q0 + npos : s0;
     auto stage = [&](uint8_t* to, size_t from, unsigned count) {   // letters as offsets into a tap's part of the table
-        for (unsigned e = tid; e < count; e += 256) to[e] = (uint8_t)((from + e < a.N ? letter_of(a.X[from + e]) : 5u) * MUT_F);
+        for (unsigned e = tid; e < count; e += MUT_NT) to[e] = (uint8_t)((from + e < a.N ? letter_of(a.X[from + e]) : 5u) * MUT_F);
     };
-    stage(let, s0, mut_reach_letters(MUT_POS, m));
+    stage(let, s0, mut_reach_letters(a.pos, m));
     // the change of the region before this one that lands in this one's leading pad
-    const bool shorter_before = a.strands == 1 && r > 0;
+    const bool shorter_before = SPILLS && r > 0;
     const unsigned pa = shorter_before ? a.R[2 * r - 2] : 0u, pb = shorter_before ? a.R[2 * r - 1] : 0u;
     auto spills = [&](unsigned pass) { return spilled_pass(pass, pad, shorter_before, pa, pb, ra); };
     bool spill_here = false;
-    for (unsigned i = 0; i < npos; ++i) spill_here |= spills(i0 + i);
+    if (SPILLS)
+        for (unsigned i = 0; i < npos; ++i) spill_here |= spills(i0 + i);
     // rows of the head that no change of these letters reaches: with a spill they are kept one by one as well
     const unsigned h1 = spill_here ? (s0 < ra + pad ? s0 : ra + pad) : ra;
     if (spill_here) stage(hlet, ra, mut_reach_letters(0, m));
@@ -204,8 +271,10 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
     for (unsigned f0 = 0; f0 < a.F; f0 += MUT_F) {
         const bool on = f0 + f < a.F;
         const float bf = on ? a.bias[f0 + f] : 0.0f;
-        __syncthreads();                                            // the previous tile's table and rows are no longer read
-        letter_table16(lut, a.W, m, a.F, f0, a.F, 256);
+        if (f0 > 0) {
+            __syncthreads();                                        // the previous tile's table and rows are no longer read
+            letter_table16(lut, a.W, m, a.F, f0, a.F, MUT_NT);
+        }
         // ---- the region as it is: rows out of reach folded, rows in reach kept
         float mx = 0.0f, sum = 0.0f;
         for (unsigned t0 = ra; t0 < rb; t0 += MUT_TILE) {
@@ -213,9 +282,9 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
             stage(tile, t0, mut_tile_letters(m));
             __syncthreads();
             const unsigned t1 = rb - t0 < MUT_TILE ? rb : t0 + MUT_TILE;
-            for (unsigned p = t0 + 4 * rl; p < t1; p += 64) {
+            for (unsigned p = t0 + 4 * rl; p < t1; p += MUT_NT / 4) {
                 float z[4];
-                scan4(lut_f, tile, p - t0, m, ~0u, 0u, z);
+                scan_rows<4>(lut_f, tile, p - t0, m, z);
 #pragma unroll
                 for (unsigned u = 0; u < 4; ++u) {
                     if (p + u >= t1) break;
@@ -228,84 +297,120 @@ __global__ __launch_bounds__(256) void k_mutation_scores(const mut_args a)
             }
         }
         fold[rl * MUT_F + f] = mx;
-        fold[(16 + rl) * MUT_F + f] = sum;
+        fold[(MUT_NT / 16 + rl) * MUT_F + f] = sum;
         __syncthreads();
         mx = 0.0f; sum = 0.0f;
 #pragma unroll
-        for (unsigned t = 0; t < 16; ++t) {
+        for (unsigned t = 0; t < MUT_NT / 16; ++t) {
             const float v = fold[t * MUT_F + f];
             mx = v > mx ? v : mx;
-            sum += fold[(16 + t) * MUT_F + f];
+            sum += fold[(MUT_NT / 16 + t) * MUT_F + f];
         }
-        // ---- one letter per wave at a time (the item behind the last one is the region unchanged): lane = (new letter, filter)
-        const unsigned c = lane >> 4, coff = c * MUT_F;
-        for (unsigned i = wave; i < npos + (i0 == 0 ? 1u : 0u); i += 4) {
-            float bm = mx, bs = sum;
-            auto pool = [&](float v) { bm = v > bm ? v : bm; bs += v; };
+        // ---- one letter per wave at a time (the item behind the last one is the region unchanged): lane = (quarter of the rows, filter)
+        const unsigned g = lane >> 4;
+        for (unsigned i = wave; i < npos + (i0 == 0 ? 1u : 0u); i += MUT_NT / 64) {
+            float bm[4] = {mx, mx, mx, mx}, bs[4] = {0.0f, 0.0f, 0.0f, 0.0f};      // with each new letter, of this quarter
+            float km = 0.0f, ks = g == 0u ? sum : 0.0f;                             // of rows that no new letter changes
+            auto kept = [&](const float* values, unsigned lo, unsigned hi) __attribute__((always_inline)) {
+                for (unsigned p = lo + g; p < hi; p += 4) { const float v = values[p * MUT_F + f]; km = v > km ? v : km; ks += v; }
+            };
             // rows [lo, hi) among the kept ones are scanned anew: those of letter q0 + i's windows, and with a spill the head as well
-            const bool both = i < npos && spills(i0 + i);
-            const unsigned q2 = pad + pa + i0 + i;
+            const bool both = SPILLS && i < npos && spills(i0 + i);
+            const unsigned q2 = pad + pa + i0 + i, rest = s1 - s0;
             unsigned hp = 0;                                         // rows of the head to scan anew
             if (both) {
                 hp = q2 + 1 - ra;                                    // rows ra .. q2 hold it
                 if (hp > h1 - ra) hp = h1 - ra;
-                for (unsigned p = 0; p < hp; p += 4) {
-                    float z[4];
-                    scan4(lut_f, hlet, p, m, q2 - ra, coff, z);
-#pragma unroll
-                    for (unsigned u = 0; u < 4; ++u)
-                        if (p + u < hp) {
-                            const float v = ((size_t)ra + p + u < n ? z[u] : 0.0f) + bf;
-                            pool(v > 0.0f ? v : 0.0f);
-                        }
-                }
             }
-            for (unsigned p = hp; p < h1 - ra; ++p) pool(head[p * MUT_F + f]);
-            const unsigned rest = s1 - s0;
+            kept(head, hp, h1 - ra);
             unsigned lo = i < npos ? i : rest, hi = i < npos ? i + m : rest;
             if (both && q2 >= s0) lo = 0;
-            for (unsigned p = 0; p < lo; ++p) pool(rows[p * MUT_F + f]);
-            for (unsigned p = lo; p < hi; p += 4) {
-                float z[4];
-                if (both) scan4<true>(lut_f, let, p, m, i + pad, coff, z, q2 - s0);
-                else scan4(lut_f, let, p, m, i + pad, coff, z);
+            kept(rows, 0u, lo);
+            kept(rows, hi, rest);
+            // the rows, then (spills) those of the head: row 0 at stream position `first`, the letters at indexes `at` and `at2` (~0: none) changed
+            unsigned first = s0, at = i + pad, at2 = both ? q2 - s0 : ~0u;
+            const uint8_t* letters = let;
+            for (unsigned part = 0; part < (both ? 2u : 1u); ++part) {
+                const unsigned each = (hi - lo + 3u) / 4u, shown = hi > lo ? hi - lo + 3u + NR + m : 0u;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                for (unsigned e = lane; e < shown; e += 64) mine[e] = lo + e == at || lo + e == at2 ? (uint8_t)(5u * MUT_F) : letters[lo + e];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const unsigned stop = n > first ? (n - first < hi ? (unsigned)(n - first) : hi) : 0u;      // rows that the scan defines
+                for (unsigned u0 = 0; u0 < each; u0 += NR) {
+                    const unsigned p0 = lo + g * each + u0;
+                    float z[NR], w[NR][4];
+                    // what the new letters put in the place of the old (no tap of this row's: nothing)
 #pragma unroll
-                for (unsigned u = 0; u < 4; ++u)
-                    if (p + u < hi) {
-                        const float v = ((size_t)s0 + p + u < n ? z[u] : 0.0f) + bf;
-                        pool(v > 0.0f ? v : 0.0f);
+                    for (unsigned u = 0; u < NR; ++u) {
+                        const bool here = at - (p0 + u) < m;        // (a row past the letter wraps round)
+                        const float* t = lut_f + (here ? at - (p0 + u) : 0u) * NL * MUT_F;
+#pragma unroll
+                        for (unsigned c = 0; c < 4; ++c) w[u][c] = here ? t[c * MUT_F] : 0.0f;
                     }
+                    if (SPILLS && both) {
+#pragma unroll
+                        for (unsigned u = 0; u < NR; ++u) {
+                            const bool there = at2 - (p0 + u) < m;
+                            const float* t = lut_f + (there ? at2 - (p0 + u) : 0u) * NL * MUT_F;
+#pragma unroll
+                            for (unsigned c = 0; c < 4; ++c) w[u][c] += there ? t[c * MUT_F] : 0.0f;
+                        }
+                    }
+                    scan_rows<NR>(lut_f, mine, p0 - lo, m, z);
+#pragma unroll
+                    for (unsigned u = 0; u < NR; ++u) {
+                        const bool counts = u0 + u < each && p0 + u < hi, in = p0 + u < stop;
+#pragma unroll
+                        for (unsigned c = 0; c < 4; ++c) {
+                            float v = (in ? z[u] + w[u][c] : 0.0f) + bf;
+                            v = counts && v > 0.0f ? v : 0.0f;
+                            bm[c] = v > bm[c] ? v : bm[c];
+                            bs[c] += v;
+                        }
+                    }
+                }
+                letters = hlet; first = ra; lo = 0u; hi = hp; at = q2 - ra; at2 = ~0u;
             }
-            for (unsigned p = hi; p < rest; ++p) pool(rows[p * MUT_F + f]);
+            // ---- the quarters together, quarter g with new letter g
+#pragma unroll
+            for (unsigned c = 0; c < 4; ++c) { bm[c] = km > bm[c] ? km : bm[c]; bs[c] += ks; }
+            const float best = quarters(bm, [](float x, float y) { return x > y ? x : y; }), total = quarters(bs, [](float x, float y) { return x + y; });
             if (on) {
-                float* to = pooled + (i * 4 + c) * a.k + (f0 + f) * kper;
-                if (a.ptype == DBK_PT_MAX) to[0] = bm;
-                else if (a.ptype == DBK_PT_AVG) to[0] = bs / count;
-                else { to[0] = bm; to[1] = bs / count; }
+                float* to = pooled + (i * 4 + g) * a.k + (f0 + f) * kper;
+                if (a.ptype == DBK_PT_MAX) to[0] = best;
+                else if (a.ptype == DBK_PT_AVG) to[0] = total / count;
+                else { to[0] = best; to[1] = total / count; }
             }
         }
     }
     __syncthreads();
     // ---- the dense head: 16 lanes per (letter, change) item, hidden units dealt over them
     const float sc = a.in_scale ? a.in_scale[0] : 1.0f;
-    const unsigned nitem = (npos + (i0 == 0 ? 1u : 0u)) * 4, g = tid >> 4, hl = tid & 15u;
-    for (unsigned it = g; it < nitem; it += 16) {
+    const float* w1 = nhead_w ? head_w : a.W1;
+    const unsigned nitem = (npos + (i0 == 0 ? 1u : 0u)) * 4;
+    for (unsigned it = tid >> 4; it < nitem; it += MUT_NT / 16) {
         const float* x = pooled + it * a.k;
         float out = 0.0f;
         if (a.hidden > 0) {
-            for (unsigned h = hl; h < a.hidden; h += 16) {
+#pragma unroll
+            for (unsigned q = 0; q < MUT_MAXH / 16; ++q) {
+                const unsigned h = hl + 16u * q;
+                if (h >= a.hidden) break;
                 float z = 0.0f;
 #pragma unroll 8
-                for (unsigned kk = 0; kk < a.k; ++kk) z = __builtin_fmaf(x[kk] * sc, a.W1[(size_t)kk * a.hidden + h], z);
-                z += a.b1[h];
-                out += (z > 0.0f ? z : 0.0f) * a.W2[h];
+                for (unsigned kk = 0; kk < a.k; ++kk) z = __builtin_fmaf(x[kk] * sc, w1[(size_t)kk * a.hidden + h], z);
+                z += hidden_b[q];
+                out += (z > 0.0f ? z : 0.0f) * hidden_w[q];
             }
         } else {
-            for (unsigned kk = hl; kk < a.k; kk += 16) out += x[kk] * sc * a.W1[kk];
+            for (unsigned kk = hl; kk < a.k; kk += 16) out += x[kk] * sc * w1[kk];
         }
 #pragma unroll
         for (int d = 8; d >= 1; d >>= 1) out += __shfl_xor(out, d, 16);
-        out += a.hidden > 0 ? a.b2[0] : a.b1[0];
+        out += last_b;
         if (a.logistic) out = 1.0f / (1.0f + expf(-out));
         if (hl == 0) {
             const unsigned i = it >> 2, c = it & 3u;
@@ -373,7 +478,7 @@ __global__ __launch_bounds__(NT) void k_predict_small(const small_args a)
         __syncthreads();
         for (unsigned p = t0 + 4 * rl; p < t1; p += NT / 4) {
             float z[4];
-            scan4(lut + f, tile, p - t0, m, ~0u, 0u, z);
+            scan4(lut + f, tile, p - t0, m, z);
 #pragma unroll
             for (unsigned u = 0; u < 4; ++u)
                 if (p + u < t1) {
@@ -487,7 +592,7 @@ __global__ __launch_bounds__(256) void k_gradient_map(const grad_args a)
         unsigned at = ~0u;
         for (unsigned p = 4 * rl; p < rows; p += 64) {
             float z[4];
-            scan4(lut + f, tile, p, m, ~0u, 0u, z);
+            scan4(lut + f, tile, p, m, z);
 #pragma unroll
             for (unsigned u = 0; u < 4; ++u) {
                 float v = z[u] + bf;
@@ -723,7 +828,7 @@ int dbk_mutation_map_takes(size_t m, size_t nfilter, int ptype, size_t hidden)
 {
     const size_t k = nfilter * (ptype == DBK_PT_ALL ? 2 : 1);
     return m >= 1 && m <= 64 && nfilter >= 1 && k <= MUT_MAXK && hidden <= MUT_MAXH &&
-           (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL) && mut_smem(16, m, k) <= 65536;
+           (ptype == DBK_PT_MAX || ptype == DBK_PT_AVG || ptype == DBK_PT_ALL) && mut_fits(m, k);
 }
 
 int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, size_t m, size_t nfilter, const uint8_t* X, size_t N,
@@ -736,10 +841,11 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     if (nregion == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(W && bias && X && regions && W1 && b1 && Z && (longest == 0 || map), "ValueError: null pointer argument");
     DBK_CHECK(hidden == 0 || (W2 && b2), "ValueError: hidden layer requested but W2/b2 are null");
-    // letters per workgroup: 16 where that still gives every CU several workgroups, else fewer, as a workgroup's first scan of
-    // its region costs less than an idle CU (64 regions of up to 101 letters: 159 us a call with 4, 179 with 16; 256 of 101: 312 / 288)
+    // letters per workgroup: 16 where that still gives every CU six workgroups, 8 where it has two, else 4, as a workgroup's first scan of
+    // its region costs less than an idle CU. Whole calls, us, 4 / 8 / 16: one sequence of 101 letters 72 / 77 / 88; 64 regions of 60-101, 24 taps
+    // 111 / 104 / 114, 32 taps 145 / 144 / 163; 100 regions of 40-80, 8 taps 132 / 130 / 136; 256 regions of 101 227 / 209 / 200.
     const size_t letters = longest > 0 ? longest : 1;
-    const unsigned pos = nregion * dbk::divup(letters, 16) >= 1024 ? 16u : nregion * dbk::divup(letters, 8) >= 1024 ? 8u : 4u;
+    const unsigned pos = nregion * dbk::divup(letters, 16) >= 1536 ? 16u : nregion * dbk::divup(letters, 8) >= 512 ? 8u : 4u;
     const unsigned gy = dbk::divup(letters, pos);
     DBK_CHECK(nregion <= 0x7fffffffu && gy <= 65535u, "ValueError: too many regions (%zu) or letters per region (%zu) for one launch", nregion, longest);
     hipStream_t st = dbk::as_stream(stream);
@@ -751,8 +857,13 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     a.m = (unsigned)m; a.F = (unsigned)nfilter; a.k = (unsigned)(nfilter * (ptype == DBK_PT_ALL ? 2 : 1)); a.hidden = (unsigned)hidden;
     a.ptype = ptype; a.logistic = apply_logistic; a.strands = strands;
     a.S = scratch; a.base = scratch + 4 * N;
-    auto kern = pos == 16 ? k_mutation_scores<16> : (pos == 8 ? k_mutation_scores<8> : k_mutation_scores<4>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(256), mut_smem(pos, m, a.k), st, a);
+    a.pos = pos;
+    // (a lane takes a quarter of the m rows)
+    auto kern = strands == 1 ? (m <= 16 ? k_mutation_scores<4, true> : (m <= 24 ? k_mutation_scores<6, true> : k_mutation_scores<8, true>))
+                             : (m <= 16 ? k_mutation_scores<4, false> : (m <= 24 ? k_mutation_scores<6, false> : k_mutation_scores<8, false>));
+    const size_t smem = mut_smem(pos, m, a.k, hidden);
+    if (smem > 65536) DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(MUT_NT), smem, st, a);
     hipLaunchKernelGGL(k_mutation_map, dim3((unsigned)(nregion / strands)), dim3(256), 0, st, regions, (unsigned)(m - 1), strands, X,
                        (const float*)a.S, (const float*)a.base, Z, map);
     DBK_LAUNCH_OK();

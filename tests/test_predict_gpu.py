@@ -122,6 +122,38 @@ def test_mutation_map_kernel_edges(pool, hidden, loss, rc, m, F):
 
 
 @pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("pool,hidden,m,F", [("max", 0, 2, 16), ("all", 64, 3, 5), ("avg", 17, 5, 16), ("all", 3, 18, 16), ("max", 32, 25, 16), ("all", 0, 33, 4),
+                                             ("avg", 9, 64, 2)])
+def test_mutation_map_quarters_of_any_number_of_taps(pool, hidden, m, F, rc):
+    """A lane scans a quarter of the rows that a letter moves, four, six or eight of them at a time: taps that leave quarters short or empty,
+    one more than a multiple, more than one round; sequences shorter than their neighbours, whose changes land in the next one's pad."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(11 * m + F)
+    p = _params(rng, m, F, pool, hidden)
+    seqs = _seqs(rng, 9, 1, 30)
+    Zr, mr = orc.gen_predictions({k: v.astype(np.float64) for k, v in p.items()}, seqs, pool, hidden, "logistic", reverse_complement=rc, want_gmaps="finite_diff")
+    Z, maps = predict.gen_predictions(_net(p, m, F, pool, hidden, "nll", rc, 0.0), seqs, want_gmaps="finite_diff")
+    assert_close(Z, Zr, ACT, "Z")
+    scale = max(np.abs(b).max() for _, b in mr)
+    for (sa, a), (sb, b) in zip(maps, mr):
+        assert sa == sb and np.abs(a - b).max() <= GRAD * scale, (len(sa), np.abs(a - b).max(), scale)
+
+
+@pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("n,length", [(80, 57), (300, 101)])
+def test_mutation_maps_do_not_depend_on_how_many_letters_a_workgroup_takes(rc, n, length):
+    """Eight and sixteen letters per workgroup (many sequences) give the bits that four do (one sequence): maxima are the same rows' sums."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(n)
+    net = _net(_params(rng, 24, 16, "max", 32), 24, 16, "max", 32, "nll", rc, 0.0)
+    seqs = _seqs(rng, n, length, length)
+    Z, maps = predict.gen_predictions(net, seqs, want_gmaps="finite_diff")
+    for k in (0, 1, n // 2, n - 1):
+        Z1, one = predict.gen_predictions(net, seqs[k:k + 1], want_gmaps="finite_diff")
+        assert np.array_equal(Z[k:k + 1], Z1) and np.array_equal(maps[k][1], one[0][1])
+
+
+@pytest.mark.parametrize("rc", [False, True])
 @pytest.mark.parametrize("pool,hidden,m,F", [("avg", 6, 24, 16), ("all", 0, 9, 33), ("max", 5, 16, 16), ("avg", 0, 1, 4)])
 def test_mutation_to_the_letter_that_is_there_is_none(pool, hidden, m, F, rc):
     """Exactly zero at every sequence's own letters, wherever in the sequence the workgroup that scores them begins. (Longer sequences
