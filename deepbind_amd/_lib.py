@@ -101,6 +101,7 @@ _SIGNATURES = {
     "dbk_train_step": [_P, _P],
     "dbk_train_steps": [_P, _Z, _P],
     "dbk_train_step_single_workspace": [_P, _P],
+    "dbk_train_step_single_pays": [_P],
     "dbk_longest_region": [_P, _P, _Z, _P],
     "dbk_train_step_single": [_P, _P, _P, _Z],
     "dbk_train_step_args_size": [],

@@ -915,6 +915,23 @@ extern "C" int dbk_train_step_single_workspace(const dbk_train_step_args* a, siz
     return 0;
 }
 
+// A workgroup takes its regions one after the other in lane groups of Fp filters (16, 32 or 64 lanes' worth), where the launches of
+// dbk_train_step spread them over the GPU and scan on the matrix cores. Measured, one launch / several, mean ratio of their times over 390 random
+// shapes of 8-32 taps, regions of 30-280 rows, every pooling, with and without a hidden layer and strands, by regions per workgroup:
+//   16 filters       1: 0.3-0.6   2: 0.66   3: 0.85   4: 0.93   5: 1.02   6: 1.03   7: 1.08   8: 1.12
+//   17-32 filters    1: 0.4-0.6   2: 0.88   3: 1.14   4: 1.30   6: 1.49   8: 1.70
+//   33-64 filters    1: 0.5-0.8   2: 1.30   3: 1.67   4: 2.01   6: 2.57   8: 2.75
+// (1466 regions of 70 rows, 4 models of 16 filters of 26 taps: 102 against 42 us a step.) With the line at 80, 3 % of the shapes are slower than
+// they were by more than 3 %, at most 13 %; the others gain up to a factor of three.
+extern "C" int dbk_train_step_single_pays(const dbk_train_step_args* a)
+{
+    single_args s;
+    unsigned MT;
+    size_t lds;
+    if (!a || !plan(a, s, MT, lds)) return 0;
+    return s.RC == 1u || s.RC * s.Fp <= 80u;
+}
+
 extern "C" int dbk_train_step_single(dbk_stream_t stream, const dbk_train_step_args* a, void* work, size_t work_bytes)
 {
     single_args s;

@@ -187,10 +187,11 @@ class SequenceNet(object):
         self._L_versions = None              # the look-ahead kept beside the parameters no longer matches them
 
     def _single_work(self, buf, R):
-        """Workspace of the single-launch step for this batch shape, or None when the step does not take it."""
+        """Workspace of the single-launch step for this batch shape, or None when the step does not take it or several launches are faster."""
         if "work" not in buf:
             need = ctypes.c_size_t(0)
-            _lib.call("dbk_train_step_single_workspace", ctypes.addressof(self._step_args), ctypes.addressof(need))
+            if _lib.dll().dbk_train_step_single_pays(ctypes.addressof(self._step_args)):
+                _lib.call("dbk_train_step_single_workspace", ctypes.addressof(self._step_args), ctypes.addressof(need))
             buf["work"] = self._workspace(need.value) if need.value else None
         if buf["work"] is None:
             return None

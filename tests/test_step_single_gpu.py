@@ -129,6 +129,28 @@ def test_single_launch_step_is_bit_stable_and_agrees_with_the_multi_launch_step(
         assert_close_per_model(outs[0][pname], outs[2][pname], GRAD, 1, 0, "single vs multi launch %s" % pname)
 
 
+@pytest.mark.parametrize("nm,B,rc,single", [(1, 1280, False, True), (1, 1281, False, False), (2, 512, False, True), (2, 514, True, False),
+                                             (4, 256, False, True), (4, 257, False, False)])
+def test_batches_of_several_regions_per_workgroup_take_the_faster_step(nm, B, rc, single):
+    """One model's 16 filters go through the single launch up to five regions per workgroup, 32 filters up to two, 64 one; beyond, the step is
+    that of several launches (its bits), and its dropout draws go on where the other's would."""
+    rng = np.random.default_rng(B)
+    m = 9
+    X, R = _batch(rng, B // (2 if rc else 1), m, 12, 20, reverse_complement=rc)
+    Y = rng.random((B, nm)).astype(np.float32)
+    nets = [_net(np.random.default_rng(1), nm, 16, m, "all", 8, "nll", rate=0.05, momentum=0.9, dropout=0.5, reverse_complement=rc, single_launch=on)[0]
+            for on in (True, False)]
+    for net in nets:
+        for _ in range(2):
+            net.train_step(dev(X), dev(R), dev(Y))
+    assert nets[0]._last_single == single and not nets[1]._last_single
+    a, b = nets[0].get_params(), nets[1].get_params()
+    for name in a:
+        assert single or np.array_equal(a[name], b[name])
+        assert_close_per_model(a[name], b[name], GRAD, 1, 0, name)
+    assert nets[0]._rng_offset == nets[1]._rng_offset and int(nets[0].rng_counter.item()) == int(nets[1].rng_counter.item())
+
+
 def test_single_launch_step_in_a_graph_and_loss_output():
     rng = np.random.default_rng(8)
     m, B = 16, 128
