@@ -226,21 +226,30 @@ bool pack_shape(const void* U, size_t F, size_t P, const void* pooled, const voi
 
 // flag[0] = 1 when regions are sorted, unit-step and non-overlapping (each map element then has a
 // single writer in the gradient kernel), else 0.
+__device__ __forceinline__ bool disjoint_at(const uint32_t* __restrict__ R, size_t P, bool per_step, size_t r)
+{
+    const unsigned rc = per_step ? 3 : 2;
+    const unsigned a = R[r * rc], b = R[r * rc + 1], step = per_step ? R[r * rc + 2] : 1u, next = r + 1 < P ? R[(r + 1) * rc] : b;
+    return b >= a && step == 1u && next >= b;
+}
+
 __global__ void regions_disjoint_kernel(const uint32_t* __restrict__ R, size_t P, bool per_step, unsigned* flag)
 {
-    __shared__ unsigned bad;
-    if (threadIdx.x == 0) bad = 0;
-    __syncthreads();
-    unsigned mine = 0;
-    const unsigned rc = per_step ? 3 : 2;
-    for (size_t r = threadIdx.x; r < P; r += blockDim.x) {
-        if (R[r * rc + 1] < R[r * rc]) mine = 1;
-        if (per_step && R[r * rc + 2] != 1) mine = 1;
-        if (r + 1 < P && R[(r + 1) * rc] < R[r * rc + 1]) mine = 1;
-    }
-    if (mine) atomicOr(&bad, 1u);
-    __syncthreads();
+    bool bad = false;
+    for (size_t r = threadIdx.x; r < P; r += blockDim.x) bad |= !disjoint_at(R, P, per_step, r);
+    bad = __syncthreads_or(bad) != 0;
     if (threadIdx.x == 0) flag[0] = bad ? 0u : 1u;
+}
+
+// Few regions: every workgroup looks through the whole table itself, and one launch takes the place of three (the look, the kernel for disjoint
+// regions, the one for others, one of which has nothing to do): 1000 regions x 64 float64 columns 13.7 -> 5.5 us. Beyond, the tables that all workgroups
+// read are more than the two launches. All threads of the workgroup come here.
+constexpr size_t CHECK_REGIONS = 2048;
+__device__ __forceinline__ bool all_disjoint(const uint32_t* __restrict__ R, unsigned P, bool per_step)
+{
+    bool bad = false;
+    for (unsigned r = threadIdx.x; r < P; r += 256u) bad |= !disjoint_at(R, P, per_step, r);
+    return __syncthreads_or(bad) == 0;
 }
 
 template <bool ATOMIC, typename T>
@@ -250,19 +259,12 @@ __device__ __forceinline__ void accumulate(T* p, T v)
     else *p += v;
 }
 
-// ATOMIC=false runs when flag says "disjoint" (plain read-modify-write, reproducible);
-// ATOMIC=true runs otherwise (overlapping regions: same accumulation races as any scatter-add).
+// One (region, column). ATOMIC=false: regions are disjoint (plain read-modify-write, reproducible); true: they may overlap (same accumulation
+// races as any scatter-add).
 template <typename T, int PT, bool ATOMIC>
-__global__ __launch_bounds__(256) void poolrgn_bprop_kernel(T* __restrict__ dU, size_t F, size_t nelem_map,
-                                                            const uint32_t* __restrict__ R, size_t P, bool per_step,
-                                                            const T* __restrict__ dP, const uint32_t* __restrict__ argmax,
-                                                            const unsigned* __restrict__ flag)
+__device__ __forceinline__ void poolrgn_bprop_element(size_t r, size_t f, T* __restrict__ dU, size_t F, const uint32_t* __restrict__ R, bool per_step,
+                                                      const T* __restrict__ dP, const uint32_t* __restrict__ argmax)
 {
-    const bool disjoint = flag[0] != 0;
-    if (disjoint == ATOMIC) return;
-    const size_t f = (size_t)blockIdx.y * 64 + (threadIdx.x & 63);
-    const size_t r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (f >= F || r >= P) return;
     const region_t g = load_region(R, r, per_step);
     const size_t j = r * F + f;
     // The argmax index is caller data. One that lies in this thread's own column and region (what the forward
@@ -296,6 +298,27 @@ __global__ __launch_bounds__(256) void poolrgn_bprop_kernel(T* __restrict__ dU, 
     if (PT == DBK_PT_ALL) scatter(dP[2 * j]);
 }
 
+template <typename T, int PT, bool ATOMIC>
+__global__ __launch_bounds__(256) void poolrgn_bprop_kernel(T* __restrict__ dU, size_t F, const uint32_t* __restrict__ R, size_t P, bool per_step,
+                                                            const T* __restrict__ dP, const uint32_t* __restrict__ argmax,
+                                                            const unsigned* __restrict__ flag)
+{
+    if ((flag[0] != 0) == ATOMIC) return;
+    const size_t f = (size_t)blockIdx.y * 64 + (threadIdx.x & 63), r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (f < F && r < P) poolrgn_bprop_element<T, PT, ATOMIC>(r, f, dU, F, R, per_step, dP, argmax);
+}
+
+template <typename T, int PT>
+__global__ __launch_bounds__(256) void poolrgn_bprop_check_kernel(T* __restrict__ dU, size_t F, const uint32_t* __restrict__ R, unsigned P, bool per_step,
+                                                                  const T* __restrict__ dP, const uint32_t* __restrict__ argmax)
+{
+    const bool disjoint = all_disjoint(R, P, per_step);
+    const size_t f = (size_t)blockIdx.y * 64 + (threadIdx.x & 63), r = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (f >= F || r >= P) return;
+    if (disjoint) poolrgn_bprop_element<T, PT, false>(r, f, dU, F, R, per_step, dP, argmax);
+    else poolrgn_bprop_element<T, PT, true>(r, f, dU, F, R, per_step, dP, argmax);
+}
+
 // The gradient of average / sum / max+average pooling with sixteen bytes per lane (regions disjoint, rows whole packs):
 // thread t adds to pack t % (F / V) of every row of region t / (F / V), as poolrgn_pack_kernel reads them; every column
 // receives what poolrgn_bprop_kernel<.., false> gives it, in the same order (the share of the average first, then the
@@ -303,18 +326,26 @@ __global__ __launch_bounds__(256) void poolrgn_bprop_kernel(T* __restrict__ dU, 
 // PASS (max+average): the maximum's share goes in as its row passes, with the same additions, instead of in four reads and writes of single
 // elements behind the loop, each of a whole line that has left the caches by then: 8192 regions x 124 rows x 256 float32 545 -> 434 us,
 // 20 000 x 60 x 64 163 -> 131. A map that stays in the caches is faster without (1000 x 123 x 64: 21 us against 24).
-template <typename T, int PT, bool PASS>
+// CHECK: the workgroup looks through the table of regions itself (flag is not read).
+template <typename T, int PT, bool PASS, bool CHECK = false>
 __global__ __launch_bounds__(256) void poolrgn_bprop_pack_kernel(T* __restrict__ dU, unsigned F, const uint32_t* __restrict__ R, unsigned P,
                                                                  bool per_step, const T* __restrict__ dP,
                                                                  const uint32_t* __restrict__ argmax, const unsigned* __restrict__ flag)
 {
     using V4 = typename pack_t<T>::type;
     constexpr int V = pack_t<T>::V;
-    if (flag[0] == 0) return;                                        // overlapping regions: the atomic kernel runs instead
+    bool disjoint = true;
+    if (CHECK) disjoint = all_disjoint(R, P, per_step);
+    else if (flag[0] == 0) return;                                   // overlapping regions: the atomic kernel runs instead
     const unsigned Fp = F / V;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)P * Fp) return;
     const unsigned r = (unsigned)(t / Fp), f = (unsigned)(t - (size_t)r * Fp) * V;
+    if (CHECK && !disjoint) {
+#pragma unroll 1
+        for (int k = 0; k < V; ++k) poolrgn_bprop_element<T, PT, true>(r, f + k, dU, F, R, per_step, dP, argmax);
+        return;
+    }
     const region_t g = load_region(R, r, per_step);
     const size_t j = (size_t)r * F + f;
     V4 dy;
@@ -420,13 +451,21 @@ void launch_bwd_pt(hipStream_t st, T* dU, size_t F, const uint32_t* R, size_t P,
     dim3 grid(dbk::divup(P, 4), dbk::divup(F, 64)), block(256);
     if (PT != DBK_PT_MAX && pack_shape<T>(dU, F, P, dP, nullptr)) {
         // (the map's rows are only known on the device: 262 144 packs of regions of ~60 rows and more leave the caches)
-        auto kern = PT == DBK_PT_ALL && P * (F / (16 / sizeof(T))) >= 262144 ? poolrgn_bprop_pack_kernel<T, PT, PT == DBK_PT_ALL> : poolrgn_bprop_pack_kernel<T, PT, false>;
-        hipLaunchKernelGGL(kern, dim3(dbk::divup(P * (F / (16 / sizeof(T))), 256)), block, PACK_LDS_CAP, st, dU, (unsigned)F, R,
-                           (unsigned)P, per_step, dP, argmax, flag);
-    }
-    else
-        hipLaunchKernelGGL((poolrgn_bprop_kernel<T, PT, false>), grid, block, 0, st, dU, F, (size_t)0, R, P, per_step, dP, argmax, flag);
-    hipLaunchKernelGGL((poolrgn_bprop_kernel<T, PT, true>), grid, block, 0, st, dU, F, (size_t)0, R, P, per_step, dP, argmax, flag);
+        const size_t packs = P * (F / (16 / sizeof(T)));
+        const dim3 wgs(dbk::divup(packs, 256));
+        if (!flag) {
+            auto kern = PT == DBK_PT_ALL && packs >= 262144 ? poolrgn_bprop_pack_kernel<T, PT, PT == DBK_PT_ALL, true> : poolrgn_bprop_pack_kernel<T, PT, false, true>;
+            hipLaunchKernelGGL(kern, wgs, block, PACK_LDS_CAP, st, dU, (unsigned)F, R, (unsigned)P, per_step, dP, argmax, flag);
+            return;
+        }
+        auto kern = PT == DBK_PT_ALL && packs >= 262144 ? poolrgn_bprop_pack_kernel<T, PT, PT == DBK_PT_ALL> : poolrgn_bprop_pack_kernel<T, PT, false>;
+        hipLaunchKernelGGL(kern, wgs, block, PACK_LDS_CAP, st, dU, (unsigned)F, R, (unsigned)P, per_step, dP, argmax, flag);
+    } else if (!flag) {
+        hipLaunchKernelGGL((poolrgn_bprop_check_kernel<T, PT>), grid, block, 0, st, dU, F, R, (unsigned)P, per_step, dP, argmax);
+        return;
+    } else
+        hipLaunchKernelGGL((poolrgn_bprop_kernel<T, PT, false>), grid, block, 0, st, dU, F, R, P, per_step, dP, argmax, flag);
+    hipLaunchKernelGGL((poolrgn_bprop_kernel<T, PT, true>), grid, block, 0, st, dU, F, R, P, per_step, dP, argmax, flag);
 }
 
 template <typename T>
@@ -434,9 +473,12 @@ int launch_bwd(hipStream_t st, T* dU, size_t F, const uint32_t* R, size_t P, boo
                const uint32_t* argmax, int ptype)
 {
     DBK_CHECK(dbk::divup(F, 64) <= 65535u, "ValueError: too many feature maps (%zu) for one launch", F);
-    unsigned* flag = (unsigned*)dbk::workspace(256, st);
-    DBK_CHECK(flag != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
-    hipLaunchKernelGGL(regions_disjoint_kernel, dim3(1), dim3(1024), 0, st, R, P, per_step, flag);
+    unsigned* flag = nullptr;
+    if (P > CHECK_REGIONS) {
+        flag = (unsigned*)dbk::workspace(256, st);
+        DBK_CHECK(flag != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
+        hipLaunchKernelGGL(regions_disjoint_kernel, dim3(1), dim3(1024), 0, st, R, P, per_step, flag);
+    }
     switch (ptype) {
     case DBK_PT_MAX: launch_bwd_pt<T, DBK_PT_MAX>(st, dU, F, R, P, per_step, dP, argmax, flag); break;
     case DBK_PT_AVG: launch_bwd_pt<T, DBK_PT_AVG>(st, dU, F, R, P, per_step, dP, argmax, flag); break;

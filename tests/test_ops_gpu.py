@@ -362,6 +362,34 @@ def test_poolrgn_bprop_all_of_many_packs(ks, dtype, P, F, stepped):
 
 
 # ------------------------------------------------------------------------------------------ fused scan + pool
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("P,F,dtype", [(2048, 5, np.float32), (2049, 5, np.float32), (2048, 8, np.float64), (2049, 8, np.float64), (300, 8, np.float32), (2048, 512, np.float32)])
+@pytest.mark.parametrize("overlap", [False, True])
+def test_poolrgn_bprop_finds_overlapping_regions(ks, overlap, P, F, dtype, ptype):
+    """One region among many that lies over others, on either side of the number of regions up to which every workgroup looks through the
+    table itself: shares of the same rows all count."""
+    rng = np.random.default_rng(P + F)
+    edges = np.concatenate([[0], np.cumsum(rng.integers(0 if ptype == "avg" else 1, 9, P))])
+    R = np.stack([edges[:-1], edges[1:]], axis=1).astype(np.uint32)
+    R = R[R[:, 1] > R[:, 0]]
+    if overlap:
+        R[len(R) // 2 + 1] = [3, 40]
+    U = rng.standard_normal((int(edges[-1]), F)).astype(dtype)
+    dP = rng.standard_normal((len(R), F * (2 if ptype == "all" else 1))).astype(dtype)
+    pooled, arg = ks.poolrgn(dev(U), dev(R), ptype, want_argmax=ptype != "avg")
+    want = U.astype(np.float64)
+    top = dP[:, 0::2] if ptype == "all" else dP
+    if ptype != "avg":
+        np.add.at(want.reshape(-1), host(arg).astype(np.int64).ravel(), top.astype(np.float64).ravel())
+    if ptype != "max":
+        mean = dP[:, 1::2] if ptype == "all" else dP
+        for r, (a, e) in enumerate(R.astype(int)):
+            want[a:e] += mean[r].astype(np.float64) / (e - a)
+    dU = dev(U.copy())
+    ks.poolrgn_bprop(dU, dev(R), dev(dP), arg if ptype != "avg" else None, ptype)
+    assert np.abs(host(dU) - want).max() <= (2e-6 if dtype == np.float32 else 4e-15)
+
+
 def _chain_oracle(W, b, X, R, ptype):
     Z = np.zeros((X.size, W.shape[1]), W.dtype)
     orc.corr1ord(W, X, Z)
