@@ -377,6 +377,39 @@ __device__ __forceinline__ float slab_sum(const float* __restrict__ slabs, size_
     return total;
 }
 
+// The same sum, bit for bit, of 64 elements by a workgroup of four waves: each takes every fourth of the trees, four of them in flight, and the first
+// adds them up. (Many slabs of few elements leave a thread per element waiting for one round after the other.) The result is the first wave's.
+constexpr unsigned SUM_TREES = 32;
+__device__ __forceinline__ float slab_sum_together(const float* __restrict__ slabs, size_t nelem, size_t e, bool active, unsigned nslab, float (&trees)[SUM_TREES][64])
+{
+    const unsigned lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    float total = 0.0f;
+    for (unsigned base = 0; base < nslab; base += 8 * SUM_TREES) {
+        const unsigned left = (nslab - base + 7) / 8, n = left < SUM_TREES ? left : SUM_TREES;
+        if (active) {
+            for (unsigned j0 = wave; j0 < n; j0 += 16) {
+                float buf[4][8];
+#pragma unroll
+                for (unsigned q = 0; q < 4; ++q)
+#pragma unroll
+                    for (unsigned s = 0; s < 8; ++s) {
+                        const unsigned slab = base + 8 * (j0 + 4 * q) + s;
+                        buf[q][s] = slab < nslab ? slabs[(size_t)slab * nelem + e] : 0.0f;
+                    }
+#pragma unroll
+                for (unsigned q = 0; q < 4; ++q)
+                    if (j0 + 4 * q < n)
+                        trees[j0 + 4 * q][lane] = ((buf[q][0] + buf[q][1]) + (buf[q][2] + buf[q][3])) + ((buf[q][4] + buf[q][5]) + (buf[q][6] + buf[q][7]));
+            }
+        }
+        __syncthreads();
+        if (active && wave == 0u)
+            for (unsigned j = 0; j < n; ++j) total += trees[j][lane];
+        __syncthreads();
+    }
+    return total;
+}
+
 inline size_t lds_limit()
 {
     // LDS bytes a workgroup may use on the current device (asked once per device)

@@ -49,23 +49,43 @@ struct reduce_update_args {
 __device__ __forceinline__ float chunk_sum(const reduce_update_args& a, unsigned b, unsigned idx)
 {
     float s = 0.0f;
-    for (unsigned c0 = 0; c0 < a.nchunk; c0 += 8) {                // eight chunks in flight per round, added in ascending order
-        float v[8];
+    for (unsigned c0 = 0; c0 < a.nchunk; c0 += 16) {               // sixteen chunks in flight per round, added in ascending order
+        float v[16];
 #pragma unroll
-        for (unsigned t = 0; t < 8; ++t) v[t] = c0 + t < a.nchunk ? a.head_partial[((size_t)(c0 + t) * a.nblock + b) * a.pstride + idx] : 0.0f;
+        for (unsigned t = 0; t < 16; ++t) v[t] = c0 + t < a.nchunk ? a.head_partial[((size_t)(c0 + t) * a.nblock + b) * a.pstride + idx] : 0.0f;
 #pragma unroll
-        for (unsigned t = 0; t < 8; ++t)
+        for (unsigned t = 0; t < 16; ++t)
             if (c0 + t < a.nchunk) s += v[t];
     }
     return s;
 }
 
+// From how many slabs on a workgroup sums 64 elements together instead of 256 one by one (slab_sum_together), and the workgroups of a vector.
+// What bounds it is latency: 256 slabs were eight rounds of loads for a thread per element, 98 workgroups in all. us a launch, one by one / together: 1024 pairs of
+// 90-200 letters x 8 models x 16 filters of 32 taps (256 slabs of 16 640 elements) 10.5 / 7.7; 700 x 100-200 x 4 of 30 taps 7.9 / 6.2. With the
+// calibration's 21 slabs a thread per element has all of them in flight.
+constexpr unsigned TOGETHER_SLABS = 32;
+inline unsigned update_grid(size_t elements, unsigned nslab) { return nslab > TOGETHER_SLABS ? dbk::ew_grid(elements, 64) : dbk::ew_grid(elements); }
+
 // bx of gx: this workgroup's place among those that share the vector
+template <bool TOGETHER>
 __device__ __forceinline__ void reduce_update_body(const reduce_update_args& a, const unsigned bx, const unsigned gx)
 {
+    __shared__ float trees[dbk_scan::SUM_TREES][64];
+    const unsigned per = TOGETHER ? 64u : blockDim.x, mine = TOGETHER ? threadIdx.x & 63u : threadIdx.x;
     const unsigned nW1m = a.k * a.h1;                              // dense weights per model
     const unsigned total = a.nparam + (a.loss ? a.nblock : 0u);
-    for (unsigned e = bx * blockDim.x + threadIdx.x; e < total; e += gx * blockDim.x) {
+    for (unsigned e0 = bx * per; e0 < total; e0 += gx * per) {
+        const unsigned e = e0 + mine;
+        float scan = 0.0f;
+        if (TOGETHER) {
+            // (the scan's weights and biases are the slabs' elements; a group of 64 may reach past either)
+            const bool weight = e < total && e - a.off_Wc < a.nWc, bias = e < total && e - a.off_bc < a.nbc;
+            if (__syncthreads_or(weight || bias))
+                scan = dbk_scan::slab_sum_together(a.slabs, a.slab_stride, weight ? e - a.off_Wc : a.nWc + (e - a.off_bc), weight || bias, a.nslab, trees);
+            if (threadIdx.x >= 64u) continue;
+        }
+        if (e >= total) continue;
         if (e >= a.nparam) {                                       // per-model loss
             const unsigned b = (unsigned)(e - a.nparam);
             const float s = chunk_sum(a, b, nW1m + 2 * a.h1 + 1);
@@ -74,8 +94,8 @@ __device__ __forceinline__ void reduce_update_body(const reduce_update_args& a, 
         }
         float g;
         bool scan_weight = false;
-        if (e - a.off_Wc < a.nWc) { g = dbk_scan::slab_sum(a.slabs, a.slab_stride, e - a.off_Wc, a.nslab); scan_weight = true; }
-        else if (e - a.off_bc < a.nbc) g = dbk_scan::slab_sum(a.slabs, a.slab_stride, a.nWc + (e - a.off_bc), a.nslab);
+        if (e - a.off_Wc < a.nWc) { g = TOGETHER ? scan : dbk_scan::slab_sum(a.slabs, a.slab_stride, e - a.off_Wc, a.nslab); scan_weight = true; }
+        else if (e - a.off_bc < a.nbc) g = TOGETHER ? scan : dbk_scan::slab_sum(a.slabs, a.slab_stride, a.nWc + (e - a.off_bc), a.nslab);
         else if (e - a.off_W1 < a.nW1) { const unsigned q = e - a.off_W1, b = q / nW1m; g = chunk_sum(a, b, q - b * nW1m); }
         else if (e - a.off_b1 < a.nb1) { const unsigned q = e - a.off_b1, b = q / a.h1; g = chunk_sum(a, b, nW1m + (q - b * a.h1)); }
         else if (e - a.off_W2 < a.nW2) { const unsigned q = e - a.off_W2, b = q / a.hidden; g = chunk_sum(a, b, nW1m + a.h1 + (q - b * a.hidden)); }
@@ -99,7 +119,13 @@ __device__ __forceinline__ void reduce_update_body(const reduce_update_args& a, 
     if (a.counter && a.counter_advance && bx == 0 && threadIdx.x == 0) a.counter[0] += a.counter_advance;
 }
 
-__global__ __launch_bounds__(256) void k_reduce_update(reduce_update_args a) { reduce_update_body(a, blockIdx.x, gridDim.x); }
+__device__ __forceinline__ void reduce_update(const reduce_update_args& a, const unsigned bx, const unsigned gx)
+{
+    if (a.nslab > TOGETHER_SLABS) reduce_update_body<true>(a, bx, gx);
+    else reduce_update_body<false>(a, bx, gx);
+}
+
+__global__ __launch_bounds__(256) void k_reduce_update(reduce_update_args a) { reduce_update(a, blockIdx.x, gridDim.x); }
 
 // The same for several model groups in one launch: workgroups first[g] .. first[g+1]-1 share group g's vector.
 struct reduce_update_multi_args {
@@ -111,7 +137,7 @@ __global__ __launch_bounds__(256) void k_reduce_update_multi(const reduce_update
 {
     unsigned g = 0;
     while (g + 1 < m.n && blockIdx.x >= m.first[g + 1]) ++g;
-    reduce_update_body(m.g[g], blockIdx.x - m.first[g], m.first[g + 1] - m.first[g]);
+    reduce_update(m.g[g], blockIdx.x - m.first[g], m.first[g + 1] - m.first[g]);
 }
 
 // Look-ahead vectors of several groups in one launch (L = P + mrate*mP, as k_lookahead forms it).
@@ -262,7 +288,7 @@ extern "C" int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* a)
         reduce_update_args u;
         rc = fill_update(u, a, z, later.slabs, later.slab_stride, later.nslab, later.head_partial, later.head_nchunk, later.head_pstride, draws);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_reduce_update, dim3(dbk::ew_grid(a->nparam + a->nmodel)), dim3(256), 0, dbk::as_stream(stream), u);
+        hipLaunchKernelGGL(k_reduce_update, dim3(update_grid(a->nparam + a->nmodel, u.nslab)), dim3(256), 0, dbk::as_stream(stream), u);
         DBK_LAUNCH_OK();
     }
     if (a->decay) {
@@ -369,7 +395,7 @@ extern "C" int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_tra
         const dbk_train_step_args* a = ord[i];
         rc = fill_update(um.g[i], a, sizes_of(a), sg[i].slabs, sg[i].slab_stride, sg[i].nslab, hg[i].partial, hg[i].nchunk, hg[i].pstride, draws[i]);
         if (rc) return rc;
-        um.first[i + 1] = um.first[i] + dbk::ew_grid(a->nparam + a->nmodel);
+        um.first[i + 1] = um.first[i] + update_grid(a->nparam + a->nmodel, um.g[i].nslab);
     }
     hipLaunchKernelGGL(k_reduce_update_multi, dim3(um.first[n]), dim3(256), 0, st, um);
     DBK_LAUNCH_OK();

@@ -741,6 +741,33 @@ def test_natively_issued_step_equals_the_step_issued_call_by_call(pool, hidden, 
                 assert np.array_equal(getattr(native, name).cpu().numpy(), getattr(stepwise, name).cpu().numpy()), (change, name)
 
 
+@pytest.mark.parametrize("ni,nf,m,pool,hidden,rows", [(1, 5, 7, "max", 0, 33), (3, 7, 11, "avg", 4, 70), (5, 13, 9, "all", 32, 300), (2, 16, 24, "max", 3, 1100),
+                                                      (9, 16, 16, "all", 0, 523)])
+def test_the_update_sums_many_slabs_as_the_gradient_does(ni, nf, m, pool, hidden, rows):
+    """From 33 slabs on four waves of the step's last kernel sum 64 elements together: the bits are those of the gradient's own kernel, whose
+    sums go one by one, for vectors that are no whole groups of 64, groups that reach from the scan's parameters into the head's, and
+    more slabs than one round takes."""
+    from deepbind_amd import data, deepity_smat as ds
+    from deepbind_amd.model import SequenceNet
+    rng = np.random.default_rng(rows)
+    seqs = ["".join(rng.choice(list("ACGT"), size=rng.integers(10, 40))) for _ in range(rows)]
+    X, R = [dev(v) for v in data.pack_sequences(seqs, m - 1)]
+    Y = dev(rng.random((rows, ni)).astype(np.float32))
+    nets = []
+    for _ in range(2):
+        net = SequenceNet(ni, nf, m, pool=pool, hidden=hidden, loss="mse", rate=0.05, momentum=0.8, decay_conv=1e-3, decay_full=1e-3,
+                          weight_decay_start=0, single_launch=False)
+        net.init_params(0.3, 0.3, 0.05, seed=4)
+        nets.append(net)
+    native, stepwise = nets
+    for _ in range(2):
+        native.train_step(X, R, Y)
+        ds.gradstep(stepwise.P, stepwise.dP, stepwise.drate, stepwise.mP, stepwise.mrate, lambda: stepwise._grad_fused(X, R, Y, None, None), nesterov=True)
+        stepwise.step_count += 1
+        for name in ("P", "dP", "mP"):
+            assert torch.equal(getattr(native, name), getattr(stepwise, name)), name
+
+
 def test_groups_stepped_in_shared_launches_match_groups_stepped_alone_across_changing_batches():
     """ModelGroup.train_step issues one launch per phase for all its architecture groups (dbk_train_steps);
     every group must end with the bits of its own dbk_train_step, across a change of targets, a smaller batch,
