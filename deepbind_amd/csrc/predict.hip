@@ -124,16 +124,17 @@ __device__ __forceinline__ void letter_table16(float* __restrict__ lut, const fl
 }
 
 // Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending. A letter is read once for the four rows it meets.
-__device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, float (&z)[4])
+// (It passes a comparison that never holds: without it the reads are ordered otherwise, 4140 windows of 55 rows 14.1 -> 15.3 us; by words of four letters 14.8.)
+__device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, float (&z)[4], unsigned at = ~0u)
 {
     z[0] = z[1] = z[2] = z[3] = 0.0f;
     unsigned l[4];
 #pragma unroll
-    for (unsigned u = 0; u < 3; ++u) l[u + 1] = let[p + u];
+    for (unsigned u = 0; u < 3; ++u) l[u + 1] = p + u == at ? 0u : let[p + u];
 #pragma unroll 4
     for (unsigned j = 0; j < m; ++j) {
         l[0] = l[1]; l[1] = l[2]; l[2] = l[3];
-        l[3] = let[p + 3 + j];
+        l[3] = p + 3 + j == at ? 0u : let[p + 3 + j];
         const float* t = lut_f + j * NL * MUT_F;
 #pragma unroll
         for (unsigned u = 0; u < 4; ++u) z[u] += t[l[u]];
