@@ -46,15 +46,17 @@ struct reduce_update_args {
     unsigned long long* counter; unsigned long long counter_advance;
 };
 
+// FLY chunks in flight per round, added in ascending order
+template <unsigned FLY>
 __device__ __forceinline__ float chunk_sum(const reduce_update_args& a, unsigned b, unsigned idx)
 {
     float s = 0.0f;
-    for (unsigned c0 = 0; c0 < a.nchunk; c0 += 16) {               // sixteen chunks in flight per round, added in ascending order
-        float v[16];
+    for (unsigned c0 = 0; c0 < a.nchunk; c0 += FLY) {
+        float v[FLY];
 #pragma unroll
-        for (unsigned t = 0; t < 16; ++t) v[t] = c0 + t < a.nchunk ? a.head_partial[((size_t)(c0 + t) * a.nblock + b) * a.pstride + idx] : 0.0f;
+        for (unsigned t = 0; t < FLY; ++t) v[t] = c0 + t < a.nchunk ? a.head_partial[((size_t)(c0 + t) * a.nblock + b) * a.pstride + idx] : 0.0f;
 #pragma unroll
-        for (unsigned t = 0; t < 16; ++t)
+        for (unsigned t = 0; t < FLY; ++t)
             if (c0 + t < a.nchunk) s += v[t];
     }
     return s;
@@ -67,65 +69,81 @@ __device__ __forceinline__ float chunk_sum(const reduce_update_args& a, unsigned
 constexpr unsigned TOGETHER_SLABS = 32;
 inline unsigned update_grid(size_t elements, unsigned nslab) { return nslab > TOGETHER_SLABS ? dbk::ew_grid(elements, 64) : dbk::ew_grid(elements); }
 
+template <unsigned FLY>
+__device__ __forceinline__ void update_loss(const reduce_update_args& a, unsigned b)
+{
+    const float s = chunk_sum<FLY>(a, b, a.k * a.h1 + 2 * a.h1 + 1);
+    a.loss[b] = dbk::loss_mean(a.loss_kind, s, (float)a.nrow);
+}
+
+// the gradient of a parameter of the head
+template <unsigned FLY>
+__device__ __forceinline__ float head_gradient(const reduce_update_args& a, unsigned e, unsigned nW1m)
+{
+    if (e - a.off_W1 < a.nW1) { const unsigned q = e - a.off_W1, b = q / nW1m; return chunk_sum<FLY>(a, b, q - b * nW1m); }
+    if (e - a.off_b1 < a.nb1) { const unsigned q = e - a.off_b1, b = q / a.h1; return chunk_sum<FLY>(a, b, nW1m + (q - b * a.h1)); }
+    if (e - a.off_W2 < a.nW2) { const unsigned q = e - a.off_W2, b = q / a.hidden; return chunk_sum<FLY>(a, b, nW1m + a.h1 + (q - b * a.hidden)); }
+    return chunk_sum<FLY>(a, e - a.off_b2, nW1m + 2 * a.h1);
+}
+
+__device__ __forceinline__ void update_parameter(const reduce_update_args& a, unsigned e, float g, bool scan_weight)
+{
+    const float look = a.L[e];
+    if (a.decay) {
+        const float sg = (float)((look > 0.0f) - (look < 0.0f));
+        g += sg * a.decay[e];
+    }
+    if (scan_weight && a.freeze_scan) g = 0.0f;
+    a.dP[e] = g;
+    const float rm = a.mrate[e];
+    const float delta = g * a.drate[e];
+    const float mom = a.mP[e] * rm - delta;
+    const float pn = look - delta;
+    a.mP[e] = mom;
+    a.P[e] = pn;
+    a.L[e] = pn + rm * mom;
+}
+
 // bx of gx: this workgroup's place among those that share the vector
 template <bool TOGETHER>
 __device__ __forceinline__ void reduce_update_body(const reduce_update_args& a, const unsigned bx, const unsigned gx)
 {
-    __shared__ float trees[dbk_scan::SUM_TREES][64];
-    const unsigned per = TOGETHER ? 64u : blockDim.x, mine = TOGETHER ? threadIdx.x & 63u : threadIdx.x;
     const unsigned nW1m = a.k * a.h1;                              // dense weights per model
     const unsigned total = a.nparam + (a.loss ? a.nblock : 0u);
-    for (unsigned e0 = bx * per; e0 < total; e0 += gx * per) {
-        const unsigned e = e0 + mine;
-        float scan = 0.0f;
-        if (TOGETHER) {
+    if constexpr (TOGETHER) {
+        __shared__ float trees[dbk_scan::SUM_TREES][64];
+        for (unsigned e0 = bx * 64u; e0 < total; e0 += gx * 64u) {
             // (the scan's weights and biases are the slabs' elements; a group of 64 may reach past either)
+            const unsigned e = e0 + (threadIdx.x & 63u);
             const bool weight = e < total && e - a.off_Wc < a.nWc, bias = e < total && e - a.off_bc < a.nbc;
+            float scan = 0.0f;
             if (__syncthreads_or(weight || bias))
                 scan = dbk_scan::slab_sum_together(a.slabs, a.slab_stride, weight ? e - a.off_Wc : a.nWc + (e - a.off_bc), weight || bias, a.nslab, trees);
-            if (threadIdx.x >= 64u) continue;
+            if (threadIdx.x >= 64u || e >= total) continue;
+            if (e >= a.nparam) update_loss<16>(a, e - a.nparam);
+            else update_parameter(a, e, weight || bias ? scan : head_gradient<16>(a, e, nW1m), weight);
         }
-        if (e >= total) continue;
-        if (e >= a.nparam) {                                       // per-model loss
-            const unsigned b = (unsigned)(e - a.nparam);
-            const float s = chunk_sum(a, b, nW1m + 2 * a.h1 + 1);
-            a.loss[b] = dbk::loss_mean(a.loss_kind, s, (float)a.nrow);
-            continue;
+    } else {
+        for (unsigned e = bx * blockDim.x + threadIdx.x; e < total; e += gx * blockDim.x) {
+            if (e >= a.nparam) {                                   // per-model loss
+                update_loss<8>(a, e - a.nparam);
+                continue;
+            }
+            float g;
+            bool scan_weight = false;
+            if (e - a.off_Wc < a.nWc) { g = dbk_scan::slab_sum(a.slabs, a.slab_stride, e - a.off_Wc, a.nslab); scan_weight = true; }
+            else if (e - a.off_bc < a.nbc) g = dbk_scan::slab_sum(a.slabs, a.slab_stride, a.nWc + (e - a.off_bc), a.nslab);
+            else g = head_gradient<8>(a, e, nW1m);
+            update_parameter(a, e, g, scan_weight);
         }
-        float g;
-        bool scan_weight = false;
-        if (e - a.off_Wc < a.nWc) { g = TOGETHER ? scan : dbk_scan::slab_sum(a.slabs, a.slab_stride, e - a.off_Wc, a.nslab); scan_weight = true; }
-        else if (e - a.off_bc < a.nbc) g = TOGETHER ? scan : dbk_scan::slab_sum(a.slabs, a.slab_stride, a.nWc + (e - a.off_bc), a.nslab);
-        else if (e - a.off_W1 < a.nW1) { const unsigned q = e - a.off_W1, b = q / nW1m; g = chunk_sum(a, b, q - b * nW1m); }
-        else if (e - a.off_b1 < a.nb1) { const unsigned q = e - a.off_b1, b = q / a.h1; g = chunk_sum(a, b, nW1m + (q - b * a.h1)); }
-        else if (e - a.off_W2 < a.nW2) { const unsigned q = e - a.off_W2, b = q / a.hidden; g = chunk_sum(a, b, nW1m + a.h1 + (q - b * a.hidden)); }
-        else { const unsigned q = e - a.off_b2; g = chunk_sum(a, q, nW1m + 2 * a.h1); }
-        const float look = a.L[e];
-        if (a.decay) {
-            const float sg = (float)((look > 0.0f) - (look < 0.0f));
-            g += sg * a.decay[e];
-        }
-        if (scan_weight && a.freeze_scan) g = 0.0f;
-        a.dP[e] = g;
-        const float rm = a.mrate[e];
-        const float delta = g * a.drate[e];
-        const float mom = a.mP[e] * rm - delta;
-        const float pn = look - delta;
-        a.mP[e] = mom;
-        a.P[e] = pn;
-        a.L[e] = pn + rm * mom;
     }
     // every workgroup of the head kernel has read the generator position long ago: move it on
     if (a.counter && a.counter_advance && bx == 0 && threadIdx.x == 0) a.counter[0] += a.counter_advance;
 }
 
-__device__ __forceinline__ void reduce_update(const reduce_update_args& a, const unsigned bx, const unsigned gx)
-{
-    if (a.nslab > TOGETHER_SLABS) reduce_update_body<true>(a, bx, gx);
-    else reduce_update_body<false>(a, bx, gx);
-}
-
-__global__ __launch_bounds__(256) void k_reduce_update(reduce_update_args a) { reduce_update(a, blockIdx.x, gridDim.x); }
+// (kernels of their own, so that few slabs are not summed at the occupancy of many)
+template <bool TOGETHER>
+__global__ __launch_bounds__(256) void k_reduce_update(reduce_update_args a) { reduce_update_body<TOGETHER>(a, blockIdx.x, gridDim.x); }
 
 // The same for several model groups in one launch: workgroups first[g] .. first[g+1]-1 share group g's vector.
 struct reduce_update_multi_args {
@@ -133,11 +151,15 @@ struct reduce_update_multi_args {
     unsigned first[dbk::MULTI_MAX + 1];
     reduce_update_args g[dbk::MULTI_MAX];
 };
+// TOGETHER: some of the groups have many slabs
+template <bool TOGETHER>
 __global__ __launch_bounds__(256) void k_reduce_update_multi(const reduce_update_multi_args m)
 {
     unsigned g = 0;
     while (g + 1 < m.n && blockIdx.x >= m.first[g + 1]) ++g;
-    reduce_update(m.g[g], blockIdx.x - m.first[g], m.first[g + 1] - m.first[g]);
+    const unsigned bx = blockIdx.x - m.first[g], gx = m.first[g + 1] - m.first[g];
+    if (TOGETHER && m.g[g].nslab > TOGETHER_SLABS) reduce_update_body<true>(m.g[g], bx, gx);
+    else reduce_update_body<false>(m.g[g], bx, gx);
 }
 
 // Look-ahead vectors of several groups in one launch (L = P + mrate*mP, as k_lookahead forms it).
@@ -288,7 +310,8 @@ extern "C" int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* a)
         reduce_update_args u;
         rc = fill_update(u, a, z, later.slabs, later.slab_stride, later.nslab, later.head_partial, later.head_nchunk, later.head_pstride, draws);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_reduce_update, dim3(update_grid(a->nparam + a->nmodel, u.nslab)), dim3(256), 0, dbk::as_stream(stream), u);
+        auto kern = u.nslab > TOGETHER_SLABS ? k_reduce_update<true> : k_reduce_update<false>;
+        hipLaunchKernelGGL(kern, dim3(update_grid(a->nparam + a->nmodel, u.nslab)), dim3(256), 0, dbk::as_stream(stream), u);
         DBK_LAUNCH_OK();
     }
     if (a->decay) {
@@ -397,7 +420,10 @@ extern "C" int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_tra
         if (rc) return rc;
         um.first[i + 1] = um.first[i] + update_grid(a->nparam + a->nmodel, um.g[i].nslab);
     }
-    hipLaunchKernelGGL(k_reduce_update_multi, dim3(um.first[n]), dim3(256), 0, st, um);
+    bool many = false;
+    for (unsigned i = 0; i < n; ++i) many |= um.g[i].nslab > TOGETHER_SLABS;
+    auto kern = many ? k_reduce_update_multi<true> : k_reduce_update_multi<false>;
+    hipLaunchKernelGGL(kern, dim3(um.first[n]), dim3(256), 0, st, um);
     DBK_LAUNCH_OK();
 }
 
