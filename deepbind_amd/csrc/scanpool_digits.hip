@@ -33,7 +33,7 @@
 // Bound: the matrix pipe, and through it the chip's power: an instruction takes its 34 clocks, at 1.5-1.6 GHz under this
 // load (2.3 GHz with all operands zero), 22 ns per SIMD. A table of 3-mer sums in LDS (one 4-byte read and add per three
 // taps), which this replaced, moved its 248 ns worth of LDS bytes per 32 x 32 tile of 24 taps; nine instructions are 198.
-// Measured, table / all digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 10.4 ms (8.1 through half of the
+// Measured, table / all digits: max pooling, 100 000 x 500 letters x 1024 filters x 24 taps 12.8 / 10.4 ms (7.35 through half of the
 // products, scanpool_digits_max_kernel below); 65 536 x 101 x 256
 // filters, 24 taps 0.721 / 0.513, 16 taps 0.552 / 0.380; 20 000 x 500 x 256 x 8 taps 0.491 / 0.261; max + average, 20 000 x
 // 30-150 x 384 x 16 taps 0.275 / 0.215 (0.19 now: launch_sets, scanpool_digits_body); with an argmax 65 536 x 101 x 256 x 24 taps 0.867 / 0.616; averages are off by
@@ -1079,7 +1079,7 @@ int launch(hipStream_t st, const digit_store& D, const float* W, const float* bi
 
 // Whether plain maxima go through half the products: filters of more than 16 taps, more than 32 of them (a wave takes 64),
 // regions of 80 rows on average and eight of them per wave. Measured, all the products / half of them, 24 taps: 100 000 x
-// 500 letters x 1024 filters 10.4 / 8.1 ms, 65 536 x 101 x 256 0.515 / 0.461, 8192 x 101 x 256 0.080 / 0.078, 100 000 x 40 x
+// 500 letters x 1024 filters 10.4 / 8.1 ms (7.35 since the halves take turns), 65 536 x 101 x 256 0.515 / 0.461, 8192 x 101 x 256 0.080 / 0.078, 100 000 x 40 x
 // 64 0.134 / 0.137, 2000 x 500 x 64 0.034 / 0.049; 16 taps, 65 536 x 101 x 256 0.361 / 0.368. A caller who asks for this
 // path by name gets them whatever the number of regions; the regions' average length still decides, so a region's last bit may differ
 // between calls of short and of long company.
