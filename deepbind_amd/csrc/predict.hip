@@ -83,8 +83,11 @@ __global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict_
 // LDS), keeps the maximum and the sum of the rows no change of its letters can reach and, one by one, the rows some change
 // can; a wave then takes a letter at a time, its lanes being 4 quarters of the m rows x 16 filters: the rows are scanned anew without that
 // letter, in two halves of its other taps, which leaves one addition for each of the four new ones, and pooled with what is kept (maps' error
-// against float64 2.1e-6 to 6.6e-6, 2.4e-6 to 6.9e-6 with every tap in one chain). (Rows of a mean are added in an order that depends on
-// where the workgroup's letters lie, so the score of the letter that is there comes from k_mutation_map.) More than 16 filters take further passes; pooled values meet the dense head in LDS.
+// against float64 2.1e-6 to 6.6e-6, 2.4e-6 to 6.9e-6 with every tap in one chain). That adds a row's taps in another order than the forward pass does, and the
+// rows of a mean in one that depends on where the workgroup's letters lie, so what a change is measured against is the score of the letter that is there
+// from the same pass (k_mutation_map): letters of equal weight differ by nothing. An unknown letter and a change in two regions (below) have no such
+// score: where filters have equal weights at a tap, their rows are scanned with each new letter in its place, in the order of the rows as they are (scan_changed).
+// More than 16 filters take further passes; pooled values meet the dense head in LDS.
 // What bounds it is instruction issue and LDS reads, one per (row, tap): m * m / 4 per letter and filter tile and lane (m * m with a lane per new
 // letter, each of which scanned the rows by itself), where the reference's way (a pass of the
 // whole net per change) scans length + m - 1 rows per change, and launches 15 kernels for it.
@@ -107,10 +110,12 @@ struct mut_args {
     float *S, *base;                                                // changed scores (4 per stream position), unchanged ones (per region)
 };
 
-// The letter table of filters c0 .. c0 + 15 (filters >= c1: zeros), [tap][letter][16], by all `nt` threads of the workgroup.
-__device__ __forceinline__ void letter_table16(float* __restrict__ lut, const float* __restrict__ W, unsigned m, size_t F, unsigned c0, unsigned c1,
+// The letter table of filters c0 .. c0 + 15 (filters >= c1: zeros), [tap][letter][16], by all `nt` threads of the workgroup. Whether one of
+// this thread's taps has the same weight, other than zero, for two letters (an unknown one counts their mean).
+__device__ __forceinline__ bool letter_table16(float* __restrict__ lut, const float* __restrict__ W, unsigned m, size_t F, unsigned c0, unsigned c1,
                                                unsigned nt)
 {
+    bool ties = false;
     for (unsigned e = threadIdx.x; e < m * MUT_F; e += nt) {
         const unsigned j = e / MUT_F, c = c0 + e % MUT_F;
         float w[4];
@@ -120,7 +125,13 @@ __device__ __forceinline__ void letter_table16(float* __restrict__ lut, const fl
         z += w[1]; z += w[2]; z += w[3];
         float* t = lut + (size_t)j * NL * MUT_F + e % MUT_F;
         t[0] = w[0]; t[MUT_F] = w[1]; t[2 * MUT_F] = w[2]; t[3 * MUT_F] = w[3]; t[4 * MUT_F] = z * 0.25f; t[5 * MUT_F] = 0.0f;
+        const float v[5] = {w[0], w[1], w[2], w[3], z * 0.25f};
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = a + 1; b < 5; ++b) ties |= v[a] == v[b] && v[a] != 0.0f;
     }
+    return ties;
 }
 
 // Rows p .. p + 3 of the staged letters (each already x 16) for this lane's filter, taps ascending. A letter is read once for the four rows it meets.
@@ -169,6 +180,31 @@ __device__ __forceinline__ void scan_rows(const float* __restrict__ lut_f, const
     taps(half, m);
 #pragma unroll
     for (unsigned u = 0; u < NR; ++u) z[u] += first[u];
+}
+
+// Row p with each of the four letters at the indexes one and two (~0: none), its taps in the order of scan_rows.
+__device__ __forceinline__ void scan_changed(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, unsigned one, unsigned two,
+                                             float (&z)[4])
+{
+    float first[4];
+#pragma unroll
+    for (unsigned c = 0; c < 4; ++c) z[c] = 0.0f;
+#pragma unroll 1
+    for (unsigned half = 0; half < 2u; ++half) {
+#pragma unroll
+        for (unsigned c = 0; c < 4; ++c) { first[c] = z[c]; z[c] = 0.0f; }
+        const unsigned to = half ? m : m / 2u;
+#pragma unroll 1
+        for (unsigned j = half ? m / 2u : 0u; j < to; ++j) {
+            const float* t = lut_f + j * NL * MUT_F;
+            const bool changed = p + j == one || p + j == two;
+            const unsigned l = let[p + j];
+#pragma unroll
+            for (unsigned c = 0; c < 4; ++c) z[c] += t[changed ? c * MUT_F : l];
+        }
+    }
+#pragma unroll
+    for (unsigned c = 0; c < 4; ++c) z[c] += first[c];
 }
 
 // LDS, in this order: letter table [m][NL][16], rows a change can reach [pos + m - 1][16] (rectified), two fold areas [2][NT / 16][16],
@@ -227,7 +263,7 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
     const unsigned nhead_w = mut_head_weights(a.k, a.hidden);
     // (the weights are on their way before the region's bounds and letters)
     for (unsigned e = tid; e < nhead_w; e += MUT_NT) head_w[e] = a.W1[e];
-    letter_table16(lut, a.W, m, a.F, 0, a.F, MUT_NT);
+    bool ties = letter_table16(lut, a.W, m, a.F, 0, a.F, MUT_NT);   // (of this thread's taps, then of the sixteen filters)
     const unsigned hl = tid & 15u;
     float hidden_b[MUT_MAXH / 16], hidden_w[MUT_MAXH / 16];         // this lane's hidden units'
 #pragma unroll
@@ -274,7 +310,7 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
         const float bf = on ? a.bias[f0 + f] : 0.0f;
         if (f0 > 0) {
             __syncthreads();                                        // the previous tile's table and rows are no longer read
-            letter_table16(lut, a.W, m, a.F, f0, a.F, MUT_NT);
+            ties = letter_table16(lut, a.W, m, a.F, f0, a.F, MUT_NT);
         }
         // ---- the region as it is: rows out of reach folded, rows in reach kept
         float mx = 0.0f, sum = 0.0f;
@@ -299,7 +335,7 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
         }
         fold[rl * MUT_F + f] = mx;
         fold[(MUT_NT / 16 + rl) * MUT_F + f] = sum;
-        __syncthreads();
+        ties = __syncthreads_or(ties) != 0;
         mx = 0.0f; sum = 0.0f;
 #pragma unroll
         for (unsigned t = 0; t < MUT_NT / 16; ++t) {
@@ -332,6 +368,21 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
             unsigned first = s0, at = i + pad, at2 = both ? q2 - s0 : ~0u;
             const uint8_t* letters = let;
             for (unsigned part = 0; part < (both ? 2u : 1u); ++part) {
+                if (ties && (both || letters[at] >= 4u * MUT_F)) {
+#pragma unroll 1
+                    for (unsigned p = lo + g; p < hi; p += 4) {
+                        float z[4];
+                        scan_changed(lut_f, letters, p, m, at, at2, z);
+#pragma unroll
+                        for (unsigned c = 0; c < 4; ++c) {
+                            float v = ((size_t)first + p < n ? z[c] : 0.0f) + bf;
+                            v = v > 0.0f ? v : 0.0f;
+                            bm[c] = v > bm[c] ? v : bm[c];
+                            bs[c] += v;
+                        }
+                    }
+                    lo = hi;                                         // (nothing left for the quarters)
+                }
                 const unsigned each = (hi - lo + 3u) / 4u, shown = hi > lo ? hi - lo + 3u + NR + m : 0u;
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -717,8 +768,9 @@ __global__ __launch_bounds__(256) void k_gradient_map(const grad_args a)
 }
 
 // The map of a sequence: (changed score - score) where the larger of the two is positive, else 0; with both strands a score
-// is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. The letter that is there is no change: its score
-// is the score, whatever order the workgroup that formed the changed one added its rows in. One workgroup per sequence.
+// is the larger of the pair's, the reverse row changed at the mirrored letter to the complement. The score to take off is that of the letter that is
+// there, its rows added in the order of the changed ones; where that is none of ACGT, or the pass changes the region twice, the score as
+// k_mutation_scores formed it of the region as it is. One workgroup per sequence.
 __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict__ R, unsigned pad, int strands, const uint8_t* __restrict__ X,
                                                       const float* __restrict__ S, const float* __restrict__ base, float* __restrict__ Z,
                                                       float* __restrict__ map)
@@ -733,14 +785,19 @@ __global__ __launch_bounds__(256) void k_mutation_map(const uint32_t* __restrict
     const unsigned pa = before ? R[2 * r - 2] : 0u, pb = before ? R[2 * r - 1] : 0u;
     for (unsigned e = threadIdx.x; e < 4 * len; e += blockDim.x) {
         const unsigned i = e >> 2, c = e & 3u;
-        float v = S[4 * ((size_t)ra + pad + i) + c];
-        if (strands == 2) {
-            const float w = S[4 * (size_t)(mirror - i) + 3 - c];
-            v = w > v ? w : v;
-        }
-        if (X[(size_t)ra + pad + i] == c && !spilled_pass(i, pad, before, pa, pb, ra)) v = z;
+        const size_t at = (size_t)ra + pad + i;
+        auto score = [&](unsigned letter) {
+            float v = S[4 * at + letter];
+            if (strands == 2) {
+                const float w = S[4 * (size_t)(mirror - i) + 3 - letter];
+                v = w > v ? w : v;
+            }
+            return v;
+        };
+        const unsigned own = X[at];
+        const float v = score(c), from = own < 4u && !spilled_pass(i, pad, before, pa, pb, ra) ? score(own) : z;
         // (a product with 1 or 0, so that scores that are infinite or not a number show)
-        const float d = v - z;
+        const float d = v - from;
         map[4 * out + e] = (z > v ? z : v) > 0.0f ? d : v == v && z == z ? d * 0.0f : d;
     }
     if (threadIdx.x == 0) Z[s] = z;

@@ -170,6 +170,45 @@ def test_mutation_to_the_letter_that_is_there_is_none(pool, hidden, m, F, rc):
 
 
 @pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("pool,hidden,m,F,n", [("max", 6, 24, 16, 5), ("max", 0, 9, 33, 70), ("avg", 5, 16, 16, 5), ("all", 8, 32, 16, 300), ("max", 32, 7, 4, 5)])
+def test_mutation_between_letters_of_equal_weight_is_none(pool, hidden, m, F, n, rc):
+    """A filter that does not tell A from G nor C from T scores a sequence the same, bit for bit, when one takes the other's place: the rows that
+    hold the letter are added in one order for all four. (Both strands: the complements are equal as well. Longer sequences first, so that
+    no change lands in the next one's pad.)"""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(5 * m + F)
+    p = _params(rng, m, F, pool, hidden)
+    W = p["Wc"].reshape(m, 4, F)
+    W[:, 2], W[:, 3] = W[:, 0], W[:, 1]
+    seqs = sorted(("".join("ACGT"[v] for v in rng.integers(0, 4, int(k))) for k in rng.integers(20, 90, n)), key=len, reverse=True)
+    _, maps = predict.gen_predictions(_net(p, m, F, pool, hidden, "nll", rc, 0.0), seqs, want_gmaps="finite_diff")
+    for s, (_, g) in zip(seqs, maps):
+        twin = ["GTAC".find(ch) for ch in s]
+        assert (g[np.arange(len(s)), twin] == 0).all()
+    assert all((g != 0).any() for _, g in maps)
+
+
+@pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("hidden,m,F", [(6, 24, 16), (0, 9, 33), (4, 30, 16), (3, 2, 5), (8, 64, 2)])
+def test_filters_that_tell_no_letters_apart_have_no_mutations(hidden, m, F, rc):
+    """Every window of such a filter has one sum, with unknown letters in it (their mean is the weight that all four have) and where a change
+    lands in the pad of the next sequence as well: maps of zeros, bit for bit, by the maximum."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(m + F)
+    p = _params(rng, m, F, "max", hidden)
+    W = p["Wc"].reshape(m, 4, F)
+    W[:] = W[:, :1]
+    W[1::3] = 0.0
+    p["bc"] += 0.5 * np.abs(W[:, 0].sum(axis=0))
+    p["b2" if hidden else "b1"] += 5.0                  # (changes count where a score is positive)
+    seqs = _seqs(rng, 60, 1, 40, 0.2) + ["N" * 12, "ACGT", "N", "GATTACA" * 5]
+    Z, maps = predict.gen_predictions(_net(p, m, F, "max", hidden, "mse", rc, 0.0), seqs, want_gmaps="finite_diff")
+    assert np.isfinite(Z).all() and (Z > 0).all()
+    for _, g in maps:
+        assert (g == 0).all()
+
+
+@pytest.mark.parametrize("rc", [False, True])
 @pytest.mark.parametrize("m,window,stride", [(1, 2, 1), (24, 20, 3), (8, 65, 7)])
 def test_text_and_windows_are_packed_as_on_the_host(rc, m, window, stride):
     from deepbind_amd import _lib, data, predict
