@@ -135,7 +135,7 @@ def _mutation_maps(net, X, R, text):
     _lib.call("dbk_mutation_map", _lib.stream(), _lib.ptr(Wc), _lib.ptr(p["bc"]), net.m, net.nfilter, _lib.ptr(X), X.numel(), _lib.ptr(R),
               R.shape[0], int(text.lens.max()), ptype, net.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")),
               _lib.ptr(p.get("b2")), _lib.ptr(scale), int(net.loss == "nll"), 2 if net.reverse_complement else 1, _lib.ptr(Z), _lib.ptr(maps))
-    host = torch.empty(out.shape, dtype=out.dtype)
+    host = torch.empty(out.shape, dtype=out.dtype, device="cpu")
     result = host.numpy()
     gmaps = list(zip(text.strings(), _split(result[n:].reshape(-1, 4), text)))               # (cut while the kernel runs, filled by the copy)
     host.copy_(out)
@@ -156,7 +156,7 @@ def _gradient_maps(net, text):
               shortest, longest, ptype, net.hidden, _lib.ptr(p["W1"]), _lib.ptr(p["b1"]), _lib.ptr(p.get("W2")), _lib.ptr(p.get("b2")),
               _lib.ptr(scale), int(net.loss == "nll"), 2 if net.reverse_complement else 1,
               _lib.ptr(Z), _lib.ptr(maps), _lib.ptr(strand))
-    host = torch.empty(out.shape, dtype=out.dtype)
+    host = torch.empty(out.shape, dtype=out.dtype, device="cpu")
     result = host.numpy()
     cut = _split(result[4 * n:4 * n + 16 * L].view(np.float32).reshape(-1, 4), text)         # (while the kernel runs; filled by the copy)
     host.copy_(out)

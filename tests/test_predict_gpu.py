@@ -372,3 +372,24 @@ def test_feature_columns_and_wide_targets():
             assert all(np.array_equal(a, b) for a, b in zip(out[0], o))
         with pytest.raises(DeepbindError):
             grp.train_step(X, R, wide[:, :2].contiguous())
+
+
+@pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("mode", [False, True, "finite_diff"])
+def test_predictions_under_a_default_device(mode, rc):
+    """Scores and maps come to the host whatever device a program's new tensors go to by default; the same bits."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(12)
+    net = _net(_params(rng, 8, 4, "max", 5), 8, 4, "max", 5, "nll", rc, 0.0)
+    seqs = _seqs(rng, 6, 10, 20)
+    want = predict.gen_predictions(net, seqs, want_gmaps=mode)
+    windows = predict.gen_predictionmaps(net, seqs, windowsize=12)[0]
+    torch.set_default_device("cuda")
+    try:
+        got = predict.gen_predictions(net, seqs, want_gmaps=mode)
+        again = predict.gen_predictionmaps(net, seqs, windowsize=12)[0]
+    finally:
+        torch.set_default_device(None)
+    assert np.array_equal(got[0], want[0]) and all(np.array_equal(a, b) for a, b in zip(again, windows))
+    for (sa, a), (sb, b) in zip(got[1] or [], want[1] or []):
+        assert sa == sb and np.array_equal(a, b)
