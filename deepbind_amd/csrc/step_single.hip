@@ -41,6 +41,7 @@
 // nothing until the host has zeroed the workspace's header again.
 // Results are deterministic (no float atomics; LDS atomics only OR bits), within the tolerances of the
 // multi-launch step but not its bits (other summation orders).
+#include <mutex>
 #include <type_traits>
 #include "dbk_common.h"
 #include "rng.h"
@@ -886,6 +887,31 @@ __global__ __launch_bounds__(256) void k_longest_region(const uint32_t* __restri
 
 }  // namespace
 
+// While a stream is being captured the look goes through a stream and a word of host memory of the library's own, one each per device, which stay for
+// the process; nothing of it is in the graph. The table has to be there, as it is where the device was waited for before the capture began.
+static int longest_region_beside(const uint32_t* regions, unsigned nregion, unsigned* rows)
+{
+    static std::mutex lock;
+    static hipStream_t streams[64];
+    static unsigned* words[64];
+    int dev = 0;
+    DBK_HIP(hipGetDevice(&dev));
+    DBK_CHECK(dev >= 0 && dev < 64, "RuntimeError: no current device below 64");
+    struct relaxed {                                               // (this thread's calls are not the capture's)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    } guard;
+    std::lock_guard<std::mutex> held(lock);
+    if (!streams[dev]) DBK_HIP(hipStreamCreateWithFlags(&streams[dev], hipStreamNonBlocking));
+    if (!words[dev]) DBK_HIP(hipHostMalloc((void**)&words[dev], sizeof(unsigned), hipHostMallocDefault));
+    hipLaunchKernelGGL(k_longest_region, dim3(1), dim3(256), 0, streams[dev], regions, nregion, words[dev]);
+    DBK_HIP(hipGetLastError());
+    DBK_HIP(hipStreamSynchronize(streams[dev]));
+    *rows = *(volatile unsigned*)words[dev];
+    return 0;
+}
+
 // A new minibatch pays for this once before its first step: one launch and one read-back (the same from elementwise
 // operations of the host's array library: five launches and a read-back, ~60 us a minibatch against ~20).
 extern "C" int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, size_t nregion, unsigned* rows)
@@ -895,6 +921,13 @@ extern "C" int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, 
     if (nregion == 0) { dbk::clear_error(); return 0; }
     DBK_CHECK(regions && nregion < ((size_t)1 << 31), "ValueError: regions must be a table of fewer than 2^31 rows");
     hipStream_t st = dbk::as_stream(stream);
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();      // (the default stream beside another one's capture)
+    if (status != hipStreamCaptureStatusNone) {
+        const int rc = longest_region_beside(regions, (unsigned)nregion, rows);
+        if (rc == 0) dbk::clear_error();
+        return rc;
+    }
     unsigned* word = (unsigned*)dbk::workspace(sizeof(unsigned), st);
     DBK_CHECK(word != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
     hipLaunchKernelGGL(k_longest_region, dim3(1), dim3(256), 0, st, regions, (unsigned)nregion, word);

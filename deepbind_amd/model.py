@@ -72,6 +72,8 @@ class SequenceNet(object):
         # Nesterov look-ahead kept beside the parameters by the natively issued step (each step's update kernel
         # leaves the next step's look-ahead there); valid while nothing else has touched P, mP or mrate
         self._L, self._L_versions = None, None
+        self._own_capture = False            # a graph that this package replays itself is being captured
+        self._replayed = False               # a program has captured a step that leaves no look-ahead: its replays are not seen here
         ni, nf = self.ninst, self.nfilter
         self.k = nf * (2 if pool == "all" else 1)          # pooled features per model
         # the reference's first dense layer (its "combiner") has a second input: a feature matrix with
@@ -187,14 +189,21 @@ class SequenceNet(object):
         self._L_versions = None              # the look-ahead kept beside the parameters no longer matches them
 
     def _single_work(self, buf, R):
-        """Workspace of the single-launch step for this batch shape, or None when the step does not take it or several launches are faster."""
+        """Workspace of the single-launch step for this batch shape, or None when the step does not take it or several launches are faster.
+        A graph that a program captures itself gets the one launch wherever it fits: it takes no scratch of the capturing stream, which may have
+        none yet and shares it among all graphs captured there, and forms the look-ahead anew whenever it is replayed."""
         if "work" not in buf:
             need = ctypes.c_size_t(0)
-            if _lib.dll().dbk_train_step_single_pays(ctypes.addressof(self._step_args)):
-                _lib.call("dbk_train_step_single_workspace", ctypes.addressof(self._step_args), ctypes.addressof(need))
-            buf["work"] = self._workspace(need.value) if need.value else None
-        if buf["work"] is None:
-            return None
+            _lib.call("dbk_train_step_single_workspace", ctypes.addressof(self._step_args), ctypes.addressof(need))
+            # (made now in either case: under capture it would be a node of the graph and be cleared by every replay)
+            buf["fits"] = need.value
+            work = self._workspace(need.value) if need.value else None
+            buf["work"] = work if _lib.dll().dbk_train_step_single_pays(ctypes.addressof(self._step_args)) else None
+        work = buf["work"]
+        if work is None:
+            if not buf["fits"] or not self._captured_by_program():
+                return None
+            work = self._workspace(buf["fits"])
         # the longest region of this very tensor object in its present state: an address alone says nothing (a new
         # tensor of a later batch can get the address of a freed one), so the entry holds a weak reference to the tensor
         ent = self._single_rows.get(id(R))
@@ -204,7 +213,10 @@ class SequenceNet(object):
             rows = ctypes.c_uint(0)          # one read-back per region table: the kernel keeps whole regions in LDS
             _lib.call("dbk_longest_region", _lib.stream(), _lib.ptr(R), R.shape[0], ctypes.addressof(rows))
             ent = self._single_rows[id(R)] = (weakref.ref(R), R._version, rows.value)
-        return buf["work"] if ent[2] <= 256 else None
+        return work if ent[2] <= 256 else None
+
+    def _captured_by_program(self):
+        return not self._own_capture and torch.cuda.is_current_stream_capturing()
 
     def _workspace(self, need):
         """A single-launch workspace of at least `need` bytes. Batches of all shapes share one: what a launch leaves in it
@@ -555,7 +567,7 @@ class SequenceNet(object):
         if a is not None and sig == self._step_sig and self._step_switches == self._switches():
             if self.nesterov:
                 versions = (self.P._version, self.mP._version, self.mrate._version)
-                a.L_ready = int(self._L_versions == versions)
+                a.L_ready = int(self._L_versions == versions and not self._replayed)
                 self._L_versions = versions
             a.decay = self.decay_vec.data_ptr() if self.weight_decay_start <= self.step_count else None
             a.freeze_scan = int(self.step_count < self.start_training)
@@ -590,7 +602,7 @@ class SequenceNet(object):
             # in-place changes made through torch (set_params, set_rates, a view written by the caller) move these counters;
             # the wrappers that write through raw pointers (the layer-by-layer and the graphed step) reset _L_versions
             versions = (self.P._version, self.mP._version, self.mrate._version)
-            a.L_ready = int(self._L_versions == versions)
+            a.L_ready = int(self._L_versions == versions and not self._replayed)
             self._L_versions = versions
         else:
             a.L, a.L_ready = None, 0
@@ -666,8 +678,11 @@ class SequenceNet(object):
             _lib.call("dbk_train_step", _lib.stream(), ctypes.addressof(self._step_args))
         self._last_single = work is not None
         self._finish_step(X, R)
-        if work is not None and not torch.cuda.is_current_stream_capturing():
-            self._count_single_launch(work)  # (may raise: a step that was abandoned must not be trained over in silence)
+        if work is not None:
+            if not torch.cuda.is_current_stream_capturing():
+                self._count_single_launch(work)      # (may raise: a step that was abandoned must not be trained over in silence)
+            elif not self._own_capture:
+                self._replayed = True
         self.enforce_constraints()
         return buf["Z"]
 
@@ -768,7 +783,12 @@ def _graphed_step(jobs):
         # the natively issued step on the capturing stream, with or without a look-ahead to start from
         for net, *_ in jobs:
             net._L_versions = versions(net) if (ready and keeps_lookahead(net)) else None
-        _native_steps(jobs)
+            net._own_capture = True
+        try:
+            _native_steps(jobs)
+        finally:
+            for net, *_ in jobs:
+                net._own_capture = False
 
     def capture():
         # The library's scratch buffers belong to a stream and cannot grow under capture: run the step
@@ -806,7 +826,7 @@ def _graphed_step(jobs):
     def step():
         if state["graphs"] is None or state["decay"] != decay_flags():
             capture()
-        ready = all(keeps_lookahead(net) and net._L_versions == versions(net) for net, *_ in jobs)
+        ready = all(keeps_lookahead(net) and net._L_versions == versions(net) and not net._replayed for net, *_ in jobs)
         state["graphs"][ready].replay()
         for net, X, R, *_ in jobs:
             # the update left the look-ahead of the new parameters (written through raw pointers: the counters stand still)

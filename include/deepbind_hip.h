@@ -549,7 +549,8 @@ int dbk_train_step_single_workspace(const dbk_train_step_args* args, size_t* wor
 /* 1 where the one launch is the faster step of a shape that it takes, 0 where dbk_train_step is (several regions per workgroup, beyond one
  * model's 16 filters) or the shape is not taken. */
 int dbk_train_step_single_pays(const dbk_train_step_args* args);
-/* Rows of the longest of nregion (start, end) regions, read back to the host (waits for the stream). */
+/* Rows of the longest of nregion (start, end) regions, read back to the host (waits for the stream; while the stream is being captured: through a
+ * stream of the library's own, the table as it is then). */
 int dbk_longest_region(dbk_stream_t stream, const uint32_t* regions, size_t nregion, unsigned* rows);
 int dbk_train_step_single(dbk_stream_t stream, const dbk_train_step_args* args, void* work, size_t work_bytes);
 /* sizeof(dbk_train_step_args) as the library was built, for bindings that mirror the block field by field. */

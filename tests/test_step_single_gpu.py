@@ -349,3 +349,37 @@ def test_graphed_step_outlives_a_larger_workspace():
         for name in a:
             assert np.array_equal(a[name], b[name]), (i, name)
     assert len(net._works) == 2 and net.step_count == ref.step_count == 6
+
+
+@pytest.mark.parametrize("nm,B,rc,pool", [(4, 300, False, "all"), (1, 1400, False, "max"), (2, 520, True, "avg"), (1, 128, False, "max")])
+def test_steps_that_a_program_captures_itself(nm, B, rc, pool):
+    """A graph of a step captured on a stream that never ran one, for batches of several regions per workgroup as for others: replays among eager
+    steps on the same and on a larger batch, and after parameters were set anew, end where eager steps through the one launch and the same sums do."""
+    rng = np.random.default_rng(B)
+    m = 9
+    batches = []
+    for rows in (B, 2 * B):
+        X, R = _batch(rng, rows // (2 if rc else 1), m, 12, 20, reverse_complement=rc)
+        batches.append((dev(X), dev(R), dev(rng.random((rows, nm)).astype(np.float32))))
+    make = lambda **kw: _net(np.random.default_rng(1), nm, 16, m, pool, 8, "nll", rate=0.05, momentum=0.9, dropout=0.5, reverse_complement=rc, **kw)
+    (net, p0), (ref, _) = make(), make()
+    for n in (net, ref):
+        for _ in range(2):
+            n.train_step(*batches[0])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        net.train_step(*batches[0])
+    assert net._last_single
+    for i in range(6):
+        if i == 3:
+            for n in (net, ref):
+                n.set_params(p0)
+        g.replay()
+        ref.train_step(*batches[0])
+        which = batches[1 if i % 2 else 0]
+        torch.cuda.synchronize()
+        net.train_step(*which)
+        ref.train_step(*which)
+        for name in ("P", "mP"):
+            assert_close_per_model(host(getattr(net, name)), host(getattr(ref, name)), GRAD, 1, 0, "%s after replay %d" % (name, i))
+        assert int(net.rng_counter.item()) == int(ref.rng_counter.item())
