@@ -73,7 +73,7 @@ class SequenceNet(object):
         # leaves the next step's look-ahead there); valid while nothing else has touched P, mP or mrate
         self._L, self._L_versions = None, None
         self._own_capture = False            # a graph that this package replays itself is being captured
-        self._replayed = False               # a program has captured a step that leaves no look-ahead: its replays are not seen here
+        self._replayed = False               # a program has captured a step: its replays move the parameters unseen
         ni, nf = self.ninst, self.nfilter
         self.k = nf * (2 if pool == "all" else 1)          # pooled features per model
         # the reference's first dense layer (its "combiner") has a second input: a feature matrix with
@@ -217,6 +217,13 @@ class SequenceNet(object):
 
     def _captured_by_program(self):
         return not self._own_capture and torch.cuda.is_current_stream_capturing()
+
+    def _start_over_in_graphs(self):
+        """A step of several launches that a program captures forms the look-ahead itself: what lies beside the parameters when the graph
+        is replayed need not be theirs. Eager steps do the same from then on."""
+        if self._captured_by_program():
+            self._step_args.L_ready = 0
+            self._replayed = True
 
     def _workspace(self, need):
         """A single-launch workspace of at least `need` bytes. Batches of all shapes share one: what a launch leaves in it
@@ -675,6 +682,7 @@ class SequenceNet(object):
             _lib.call("dbk_train_step_single", _lib.stream(), ctypes.addressof(self._step_args), _lib.ptr(work), work.numel())
             self._L_versions = None          # (this kernel forms the look-ahead itself and leaves none behind)
         else:
+            self._start_over_in_graphs()
             _lib.call("dbk_train_step", _lib.stream(), ctypes.addressof(self._step_args))
         self._last_single = work is not None
         self._finish_step(X, R)
@@ -738,6 +746,7 @@ def _native_steps(jobs):
         blocks = (ctypes.c_void_p * len(chunk))()
         for j, (net, X, R, Y, Ymask, *rest) in enumerate(chunk):
             net._prepare_step(X, R, Y, Ymask, *rest)
+            net._start_over_in_graphs()
             blocks[j] = ctypes.addressof(net._step_args)
         _lib.call("dbk_train_steps", _lib.stream(), len(chunk), blocks)
         for net, X, R, *_ in chunk:

@@ -908,3 +908,50 @@ def test_group_reads_its_models_columns_of_the_shared_targets(masked):
             net.train_step(Xd, Rd, dev(np.ascontiguousarray(Y[:, idx])), dev(np.ascontiguousarray(M[:, idx])) if masked else None)
     for (idx, net), own in zip(grp.groups, nets):
         assert np.array_equal(host(net.P), host(own.P)) and np.array_equal(host(net.mP), host(own.mP)), idx
+
+
+@pytest.mark.parametrize("grouped", [False, True])
+def test_captured_steps_of_several_launches_start_from_the_parameters_as_they_are(grouped):
+    """A graph that a program captures of a step of several launches, replayed among eager steps and after parameters and momentum were set
+    anew, gives the bits of eager steps: neither side takes a look-ahead that the other's updates have outdated."""
+    from deepbind_amd import data
+    from deepbind_amd.model import ModelGroup, SequenceNet
+    rng = np.random.default_rng(8)
+    ni, m = (6, 11)
+    seqs = ["".join(rng.choice(list("ACGT"), size=rng.integers(15, 40))) for _ in range(60)]
+    X, R = [dev(v) for v in data.pack_sequences(seqs, m - 1)]
+    Y = dev((rng.random((60, ni)) < 0.5).astype(np.float32))
+
+    def make():
+        if grouped:
+            it = ModelGroup(["max", "all"] * 3, [0, 4] * 3, 8, m, loss="nll", rate=0.05, momentum=0.9, dropout=0.5)
+            nets = [n for _, n in it.groups]
+        else:
+            it = SequenceNet(ni, 8, m, pool="all", hidden=4, loss="nll", rate=0.05, momentum=0.9, dropout=0.5)
+            nets = [it]
+        for k, n in enumerate(nets):
+            n.init_params(0.3, 0.3, 0.05, seed=k)
+        return it, nets
+
+    (one, nets), (ref, refs) = make(), make()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            one.train_step(X, R, Y)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        one.train_step(X, R, Y)
+    for _ in range(2):
+        ref.train_step(X, R, Y)
+    for i in range(6):
+        if i in (2, 5):
+            for n in nets + refs:
+                n.P.mul_(0.5)
+                n.mP.zero_()
+        for step in ((g.replay, lambda: one.train_step(X, R, Y)) if i != 4 else (lambda: one.train_step(X, R, Y), g.replay)):
+            step()
+            torch.cuda.synchronize()
+            ref.train_step(X, R, Y)
+            for a, b in zip(nets, refs):
+                assert torch.equal(a.P, b.P) and torch.equal(a.mP, b.mP), i
