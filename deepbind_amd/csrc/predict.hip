@@ -4,6 +4,7 @@
 // Reference: kangaroo/kangaroo/util.py:50-56,68-74 (letters), data.py:274-354 (packed stream, reverse-complement rows),
 // predict.py:145-345 (predictions, mutation maps, window scans). There every change is one full pass of the net over the
 // whole batch, the stream mutated on the host.
+#include <type_traits>
 #include "dbk_common.h"
 #include "scan_common.h"
 
@@ -152,8 +153,8 @@ __device__ __forceinline__ void scan4(const float* __restrict__ lut_f, const uin
     }
 }
 
-// Rows p .. p + NR - 1, in two halves of the taps, each ascending.
-template <unsigned NR>
+// Rows p .. p + NR - 1, in two halves of the taps, each ascending. FLY: taps whose reads are in flight.
+template <unsigned NR, unsigned FLY>
 __device__ __forceinline__ void scan_rows(const float* __restrict__ lut_f, const uint8_t* __restrict__ let, unsigned p, unsigned m, float (&z)[NR])
 {
     float first[NR];
@@ -163,7 +164,7 @@ __device__ __forceinline__ void scan_rows(const float* __restrict__ lut_f, const
 #pragma unroll
     for (unsigned u = 0; u + 1 < NR; ++u) l[u + 1] = let[p + u];
     auto taps = [&](unsigned from, unsigned to) __attribute__((always_inline)) {
-#pragma unroll 4
+#pragma unroll FLY
         for (unsigned j = from; j < to; ++j) {
 #pragma unroll
             for (unsigned u = 0; u + 1 < NR; ++u) l[u] = l[u + 1];
@@ -232,7 +233,6 @@ __device__ __forceinline__ bool spilled_pass(unsigned pass, unsigned pad, bool b
     return before && pb - pa > pass && pad + pa + pass >= pb && pad + pa + pass < ra + pad;
 }
 
-// NR: rows that a lane scans at a time. SPILLS: one strand only, where a change may lie in two regions (above).
 // v[c] of the four quarters of a wave put together: lanes 16 c .. 16 c + 15 get the one of v[c]
 template <typename Op>
 __device__ __forceinline__ float quarters(const float (&v)[4], Op op)
@@ -247,9 +247,17 @@ __device__ __forceinline__ float quarters(const float (&v)[4], Op op)
     return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
+// NR: rows that a lane scans at a time, of the quarter that it has. SPILLS: one strand only, where a change may lie in two regions (above).
+// Few taps are all latency: a letter's rows take less than fetching them, so their kernels keep fewer reads in flight for the registers' sake and six
+// or five waves per SIMD instead of four. (m <= 8 and m <= 12 went through the kernel of four rows, half and a quarter of which were none. us, with the letters
+// per workgroup chosen below, and the kernel of a lane per new letter: 128 sequences of 60-101, one strand, 4 taps 33 -> 24 / 21, 8 taps 34 -> 27 / 27, 12 taps
+// 39 -> 33 / 35; 64 on both strands 8 taps 28 -> 22 / 24, 12 taps 32 -> 25 / 30.) Eight rows at a time (25 to 64 taps) do not fit the registers of four waves:
+// 26 spills of 108 bytes a lane. Four rows take none, and 79 against 87 us at 25 taps (128 sequences, both strands), but 91 against 88 at 32 and 238 against 227 at 64.
+constexpr int mut_waves(unsigned nr) { return nr <= 2 ? 6 : nr == 3 ? 5 : 4; }
 template <unsigned NR, bool SPILLS>
-__global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
+__global__ __launch_bounds__(MUT_NT, mut_waves(NR)) void k_mutation_scores(const mut_args a)
 {
+    constexpr unsigned FLY = NR <= 3 ? 2 : 4;
     extern __shared__ __align__(16) float msm[];
     const unsigned m = a.m, pad = m - 1;
     const size_t r = blockIdx.x;
@@ -321,7 +329,7 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
             const unsigned t1 = rb - t0 < MUT_TILE ? rb : t0 + MUT_TILE;
             for (unsigned p = t0 + 4 * rl; p < t1; p += MUT_NT / 4) {
                 float z[4];
-                scan_rows<4>(lut_f, tile, p - t0, m, z);
+                scan_rows<4, FLY>(lut_f, tile, p - t0, m, z);
 #pragma unroll
                 for (unsigned u = 0; u < 4; ++u) {
                     if (p + u >= t1) break;
@@ -411,7 +419,7 @@ __global__ __launch_bounds__(MUT_NT, 4) void k_mutation_scores(const mut_args a)
                             for (unsigned c = 0; c < 4; ++c) w[u][c] += there ? t[c * MUT_F] : 0.0f;
                         }
                     }
-                    scan_rows<NR>(lut_f, mine, p0 - lo, m, z);
+                    scan_rows<NR, FLY>(lut_f, mine, p0 - lo, m, z);
 #pragma unroll
                     for (unsigned u = 0; u < NR; ++u) {
                         const bool counts = u0 + u < each && p0 + u < hi, in = p0 + u < stop;
@@ -902,8 +910,12 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     // letters per workgroup: 16 where that still gives every CU six workgroups, 8 where it has two, else 4, as a workgroup's first scan of
     // its region costs less than an idle CU. Whole calls, us, 4 / 8 / 16: one sequence of 101 letters 72 / 77 / 88; 64 regions of 60-101, 24 taps
     // 111 / 104 / 114, 32 taps 145 / 144 / 163; 100 regions of 40-80, 8 taps 132 / 130 / 136; 256 regions of 101 227 / 209 / 200.
+    // Up to 12 taps a letter costs little beside the first scan and the workgroups are to be on the GPU all at once: the next larger number where
+    // they would not be (regions count as long as the longest). us, 4 / 8 / 16, 8 taps: 50 regions of 60-101 19 / 21 / 26, 64 on both strands 20 / 16 / 20, 128 of one strand
+    // 30 / 27 / 28, 200 on both strands 37 / 31 / 28; 12 taps: 50 regions 20 / 23 / 30, 128 37 / 35 / 33.
     const size_t letters = longest > 0 ? longest : 1;
-    const unsigned pos = nregion * dbk::divup(letters, 16) >= 1536 ? 16u : nregion * dbk::divup(letters, 8) >= 512 ? 8u : 4u;
+    const unsigned pos = m <= 12 ? (nregion * dbk::divup(letters, 8) > (m <= 8 ? 1920 : 1600) ? 16u : nregion * dbk::divup(letters, 4) > 1400 ? 8u : 4u)
+                                 : (nregion * dbk::divup(letters, 16) >= 1536 ? 16u : nregion * dbk::divup(letters, 8) >= 512 ? 8u : 4u);
     const unsigned gy = dbk::divup(letters, pos);
     DBK_CHECK(nregion <= 0x7fffffffu && gy <= 65535u, "ValueError: too many regions (%zu) or letters per region (%zu) for one launch", nregion, longest);
     hipStream_t st = dbk::as_stream(stream);
@@ -917,8 +929,11 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     a.S = scratch; a.base = scratch + 4 * N;
     a.pos = pos;
     // (a lane takes a quarter of the m rows)
-    auto kern = strands == 1 ? (m <= 16 ? k_mutation_scores<4, true> : (m <= 24 ? k_mutation_scores<6, true> : k_mutation_scores<8, true>))
-                             : (m <= 16 ? k_mutation_scores<4, false> : (m <= 24 ? k_mutation_scores<6, false> : k_mutation_scores<8, false>));
+    auto pick = [&](auto spills) {
+        constexpr bool S = decltype(spills)::value;
+        return m <= 8 ? k_mutation_scores<2, S> : m <= 12 ? k_mutation_scores<3, S> : m <= 16 ? k_mutation_scores<4, S> : m <= 24 ? k_mutation_scores<6, S> : k_mutation_scores<8, S>;
+    };
+    auto kern = strands == 1 ? pick(std::true_type{}) : pick(std::false_type{});
     const size_t smem = mut_smem(pos, m, a.k, hidden);
     if (smem > 65536) DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
     hipLaunchKernelGGL(kern, dim3((unsigned)nregion, gy), dim3(MUT_NT), smem, st, a);

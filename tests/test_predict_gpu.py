@@ -154,6 +154,28 @@ def test_mutation_maps_do_not_depend_on_how_many_letters_a_workgroup_takes(rc, n
 
 
 @pytest.mark.parametrize("rc", [False, True])
+@pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 12, 13])
+def test_mutation_maps_of_few_taps(m, rc):
+    """Two rows at a time up to 8 taps, three up to 12: against the oracle with four letters per workgroup, the same bits with eight and sixteen."""
+    from deepbind_amd import predict
+    rng = np.random.default_rng(40 + m)
+    p = _params(rng, m, 16, "max", 32)
+    net = _net(p, m, 16, "max", 32, "nll", rc, 0.0)
+    seqs = _seqs(rng, 270, 57, 57)
+    Z, maps = predict.gen_predictions(net, seqs[:6], want_gmaps="finite_diff")
+    Zr, mr = orc.gen_predictions({k: v.astype(np.float64) for k, v in p.items()}, seqs[:6], "max", 32, "logistic", reverse_complement=rc, want_gmaps="finite_diff")
+    assert_close(Z, Zr, ACT, "Z")
+    scale = max(np.abs(b).max() for _, b in mr)
+    for (_, a), (_, b) in zip(maps, mr):
+        assert np.abs(a - b).max() <= GRAD * scale
+    for n in (130, 270):
+        Zn, more = predict.gen_predictions(net, seqs[:n], want_gmaps="finite_diff")
+        assert np.array_equal(Zn[:6], Z)
+        for (_, a), (_, b) in zip(maps, more):
+            assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("rc", [False, True])
 @pytest.mark.parametrize("pool,hidden,m,F", [("avg", 6, 24, 16), ("all", 0, 9, 33), ("max", 5, 16, 16), ("avg", 0, 1, 4)])
 def test_mutation_to_the_letter_that_is_there_is_none(pool, hidden, m, F, rc):
     """Exactly zero at every sequence's own letters, wherever in the sequence the workgroup that scores them begins. (Longer sequences
