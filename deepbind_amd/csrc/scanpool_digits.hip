@@ -998,13 +998,13 @@ void scanpool_digits_max_kernel(digit_store D, unsigned ntile, const float* __re
         scanpool_digits_max_body<WANT_ARGMAX, TB, false>(D, tile, split, two, W, bias, f0, m, F, X, N, ndef, R, P, nsplit, pooled, argmax);
 }
 
-// workgroups per group of filters: one workgroup per CU in all, no more waves than regions
-inline unsigned splits(unsigned groups, unsigned waves, size_t P)
+// workgroups per group of filters: one workgroup per CU in all, each with a region at least. (Fewer regions than waves lie side by side on all the
+// CUs, with waves that have none, not in full workgroups on some: one set of filters, 600 regions of 500 rows x 64 filters of 8 taps 19.3 -> 16.5 us, max + average.)
+inline unsigned splits(unsigned groups, size_t P)
 {
     unsigned n = 256u / groups;
     if (n < 1) n = 1;
-    while (n > 1 && (size_t)(n - 1) * waves >= P) --n;
-    return n;
+    return n < P ? n : (unsigned)P;
 }
 
 constexpr size_t max_smem(int tb)
@@ -1019,7 +1019,7 @@ int launch_max(hipStream_t st, const digit_store& D, const float* W, const float
 {
     auto kern = scanpool_digits_max_kernel<WANT_ARGMAX, TB>;
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_smem(TB)));
-    const unsigned groups = (ntile + 1) / 2, nsplit = splits(groups, MAX_WAVES, P);
+    const unsigned groups = (ntile + 1) / 2, nsplit = splits(groups, P);
     hipLaunchKernelGGL(kern, dim3(groups * nsplit), dim3(MAX_WAVES * 64), max_smem(TB), st, D, ntile, W, bias, f0, (unsigned)m, (unsigned)F, X, N, ndef, R,
                        (unsigned)P, nsplit, pooled, argmax);
     return 0;
@@ -1029,10 +1029,20 @@ template <int TB, int NT> constexpr size_t scan_smem() { return 16 + (size_t)WAV
 
 // Whether a wave takes two sets of 32 filters at a time: one staging of the letters, one read of a tile's operands and one walk serve both,
 // and their products take turns instead of waiting for each other's sums. Up to 16 taps, whose digits leave the registers for it (24 taps, us, one /
-// two: average, 30 000 x 101 x 256 251 / 254, max + average 271 / 303). An odd last set is scanned beside nothing, which many others pay for.
+// two: average, 30 000 x 101 x 256 251 / 254, max + average 271 / 303). An odd last set is scanned beside nothing, which many others pay for. Of the
+// 3072 waves of two sets (4096 of one) the last round is to have most at work, or to be one of many: a wave has twice the products and no more
+// than two others beside it. us, one / two, max + average, 500 rows x 128 filters: 16 taps, 600 regions (0.4 rounds of the waves of two sets) 22.3 / 25.4, 1200 (0.8) 27.8 / 28.4, 2000 (1.3)
+// 34.7 / 40.6, 3000 (1.95) 44.3 / 44.4; 64 filters, 3000 (0.98) 31.0 / 29.5; 256 filters, 2000 (2.6) 55.5 / 53.1; 8 taps, 128 filters, 600 18.7 / 20.2, 2000 27.6 / 31.3,
+// 3000 32.6 / 32.9 (average 32.9 / 30.6), 256 filters, 1200 (1.6) 29.8 / 32.1, 2000 41.0 / 38.3.
 // Whole calls, us, one / two: max + average, 20 000 x 30-150 letters x 384 filters x 16 taps 205 / 193, 60 000 x 20-40 x 128 142 / 131; maximum,
 // 60 000 x 101 x 256, 8 taps 225 / 195, 16 taps 328 / 304; average, 30 000 x 101 x 256 x 12 taps 186 / 174; 5000 x 101 x 64 x 16 taps 25.5 / 25.4.
-inline bool takes_two(unsigned ntile) { return ntile % 2 == 0 || ntile > 16; }
+template <int TB>
+inline bool takes_two(unsigned ntile, size_t P)
+{
+    if (ntile % 2 != 0 && ntile <= 16) return false;
+    const double rounds = (double)((ntile + 1) / 2) * (double)P / (256 * WAVES<2>);
+    return rounds <= 1.0 ? rounds >= 0.75 : rounds >= (TB == 1 ? 1.8 : 2.2);
+}
 
 template <int PT, bool WANT_ARGMAX, int TB, int NT>
 int launch_sets(hipStream_t st, const digit_store& D, const float* bias, unsigned f0, unsigned ntile, size_t F, const uint8_t* X, size_t N, size_t ndef,
@@ -1041,7 +1051,7 @@ int launch_sets(hipStream_t st, const digit_store& D, const float* bias, unsigne
     auto kern = scanpool_digits_kernel<PT, WANT_ARGMAX, TB, NT>;
     constexpr size_t smem = scan_smem<TB, NT>();
     DBK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
-    const unsigned groups = (ntile + NT - 1) / NT, nsplit = splits(groups, WAVES<NT>, P);
+    const unsigned groups = (ntile + NT - 1) / NT, nsplit = splits(groups, P);
     hipLaunchKernelGGL(kern, dim3(groups * nsplit), dim3(WAVES<NT> * 64), smem, st, D, bias, f0, (unsigned)F, X, N, ndef, R, (unsigned)P, nsplit, pooled, argmax);
     return 0;
 }
@@ -1051,7 +1061,7 @@ int launch_pt(hipStream_t st, const digit_store& D, const float* bias, unsigned 
               const uint32_t* R, size_t P, float* pooled, uint32_t* argmax)
 {
     if constexpr (TB <= 2) {
-        if (takes_two(ntile)) return launch_sets<PT, WANT_ARGMAX, TB, 2>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
+        if (takes_two<TB>(ntile, P)) return launch_sets<PT, WANT_ARGMAX, TB, 2>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
     }
     return launch_sets<PT, WANT_ARGMAX, TB, 1>(st, D, bias, f0, ntile, F, X, N, ndef, R, P, pooled, argmax);
 }

@@ -1630,6 +1630,26 @@ def test_bulk_scan_of_two_sets_of_filters_at_a_time(ks, F, closed, m, ptype):
 
 
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
+@pytest.mark.parametrize("m", [7, 16])
+@pytest.mark.parametrize("F,P,closed", [(33, 2300, ()), (64, 2310, (1,)), (64, 3080, ()), (96, 2500, (2,)), (128, 1160, (0, 3)), (128, 2800, (1,)), (520, 300, (16,)),
+                                        (520, 800, (16, 3)), (64, 255, ()), (64, 257, (0,)), (32, 1, ())])
+def test_bulk_scan_of_one_and_two_sets_of_filters_by_the_number_of_regions(ks, F, P, closed, m, ptype):
+    """Either side of the numbers of regions from which a wave takes 64 filters (0.75 to 1 round of its waves, then 1.8 or 2.2 on), where
+    it takes 32 whatever the regions (three sets), an odd last set among many, fewer regions than workgroups; weights that close windows in some sets."""
+    rng, W, b, X, R = _bulk_case(F + P, np.random.default_rng(P).integers(1, 41, P), m, F)
+    R[-1, 1] = X.size                                                   # the last region runs into rows the scan does not define
+    _closed_tiles(W, closed, np.float32(-1e9))
+    A, want, rows = _chain_oracle(W.astype(np.float64), b.astype(np.float64), X, R, ptype)
+    Pd, _ = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, path="kmer")
+    _within_rounding(host(Pd), want, np.where(W < -1e8, 0.0, W), b, ptype)
+    if ptype != "avg":
+        Pa, I = ks.scanpool_fprop(dev(W), dev(b), dev(X), dev(R), ptype, want_argmax=True, path="kmer")
+        assert np.array_equal(host(Pa), host(Pd))
+        moved = host(I) != rows
+        assert np.abs(A.ravel()[host(I)[moved]] - A.ravel()[rows[moved]]).max(initial=0.0) <= 1e-5
+
+
+@pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("m", [4, 16, 24])
 @pytest.mark.parametrize("size,bias", [(1e-24, 0.0), (1e28, 0.0), (1e-20, 1e25), (1e-20, -1e25), (1e-12, 1e-3), (1e20, 1e-20), (1.0, -1e29)])
 def test_bulk_scan_of_weights_and_biases_of_any_size(ks, size, bias, m, ptype):
