@@ -242,9 +242,12 @@ __global__ void regions_disjoint_kernel(const uint32_t* __restrict__ R, size_t P
 }
 
 // Few regions: every workgroup looks through the whole table itself, and one launch takes the place of three (the look, the kernel for disjoint
-// regions, the one for others, one of which has nothing to do): 1000 regions x 64 float64 columns 13.7 -> 5.5 us. Beyond, the tables that all workgroups
-// read are more than the two launches. All threads of the workgroup come here.
-constexpr size_t CHECK_REGIONS = 2048;
+// regions, the one for others, one of which has nothing to do). Up to 1024 regions that is no slower whatever the columns; up to 2048 while all
+// workgroups together read no more than 4.6 M entries of the table (the kernel of single columns, which maxima take, has one per 4 regions and 64 columns).
+// us, three launches / one, regions of 60 rows: maxima, float32, 1000 regions x 64 columns 6.3 / 4.1, x 1024 31.9 / 30.7, x 4096 182 / 177; 1500 x 512 (4.5 M) 25.7 / 25.4, x 1024 (9 M)
+// 49.9 / 52.9; 2048 x 256 19.4 / 18.6, x 512 (8 M) 33.3 / 34.7, x 1024 73.5 / 82.1, float64 76.9 / 90.1; average, rows of 12, 2048 x 512 (2 M) 21.9 / 22.1, x 1024 (4 M)
+// 37.9 / 38.2, x 4096 165 / 170, float64 x 1024 67.5 / 71.4. All threads of the workgroup come here.
+constexpr size_t CHECK_ALWAYS = 1024, CHECK_REGIONS = 2048, CHECK_ENTRIES = 4600000;
 __device__ __forceinline__ bool all_disjoint(const uint32_t* __restrict__ R, unsigned P, bool per_step)
 {
     bool bad = false;
@@ -473,11 +476,14 @@ int launch_bwd(hipStream_t st, T* dU, size_t F, const uint32_t* R, size_t P, boo
                const uint32_t* argmax, int ptype)
 {
     DBK_CHECK(dbk::divup(F, 64) <= 65535u, "ValueError: too many feature maps (%zu) for one launch", F);
+    const bool packs = ptype != DBK_PT_MAX && pack_shape<T>(dU, F, P, dP, nullptr);
+    const size_t wgs = packs ? dbk::divup(P * (F / (16 / sizeof(T))), 256) : (size_t)dbk::divup(P, 4) * dbk::divup(F, 64);
     unsigned* flag = nullptr;
-    if (P > CHECK_REGIONS) {
+    if (P > CHECK_REGIONS || (P > CHECK_ALWAYS && wgs * P > CHECK_ENTRIES)) {
         flag = (unsigned*)dbk::workspace(256, st);
-        DBK_CHECK(flag != nullptr, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
-        hipLaunchKernelGGL(regions_disjoint_kernel, dim3(1), dim3(1024), 0, st, R, P, per_step, flag);
+        // (without the word - a stream under capture that has no scratch yet - few enough regions are looked at by every workgroup all the same)
+        DBK_CHECK(flag != nullptr || P <= CHECK_REGIONS, "MemoryError: could not allocate scratch (%s)", dbk::workspace_error());
+        if (flag) hipLaunchKernelGGL(regions_disjoint_kernel, dim3(1), dim3(1024), 0, st, R, P, per_step, flag);
     }
     switch (ptype) {
     case DBK_PT_MAX: launch_bwd_pt<T, DBK_PT_MAX>(st, dU, F, R, P, per_step, dP, argmax, flag); break;

@@ -390,6 +390,37 @@ def test_poolrgn_bprop_finds_overlapping_regions(ks, overlap, P, F, dtype, ptype
     assert np.abs(host(dU) - want).max() <= (2e-6 if dtype == np.float32 else 4e-15)
 
 
+@pytest.mark.parametrize("ptype", ["max", "avg"])
+@pytest.mark.parametrize("P,F", [(1024, 2048), (1025, 2048), (2048, 1024), (2048, 64)])
+def test_poolrgn_bprop_of_many_columns_captured_without_scratch(ks, P, F, ptype):
+    """Many columns of up to 2048 regions: the look at the table has a launch of its own where workgroups would read it too often, and none where
+    a capturing stream has no scratch for its answer. Both give the same bits, regions that lie over each other included."""
+    rng = np.random.default_rng(P + F)
+    edges = np.concatenate([[0], np.cumsum(rng.integers(1, 5, P))])
+    R = np.stack([edges[:-1], edges[1:]], axis=1).astype(np.uint32)
+    R[P // 2] = [3, 9]                                                  # over others; whole numbers are added, so any order gives the same
+    U = dev(rng.integers(-8, 9, (int(edges[-1]), F)).astype(np.float32))
+    Rd = dev(R)
+    pooled, arg = ks.poolrgn(U, Rd, ptype, want_argmax=ptype == "max")
+    length = torch.from_numpy((R[:, 1].astype(np.int64) - R[:, 0])).cuda().float().view(-1, 1)
+    dP = torch.randint(-8, 9, (P, F), device="cuda").float() * (length if ptype == "avg" else 1.0)
+    want, got = U.clone(), U.clone()
+    ks.poolrgn_bprop(want, Rd, dP, arg, ptype)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        ks.poolrgn_bprop(got, Rd, dP, arg, ptype)
+    g.replay()
+    torch.cuda.synchronize()
+    ref = host(U).astype(np.float64)
+    if ptype == "max":
+        np.add.at(ref.reshape(-1), host(arg).astype(np.int64).ravel(), host(dP).astype(np.float64).ravel())
+    else:
+        for r, (a, e) in enumerate(R.astype(int)):
+            ref[a:e] += host(dP[r] / float(e - a)).astype(np.float64)
+    assert np.array_equal(host(want), ref) and torch.equal(got, want)
+
+
 def _chain_oracle(W, b, X, R, ptype):
     Z = np.zeros((X.size, W.shape[1]), W.dtype)
     orc.corr1ord(W, X, Z)
