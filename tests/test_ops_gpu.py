@@ -234,6 +234,21 @@ def test_corr1ord_gradients_on_the_small_matrix_instructions(ks, n, m, F, dtype)
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,m,F", [(200, 7, 5), (600, 9, 17), (2048, 5, 13), (2304, 5, 13), (2400, 24, 48), (5000, 4, 1000), (20000, 24, 3)])
+def test_corr1ord_bprop_W_of_few_and_many_slabs(ks, n, m, F, dtype):
+    """One, two and eight partial sums of an element, which a thread adds up, nine and more, which four waves do; elements that are no groups of 64."""
+    rng = np.random.default_rng(n + m)
+    X = random_codes(rng, n + m - 1, 0.05, 0.05).reshape(-1, 1)
+    dZ = np.zeros((n + m - 1, F), dtype); dZ[:n] = rng.standard_normal((n, F))
+    ref = np.ones((4 * m, F)); orc.corr1ord_bprop_W(ref, X, dZ.astype(np.float64))
+    dW, again = dev(np.ones((4 * m, F), dtype)), dev(np.ones((4 * m, F), dtype))
+    for out in (dW, again):
+        ks.corr1ord_bprop_W(out, dev(X), dev(dZ), 4)
+    assert_close(host(dW), ref, GRAD if dtype == np.float32 else 1e-12, "dW")
+    assert np.array_equal(host(dW), host(again))
+
+
 @pytest.mark.parametrize("N,m,F", [(750030, 24, 17), (750021, 5, 31), (749990, 16, 20)])
 def test_corr1ord_bprop_W_many_rows_of_few_filters(ks, N, m, F):
     """Either side of the row count from which 17 to 31 filters go through the register-plane kernel."""
