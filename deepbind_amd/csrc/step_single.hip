@@ -954,8 +954,9 @@ extern "C" int dbk_train_step_single_workspace(const dbk_train_step_args* a, siz
 //   16 filters       1: 0.3-0.6   2: 0.66   3: 0.85   4: 0.93   5: 1.02   6: 1.03   7: 1.08   8: 1.12
 //   17-32 filters    1: 0.4-0.6   2: 0.88   3: 1.14   4: 1.30   6: 1.49   8: 1.70
 //   33-64 filters    1: 0.5-0.8   2: 1.30   3: 1.67   4: 2.01   6: 2.57   8: 2.75
-// (1466 regions of 70 rows, 4 models of 16 filters of 26 taps: 102 against 42 us a step.) With the line at 80, 3 % of the shapes are slower than
-// they were by more than 3 %, at most 13 %; the others gain up to a factor of three.
+// (1466 regions of 70 rows, 4 models of 16 filters of 26 taps: 102 against 42 us a step.) The line lies at 80: with five regions of 16 filters the two are level on average,
+// and of the 263 shapes of several regions per workgroup 2.9 % are then slower than in one launch by more than 3 % (at most 13 %, those of up to 16 taps
+// or without a hidden layer); at 64 4.5 % are, for the same mean of all (0.858). The others gain up to a factor of three.
 extern "C" int dbk_train_step_single_pays(const dbk_train_step_args* a)
 {
     single_args s;

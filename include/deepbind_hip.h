@@ -546,8 +546,8 @@ int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_train_step_arg
  * (use dbk_train_step).
  * reference: the body of the trainer's loop, deepity/deepity/sgd.py:98-135, as dbk_train_step. */
 int dbk_train_step_single_workspace(const dbk_train_step_args* args, size_t* work_bytes);
-/* 1 where the one launch is the faster step of a shape that it takes, 0 where dbk_train_step is (several regions per workgroup, beyond one
- * model's 16 filters) or the shape is not taken. */
+/* 1 where the one launch is the step to take of a shape that it takes, 0 where dbk_train_step is faster on average (more than five regions per
+ * workgroup with up to 16 filters, two with 32, one with 64) or the shape is not taken. */
 int dbk_train_step_single_pays(const dbk_train_step_args* args);
 /* Rows of the longest of nregion (start, end) regions, read back to the host (waits for the stream; while the stream is being captured: through a
  * stream of the library's own, the table as it is then). */

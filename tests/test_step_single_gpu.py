@@ -383,3 +383,33 @@ def test_steps_that_a_program_captures_itself(nm, B, rc, pool):
         for name in ("P", "mP"):
             assert_close_per_model(host(getattr(net, name)), host(getattr(ref, name)), GRAD, 1, 0, "%s after replay %d" % (name, i))
         assert int(net.rng_counter.item()) == int(ref.rng_counter.item())
+
+
+@pytest.mark.parametrize("nm,nf,B,rc,pool,hidden", [(1, 16, 4096, False, "max", 8), (1, 12, 2000, True, "all", 0), (2, 16, 2048, False, "avg", 8), (4, 16, 1030, False, "max", 0),
+                                                    (3, 12, 700, True, "all", 4)])
+def test_single_launch_of_more_regions_per_workgroup_than_pays(nm, nf, B, rc, pool, hidden):
+    """The entry point takes up to sixteen regions per workgroup, also where the net would step in several launches: the same sums in another order."""
+    from deepbind_amd import _lib
+    rng = np.random.default_rng(B)
+    m = 9
+    X, R = _batch(rng, B // (2 if rc else 1), m, 12, 20, reverse_complement=rc)
+    Xd, Rd, Yd = dev(X), dev(R), dev(rng.random((B, nm)).astype(np.float32))
+    make = lambda: _net(np.random.default_rng(1), nm, nf, m, pool, hidden, "nll", rate=0.05, momentum=0.9, dropout=0.5, reverse_complement=rc)[0]
+    net, ref = make(), make()
+    work = None
+    for _ in range(2):
+        net._prepare_step(Xd, Rd, Yd)
+        need = ctypes.c_size_t(0)
+        _lib.call("dbk_train_step_single_workspace", ctypes.addressof(net._step_args), ctypes.addressof(need))
+        assert need.value > 0 and not _lib.dll().dbk_train_step_single_pays(ctypes.addressof(net._step_args))
+        work = torch.zeros(need.value, dtype=torch.uint8, device="cuda") if work is None else work
+        _lib.call("dbk_train_step_single", _lib.stream(), ctypes.addressof(net._step_args), _lib.ptr(work), work.numel())
+        net._L_versions = None
+        net._finish_step(Xd, Rd)
+        ref.train_step(Xd, Rd, Yd)
+        assert not ref._last_single
+    torch.cuda.synchronize()
+    assert work[0:8].view(torch.int32).tolist() == [2, 0]
+    for name in ("P", "mP"):
+        assert_close_per_model(host(getattr(net, name)), host(getattr(ref, name)), GRAD, 1, 0, name)
+    assert int(net.rng_counter.item()) == int(ref.rng_counter.item())
