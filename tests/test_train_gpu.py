@@ -741,12 +741,13 @@ def test_natively_issued_step_equals_the_step_issued_call_by_call(pool, hidden, 
                 assert np.array_equal(getattr(native, name).cpu().numpy(), getattr(stepwise, name).cpu().numpy()), (change, name)
 
 
-@pytest.mark.parametrize("ni,nf,m,pool,hidden,rows", [(1, 5, 7, "max", 0, 33), (3, 7, 11, "avg", 4, 70), (5, 13, 9, "all", 32, 300), (2, 16, 24, "max", 3, 1100),
-                                                      (9, 16, 16, "all", 0, 523)])
+@pytest.mark.parametrize("ni,nf,m,pool,hidden,rows", [(1, 5, 7, "max", 0, 290), (3, 7, 11, "avg", 4, 270), (5, 13, 9, "all", 32, 300), (2, 16, 24, "max", 3, 1100),
+                                                      (9, 16, 16, "all", 0, 523), (1, 16, 8, "max", 0, 3500), (2, 16, 12, "all", 4, 2600)])
 def test_the_update_sums_many_slabs_as_the_gradient_does(ni, nf, m, pool, hidden, rows):
     """From 33 slabs on four waves of the step's last kernel sum 64 elements together: the bits are those of the gradient's own kernel, whose
     sums go one by one, for vectors that are no whole groups of 64, groups that reach from the scan's parameters into the head's, and
-    more slabs than one round takes."""
+    more slabs than the 256 of one round. (Short regions of few filters: eight regions a slab.)"""
+    assert (rows + 7) // 8 > 32 and (rows <= 2048 or (rows + 7) // 8 > 256)
     from deepbind_amd import data, deepity_smat as ds
     from deepbind_amd.model import SequenceNet
     rng = np.random.default_rng(rows)
@@ -808,6 +809,36 @@ def test_groups_stepped_in_shared_launches_match_groups_stepped_alone_across_cha
         assert np.array_equal(host(a.mP), host(b.mP)) and np.array_equal(host(a.dP), host(b.dP))
         assert a.step_count == b.step_count == len(batches) and a._rng_offset == b._rng_offset
         assert host(a.rng_counter) == host(b.rng_counter)
+
+
+@pytest.mark.parametrize("small", ["max", "all"])
+def test_groups_of_few_and_many_slabs_in_one_launch(small):
+    """A group of 64 models, whose 16 tiles of filters leave 30 partial sums of an element, beside one of a single model, which has 38: the update's shared
+    launch sums the first one by one and the second four waves at a time, with the bits of each group's own launch."""
+    from deepbind_amd import data
+    from deepbind_amd.model import ModelGroup
+    rng = np.random.default_rng(9)
+    seqs = ["".join(rng.choice(list("ACGT"), size=rng.integers(10, 40))) for _ in range(300)]
+    X, R = [dev(v) for v in data.pack_sequences(seqs, 15)]
+    Y = dev((rng.random((300, 65)) < 0.5).astype(np.float32))
+
+    def make():
+        grp = ModelGroup(["all"] * 64 + [small], [4] * 64 + [0], 16, 16, loss="nll", rate=0.05, momentum=0.9, dropout=0.5, decay_conv=1e-3,
+                         decay_full=1e-3, weight_decay_start=0, single_launch=False)
+        for gi, (_, net) in enumerate(grp.groups):
+            net.rng_seed = gi
+            net.init_params(0.3, 0.3, 0.05, seed=gi)
+        return grp
+
+    together, alone = make(), make()
+    assert sorted(len(idx) for idx, _ in together.groups) == [1, 64]
+    for _ in range(3):
+        together.train_step(X, R, Y)
+        for idx, net in alone.groups:
+            net.train_step(X, R, Y[:, idx].contiguous())
+    for (_, a), (_, b) in zip(together.groups, alone.groups):
+        for name in ("P", "dP", "mP"):
+            assert torch.equal(getattr(a, name), getattr(b, name)), (a.pool, name)
 
 
 @pytest.mark.parametrize("case", ["mixed_pools_revcomp_input_dropout", "eight_taps", "ten_nets", "different_lengths", "plain_momentum",
