@@ -216,7 +216,7 @@ class SequenceNet(object):
         return work if ent[2] <= 256 else None
 
     def _captured_by_program(self):
-        return not self._own_capture and torch.cuda.is_current_stream_capturing()
+        return not self._own_capture and torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
     def _start_over_in_graphs(self):
         """A step of several launches that a program captures forms the look-ahead itself: what lies beside the parameters when the graph
