@@ -62,12 +62,15 @@ __device__ __forceinline__ float chunk_sum(const reduce_update_args& a, unsigned
     return s;
 }
 
-// From how many slabs on a workgroup sums 64 elements together instead of 256 one by one (slab_sum_together), and the workgroups of a vector.
+// Whether a workgroup sums 64 elements together instead of 256 one by one (slab_sum_together), and the workgroups of a vector.
 // What bounds it is latency: 256 slabs were eight rounds of loads for a thread per element, 98 workgroups in all. us a launch, one by one / together: 1024 pairs of
 // 90-200 letters x 8 models x 16 filters of 32 taps (256 slabs of 16 640 elements) 10.5 / 7.7; 700 x 100-200 x 4 of 30 taps 7.9 / 6.2. With the
-// calibration's 21 slabs a thread per element has all of them in flight.
-constexpr unsigned TOGETHER_SLABS = 32;
-inline unsigned update_grid(size_t elements, unsigned nslab) { return nslab > TOGETHER_SLABS ? dbk::ew_grid(elements, 64) : dbk::ew_grid(elements); }
+// calibration's 21 slabs a thread per element has all of them in flight, and from some 200 workgroups of 256 elements on those hide the rounds of each
+// other: 38 slabs of 102 400 elements 5.3 / 6.5. us a step, together against one by one, mean of 8 to 32 taps, 33-40 / 71-100 / 101-150 slabs: up to 16 000 elements -0.4 /
+// -1.1 / -1.7, 32 000 -0.5 / -0.9 / -1.6, 48 000 -0.3 / -0.5 / -0.7, 64 000 +0.1 / -0.1 / +0.2, 90 000 +0.4 / -0.4, 120 000 +1.0.
+constexpr unsigned TOGETHER_SLABS = 32, TOGETHER_ELEMENTS = 49152;
+__host__ __device__ inline bool sums_together(size_t elements, unsigned nslab) { return nslab > TOGETHER_SLABS && elements <= TOGETHER_ELEMENTS; }
+inline unsigned update_grid(size_t elements, unsigned nslab, size_t losses) { return dbk::ew_grid(elements + losses, sums_together(elements, nslab) ? 64 : 256); }
 
 template <unsigned FLY>
 __device__ __forceinline__ void update_loss(const reduce_update_args& a, unsigned b)
@@ -151,14 +154,14 @@ struct reduce_update_multi_args {
     unsigned first[dbk::MULTI_MAX + 1];
     reduce_update_args g[dbk::MULTI_MAX];
 };
-// TOGETHER: some of the groups have many slabs
+// TOGETHER: some of the groups have many slabs of few elements
 template <bool TOGETHER>
 __global__ __launch_bounds__(256) void k_reduce_update_multi(const reduce_update_multi_args m)
 {
     unsigned g = 0;
     while (g + 1 < m.n && blockIdx.x >= m.first[g + 1]) ++g;
     const unsigned bx = blockIdx.x - m.first[g], gx = m.first[g + 1] - m.first[g];
-    if (TOGETHER && m.g[g].nslab > TOGETHER_SLABS) reduce_update_body<true>(m.g[g], bx, gx);
+    if (TOGETHER && sums_together(m.g[g].nparam, m.g[g].nslab)) reduce_update_body<true>(m.g[g], bx, gx);
     else reduce_update_body<false>(m.g[g], bx, gx);
 }
 
@@ -310,8 +313,8 @@ extern "C" int dbk_train_step(dbk_stream_t stream, const dbk_train_step_args* a)
         reduce_update_args u;
         rc = fill_update(u, a, z, later.slabs, later.slab_stride, later.nslab, later.head_partial, later.head_nchunk, later.head_pstride, draws);
         if (rc) return rc;
-        auto kern = u.nslab > TOGETHER_SLABS ? k_reduce_update<true> : k_reduce_update<false>;
-        hipLaunchKernelGGL(kern, dim3(update_grid(a->nparam + a->nmodel, u.nslab)), dim3(256), 0, dbk::as_stream(stream), u);
+        auto kern = sums_together(a->nparam, u.nslab) ? k_reduce_update<true> : k_reduce_update<false>;
+        hipLaunchKernelGGL(kern, dim3(update_grid(a->nparam, u.nslab, a->nmodel)), dim3(256), 0, dbk::as_stream(stream), u);
         DBK_LAUNCH_OK();
     }
     if (a->decay) {
@@ -418,10 +421,10 @@ extern "C" int dbk_train_steps(dbk_stream_t stream, size_t ngroup, const dbk_tra
         const dbk_train_step_args* a = ord[i];
         rc = fill_update(um.g[i], a, sizes_of(a), sg[i].slabs, sg[i].slab_stride, sg[i].nslab, hg[i].partial, hg[i].nchunk, hg[i].pstride, draws[i]);
         if (rc) return rc;
-        um.first[i + 1] = um.first[i] + update_grid(a->nparam + a->nmodel, um.g[i].nslab);
+        um.first[i + 1] = um.first[i] + update_grid(a->nparam, um.g[i].nslab, a->nmodel);
     }
     bool many = false;
-    for (unsigned i = 0; i < n; ++i) many |= um.g[i].nslab > TOGETHER_SLABS;
+    for (unsigned i = 0; i < n; ++i) many |= sums_together(um.g[i].nparam, um.g[i].nslab);
     auto kern = many ? k_reduce_update_multi<true> : k_reduce_update_multi<false>;
     hipLaunchKernelGGL(kern, dim3(um.first[n]), dim3(256), 0, st, um);
     DBK_LAUNCH_OK();

@@ -742,11 +742,12 @@ def test_natively_issued_step_equals_the_step_issued_call_by_call(pool, hidden, 
 
 
 @pytest.mark.parametrize("ni,nf,m,pool,hidden,rows", [(1, 5, 7, "max", 0, 290), (3, 7, 11, "avg", 4, 270), (5, 13, 9, "all", 32, 300), (2, 16, 24, "max", 3, 1100),
-                                                      (9, 16, 16, "all", 0, 523), (1, 16, 8, "max", 0, 3500), (2, 16, 12, "all", 4, 2600)])
+                                                      (9, 16, 16, "all", 0, 523), (1, 16, 8, "max", 0, 3500), (2, 16, 12, "all", 4, 2600), (64, 16, 12, "max", 0, 800)])
 def test_the_update_sums_many_slabs_as_the_gradient_does(ni, nf, m, pool, hidden, rows):
     """From 33 slabs on four waves of the step's last kernel sum 64 elements together: the bits are those of the gradient's own kernel, whose
     sums go one by one, for vectors that are no whole groups of 64, groups that reach from the scan's parameters into the head's, and
-    more slabs than the 256 of one round. (Short regions of few filters: eight regions a slab.)"""
+    more slabs than the 256 of one round, and a vector (64 models) that is summed one by one for its length. (Short regions of few filters:
+    eight regions a slab; 64 models: 40 slabs.)"""
     assert (rows + 7) // 8 > 32 and (rows <= 2048 or (rows + 7) // 8 > 256)
     from deepbind_amd import data, deepity_smat as ds
     from deepbind_amd.model import SequenceNet
