@@ -1031,7 +1031,8 @@ template <int TB, int NT> constexpr size_t scan_smem() { return 16 + (size_t)WAV
 // and their products take turns instead of waiting for each other's sums. Up to 16 taps, whose digits leave the registers for it (24 taps, us, one /
 // two: average, 30 000 x 101 x 256 251 / 254, max + average 271 / 303). An odd last set is scanned beside nothing, which many others pay for. Of the
 // 3072 waves of two sets (4096 of one) the last round is to have most at work, or to be one of many: a wave has twice the products and no more
-// than two others beside it. us, one / two, max + average, 500 rows x 128 filters: 16 taps, 600 regions (0.4 rounds of the waves of two sets) 22.3 / 25.4, 1200 (0.8) 27.8 / 28.4, 2000 (1.3)
+// than two others beside it. us, one / two, max + average, 500 rows x 128 filters: 16 taps, 600 regions (0.4 rounds of the waves of two sets) 22.3 / 25.4, 1200 (0.8) 27.8 / 28.4
+// (maxima with their places, 12 taps, 27.8 / 29.8), 2000 (1.3)
 // 34.7 / 40.6, 3000 (1.95) 44.3 / 44.4; 64 filters, 3000 (0.98) 31.0 / 29.5; 256 filters, 2000 (2.6) 55.5 / 53.1; 8 taps, 128 filters, 600 18.7 / 20.2, 2000 27.6 / 31.3,
 // 3000 32.6 / 32.9 (average 32.9 / 30.6), 256 filters, 1200 (1.6) 29.8 / 32.1, 2000 41.0 / 38.3.
 // Whole calls, us, one / two: max + average, 20 000 x 30-150 letters x 384 filters x 16 taps 205 / 193, 60 000 x 20-40 x 128 142 / 131; maximum,
@@ -1041,7 +1042,7 @@ inline bool takes_two(unsigned ntile, size_t P)
 {
     if (ntile % 2 != 0 && ntile <= 16) return false;
     const double rounds = (double)((ntile + 1) / 2) * (double)P / (256 * WAVES<2>);
-    return rounds <= 1.0 ? rounds >= 0.75 : rounds >= (TB == 1 ? 1.8 : 2.2);
+    return rounds <= 1.0 ? rounds >= (TB == 1 ? 0.75 : 0.9) : rounds >= (TB == 1 ? 1.8 : 2.2);
 }
 
 template <int PT, bool WANT_ARGMAX, int TB, int NT>

@@ -1677,10 +1677,10 @@ def test_bulk_scan_of_two_sets_of_filters_at_a_time(ks, F, closed, m, ptype):
 
 @pytest.mark.parametrize("ptype", ["max", "avg", "all"])
 @pytest.mark.parametrize("m", [7, 16])
-@pytest.mark.parametrize("F,P,closed", [(33, 2300, ()), (64, 2310, (1,)), (64, 3080, ()), (96, 2500, (2,)), (128, 1160, (0, 3)), (128, 2800, (1,)), (520, 300, (16,)),
+@pytest.mark.parametrize("F,P,closed", [(33, 2300, ()), (64, 2310, (1,)), (64, 2900, (0,)), (64, 3080, ()), (96, 2500, (2,)), (128, 1160, (0, 3)), (128, 2800, (1,)), (520, 300, (16,)),
                                         (520, 800, (16, 3)), (64, 255, ()), (64, 257, (0,)), (32, 1, ())])
 def test_bulk_scan_of_one_and_two_sets_of_filters_by_the_number_of_regions(ks, F, P, closed, m, ptype):
-    """Either side of the numbers of regions from which a wave takes 64 filters (0.75 to 1 round of its waves, then 1.8 or 2.2 on), where
+    """Either side of the numbers of regions from which a wave takes 64 filters (0.75 or 0.9 to 1 round of its waves, then 1.8 or 2.2 on), where
     it takes 32 whatever the regions (three sets), an odd last set among many, fewer regions than workgroups; weights that close windows in some sets."""
     rng, W, b, X, R = _bulk_case(F + P, np.random.default_rng(P).integers(1, 41, P), m, F)
     R[-1, 1] = X.size                                                   # the last region runs into rows the scan does not define
