@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict_
 // LDS), keeps the maximum and the sum of the rows no change of its letters can reach and, one by one, the rows some change
 // can; a wave then takes a letter at a time, its lanes being 4 quarters of the m rows x 16 filters: the rows are scanned anew without that
 // letter, in two halves of its other taps, which leaves one addition for each of the four new ones, and pooled with what is kept (maps' error
-// against float64 2.1e-6 to 6.6e-6, 2.4e-6 to 6.9e-6 with every tap in one chain). That adds a row's taps in another order than the forward pass does, and the
+// against float64 1.1e-6 to 7.1e-6, 1.3e-6 to 8.8e-6 with every tap in one chain). That adds a row's taps in another order than the forward pass does, and the
 // rows of a mean in one that depends on where the workgroup's letters lie, so what a change is measured against is the score of the letter that is there
 // from the same pass (k_mutation_map): letters of equal weight differ by nothing. An unknown letter and a change in two regions (below) have no such
 // score: where filters have equal weights at a tap, their rows are scanned with each new letter in its place, in the order of the rows as they are (scan_changed).
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void k_pack_windows(const uint8_t* __restrict_
 // letter, each of which scanned the rows by itself), where the reference's way (a pass of the
 // whole net per change) scans length + m - 1 rows per change, and launches 15 kernels for it.
 // Measured: 32 sequences of 60-101 letters, both strands, 16 filters of 24 taps: 25 us (a lane per new letter 47), the whole call
-// 104 us from strings to host arrays (125) (74-84 ms when the batch was re-scored once per letter and base).
+// 98 us from strings to host arrays (127) (74-84 ms when the batch was re-scored once per letter and base).
 //
 // The reference changes letter i of EVERY region in pass i; where a region is shorter than its neighbour's i that lands in
 // the pad behind it, which is the next region's leading pad. Those entries are scored with both changes, the rows of either window anew.
