@@ -250,8 +250,8 @@ __device__ __forceinline__ float quarters(const float (&v)[4], Op op)
 
 // NR: rows that a lane scans at a time, of the quarter that it has. SPILLS: one strand only, where a change may lie in two regions (above).
 // Few taps are all latency: a letter's rows take less than fetching them, so their kernels keep fewer reads in flight for the registers' sake and six
-// or five waves per SIMD instead of four. (m <= 8 and m <= 12 went through the kernel of four rows, half and a quarter of which were none. us, with the letters
-// per workgroup chosen below, and the kernel of a lane per new letter: 128 sequences of 60-101, one strand, 4 taps 33 -> 24 / 21, 8 taps 34 -> 27 / 27, 12 taps
+// or five waves per SIMD instead of four. (Up to 12 taps went through the kernel of four rows, of which one, two or three were any. us, with the letters
+// per workgroup chosen below, and the kernel of a lane per new letter: 128 sequences of 60-101, one strand, 4 taps 33 -> 23 / 21, 8 taps 34 -> 27 / 27, 12 taps
 // 39 -> 33 / 35; 64 on both strands 8 taps 28 -> 22 / 24, 12 taps 32 -> 25 / 30.) Eight rows at a time (25 to 64 taps) do not fit the registers of four waves:
 // 26 spills of 108 bytes a lane. Four rows take none, and 79 against 87 us at 25 taps (128 sequences, both strands), but 91 against 88 at 32 and 238 against 227 at 64.
 constexpr int mut_waves(unsigned nr) { return nr <= 2 ? 6 : nr == 3 ? 5 : 4; }
@@ -932,7 +932,7 @@ int dbk_mutation_map(dbk_stream_t stream, const float* W, const float* bias, siz
     // (a lane takes a quarter of the m rows)
     auto pick = [&](auto spills) {
         constexpr bool S = decltype(spills)::value;
-        return m <= 8 ? k_mutation_scores<2, S> : m <= 12 ? k_mutation_scores<3, S> : m <= 16 ? k_mutation_scores<4, S> : m <= 24 ? k_mutation_scores<6, S> : k_mutation_scores<8, S>;
+        return m <= 4 ? k_mutation_scores<1, S> : m <= 8 ? k_mutation_scores<2, S> : m <= 12 ? k_mutation_scores<3, S> : m <= 16 ? k_mutation_scores<4, S> : m <= 24 ? k_mutation_scores<6, S> : k_mutation_scores<8, S>;
     };
     auto kern = strands == 1 ? pick(std::true_type{}) : pick(std::false_type{});
     const size_t smem = mut_smem(pos, m, a.k, hidden);
